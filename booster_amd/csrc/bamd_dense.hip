@@ -1,10 +1,14 @@
 // bamd_dense.hip — products with dense bfloat16 matrices in the packed layout of bamd_dense.h.
-//   dense_gemm_kernel: many rows (prompts).  Weight and activation tiles through two LDS stages in operand order (every LDS access is one contiguous kilobyte per
-//     wave), the next stage's global loads in flight under the matrix instructions.
+//   dense_tile_kernel: many rows (prompts), bfloat16.  Weight and activation tiles global -> LDS by DMA, four or eight stages deep, under the matrix instructions.
+//   dense_gemm_kernel: many rows, 32-bit.  Tiles through two LDS stages in operand order (every LDS access is one contiguous kilobyte per wave), the next stage's global
+//     loads in flight under the matrix instructions.
 //   dense_mv_kernel: few rows (decoding).  The eight or sixteen waves of a block split K; every wave streams its share of a 16-row tile straight from HBM into matrix operands.  With
 //     a single row the mechanism in front of the product (residual + norm + token shift or layer norms, PolyNorm, clamped gated unit, grouped norm, last norm) runs as its prologue, its weights
 //     already requested.
 #include "bamd_dense_device.h"
+#include "bamd_mfma_common.h"
+#include <algorithm>
+#include <type_traits>
 
 // ---- packing at load: value (row, col) of the packed matrix = src[row_off[row] + col_off[col]], zero where either is negative; row tiles go to every step-th row tile of
 // a matrix of ld column blocks ------------------------------------------------------------------------------------------------------------------------------
@@ -19,6 +23,36 @@ void bamd_launch_pack(const uint16_t * src, const int32_t * row_off, const int32
 }
 
 // ---- many rows --------------------------------------------------------------------------------------------------------------------------------------
+// one 16 x 16 result tile of a wave: activation rows from mb, matrix rows from nb; a: the tiles of the same activation rows, j: which one
+template <typename T, int OUT, int NI>
+__device__ __forceinline__ void store_tile(const bamd_v4 (&a)[NI], int j, int mb, int nb, int n_lim, int n_rows, int rows, void * out, int ldo, float limit, int lane) {
+    if (nb >= n_lim) return;
+    if constexpr (OUT == BAMD_OUT_ACT_T) {
+        const int n = nb + (lane & 15), m = mb + (lane >> 4) * 4;
+        if (n >= n_rows) return;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) if (m + k < rows) ((T *) out)[(size_t) n * ldo + m + k] = to_act<T>(a[j][k]);
+    } else if constexpr (OUT == BAMD_OUT_GLU) {                   // tiles in turn: gate, up
+        const int n = (nb >> 1) + (lane >> 4) * 4, m = mb + (lane & 15);
+        if ((j & 1) || m >= rows) return;
+        bamd_v4 o;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) o[k] = clamped_glu(a[j][k], a[j | 1][k], limit);
+        store4<T>((T *) out + (size_t) m * ldo + n, o);
+    } else {
+        const int n = nb + (lane >> 4) * 4, m = mb + (lane & 15);
+        if (m >= rows) return;
+        if constexpr (OUT == BAMD_OUT_F32) {
+            float * o = (float *) out + (size_t) m * ldo + n;
+            if (n + 3 < n_rows) *(bamd_v4 *) o = a[j];
+            else for (int k = 0; k < 4; ++k) if (n + k < n_rows) o[k] = a[j][k];
+        } else {
+            T * o = (T *) out + (size_t) m * ldo + n;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) if (n + k < n_rows) o[k] = to_act<T>(a[j][k]);
+        }
+    }
+}
 // TM activation rows x TN matrix rows per block of four waves (2 x 2); KT 32-column blocks per stage
 template <typename T, int TM, int TN, int KT, int OUT>
 __global__ void __launch_bounds__(256) dense_gemm_kernel(bamd_dense w, const T * x, int ldx, int rows, void * out, int ldo, int n_mt, int n_nt, float limit) {
@@ -96,47 +130,126 @@ __global__ void __launch_bounds__(256) dense_gemm_kernel(bamd_dense w, const T *
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < NI; ++j) {
-            const int mb = m0 + (wm * MI + i) * 16, nb = (n0t + wn * NI + j) * 16;
-            if (nb >= n_lim) continue;
-            if constexpr (OUT == BAMD_OUT_ACT_T) {
-                const int n = nb + (lane & 15), m = mb + (lane >> 4) * 4;
-                if (n >= w.rows) continue;
-#pragma unroll
-                for (int k = 0; k < 4; ++k) if (m + k < rows) ((T *) out)[(size_t) n * ldo + m + k] = to_act<T>(acc[i][j][k]);
-            } else if constexpr (OUT == BAMD_OUT_GLU) {           // tiles in turn: gate, up
-                const int n = (nb >> 1) + (lane >> 4) * 4, m = mb + (lane & 15);
-                if ((j & 1) || m >= rows) continue;
-                bamd_v4 o;
-#pragma unroll
-                for (int k = 0; k < 4; ++k) o[k] = clamped_glu(acc[i][j][k], acc[i][j | 1][k], limit);
-                store4<T>((T *) out + (size_t) m * ldo + n, o);
-            } else {
-                const int n = nb + (lane >> 4) * 4, m = mb + (lane & 15);
-                if (m >= rows) continue;
-                if constexpr (OUT == BAMD_OUT_F32) {
-                    float * o = (float *) out + (size_t) m * ldo + n;
-                    if (n + 3 < w.rows) *(bamd_v4 *) o = acc[i][j];
-                    else for (int k = 0; k < 4; ++k) if (n + k < w.rows) o[k] = acc[i][j][k];
-                } else {
-                    T * o = (T *) out + (size_t) m * ldo + n;
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) if (n + k < w.rows) o[k] = to_act<T>(acc[i][j][k]);
-                }
-            }
-        }
+        for (int j = 0; j < NI; ++j) store_tile<T, OUT>(acc[i], j, m0 + (wm * MI + i) * 16, (n0t + wn * NI + j) * 16, n_lim, w.rows, rows, out, ldo, limit, lane);
 }
-template <typename T, int TM, int TN, int KT, int OUT>
-static int gemm_go(const bamd_dense & w, const void * x, int ldx, int rows, void * out, int ldo, float limit, hipStream_t s) {
+// ---- many rows, bfloat16 -------------------------------------------------------------------------------------------------------------------------------
+// TM activation rows x TN matrix rows per block of WM x WN waves.  Both operands travel global -> LDS by DMA (a kilobyte per instruction: 16 rows x 32 columns), NS stages
+// of 32 columns deep: while the matrix instructions of column block k run from registers, the fragments of k + 1 are read from LDS and the copies of the NS - 2 blocks
+// behind it are under way; one barrier per column block, which waits for copies issued NS - 2 blocks ago.  What bounded the kernel before it (128 x 128, staged through registers) was LDS
+// traffic: a wave tile of 64 x 64 reads as many bytes per matrix instruction as 128 x 64 does per 1.3.  Reads and copies are spread between the rows of matrix instructions:
+// all of them in front of the first costs 15 %.
+// Activations lie in LDS as they come from memory, four lanes on 64 consecutive bytes of a row (one 16-byte piece of 16 rows per four lanes costs the vector memory path
+// four times the lookups: 446 -> 409 us below), the pieces of a row turned by half its number: sixteen rows of one piece then fall on different banks.
+// 2048 x 28672 x 4096: 676 -> 409 us (1176 TFLOP/s); 2048 x 4096 x 14336: 284 -> 185 us (1303); 2048 x 2048 x 2048: 41 -> 22 us; 131 x 8192 x 2048: 23 -> 16 us.
+template <int TM, int TN, int WM, int WN, int NS, int OUT>
+__global__ void __launch_bounds__(64 * WM * WN) dense_tile_kernel(bamd_dense w, const bamd_bf * x, int ldx, int rows, void * out, int ldo, int n_mt, int n_nt, float limit) {
+    constexpr int XT = TM / 16, WT = TN / 16, NW = WM * WN, MI = XT / WM, NI = WT / WN, PX = XT / NW, PW = WT / NW, PER = PX + PW, STAGE = (XT + WT) * 1024;
+    static_assert(XT % NW == 0 && WT % NW == 0 && MI * WM == XT && NI * WN == WT && NS >= 4 && (NS & (NS - 1)) == 0, "");
+    extern __shared__ __align__(16) unsigned char lds[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int total = n_mt * n_nt;
+    int id = blockIdx.x;
+    { const int per = (total + 7) / 8, xcd = id & 7, k = id >> 3; id = xcd * per + k; if (k >= per || id >= total) return; }
+    const int mt = id % n_mt, nt = id / n_mt, m0 = mt * TM, n0t = nt * WT;
+    // this wave's share of a stage: PX operand blocks of activations, PW of weights
+    const unsigned char * xbase = (const unsigned char *) (x + (size_t) m0 * ldx), * wbase = (const unsigned char *) (w.w + (size_t) n0t * w.k_tiles * 512);
+    uint32_t xo[PX], wo[PW];
+#pragma unroll
+    for (int i = 0; i < PX; ++i) { int row = (wave * PX + i) * 16 + (lane >> 2); row = m0 + row < rows ? row : rows - 1 - m0; xo[i] = (uint32_t) row * (uint32_t) ldx * 2u + (uint32_t) ((lane & 3) ^ ((lane >> 3) & 3)) * 16u; }
+#pragma unroll
+    for (int i = 0; i < PW; ++i) { int tile = wave * PW + i; tile = n0t + tile < w.row_tiles ? tile : w.row_tiles - 1 - n0t; wo[i] = (uint32_t) tile * (uint32_t) w.k_tiles * 1024u + (uint32_t) lane * 16u; }
+    const uint32_t xd = (uint32_t) (size_t) (bamd_lds_vp) lds + (uint32_t) wave * PX * 1024u, wd = (uint32_t) (size_t) (bamd_lds_vp) lds + (uint32_t) (XT + wave * PW) * 1024u;
+    const int nk = w.k_tiles;
+    // copy i of PER of stage k (behind the last column block: the last one again, into a stage nobody reads)
+    auto copy = [&](int k, int i) {
+        const int kk = k < nk ? k : nk - 1;
+        const uint32_t st = (uint32_t) (k & (NS - 1)) * STAGE;
+        if (i < PX) lds_dma16_s(xbase + (size_t) kk * 64, xo[i], xd + st + i * 1024u);
+        else lds_dma16_s(wbase + (size_t) kk * 1024, wo[i - PX], wd + st + (i - PX) * 1024u);
+    };
+    const int wm = wave % WM, wn = wave / WM;
+    const unsigned char * xb = lds + (size_t) wm * MI * 1024 + ((lane & 15) * 4 + ((lane >> 4) ^ ((lane >> 1) & 3))) * 16, * wb = lds + (size_t) (XT + wn * NI) * 1024 + lane * 16;
+    bamd_v4 acc[MI][NI];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NI; ++j) acc[i][j] = bamd_v4{ 0, 0, 0, 0 };
+    bamd_bf8 xf[2][MI], wf[2][NI];
+    auto read_x = [&](int k, int p, int i) { xf[p][i] = *(const bamd_bf8 *) (xb + (k & (NS - 1)) * STAGE + i * 1024); };
+    auto read_w = [&](int k, int p, int j) { wf[p][j] = *(const bamd_bf8 *) (wb + (k & (NS - 1)) * STAGE + j * 1024); };
+    auto wait = [&] {                                             // all but the last stage's copies of this wave have landed; then every wave's
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"((NS - 3) * PER) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    auto block = [&](int k, auto par) {
+        constexpr int P = decltype(par)::value;
+        wait();                                                   // stage k + 1 is whole; stage k - 1 is free
+        // MI groups: a row of matrix instructions, and spread over them the copies of stage k + NS - 1 and the reads of stage k + 1
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+#pragma unroll
+            for (int c = i * PER / MI; c < (i + 1) * PER / MI; ++c) copy(k + NS - 1, c);
+#pragma unroll
+            for (int j = i * NI / MI; j < (i + 1) * NI / MI; ++j) read_w(k + 1, P ^ 1, j);
+            read_x(k + 1, P ^ 1, i);
+#pragma unroll
+            for (int j = 0; j < NI; ++j) {
+                if constexpr (OUT == BAMD_OUT_ACT_T) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf[P][i], wf[P][j], acc[i][j], 0, 0, 0);
+                else acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[P][j], xf[P][i], acc[i][j], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+#pragma unroll
+    for (int st = 0; st < NS - 1; ++st)
+#pragma unroll
+        for (int i = 0; i < PER; ++i) copy(st, i);
+    asm volatile("s_waitcnt vmcnt(%0)" :: "n"((NS - 2) * PER) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < MI; ++i) read_x(0, 0, i);
+#pragma unroll
+    for (int j = 0; j < NI; ++j) read_w(0, 0, j);
+    int k = 0;
+    for (; k + 2 <= nk; k += 2) { block(k, std::integral_constant<int, 0>()); block(k + 1, std::integral_constant<int, 1>()); }
+    if (k < nk) block(k, std::integral_constant<int, 0>());
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");              // (no copy outlives the block)
+    const int n_lim = w.row_tiles * 16;
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NI; ++j) store_tile<bamd_bf, OUT>(acc[i], j, m0 + (wm * MI + i) * 16, (n0t + wn * NI + j) * 16, n_lim, w.rows, rows, out, ldo, limit, lane);
+}
+template <int TM, int TN, int WM, int WN, int NS, int OUT>
+static int tile_go(const bamd_dense & w, const void * x, int ldx, int rows, void * out, int ldo, float limit, hipStream_t s) {
     const int n_mt = (rows + TM - 1) / TM, n_nt = (w.row_tiles + TN / 16 - 1) / (TN / 16), per = (n_mt * n_nt + 7) / 8;
-    const size_t lds = 2 * ((size_t) TM / 16 * KT * 64 * 8 * sizeof(T) + (size_t) TN / 16 * KT * 1024);
-    hipLaunchKernelGGL((dense_gemm_kernel<T, TM, TN, KT, OUT>), dim3(per * 8), dim3(256), lds, s, w, (const T *) x, ldx, rows, out, ldo, n_mt, n_nt, limit);
+    hipLaunchKernelGGL((dense_tile_kernel<TM, TN, WM, WN, NS, OUT>), dim3(per * 8), dim3(64 * WM * WN), (size_t) NS * (TM / 16 + TN / 16) * 1024, s, w, (const bamd_bf *) x, ldx, rows, out, ldo, n_mt, n_nt, limit);
     return 0;
 }
+// The tile whose rounds over the 256 CUs end first.  Measured per block of 32 columns, all CUs busy (ns): 256 x 256 700, 128 x 256 450, 128 x 128 250, all three one block per CU,
+// so that a round started is a round paid; 64 x 128 190 and 64 x 64 130 share a CU with two to four others and never take less than 250 and 160.
 template <typename T, int OUT>
 static int gemm_tiles(const bamd_dense & w, const void * x, int ldx, int rows, void * out, int ldo, float limit, hipStream_t s) {
-    if constexpr (sizeof(T) == 2) if ((long) ((rows + 127) / 128) * ((w.row_tiles + 7) / 8) >= 192) return gemm_go<T, 128, 128, 2, OUT>(w, x, ldx, rows, out, ldo, limit, s);
-    return gemm_go<T, 64, 64, sizeof(T) == 2 ? 4 : 2, OUT>(w, x, ldx, rows, out, ldo, limit, s);
+    if constexpr (sizeof(T) == 4) {
+        const int n_mt = (rows + 63) / 64, n_nt = (w.row_tiles + 3) / 4, per = (n_mt * n_nt + 7) / 8;
+        hipLaunchKernelGGL((dense_gemm_kernel<T, 64, 64, 2, OUT>), dim3(per * 8), dim3(256), 2 * (4 * 2 * 64 * 8 * sizeof(T) + 4 * 2 * 1024), s, w, (const T *) x, ldx, rows, out, ldo, n_mt, n_nt, limit);
+        return 0;
+    } else {
+        auto tiles = [&](int tm, int tn) { return (long) ((rows + tm - 1) / tm) * ((w.row_tiles * 16 + tn - 1) / tn); };
+        auto rounds = [&](int tm, int tn, long cost) { return (tiles(tm, tn) + 255) / 256 * 256 * cost; };
+        const long t[5] = { rounds(256, 256, 700), rounds(128, 256, 450), rounds(128, 128, 250), std::max(tiles(64, 128) * 190, 256l * 250), std::max(tiles(64, 64) * 130, 256l * 160) };
+        switch (std::min_element(t, t + 5) - t) {
+            case 0: return tile_go<256, 256, 2, 4, 4, OUT>(w, x, ldx, rows, out, ldo, limit, s);
+            case 1: return tile_go<128, 256, 2, 4, 4, OUT>(w, x, ldx, rows, out, ldo, limit, s);
+            case 2: return tile_go<128, 128, 2, 4, 8, OUT>(w, x, ldx, rows, out, ldo, limit, s);
+            case 3: return tile_go<64, 128, 2, 2, 4, OUT>(w, x, ldx, rows, out, ldo, limit, s);
+        }
+        // one tile per CU at most: twice the stages hide more of the memory's latency (131 x 2048 x 8192: 49 -> 38 us); with more, blocks hide each other's
+        if (tiles(64, 64) <= 256) return tile_go<64, 64, 2, 2, 8, OUT>(w, x, ldx, rows, out, ldo, limit, s);
+        return tile_go<64, 64, 2, 2, 4, OUT>(w, x, ldx, rows, out, ldo, limit, s);
+    }
 }
 // f32 rows are stored four matrix rows at a time: ldo % 4 == 0; x rows start on 16 bytes and hold k_tiles * 32 columns
 template <typename T>

@@ -53,6 +53,20 @@ def test_dense(bamd, dtype, n, k, rows):
                 assert np.abs(bamd.op_dense(w, x, dtype, impl) - want).max() < 8e-6 * scale
 
 
+# one size per tile of the many-row product (256 x 256, 128 x 256, 128 x 128, 64 x 128, 64 x 64 with four and with eight stages), ragged in every dimension, fewer and more column blocks than stages
+@pytest.mark.parametrize("n,rows", [(8170, 2045), (8170, 1000), (4090, 1000), (4090, 1100), (8190, 131), (2047, 131)])
+@pytest.mark.parametrize("k", [1, 70, 300])
+def test_dense_tiles(bamd, n, rows, k):
+    r = np.random.default_rng(n + k + rows)
+    w = so.f32_to_bf16(r.standard_normal((n, k)).astype(np.float32))
+    x = so.round_bf16(r.standard_normal((rows, k)).astype(np.float32))
+    want = x.astype(np.float64) @ so.bf16_to_f32(w).T.astype(np.float64)
+    scale = np.sqrt(np.abs(x).astype(np.float64) ** 2 @ np.abs(so.bf16_to_f32(w)).T.astype(np.float64) ** 2) + 1e-30      # of a sum of k products with random signs
+    for impl, tol in ((0, 8e-6), (2, 2.0 ** -8), (3, 2.0 ** -8)):                    # k <= 300 roundings of 2^-24 | the result rounded to bfloat16 (2^-9 of it)
+        e = np.abs(bamd.op_dense(w, x, "bfloat16", impl) - want)
+        assert (e <= tol * (scale if impl == 0 else np.abs(want) + 0.01 * scale)).all(), impl
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("E,rows,pos0,with_y,with_mu", [(75, 5, 0, True, True), (75, 5, 9, True, True), (33, 1, 4, True, True), (1, 3, 0, True, True), (300, 4, 0, False, True), (96, 3, 2, True, False), (2000, 2, 7, True, True)])
 def test_residual_norm_and_token_shift(bamd, dtype, E, rows, pos0, with_y, with_mu):
