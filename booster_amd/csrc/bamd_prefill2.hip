@@ -542,6 +542,232 @@ __global__ void __launch_bounds__(1024) matmul_mfma3_q4k_kernel(bamd_mma2_args a
     }
 }
 
+// ==== few tokens ==============================================================================================================================
+// A prompt of up to 64 tokens leaves the kernels above without work for the chip: 64-row blocks make 64 of them at 4096 rows, and each walks all of K behind a barrier per
+// super-block that waits for everything it has requested (1.5 us per super-block: 24 us at K = 4096, 84 and, Q6_K, 105 us at K = 14336, whatever the tokens).  Here a block is ONE
+// row tile (16 rows) x up to 16 NTT tokens on twelve waves, one of each kind per SIMD: wave tt < 4 takes token tile tt, four build a quarter of the next super-block's fragments
+// each, four copy (all of it one after the other on four waves: 1230 ns a super-block at 37 tokens; copies spread over consumers and builders: 930 — a copy holds its wave until
+// the vector memory path takes it); the arithmetic, its order and the layouts are those above.  Everything a step reads travels global -> LDS by DMA — token records two
+// super-blocks ahead, the row tile's quants, scales and headers four — and the wait at the end of a step leaves what was issued in it (and the weights issued in the one before)
+// in flight, so that a step is not as long as the memory's latency.  37 tokens, 4096 rows: K = 4096 24.0 -> 12.7 us, K = 14336 84 -> 38 us (Q6_K 105 -> 46 us); the copies of
+// the token records, the same to every block, are 24 us of the 38.
+//   W slot of a super-block   Q4_K / Q5_K: 2 x 1 KiB quants of the two record groups | 1 KiB builder operands | 1 KiB consumer header | Q5_K: 2 x 256 B fifth bits
+//                             Q6_K: 2 x 1 KiB low bits | 2 x 512 B high bits | 2 x 1 KiB builder operands of the e-halves | 64 B of d
+template <int TYPE> struct FewW { static constexpr int SLOT = TYPE == BAMD_Q6_K ? 5184 : TYPE == BAMD_Q5_K ? 4608 : 4096, COPIES = TYPE == BAMD_Q4_K ? 1 : 2; };
+#define XF_RING 3                                         /* super-blocks of token records in LDS */
+#define XF_WRING 5                                        /* of the row tile's operands */
+constexpr int few_records(int ntt) { return (ntt * 16 * BAMD_B16_Q + 63) / 64; }       /* KiB of token records of a super-block */
+template <int TYPE, int NTT> constexpr size_t few_lds() { return (size_t) 16 * X_FR + (size_t) XF_RING * few_records(NTT) * 1024 + (size_t) XF_WRING * FewW<TYPE>::SLOT + 32; }
+template <int TYPE, int EPI, int NTT>
+__global__ void __launch_bounds__(768) matmul_few_kernel(bamd_mma2_args a) {
+    constexpr bool Q5 = TYPE == BAMD_Q5_K, Q6 = TYPE == BAMD_Q6_K;
+    constexpr uint32_t RECB = Q6 ? 1680u : Q5 ? BAMD_RECB_Q5K : BAMD_RECB_Q4K;
+    constexpr int RI = few_records(NTT), RS = RI * 1024, NR = (RI + 3) / 4, NW = FewW<TYPE>::COPIES, WS = FewW<TYPE>::SLOT;
+    constexpr int REC0 = 16 * X_FR, W0 = REC0 + XF_RING * RS, Z0 = W0 + XF_WRING * WS;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = wave_id(), tt = wave, bw = wave & 3, m = lane & 15, g = lane >> 4;
+    const int nb = a.K >> 8, rtg = blockIdx.y, rb = rtg >> 2, rtl = rtg & 3, t0 = blockIdx.x * (16 * NTT);
+    const size_t b16 = BAMD_BLOB16_BYTES(nb);
+    const uint32_t lds0 = (uint32_t) (size_t) (bamd_lds_vp) smem;
+    const bool active = tt < NTT && t0 + tt * 16 < a.T, builder = (wave >> 2) == 1, copier = wave >= 8;
+    // ---- copies.  Token records: RI instructions of 64 16-byte pieces, copier w issues w, w + 4, ... (one short of an instruction repeats its last)
+    uint32_t ro[NR], rd[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+        int k = r * 4 + bw; if (k >= RI) k -= 4;
+        const int idx = k * 64 + lane, tok = idx / BAMD_B16_Q, q = idx - tok * BAMD_B16_Q, tg = t0 + tok < a.T ? t0 + tok : a.T - 1;
+        ro[r] = (uint32_t) ((size_t) tg * b16 + (size_t) q * 16); rd[r] = lds0 + REC0 + (uint32_t) k * 1024u;
+    }
+    auto copy_records = [&](int ci, int slot) {
+        const void * src = uniform_ptr(a.blob16 + (size_t) (ci < nb ? ci : nb - 1) * BAMD_B16_REC);
+#pragma unroll
+        for (int r = 0; r < NR; ++r) lds_dma16_s(src, ro[r], rd[r] + (uint32_t) slot * RS);
+    };
+    // the row tile's operands: a kilobyte per copier, and the fifth bits / high bits and d of Q5_K / Q6_K.  A last tile of 8 (padded) rows takes its first record group twice
+    // (rows 8..15 are never stored)
+    const int rgq = 2 * rtg + (bw & 1), rgc = rgq * 8 < a.nrows_pad ? rgq : rgq - 1;
+    const uint8_t * rec = a.w + (size_t) rgc * nb * RECB, * s1, * s2; uint32_t st1, st2, d1, d2; int n2;
+    if (bw < 2) { s1 = rec; st1 = RECB; d1 = (uint32_t) bw * 1024u; s2 = rec + 1024; st2 = RECB; d2 = Q6 ? 2048u + bw * 512u : 4096u + bw * 256u; n2 = Q6 ? 32 : 16; }
+    else {
+        if (Q6) { s1 = a.ph + ((size_t) rb * nb * 2 + (bw & 1)) * 4096 + (size_t) rtl * 1024; st1 = 8192u; d1 = 3072u + (bw & 1) * 1024u; }
+        else if (bw == 2) { s1 = a.ph + (size_t) rb * nb * 4096 + (size_t) rtl * 1024; st1 = 4096u; d1 = 2048u; }
+        else { s1 = a.ch + (size_t) rb * nb * X3_CHS + (size_t) rtl * X_CH4_RT; st1 = X3_CHS; d1 = 3072u; }       // (640 B are used; a kilobyte from the last row tile ends inside the 3 KiB)
+        s2 = s1; st2 = st1; d2 = d1; n2 = 1;                      // (every copier issues the same number of instructions: this one copies its first bytes again)
+        if (Q6 && bw == 2) { s2 = a.ch + ((size_t) rb * nb * 4 + rtl) * X_CH6_RT; st2 = 4 * X_CH6_RT; d2 = 5120u; n2 = 4; }
+    }
+    auto copy_weights = [&](int ci, int slot) {
+        const size_t k = (size_t) (ci < nb ? ci : nb - 1);
+        const uint32_t w = lds0 + W0 + (uint32_t) slot * WS;
+        const void * p1 = uniform_ptr(s1 + k * st1), * p2 = uniform_ptr(s2 + k * st2);
+        lds_dma16_s(p1, (uint32_t) lane * 16u, w + d1);
+        if (NW == 2 && lane < n2) lds_dma16_s(p2, (uint32_t) lane * 16u, w + d2);
+    };
+    // ---- builder: Q4_K / Q5_K as in the sixteen-wave kernel (record group bq, pieces 2 gh, 2 gh + 1); Q6_K: record group bq, piece gh of both pairs
+    const int bq = bw & 1, gh = bw >> 1, br = Q6 ? (lane >> 2) & 7 : lane >> 3, be = Q6 ? lane & 3 : lane & 7, bp = lane >> 5;
+    auto build45 = [&](const unsigned char * w, unsigned char * fr) {
+        const uint2 raw = *(const uint2 *) (w + bq * 1024 + lane * 16 + gh * 8);
+        const uint32_t q = Q5 ? *(const uint32_t *) (w + 4096 + bq * 256 + lane * 4) : 0u, qs0 = 4u * (uint32_t) gh;
+        const unsigned char * p = w + 2048 + (2 * gh) * 256 + (8 * bq + br) * 16;
+        unsigned char * dst = fr + be * X_FR + ((2 * gh) * 16 + 8 * bq + br) * 16;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const uint32_t wq = j ? raw.y : raw.x;
+            const uint4 s = *(const uint4 *) (p + j * 256);
+            uint32_t lo = wq & 0x0f0f0f0fu, hi = Q5 ? (wq >> 4) & 0x0f0f0f0fu : wq & 0xf0f0f0f0u;      // Q4_K: the high nibbles stay in place (16 n; the scale operand is s / 16)
+            if (Q5) { lo |= ((q >> (qs0 + 2 * j)) & 0x01010101u) << 4; hi |= ((q >> (qs0 + 2 * j + 1)) & 0x01010101u) << 4; }
+            bamd_h2u c0, c1, c2, c3, s0, n0, s1h, n1, a0, a1, a2, a3; s0.u = s.x; n0.u = s.y; s1h.u = s.z; n1.u = s.w;
+            c0.u = __builtin_amdgcn_perm(0x64646464u, lo, 0x04010400u); c1.u = __builtin_amdgcn_perm(0x64646464u, lo, 0x04030402u);
+            c2.u = __builtin_amdgcn_perm(0x64646464u, hi, 0x04010400u); c3.u = __builtin_amdgcn_perm(0x64646464u, hi, 0x04030402u);
+            a0.h = __builtin_elementwise_fma(c0.h, s0.h, n0.h); a1.h = __builtin_elementwise_fma(c1.h, s0.h, n0.h);     // (1024 + n) s - 1024 s = n s, one rounding, exact
+            a2.h = __builtin_elementwise_fma(c2.h, s1h.h, n1.h); a3.h = __builtin_elementwise_fma(c3.h, s1h.h, n1.h);
+            *(uint4 *) (dst + j * 256) = (uint4) { a0.u, a1.u, a2.u, a3.u };
+        }
+    };
+    auto build6 = [&](const unsigned char * w, int h, unsigned char * fr) {
+        const uint2 q = *(const uint2 *) (w + bq * 1024 + (br * 8 + be) * 16 + bp * 8 + h * 64);
+        const uint32_t hq = *(const uint32_t *) (w + 2048 + bq * 512 + (br * 8 + be) * 8 + bp * 4 + h * 32), sh = 4u * (uint32_t) gh;
+        const uint4 s = *(const uint4 *) (w + 3072 + h * 1024 + (2 * bp + gh) * 256 + (8 * bq + br) * 16);
+        const bamd_h2 k1056 = { (_Float16) -1056.f, (_Float16) -1056.f };
+        const uint32_t uA = (__builtin_amdgcn_alignbit(hq, hq, (28u + sh) & 31u) & 0x30303030u) | ((q.x >> sh) & 0x0f0f0f0fu);
+        const uint32_t uB = (__builtin_amdgcn_alignbit(hq, hq, (30u + sh) & 31u) & 0x30303030u) | ((q.y >> sh) & 0x0f0f0f0fu);
+        bamd_h2u c, sa0, sl0, sa1, sl1, x0, x1, x2, x3; sa0.u = s.x; sl0.u = s.y; sa1.u = s.z; sl1.u = s.w;
+        bamd_h2 v0, v1, v2, v3;
+        c.u = __builtin_amdgcn_perm(0x64646464u, uA, 0x04010400u); v0 = c.h + k1056;      // (1024 + q) - 1056 = q - 32, exact
+        c.u = __builtin_amdgcn_perm(0x64646464u, uA, 0x04030402u); v1 = c.h + k1056;
+        c.u = __builtin_amdgcn_perm(0x64646464u, uB, 0x04010400u); v2 = c.h + k1056;
+        c.u = __builtin_amdgcn_perm(0x64646464u, uB, 0x04030402u); v3 = c.h + k1056;
+        unsigned char * dst = fr + be * (2 * X_FR) + ((2 * bp + gh) * 16 + 8 * bq + br) * 16;
+        x0.h = v0 * sa0.h; x1.h = v1 * sa0.h; x2.h = v2 * sa1.h; x3.h = v3 * sa1.h;
+        *(uint4 *) dst = (uint4) { x0.u, x1.u, x2.u, x3.u };
+        x0.h = v0 * sl0.h; x1.h = v1 * sl0.h; x2.h = v2 * sl1.h; x3.h = v3 * sl1.h;
+        *(uint4 *) (dst + X_FR) = (uint4) { x0.u, x1.u, x2.u, x3.u };
+    };
+    unsigned char * const fr0 = smem, * const fr1 = smem + 8 * X_FR;
+    bamd_f4 acc[8], accm[4];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] = (bamd_f4) { 0.f, 0.f, 0.f, 0.f };
+#pragma unroll
+    for (int l = 0; l < 4; ++l) accm[l] = (bamd_f4) { 0.f, 0.f, 0.f, 0.f };
+    const bamd_f4 z = { 0.f, 0.f, 0.f, 0.f };
+    const unsigned char * const zero = smem + Z0;
+    auto consume45 = [&](const unsigned char * recs, const unsigned char * w, const unsigned char * fr) {
+        const unsigned char * tok = recs + (size_t) (tt * 16 + m) * BAMD_B16_REC, * ch = w + 3072;
+        // every operand of the super-block is requested before the first matrix instruction (left to itself the compiler reads two, waits, multiplies: eight LDS latencies in a row)
+        bamd_h8 A[8], B[8]; uint4 ma, mb, sfa, sfb; uint2 m5, s5;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) { A[e] = *(const bamd_h8 *) (fr + e * X_FR + lane * 16); B[e] = *(const bamd_h8 *) (tok + g * 16 + e * 64); }
+        const bamd_f4 h0 = *(const bamd_f4 *) (ch + g * 16), h1 = *(const bamd_f4 *) (ch + 64 + g * 16);
+        const float ydv = *(const float *) (tok + 560);
+        if constexpr (Q5) { m5 = *(const uint2 *) (ch + 128 + m * 32 + g * 8); s5 = *(const uint2 *) (tok + 512 + g * 8); }
+        else {
+            const unsigned char * cm = g == 0 ? ch + 128 + m * 32 : zero;
+            ma = *(const uint4 *) cm; mb = *(const uint4 *) (cm + 16); sfa = *(const uint4 *) (tok + 512); sfb = *(const uint4 *) (tok + 528);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        bamd_f4 si[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) si[e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[e], B[e], z, 0, 0, 0);
+        float D[4], Dm[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { D[i] = ydv * h0[i]; Dm[i] = (-ydv) * h1[i]; }
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[e][i] = fmaf(D[i], si[e][i], acc[e][i]);
+        if constexpr (Q5) {
+            union { uint2 u; bamd_h4 h; } av, bv; av.u = m5; bv.u = s5;
+            const bamd_f4 pm = __builtin_amdgcn_mfma_f32_16x16x16f16(av.h, bv.h, z, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) { const float t = Dm[i] * pm[i]; accm[0][i] = accm[0][i] + t; }
+        } else {
+            const uint2 al[4] = { { ma.x, ma.y }, { ma.z, ma.w }, { mb.x, mb.y }, { mb.z, mb.w } };
+            const uint2 bl[4] = { { sfa.x, sfa.y }, { sfa.z, sfa.w }, { sfb.x, sfb.y }, { sfb.z, sfb.w } };
+            bamd_f4 pm[4];
+#pragma unroll
+            for (int l = 0; l < 4; ++l) { union { uint2 u; bamd_h4 h; } av, bv; av.u = al[l]; bv.u = bl[l]; pm[l] = __builtin_amdgcn_mfma_f32_16x16x16f16(av.h, bv.h, z, 0, 0, 0); }
+#pragma unroll
+            for (int l = 0; l < 4; ++l)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) accm[l][i] = fmaf(Dm[i], pm[l][i], accm[l][i]);
+        }
+    };
+    auto consume6 = [&](const unsigned char * recs, const unsigned char * w, const unsigned char * fr, auto h_tag) {
+        constexpr int H = decltype(h_tag)::value;
+        const unsigned char * tok = recs + (size_t) (tt * 16 + m) * BAMD_B16_REC;
+        const bamd_f4 dw = *(const bamd_f4 *) (w + 5120 + g * 16);
+        const float ydv = *(const float *) (tok + 560);
+        float D[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) D[i] = ydv * dw[i];
+        bamd_f4 s[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {                             // (requested all at once, as above, they hold up the builders, who set the pace here: 52 instead of 46 us)
+            const bamd_h8 b = *(const bamd_h8 *) (tok + g * 16 + (4 * H + e) * 64);
+            const bamd_f4 hi = __builtin_amdgcn_mfma_f32_16x16x32_f16(*(const bamd_h8 *) (fr + e * (2 * X_FR) + lane * 16), b, z, 0, 0, 0);
+            s[e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(*(const bamd_h8 *) (fr + e * (2 * X_FR) + X_FR + lane * 16), b, hi, 0, 0, 0);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[4 * H + e][i] = fmaf(D[i], s[e][i], acc[4 * H + e][i]);
+    };
+    // records of 0 and the operands of 0 and 1 have landed when all but the last NR + 2 NW copies have; so it stays: at the end of step ci the records of ci + 1 (issued in ci - 1) and
+    // the operands of ci + 2 (issued in ci - 2) have landed
+    auto publish = [&] { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(NR + 2 * NW) : "memory"); __builtin_amdgcn_s_barrier(); asm volatile("" ::: "memory"); };
+    auto barrier = [&] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); __builtin_amdgcn_s_barrier(); asm volatile("" ::: "memory"); };
+    if (tid < 8) *(uint32_t *) (smem + Z0 + tid * 4) = 0u;
+    // a loop per kind of wave, barrier for barrier alike (one loop with branches inside moves the 48 accumulators through every join)
+    auto after = [](int s, int by, int ring) { s += by; return s < ring ? s : s - ring; };
+    if (copier) { copy_records(0, 0); copy_weights(0, 0); copy_weights(1, 1); copy_records(1, 1); copy_weights(2, 2); copy_weights(3, 3); }
+    publish();
+    if (copier) {
+        barrier();
+        for (int ci = 0, rs = 0, ws = 0; ci < nb; ++ci, rs = after(rs, 1, XF_RING), ws = after(ws, 1, XF_WRING)) {
+            copy_records(ci + 2, after(rs, 2, XF_RING)); copy_weights(ci + 4, after(ws, 4, XF_WRING));
+            if (Q6) barrier();
+            publish();
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");          // (no copy outlives the block)
+        return;
+    }
+    if (builder) {
+        if constexpr (Q6) build6(smem + W0, 0, fr0); else build45(smem + W0, fr0);
+        barrier();
+        for (int ci = 0, ws = 0; ci < nb; ++ci) {
+            const unsigned char * w = smem + W0 + ws * WS;
+            ws = after(ws, 1, XF_WRING);
+            const unsigned char * wn = smem + W0 + ws * WS;
+            if constexpr (Q6) { build6(w, 1, fr1); barrier(); build6(wn, 0, fr0); }
+            else build45(wn, (ci & 1) ? fr0 : fr1);
+            barrier();
+        }
+        return;
+    }
+    barrier();
+    for (int ci = 0, rs = 0, ws = 0; ci < nb; ++ci, rs = after(rs, 1, XF_RING), ws = after(ws, 1, XF_WRING)) {
+        const unsigned char * recs = smem + REC0 + rs * RS, * w = smem + W0 + ws * WS;
+        if (!active) { if (Q6) barrier(); }
+        else if constexpr (Q6) {
+            consume6(recs, w, fr0, std::integral_constant<int, 0>());
+            barrier();
+            consume6(recs, w, fr1, std::integral_constant<int, 1>());
+        } else consume45(recs, w, (ci & 1) ? fr1 : fr0);
+        barrier();
+    }
+    const int t = t0 + tt * 16 + m, row0 = rtg * 16 + 4 * g;
+    if (!active || t >= a.T) return;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float v = ((acc[0][i] + acc[4][i]) + (acc[2][i] + acc[6][i])) + ((acc[1][i] + acc[5][i]) + (acc[3][i] + acc[7][i]));
+        float val = v;
+        if constexpr (!Q6) { const float mm = Q5 ? accm[0][i] : (accm[0][i] + accm[2][i]) + (accm[1][i] + accm[3][i]); val = v + mm; }
+        if (row0 + i < a.nrows) {
+            const size_t o = (size_t) t * a.ldo + row0 + i;
+            a.out[o] = EPI == BAMD_EPI_ADD ? val + a.res[o] : EPI == BAMD_EPI_SILU_MUL ? v_silu(a.res[o]) * val : val;
+        }
+    }
+}
+
 // ---- host side -----------------------------------------------------------------------------------------------------------------------------
 static inline int x_row_blocks(int nrows_pad) { return (nrows_pad + 63) / 64; }
 static unsigned long long * g_prefill_dbg = nullptr;      // -DX_TIMING builds: where the kernels of the next launches leave their phase clocks (bamd_prefill_dbg)
@@ -590,6 +816,22 @@ int bamd_launch_matmul_mfma2(const void * w_stream, const void * aux, int type, 
         if (epi == BAMD_EPI_ADD)           hipLaunchKernelGGL((KERNEL<BAMD_EPI_ADD __VA_ARGS__>),      grid3, dim3(1024), X3_LDS_BYTES, s, a); \
         else if (epi == BAMD_EPI_SILU_MUL) hipLaunchKernelGGL((KERNEL<BAMD_EPI_SILU_MUL __VA_ARGS__>), grid3, dim3(1024), X3_LDS_BYTES, s, a); \
         else                               hipLaunchKernelGGL((KERNEL<BAMD_EPI_STORE __VA_ARGS__>),    grid3, dim3(1024), X3_LDS_BYTES, s, a); } while (0)
+    // up to 64 tokens: whichever ends first, measured per super-block of a round of 256 blocks (Q4_K): 64-row blocks 1500 ns at any number of tokens, 16-row blocks 480 up to
+    // 32 tokens, 700 up to 48 (790 at K = 4096), 800 above
+    const long c16 = T <= 32 ? 480 : T <= 48 ? 700 : 800;
+    if (T <= 64 && ((nrows_pad + 15) / 16 + 255) / 256 * c16 < ((long) grid.y + 255) / 256 * 1500) {
+#define XF_LAUNCH(TYPE_, NTT_) do { const dim3 gf((T + 16 * NTT_ - 1) / (16 * NTT_), (nrows_pad + 15) / 16); \
+        if (epi == BAMD_EPI_ADD)           hipLaunchKernelGGL((matmul_few_kernel<TYPE_, BAMD_EPI_ADD, NTT_>),      gf, dim3(768), (few_lds<TYPE_, NTT_>()), s, a); \
+        else if (epi == BAMD_EPI_SILU_MUL) hipLaunchKernelGGL((matmul_few_kernel<TYPE_, BAMD_EPI_SILU_MUL, NTT_>), gf, dim3(768), (few_lds<TYPE_, NTT_>()), s, a); \
+        else                               hipLaunchKernelGGL((matmul_few_kernel<TYPE_, BAMD_EPI_STORE, NTT_>),    gf, dim3(768), (few_lds<TYPE_, NTT_>()), s, a); } while (0)
+#define XF_TYPE(TYPE_) do { if (T <= 32) XF_LAUNCH(TYPE_, 2); else if (T <= 48) XF_LAUNCH(TYPE_, 3); else XF_LAUNCH(TYPE_, 4); } while (0)
+        if (type == BAMD_Q6_K)      XF_TYPE(BAMD_Q6_K);
+        else if (type == BAMD_Q5_K) XF_TYPE(BAMD_Q5_K);
+        else                        XF_TYPE(BAMD_Q4_K);
+#undef XF_TYPE
+#undef XF_LAUNCH
+        return 0;
+    }
     if (type == BAMD_Q6_K)      X_LAUNCH(matmul_mfma2_q6k_kernel);
     else if (type == BAMD_Q5_K) X3_LAUNCH(matmul_mfma3_q4k_kernel, , true);
     else                        X3_LAUNCH(matmul_mfma3_q4k_kernel, , false);

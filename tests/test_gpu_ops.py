@@ -247,6 +247,25 @@ def test_mul_mat_batch(bamd, po, t, K, rows, T, impl):
         assert_bits(got[i], want, "mul_mat_batch type %d K %d T %d impl %d token %d" % (t, K, T, impl, i))
 
 
+@pytest.mark.parametrize("t", [12, 13, 14])
+@pytest.mark.parametrize("nb,rows", [(1, 8), (2, 16), (3, 24), (5, 72), (7, 40), (9, 4104)])
+def test_mul_mat_batch_few_tokens(bamd, po, t, nb, rows):
+    """one row tile per block: fewer and more super-blocks than its rings hold, a last tile of eight rows, every edge of the token tiles; the
+    integer-dot kernel is the reference (itself compared with the oracle above), the first and last token are compared with the oracle"""
+    K = nb * 256
+    rng = np.random.default_rng(900 * t + nb)
+    W = random_kquant_tensor(t, K, rows, rng)
+    for T in (1, 2, 16, 17, 32, 33, 48, 49, 64):
+        X = (rng.standard_normal((T, K)) * 3).astype(np.float32)
+        res = rng.standard_normal((T, rows)).astype(np.float32) if T % 2 else None
+        got = bamd.op_mul_mat_batch(t, W, rows, K, X, residual=res, impl=2)
+        want = bamd.op_mul_mat_batch(t, W, rows, K, X, residual=res, impl=0)
+        assert_bits(got, want, "type %d nb %d rows %d T %d" % (t, nb, rows, T))
+        for i in {0, T - 1}:
+            ref = po.mul_mat_q(t, W, rows, K, X[i], nthreads=8)[0]
+            assert_bits(got[i], ref + res[i] if res is not None else ref, "type %d nb %d rows %d T %d token %d" % (t, nb, rows, T, i))
+
+
 def test_attention_long_context_eight_heads_per_kv_head(bamd, po):
     """the 70B head layout at a long context: gq = 8 -> four query heads per workgroup of the softmax + P.V launch (128 KB of probability rows in
     LDS at n_ctx 8192), the V^T ring over 125 blocks, a half block at the end (n_kv % 64 == 32)"""
