@@ -2,7 +2,8 @@
 //   dense_tile_kernel: many rows (prompts), bfloat16.  Weight and activation tiles global -> LDS by DMA, four or eight stages deep, under the matrix instructions.
 //   dense_gemm_kernel: many rows, 32-bit.  Tiles through two LDS stages in operand order (every LDS access is one contiguous kilobyte per wave), the next stage's global
 //     loads in flight under the matrix instructions.
-//   dense_mv_kernel: few rows (decoding).  The eight or sixteen waves of a block split K; every wave streams its share of a 16-row tile straight from HBM into matrix operands.  With
+//   dense_few_kernel: up to 64 rows (decoding several sequences, short prompts), bfloat16.  The waves of a block split K, each with a DMA ring of weights and rows.
+//   dense_mv_kernel: a row (decoding), and up to 64 in 32-bit.  The eight or sixteen waves of a block split K; every wave streams its share of a 16-row tile straight from HBM into matrix operands.  With
 //     a single row the mechanism in front of the product (residual + norm + token shift or layer norms, PolyNorm, clamped gated unit, grouped norm, last norm) runs as its prologue, its weights
 //     already requested.
 #include "bamd_dense_device.h"
@@ -335,6 +336,104 @@ __global__ void __launch_bounds__(64 * NW) dense_mv_kernel(bamd_dense w, bamd_ba
         }
     }
 }
+// Up to 64 rows, bfloat16: NT groups of 16 rows, RT row tiles of the matrix.  Every block reads all the rows: bytes out of L2 (NT per RT of weights) and, read by the lanes of a
+// fragment as above, four times the lookups of the same bytes in one piece, were what the product took (16 rows x 14336 x 4096: 32 us, of which the weights are 19).  Here every
+// wave streams its share of K — RT KiB of weights and NT of the rows per step — by DMA through a ring of NS steps of its own: 64 consecutive bytes of a row per four lanes, read
+// back in fragment order (dense_tile_kernel's layout), no barrier between steps, and while the sums of a group of tiles meet, the next group's first steps are under way.  LDS holds
+// one block of eight waves per CU.  16 x 14336 x 4096: 32.3 -> 27.1 us (4.3 TB/s of weights), 16 x 32000 x 4096: 62 -> 50 (5.3), 45 x 4096 x 14336: 57 -> 48 us.
+template <int NT, int RT, int NS>
+__global__ void __launch_bounds__(512) dense_few_kernel(bamd_dense w, const bamd_bf * x, int ldx, int rows, float * out, int ldo) {
+    constexpr int NW = 8, STEP = (NT + RT) * 1024, RING = NS * STEP;
+    extern __shared__ __align__(16) unsigned char lds[];
+    float * red = (float *) (lds + NW * RING);                    // [wave][RT][NT][64 lanes][4]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int k0 = w.k_tiles * wave / NW, n = w.k_tiles * (wave + 1) / NW - k0, groups = (w.row_tiles + RT - 1) / RT;
+    uint32_t xo[NT];
+#pragma unroll
+    for (int g = 0; g < NT; ++g) { int r = g * 16 + (lane >> 2); r = r < rows ? r : rows - 1; xo[g] = (uint32_t) r * (uint32_t) ldx * 2u + (uint32_t) ((lane & 3) ^ ((lane >> 3) & 3)) * 16u; }
+    const uint32_t ring = (uint32_t) (size_t) (bamd_lds_vp) lds + (uint32_t) wave * RING;
+    const unsigned char * mine = lds + (size_t) wave * RING, * xs = mine + 1024 * RT + ((lane & 15) * 4 + ((lane >> 4) ^ ((lane >> 1) & 3))) * 16;
+    int ct = blockIdx.x, ck = 0, cs = 0;                          // next copy: group of RT row tiles, step, slot
+    auto copy = [&] {                                             // (behind the last step: its bytes again, into slots nobody reads)
+        const size_t k = (size_t) (k0 + ck);
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+            int tile = ct * RT + t; tile = tile < w.row_tiles ? tile : w.row_tiles - 1;
+            lds_dma16_s(w.w + ((size_t) tile * w.k_tiles + k) * 512, (uint32_t) lane * 16u, ring + (uint32_t) cs * STEP + 1024u * t);
+        }
+#pragma unroll
+        for (int g = 0; g < NT; ++g) lds_dma16_s((const unsigned char *) x + k * 64, xo[g], ring + (uint32_t) cs * STEP + 1024u * (g + RT));
+        cs = cs + 1 < NS ? cs + 1 : 0;
+        if (ck + 1 < n) ++ck; else if (ct + (int) gridDim.x < groups) { ck = 0; ct += gridDim.x; }
+    };
+    if (n > 0)
+        for (int i = 0; i < NS - 1; ++i) copy();
+    int slot = 0;
+    for (int grp = blockIdx.x; grp < groups; grp += gridDim.x) {
+        bamd_v4 acc[RT][NT];
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int g = 0; g < NT; ++g) acc[t][g] = bamd_v4{ 0, 0, 0, 0 };
+        for (int i = 0; i < n; ++i) {
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"((NS - 2) * (NT + RT)) : "memory");      // this step has landed; the step before is read
+            copy();
+            const int at = slot * STEP;
+            slot = slot + 1 < NS ? slot + 1 : 0;
+            bamd_bf8 wf[RT], xf[NT];
+#pragma unroll
+            for (int t = 0; t < RT; ++t) wf[t] = *(const bamd_bf8 *) (mine + at + t * 1024 + lane * 16);
+#pragma unroll
+            for (int g = 0; g < NT; ++g) xf[g] = *(const bamd_bf8 *) (xs + at + g * 1024);
+#pragma unroll
+            for (int t = 0; t < RT; ++t)
+#pragma unroll
+                for (int g = 0; g < NT; ++g) acc[t][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[t], xf[g], acc[t][g], 0, 0, 0);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();                             // (the sums of the tiles before are read)
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int g = 0; g < NT; ++g) *(bamd_v4 *) (red + (((wave * RT + t) * NT + g) * 64 + lane) * 4) = acc[t][g];
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        for (int i = tid; i < RT * NT * 256; i += 64 * NW) {
+            const int c = i >> 8, l = (i >> 2) & 63, k = i & 3, r = (c % NT) * 16 + (l & 15), o = (grp * RT + c / NT) * 16 + (l >> 4) * 4 + k;
+            if (r < rows && o < w.rows) {
+                float v = 0.f;
+#pragma unroll
+                for (int q = 0; q < NW; ++q) v += red[((q * RT * NT + c) * 64 + l) * 4 + k];
+                out[(size_t) r * ldo + o] = v;
+            }
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");              // (no copy outlives the block)
+}
+template <int NT, int RT, int NS>
+static void few_go(const bamd_dense & w, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s) {
+    const int groups = (w.row_tiles + RT - 1) / RT;
+    hipLaunchKernelGGL((dense_few_kernel<NT, RT, NS>), dim3(groups < 256 ? groups : 256), dim3(512), (size_t) 8 * (NS * (NT + RT) + NT * RT) * 1024, s, w, (const bamd_bf *) x, ldx, rows, out, ldo);
+}
+// RT by the rounds over the CUs; a round of 1, 2 or 3 tiles at K = 4096 takes 7.1, 12.7 and 16 us with up to 16 rows, one of 1 or 2 tiles 9.0 and 15.1 us with up to 32.
+// With more rows the 64 x 64 tiles of prompts are ahead once they fill the CUs (45 x 22672 x 4096: 49 against 74 us) and behind before (45 x 4096 x 14336: 136 against 48)
+static int few_pick(const bamd_dense & w, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s) {
+    const long rounds[3] = { (w.row_tiles + 255) / 256, (w.row_tiles + 511) / 512, (w.row_tiles + 767) / 768 };
+    if (rows > 32) {
+        if (w.row_tiles > 768 && (ldo & 3) == 0) return gemm_tiles<bamd_bf, BAMD_OUT_F32>(w, x, ldx, rows, out, ldo, 0.f, s);
+        few_go<4, 1, 3>(w, x, ldx, rows, out, ldo, s);
+    } else if (rows > 16) {
+        if (rounds[0] * 90 <= rounds[1] * 151) few_go<2, 1, 5>(w, x, ldx, rows, out, ldo, s); else few_go<2, 2, 4>(w, x, ldx, rows, out, ldo, s);
+    } else {
+        const long t1 = rounds[0] * 71, t2 = rounds[1] * 127, t3 = rounds[2] * 160;
+        if (t1 <= t2 && t1 <= t3) few_go<1, 1, 5>(w, x, ldx, rows, out, ldo, s);
+        else if (t2 <= t3) few_go<1, 2, 5>(w, x, ldx, rows, out, ldo, s);
+        else few_go<1, 3, 4>(w, x, ldx, rows, out, ldo, s);
+    }
+    return 0;
+}
 size_t bamd_dense_mv_lds(int act, int K) { return (size_t) (K + 31) / 32 * 32 * (act == BAMD_ACT_F32 ? 4 : 2); }
 template <typename T, int NT, int NW, int PRE>
 static void mv_go(const bamd_dense & w, const bamd_batch_dev & b, const bamd_pre_args & p, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s) {
@@ -363,7 +462,8 @@ static int mv_pick(const bamd_dense & w, int pre, const bamd_batch_dev & b, cons
         return 0;
     }
     if (rows < 1 || rows > BAMD_MV_ROWS || ldx < w.k_tiles * 32 || (ldx & 7)) return 1;
-    if (rows <= 16) mv_one<T, BAMD_PRE_ROWS>(w, b, p, x, ldx, rows, out, ldo, s);
+    if constexpr (sizeof(T) == 2) return few_pick(w, x, ldx, rows, out, ldo, s);
+    else if (rows <= 16) mv_one<T, BAMD_PRE_ROWS>(w, b, p, x, ldx, rows, out, ldo, s);
     else if (rows <= 32) mv_go<T, 2, 8, BAMD_PRE_ROWS>(w, b, p, x, ldx, rows, out, ldo, s);
     else mv_go<T, 4, 8, BAMD_PRE_ROWS>(w, b, p, x, ldx, rows, out, ldo, s);
     return 0;

@@ -67,6 +67,18 @@ def test_dense_tiles(bamd, n, rows, k):
         assert (e <= tol * (scale if impl == 0 else np.abs(want) + 0.01 * scale)).all(), impl
 
 
+# one, two and three row tiles per step with a remainder, every group of rows and its edges, fewer column blocks than waves and more than a ring holds
+@pytest.mark.parametrize("n,rows", [(2030, 1), (2030, 16), (4620, 2), (11000, 15), (4100, 17), (4620, 32), (4620, 33), (12400, 33), (520, 64)])
+@pytest.mark.parametrize("k", [1, 230, 2050])
+def test_dense_few_rows(bamd, n, rows, k):
+    r = np.random.default_rng(n + k + rows)
+    w = so.f32_to_bf16(r.standard_normal((n, k)).astype(np.float32))
+    x = so.round_bf16(r.standard_normal((rows, k)).astype(np.float32))
+    want = x.astype(np.float64) @ so.bf16_to_f32(w).T.astype(np.float64)
+    scale = np.sqrt(np.abs(x).astype(np.float64) ** 2 @ np.abs(so.bf16_to_f32(w)).T.astype(np.float64) ** 2) + 1e-30      # of a sum of k products with random signs
+    assert (np.abs(bamd.op_dense(w, x, "bfloat16", 1) - want) <= 1e-5 * scale).all()                 # sqrt(k) <= 46 roundings of 2^-24 in a row, three times over
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("E,rows,pos0,with_y,with_mu", [(75, 5, 0, True, True), (75, 5, 9, True, True), (33, 1, 4, True, True), (1, 3, 0, True, True), (300, 4, 0, False, True), (96, 3, 2, True, False), (2000, 2, 7, True, True)])
 def test_residual_norm_and_token_shift(bamd, dtype, E, rows, pos0, with_y, with_mu):
