@@ -35,6 +35,7 @@ struct bamd_batch_dev {            // device arrays of a step
 enum { BAMD_NORM_RMS = 0, BAMD_NORM_LAYER = 1 };
 struct bamd_residual_args {
     const float * x, * y; int ldy, norm; const float * g; float eps;
+    int parts; size_t plane;                       // y is the sum of so many planes (a product whose K was halved: 2; 0 or 1: one)
     const float * mu; float * prev;                // prev: [2][n_seq][E]
     const float * gi;
     float * xo; void * h; int E, ldh;              // xo [rows][E]; h [rows][ldh], zero beyond E (null: not wanted)
@@ -62,12 +63,13 @@ void bamd_launch_advance(bamd_entry * ent, int32_t * tokens, unsigned long long 
 // ---- dense matrices -------------------------------------------------------------------------------------------------------------------------------
 // f32 [rows][ldo] | activation type [rows][ldo] | activation type, transposed [n][ldo] | activation type, the clamped gated unit of alternating 16-row tiles [rows][ldo]
 enum { BAMD_OUT_F32 = 0, BAMD_OUT_ACT = 1, BAMD_OUT_ACT_T = 2, BAMD_OUT_GLU = 3 };
-int bamd_launch_dense_gemm(int act, const bamd_dense & w, const void * x, int ldx, int rows, void * out, int ldo, int out_kind, hipStream_t s, float limit = 0.f);
+// parts: in, how many shares of K the caller can take (f32 results only; share i goes to out + i * rows * ldo); out, how many there are: one or two
+int bamd_launch_dense_gemm(int act, const bamd_dense & w, const void * x, int ldx, int rows, void * out, int ldo, int out_kind, hipStream_t s, float limit = 0.f, int * parts = nullptr);
 // few rows (<= BAMD_MV_ROWS): the weights stream once; out f32 [rows][ldo].  pre: how the operand comes about —
 enum { BAMD_PRE_ROWS = 0, BAMD_PRE_RESIDUAL = 1, BAMD_PRE_POLY = 2, BAMD_PRE_GROUP = 3, BAMD_PRE_FINAL = 4, BAMD_PRE_GLU = 5, BAMD_PRE_LAYER = 6 };     // (LAYER: RESIDUAL and FINAL with layer norms, chosen by res.norm); x given | one row, built in front of the product from the argument block
 struct bamd_pre_args { bamd_residual_args res; bamd_poly_args poly; bamd_group_norm_args grp; bamd_glu_args glu; const float * gf; const int32_t * want; };
 #define BAMD_MV_ROWS 64
-int bamd_launch_dense_mv(int act, const bamd_dense & w, int pre, const bamd_batch_dev & b, const bamd_pre_args * p, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s);
+int bamd_launch_dense_mv(int act, const bamd_dense & w, int pre, const bamd_batch_dev & b, const bamd_pre_args * p, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s, int * parts = nullptr);
 size_t bamd_dense_mv_lds(int act, int K);         // operand bytes of a built row: must stay within BAMD_MV_LDS
 #define BAMD_MV_LDS (96 * 1024)
 

@@ -144,6 +144,7 @@ __global__ void __launch_bounds__(256) dense_gemm_kernel(bamd_dense w, const T *
 // 2048 x 28672 x 4096: 676 -> 409 us (1176 TFLOP/s); 2048 x 4096 x 14336: 284 -> 185 us (1303); 2048 x 2048 x 2048: 41 -> 22 us; 131 x 8192 x 2048: 23 -> 16 us.
 template <int TM, int TN, int WM, int WN, int NS, int OUT>
 __global__ void __launch_bounds__(64 * WM * WN) dense_tile_kernel(bamd_dense w, const bamd_bf * x, int ldx, int rows, void * out, int ldo, int n_mt, int n_nt, float limit) {
+    const int kb = (int) ((long) w.k_tiles * blockIdx.y / gridDim.y), nk = (int) ((long) w.k_tiles * (blockIdx.y + 1) / gridDim.y) - kb;      // this block's share of K
     constexpr int XT = TM / 16, WT = TN / 16, NW = WM * WN, MI = XT / WM, NI = WT / WN, PX = XT / NW, PW = WT / NW, PER = PX + PW, STAGE = (XT + WT) * 1024;
     static_assert(XT % NW == 0 && WT % NW == 0 && MI * WM == XT && NI * WN == WT && NS >= 4 && (NS & (NS - 1)) == 0, "");
     extern __shared__ __align__(16) unsigned char lds[];
@@ -153,14 +154,13 @@ __global__ void __launch_bounds__(64 * WM * WN) dense_tile_kernel(bamd_dense w, 
     { const int per = (total + 7) / 8, xcd = id & 7, k = id >> 3; id = xcd * per + k; if (k >= per || id >= total) return; }
     const int mt = id % n_mt, nt = id / n_mt, m0 = mt * TM, n0t = nt * WT;
     // this wave's share of a stage: PX operand blocks of activations, PW of weights
-    const unsigned char * xbase = (const unsigned char *) (x + (size_t) m0 * ldx), * wbase = (const unsigned char *) (w.w + (size_t) n0t * w.k_tiles * 512);
+    const unsigned char * xbase = (const unsigned char *) (x + (size_t) m0 * ldx + (size_t) kb * 32), * wbase = (const unsigned char *) (w.w + ((size_t) n0t * w.k_tiles + kb) * 512);
     uint32_t xo[PX], wo[PW];
 #pragma unroll
     for (int i = 0; i < PX; ++i) { int row = (wave * PX + i) * 16 + (lane >> 2); row = m0 + row < rows ? row : rows - 1 - m0; xo[i] = (uint32_t) row * (uint32_t) ldx * 2u + (uint32_t) ((lane & 3) ^ ((lane >> 3) & 3)) * 16u; }
 #pragma unroll
     for (int i = 0; i < PW; ++i) { int tile = wave * PW + i; tile = n0t + tile < w.row_tiles ? tile : w.row_tiles - 1 - n0t; wo[i] = (uint32_t) tile * (uint32_t) w.k_tiles * 1024u + (uint32_t) lane * 16u; }
     const uint32_t xd = (uint32_t) (size_t) (bamd_lds_vp) lds + (uint32_t) wave * PX * 1024u, wd = (uint32_t) (size_t) (bamd_lds_vp) lds + (uint32_t) (XT + wave * PW) * 1024u;
-    const int nk = w.k_tiles;
     // copy i of PER of stage k (behind the last column block: the last one again, into a stage nobody reads)
     auto copy = [&](int k, int i) {
         const int kk = k < nk ? k : nk - 1;
@@ -218,54 +218,66 @@ __global__ void __launch_bounds__(64 * WM * WN) dense_tile_kernel(bamd_dense w, 
     if (k < nk) block(k, std::integral_constant<int, 0>());
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");              // (no copy outlives the block)
     const int n_lim = w.row_tiles * 16;
+    if constexpr (OUT == BAMD_OUT_F32) out = (float *) out + (size_t) blockIdx.y * rows * ldo;
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < NI; ++j) store_tile<bamd_bf, OUT>(acc[i], j, m0 + (wm * MI + i) * 16, (n0t + wn * NI + j) * 16, n_lim, w.rows, rows, out, ldo, limit, lane);
 }
 template <int TM, int TN, int WM, int WN, int NS, int OUT>
-static int tile_go(const bamd_dense & w, const void * x, int ldx, int rows, void * out, int ldo, float limit, hipStream_t s) {
+static int tile_go(const bamd_dense & w, const void * x, int ldx, int rows, void * out, int ldo, float limit, int parts, hipStream_t s) {
     const int n_mt = (rows + TM - 1) / TM, n_nt = (w.row_tiles + TN / 16 - 1) / (TN / 16), per = (n_mt * n_nt + 7) / 8;
-    hipLaunchKernelGGL((dense_tile_kernel<TM, TN, WM, WN, NS, OUT>), dim3(per * 8), dim3(64 * WM * WN), (size_t) NS * (TM / 16 + TN / 16) * 1024, s, w, (const bamd_bf *) x, ldx, rows, out, ldo, n_mt, n_nt, limit);
+    hipLaunchKernelGGL((dense_tile_kernel<TM, TN, WM, WN, NS, OUT>), dim3(per * 8, parts), dim3(64 * WM * WN), (size_t) NS * (TM / 16 + TN / 16) * 1024, s, w, (const bamd_bf *) x, ldx, rows, out, ldo, n_mt, n_nt, limit);
     return 0;
 }
 // The tile whose rounds over the 256 CUs end first.  Measured per block of 32 columns, all CUs busy (ns): 256 x 256 700, 128 x 256 450, 128 x 128 250, all three one block per CU,
-// so that a round started is a round paid; 64 x 128 190 and 64 x 64 130 share a CU with two to four others and never take less than 250 and 160.
+// so that a round started is a round paid; 64 x 128 190 and 64 x 64 160 share a CU with two to four others and never take less than 250 and 160.  Where even the small tiles leave
+// CUs idle and the reader of the result can add planes, K is halved: two planes cost their bytes twice (at 4 TB/s) and blocks their
+// start and end once more (4 us).  131 x 2048 x 8192: 38 -> 22 us, 412 x 4096 x 8192: 85 -> 39; four shares were no faster (24 and 43 us)
 template <typename T, int OUT>
-static int gemm_tiles(const bamd_dense & w, const void * x, int ldx, int rows, void * out, int ldo, float limit, hipStream_t s) {
+static int gemm_tiles(const bamd_dense & w, const void * x, int ldx, int rows, void * out, int ldo, float limit, hipStream_t s, int * parts = nullptr) {
     if constexpr (sizeof(T) == 4) {
+        if (parts) *parts = 1;
         const int n_mt = (rows + 63) / 64, n_nt = (w.row_tiles + 3) / 4, per = (n_mt * n_nt + 7) / 8;
         hipLaunchKernelGGL((dense_gemm_kernel<T, 64, 64, 2, OUT>), dim3(per * 8), dim3(256), 2 * (4 * 2 * 64 * 8 * sizeof(T) + 4 * 2 * 1024), s, w, (const T *) x, ldx, rows, out, ldo, n_mt, n_nt, limit);
         return 0;
     } else {
         auto tiles = [&](int tm, int tn) { return (long) ((rows + tm - 1) / tm) * ((w.row_tiles * 16 + tn - 1) / tn); };
-        auto rounds = [&](int tm, int tn, long cost) { return (tiles(tm, tn) + 255) / 256 * 256 * cost; };
-        const long t[5] = { rounds(256, 256, 700), rounds(128, 256, 450), rounds(128, 128, 250), std::max(tiles(64, 128) * 190, 256l * 250), std::max(tiles(64, 64) * 130, 256l * 160) };
-        switch (std::min_element(t, t + 5) - t) {
-            case 0: return tile_go<256, 256, 2, 4, 4, OUT>(w, x, ldx, rows, out, ldo, limit, s);
-            case 1: return tile_go<128, 256, 2, 4, 4, OUT>(w, x, ldx, rows, out, ldo, limit, s);
-            case 2: return tile_go<128, 128, 2, 4, 8, OUT>(w, x, ldx, rows, out, ldo, limit, s);
-            case 3: return tile_go<64, 128, 2, 2, 4, OUT>(w, x, ldx, rows, out, ldo, limit, s);
+        long best = 0; int pick = 0, share = 1;
+        for (int p = 1; p <= (OUT == BAMD_OUT_F32 && parts ? *parts : 1) && p <= 2 && (p == 1 || w.k_tiles >= 32); ++p) {
+            auto rounds = [&](int tm, int tn, long cost) { return (tiles(tm, tn) * p + 255) / 256 * cost; };
+            const long t[5] = { rounds(256, 256, 700), rounds(128, 256, 450), rounds(128, 128, 250), std::max(tiles(64, 128) * p * 190 / 256, 250l), std::max(tiles(64, 64) * p * 160 / 256, 160l) };
+            const int i = (int) (std::min_element(t, t + 5) - t);
+            const long ns = t[i] * ((w.k_tiles + p - 1) / p) + (p > 1 ? 4000 + (long) p * rows * w.row_tiles * 16 / 500 : 0);
+            if (p == 1 || ns < best) { best = ns; pick = i; share = p; }
+        }
+        if (parts) *parts = share;
+        switch (pick) {
+            case 0: return tile_go<256, 256, 2, 4, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
+            case 1: return tile_go<128, 256, 2, 4, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
+            case 2: return tile_go<128, 128, 2, 4, 8, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
+            case 3: return tile_go<64, 128, 2, 2, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
         }
         // one tile per CU at most: twice the stages hide more of the memory's latency (131 x 2048 x 8192: 49 -> 38 us); with more, blocks hide each other's
-        if (tiles(64, 64) <= 256) return tile_go<64, 64, 2, 2, 8, OUT>(w, x, ldx, rows, out, ldo, limit, s);
-        return tile_go<64, 64, 2, 2, 4, OUT>(w, x, ldx, rows, out, ldo, limit, s);
+        if (tiles(64, 64) * share <= 256) return tile_go<64, 64, 2, 2, 8, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
+        return tile_go<64, 64, 2, 2, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
     }
 }
 // f32 rows are stored four matrix rows at a time: ldo % 4 == 0; x rows start on 16 bytes and hold k_tiles * 32 columns
 template <typename T>
-static int gemm_out(const bamd_dense & w, const void * x, int ldx, int rows, void * out, int ldo, int kind, float limit, hipStream_t s) {
+static int gemm_out(const bamd_dense & w, const void * x, int ldx, int rows, void * out, int ldo, int kind, float limit, hipStream_t s, int * parts) {
+    if (kind != BAMD_OUT_F32 && parts) *parts = 1;
     switch (kind) {
-        case BAMD_OUT_F32: return gemm_tiles<T, BAMD_OUT_F32>(w, x, ldx, rows, out, ldo, limit, s);
+        case BAMD_OUT_F32: return gemm_tiles<T, BAMD_OUT_F32>(w, x, ldx, rows, out, ldo, limit, s, parts);
         case BAMD_OUT_ACT: return gemm_tiles<T, BAMD_OUT_ACT>(w, x, ldx, rows, out, ldo, limit, s);
         case BAMD_OUT_ACT_T: return gemm_tiles<T, BAMD_OUT_ACT_T>(w, x, ldx, rows, out, ldo, limit, s);
         case BAMD_OUT_GLU: return (w.row_tiles & 1) || ldo < w.row_tiles * 8 ? 1 : gemm_tiles<T, BAMD_OUT_GLU>(w, x, ldx, rows, out, ldo, limit, s);
     }
     return 1;
 }
-int bamd_launch_dense_gemm(int act, const bamd_dense & w, const void * x, int ldx, int rows, void * out, int ldo, int kind, hipStream_t s, float limit) {
+int bamd_launch_dense_gemm(int act, const bamd_dense & w, const void * x, int ldx, int rows, void * out, int ldo, int kind, hipStream_t s, float limit, int * parts) {
     if (rows < 1 || w.row_tiles < 1 || w.k_tiles < 1 || ldx < w.k_tiles * 32 || (ldx & 7) || (ldo & 3)) return 1;
-    return act == BAMD_ACT_F32 ? gemm_out<float>(w, x, ldx, rows, out, ldo, kind, limit, s) : gemm_out<bamd_bf>(w, x, ldx, rows, out, ldo, kind, limit, s);
+    return act == BAMD_ACT_F32 ? gemm_out<float>(w, x, ldx, rows, out, ldo, kind, limit, s, parts) : gemm_out<bamd_bf>(w, x, ldx, rows, out, ldo, kind, limit, s, parts);
 }
 
 // ---- few rows ---------------------------------------------------------------------------------------------------------------------------------------
@@ -276,7 +288,9 @@ __global__ void __launch_bounds__(64 * NW) dense_mv_kernel(bamd_dense w, bamd_ba
     extern __shared__ __align__(16) unsigned char lds[];
     __shared__ float red[NW * NT * 256];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int k0 = w.k_tiles * wave / NW, k1 = w.k_tiles * (wave + 1) / NW, kn = (w.k_tiles + NW - 1) / NW, nc = (kn + U - 1) / U;
+    const int kb = w.k_tiles * blockIdx.y / gridDim.y, ke = w.k_tiles * (blockIdx.y + 1) / gridDim.y;      // the block's share of K, and the wave's
+    const int k0 = kb + (ke - kb) * wave / NW, k1 = kb + (ke - kb) * (wave + 1) / NW, kn = (ke - kb + NW - 1) / NW, nc = (kn + U - 1) / U;
+    out += (size_t) blockIdx.y * rows * ldo;
     bamd_u4 cur[U], nxt[U] = {};
     auto request = [&](int tile, int c, bamd_u4 * d) {
         const uint16_t * base = w.w + ((size_t) tile * w.k_tiles * 64 + lane) * 8;
@@ -347,7 +361,9 @@ __global__ void __launch_bounds__(512) dense_few_kernel(bamd_dense w, const bamd
     extern __shared__ __align__(16) unsigned char lds[];
     float * red = (float *) (lds + NW * RING);                    // [wave][RT][NT][64 lanes][4]
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int k0 = w.k_tiles * wave / NW, n = w.k_tiles * (wave + 1) / NW - k0, groups = (w.row_tiles + RT - 1) / RT;
+    const int kb = w.k_tiles * blockIdx.y / gridDim.y, ke = w.k_tiles * (blockIdx.y + 1) / gridDim.y, k0 = kb + (ke - kb) * wave / NW, n = kb + (ke - kb) * (wave + 1) / NW - k0;      // the block's share of K, and the wave's
+    const int groups = (w.row_tiles + RT - 1) / RT;
+    out += (size_t) blockIdx.y * rows * ldo;
     uint32_t xo[NT];
 #pragma unroll
     for (int g = 0; g < NT; ++g) { int r = g * 16 + (lane >> 2); r = r < rows ? r : rows - 1; xo[g] = (uint32_t) r * (uint32_t) ldx * 2u + (uint32_t) ((lane & 3) ^ ((lane >> 3) & 3)) * 16u; }
@@ -413,22 +429,22 @@ __global__ void __launch_bounds__(512) dense_few_kernel(bamd_dense w, const bamd
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");              // (no copy outlives the block)
 }
 template <int NT, int RT, int NS>
-static void few_go(const bamd_dense & w, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s) {
+static void few_go(const bamd_dense & w, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s, int parts = 1) {
     const int groups = (w.row_tiles + RT - 1) / RT;
-    hipLaunchKernelGGL((dense_few_kernel<NT, RT, NS>), dim3(groups < 256 ? groups : 256), dim3(512), (size_t) 8 * (NS * (NT + RT) + NT * RT) * 1024, s, w, (const bamd_bf *) x, ldx, rows, out, ldo);
+    hipLaunchKernelGGL((dense_few_kernel<NT, RT, NS>), dim3(groups < 256 ? groups : 256, parts), dim3(512), (size_t) 8 * (NS * (NT + RT) + NT * RT) * 1024, s, w, (const bamd_bf *) x, ldx, rows, out, ldo);
 }
 // RT by the rounds over the CUs; a round of 1, 2 or 3 tiles at K = 4096 takes 7.1, 12.7 and 16 us with up to 16 rows, one of 1 or 2 tiles 9.0 and 15.1 us with up to 32.
 // With more rows the 64 x 64 tiles of prompts are ahead once they fill the CUs (45 x 22672 x 4096: 49 against 74 us) and behind before (45 x 4096 x 14336: 136 against 48)
-static int few_pick(const bamd_dense & w, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s) {
+static int few_pick(const bamd_dense & w, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s, int parts) {
     const long rounds[3] = { (w.row_tiles + 255) / 256, (w.row_tiles + 511) / 512, (w.row_tiles + 767) / 768 };
     if (rows > 32) {
         if (w.row_tiles > 768 && (ldo & 3) == 0) return gemm_tiles<bamd_bf, BAMD_OUT_F32>(w, x, ldx, rows, out, ldo, 0.f, s);
-        few_go<4, 1, 3>(w, x, ldx, rows, out, ldo, s);
+        few_go<4, 1, 3>(w, x, ldx, rows, out, ldo, s, parts);
     } else if (rows > 16) {
-        if (rounds[0] * 90 <= rounds[1] * 151) few_go<2, 1, 5>(w, x, ldx, rows, out, ldo, s); else few_go<2, 2, 4>(w, x, ldx, rows, out, ldo, s);
+        if (rounds[0] * 90 <= rounds[1] * 151) few_go<2, 1, 5>(w, x, ldx, rows, out, ldo, s, parts); else few_go<2, 2, 4>(w, x, ldx, rows, out, ldo, s);
     } else {
         const long t1 = rounds[0] * 71, t2 = rounds[1] * 127, t3 = rounds[2] * 160;
-        if (t1 <= t2 && t1 <= t3) few_go<1, 1, 5>(w, x, ldx, rows, out, ldo, s);
+        if (t1 <= t2 && t1 <= t3) few_go<1, 1, 5>(w, x, ldx, rows, out, ldo, s, parts);
         else if (t2 <= t3) few_go<1, 2, 5>(w, x, ldx, rows, out, ldo, s);
         else few_go<1, 3, 4>(w, x, ldx, rows, out, ldo, s);
     }
@@ -436,39 +452,45 @@ static int few_pick(const bamd_dense & w, const void * x, int ldx, int rows, flo
 }
 size_t bamd_dense_mv_lds(int act, int K) { return (size_t) (K + 31) / 32 * 32 * (act == BAMD_ACT_F32 ? 4 : 2); }
 template <typename T, int NT, int NW, int PRE>
-static void mv_go(const bamd_dense & w, const bamd_batch_dev & b, const bamd_pre_args & p, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s) {
+static void mv_go(const bamd_dense & w, const bamd_batch_dev & b, const bamd_pre_args & p, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s, int parts = 1) {
     const int grid = w.row_tiles < 4096 / NW ? w.row_tiles : 4096 / NW;       // what is resident at once; blocks walk the tiles
     const size_t lds = PRE == BAMD_PRE_ROWS ? 0 : bamd_dense_mv_lds(sizeof(T) == 4 ? BAMD_ACT_F32 : BAMD_ACT_BF16, w.k_tiles * 32);
-    hipLaunchKernelGGL((dense_mv_kernel<T, NT, NW, PRE>), dim3(grid), dim3(64 * NW), lds, s, w, b, p, (const T *) x, ldx, rows, out, ldo);
+    hipLaunchKernelGGL((dense_mv_kernel<T, NT, NW, PRE>), dim3(grid, parts), dim3(64 * NW), lds, s, w, b, p, (const T *) x, ldx, rows, out, ldo);
 }
 // sixteen waves where the tiles alone would leave the chip half empty
 template <typename T, int PRE>
-static void mv_one(const bamd_dense & w, const bamd_batch_dev & b, const bamd_pre_args & p, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s) {
-    if (w.row_tiles <= 256) mv_go<T, 1, 16, PRE>(w, b, p, x, ldx, rows, out, ldo, s);
+static void mv_one(const bamd_dense & w, const bamd_batch_dev & b, const bamd_pre_args & p, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s, int parts = 1) {
+    if (w.row_tiles <= 256) mv_go<T, 1, 16, PRE>(w, b, p, x, ldx, rows, out, ldo, s, parts);
     else mv_go<T, 1, 8, PRE>(w, b, p, x, ldx, rows, out, ldo, s);
 }
+// Two shares of K where a matrix has too few row tiles for the CUs and enough columns that halves are still worth a block; a prologue that writes state stays whole
+static int few_parts(const bamd_dense & w, int pre, const int * parts) {
+    return parts && *parts > 1 && w.row_tiles <= 128 && w.k_tiles >= 64 && pre != BAMD_PRE_RESIDUAL && pre != BAMD_PRE_FINAL && pre != BAMD_PRE_LAYER ? 2 : 1;
+}
 template <typename T>
-static int mv_pick(const bamd_dense & w, int pre, const bamd_batch_dev & b, const bamd_pre_args & p, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s) {
+static int mv_pick(const bamd_dense & w, int pre, const bamd_batch_dev & b, const bamd_pre_args & p, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s, int * parts) {
+    const int n = few_parts(w, pre, parts);
+    if (parts) *parts = n;
     if (pre != BAMD_PRE_ROWS) {
         if (rows != 1 || bamd_dense_mv_lds(sizeof(T) == 4 ? BAMD_ACT_F32 : BAMD_ACT_BF16, w.k_tiles * 32) > BAMD_MV_LDS) return 1;
         const int ldh = pre == BAMD_PRE_POLY ? p.poly.ldh : pre == BAMD_PRE_GROUP ? p.grp.ldh : pre == BAMD_PRE_GLU ? p.glu.ldh : p.res.ldh;
         if (ldh != w.k_tiles * 32) return 1;
         if (pre == BAMD_PRE_RESIDUAL && p.res.norm != BAMD_NORM_LAYER) mv_one<T, BAMD_PRE_RESIDUAL>(w, b, p, x, ldx, rows, out, ldo, s);
-        else if (pre == BAMD_PRE_POLY) mv_one<T, BAMD_PRE_POLY>(w, b, p, x, ldx, rows, out, ldo, s);
-        else if (pre == BAMD_PRE_GROUP) mv_one<T, BAMD_PRE_GROUP>(w, b, p, x, ldx, rows, out, ldo, s);
-        else if (pre == BAMD_PRE_GLU) mv_one<T, BAMD_PRE_GLU>(w, b, p, x, ldx, rows, out, ldo, s);
+        else if (pre == BAMD_PRE_POLY) mv_one<T, BAMD_PRE_POLY>(w, b, p, x, ldx, rows, out, ldo, s, n);
+        else if (pre == BAMD_PRE_GROUP) mv_one<T, BAMD_PRE_GROUP>(w, b, p, x, ldx, rows, out, ldo, s, n);
+        else if (pre == BAMD_PRE_GLU) mv_one<T, BAMD_PRE_GLU>(w, b, p, x, ldx, rows, out, ldo, s, n);
         else if (p.res.norm == BAMD_NORM_LAYER) mv_one<T, BAMD_PRE_LAYER>(w, b, p, x, ldx, rows, out, ldo, s);
         else mv_one<T, BAMD_PRE_FINAL>(w, b, p, x, ldx, rows, out, ldo, s);
         return 0;
     }
     if (rows < 1 || rows > BAMD_MV_ROWS || ldx < w.k_tiles * 32 || (ldx & 7)) return 1;
-    if constexpr (sizeof(T) == 2) return few_pick(w, x, ldx, rows, out, ldo, s);
-    else if (rows <= 16) mv_one<T, BAMD_PRE_ROWS>(w, b, p, x, ldx, rows, out, ldo, s);
-    else if (rows <= 32) mv_go<T, 2, 8, BAMD_PRE_ROWS>(w, b, p, x, ldx, rows, out, ldo, s);
-    else mv_go<T, 4, 8, BAMD_PRE_ROWS>(w, b, p, x, ldx, rows, out, ldo, s);
+    if constexpr (sizeof(T) == 2) return few_pick(w, x, ldx, rows, out, ldo, s, n);
+    else if (rows <= 16) mv_one<T, BAMD_PRE_ROWS>(w, b, p, x, ldx, rows, out, ldo, s, n);
+    else if (rows <= 32) mv_go<T, 2, 8, BAMD_PRE_ROWS>(w, b, p, x, ldx, rows, out, ldo, s, n);
+    else mv_go<T, 4, 8, BAMD_PRE_ROWS>(w, b, p, x, ldx, rows, out, ldo, s, n);
     return 0;
 }
-int bamd_launch_dense_mv(int act, const bamd_dense & w, int pre, const bamd_batch_dev & b, const bamd_pre_args * p, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s) {
+int bamd_launch_dense_mv(int act, const bamd_dense & w, int pre, const bamd_batch_dev & b, const bamd_pre_args * p, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s, int * parts) {
     static const bamd_pre_args none = {};
-    return act == BAMD_ACT_F32 ? mv_pick<float>(w, pre, b, p ? *p : none, x, ldx, rows, out, ldo, s) : mv_pick<bamd_bf>(w, pre, b, p ? *p : none, x, ldx, rows, out, ldo, s);
+    return act == BAMD_ACT_F32 ? mv_pick<float>(w, pre, b, p ? *p : none, x, ldx, rows, out, ldo, s, parts) : mv_pick<bamd_bf>(w, pre, b, p ? *p : none, x, ldx, rows, out, ldo, s, parts);
 }

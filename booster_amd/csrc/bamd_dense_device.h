@@ -95,6 +95,14 @@ template <int RC> struct RowRegs {
 #pragma unroll
         for (int c = 0; c < RC; ++c) v[c] = at(c) < n ? *(const bamd_v4 *) (p + at(c)) : bamd_v4{ 0, 0, 0, 0 };
     }
+    // the sum of one or two planes
+    __device__ __forceinline__ void load(const float * p, int n, int parts, size_t plane) {
+        load(p, n);
+        if (parts <= 1) return;
+        RowRegs b; b.load(p + plane, n);
+#pragma unroll
+        for (int i = 0; i < RC; ++i) v[i] = v[i] + b.v[i];
+    }
     __device__ __forceinline__ void clear() {
 #pragma unroll
         for (int c = 0; c < RC; ++c) v[c] = bamd_v4{ 0, 0, 0, 0 };
@@ -115,6 +123,8 @@ template <> __device__ __forceinline__ void store4<bamd_bf>(bamd_bf * h, bamd_v4
     *(bf4 *) h = bf4{ (bamd_bf) v[0], (bamd_bf) v[1], (bamd_bf) v[2], (bamd_bf) v[3] };
 }
 template <typename T> __device__ __forceinline__ void zero_tail(T * h, int n, int ld) { for (int i = n + threadIdx.x; i < ld; i += blockDim.x) h[i] = to_act<T>(0.f); }
+
+__device__ __forceinline__ float parts_sum(const float * p, int parts, size_t plane) { return parts > 1 ? p[0] + p[plane] : p[0]; }
 
 // mean and variance (mean of the squared deviations) of a row in registers: per wave around its own mean, then over the waves.  red: 48 floats of LDS
 template <int RC> __device__ __forceinline__ void row_moments(const RowRegs<RC> & r, int n, float * red, float & mean, float & var) {
@@ -149,7 +159,7 @@ __device__ __forceinline__ void layer_row(const bamd_residual_args & a, int row,
         RowRegs<RC> xr, yr;
         bamd_v4 g[RC], w[RC];
         xr.load(x, E);
-        if (y) yr.load(y, E);
+        if (y) yr.load(y, E, a.parts, a.plane);
 #pragma unroll
         for (int c = 0; c < RC; ++c) {
             const int i = RowRegs<RC>::at(c);
@@ -178,14 +188,14 @@ __device__ __forceinline__ void layer_row(const bamd_residual_args & a, int row,
     float my = 0.f, ry = 0.f, v[1];
     if (y) {
         v[0] = 0.f;
-        for (int i = threadIdx.x; i < E; i += blockDim.x) v[0] += y[i];
+        for (int i = threadIdx.x; i < E; i += blockDim.x) v[0] += parts_sum(y + i, a.parts, a.plane);
         block_sum<1>(v, red);
         my = v[0] / (float) E; v[0] = 0.f;
-        for (int i = threadIdx.x; i < E; i += blockDim.x) { const float d = y[i] - my; v[0] += d * d; }
+        for (int i = threadIdx.x; i < E; i += blockDim.x) { const float d = parts_sum(y + i, a.parts, a.plane) - my; v[0] += d * d; }
         block_sum<1>(v, red);
         ry = 1.0f / sqrtf(v[0] / (float) E + a.eps);
     }
-    auto at = [&](int i) { return y ? x[i] + (y[i] - my) * ry * a.g[i] : x[i]; };
+    auto at = [&](int i) { return y ? x[i] + (parts_sum(y + i, a.parts, a.plane) - my) * ry * a.g[i] : x[i]; };
     float mx = 0.f, rx = 1.f;
     if (gi && h) {
         v[0] = 0.f;
@@ -237,8 +247,8 @@ __device__ __forceinline__ void residual_row(const bamd_batch_dev & b, const bam
     if (RowRegs<RC>::fits(E)) {
         RowRegs<RC> xr, yr, pr, qr, mu;
         xr.load(x, E);
-        if (y) yr.load(y, E);
-        if (shifted) { mu.load(a.mu, E); if (before) { pr.load(xp, E); if (yp) qr.load(yp, E); } else if (sp) pr.load(sp, E); else pr.clear(); }
+        if (y) yr.load(y, E, a.parts, a.plane);
+        if (shifted) { mu.load(a.mu, E); if (before) { pr.load(xp, E); if (yp) qr.load(yp, E, a.parts, a.plane); } else if (sp) pr.load(sp, E); else pr.clear(); }
         float r = 0.f, rp = 0.f;
         if (y) {
             const float g = a.g[0];
@@ -262,16 +272,16 @@ __device__ __forceinline__ void residual_row(const bamd_batch_dev & b, const bam
     float r = 0.f, rp = 0.f;
     if (y) {
         float v[2] = { 0.f, 0.f };
-        for (int i = threadIdx.x; i < E; i += blockDim.x) { const float t = y[i]; v[0] += t * t; if (yp) { const float u = yp[i]; v[1] += u * u; } }
+        for (int i = threadIdx.x; i < E; i += blockDim.x) { const float t = parts_sum(y + i, a.parts, a.plane); v[0] += t * t; if (yp) { const float u = parts_sum(yp + i, a.parts, a.plane); v[1] += u * u; } }
         block_sum<2>(v, red);
         const float g = a.g[0];
         r = g / sqrtf(v[0] / (float) E + a.eps); rp = g / sqrtf(v[1] / (float) E + a.eps);
     }
     for (int i = threadIdx.x; i < E; i += blockDim.x) {
-        const float xn = y ? x[i] + y[i] * r : x[i];
+        const float xn = y ? x[i] + parts_sum(y + i, a.parts, a.plane) * r : x[i];
         float hn = xn;
         if (shifted) {
-            const float pv = before ? (yp ? xp[i] + yp[i] * rp : xp[i]) : (sp ? sp[i] : 0.f);
+            const float pv = before ? (yp ? xp[i] + parts_sum(yp + i, a.parts, a.plane) * rp : xp[i]) : (sp ? sp[i] : 0.f);
             hn = xn + (pv - xn) * a.mu[i];
         }
         if (write) { a.xo[(size_t) row * E + i] = xn; if (so) so[i] = xn; }
@@ -289,7 +299,7 @@ __device__ __forceinline__ void final_row(const bamd_residual_args & a, int row,
         RowRegs<RC> xr, yr;
         xr.load(x, E);
         if (y) {
-            yr.load(y, E);
+            yr.load(y, E, a.parts, a.plane);
             v[0] = yr.squares();
             block_sum<1>(v, red);
             const float r = a.g[0] / sqrtf(v[0] / (float) E + a.eps);
@@ -306,14 +316,14 @@ __device__ __forceinline__ void final_row(const bamd_residual_args & a, int row,
     }
     float r = 0.f;
     if (y) {
-        for (int i = threadIdx.x; i < E; i += blockDim.x) v[0] += y[i] * y[i];
+        for (int i = threadIdx.x; i < E; i += blockDim.x) { const float t = parts_sum(y + i, a.parts, a.plane); v[0] += t * t; }
         block_sum<1>(v, red);
         r = a.g[0] / sqrtf(v[0] / (float) E + a.eps);
     }
-    for (int i = threadIdx.x; i < E; i += blockDim.x) { const float xn = y ? x[i] + y[i] * r : x[i]; w[0] += xn * xn; }
+    for (int i = threadIdx.x; i < E; i += blockDim.x) { const float xn = y ? x[i] + parts_sum(y + i, a.parts, a.plane) * r : x[i]; w[0] += xn * xn; }
     block_sum<1>(w, red);
     const float rf = gf[0] / sqrtf(w[0] / (float) E + a.eps);
-    for (int i = threadIdx.x; i < E; i += blockDim.x) h[i] = to_act<T>((y ? x[i] + y[i] * r : x[i]) * rf);
+    for (int i = threadIdx.x; i < E; i += blockDim.x) h[i] = to_act<T>((y ? x[i] + parts_sum(y + i, a.parts, a.plane) * r : x[i]) * rf);
     zero_tail(h, E, a.ldh);
 }
 template <typename T>

@@ -204,7 +204,7 @@ struct Ctx {
 };
 struct Pass {                                      // one pass through the layers
     Ctx & c; Stack & st; hipStream_t s; bamd_batch_dev b; bool decode = false;
-    int n_tiles = 0, k_rows = 0, max_n = 1, n_segs = 0; float * x; float * xo; const float * pend = nullptr; int ldp = 0; const float * pend_g = nullptr;
+    int n_tiles = 0, k_rows = 0, max_n = 1, n_segs = 0; float * x; float * xo; const float * pend = nullptr; int ldp = 0; const float * pend_g = nullptr; int pend_parts = 1;
     Timer * tm = nullptr;
     void begin(int kind, double bytes) { if (!tm) return; hipEvent_t e; hipEventCreate(&e); hipEventRecord(e, s); tm->ev.push_back(e); tm->kind.push_back(kind); tm->bytes.push_back(bytes); }
     void end() { if (!tm) return; hipEvent_t e; hipEventCreate(&e); hipEventRecord(e, s); tm->ev.push_back(e); }
@@ -212,23 +212,24 @@ struct Pass {                                      // one pass through the layer
     bamd_residual_args residual(const float * mu, float * prev, const float * gi) {
         bamd_residual_args a; memset(&a, 0, sizeof a);
         a.norm = st.d.norm == STACK_NORM_SANDWICH ? BAMD_NORM_LAYER : BAMD_NORM_RMS; a.gi = gi;
-        a.x = x; a.y = pend; a.ldy = ldp; a.g = pend_g; a.eps = st.eps; a.mu = mu; a.prev = prev; a.xo = xo; a.h = c.h; a.E = st.E; a.ldh = up(st.E, 32);
+        a.x = x; a.y = pend; a.ldy = ldp; a.parts = pend_parts; a.plane = (size_t) b.rows * ldp; a.g = pend_g; a.eps = st.eps; a.mu = mu; a.prev = prev; a.xo = xo; a.h = c.h; a.E = st.E; a.ldh = up(st.E, 32);
         return a;
     }
-    void advanced(const float * y, int ld, const float * g) { std::swap(x, xo); pend = y; ldp = ld; pend_g = g; }
+    void advanced(const float * y, int ld, const float * g, int parts) { std::swap(x, xo); pend = y; ldp = ld; pend_g = g; pend_parts = parts; }
     // a product whose operand rows exist; small row counts stream the weights once
-    int product(const bamd_dense & w, const void * in, int ldx, float * out, int ldo, int kind) {
+    // parts: in, shares of K the result's buffer can hold; out, shares there are (the rows' residual sum adds them)
+    int product(const bamd_dense & w, const void * in, int ldx, float * out, int ldo, int kind, int * parts = nullptr) {
         begin(kind, (double) w.bytes);
-        const int rc = b.rows <= BAMD_MV_ROWS ? bamd_launch_dense_mv(st.act, w, BAMD_PRE_ROWS, b, nullptr, in, ldx, b.rows, out, ldo, s)
-                                              : bamd_launch_dense_gemm(st.act, w, in, ldx, b.rows, out, ldo, BAMD_OUT_F32, s);
+        const int rc = b.rows <= BAMD_MV_ROWS ? bamd_launch_dense_mv(st.act, w, BAMD_PRE_ROWS, b, nullptr, in, ldx, b.rows, out, ldo, s, parts)
+                                              : bamd_launch_dense_gemm(st.act, w, in, ldx, b.rows, out, ldo, BAMD_OUT_F32, s, 0.f, parts);
         end();
         return rc ? fail("dense product: unsupported shape") : 0;
     }
     bool fused(const bamd_dense & w) const { return b.rows == 1 && decode && bamd_dense_mv_lds(st.act, w.K) <= BAMD_MV_LDS; }
-    int product_pre(const bamd_dense & w, int pre, const bamd_pre_args & p, float * out, int ldo, int kind) {
+    int product_pre(const bamd_dense & w, int pre, const bamd_pre_args & p, float * out, int ldo, int kind, int * parts = nullptr) {
         if (fused(w)) {
             begin(kind, (double) w.bytes);
-            const int rc = bamd_launch_dense_mv(st.act, w, pre, b, &p, nullptr, 0, 1, out, ldo, s);
+            const int rc = bamd_launch_dense_mv(st.act, w, pre, b, &p, nullptr, 0, 1, out, ldo, s, parts);
             end();
             return rc ? fail("dense product: unsupported shape") : 0;
         }
@@ -239,7 +240,7 @@ struct Pass {                                      // one pass through the layer
         else if (pre == BAMD_PRE_POLY) { bamd_launch_poly_rows(st.act, b.rows, p.poly, s); ldx = p.poly.ldh; }
         else { bamd_launch_group_norm_rows(st.act, b.rows, p.grp, s); ldx = p.grp.ldh; }
         end();
-        return product(w, c.h, ldx, out, ldo, kind);
+        return product(w, c.h, ldx, out, ldo, kind, parts);
     }
     int layers();
     int head(const int32_t * want, int n, float * logits);
@@ -721,17 +722,20 @@ int Parallel::run(Pass & p, MixState & st, Operand & o) {
 }
 int Pass::layers() {
     bamd_pre_args pa; memset((void *) &pa, 0, sizeof pa);
+    const int room = std::min(2, c.rows_cap / b.rows);             // planes of these rows that fit the result's buffer
     for (size_t i = 0; i < st.layers.size(); ++i) {
+        int parts = room;
         Layer & ly = st.layers[i];
         Mixer & mx = *ly.mix;
         pa.res = residual(ly.shift, c.prev[i], ly.pre1);
         if (product_pre(mx.in, BAMD_PRE_RESIDUAL, pa, c.y, ld_of(mx.in), 0)) return 1;
         Operand o;
         if (mx.run(*this, c.mix[i], o)) return 1;
-        if (o.pre == BAMD_PRE_ROWS) { if (product(mx.out, o.x, o.ldx, c.y2, c.ldy2, 3)) return 1; }
-        else { pa.grp = o.grp; if (product_pre(mx.out, o.pre, pa, c.y2, c.ldy2, 3)) return 1; }
-        advanced(c.y2, c.ldy2, ly.norm1);
+        if (o.pre == BAMD_PRE_ROWS) { if (product(mx.out, o.x, o.ldx, c.y2, c.ldy2, 3, &parts)) return 1; }
+        else { pa.grp = o.grp; if (product_pre(mx.out, o.pre, pa, c.y2, c.ldy2, 3, &parts)) return 1; }
+        advanced(c.y2, c.ldy2, ly.norm1, parts);
         if (!ly.mlp) continue;
+        parts = room;
         pa.res = residual(nullptr, nullptr, ly.pre2);
         const bool glu = st.d.mlp_act == STACK_ACT_CLAMPED_GLU;
         if (glu && b.rows > BAMD_MV_ROWS) {                        // the product's tiles write the down-projection's operand
@@ -740,14 +744,14 @@ int Pass::layers() {
             const int rc = bamd_launch_dense_gemm(st.act, ly.up, c.h, pa.res.ldh, b.rows, c.y, ly.down.K, BAMD_OUT_GLU, s, ly.limit);
             end();
             if (rc) return fail("dense product: unsupported shape");
-            if (product(ly.down, c.y, ly.down.K, c.y2, c.ldy2, 5)) return 1;
+            if (product(ly.down, c.y, ly.down.K, c.y2, c.ldy2, 5, &parts)) return 1;
         } else {
             if (product_pre(ly.up, BAMD_PRE_RESIDUAL, pa, c.y, ld_of(ly.up), 4)) return 1;
             if (glu) pa.glu = { c.y, ld_of(ly.up), ly.limit, c.h, ly.down.K };
             else pa.poly = { c.y, ld_of(ly.up), ly.act, st.eps, c.h, ly.F, ly.down.K };
-            if (product_pre(ly.down, glu ? BAMD_PRE_GLU : BAMD_PRE_POLY, pa, c.y2, c.ldy2, 5)) return 1;
+            if (product_pre(ly.down, glu ? BAMD_PRE_GLU : BAMD_PRE_POLY, pa, c.y2, c.ldy2, 5, &parts)) return 1;
         }
-        advanced(c.y2, c.ldy2, ly.norm2);
+        advanced(c.y2, c.ldy2, ly.norm2, parts);
     }
     return 0;
 }
@@ -823,7 +827,7 @@ int send(Pass & p, const std::vector<Piece> & pc, const std::vector<int32_t> & w
     HIPC(hipEventRecord(c.ev[r], p.s));
     p.b = { (bamd_entry *) (c.dev + c.lay.ent), (int32_t *) (c.dev + c.lay.row), (int32_t *) (c.dev + c.lay.tok), (int) pc.size(), rows, c.c->n_seq, c.pages, c.max_pages };
     p.k_rows = kb * BAMD_PAGE; p.n_tiles = nt; p.n_segs = ns;
-    p.x = c.xa; p.xo = c.xb; p.pend = nullptr; p.ldp = 0; p.pend_g = nullptr;
+    p.x = c.xa; p.xo = c.xb; p.pend = nullptr; p.ldp = 0; p.pend_g = nullptr; p.pend_parts = 1;
     return 0;
 }
 int embed(Pass & p) { bamd_launch_embed_rows(p.b, p.st.embd, p.st.pos, p.st.scale, p.st.E, p.st.V, p.x, p.s); return 0; }
@@ -1102,13 +1106,22 @@ BAMD_OP bamd_op_dense(int act, const uint16_t * w, int nrows, int k, const float
     const SafeTensor t = bf16_tensor(w, { nrows, k });
     if (s.l.alloc(d, nrows, k) || s.l.pack(&t, Loader::steps(nrows, k), Loader::steps(k, 1), const_cast<uint16_t *>(d.w)) || s.act_rows(x, rows, k, d.K, &dx)) return 1;
     const int ldo = impl == 3 ? up(rows, 64) : ld_of(d);
-    if (s.alloc((void **) &dy, (size_t) (impl == 3 ? ld_of(d) : rows) * ldo * 4)) return 1;
+    int parts = impl == 4 || impl == 5 ? 2 : 1;
+    if (s.alloc((void **) &dy, (size_t) (impl == 3 ? ld_of(d) : rows) * ldo * 4 * parts)) return 1;
     bamd_batch_dev b; memset((void *) &b, 0, sizeof b);
     int rc;
-    if (impl == 1) rc = bamd_launch_dense_mv(act, d, BAMD_PRE_ROWS, b, nullptr, dx, d.K, rows, dy, ldo, s.l.s);
+    if (impl == 4) rc = bamd_launch_dense_gemm(act, d, dx, d.K, rows, dy, ldo, BAMD_OUT_F32, s.l.s, 0.f, &parts);
+    else if (impl == 5) rc = bamd_launch_dense_mv(act, d, BAMD_PRE_ROWS, b, nullptr, dx, d.K, rows, dy, ldo, s.l.s, &parts);
+    else if (impl == 1) rc = bamd_launch_dense_mv(act, d, BAMD_PRE_ROWS, b, nullptr, dx, d.K, rows, dy, ldo, s.l.s);
     else rc = bamd_launch_dense_gemm(act, d, dx, d.K, rows, dy, ldo, impl == 0 ? BAMD_OUT_F32 : impl == 2 ? BAMD_OUT_ACT : BAMD_OUT_ACT_T, s.l.s);
     if (rc) return fail("bamd_op_dense: unsupported shape");
     HIPC(hipGetLastError());
+    if (impl >= 4) {                                              // the shares, added as their reader adds them
+        std::vector<float> all((size_t) rows * nrows * parts);
+        for (int p = 0; p < parts; ++p) if (s.rows_back(dy + (size_t) p * rows * ldo, rows, nrows, ldo, all.data() + (size_t) p * rows * nrows, true)) return 1;
+        for (size_t i = 0, n = (size_t) rows * nrows; i < n; ++i) y[i] = parts == 2 ? all[i] + all[n + i] : all[i];
+        return 0;
+    }
     if (impl != 3) return s.rows_back(dy, rows, nrows, ldo, y, impl != 2 || act == BAMD_ACT_F32);
     std::vector<float> tr((size_t) nrows * rows);
     if (s.rows_back(dy, nrows, rows, ldo, tr.data(), act == BAMD_ACT_F32)) return 1;

@@ -228,7 +228,8 @@ int bamd_op_attention(const float * q, const float * k, const float * v, uint16_
                       const float * rope_row, int H, int Hkv, int hd, int n_ctx, int pos, int prefill_mode, float * out,
                       float * probs_h0);
 /* mechanisms of the configured layer stacks (csrc/bamd_dense.h); act: 0 bfloat16, 1 float; matrices bfloat16 [nrows][k] */
-/* y[rows][nrows] = x[rows][k] . w^T; impl 0: many-row kernel, 1: few-row kernel (rows <= 64), 2: many-row kernel with an activation-typed result, 3: the same, transposed */
+/* y[rows][nrows] = x[rows][k] . w^T; impl 0: many-row kernel, 1: few-row kernel (rows <= 64), 2: many-row kernel with an activation-typed result, 3: the same, transposed,
+ * 4 / 5: as 0 / 1 with K halved where that is faster, the halves added */
 int bamd_op_dense(int act, const uint16_t * w, int nrows, int k, const float * x, int rows, int impl, float * y);
 /* xo = x + rms_norm(y) * g (y NULL: x), h = xo + (xo of the row in front - xo) * mu (mu NULL: xo); prev [E]: the row in front of the first (used when pos0 > 0), replaced by the last */
 int bamd_op_residual_rows(int act, const float * x, const float * y, float g, float eps, const float * mu, float * prev, int pos0, int rows, int E, float * xo, float * h);

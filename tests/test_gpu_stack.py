@@ -11,6 +11,7 @@ import pytest
 
 from conftest import ROOT
 from oracle import stack_oracle as so
+import stack_cases
 from stack_cases import CONFIGS, ROWS, SEEDS, attend, config, latent, mafurax, mamba, parallel, tokens
 
 pytestmark = pytest.mark.gpu
@@ -77,6 +78,19 @@ def test_dense_few_rows(bamd, n, rows, k):
     want = x.astype(np.float64) @ so.bf16_to_f32(w).T.astype(np.float64)
     scale = np.sqrt(np.abs(x).astype(np.float64) ** 2 @ np.abs(so.bf16_to_f32(w)).T.astype(np.float64) ** 2) + 1e-30      # of a sum of k products with random signs
     assert (np.abs(bamd.op_dense(w, x, "bfloat16", 1) - want) <= 1e-5 * scale).all()                 # sqrt(k) <= 46 roundings of 2^-24 in a row, three times over
+
+
+# K in two shares (few row tiles, many columns: an odd number of column blocks among them), and sizes just below that
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n,k,rows", [(500, 2100, 131), (77, 2049, 300), (500, 1000, 70), (500, 2100, 1), (2048, 2080, 6), (2049, 2080, 6), (77, 2049, 20), (500, 2100, 45), (500, 2000, 6)])
+def test_dense_halves(bamd, dtype, n, k, rows):
+    r = np.random.default_rng(n + k + rows)
+    w = so.f32_to_bf16(r.standard_normal((n, k)).astype(np.float32))
+    x = so.round_bf16(r.standard_normal((rows, k)).astype(np.float32))
+    want = x.astype(np.float64) @ so.bf16_to_f32(w).T.astype(np.float64)
+    scale = np.sqrt(np.abs(x).astype(np.float64) ** 2 @ np.abs(so.bf16_to_f32(w)).T.astype(np.float64) ** 2)
+    for impl in (4,) if rows > 64 else (4, 5):
+        assert (np.abs(bamd.op_dense(w, x, dtype, impl) - want) <= 1e-5 * scale).all(), impl
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
@@ -256,6 +270,32 @@ def run(request, bamd, cases):
 
 def everywhere(toks):
     return list(range(len(toks)))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width", [75, 76])
+@pytest.mark.parametrize("design", ["Tupitar", "Mafurax"])
+def test_models_whose_products_are_halved(bamd, dtype, width, design, tmp_path):
+    """output and down projections of 5 row tiles and 66 column blocks: their halves meet in the residual sum behind them, of prompts, of a few sequences and of one, in rows that are kept in
+    registers and in rows that are not"""
+    if design == "Tupitar":
+        cfg = stack_cases.config(width, 131, [stack_cases.mamba(33, 64, 8, 1, 1, 2, ff=2100), stack_cases.latent(9, 24, 250, 36, 0.31, ff=2100)])
+    else:
+        cfg = stack_cases.mafurax(width, 131, [stack_cases.parallel(stack_cases.attend(17, 1, 24, 120, 0.4, 6.0, 50, 19, 3), 0.7, (3, 10, 14, 8.0), 1.3, ff=2100, limit=0.8)])
+    case = Case(str(tmp_path / "m"), cfg, 3, dict(rel=8, rank=5))
+    m = bamd.Model(case.folder, dtype=dtype)
+    c = bamd.Context(m, 512, 3)
+    t = [tokens(cfg, 76, 30 + i) for i in range(3)]
+    for n in (70, 9, 1):
+        near(c.decode_batch([(0, t[0][:n], everywhere(t[0][:n]))]), case.logits(t[0])[:n], dtype)
+        c.seq_free(0)
+    got = c.decode_batch([(i, t[i][:70 - i], [69 - i]) for i in range(3)])
+    near(got, np.stack([case.logits(t[i])[69 - i] for i in range(3)]), dtype)
+    for k in range(3):
+        got = c.decode_batch([(i, [t[i][70 - i + k]], [0]) for i in range(3)])
+        near(got, np.stack([case.logits(t[i])[70 - i + k] for i in range(3)]), dtype)
+    near(c.decode_batch([(1, [t[1][72]], [0])])[0], case.logits(t[1])[72], dtype)
+    c.close(); m.close()
 
 
 @pytest.mark.parametrize("n", [1, 2, 3, 5, 64, 65, 150])
