@@ -1,13 +1,11 @@
 // bamd_ssm.hip — the state-space recurrence (Mamba-2 form): S_t = exp(-exp(A_log) dt_t) S_(t-1) + dt_t B_t x_t^T, y_t = S_t^T C_t + D x_t, gated by silu(z_t).
 //
-// ssm_scan_kernel: one block per (PT value columns, head, sequence) walks the sequence's tokens of this step.  A lane keeps four columns of NPL state rows in
-// registers (lane = column quad + group of state rows, so that a row's B and C serve four columns from one LDS read); y is summed over a lane's rows at once and over
-// the row groups once per chunk of tokens.  The state is read and written once per step; everything is 32-bit.
-//   prompts: ssm_conv_kernel filters x, B and C and computes step sizes and decays for all tokens in front of it; the scan only streams them, a chunk ahead;
-//   decoding (one token): the block filters its own channels, one launch in all.
+//   prompts: ssm_conv_kernel filters x, B and C and computes step sizes and decays for all tokens, ssm_chunk_kernel takes them sixteen at a time on the f32 matrix cores;
+//   decoding (one token): ssm_step_kernel, a block per (PT value columns, head, sequence), filters its own channels, one launch in all.  A lane keeps four columns of NPL state
+//     rows in registers (lane = column quad + group of state rows, so that a row's B and C serve four columns from one LDS read); y is summed over a lane's rows, then over the groups.
+// The state is read and written once per step; everything is 32-bit.
 #include "bamd_dense_device.h"
-
-#define SSM_CT 16
+#include <type_traits>
 
 struct SsmIndex {                                                  // channels of one (column block, head): [x columns | B | C]
     int h, g, p0, pw, inner, ch, N, groups, P;
@@ -69,14 +67,13 @@ __global__ void __launch_bounds__(256) ssm_conv_kernel(bamd_batch_dev b, bamd_ss
     }
 }
 
-// PT columns per block (16, 32, 64); NPL state rows per lane; 4 * (256 / PT) row groups over the four waves
-template <int PT, int NPL, bool PROMPT>
-__global__ void __launch_bounds__(256) ssm_scan_kernel(bamd_batch_dev b, bamd_ssm_args a) {
-    constexpr int Q = PT / 4, NG = 64 / Q, GROUPS = 4 * NG, NP = GROUPS * NPL, CT = PROMPT ? SSM_CT : 1;     // NP >= N state rows
-    constexpr int PF = PROMPT ? (CT * (PT + 2 * NP) + 255) / 256 : 1, ZF = PROMPT ? (CT * PT + 255) / 256 : 1;
-    __shared__ __align__(16) float ops[CT * (PT + 2 * NP)], yp[CT][GROUPS][PT];
-    float (*xs)[PT] = (float (*)[PT]) ops, (*Bs)[NP] = (float (*)[NP]) (ops + CT * PT), (*Cs)[NP] = (float (*)[NP]) (ops + CT * (PT + NP));
-    __shared__ float dts[CT], dec[CT];
+// Decoding, one token.  PT columns per block (16, 32, 64); NPL state rows per lane; 4 * (256 / PT) row groups over the four waves
+template <int PT, int NPL>
+__global__ void __launch_bounds__(256) ssm_step_kernel(bamd_batch_dev b, bamd_ssm_args a) {
+    constexpr int Q = PT / 4, NG = 64 / Q, GROUPS = 4 * NG, NP = GROUPS * NPL;     // NP >= N state rows
+    __shared__ __align__(16) float ops[PT + 2 * NP], yp[GROUPS][PT];
+    float * xs = ops, * Bs = ops + PT, * Cs = ops + PT + NP;
+    __shared__ float sdt, sdec;
     const bamd_entry e = b.ent[blockIdx.z];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, quad = lane % Q, grp = wave * NG + lane / Q;
     SsmIndex ix;
@@ -91,111 +88,200 @@ __global__ void __launch_bounds__(256) ssm_scan_kernel(bamd_batch_dev b, bamd_ss
 #pragma unroll
         for (int k = 0; k < 4; ++k) { const int n = grp * NPL + j, p = quad * 4 + k; s[j][k] = (e.pos0 > 0 && n < N && p < ix.pw) ? st[(size_t) n * a.P + p] : 0.f; }
     const float D = a.D[ix.h];
-    for (int i = tid; i < CT * (PT + 2 * NP); i += 256) ops[i] = 0.f;
-    auto slot = [&](int t, int c) { return c < ix.pw ? t * PT + c : c < ix.pw + N ? CT * PT + t * NP + (c - ix.pw) : CT * (PT + NP) + t * NP + (c - ix.pw - N); };
-    float pf[PF], zf[ZF], zc[ZF], pdt = 0.f, pdec = 0.f;
-    int src[PF], dst[PF];                                          // of this thread's share of a chunk: place in `filtered` behind the chunk's first row, place in LDS
-    if constexpr (PROMPT) {
-#pragma unroll
-        for (int i = 0; i < PF; ++i) {
-            const int k = tid + 256 * i, t = k / CH, c = k % CH;
-            src[i] = t < CT ? t * ix.ch + ix.channel(c) : 0x7fffffff; dst[i] = t < CT ? slot(t, c) : 0;
-        }
+    for (int i = tid; i < PT + 2 * NP; i += 256) ops[i] = 0.f;
+    auto slot = [&](int c) { return c < ix.pw ? c : c < ix.pw + N ? PT + (c - ix.pw) : PT + NP + (c - ix.pw - N); };
+    __syncthreads();                                               // zeroes are in
+    const float * hist = e.pos0 > 0 ? a.hist + ((size_t) e.par * b.n_seq + e.seq) * T1 * ix.ch : nullptr;
+    float * ho = a.hist + ((size_t) (e.par ^ 1) * b.n_seq + e.seq) * T1 * ix.ch;
+    const int own = (ix.h % per == 0 && ix.p0 == 0) ? CH : ix.pw;     // B and C belong to the group: its first head's first block stores their inputs
+    for (int c = tid; c < CH; c += 256) {
+        const int q = ix.channel(c);
+        ops[slot(c)] = ssm_filter(a, in, hist, 0, q, ix.inner, ix.ch);
+        if (c < own) for (int r = 0; r < T1; ++r) ho[(size_t) r * ix.ch + q] = ssm_raw(a, in, hist, 1 - T1 + r, q, ix.inner, ix.ch);
     }
-    auto request = [&](int t0) {                                   // the chunk's filtered values, in registers until the chunk in front is done
-        const float * f = a.filtered + (size_t) (e.row0 + t0) * ix.ch;
-        const int lim = min(CT, e.n - t0) * ix.ch;
+    if (tid == 0) { const float dt = softplus_f(in[ix.inner + ix.ch + ix.h] + a.dt_bias[ix.h]); sdt = dt; sdec = expf(-expf(a.A_log[ix.h]) * dt); }
+    __syncthreads();
+    {
+        const float d = sdec, dt = sdt;
+        const bamd_v4 x4 = *(const bamd_v4 *) &xs[quad * 4];
+        float xv[4], y[4] = { 0.f, 0.f, 0.f, 0.f };
 #pragma unroll
-        for (int i = 0; i < PF; ++i) pf[i] = src[i] < lim ? f[src[i]] : 0.f;
+        for (int k = 0; k < 4; ++k) xv[k] = dt * x4[k];
 #pragma unroll
-        for (int i = 0; i < ZF; ++i) { const int k = tid + 256 * i, t = k / PT, c = k % PT; zf[i] = t < CT && t0 + t < e.n && c < ix.pw ? in[(size_t) (t0 + t) * a.ld + ix.h * a.P + ix.p0 + c] : 0.f; }
-        if (tid < CT && t0 + tid < e.n) { const float * p = a.steps + ((size_t) (e.row0 + t0 + tid) * a.heads + ix.h) * 2; pdt = p[0]; pdec = p[1]; }
-    };
-    if constexpr (PROMPT) request(0);
-    for (int t0 = 0; t0 < e.n; t0 += CT) {
-        const int nt = min(CT, e.n - t0);
-        __syncthreads();                                           // zeroes are in, or the chunk before is done with LDS
-        if constexpr (PROMPT) {
+        for (int j = 0; j < NPL; ++j) {
+            const float B = Bs[grp * NPL + j], C = Cs[grp * NPL + j];
 #pragma unroll
-            for (int i = 0; i < PF; ++i) if (src[i] < nt * ix.ch) ops[dst[i]] = pf[i];
-            if (tid < nt) { dts[tid] = pdt; dec[tid] = pdec; }
-#pragma unroll
-            for (int i = 0; i < ZF; ++i) zc[i] = zf[i];
-        } else {
-            const float * hist = e.pos0 > 0 ? a.hist + ((size_t) e.par * b.n_seq + e.seq) * T1 * ix.ch : nullptr;
-            float * ho = a.hist + ((size_t) (e.par ^ 1) * b.n_seq + e.seq) * T1 * ix.ch;
-            const int own = (ix.h % per == 0 && ix.p0 == 0) ? CH : ix.pw;     // B and C belong to the group: its first head's first block stores their inputs
-            for (int c = tid; c < CH; c += 256) {
-                const int q = ix.channel(c);
-                ops[slot(0, c)] = ssm_filter(a, in, hist, 0, q, ix.inner, ix.ch);
-                if (c < own) for (int r = 0; r < T1; ++r) ho[(size_t) r * ix.ch + q] = ssm_raw(a, in, hist, 1 - T1 + r, q, ix.inner, ix.ch);
-            }
-            if (tid == 0) { const float dt = softplus_f(in[ix.inner + ix.ch + ix.h] + a.dt_bias[ix.h]); dts[0] = dt; dec[0] = expf(-expf(a.A_log[ix.h]) * dt); }
+            for (int k = 0; k < 4; ++k) { s[j][k] = fmaf(d, s[j][k], B * xv[k]); y[k] = fmaf(C, s[j][k], y[k]); }
         }
-        __syncthreads();
-        if constexpr (PROMPT) if (t0 + CT < e.n) request(t0 + CT);
-        auto token = [&](int t) {
-            const float d = dec[t], dt = dts[t];
-            const bamd_v4 x4 = *(const bamd_v4 *) &xs[t][quad * 4];
-            float xv[4], y[4] = { 0.f, 0.f, 0.f, 0.f };
+        *(bamd_v4 *) &yp[grp][quad * 4] = bamd_v4{ y[0], y[1], y[2], y[3] };
+    }
+    __syncthreads();
+    if (tid < ix.pw) {
+        float y[4] = { 0.f, 0.f, 0.f, 0.f };
 #pragma unroll
-            for (int k = 0; k < 4; ++k) xv[k] = dt * x4[k];
-#pragma unroll
-            for (int j = 0; j < NPL; ++j) {
-                const float B = Bs[t][grp * NPL + j], C = Cs[t][grp * NPL + j];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) { s[j][k] = fmaf(d, s[j][k], B * xv[k]); y[k] = fmaf(C, s[j][k], y[k]); }
-            }
-            *(bamd_v4 *) &yp[t][grp][quad * 4] = bamd_v4{ y[0], y[1], y[2], y[3] };
-        };
-        if (nt == CT) {                                            // a whole chunk: unrolled, the next token's operands are read under this one's arithmetic
-#pragma unroll
-            for (int t = 0; t < CT; ++t) token(t);
-        } else for (int t = 0; t < nt; ++t) token(t);
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < ZF; ++i) {
-            const int k = tid + 256 * i, t = k / PT, c = k % PT;
-            if (t < nt && c < ix.pw) {
-                float y[4] = { 0.f, 0.f, 0.f, 0.f };
-#pragma unroll
-                for (int g = 0; g < GROUPS; ++g) y[g & 3] += yp[t][g][c];
-                const float z = PROMPT ? zc[i] : in[ix.h * a.P + ix.p0 + c];
-                a.out[(size_t) (e.row0 + t0 + t) * a.ldo + ix.h * a.P + ix.p0 + c] = ((y[0] + y[1]) + (y[2] + y[3]) + D * xs[t][c]) * silu_f(z);
-            }
-        }
+        for (int g = 0; g < GROUPS; ++g) y[g & 3] += yp[g][tid];
+        const float z = in[ix.h * a.P + ix.p0 + tid];
+        a.out[(size_t) e.row0 * a.ldo + ix.h * a.P + ix.p0 + tid] = ((y[0] + y[1]) + (y[2] + y[3]) + D * xs[tid]) * silu_f(z);
     }
 #pragma unroll
     for (int j = 0; j < NPL; ++j)
 #pragma unroll
         for (int k = 0; k < 4; ++k) { const int n = grp * NPL + j, p = quad * 4 + k; if (n < N && p < ix.pw) st[(size_t) n * a.P + p] = s[j][k]; }
 }
-template <int PT, bool PROMPT> static void scan_go(const bamd_batch_dev & b, const bamd_ssm_args & a, hipStream_t s) {
+
+// Prompts: the tokens of a sequence sixteen at a time on the f32 matrix cores.  With p_t the product of the decays up to t inside a chunk and f_s that of the decays behind s,
+//     y_t = p_t C_t^T S + sum over s <= t of (C_t . B_s) (product of the decays s + 1 .. t) dt_s x_s,     S <- p_15 S + sum over s of B_s (f_s dt_s x_s)^T;
+// every factor is a product of at most fifteen decays, nothing is divided or taken from a difference of sums.  A block is 32 value columns of a head: eight waves, two tiles of 16
+// columns x four quarters of the state rows (y is summed over the quarters); a wave keeps its NT 16 x 16 tiles of S as accumulators, which are at once the operand that C^T S needs
+// (the four rows a lane holds are the four steps of a 16x16x4 product), as B^T C comes out in the order that its product with x wants.  Chunk c + 2 is requested and chunk c + 1 put
+// into LDS while c is computed.  One token after the other on the vector ALUs was a chain of 283 ns per token: 2048 tokens of 128 heads x 64 x 128 took 525 us; now 271.  A chunk's
+// matrix instructions take 0.4 us of a SIMD's time; the rest is what stands between them, which is why two waves share a SIMD (four waves a block: 331 us).
+template <int NT>
+__global__ void __launch_bounds__(512) ssm_chunk_kernel(bamd_batch_dev b, bamd_ssm_args a) {
+    constexpr int NQ = 4, NP = 16 * NQ * NT, LB = NP + 4, LX = 36, LD = 20, PF = 16 * NP / 512, KS = 512 / NP;      // row lengths in LDS: four rows on, 16 banks on
+    __shared__ __align__(16) float Bs[2][16 * LB], Cs[2][16 * LB], xs[2][16 * LX], yp[2][NQ][16 * LX], dm[2][16 * LD];
+    __shared__ __align__(16) float pre[2][16], fd[2][16], dts[2][16];
+    const bamd_entry e = b.ent[blockIdx.z];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 15, q = lane >> 4, ct = wave & 1, part = wave >> 1;
+    const int h = blockIdx.y, p0 = blockIdx.x * 32, pw = min(32, a.P - p0), N = a.N, inner = a.heads * a.P, ch = inner + 2 * a.groups * N, g = h / (a.heads / a.groups);
+    const int n0 = part * NT * 16;                                 // first state row of this wave
+    float * st = a.state + (((size_t) e.seq * a.heads + h) * N) * a.P + p0;
+    bamd_v4 S[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { const int n = n0 + j * 16 + q * 4 + i, p = ct * 16 + col; S[j][i] = e.pos0 > 0 && n < N && p < pw ? st[(size_t) n * a.P + p] : 0.f; }
+    const float D = a.D[h];
+    // Chunks on their way, by the parity of the chunk.  Every load is unconditional (a row or column clamped into range, zeroed on its way to LDS): a branch around each costs more
+    // than the chunk's arithmetic.  Thread: state row kn of the tokens kt, kt + KS, .., column xc of token xt, step size and decay of token col
+    float bf[2][PF], cf[2][PF], xf[2], zf[2], fdt[2], fdec[2];
+    const int kn = tid % NP, kt = tid / NP, xc = tid & 31, xt = tid >> 5;
+    const uint32_t kb = (uint32_t) (inner + g * N + min(kn, N - 1)), kc = kb + (uint32_t) (a.groups * N), xo = (uint32_t) (h * a.P + p0 + min(xc, pw - 1));
+    auto request = [&](int t0, auto par) {
+        constexpr int R = decltype(par)::value;
+        const int nt = e.n - t0;
+        if (nt <= 0) return;
+        const float * f = a.filtered + (size_t) (e.row0 + t0) * ch, * z = a.in + (size_t) (e.row0 + t0) * a.ld;
+        if (nt >= 16) {
+            const uint32_t r = (uint32_t) (kt * ch);
+#pragma unroll
+            for (int i = 0; i < PF; ++i) { const float * fi = f + (size_t) (i * KS) * ch; bf[R][i] = fi[r + kb]; cf[R][i] = fi[r + kc]; }
+        } else {
+#pragma unroll
+            for (int i = 0; i < PF; ++i) { const uint32_t r = (uint32_t) (min(kt + i * KS, nt - 1) * ch); bf[R][i] = f[r + kb]; cf[R][i] = f[r + kc]; }
+        }
+        const int t = min(xt, nt - 1);
+        xf[R] = f[(uint32_t) (t * ch) + xo]; zf[R] = z[(uint32_t) (t * a.ld) + xo];
+        const float * p = a.steps + ((size_t) (e.row0 + t0 + min(col, nt - 1)) * a.heads + h) * 2;
+        fdt[R] = col < nt ? p[0] : 0.f; fdec[R] = col < nt ? p[1] : 1.f;
+    };
+    // data-parallel moves inside a row of sixteen lanes (row_shr, row_shl); a lane without a source gets 1
+    auto moved = [](float v, auto ctrl) { return __int_as_float(__builtin_amdgcn_update_dpp(0x3f800000, __float_as_int(v), decltype(ctrl)::value, 0xf, 0xf, false)); };
+    auto scan_up = [&](float v) {                                  // products of lanes 0 .. col
+        v *= moved(v, std::integral_constant<int, 0x111>()); v *= moved(v, std::integral_constant<int, 0x112>());
+        v *= moved(v, std::integral_constant<int, 0x114>()); return v * moved(v, std::integral_constant<int, 0x118>());
+    };
+    auto put = [&](int nt, auto par) {                             // nt: the chunk's tokens and those behind
+        constexpr int w = decltype(par)::value;
+        if (nt >= 16 && N == NP) {
+#pragma unroll
+            for (int i = 0; i < PF; ++i) { Bs[w][(kt + i * KS) * LB + kn] = bf[w][i]; Cs[w][(kt + i * KS) * LB + kn] = cf[w][i]; }
+        } else {
+#pragma unroll
+            for (int i = 0; i < PF; ++i) { const bool in = kn < N && kt + i * KS < nt; Bs[w][(kt + i * KS) * LB + kn] = in ? bf[w][i] : 0.f; Cs[w][(kt + i * KS) * LB + kn] = in ? cf[w][i] : 0.f; }
+        }
+        xf[w] = xc < pw && xt < nt ? xf[w] : 0.f;
+        xs[w][xt * LX + xc] = xf[w];
+        if (wave < 4) {                                            // row s = tid / 16: the products of the decays s + 1 .. t = col (zero above the diagonal)
+            const int s = tid >> 4;
+            const float v = scan_up(col > s ? fdec[w] : 1.f);
+            dm[w][col * LD + s] = col < s ? 0.f : v;
+        } else if (wave == 4) {                                    // up to each token, and behind it
+            const float p = scan_up(fdec[w]);
+            float f = fdec[w];
+            f *= moved(f, std::integral_constant<int, 0x101>()); f *= moved(f, std::integral_constant<int, 0x102>());
+            f *= moved(f, std::integral_constant<int, 0x104>()); f *= moved(f, std::integral_constant<int, 0x108>());
+            f = moved(f, std::integral_constant<int, 0x101>());
+            if (lane < 16) { dts[w][lane] = fdt[w]; pre[w][lane] = p; fd[w][lane] = f * fdt[w]; }
+        }
+    };
+    request(0, std::integral_constant<int, 0>()); request(16, std::integral_constant<int, 1>());
+    put(e.n, std::integral_constant<int, 0>());
+    __syncthreads();
+    auto chunk = [&](int t0, auto par) {
+        constexpr int w = decltype(par)::value;
+        const int nt = e.n - t0;
+        const float xk = xf[w], zk = zf[w];
+        request(t0 + 32, par);
+        bamd_v4 cr[NT], br[NT], gt = { 0, 0, 0, 0 }, g2 = { 0, 0, 0, 0 }, y = { 0, 0, 0, 0 }, y2 = { 0, 0, 0, 0 };
+        float ba[NT][4], xw[4], xd[4];
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            cr[j] = *(const bamd_v4 *) &Cs[w][col * LB + n0 + j * 16 + q * 4]; br[j] = *(const bamd_v4 *) &Bs[w][col * LB + n0 + j * 16 + q * 4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) ba[j][i] = Bs[w][(q * 4 + i) * LB + n0 + j * 16 + col];
+        }
+        const bamd_v4 pr = *(const bamd_v4 *) &pre[w][q * 4], dv = *(const bamd_v4 *) &dm[w][col * LD + q * 4], d4 = *(const bamd_v4 *) &dts[w][q * 4], f4 = *(const bamd_v4 *) &fd[w][q * 4];
+        const float all = pre[w][15];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { const float x = xs[w][(q * 4 + i) * LX + ct * 16 + col]; xd[i] = x * d4[i]; xw[i] = x * f4[i]; }
+        if (nt > 16) put(nt - 16, std::integral_constant<int, w ^ 1>());       // (requested a chunk ago; its place was read before the last barrier)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (i & 1) { g2 = __builtin_amdgcn_mfma_f32_16x16x4f32(br[j][i], cr[j][i], g2, 0, 0, 0); y2 = __builtin_amdgcn_mfma_f32_16x16x4f32(cr[j][i], S[j][i], y2, 0, 0, 0); }
+                else { gt = __builtin_amdgcn_mfma_f32_16x16x4f32(br[j][i], cr[j][i], gt, 0, 0, 0); y = __builtin_amdgcn_mfma_f32_16x16x4f32(cr[j][i], S[j][i], y, 0, 0, 0); }
+            }
+#pragma unroll
+        for (int j = 0; j < NT; ++j) S[j] = S[j] * all;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) S[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ba[j][i], xw[i], S[j], 0, 0, 0);
+        y = (y + y2) * pr;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) y = __builtin_amdgcn_mfma_f32_16x16x4f32((gt[i] + g2[i]) * dv[i], xd[i], y, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) yp[w][part][(q * 4 + i) * LX + ct * 16 + col] = y[i];
+        __syncthreads();
+        const int o = xt * LX + xc;
+        if (xt < nt && xc < pw) a.out[(size_t) (e.row0 + t0 + xt) * a.ldo + h * a.P + p0 + xc] = ((yp[w][0][o] + yp[w][1][o]) + (yp[w][2][o] + yp[w][3][o]) + D * xk) * silu_f(zk);
+    };
+    for (int t0 = 0; t0 < e.n; t0 += 32) { chunk(t0, std::integral_constant<int, 0>()); if (t0 + 16 < e.n) chunk(t0 + 16, std::integral_constant<int, 1>()); }
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { const int n = n0 + j * 16 + q * 4 + i, p = ct * 16 + col; if (n < N && p < pw) st[(size_t) n * a.P + p] = S[j][i]; }
+}
+template <int PT> static void step_go(const bamd_batch_dev & b, const bamd_ssm_args & a, hipStream_t s) {
     constexpr int GROUPS = 4 * 64 / (PT / 4);                      // 16 (64 columns), 32, 64
     const dim3 grid((a.P + PT - 1) / PT, a.heads, b.n_entries);
     const int npl = (a.N + GROUPS - 1) / GROUPS;
-    if (npl <= 1) hipLaunchKernelGGL((ssm_scan_kernel<PT, 1, PROMPT>), grid, dim3(256), 0, s, b, a);
-    else if (npl <= 2) hipLaunchKernelGGL((ssm_scan_kernel<PT, 2, PROMPT>), grid, dim3(256), 0, s, b, a);
-    else if (npl <= 4) hipLaunchKernelGGL((ssm_scan_kernel<PT, 4, PROMPT>), grid, dim3(256), 0, s, b, a);
+    if (npl <= 1) hipLaunchKernelGGL((ssm_step_kernel<PT, 1>), grid, dim3(256), 0, s, b, a);
+    else if (npl <= 2) hipLaunchKernelGGL((ssm_step_kernel<PT, 2>), grid, dim3(256), 0, s, b, a);
+    else if (npl <= 4) hipLaunchKernelGGL((ssm_step_kernel<PT, 4>), grid, dim3(256), 0, s, b, a);
     else if constexpr (PT >= 32) {
-        if (npl <= 8) hipLaunchKernelGGL((ssm_scan_kernel<PT, 8, PROMPT>), grid, dim3(256), 0, s, b, a);
-        else if constexpr (PT >= 64) hipLaunchKernelGGL((ssm_scan_kernel<PT, 16, PROMPT>), grid, dim3(256), 0, s, b, a);
+        if (npl <= 8) hipLaunchKernelGGL((ssm_step_kernel<PT, 8>), grid, dim3(256), 0, s, b, a);
+        else if constexpr (PT >= 64) hipLaunchKernelGGL((ssm_step_kernel<PT, 16>), grid, dim3(256), 0, s, b, a);
     }
 }
 // max_n: most tokens any entry brings.  a.filtered [rows][channels] and a.steps [rows][heads][2] are scratch of prompts
 int bamd_launch_ssm(const bamd_batch_dev & b, const bamd_ssm_args & a, int max_n, hipStream_t s) {
     if (a.N < 1 || a.N > 256 || a.taps < 1 || a.groups < 1 || a.heads % a.groups || max_n < 1) return 1;
     const int ch = a.heads * a.P + 2 * a.groups * a.N;
-    // enough blocks for the chip; narrower blocks only as far as they are filled
-    const long wide = (long) ((a.P + 63) / 64) * a.heads * b.n_entries;
-    const int pt = a.P <= 16 || (max_n == 1 && wide * 2 < 256) ? 16 : a.P <= 32 || wide < 256 ? 32 : 64;
     if (max_n == 1) {
-        if (pt == 16) scan_go<16, false>(b, a, s); else if (pt == 32) scan_go<32, false>(b, a, s); else scan_go<64, false>(b, a, s);
+        // enough blocks for the chip; narrower blocks only as far as they are filled
+        const long wide = (long) ((a.P + 63) / 64) * a.heads * b.n_entries;
+        const int pt = a.P <= 16 || wide * 2 < 256 ? 16 : a.P <= 32 || wide < 256 ? 32 : 64;
+        if (pt == 16) step_go<16>(b, a, s); else if (pt == 32) step_go<32>(b, a, s); else step_go<64>(b, a, s);
         return 0;
     }
     if (!a.filtered || !a.steps) return 1;
-    const dim3 cg((ch + 255) / 256, (b.rows + SSM_STRIP - 1) / SSM_STRIP);
+    const dim3 cg((ch + 255) / 256, (b.rows + SSM_STRIP - 1) / SSM_STRIP), grid((a.P + 31) / 32, a.heads, b.n_entries);
     if (a.taps == 4) hipLaunchKernelGGL(ssm_conv_kernel<true>, cg, dim3(256), 0, s, b, a); else hipLaunchKernelGGL(ssm_conv_kernel<false>, cg, dim3(256), 0, s, b, a);
-    if (pt == 16) scan_go<16, true>(b, a, s); else if (pt == 32) scan_go<32, true>(b, a, s); else scan_go<64, true>(b, a, s);
+    if (a.N <= 64) hipLaunchKernelGGL(ssm_chunk_kernel<1>, grid, dim3(512), 0, s, b, a);
+    else if (a.N <= 128) hipLaunchKernelGGL(ssm_chunk_kernel<2>, grid, dim3(512), 0, s, b, a);
+    else hipLaunchKernelGGL(ssm_chunk_kernel<4>, grid, dim3(512), 0, s, b, a);
     return 0;
 }

@@ -164,6 +164,26 @@ def test_ssm(bamd, H, P, N, G, taps):
         pos += n
 
 
+@pytest.mark.parametrize("H,P,N,G", [(2, 32, 64, 1), (1, 33, 65, 1), (3, 64, 128, 3), (1, 31, 129, 1), (2, 100, 200, 2), (1, 16, 256, 1)])
+def test_ssm_chunks(bamd, H, P, N, G):
+    """prompts through every number of state tiles, around the width of a block and the sixteen tokens of a chunk, with decays down to zero and up to one; portions continue one another"""
+    r = np.random.default_rng(H * P + N)
+    inner, ch = H * P, H * P + 2 * G * N
+    f = lambda a: np.asarray(a, np.float32)
+    conv, cb, dtb, A, D = map(f, (r.standard_normal((ch, 4)), r.standard_normal(ch) * 0.3, r.uniform(-6, 1, H), r.uniform(-4, 3, H), r.standard_normal(H)))
+    rows = f(r.standard_normal((200, inner + ch + H)))
+    rows[::9, -H:] -= 30
+    rows[5::11, -H:] += 90                                # exp(-exp(A) dt) is zero
+    hist, S = np.zeros((3, ch)), np.zeros((H, N, P))
+    gh, gs, pos = f(hist), f(S) + 7, 0
+    for n in (31, 32, 33, 2, 48, 54):
+        part = rows[pos:pos + n]
+        want, hist, S = plain_ssm(part.astype(np.float64), H, P, N, G, conv, cb, dtb, A, D, hist, S)
+        got, gh, gs = bamd.op_ssm(part, pos, H, P, N, G, conv, cb, dtb, A, D, gh, gs)
+        assert rel(got, want) < 2e-5 and rel(gs, S) < 2e-5, pos      # as test_ssm
+        pos += n
+
+
 def plain_attention(q, c, gate, past, uk, uv, c_norm, sink, scale, eps, H):
     T, _, d = q.shape
     lat = np.stack([so.rms(v, eps) * c_norm for v in c])
