@@ -1,7 +1,5 @@
 // bamd_dense.hip — products with dense bfloat16 matrices in the packed layout of bamd_dense.h.
-//   dense_tile_kernel: many rows (prompts), bfloat16.  Weight and activation tiles global -> LDS by DMA, four or eight stages deep, under the matrix instructions.
-//   dense_gemm_kernel: many rows, 32-bit.  Tiles through two LDS stages in operand order (every LDS access is one contiguous kilobyte per wave), the next stage's global
-//     loads in flight under the matrix instructions.
+//   dense_tile_kernel: many rows (prompts).  Weight and activation tiles global -> LDS by DMA, four or eight stages deep, under the matrix instructions.
 //   dense_few_kernel: up to 64 rows (decoding several sequences, short prompts), bfloat16.  The waves of a block split K, each with a DMA ring of weights and rows.
 //   dense_mv_kernel: a row (decoding), and up to 64 in 32-bit.  The eight or sixteen waves of a block split K; every wave streams its share of a 16-row tile straight from HBM into matrix operands.  With
 //     a single row the mechanism in front of the product (residual + norm + token shift or layer norms, PolyNorm, clamped gated unit, grouped norm, last norm) runs as its prologue, its weights
@@ -54,86 +52,6 @@ __device__ __forceinline__ void store_tile(const bamd_v4 (&a)[NI], int j, int mb
         }
     }
 }
-// TM activation rows x TN matrix rows per block of four waves (2 x 2); KT 32-column blocks per stage
-template <typename T, int TM, int TN, int KT, int OUT>
-__global__ void __launch_bounds__(256) dense_gemm_kernel(bamd_dense w, const T * x, int ldx, int rows, void * out, int ldo, int n_mt, int n_nt, float limit) {
-    constexpr int FB = 64 * 8 * sizeof(T);                        // bytes of one operand block (16 rows x 32 columns)
-    constexpr int XT = TM / 16, WT = TN / 16, XC = XT * KT * FB / 4096, WC = WT * KT * 1024 / 4096;   // 16-byte pieces per thread and stage
-    constexpr int WF = 1024;                                      // weights stay bfloat16 in LDS
-    constexpr int STAGE = XT * KT * FB + WT * KT * WF;
-    extern __shared__ __align__(16) unsigned char lds[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    // blocks of one XCD (every eighth) take neighbouring tiles: the row tiles of one column strip follow one another, so the strip's weights stay in that XCD's L2
-    const int total = n_mt * n_nt;
-    int id = blockIdx.x;
-    { const int per = (total + 7) / 8, xcd = id & 7, k = id >> 3; id = xcd * per + k; if (k >= per || id >= total) return; }
-    const int mt = id % n_mt, nt = id / n_mt, m0 = mt * TM, n0t = nt * WT;
-    bamd_u4 xr[XC], wr[WC];
-    auto fetch = [&](int ks) {
-#pragma unroll
-        for (int i = 0; i < XC; ++i) {
-            const int c = tid + 256 * i, per = FB / 16, blk = c / per, in = c % per;        // piece `in` of operand block blk
-            const int l = in & 63, half = in >> 6, tile = blk / KT, kt = ks * KT + blk % KT;
-            int row = m0 + tile * 16 + (l & 15); row = row < rows ? row : rows - 1;
-            const int k = kt * 32 + (l >> 4) * 8 + half * 4;
-            xr[i] = kt < w.k_tiles ? *(const bamd_u4 *) (x + (size_t) row * ldx + k) : bamd_u4{ 0, 0, 0, 0 };
-        }
-#pragma unroll
-        for (int i = 0; i < WC; ++i) {
-            const int c = tid + 256 * i, blk = c >> 6, l = c & 63, kt = ks * KT + blk % KT;
-            int tile = n0t + blk / KT; tile = tile < w.row_tiles ? tile : w.row_tiles - 1;
-            wr[i] = kt < w.k_tiles ? *(const bamd_u4 *) (w.w + (((size_t) tile * w.k_tiles + kt) * 64 + l) * 8) : bamd_u4{ 0, 0, 0, 0 };
-        }
-    };
-    auto put = [&](int st) {
-        unsigned char * base = lds + st * STAGE;
-#pragma unroll
-        for (int i = 0; i < XC; ++i) *(bamd_u4 *) (base + (tid + 256 * i) * 16) = xr[i];
-#pragma unroll
-        for (int i = 0; i < WC; ++i) *(bamd_u4 *) (base + XT * KT * FB + (tid + 256 * i) * 16) = wr[i];
-    };
-    constexpr int MI = XT / 2, NI = WT / 2;
-    const int wm = wave & 1, wn = wave >> 1;
-    bamd_v4 acc[MI][NI];
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < NI; ++j) acc[i][j] = bamd_v4{ 0, 0, 0, 0 };
-    const int nks = (w.k_tiles + KT - 1) / KT;
-    fetch(0); put(0);
-    __syncthreads();
-    for (int ks = 0; ks < nks; ++ks) {
-        if (ks + 1 < nks) fetch(ks + 1);
-        const unsigned char * base = lds + (ks & 1) * STAGE;
-#pragma unroll
-        for (int h = 0; h < KT; ++h) {
-            Frag<T> xf[MI], wf[NI];
-#pragma unroll
-            for (int i = 0; i < MI; ++i) {
-                const unsigned char * p = base + ((wm * MI + i) * KT + h) * FB;
-                if constexpr (sizeof(T) == 2) xf[i].load((const T *) (p + lane * 16));
-                else { xf[i].a = *(const bamd_v4 *) (p + lane * 16); xf[i].b = *(const bamd_v4 *) (p + 1024 + lane * 16); }
-            }
-#pragma unroll
-            for (int j = 0; j < NI; ++j) wf[j].weight(*(const bamd_u4 *) (base + XT * KT * FB + ((wn * NI + j) * KT + h) * WF + lane * 16));
-#pragma unroll
-            for (int i = 0; i < MI; ++i)
-#pragma unroll
-                for (int j = 0; j < NI; ++j) {
-                    if constexpr (OUT == BAMD_OUT_ACT_T) acc[i][j] = mma(xf[i], wf[j], acc[i][j]);     // lane: four activation rows of one matrix row
-                    else acc[i][j] = mma(wf[j], xf[i], acc[i][j]);                                      // lane: four matrix rows of one activation row
-                }
-        }
-        if (ks + 1 < nks) put((ks + 1) & 1);
-        __syncthreads();
-    }
-    const int n_lim = w.row_tiles * 16;
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < NI; ++j) store_tile<T, OUT>(acc[i], j, m0 + (wm * MI + i) * 16, (n0t + wn * NI + j) * 16, n_lim, w.rows, rows, out, ldo, limit, lane);
-}
-// ---- many rows, bfloat16 -------------------------------------------------------------------------------------------------------------------------------
 // TM activation rows x TN matrix rows per block of WM x WN waves.  Both operands travel global -> LDS by DMA (a kilobyte per instruction: 16 rows x 32 columns), NS stages
 // of 32 columns deep: while the matrix instructions of column block k run from registers, the fragments of k + 1 are read from LDS and the copies of the NS - 2 blocks
 // behind it are under way; one barrier per column block, which waits for copies issued NS - 2 blocks ago.  What bounded the kernel before it (128 x 128, staged through registers) was LDS
@@ -142,11 +60,11 @@ __global__ void __launch_bounds__(256) dense_gemm_kernel(bamd_dense w, const T *
 // Activations lie in LDS as they come from memory, four lanes on 64 consecutive bytes of a row (one 16-byte piece of 16 rows per four lanes costs the vector memory path
 // four times the lookups: 446 -> 409 us below), the pieces of a row turned by half its number: sixteen rows of one piece then fall on different banks.
 // 2048 x 28672 x 4096: 676 -> 409 us (1176 TFLOP/s); 2048 x 4096 x 14336: 284 -> 185 us (1303); 2048 x 2048 x 2048: 41 -> 22 us; 131 x 8192 x 2048: 23 -> 16 us.
-template <int TM, int TN, int WM, int WN, int NS, int OUT>
-__global__ void __launch_bounds__(64 * WM * WN) dense_tile_kernel(bamd_dense w, const bamd_bf * x, int ldx, int rows, void * out, int ldo, int n_mt, int n_nt, float limit) {
+template <typename T, int TM, int TN, int WM, int WN, int NS, int OUT>
+__global__ void __launch_bounds__(64 * WM * WN) dense_tile_kernel(bamd_dense w, const T * x, int ldx, int rows, void * out, int ldo, int n_mt, int n_nt, float limit) {
     const int kb = (int) ((long) w.k_tiles * blockIdx.y / gridDim.y), nk = (int) ((long) w.k_tiles * (blockIdx.y + 1) / gridDim.y) - kb;      // this block's share of K
-    constexpr int XT = TM / 16, WT = TN / 16, NW = WM * WN, MI = XT / WM, NI = WT / WN, PX = XT / NW, PW = WT / NW, PER = PX + PW, STAGE = (XT + WT) * 1024;
-    static_assert(XT % NW == 0 && WT % NW == 0 && MI * WM == XT && NI * WN == WT && NS >= 4 && (NS & (NS - 1)) == 0, "");
+    constexpr int XT = TM / 16, WT = TN / 16, NW = WM * WN, MI = XT / WM, NI = WT / WN, XK = sizeof(T) / 2, PX = XT * XK / NW, PW = WT / NW, PER = PX + PW, STAGE = (XT * XK + WT) * 1024;       // XK: KiB of an activation block
+    static_assert(XT * XK % NW == 0 && WT % NW == 0 && MI * WM == XT && NI * WN == WT && NS >= 4 && (NS & (NS - 1)) == 0, "");
     extern __shared__ __align__(16) unsigned char lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int total = n_mt * n_nt;
@@ -157,27 +75,38 @@ __global__ void __launch_bounds__(64 * WM * WN) dense_tile_kernel(bamd_dense w, 
     const unsigned char * xbase = (const unsigned char *) (x + (size_t) m0 * ldx + (size_t) kb * 32), * wbase = (const unsigned char *) (w.w + ((size_t) n0t * w.k_tiles + kb) * 512);
     uint32_t xo[PX], wo[PW];
 #pragma unroll
-    for (int i = 0; i < PX; ++i) { int row = (wave * PX + i) * 16 + (lane >> 2); row = m0 + row < rows ? row : rows - 1 - m0; xo[i] = (uint32_t) row * (uint32_t) ldx * 2u + (uint32_t) ((lane & 3) ^ ((lane >> 3) & 3)) * 16u; }
+    for (int i = 0; i < PX; ++i) {                                // bfloat16: 16 rows of four 16-byte pieces; 32-bit: 8 rows of eight
+        int row = XK == 1 ? (wave * PX + i) * 16 + (lane >> 2) : (wave * PX + i) * 8 + (lane >> 3);
+        row = m0 + row < rows ? row : rows - 1 - m0;
+        xo[i] = (uint32_t) row * (uint32_t) ldx * (uint32_t) sizeof(T) + (uint32_t) (XK == 1 ? (lane & 3) ^ ((lane >> 3) & 3) : (lane & 7) ^ (lane >> 3)) * 16u;
+    }
 #pragma unroll
     for (int i = 0; i < PW; ++i) { int tile = wave * PW + i; tile = n0t + tile < w.row_tiles ? tile : w.row_tiles - 1 - n0t; wo[i] = (uint32_t) tile * (uint32_t) w.k_tiles * 1024u + (uint32_t) lane * 16u; }
-    const uint32_t xd = (uint32_t) (size_t) (bamd_lds_vp) lds + (uint32_t) wave * PX * 1024u, wd = (uint32_t) (size_t) (bamd_lds_vp) lds + (uint32_t) (XT + wave * PW) * 1024u;
+    const uint32_t xd = (uint32_t) (size_t) (bamd_lds_vp) lds + (uint32_t) wave * PX * 1024u, wd = (uint32_t) (size_t) (bamd_lds_vp) lds + (uint32_t) (XT * XK + wave * PW) * 1024u;
     // copy i of PER of stage k (behind the last column block: the last one again, into a stage nobody reads)
     auto copy = [&](int k, int i) {
         const int kk = k < nk ? k : nk - 1;
         const uint32_t st = (uint32_t) (k & (NS - 1)) * STAGE;
-        if (i < PX) lds_dma16_s(xbase + (size_t) kk * 64, xo[i], xd + st + i * 1024u);
+        if (i < PX) lds_dma16_s(xbase + (size_t) kk * (32 * sizeof(T)), xo[i], xd + st + i * 1024u);
         else lds_dma16_s(wbase + (size_t) kk * 1024, wo[i - PX], wd + st + (i - PX) * 1024u);
     };
     const int wm = wave % WM, wn = wave / WM;
-    const unsigned char * xb = lds + (size_t) wm * MI * 1024 + ((lane & 15) * 4 + ((lane >> 4) ^ ((lane >> 1) & 3))) * 16, * wb = lds + (size_t) (XT + wn * NI) * 1024 + lane * 16;
+    const int r = lane & 15, q = lane >> 4;                       // the lane's row of a block and its eight columns
+    const unsigned char * xb = lds + (size_t) wm * MI * XK * 1024 + (XK == 1 ? (r * 4 + (q ^ ((r >> 1) & 3))) * 16 : (r * 8 + ((2 * q) ^ (r & 7))) * 16), * wb = lds + (size_t) (XT * XK + wn * NI) * 1024 + lane * 16;
+    const int xb2 = XK == 1 ? 0 : (((2 * q + 1) ^ (r & 7)) - ((2 * q) ^ (r & 7))) * 16;      // 32-bit: from the first four columns to the other four
     bamd_v4 acc[MI][NI];
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < NI; ++j) acc[i][j] = bamd_v4{ 0, 0, 0, 0 };
-    bamd_bf8 xf[2][MI], wf[2][NI];
-    auto read_x = [&](int k, int p, int i) { xf[p][i] = *(const bamd_bf8 *) (xb + (k & (NS - 1)) * STAGE + i * 1024); };
-    auto read_w = [&](int k, int p, int j) { wf[p][j] = *(const bamd_bf8 *) (wb + (k & (NS - 1)) * STAGE + j * 1024); };
+    Frag<T> xf[2][MI];
+    bamd_u4 wr[2][NI];                                            // as packed; 32-bit operands are widened where they are used
+    auto read_x = [&](int k, int p, int i) {
+        const unsigned char * at = xb + (k & (NS - 1)) * STAGE + i * (XK * 1024);
+        if constexpr (XK == 1) xf[p][i].load((const T *) at);
+        else { xf[p][i].a = *(const bamd_v4 *) at; xf[p][i].b = *(const bamd_v4 *) (at + xb2); }
+    };
+    auto read_w = [&](int k, int p, int j) { wr[p][j] = *(const bamd_u4 *) (wb + (k & (NS - 1)) * STAGE + j * 1024); };
     auto wait = [&] {                                             // all but the last stage's copies of this wave have landed; then every wave's
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"((NS - 3) * PER) : "memory");
         __builtin_amdgcn_s_barrier();
@@ -186,6 +115,9 @@ __global__ void __launch_bounds__(64 * WM * WN) dense_tile_kernel(bamd_dense w, 
     auto block = [&](int k, auto par) {
         constexpr int P = decltype(par)::value;
         wait();                                                   // stage k + 1 is whole; stage k - 1 is free
+        Frag<T> wf[NI];
+#pragma unroll
+        for (int j = 0; j < NI; ++j) wf[j].weight(wr[P][j]);
         // MI groups: a row of matrix instructions, and spread over them the copies of stage k + NS - 1 and the reads of stage k + 1
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
@@ -196,8 +128,8 @@ __global__ void __launch_bounds__(64 * WM * WN) dense_tile_kernel(bamd_dense w, 
             read_x(k + 1, P ^ 1, i);
 #pragma unroll
             for (int j = 0; j < NI; ++j) {
-                if constexpr (OUT == BAMD_OUT_ACT_T) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf[P][i], wf[P][j], acc[i][j], 0, 0, 0);
-                else acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[P][j], xf[P][i], acc[i][j], 0, 0, 0);
+                if constexpr (OUT == BAMD_OUT_ACT_T) acc[i][j] = mma(xf[P][i], wf[j], acc[i][j]);      // lane: four activation rows of one matrix row
+                else acc[i][j] = mma(wf[j], xf[P][i], acc[i][j]);                                       // lane: four matrix rows of one activation row
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -222,12 +154,12 @@ __global__ void __launch_bounds__(64 * WM * WN) dense_tile_kernel(bamd_dense w, 
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < NI; ++j) store_tile<bamd_bf, OUT>(acc[i], j, m0 + (wm * MI + i) * 16, (n0t + wn * NI + j) * 16, n_lim, w.rows, rows, out, ldo, limit, lane);
+        for (int j = 0; j < NI; ++j) store_tile<T, OUT>(acc[i], j, m0 + (wm * MI + i) * 16, (n0t + wn * NI + j) * 16, n_lim, w.rows, rows, out, ldo, limit, lane);
 }
-template <int TM, int TN, int WM, int WN, int NS, int OUT>
+template <typename T, int TM, int TN, int WM, int WN, int NS, int OUT>
 static int tile_go(const bamd_dense & w, const void * x, int ldx, int rows, void * out, int ldo, float limit, int parts, hipStream_t s) {
     const int n_mt = (rows + TM - 1) / TM, n_nt = (w.row_tiles + TN / 16 - 1) / (TN / 16), per = (n_mt * n_nt + 7) / 8;
-    hipLaunchKernelGGL((dense_tile_kernel<TM, TN, WM, WN, NS, OUT>), dim3(per * 8, parts), dim3(64 * WM * WN), (size_t) NS * (TM / 16 + TN / 16) * 1024, s, w, (const bamd_bf *) x, ldx, rows, out, ldo, n_mt, n_nt, limit);
+    hipLaunchKernelGGL((dense_tile_kernel<T, TM, TN, WM, WN, NS, OUT>), dim3(per * 8, parts), dim3(64 * WM * WN), (size_t) NS * (TM / 16 * sizeof(T) / 2 + TN / 16) * 1024, s, w, (const T *) x, ldx, rows, out, ldo, n_mt, n_nt, limit);
     return 0;
 }
 // The tile whose rounds over the 256 CUs end first.  Measured per block of 32 columns, all CUs busy (ns): 256 x 256 700, 128 x 256 450, 128 x 128 250, all three one block per CU,
@@ -236,11 +168,11 @@ static int tile_go(const bamd_dense & w, const void * x, int ldx, int rows, void
 // start and end once more (4 us).  131 x 2048 x 8192: 38 -> 22 us, 412 x 4096 x 8192: 85 -> 39; four shares were no faster (24 and 43 us)
 template <typename T, int OUT>
 static int gemm_tiles(const bamd_dense & w, const void * x, int ldx, int rows, void * out, int ldo, float limit, hipStream_t s, int * parts = nullptr) {
-    if constexpr (sizeof(T) == 4) {
-        if (parts) *parts = 1;
-        const int n_mt = (rows + 63) / 64, n_nt = (w.row_tiles + 3) / 4, per = (n_mt * n_nt + 7) / 8;
-        hipLaunchKernelGGL((dense_gemm_kernel<T, 64, 64, 2, OUT>), dim3(per * 8), dim3(256), 2 * (4 * 2 * 64 * 8 * sizeof(T) + 4 * 2 * 1024), s, w, (const T *) x, ldx, rows, out, ldo, n_mt, n_nt, limit);
-        return 0;
+    if constexpr (sizeof(T) == 4) {                               // bound by the f32 matrix instructions: small tiles, several blocks per CU
+        const long tiles = (long) ((rows + 63) / 64) * ((w.row_tiles + 3) / 4);
+        const int share = OUT == BAMD_OUT_F32 && parts && *parts > 1 && tiles <= 192 && w.k_tiles >= 32 ? 2 : 1;
+        if (parts) *parts = share;
+        return tile_go<T, 64, 64, 2, 2, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
     } else {
         auto tiles = [&](int tm, int tn) { return (long) ((rows + tm - 1) / tm) * ((w.row_tiles * 16 + tn - 1) / tn); };
         long best = 0; int pick = 0, share = 1;
@@ -253,14 +185,14 @@ static int gemm_tiles(const bamd_dense & w, const void * x, int ldx, int rows, v
         }
         if (parts) *parts = share;
         switch (pick) {
-            case 0: return tile_go<256, 256, 2, 4, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
-            case 1: return tile_go<128, 256, 2, 4, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
-            case 2: return tile_go<128, 128, 2, 4, 8, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
-            case 3: return tile_go<64, 128, 2, 2, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
+            case 0: return tile_go<T, 256, 256, 2, 4, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
+            case 1: return tile_go<T, 128, 256, 2, 4, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
+            case 2: return tile_go<T, 128, 128, 2, 4, 8, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
+            case 3: return tile_go<T, 64, 128, 2, 2, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
         }
         // one tile per CU at most: twice the stages hide more of the memory's latency (131 x 2048 x 8192: 49 -> 38 us); with more, blocks hide each other's
-        if (tiles(64, 64) * share <= 256) return tile_go<64, 64, 2, 2, 8, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
-        return tile_go<64, 64, 2, 2, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
+        if (tiles(64, 64) * share <= 256) return tile_go<T, 64, 64, 2, 2, 8, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
+        return tile_go<T, 64, 64, 2, 2, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
     }
 }
 // f32 rows are stored four matrix rows at a time: ldo % 4 == 0; x rows start on 16 bytes and hold k_tiles * 32 columns
