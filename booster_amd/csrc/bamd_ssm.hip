@@ -82,11 +82,21 @@ __global__ void __launch_bounds__(256) ssm_step_kernel(bamd_batch_dev b, bamd_ss
     ix.g = ix.h / per;
     const float * in = a.in + (size_t) e.row0 * a.ld;
     float * st = a.state + (((size_t) e.seq * a.heads + ix.h) * N) * a.P + ix.p0;
-    float s[NPL][4];
+    // sixteen bytes at a time where rows start on sixteen bytes (pw is then a multiple of four as well), from a place clamped into the state: a branch around each of 4 NPL single values
+    // made sixteen sequences of 128 heads x 64 x 128 take 48 us for 134 MB, now 31
+    const bool wide = (a.P & 3) == 0;
+    bamd_v4 s[NPL];
+    if (wide) {
 #pragma unroll
-    for (int j = 0; j < NPL; ++j)
+        for (int j = 0; j < NPL; ++j) s[j] = *(const bamd_v4 *) (st + (size_t) min(grp * NPL + j, N - 1) * a.P + min(quad * 4, ix.pw - 4));
 #pragma unroll
-        for (int k = 0; k < 4; ++k) { const int n = grp * NPL + j, p = quad * 4 + k; s[j][k] = (e.pos0 > 0 && n < N && p < ix.pw) ? st[(size_t) n * a.P + p] : 0.f; }
+        for (int j = 0; j < NPL; ++j) if (!(e.pos0 > 0 && grp * NPL + j < N && quad * 4 < ix.pw)) s[j] = bamd_v4{ 0, 0, 0, 0 };
+    } else {
+#pragma unroll
+        for (int j = 0; j < NPL; ++j)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) { const int n = grp * NPL + j, p = quad * 4 + k; s[j][k] = (e.pos0 > 0 && n < N && p < ix.pw) ? st[(size_t) n * a.P + p] : 0.f; }
+    }
     const float D = a.D[ix.h];
     for (int i = tid; i < PT + 2 * NP; i += 256) ops[i] = 0.f;
     auto slot = [&](int c) { return c < ix.pw ? c : c < ix.pw + N ? PT + (c - ix.pw) : PT + NP + (c - ix.pw - N); };
@@ -122,6 +132,11 @@ __global__ void __launch_bounds__(256) ssm_step_kernel(bamd_batch_dev b, bamd_ss
         for (int g = 0; g < GROUPS; ++g) y[g & 3] += yp[g][tid];
         const float z = in[ix.h * a.P + ix.p0 + tid];
         a.out[(size_t) e.row0 * a.ldo + ix.h * a.P + ix.p0 + tid] = ((y[0] + y[1]) + (y[2] + y[3]) + D * xs[tid]) * silu_f(z);
+    }
+    if (wide) {
+#pragma unroll
+        for (int j = 0; j < NPL; ++j) if (grp * NPL + j < N && quad * 4 < ix.pw) *(bamd_v4 *) (st + (size_t) (grp * NPL + j) * a.P + quad * 4) = s[j];
+        return;
     }
 #pragma unroll
     for (int j = 0; j < NPL; ++j)
