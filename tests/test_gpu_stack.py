@@ -54,13 +54,10 @@ def test_dense(bamd, dtype, n, k, rows):
                 assert np.abs(bamd.op_dense(w, x, dtype, impl) - want).max() < 8e-6 * scale
 
 
-# one size per tile of the many-row product (256 x 256, 128 x 256, 128 x 128, 64 x 128, 64 x 64 with four and with eight stages), ragged in every dimension, fewer and more column blocks than stages
-@pytest.mark.parametrize("n,rows", [(8170, 2045), (8170, 1000), (4090, 1000), (4090, 1100), (8190, 131), (2047, 131)])
+# one size per tile of the many-row product (256 x 256, 128 x 256, 128 x 128, 64 x 128, 64 x 64 with four and with eight stages; 32-bit: 64 x 64), ragged in every dimension, fewer and more column blocks than stages
+@pytest.mark.parametrize("dtype,n,rows", [("bfloat16", 8170, 2045), ("bfloat16", 8170, 1000), ("bfloat16", 4090, 1000), ("bfloat16", 4090, 1100), ("bfloat16", 8190, 131), ("bfloat16", 2047, 131), ("float32", 2047, 131)])
 @pytest.mark.parametrize("k", [1, 70, 300])
-@pytest.mark.parametrize("dtype", DTYPES)
 def test_dense_tiles(bamd, dtype, n, rows, k):
-    if dtype == "float32" and n > 2047:
-        pytest.skip("one tile only")
     r = np.random.default_rng(n + k + rows)
     w = so.f32_to_bf16(r.standard_normal((n, k)).astype(np.float32))
     x = r.standard_normal((rows, k)).astype(np.float32)
