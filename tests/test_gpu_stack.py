@@ -185,6 +185,34 @@ def test_ssm_chunks(bamd, H, P, N, G):
         pos += n
 
 
+# a token of a prompt that is not finite leaves the tokens in front of it as they are (in B, C, x and the step size, at several places of a chunk), and so does a state handed over that is not;
+# "far": finite values whose product with a token further back overflows
+@pytest.mark.parametrize("N,at", [(40, 20), (128, 30), (200, 17)])
+@pytest.mark.parametrize("what,value", [("x", np.inf), ("x", np.nan), ("B", np.inf), ("C", np.nan), ("dt", np.inf), ("far", 1e20), ("state", np.inf)])
+def test_ssm_tokens_that_are_not_finite(bamd, N, at, what, value):
+    H, P, n = 2, 40, 70
+    r = np.random.default_rng(N)
+    inner, ch = H * P, H * P + 2 * N
+    f = lambda a: np.asarray(a, np.float32)
+    conv, cb, dtb, A, D = map(f, (r.uniform(0.5, 2, (ch, 1)), np.zeros(ch), r.uniform(-2, 1, H), r.uniform(-2, 1, H), r.standard_normal(H)))
+    rows, S = f(r.standard_normal((n, inner + ch + H))), f(r.standard_normal((H, N, P)))
+    x, B, C = inner + P + 33, 2 * inner + N // 2, 2 * inner + N + 1                  # a column of the second head, a state row of both
+    if what == "state":
+        S[1, N - 1, 5] = value
+    elif what == "far":
+        rows[at, 2 * inner + N + N // 2] = rows[at + 1, B] = value
+    else:
+        rows[at, {"x": x, "B": B, "C": C, "dt": -1}[what]] = value
+    with np.errstate(all="ignore"):
+        want, _, _ = plain_ssm(rows.astype(np.float64), H, P, N, 1, conv, cb, dtb, A, D, np.zeros((0, ch)), S.astype(np.float64))
+    got, _, _ = bamd.op_ssm(rows, 1, H, P, N, 1, conv, cb, dtb, A, D, np.zeros((0, ch)), S)
+    assert np.isfinite(want[:at] if what != "state" else want[:, :P]).all() and (what == "far" or not np.isfinite(want).all())
+    for t in range(n):
+        ok = np.isfinite(want[t])
+        assert (np.isfinite(got[t]) == ok).all(), t
+        assert not ok.any() or rel(got[t][ok], want[t][ok]) < 2e-5, t                # as test_ssm
+
+
 def plain_attention(q, c, gate, past, uk, uv, c_norm, sink, scale, eps, H):
     T, _, d = q.shape
     lat = np.stack([so.rms(v, eps) * c_norm for v in c])
