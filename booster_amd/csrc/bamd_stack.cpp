@@ -180,6 +180,7 @@ struct Timer {                                     // per-launch HIP events (pro
 };
 #define STACK_CTX 8192                             /* positions of a context that asks for none, where the model sets no bound */
 #define STACK_ROWS 2048                            /* token rows of one pass */
+#define Y2_PLANES 2                                /* shares of K of an output or down projection: there is room for them whatever the rows, so that whether K is halved goes by the shape alone */
 #define SEG_MIN 64                                 /* tokens of the shortest scan segment */
 #define PAIR_ROWS 4                                /* decoding rows up to which two branches share their launches */
 #define SEG_BLOCKS 768                             /* blocks a scan wants */
@@ -576,7 +577,7 @@ int Stack::context_init(bamd_context * bc) {
     }
     const size_t R = (size_t) c.rows_cap;
     if (dev_alloc(bc->allocs, (void **) &c.xa, R * E * 4) || dev_alloc(bc->allocs, (void **) &c.xb, R * E * 4) || dev_alloc(bc->allocs, (void **) &c.y, R * std::max(c.ldy, 16) * 4) ||
-        dev_alloc(bc->allocs, (void **) &c.y2, R * c.ldy2 * 4) || dev_alloc(bc->allocs, (void **) &c.y3, R * std::max(c.ldy3, 16) * 4) || dev_alloc(bc->allocs, &c.h, R * c.ldh * el())) return 1;
+        dev_alloc(bc->allocs, (void **) &c.y2, R * c.ldy2 * 4 * Y2_PLANES) || dev_alloc(bc->allocs, (void **) &c.y3, R * std::max(c.ldy3, 16) * 4) || dev_alloc(bc->allocs, &c.h, R * c.ldh * el())) return 1;
     if (qp && dev_alloc(bc->allocs, &c.qp, qp * el())) return 1;
     if (po && (dev_alloc(bc->allocs, (void **) &c.part_o, po * 4) || dev_alloc(bc->allocs, (void **) &c.part_ml, pm * 4))) return 1;
     if (qp) HIPC(hipMemset(c.qp, 0, qp * el()));                  // rows of absent heads stay zero
@@ -722,9 +723,8 @@ int Parallel::run(Pass & p, MixState & st, Operand & o) {
 }
 int Pass::layers() {
     bamd_pre_args pa; memset((void *) &pa, 0, sizeof pa);
-    const int room = std::min(2, c.rows_cap / b.rows);             // planes of these rows that fit the result's buffer
     for (size_t i = 0; i < st.layers.size(); ++i) {
-        int parts = room;
+        int parts = Y2_PLANES;
         Layer & ly = st.layers[i];
         Mixer & mx = *ly.mix;
         pa.res = residual(ly.shift, c.prev[i], ly.pre1);
@@ -735,7 +735,7 @@ int Pass::layers() {
         else { pa.grp = o.grp; if (product_pre(mx.out, o.pre, pa, c.y2, c.ldy2, 3, &parts)) return 1; }
         advanced(c.y2, c.ldy2, ly.norm1, parts);
         if (!ly.mlp) continue;
-        parts = room;
+        parts = Y2_PLANES;
         pa.res = residual(nullptr, nullptr, ly.pre2);
         const bool glu = st.d.mlp_act == STACK_ACT_CLAMPED_GLU;
         if (glu && b.rows > BAMD_MV_ROWS) {                        // the product's tiles write the down-projection's operand

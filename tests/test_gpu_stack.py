@@ -347,6 +347,25 @@ def test_models_whose_products_are_halved(bamd, dtype, width, design, tmp_path):
     c.close(); m.close()
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("design", ["Tupitar", "Mafurax"])
+def test_a_context_that_is_just_large_enough_gives_the_same_bits(bamd, dtype, design, tmp_path):
+    """products of 5 row tiles and 66 column blocks, which are halved: with every row of the context's scratch in use as with a fraction of it"""
+    if design == "Tupitar":
+        cfg = stack_cases.config(76, 131, [stack_cases.mamba(33, 64, 8, 1, 1, 2, ff=2100), stack_cases.latent(9, 24, 250, 36, 0.31, ff=2100)], max_positions=1024)
+    else:
+        cfg = stack_cases.mafurax(76, 131, [stack_cases.parallel(stack_cases.attend(17, 1, 24, 120, 0.4, 6.0, 50, 19, 3), 0.7, (3, 10, 14, 8.0), 1.3, ff=2100, limit=0.8)])
+    m = bamd.Model(Case(str(tmp_path / "m"), cfg, 3, dict(rel=8, rank=5)).folder, dtype=dtype)
+    for n in (64, 320):
+        got = []
+        for n_ctx in (n, 1024):
+            c = bamd.Context(m, n_ctx, 1)
+            got.append(c.decode(tokens(cfg, n, 30), 0))
+            c.close()
+        assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32)), n
+    m.close()
+
+
 @pytest.mark.parametrize("n", [1, 2, 3, 5, 64, 65, 150])
 def test_prompt(run, n):
     case, c, dtype = run
