@@ -42,6 +42,7 @@ struct bamd_residual_args {
 };
 void bamd_launch_embed_rows(const bamd_batch_dev & b, const uint16_t * embd, const uint16_t * pos, float scale, int E, int V, float * x, hipStream_t s);
 void bamd_launch_residual_rows(int act, const bamd_batch_dev & b, const bamd_residual_args & a, hipStream_t s);
+int bamd_norm_threads(int n, int rows);            // threads of a block that norms one of so many rows of n
 // a N(z) + b N(z^2) + c N(z^3) + e with coef = {a, b, c, e}, N = division by the root mean square over the F values
 struct bamd_poly_args { const float * z; int ldz; const float * coef; float eps; void * h; int F, ldh; };
 void bamd_launch_poly_rows(int act, int rows, const bamd_poly_args & a, hipStream_t s);

@@ -72,25 +72,28 @@ __global__ void __launch_bounds__(64) advance_kernel(bamd_entry * ent, int32_t *
 }
 
 static dim3 row_block(int n) { return dim3(n > 1024 ? 1024 : 256); }
-// rows that two pieces of four floats per thread hold (RowRegs<2>): no more waves than that takes, since every sum over the row waits for all of them
-// (layer norms of six rows of 2048: 6.6 -> 5.5 us, of 2048 rows of 4096: 32 -> 23 us; up to 1024 threads before)
-static dim3 sum_block(int n) { return dim3(std::min(1024, std::max(256, (n / 8 + 63) / 64 * 64))); }
+// Rows that two pieces of four floats per thread hold (RowRegs<2>): no more waves than that takes, since every sum over the row waits for all of them
+// (layer norms of six rows of 2048: 6.6 -> 5.5 us, of 2048 rows of 4096: 32 -> 23 us; up to 1024 threads before; six rows of 2052: 5.3 -> 4.8 us, 14.1 on the 256 threads that fall four floats short).  Rows that are not held (no multiple of four) are read again for every
+// sum, one float per thread and step: all the threads there are (six rows of 2050 on 256 threads: 13.9 us, on 1024: 7.8), unless there are rows for more blocks than are resident at once
+// (a prompt of 2048 tokens of width 1030 on 1024 threads: 855 us, on 256: 815)
+int bamd_norm_threads(int n, int rows) { return (n & 3) && rows <= 512 ? (int) row_block(n).x : std::min(1024, std::max(256, ((n + 7) / 8 + 63) / 64 * 64)); }
+static dim3 sum_block(int n, int rows) { return dim3(bamd_norm_threads(n, rows)); }
 void bamd_launch_embed_rows(const bamd_batch_dev & b, const uint16_t * embd, const uint16_t * pos, float scale, int E, int V, float * x, hipStream_t s) {
     hipLaunchKernelGGL(embed_rows_kernel, dim3((E + 1023) / 1024, b.rows), dim3(256), 0, s, b, embd, pos, scale, E, V, x);
 }
 void bamd_launch_residual_rows(int act, const bamd_batch_dev & b, const bamd_residual_args & a, hipStream_t s) {
     if (a.norm == BAMD_NORM_LAYER) {
-        if (act == BAMD_ACT_F32) hipLaunchKernelGGL(layer_rows_kernel<float>, dim3(b.rows), sum_block(a.E), 0, s, a, nullptr, a.gi);
-        else hipLaunchKernelGGL(layer_rows_kernel<bamd_bf>, dim3(b.rows), sum_block(a.E), 0, s, a, nullptr, a.gi);
-    } else if (act == BAMD_ACT_F32) hipLaunchKernelGGL(residual_rows_kernel<float>, dim3(b.rows), sum_block(a.E), 0, s, b, a);
-    else hipLaunchKernelGGL(residual_rows_kernel<bamd_bf>, dim3(b.rows), sum_block(a.E), 0, s, b, a);
+        if (act == BAMD_ACT_F32) hipLaunchKernelGGL(layer_rows_kernel<float>, dim3(b.rows), sum_block(a.E, b.rows), 0, s, a, nullptr, a.gi);
+        else hipLaunchKernelGGL(layer_rows_kernel<bamd_bf>, dim3(b.rows), sum_block(a.E, b.rows), 0, s, a, nullptr, a.gi);
+    } else if (act == BAMD_ACT_F32) hipLaunchKernelGGL(residual_rows_kernel<float>, dim3(b.rows), sum_block(a.E, b.rows), 0, s, b, a);
+    else hipLaunchKernelGGL(residual_rows_kernel<bamd_bf>, dim3(b.rows), sum_block(a.E, b.rows), 0, s, b, a);
 }
 void bamd_launch_final_rows(int act, const bamd_residual_args & a, const int32_t * want, int n_want, const float * gf, hipStream_t s) {
     if (a.norm == BAMD_NORM_LAYER) {
-        if (act == BAMD_ACT_F32) hipLaunchKernelGGL(layer_rows_kernel<float>, dim3(n_want), sum_block(a.E), 0, s, a, want, gf);
-        else hipLaunchKernelGGL(layer_rows_kernel<bamd_bf>, dim3(n_want), sum_block(a.E), 0, s, a, want, gf);
-    } else if (act == BAMD_ACT_F32) hipLaunchKernelGGL(final_rows_kernel<float>, dim3(n_want), sum_block(a.E), 0, s, a, want, gf);
-    else hipLaunchKernelGGL(final_rows_kernel<bamd_bf>, dim3(n_want), sum_block(a.E), 0, s, a, want, gf);
+        if (act == BAMD_ACT_F32) hipLaunchKernelGGL(layer_rows_kernel<float>, dim3(n_want), sum_block(a.E, n_want), 0, s, a, want, gf);
+        else hipLaunchKernelGGL(layer_rows_kernel<bamd_bf>, dim3(n_want), sum_block(a.E, n_want), 0, s, a, want, gf);
+    } else if (act == BAMD_ACT_F32) hipLaunchKernelGGL(final_rows_kernel<float>, dim3(n_want), sum_block(a.E, n_want), 0, s, a, want, gf);
+    else hipLaunchKernelGGL(final_rows_kernel<bamd_bf>, dim3(n_want), sum_block(a.E, n_want), 0, s, a, want, gf);
 }
 void bamd_launch_poly_rows(int act, int rows, const bamd_poly_args & a, hipStream_t s) {
     if (act == BAMD_ACT_F32) hipLaunchKernelGGL(poly_rows_kernel<float>, dim3(rows), row_block(a.F), 0, s, a);

@@ -1100,6 +1100,7 @@ SafeTensor bf16_tensor(const uint16_t * p, std::vector<int64_t> shape) { SafeTen
 }  // namespace
 #define BAMD_OP extern "C" __attribute__((visibility("default"))) int
 
+BAMD_OP bamd_op_norm_threads(int n, int rows) { return bamd_norm_threads(n, rows); }
 BAMD_OP bamd_op_dense(int act, const uint16_t * w, int nrows, int k, const float * x, int rows, int impl, float * y) {
     OpScratch s; bamd_dense d; void * dx; float * dy = nullptr;
     if (!w || !x || !y || nrows < 1 || k < 1 || rows < 1 || s.init(act)) return fail("bamd_op_dense: bad arguments");

@@ -32,6 +32,24 @@ def test_layer_norms_around_a_sublayer(bamd, dtype, E, rows, with_y, with_pre):
     near(h, np.stack([so.layer_norm(a, gi, 1e-4) for a in ref]) if with_pre else ref, dtype)
 
 
+# widths just inside and outside of what a block of four or five waves keeps in registers, and widths that no block keeps
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("E", [1030, 2044, 2048, 2050, 2052, 2560, 2564, 4100])
+def test_norms_of_rows_at_the_edge_of_a_block(bamd, dtype, E):
+    r = np.random.default_rng(E)
+    f = lambda a: np.asarray(a, np.float32).astype(np.float64)
+    x, y, g, gi, mu, prev = f(r.standard_normal((3, E))), f(r.standard_normal((3, E)) - 2), f(r.standard_normal(E)), f(1 + 0.3 * r.standard_normal(E)), f(r.uniform(0, 1, E)), f(r.standard_normal(E))
+    xo, h = bamd.op_layer_rows(x, y, g, gi, 1e-4, dtype)
+    ref = np.stack([a + so.layer_norm(b, g, 1e-4) for a, b in zip(x, y)])
+    near(xo, ref, "float32")
+    near(h, np.stack([so.layer_norm(a, gi, 1e-4) for a in ref]), dtype)
+    xo, h, last = bamd.op_residual_rows(x, y, 0.7, 1e-3, mu, prev, 5, dtype)
+    ref = np.stack([a + so.scalar_norm(b, 0.7, 1e-3) for a, b in zip(x, y)])
+    near(xo, ref, "float32")
+    near(h, np.stack([so.token_shift(a, b, mu) for a, b in zip(ref, np.concatenate([prev[None], ref[:-1]]))]), dtype)
+    near(last, ref[-1], "float32")
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("F,rows,limit", [(1, 1, 1.0), (40, 3, 0.5), (333, 2, 2.0), (3000, 2, 7.0)])
 def test_clamped_glu(bamd, dtype, F, rows, limit):
