@@ -1451,6 +1451,13 @@ extern "C" __attribute__((visibility("default"))) int bamd_op_mul_mat_vec(int ty
                                    const float * residual, float * y, int mode) {
     return op_matvec(type, w_raw, nullptr, nrows, k, x, norm_w, eps, residual, y, residual ? BAMD_EPI_ADD : BAMD_EPI_STORE, mode);
 }
+extern "C" __attribute__((visibility("default"))) int bamd_op_prefill_route(int type, int nrows, int k, int T, int * few_tiles, int * lds, int * most) {
+    if (!bamd_is_kquant(type) || k <= 0 || k % 256 || nrows <= 0 || T <= 0 || !few_tiles || !lds || !most) return fail("bad type/shape");
+    size_t m = 0;
+    *lds = (int) bamd_prefill_route(type, (nrows + 7) / 8 * 8, k, T, few_tiles, &m);
+    *most = (int) m;
+    return 0;
+}
 // batched mat-mul of T activation rows against one matrix through the prefill kernels: impl 0 = integer-dot kernel, 2 = matrix-core kernel (1 and 3 were the generations removed in round 6)
 extern "C" __attribute__((visibility("default"))) int bamd_op_mul_mat_batch(int type, const void * w_raw, int nrows, int k, const float * x, int T, const float * norm_w,
                                                                               float eps, const float * residual, float * y, int impl) {

@@ -94,6 +94,7 @@ void bamd_launch_quantize_batch(const float * x, const float * nw, float eps, in
 // BAMD_EPI_SILU_MUL: out = silu(res) * y (res = the gate projection, may alias out).  The A fragments are built once per 64-row x 64-token workgroup from the
 // wave-stream copy and the matrix's load-time side table (aux: bamd_prefill_aux_bytes bytes, filled by bamd_launch_prefill_aux).  1 = type / shape not supported or no table
 int  bamd_prefill_mfma_supported(void);      // the current device accepts the kernels' LDS size (asked at model load)
+size_t bamd_prefill_route(int type, int nrows_pad, int K, int T, int * few_tiles, size_t * most);      // dynamic LDS of the launch such a product takes; the few-token kernel's token tiles (0: another kernel); the most that is asked for at model load
 size_t bamd_prefill_aux_bytes(int type, int nrows_pad, int K);
 void bamd_launch_prefill_aux(const void * w_stream, int type, int nrows_pad, int K, void * aux, hipStream_t s);
 int  bamd_launch_matmul_mfma2(const void * w_stream, const void * aux, int type, int nrows, int nrows_pad, int K, const void * blob16, int T, float * out, const float * res,

@@ -557,7 +557,9 @@ template <int TYPE> struct FewW { static constexpr int SLOT = TYPE == BAMD_Q6_K 
 #define XF_RING 3                                         /* super-blocks of token records in LDS */
 #define XF_WRING 5                                        /* of the row tile's operands */
 constexpr int few_records(int ntt) { return (ntt * 16 * BAMD_B16_Q + 63) / 64; }       /* KiB of token records of a super-block */
-template <int TYPE, int NTT> constexpr size_t few_lds() { return (size_t) 16 * X_FR + (size_t) XF_RING * few_records(NTT) * 1024 + (size_t) XF_WRING * FewW<TYPE>::SLOT + 32; }
+constexpr size_t few_lds(int type, int ntt) {
+    return (size_t) 16 * X_FR + (size_t) XF_RING * few_records(ntt) * 1024 + (size_t) XF_WRING * (type == BAMD_Q6_K ? FewW<BAMD_Q6_K>::SLOT : type == BAMD_Q5_K ? FewW<BAMD_Q5_K>::SLOT : FewW<BAMD_Q4_K>::SLOT) + 32;
+}
 template <int TYPE, int EPI, int NTT>
 __global__ void __launch_bounds__(768) matmul_few_kernel(bamd_mma2_args a) {
     constexpr bool Q5 = TYPE == BAMD_Q5_K, Q6 = TYPE == BAMD_Q6_K;
@@ -788,15 +790,35 @@ void bamd_launch_prefill_aux(const void * w_stream, int type, int nrows_pad, int
     else if (type == BAMD_Q5_K) hipLaunchKernelGGL((prefill_aux_q4k_kernel<true>), grid, dim3(64), 0, s, (const uint8_t *) w_stream, nrows_pad, nb, ph, ch);
     else                        hipLaunchKernelGGL((prefill_aux_q4k_kernel<false>), grid, dim3(64), 0, s, (const uint8_t *) w_stream, nrows_pad, nb, ph, ch);
 }
-// 1 when the current device takes the matrix-core kernels' launches (158 784 B of dynamic LDS at 1024 threads): asked once per model load, before any side table is
-// built (a rejected launch would otherwise leave stale output behind a success code)
+// the most dynamic LDS any launch below takes
+static constexpr size_t x_max_lds() {
+    size_t m = few_lds(BAMD_Q6_K, 4);
+    for (const size_t v : { (size_t) X3_LDS_BYTES, (size_t) X_LDS_BYTES, few_lds(BAMD_Q4_K, 4), few_lds(BAMD_Q5_K, 4) }) m = v > m ? v : m;
+    return m;
+}
+static bool x_takes(const void * kernel, size_t lds) { return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds) == hipSuccess; }
+// 1 when the current device takes the matrix-core kernels' launches (159 328 B of dynamic LDS, up to 1024 threads): asked once per model load, before any side table is built, since a
+// rejected launch would leave stale output behind a success code
 int bamd_prefill_mfma_supported(void) {
     int dev = 0, lds = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess) { (void) hipGetLastError(); return 0; }
-    if ((size_t) lds < (size_t) X3_LDS_BYTES || (size_t) lds < (size_t) X_LDS_BYTES) return 0;
-    if (hipFuncSetAttribute((const void *) matmul_mfma3_q4k_kernel<BAMD_EPI_STORE, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) X3_LDS_BYTES) != hipSuccess ||
-        hipFuncSetAttribute((const void *) matmul_mfma2_q6k_kernel<BAMD_EPI_STORE>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) X_LDS_BYTES) != hipSuccess) { (void) hipGetLastError(); return 0; }
+    if ((size_t) lds < x_max_lds()) return 0;
+    if (!x_takes((const void *) matmul_mfma3_q4k_kernel<BAMD_EPI_STORE, false>, X3_LDS_BYTES) || !x_takes((const void *) matmul_mfma2_q6k_kernel<BAMD_EPI_STORE>, X_LDS_BYTES) ||
+        !x_takes((const void *) matmul_few_kernel<BAMD_Q6_K, BAMD_EPI_STORE, 4>, few_lds(BAMD_Q6_K, 4))) { (void) hipGetLastError(); return 0; }
     return 1;
+}
+// Token tiles (of 16) per block of the few-token kernel for this product, 0: one of the kernels with 64-row blocks.
+// Up to 64 tokens: whichever ends first, measured per super-block of a round of 256 blocks (Q4_K): 64-row blocks 1500 ns at any number of tokens, 16-row blocks 480 up to
+// 32 tokens, 700 up to 48 (790 at K = 4096), 800 above
+static int x_few_tiles(int nrows_pad, int T) {
+    if (T > 64) return 0;
+    const long c16 = T <= 32 ? 480 : T <= 48 ? 700 : 800;
+    if (((nrows_pad + 15) / 16 + 255) / 256 * c16 >= ((long) x_row_blocks(nrows_pad) + 255) / 256 * 1500) return 0;
+    return T <= 32 ? 2 : T <= 48 ? 3 : 4;
+}
+size_t bamd_prefill_route(int type, int nrows_pad, int, int T, int * few_tiles, size_t * most) {
+    *few_tiles = x_few_tiles(nrows_pad, T); *most = x_max_lds();
+    return *few_tiles ? few_lds(type, *few_tiles) : type == BAMD_Q6_K ? X_LDS_BYTES : X3_LDS_BYTES;
 }
 int bamd_launch_matmul_mfma2(const void * w_stream, const void * aux, int type, int nrows, int nrows_pad, int K, const void * blob16, int T, float * out, const float * res,
                              int epi, int ldo, hipStream_t s) {
@@ -816,15 +838,12 @@ int bamd_launch_matmul_mfma2(const void * w_stream, const void * aux, int type, 
         if (epi == BAMD_EPI_ADD)           hipLaunchKernelGGL((KERNEL<BAMD_EPI_ADD __VA_ARGS__>),      grid3, dim3(1024), X3_LDS_BYTES, s, a); \
         else if (epi == BAMD_EPI_SILU_MUL) hipLaunchKernelGGL((KERNEL<BAMD_EPI_SILU_MUL __VA_ARGS__>), grid3, dim3(1024), X3_LDS_BYTES, s, a); \
         else                               hipLaunchKernelGGL((KERNEL<BAMD_EPI_STORE __VA_ARGS__>),    grid3, dim3(1024), X3_LDS_BYTES, s, a); } while (0)
-    // up to 64 tokens: whichever ends first, measured per super-block of a round of 256 blocks (Q4_K): 64-row blocks 1500 ns at any number of tokens, 16-row blocks 480 up to
-    // 32 tokens, 700 up to 48 (790 at K = 4096), 800 above
-    const long c16 = T <= 32 ? 480 : T <= 48 ? 700 : 800;
-    if (T <= 64 && ((nrows_pad + 15) / 16 + 255) / 256 * c16 < ((long) grid.y + 255) / 256 * 1500) {
+    if (const int ntt = x_few_tiles(nrows_pad, T)) {
 #define XF_LAUNCH(TYPE_, NTT_) do { const dim3 gf((T + 16 * NTT_ - 1) / (16 * NTT_), (nrows_pad + 15) / 16); \
-        if (epi == BAMD_EPI_ADD)           hipLaunchKernelGGL((matmul_few_kernel<TYPE_, BAMD_EPI_ADD, NTT_>),      gf, dim3(768), (few_lds<TYPE_, NTT_>()), s, a); \
-        else if (epi == BAMD_EPI_SILU_MUL) hipLaunchKernelGGL((matmul_few_kernel<TYPE_, BAMD_EPI_SILU_MUL, NTT_>), gf, dim3(768), (few_lds<TYPE_, NTT_>()), s, a); \
-        else                               hipLaunchKernelGGL((matmul_few_kernel<TYPE_, BAMD_EPI_STORE, NTT_>),    gf, dim3(768), (few_lds<TYPE_, NTT_>()), s, a); } while (0)
-#define XF_TYPE(TYPE_) do { if (T <= 32) XF_LAUNCH(TYPE_, 2); else if (T <= 48) XF_LAUNCH(TYPE_, 3); else XF_LAUNCH(TYPE_, 4); } while (0)
+        if (epi == BAMD_EPI_ADD)           hipLaunchKernelGGL((matmul_few_kernel<TYPE_, BAMD_EPI_ADD, NTT_>),      gf, dim3(768), few_lds(TYPE_, NTT_), s, a); \
+        else if (epi == BAMD_EPI_SILU_MUL) hipLaunchKernelGGL((matmul_few_kernel<TYPE_, BAMD_EPI_SILU_MUL, NTT_>), gf, dim3(768), few_lds(TYPE_, NTT_), s, a); \
+        else                               hipLaunchKernelGGL((matmul_few_kernel<TYPE_, BAMD_EPI_STORE, NTT_>),    gf, dim3(768), few_lds(TYPE_, NTT_), s, a); } while (0)
+#define XF_TYPE(TYPE_) do { if (ntt == 2) XF_LAUNCH(TYPE_, 2); else if (ntt == 3) XF_LAUNCH(TYPE_, 3); else XF_LAUNCH(TYPE_, 4); } while (0)
         if (type == BAMD_Q6_K)      XF_TYPE(BAMD_Q6_K);
         else if (type == BAMD_Q5_K) XF_TYPE(BAMD_Q5_K);
         else                        XF_TYPE(BAMD_Q4_K);

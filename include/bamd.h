@@ -241,8 +241,10 @@ int bamd_op_ssm(const float * in, int rows, int pos0, int heads, int P, int N, i
 /* q [rows][heads][dim], c [rows][rank] and gate [rows][heads] (or NULL) as projected; past [pos0][rank]: the cached latents in front; decode: the one-row kernels */
 int bamd_op_latent_attention(int act, const float * q, const float * c, const float * gate, int rows, const float * past, int pos0, int heads, int dim, int vdim, int rank, float scale, float eps,
                              const float * c_norm, const uint16_t * uk, const uint16_t * uv, const float * sink, int decode, float * out);
-/* which form of a kernel a size takes (host arithmetic, no device needed): threads of a block that norms one of so many rows of n floats */
+/* which form of a kernel a size takes (host arithmetic, no device needed).  Threads of a block that norms one of so many rows of n floats */
 int bamd_op_norm_threads(int n, int rows);
+/* the matrix-core product of T tokens with a K-quant matrix: token tiles per block of the few-token kernel (0: 64-row blocks), the launch's dynamic LDS, and the most any such launch takes */
+int bamd_op_prefill_route(int type, int nrows, int k, int T, int * few_tiles, int * lds, int * most);
 /* RoPE (cos,sin) table row as built on the host for position pos (ggml_rope_cache_init, ggml.c:14017) */
 int bamd_op_rope_row(int pos, int n_dims, float freq_base, float freq_scale, const float * freq_factors, float * row);
 
