@@ -808,16 +808,24 @@ int bamd_prefill_mfma_supported(void) {
     return 1;
 }
 // Token tiles (of 16) per block of the few-token kernel for this product, 0: one of the kernels with 64-row blocks.
-// Up to 64 tokens: whichever ends first, measured per super-block of a round of 256 blocks (Q4_K): 64-row blocks 1500 ns at any number of tokens, 16-row blocks 480 up to
-// 32 tokens, 700 up to 48 (790 at K = 4096), 800 above
-static int x_few_tiles(int nrows_pad, int T) {
+// Up to 64 tokens: whichever ends first.  Both take a start and a time per super-block, for every round of 256 blocks.  The few-token kernel's goes by its token tiles, and with three (33 to
+// 48 tokens) by how the records of neighbouring tokens lie to the 128-byte lines that they are copied in: a stride of about half a line more or less is the fast one.  Constants in ns,
+// fitted to 1323 sizes (three types, 8 to 64 tokens, 1024 to 24576 rows, K 1024 to 14336), of which this rule takes the slower kernel for 23 by more than 1.5 %, at most 4 %.
+// Where the two part, K = 4096, 64-row blocks against 16-row ones in us: 8192 rows Q4_K 32 tokens 24.1 | 18.4, 48 tokens 24.0 | 22.7, 64 tokens 24.1 | 25.5; 12288 rows 32 tokens 25.2 | 27.9;
+// Q6_K 8192 rows 64 tokens 34.7 | 31.2; and by the lines, Q4_K, 6144 rows, 36 tokens: K = 4096 23.9 | 22.8, K = 3840 22.7 | 25.2
+struct x_cost { int start64, step64, extra, start[3], near_half[3], other[3]; };      // extra: what the few-token kernel's launch takes more, whatever its rounds
+static int x_few_tiles(int type, int nrows_pad, int nb, int T) {
+    static const x_cost costs[3] = { { 3010, 1300, 1150, { 1790, 2140, 2400 }, { 410, 530, 590 }, { 420, 640, 600 } },         // Q4_K
+                                     { 3410, 1240, 1800, { 1900, 2180, 2600 }, { 416, 520, 580 }, { 420, 563, 590 } },         // Q5_K
+                                     { 3590, 1815, 1150, { 2040, 2400, 2740 }, { 680, 710, 750 }, { 685, 740, 783 } } };       // Q6_K
     if (T > 64) return 0;
-    const long c16 = T <= 32 ? 480 : T <= 48 ? 700 : 800;
-    if (((nrows_pad + 15) / 16 + 255) / 256 * c16 >= ((long) x_row_blocks(nrows_pad) + 255) / 256 * 1500) return 0;
-    return T <= 32 ? 2 : T <= 48 ? 3 : 4;
+    const x_cost & c = costs[type == BAMD_Q6_K ? 2 : type == BAMD_Q5_K ? 1 : 0];
+    const int i = T <= 32 ? 0 : T <= 48 ? 1 : 2, line = (int) (BAMD_BLOB16_BYTES(nb) & 127);
+    const long few = c.extra + (long) ((nrows_pad + 15) / 16 + 255) / 256 * (c.start[i] + (long) (line >= 48 && line <= 80 ? c.near_half : c.other)[i] * nb);
+    return few < ((long) x_row_blocks(nrows_pad) + 255) / 256 * (c.start64 + (long) c.step64 * nb) ? i + 2 : 0;
 }
-size_t bamd_prefill_route(int type, int nrows_pad, int, int T, int * few_tiles, size_t * most) {
-    *few_tiles = x_few_tiles(nrows_pad, T); *most = x_max_lds();
+size_t bamd_prefill_route(int type, int nrows_pad, int K, int T, int * few_tiles, size_t * most) {
+    *few_tiles = x_few_tiles(type, nrows_pad, K >> 8, T); *most = x_max_lds();
     return *few_tiles ? few_lds(type, *few_tiles) : type == BAMD_Q6_K ? X_LDS_BYTES : X3_LDS_BYTES;
 }
 int bamd_launch_matmul_mfma2(const void * w_stream, const void * aux, int type, int nrows, int nrows_pad, int K, const void * blob16, int T, float * out, const float * res,
@@ -838,7 +846,7 @@ int bamd_launch_matmul_mfma2(const void * w_stream, const void * aux, int type, 
         if (epi == BAMD_EPI_ADD)           hipLaunchKernelGGL((KERNEL<BAMD_EPI_ADD __VA_ARGS__>),      grid3, dim3(1024), X3_LDS_BYTES, s, a); \
         else if (epi == BAMD_EPI_SILU_MUL) hipLaunchKernelGGL((KERNEL<BAMD_EPI_SILU_MUL __VA_ARGS__>), grid3, dim3(1024), X3_LDS_BYTES, s, a); \
         else                               hipLaunchKernelGGL((KERNEL<BAMD_EPI_STORE __VA_ARGS__>),    grid3, dim3(1024), X3_LDS_BYTES, s, a); } while (0)
-    if (const int ntt = x_few_tiles(nrows_pad, T)) {
+    if (const int ntt = x_few_tiles(type, nrows_pad, K >> 8, T)) {
 #define XF_LAUNCH(TYPE_, NTT_) do { const dim3 gf((T + 16 * NTT_ - 1) / (16 * NTT_), (nrows_pad + 15) / 16); \
         if (epi == BAMD_EPI_ADD)           hipLaunchKernelGGL((matmul_few_kernel<TYPE_, BAMD_EPI_ADD, NTT_>),      gf, dim3(768), few_lds(TYPE_, NTT_), s, a); \
         else if (epi == BAMD_EPI_SILU_MUL) hipLaunchKernelGGL((matmul_few_kernel<TYPE_, BAMD_EPI_SILU_MUL, NTT_>), gf, dim3(768), few_lds(TYPE_, NTT_), s, a); \

@@ -42,3 +42,20 @@ def test_the_launch_probe_covers_every_prompt_product(L):
                 assert lds <= most <= 160 * 1024
                 seen.add((tiles, lds))
     assert {s[0] for s in seen} == {0, 2, 3, 4} and max(s[1] for s in seen) == 159328 == most
+
+
+# type, K, rows, tokens, measured us of 64-row blocks and of the few-token kernel
+@pytest.mark.parametrize("t,k,rows,T,wide,few", [
+    (Q4_K, 4096, 4096, 37, 23.8, 12.3), (Q4_K, 4096, 8192, 32, 24.1, 18.4), (Q4_K, 4096, 8192, 48, 24.0, 22.7), (Q4_K, 4096, 8192, 64, 24.1, 25.5), (Q4_K, 3840, 6144, 36, 22.7, 25.2), (Q4_K, 4096, 6144, 36, 23.9, 22.8),
+    (Q4_K, 2048, 4352, 40, 13.8, 15.9), (Q4_K, 1536, 5120, 32, 11.2, 10.4), (Q4_K, 1536, 6144, 40, 11.4, 13.5), (Q4_K, 1024, 8192, 48, 8.9, 11.4), (Q4_K, 8960, 6144, 36, 48.8, 43.1), (Q4_K, 4096, 12288, 32, 25.2, 27.9),
+    (Q4_K, 2048, 24576, 16, 27.1, 33.5), (Q5_K, 3072, 6144, 64, 17.6, 20.5), (Q5_K, 2048, 6144, 48, 13.0, 14.9), (Q5_K, 13312, 6144, 48, 68.7, 59.7), (Q5_K, 14336, 4352, 32, 69.6, 52.5), (Q5_K, 4096, 14336, 48, 26.0, 44.8),
+    (Q6_K, 4096, 8192, 64, 34.7, 31.2), (Q6_K, 2048, 4352, 32, 18.2, 16.8), (Q6_K, 1024, 8192, 64, 12.1, 13.6), (Q6_K, 8192, 6144, 40, 62.2, 53.8), (Q6_K, 14336, 14336, 40, 108.0, 175.3), (Q6_K, 4096, 12288, 32, 33.9, 41.9)])
+def test_few_token_products_take_the_faster_kernel(L, t, k, rows, T, wide, few):
+    assert (prefill(L, t, rows, k, T)[0] > 0) == (few < wide)
+
+
+def test_few_token_kernel_covers_its_tokens(L):
+    for t in (Q4_K, Q5_K, Q6_K):
+        for T in range(1, 130):
+            tiles = prefill(L, t, 1024, 4096, T)[0]
+            assert tiles == (0 if T > 64 else 2 if T <= 32 else 3 if T <= 48 else 4)
