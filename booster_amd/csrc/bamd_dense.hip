@@ -165,35 +165,44 @@ static int tile_go(const bamd_dense & w, const void * x, int ldx, int rows, void
 // The tile whose rounds over the 256 CUs end first.  Measured per block of 32 columns, all CUs busy (ns): 256 x 256 700, 128 x 256 450, 128 x 128 250, all three one block per CU,
 // so that a round started is a round paid; 64 x 128 190 and 64 x 64 160 share a CU with two to four others and never take less than 250 and 160.  Where even the small tiles leave
 // CUs idle and the reader of the result can add planes, K is halved: two planes cost their bytes twice (at 4 TB/s) and blocks their
-// start and end once more (4 us).  131 x 2048 x 8192: 38 -> 22 us, 412 x 4096 x 8192: 85 -> 39; four shares were no faster (24 and 43 us)
+// start and end once more (4 us).  131 x 2048 x 8192: 38 -> 22 us, 412 x 4096 x 8192: 85 -> 39; four shares were no faster (24 and 43 us).  Halves of 64 x 64 tiles that put a second block on
+// a CU take 300 where each half is longer than 2048 columns: 131 x 4096 x 14336 whole 70 us, in halves of such tiles 74, of 128 x 128 58 (8192 columns: 41, 43, 36); at K = 4096 they are
+// level or ahead (131 x 3072: 24.0 and 24.4, 300 x 2048: 24.4 and 19.9).  Of 187 halved sizes (K 1056 to 14336) nine are slower than whole by more than 2 %, at most 7 % (17 and 11 % without).
+// 32-bit: bound by the f32 matrix instructions: small tiles, several blocks per CU.  Halves take half as long up to 128 tiles (K = 4096: 76 -> 41 us), from there to 192 they share CUs and
+// take 0 to 8 % less (K = 1024: 24.4 and 24.7, K = 4096: 76.9 -> 72.5)
+enum { TILE_256_256 = 0, TILE_128_256 = 1, TILE_128_128 = 2, TILE_64_128 = 3, TILE_64_64 = 4, TILE_64_64_DEEP = 5 };
+static int pick_tile(int act, const bamd_dense & w, int rows, int most, int & share) {
+    share = 1;
+    if (act == BAMD_ACT_F32) {
+        if (most > 1 && (long) ((rows + 63) / 64) * ((w.row_tiles + 3) / 4) <= 192 && w.k_tiles >= 32) share = 2;
+        return TILE_64_64;
+    }
+    auto tiles = [&](int tm, int tn) { return (long) ((rows + tm - 1) / tm) * ((w.row_tiles * 16 + tn - 1) / tn); };
+    long best = 0; int pick = 0;
+    for (int p = 1; p <= most && p <= 2 && (p == 1 || w.k_tiles >= 32); ++p) {
+        auto rounds = [&](int tm, int tn, long cost) { return (tiles(tm, tn) * p + 255) / 256 * cost; };
+        const long pairs = p == 2 && w.k_tiles > 128 && tiles(64, 64) * 2 > 256 ? 300 : 160;
+        const long t[5] = { rounds(256, 256, 700), rounds(128, 256, 450), rounds(128, 128, 250), std::max(tiles(64, 128) * p * 190 / 256, 250l), std::max(tiles(64, 64) * p * 160 / 256, pairs) };
+        const int i = (int) (std::min_element(t, t + 5) - t);
+        const long ns = t[i] * ((w.k_tiles + p - 1) / p) + (p > 1 ? 4000 + (long) p * rows * w.row_tiles * 16 / 500 : 0);
+        if (p == 1 || ns < best) { best = ns; pick = i; share = p; }
+    }
+    // one tile per CU at most: twice the stages hide more of the memory's latency (131 x 2048 x 8192: 49 -> 38 us); with more, blocks hide each other's
+    return pick == TILE_64_64 && tiles(64, 64) * share <= 256 ? TILE_64_64_DEEP : pick;
+}
 template <typename T, int OUT>
 static int gemm_tiles(const bamd_dense & w, const void * x, int ldx, int rows, void * out, int ldo, float limit, hipStream_t s, int * parts = nullptr) {
-    if constexpr (sizeof(T) == 4) {                               // bound by the f32 matrix instructions: small tiles, several blocks per CU
-        const long tiles = (long) ((rows + 63) / 64) * ((w.row_tiles + 3) / 4);
-        const int share = OUT == BAMD_OUT_F32 && parts && *parts > 1 && tiles <= 192 && w.k_tiles >= 32 ? 2 : 1;
-        if (parts) *parts = share;
-        return tile_go<T, 64, 64, 2, 2, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
-    } else {
-        auto tiles = [&](int tm, int tn) { return (long) ((rows + tm - 1) / tm) * ((w.row_tiles * 16 + tn - 1) / tn); };
-        long best = 0; int pick = 0, share = 1;
-        for (int p = 1; p <= (OUT == BAMD_OUT_F32 && parts ? *parts : 1) && p <= 2 && (p == 1 || w.k_tiles >= 32); ++p) {
-            auto rounds = [&](int tm, int tn, long cost) { return (tiles(tm, tn) * p + 255) / 256 * cost; };
-            const long t[5] = { rounds(256, 256, 700), rounds(128, 256, 450), rounds(128, 128, 250), std::max(tiles(64, 128) * p * 190 / 256, 250l), std::max(tiles(64, 64) * p * 160 / 256, 160l) };
-            const int i = (int) (std::min_element(t, t + 5) - t);
-            const long ns = t[i] * ((w.k_tiles + p - 1) / p) + (p > 1 ? 4000 + (long) p * rows * w.row_tiles * 16 / 500 : 0);
-            if (p == 1 || ns < best) { best = ns; pick = i; share = p; }
-        }
-        if (parts) *parts = share;
-        switch (pick) {
-            case 0: return tile_go<T, 256, 256, 2, 4, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
-            case 1: return tile_go<T, 128, 256, 2, 4, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
-            case 2: return tile_go<T, 128, 128, 2, 4, 8, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
-            case 3: return tile_go<T, 64, 128, 2, 2, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
-        }
-        // one tile per CU at most: twice the stages hide more of the memory's latency (131 x 2048 x 8192: 49 -> 38 us); with more, blocks hide each other's
-        if (tiles(64, 64) * share <= 256) return tile_go<T, 64, 64, 2, 2, 8, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
-        return tile_go<T, 64, 64, 2, 2, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
+    int share;
+    const int tile = pick_tile(sizeof(T) == 4 ? BAMD_ACT_F32 : BAMD_ACT_BF16, w, rows, OUT == BAMD_OUT_F32 && parts ? *parts : 1, share);
+    if (parts) *parts = share;
+    if constexpr (sizeof(T) == 2) switch (tile) {
+        case TILE_256_256: return tile_go<T, 256, 256, 2, 4, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
+        case TILE_128_256: return tile_go<T, 128, 256, 2, 4, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
+        case TILE_128_128: return tile_go<T, 128, 128, 2, 4, 8, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
+        case TILE_64_128: return tile_go<T, 64, 128, 2, 2, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
+        case TILE_64_64_DEEP: return tile_go<T, 64, 64, 2, 2, 8, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
     }
+    return tile_go<T, 64, 64, 2, 2, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
 }
 // f32 rows are stored four matrix rows at a time: ldo % 4 == 0; x rows start on 16 bytes and hold k_tiles * 32 columns
 template <typename T>
@@ -396,12 +405,17 @@ static void mv_one(const bamd_dense & w, const bamd_batch_dev & b, const bamd_pr
     else mv_go<T, 1, 8, PRE>(w, b, p, x, ldx, rows, out, ldo, s);
 }
 // Two shares of K where a matrix has too few row tiles for the CUs and enough columns that halves are still worth a block; a prologue that writes state stays whole
-static int few_parts(const bamd_dense & w, int pre, const int * parts) {
-    return parts && *parts > 1 && w.row_tiles <= 128 && w.k_tiles >= 64 && pre != BAMD_PRE_RESIDUAL && pre != BAMD_PRE_FINAL && pre != BAMD_PRE_LAYER ? 2 : 1;
+static int few_parts(int, const bamd_dense & w, int pre, int most) {
+    return most > 1 && w.row_tiles <= 128 && w.k_tiles >= 64 && pre != BAMD_PRE_RESIDUAL && pre != BAMD_PRE_FINAL && pre != BAMD_PRE_LAYER ? 2 : 1;
+}
+int bamd_dense_route(int act, const bamd_dense & w, int rows, int pre, int most, int & share) {
+    if (pre < 0) return pick_tile(act, w, rows, most, share);
+    share = few_parts(act, w, pre, most);
+    return -1;
 }
 template <typename T>
 static int mv_pick(const bamd_dense & w, int pre, const bamd_batch_dev & b, const bamd_pre_args & p, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s, int * parts) {
-    const int n = few_parts(w, pre, parts);
+    const int n = few_parts(sizeof(T) == 4 ? BAMD_ACT_F32 : BAMD_ACT_BF16, w, pre, parts ? *parts : 1);
     if (parts) *parts = n;
     if (pre != BAMD_PRE_ROWS) {
         if (rows != 1 || bamd_dense_mv_lds(sizeof(T) == 4 ? BAMD_ACT_F32 : BAMD_ACT_BF16, w.k_tiles * 32) > BAMD_MV_LDS) return 1;

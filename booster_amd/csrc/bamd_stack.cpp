@@ -1101,6 +1101,12 @@ SafeTensor bf16_tensor(const uint16_t * p, std::vector<int64_t> shape) { SafeTen
 #define BAMD_OP extern "C" __attribute__((visibility("default"))) int
 
 BAMD_OP bamd_op_norm_threads(int n, int rows) { return bamd_norm_threads(n, rows); }
+BAMD_OP bamd_op_dense_route(int act, int nrows, int k, int rows, int pre, int most, int * shares) {
+    if (nrows < 1 || k < 1 || rows < 1 || !shares) { fail("bamd_op_dense_route: bad arguments"); return -2; }
+    bamd_dense d;
+    d.rows = nrows; d.K = up(k, 32); d.row_tiles = up(nrows, 16) / 16; d.k_tiles = d.K / 32;
+    return bamd_dense_route(act, d, rows, pre, most, *shares);
+}
 BAMD_OP bamd_op_dense(int act, const uint16_t * w, int nrows, int k, const float * x, int rows, int impl, float * y) {
     OpScratch s; bamd_dense d; void * dx; float * dy = nullptr;
     if (!w || !x || !y || nrows < 1 || k < 1 || rows < 1 || s.init(act)) return fail("bamd_op_dense: bad arguments");

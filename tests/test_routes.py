@@ -59,3 +59,22 @@ def test_few_token_kernel_covers_its_tokens(L):
         for T in range(1, 130):
             tiles = prefill(L, t, 1024, 4096, T)[0]
             assert tiles == (0 if T > 64 else 2 if T <= 32 else 3 if T <= 48 else 4)
+
+
+BF16, F32 = 0, 1
+T256x256, T128x256, T128x128, T64x128, T64x64, T64x64_DEEP = range(6)
+
+
+def dense(L, act, n, k, rows, pre=-1, most=2):
+    share = C.c_int(0)
+    tile = L.bamd_op_dense_route(act, n, k, rows, pre, most, C.byref(share))
+    return tile, share.value
+
+
+# activation rows, matrix rows, K, the shares of the faster form: where a second 64 x 64 block per CU would make halves slower than the whole, and around it
+@pytest.mark.parametrize("rows,n,k,want", [(131, 4096, 14336, (T128x128, 2)), (131, 3072, 8192, (T128x128, 2)), (300, 2048, 8192, (T128x128, 2)), (192, 4096, 8192, (T128x128, 2)), (65, 6144, 8192, (T128x128, 2)),
+                                           (300, 2048, 4096, (T64x64, 2)), (640, 1024, 4096, (T64x64, 2)), (131, 2048, 8192, (T64x64_DEEP, 2)), (412, 4096, 8192, (T128x128, 2)), (131, 8192, 2048, (T64x64, 1))])
+def test_many_rows_are_halved_where_that_is_faster(L, rows, n, k, want):
+    assert dense(L, BF16, n, k, rows) == want
+    assert dense(L, BF16, n, k, rows, most=1)[1] == 1
+
