@@ -63,6 +63,7 @@ def test_few_token_kernel_covers_its_tokens(L):
 
 BF16, F32 = 0, 1
 T256x256, T128x256, T128x128, T64x128, T64x64, T64x64_DEEP = range(6)
+ROWS, POLY, GROUP, GLU = 0, 2, 3, 5
 
 
 def dense(L, act, n, k, rows, pre=-1, most=2):
@@ -78,3 +79,14 @@ def test_many_rows_are_halved_where_that_is_faster(L, rows, n, k, want):
     assert dense(L, BF16, n, k, rows) == want
     assert dense(L, BF16, n, k, rows, most=1)[1] == 1
 
+
+def test_few_rows_are_halved_where_that_is_faster(L):
+    share = lambda act, n, k, pre, rows=1: dense(L, act, n, k, rows, pre)[1]
+    for pre in (POLY, GROUP, GLU):
+        # measured, 2048 and 1536 outputs: slower in halves up to K = 4096, faster from 5632; 1024 and 512 outputs: never slower
+        assert [share(BF16, n, k, pre) for n in (2048, 1536) for k in (2048, 4096, 5632, 14336)] == [1, 1, 2, 2] * 2
+        assert [share(BF16, n, k, pre) for n in (1024, 512) for k in (2048, 4096, 5632, 14336)] == [2] * 8
+        assert [share(F32, 2048, k, pre) for k in (2016, 2048, 14336)] == [1, 2, 2]
+    for act in (BF16, F32):
+        assert [share(act, n, k, ROWS, rows) for rows in (1, 64) for n, k in ((2048, 2048), (2049, 2048), (2048, 2016))] == [2, 1, 1] * 2
+    assert [share(BF16, 512, 4096, pre) for pre in (1, 4, 6)] == [1, 1, 1]           # prologues that write state
