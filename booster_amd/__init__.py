@@ -78,6 +78,7 @@ def lib():
         L.bamd_op_poly_norm.argtypes = [ci, vp, vp, cf, ci, ci, vp]
         L.bamd_op_group_norm.argtypes = [ci, vp, vp, ci, cf, ci, ci, vp]
         L.bamd_op_ssm.argtypes = [vp, ci, ci, ci, ci, ci, ci, ci, vp, vp, vp, vp, vp, vp, vp, vp]
+        L.bamd_op_dense_glu.argtypes = [ci, vp, vp, ci, ci, vp, ci, cf, vp]; L.bamd_op_dense_route.argtypes = [ci, ci, ci, ci, ci, ci, vp]
         L.bamd_op_latent_attention.argtypes = [ci, vp, vp, vp, ci, vp, ci, ci, ci, ci, ci, cf, cf, vp, vp, vp, vp, ci, vp]
         L.bamd_op_layer_rows.argtypes = [ci, vp, vp, vp, vp, cf, ci, ci, vp, vp]
         L.bamd_op_clamped_glu.argtypes = [ci, vp, vp, cf, ci, ci, vp]
@@ -370,6 +371,23 @@ def op_dense(w, x, dtype, impl=0):
     y = np.zeros((x.shape[0], w.shape[0]), np.float32)
     _chk(lib().bamd_op_dense(_act(dtype), _p(w), w.shape[0], w.shape[1], _p(x), x.shape[0], impl, _p(y)))
     return y
+
+
+def op_dense_glu(gate, up, x, limit, dtype):
+    """the clamped gated unit of x . gate^T and x . up^T, written by the many-row product"""
+    gate, up, x = np.ascontiguousarray(gate, np.uint16), np.ascontiguousarray(up, np.uint16), _f32(x)
+    y = np.zeros((x.shape[0], gate.shape[0]), np.float32)
+    _chk(lib().bamd_op_dense_glu(_act(dtype), _p(gate), _p(up), gate.shape[0], gate.shape[1], _p(x), x.shape[0], limit, _p(y)))
+    return y
+
+
+def op_dense_route(n, k, rows, dtype, pre=-1, most=2):
+    """(tile, shares of K) that a product takes, no device needed; pre -1: the many-row kernel, else the few-row ones (tile -1)"""
+    shares = C.c_int(0)
+    tile = lib().bamd_op_dense_route(_act(dtype), n, k, rows, pre, most, C.byref(shares))
+    if tile < -1:
+        _chk(1)
+    return tile, shares.value
 
 
 def op_residual_rows(x, y, g, eps, mu, prev, pos0, dtype):

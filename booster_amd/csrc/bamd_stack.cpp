@@ -1135,6 +1135,19 @@ BAMD_OP bamd_op_dense(int act, const uint16_t * w, int nrows, int k, const float
     for (int n = 0; n < nrows; ++n) for (int r = 0; r < rows; ++r) y[(size_t) r * nrows + n] = tr[(size_t) n * rows + r];
     return 0;
 }
+BAMD_OP bamd_op_dense_glu(int act, const uint16_t * gate, const uint16_t * upw, int F, int k, const float * x, int rows, float limit, float * y) {
+    OpScratch s; bamd_dense d; void * dx; float * dy = nullptr;
+    if (!gate || !upw || !x || !y || F < 1 || k < 1 || rows < 1 || s.init(act)) return fail("bamd_op_dense_glu: bad arguments");
+    const int ldo = up(F, 32);
+    const SafeTensor tg = bf16_tensor(gate, { F, k }), tu = bf16_tensor(upw, { F, k });
+    std::vector<int32_t> at = Loader::steps(F, k); at.resize((size_t) ldo, -1);
+    if (s.l.alloc(d, 2 * ldo, k) || s.act_rows(x, rows, k, d.K, &dx) || s.alloc((void **) &dy, (size_t) rows * ldo * 4)) return 1;
+    uint16_t * w = const_cast<uint16_t *>(d.w);
+    if (s.l.pack(&tg, at, Loader::steps(k, 1), w, 2) || s.l.pack(&tu, at, Loader::steps(k, 1), w + (size_t) 16 * d.K, 2)) return 1;
+    if (bamd_launch_dense_gemm(act, d, dx, d.K, rows, dy, ldo, BAMD_OUT_GLU, s.l.s, limit)) return fail("bamd_op_dense_glu: unsupported shape");
+    HIPC(hipGetLastError());
+    return s.rows_back(dy, rows, F, ldo, y, act == BAMD_ACT_F32);
+}
 BAMD_OP bamd_op_residual_rows(int act, const float * x, const float * y, float g, float eps, const float * mu, float * prev, int pos0, int rows, int E, float * xo, float * h) {
     OpScratch s; bamd_batch_dev b; bamd_residual_args a; memset((void *) &a, 0, sizeof a);
     if (!x || !xo || !h || rows < 1 || E < 1 || (mu && !prev) || s.init(act) || s.one_entry(rows, pos0, b)) return fail("bamd_op_residual_rows: bad arguments");

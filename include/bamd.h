@@ -231,6 +231,8 @@ int bamd_op_attention(const float * q, const float * k, const float * v, uint16_
 /* y[rows][nrows] = x[rows][k] . w^T; impl 0: many-row kernel, 1: few-row kernel (rows <= 64), 2: many-row kernel with an activation-typed result, 3: the same, transposed,
  * 4 / 5: as 0 / 1 with K halved where that is faster, the halves added */
 int bamd_op_dense(int act, const uint16_t * w, int nrows, int k, const float * x, int rows, int impl, float * y);
+/* y[rows][F] = the clamped gated unit of x . gate^T and x . up^T (bfloat16 [F][k]), by the many-row kernel that writes it itself, in the activation type */
+int bamd_op_dense_glu(int act, const uint16_t * gate, const uint16_t * up, int F, int k, const float * x, int rows, float limit, float * y);
 /* xo = x + rms_norm(y) * g (y NULL: x), h = xo + (xo of the row in front - xo) * mu (mu NULL: xo); prev [E]: the row in front of the first (used when pos0 > 0), replaced by the last */
 int bamd_op_residual_rows(int act, const float * x, const float * y, float g, float eps, const float * mu, float * prev, int pos0, int rows, int E, float * xo, float * h);
 int bamd_op_poly_norm(int act, const float * z, const float * coef, float eps, int rows, int F, float * out);

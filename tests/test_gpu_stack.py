@@ -54,10 +54,14 @@ def test_dense(bamd, dtype, n, k, rows):
                 assert np.abs(bamd.op_dense(w, x, dtype, impl) - want).max() < 8e-6 * scale
 
 
+TILES = {("bfloat16", 8170, 2045): 0, ("bfloat16", 8170, 1000): 1, ("bfloat16", 4090, 1000): 2, ("bfloat16", 4090, 1100): 3, ("bfloat16", 8190, 131): 4, ("bfloat16", 2047, 131): 5, ("float32", 2047, 131): 4}
+
+
 # one size per tile of the many-row product (256 x 256, 128 x 256, 128 x 128, 64 x 128, 64 x 64 with four and with eight stages; 32-bit: 64 x 64), ragged in every dimension, fewer and more column blocks than stages
 @pytest.mark.parametrize("dtype,n,rows", [("bfloat16", 8170, 2045), ("bfloat16", 8170, 1000), ("bfloat16", 4090, 1000), ("bfloat16", 4090, 1100), ("bfloat16", 8190, 131), ("bfloat16", 2047, 131), ("float32", 2047, 131)])
 @pytest.mark.parametrize("k", [1, 70, 300])
 def test_dense_tiles(bamd, dtype, n, rows, k):
+    assert bamd.op_dense_route(n, k, rows, dtype, most=1) == (TILES[dtype, n, rows], 1)
     r = np.random.default_rng(n + k + rows)
     w = so.f32_to_bf16(r.standard_normal((n, k)).astype(np.float32))
     x = r.standard_normal((rows, k)).astype(np.float32)
@@ -67,6 +71,25 @@ def test_dense_tiles(bamd, dtype, n, rows, k):
     for impl, tol in ((0, 8e-6), (2, 2.0 ** -8), (3, 2.0 ** -8)):                    # k <= 300 roundings of 2^-24 | the result rounded to bfloat16 (2^-9 of it)
         e = np.abs(bamd.op_dense(w, x, dtype, impl) - want)
         assert (e <= tol * (scale if impl == 0 else np.abs(want) + 0.01 * scale)).all(), impl
+
+
+# the same tiles where they write the clamped gated unit of their gate and up tiles in turn: widths that end inside a pair of tiles, on its edge and inside a group of four
+@pytest.mark.parametrize("dtype,F,rows,tile", [("bfloat16", 4085, 2045, 0), ("bfloat16", 4085, 1000, 1), ("bfloat16", 2032, 1000, 2), ("bfloat16", 2046, 1100, 3), ("bfloat16", 4090, 131, 4), ("bfloat16", 1001, 131, 5), ("bfloat16", 35, 70, 5),
+                                                ("float32", 1001, 131, 4)])
+@pytest.mark.parametrize("k", [1, 70, 300])
+def test_dense_gated_tiles(bamd, dtype, F, rows, tile, k):
+    assert bamd.op_dense_route(2 * ((F + 31) // 32 * 32), k, rows, dtype, most=1) == (tile, 1)
+    r = np.random.default_rng(F + k + rows)
+    gate, up = (so.f32_to_bf16(r.standard_normal((F, k)).astype(np.float32)) for _ in range(2))
+    x, limit = r.standard_normal((rows, k)).astype(np.float32), 7.0
+    x = x if dtype == "float32" else so.round_bf16(x)
+    both = [x.astype(np.float64) @ so.bf16_to_f32(w).T.astype(np.float64) for w in (gate, up)]
+    scale = [np.sqrt(np.abs(x).astype(np.float64) ** 2 @ np.abs(so.bf16_to_f32(w)).T.astype(np.float64) ** 2) for w in (gate, up)]
+    g, u = np.minimum(both[0], limit), np.clip(both[1], -limit, limit)
+    want = g * so.sigmoid(1.702 * g) * (u + 1)
+    # errors of the sums (test_dense_tiles) through slopes of at most 1.13 |u + 1| and |g sigmoid| <= limit, and the result's own rounding
+    e = np.abs(bamd.op_dense_glu(gate, up, x, limit, dtype) - want)
+    assert (e <= 8e-6 * (1.13 * (limit + 1) * scale[0] + limit * scale[1]) + (1e-5 if dtype == "float32" else 2.0 ** -8) * np.abs(want) + 1e-30).all()
 
 
 # one, two and three row tiles per step with a remainder, every group of rows and its edges, fewer column blocks than waves and more than a ring holds
@@ -85,6 +108,8 @@ def test_dense_few_rows(bamd, n, rows, k):
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("n,k,rows", [(500, 2100, 131), (77, 2049, 300), (500, 1000, 70), (500, 2100, 1), (2048, 2080, 6), (2049, 2080, 6), (77, 2049, 20), (500, 2100, 45), (500, 2000, 6)])
 def test_dense_halves(bamd, dtype, n, k, rows):
+    halved = 2 if (n, k, rows) not in ((500, 1000, 70), (2049, 2080, 6), (500, 2000, 6)) else 1
+    assert bamd.op_dense_route(n, k, rows, dtype, pre=-1 if rows > 64 else 0)[1] == (halved if k != 1000 or dtype == "bfloat16" else 2)
     r = np.random.default_rng(n + k + rows)
     w = so.f32_to_bf16(r.standard_normal((n, k)).astype(np.float32))
     x = so.round_bf16(r.standard_normal((rows, k)).astype(np.float32))
@@ -92,6 +117,19 @@ def test_dense_halves(bamd, dtype, n, k, rows):
     scale = np.sqrt(np.abs(x).astype(np.float64) ** 2 @ np.abs(so.bf16_to_f32(w)).T.astype(np.float64) ** 2)
     for impl in (4,) if rows > 64 else (4, 5):
         assert (np.abs(bamd.op_dense(w, x, dtype, impl) - want) <= 1e-5 * scale).all(), impl
+
+
+# and of the larger tiles, whose halves need larger matrices
+@pytest.mark.parametrize("n,k,rows,tile", [(4247, 8200, 65, 2), (8247, 4130, 131, 3), (2045, 4090, 300, 4), (8247, 8200, 513, 0)])
+def test_dense_halves_of_large_tiles(bamd, n, k, rows, tile):
+    assert bamd.op_dense_route(n, k, rows, "bfloat16") == (tile, 2)
+    r = np.random.default_rng(n + k + rows)
+    w = so.f32_to_bf16(r.standard_normal((n, k), np.float32))
+    x = so.round_bf16(r.standard_normal((rows, k), np.float32))
+    wf = so.bf16_to_f32(w)
+    want = x.astype(np.float64) @ wf.T.astype(np.float64)
+    scale = np.sqrt((x * x) @ (wf * wf).T)
+    assert (np.abs(bamd.op_dense(w, x, "bfloat16", 4) - want) <= 1e-5 * scale).all()               # as above: sqrt(k) <= 91 roundings of 2^-24 in a row, twice over
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
