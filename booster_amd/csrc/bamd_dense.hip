@@ -107,7 +107,7 @@ __global__ void __launch_bounds__(64 * WM * WN) dense_tile_kernel(bamd_dense w, 
         else { xf[p][i].a = *(const bamd_v4 *) at; xf[p][i].b = *(const bamd_v4 *) (at + xb2); }
     };
     auto read_w = [&](int k, int p, int j) { wr[p][j] = *(const bamd_u4 *) (wb + (k & (NS - 1)) * STAGE + j * 1024); };
-    auto wait = [&] {                                             // all but the last stage's copies of this wave have landed; then every wave's
+    auto wait = [&] {                                             // in block k: leaves NS - 3 stages of this wave's copies under way, so that stage k + 1 is whole; then every wave's
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"((NS - 3) * PER) : "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");

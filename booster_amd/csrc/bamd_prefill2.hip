@@ -544,12 +544,12 @@ __global__ void __launch_bounds__(1024) matmul_mfma3_q4k_kernel(bamd_mma2_args a
 
 // ==== few tokens ==============================================================================================================================
 // A prompt of up to 64 tokens leaves the kernels above without work for the chip: 64-row blocks make 64 of them at 4096 rows, and each walks all of K behind a barrier per
-// super-block that waits for everything it has requested (1.5 us per super-block: 24 us at K = 4096, 84 and, Q6_K, 105 us at K = 14336, whatever the tokens).  Here a block is ONE
+// super-block that waits for everything it has requested (1.5 us per super-block: 25 us at K = 4096, 77 and, Q6_K, 105 us at K = 14336, whatever the tokens).  Here a block is ONE
 // row tile (16 rows) x up to 16 NTT tokens on twelve waves, one of each kind per SIMD: wave tt < 4 takes token tile tt, four build a quarter of the next super-block's fragments
 // each, four copy (all of it one after the other on four waves: 1230 ns a super-block at 37 tokens; copies spread over consumers and builders: 930 — a copy holds its wave until
 // the vector memory path takes it); the arithmetic, its order and the layouts are those above.  Everything a step reads travels global -> LDS by DMA — token records two
 // super-blocks ahead, the row tile's quants, scales and headers four — and the wait at the end of a step leaves what was issued in it (and the weights issued in the one before)
-// in flight, so that a step is not as long as the memory's latency.  37 tokens, 4096 rows: K = 4096 24.0 -> 12.7 us, K = 14336 84 -> 38 us (Q6_K 105 -> 46 us); the copies of
+// in flight, so that a step is not as long as the memory's latency.  37 tokens, 4096 rows: K = 4096 25.0 -> 12.9 us, K = 14336 77 -> 38 us (Q6_K 105 -> 46 us); the copies of
 // the token records, the same to every block, are 24 us of the 38.
 //   W slot of a super-block   Q4_K / Q5_K: 2 x 1 KiB quants of the two record groups | 1 KiB builder operands | 1 KiB consumer header | Q5_K: 2 x 256 B fifth bits
 //                             Q6_K: 2 x 1 KiB low bits | 2 x 512 B high bits | 2 x 1 KiB builder operands of the e-halves | 64 B of d
