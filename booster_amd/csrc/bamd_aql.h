@@ -1,4 +1,4 @@
-// bamd_aql.h — a decode step replayed from the library's OWN AQL queue instead of a hipGraph (round 6).
+// bamd_aql.h — a decode step replayed from the library's OWN AQL queue instead of a hipGraph.
 //
 // Why: between two dependent launches the HIP runtime (stream or graph alike) puts agent-scope acquire / release fences — an L2 write-back at the end of
 // one kernel, an L1 / L2 / scalar-cache invalidate at the start of the next.  tools/aql_probe.hip measured that pair at 0.38 us per launch on a mat-vec

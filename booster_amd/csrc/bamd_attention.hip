@@ -10,8 +10,8 @@
 template <int GQ, int LG, bool SH, int NT = BAMD_QK_NT>       // LG = head_dim / 64 = 16-byte groups of a K row per lane; NT = tiles of 64 positions per workgroup in flight together
 // (the launcher picks 2 when the context has no more than two tiles per workgroup: no request for a tile that cannot exist)
 __global__ void __launch_bounds__(512) attn_qk_kernel(bamd_attn_args a) {
-    // Round 6: the launch is a chain of latencies, not bytes — 16 MB of K at 8000 positions are 2.7 us at the HBM rate and the kernel took 7.9.
-    // A wave's loads return in order, so the q / k / RoPE requests that rounds 2-5 issued BEHIND the K prefetch (the prefetch clamp needed the position first)
+    // The launch is a chain of latencies, not bytes — 16 MB of K at 8000 positions are 2.7 us at the HBM rate and the kernel took 7.9.
+    // A wave's loads return in order, so the q / k / RoPE requests that were once issued BEHIND the K prefetch (the prefetch clamp needed the position first)
     // came back behind 64 KB of K rows per CU, and the prologue's barrier stood at 4.7 us.  Now: (1) the small requests go out first — this token's q / k / v pairs
     // and the cos / sin row of the current position, which step_begin_kernel leaves at a FIXED address (a.rope_cur: no dependent load of the position in front of
     // them); (2) the K rows of the first NT tiles right behind, unclamped (rows past the sequence are masked by a select; the cache is finite everywhere);

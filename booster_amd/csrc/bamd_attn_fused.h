@@ -15,8 +15,8 @@
 // flag (MI355X_MICROARCH.md, R2): the wo workgroups of the same launch re-read their granules until every tag is this launch's tag, with no drain,
 // barrier or flag hop on this side.  done_flags then points at the granule array [H * hd].
 // ENV: where the body runs.  AttnEnvWG = a whole 512-thread workgroup (attn_fused_kernel, attn_wo_kernel): thread / wave ids from the hardware,
-// __syncthreads, this token's q / k / v read from the f32 vectors of the argument block.  (Round 4's weight-stream engine ran the same body on eight of its
-// consumer waves through another ENV; the engine was removed in round 6 — profiles/r04_engine_vs_launches.txt — the parameter stays for a role that
+// __syncthreads, this token's q / k / v read from the f32 vectors of the argument block.  (A weight-stream engine ran the same body on eight of its
+// consumer waves through another ENV; the engine is gone — profiles/r04_engine_vs_launches.txt — the parameter stays for a role that
 // takes its inputs from somewhere else.)
 struct AttnEnvWG {
     int tid, wave, nthr;

@@ -87,7 +87,7 @@ struct Job {
     void append(const std::string & piece) {
         if (piece.empty()) return;
         if (!cur_buf || len + piece.size() + 1 > cap) grow(len + piece.size() + 1);
-        // every byte is a RELEASE store (round 6: rounds 3-5 used volatile stores and relied on x86-64's store order): each one is ordered behind the new
+        // every byte is a RELEASE store (volatile stores would rely on x86-64's store order): each one is ordered behind the new
         // terminator and the bytes after it on any host, so a reader that sees byte i also sees a terminator somewhere behind it.  (The reader is
         // C.GoString on a bare char *: its side of the contract cannot be made atomic from here; the reference does not order anything.)
         char * b = cur_buf;
@@ -292,7 +292,7 @@ int sample_janus(Pod & p, float * logits, const std::vector<int> & last_tokens, 
     return janus_draw(p, cand);
 }
 
-// The same sampler with the O(n_vocab) passes on the device (SURVEY 8f-4): the penalties become a short list of per-token factors
+// The same sampler with the O(n_vocab) passes on the device: the penalties become a short list of per-token factors
 // (a token that occurs k times in the window is multiplied k times, in sequence, as the reference's loop does), the x0.5 pass and
 // the ratio test run where the logits are, and only the shortlist comes back.  Whenever the order of the result could depend on the
 // reference's full sort the (already penalised) logits are read back and the host shortlist runs on them: same result either way.
@@ -360,7 +360,7 @@ int sample_janus_device(Pod & p, const std::vector<int> & last_tokens, size_t pr
 // only the first `device_count` entries of the split count; if those are all zero the reference splits by free device memory (equal
 // here: identical GPUs); layer i lives on upper_bound(cumulative normalised splits, i / act), the output layer with fraction (act-1)/act.
 // BAMD_MAX_GPUS = 8: the nine symbols carry four weights (gpu1..gpu4, cpp/bridge.cpp:745-750 -> tensor_split[0..3]); the environment
-// variable BOOSTER_GPUS="w0,w1,...,w7"  replaces them with up to eight — same rule, more devices.
+// variable BOOSTER_GPUS="w0,w1,...,w7" replaces them with up to eight — same rule, more devices.
 #define BAMD_MAX_GPUS 8
 bool plan_stages(int n_layer, const int * gpu, int n_gpu, int device_count, std::vector<std::pair<int, std::pair<int, int>>> & out, std::string & err) {
     if (n_layer < 1) { err = "model has no layers"; return false; }
@@ -578,7 +578,7 @@ static int64_t do_inference_impl(int idx, void * ctx, char * jobID, char * promp
     const std::string job = jobID, text = prompt;
     p.t_p_eval_ms = p.t_eval_ms = 0; p.n_p_eval = p.n_eval = 0; p.eval_open = false;   // llama_reset_timings
     // an evaluation that no sampler call followed (stopInference during the prompt, the n_ctx - 4 exit, an error return) was never waited for: wait on every
-    // way out, close its timing interval and report a give-up of that evaluation (ADVICE r5)
+    // way out, close its timing interval and report a give-up of that evaluation
     struct OpenEval { Pod & p; bool failed = false; void close() { if (p.eval_open) { if (bamd_synchronize(p.stages[0].ctx)) { fprintf(stderr, "doInference: %s\n", bamd_last_error()); failed = true; } pod_eval_done(p); } }
                       ~OpenEval() { close(); } } open_eval{ p };
     p.stop.store(false);

@@ -171,7 +171,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
 }
 
 static const bool g_colaunch = [] { const char * e = getenv("BAMD_COLAUNCH"); return !(e && e[0] == '0'); }();
-static const int g_ring_delay = [] { const char * e = getenv("BAMD_COLAUNCH_DELAY"); return e ? atoi(e) : 12 + 256; }();   // low byte: x ~0.2 us; + 256: s_sleep between polls (A/B on the MI355X, round 3 end: 707 / 708 / 710 / 713-717 / 712 / 705 / 694 tok/s at 6 / 8 / 10 / 12 / 14 / 16 / 20, all + sleep)      // x ~0.2 us before the wo role requests its weights
+static const int g_ring_delay = [] { const char * e = getenv("BAMD_COLAUNCH_DELAY"); return e ? atoi(e) : 12 + 256; }();   // low byte: x ~0.2 us; + 256: s_sleep between polls (A/B on the MI355X: 707 / 708 / 710 / 713-717 / 712 / 705 / 694 tok/s at 6 / 8 / 10 / 12 / 14 / 16 / 20, all + sleep)      // x ~0.2 us before the wo role requests its weights
 
 // 0 = launched; 1 = this shape has no co-launch kernel (the caller issues the two ordinary launches)
 int bamd_launch_attn_wo(const bamd_attn_args & t, int gq, const bamd_mv_args & wo, int n_cu, unsigned long long * gran, int il, uint32_t * err, hipStream_t s) {
@@ -184,7 +184,7 @@ int bamd_launch_attn_wo(const bamd_attn_args & t, int gq, const bamd_mv_args & w
     if (G < 8) return 1;
     if (nb == 16 && nrg / G != 2) return 1;                                                   // two or three row-groups per wo workgroup
     if (nb == 32) {
-        // the 70B width: MEASURED NEUTRAL (round 4: a 10-layer stage 1.267 ms per token co-launched against 1.260 with the two launches; the whole model 110.9
+        // the 70B width: MEASURED NEUTRAL (a 10-layer stage 1.267 ms per token co-launched against 1.260 with the two launches; the whole model 110.9
         // against 115.2 tok/s in one bench.py pairing) — the wo role's 5 - 6 row-groups x 32 records are 190 KB per workgroup, of which only the first
         // batch can be in flight while the attention role works, and the hand-over costs what the boundary did.  BAMD_COLAUNCH70=1 selects it.
         static const bool on70 = [] { const char * e = getenv("BAMD_COLAUNCH70"); return e && e[0] == '1'; }();

@@ -247,7 +247,7 @@ __device__ __forceinline__ double seq_expsum8(const float * vals, int n) {
 // LDS layout of the quantised activations of one mat-vec: q8[nb][64] u32 | S[nb][8] i32 | yd[nb] f32 | (16-byte aligned) red[16] f64
 #ifndef BAMD_CEILING
 #define BAMD_CEILING 0               /* timing-only builds (never shipped): 1 = mat-vec prologues without the Q8_K / RMSNorm statistics, 2 = split-K kernels without the
-                                        barrier + sequential chain replay: what the reference's arithmetic costs per launch (DESIGN 7b, profiles/r05_ceiling.txt) */
+                                        barrier + sequential chain replay: what the reference's arithmetic costs per launch (profiles/r05_ceiling.txt) */
 #endif
 #define BAMD_ACT_RED_OFF(nb) ((((size_t) (nb) * (256 + 32 + 4)) + 15) & ~(size_t) 15)
 template <bool NORM>
@@ -823,7 +823,7 @@ __device__ __forceinline__ void embed_row(const uint8_t * embd, int embd_type, i
 // KV cache, "chain-major" physical order (logically the reference's K [n_ctx][Hkv*hd] f16 and V^T [Hkv*hd][n_ctx] f16,
 // llama.cpp:7845-7875; bamd_op_attention converts at the boundary):
 //   K : inside each head row, element n = 8l + e (lane e, chain step l) is stored at index (l >> 3)*64 + e*8 + (l & 7): the 16-byte group g = l >> 3 of
-//       the eight lanes is ONE 128-byte line, so a wave's load instruction for group g covers whole lines (round 6; rounds 1-5 kept a lane's L = hd/8
+//       the eight lanes is ONE 128-byte line, so a wave's load instruction for group g covers whole lines (the order before kept a lane's L = hd/8
 //       halves contiguous — e*L + l — and every load instruction touched HALF of two lines per position: harmless while the vector L1 caught the second
 //       half, 1.4 us per attention launch once the loads had to bypass it — sc1, "Inter-kernel data" above; profiles/r06_levers.txt)
 //   V^T: inside each row, position p = 64B + 8l + e is stored at index 64B + 8e + l

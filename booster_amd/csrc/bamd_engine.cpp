@@ -36,7 +36,7 @@ static const int g_stage_graph = [] { const char * e = getenv("BAMD_STAGE_GRAPH"
 static const bool g_attn_fused = [] { const char * e = getenv("BAMD_ATTN_FUSED"); return !(e && e[0] == '0'); }();   // default: fused single-launch attention (BAMD_ATTN_FUSED=0: three-kernel path)
 int bamd_fail(const std::string & m) { g_err = m; return 1; }
 static int fail(const std::string & m) { return bamd_fail(m); }
-// BAMD_AQL=0: the device-side greedy loop replays one hipGraph per step on the context's HIP stream (rounds 1-5) instead of AQL packets with fence scope
+// BAMD_AQL=0: the device-side greedy loop replays one hipGraph per step on the context's HIP stream instead of AQL packets with fence scope
 // NONE on the library's own queue (bamd_aql.h).  Same kernels, same bits; BAMD_AQL_VERBOSE=1 says why when the own queue is not used
 static int g_aql = [] { const char * e = getenv("BAMD_AQL"); return (e && e[0] == '0') ? 0 : 1; }();
 extern "C" __attribute__((visibility("default"))) void bamd_set_aql(int on) { g_aql = on ? 1 : 0; }
@@ -497,7 +497,7 @@ static void enqueue_begin(bamd_context * c, int n_forced, int do_embed, hipStrea
 // The tag of a granule hand-over (bamd_colaunch.hip) is (host serial : 12, device step : 12, layer : 8); a word must never already hold the tag a
 // consumer is about to wait for.  The serial runs 1 .. 0xffe (0 is what zero-initialised granules carry, 0xfff is reserved) and every time it wraps ALL granule
 // vectors of the context are overwritten with 0xff bytes — tag 0xffffffff, which no launch produces — in stream order ahead of the launch that reuses serial 1
-// (ADVICE r4: with a bare 12-bit counter a stale granule of 4096 host calls ago carried the awaited tag and a gather passed without waiting).
+// (with a bare 12-bit counter a stale granule of 4096 host calls ago carried the awaited tag and a gather passed without waiting).
 static int next_serial(bamd_context * c, hipStream_t s) {
     if (++c->host_serial > 0xffe) {
         c->host_serial = 1;
@@ -683,8 +683,8 @@ static bool prefill_batch_supported(const bamd_context * c, int pos_hi) {
         if (!ok(ly.wq.type, m->E) || !ok(ly.wk.type, m->E) || !ok(ly.wv.type, m->E) || !ok(ly.wo.type, m->E) || !ok(ly.wg.type, m->E) || !ok(ly.wu.type, m->E) || !ok(ly.wd.type, m->F)) return false;
     return true;
 }
-// prefill side tables of every layer matrix (bamd_prefill2.hip), built at model load (round 6; round 5 built them lazily inside the first batched evaluation — a
-// multi-gigabyte allocation after the contexts existed, and a partial failure mixed kernel generations).  The QKV segments are the ones
+// prefill side tables of every layer matrix (bamd_prefill2.hip), built at model load (built inside the first batched evaluation they would be a
+// multi-gigabyte allocation after the contexts exist, and a partial failure would mix kernels).  The QKV segments are the ones
 // enqueue_prefill_batch forms (equal-typed neighbours of the fused wq | wk | wv stream merge into one matrix).  All or nothing.
 static void build_prefill_aux(bamd_model * m, hipStream_t s) {
     if (!g_prefill_aux) { m->aux_why = "switched off (BAMD_PREFILL_AUX=0)"; return; }
@@ -810,7 +810,7 @@ static int enqueue_prefill_batch(bamd_context * c, int T, int n_past, hipStream_
                 // ~ H * T * ld * 4 bytes (0.5 GB at 8 K positions on the 8B shape, 2.4 GB at 18 K on a 70B stage).  If the device cannot spare it the
                 // prompt is not lost: without a scratch block the matrix-core launcher declines and attn_batch_kernel (VALU, no scratch) runs
                 if (hipMalloc((void **) &c->attn_bscr, need) == hipSuccess) c->attn_bscr_bytes = need;
-                else { (void) hipGetLastError(); c->attn_bscr = nullptr; c->attn_bscr_failed = need; }   // not retried for this size or larger (every layer of every micro-batch drained the stream and failed again)
+                else { (void) hipGetLastError(); c->attn_bscr = nullptr; c->attn_bscr_failed = need; }   // not retried for this size or larger (or every layer of every micro-batch drains the stream and fails again)
             }
             t.batch_scratch = need && c->attn_bscr_bytes >= need ? c->attn_bscr : nullptr;
         }
@@ -908,7 +908,7 @@ extern "C" __attribute__((visibility("default"))) int bamd_decode(bamd_context *
     if (!c->logits_readback) {
         // nothing of this evaluation is read on the host yet (bamd_set_logits_readback(c, 0): the sampler prefilter runs where the lm_head left the logits): do not wait
         // here — the caller's next synchronising call (bamd_logits_shortlist, bamd_get_logits) enqueues behind this evaluation, waits ONCE and checks the status words
-        // then.  One host round trip per token instead of two (round 5: 2.31 -> 2.27 ms per token through the bridge at 7850 cached positions)
+        // then.  One host round trip per token instead of two (2.31 -> 2.27 ms per token through the bridge at 7850 cached positions)
         c->status_pending = true;
         return 0;
     }
@@ -984,7 +984,7 @@ extern "C" __attribute__((visibility("default"))) const float * bamd_get_logits(
     return c->logits_host;
 }
 // waits for everything enqueued on the context's stream and reports what a bamd_decode without read-back left pending (the co-launch give-up words): the
-// synchronisation point of a caller that evaluated without sampling afterwards (ADVICE r5: a request that stops during its prompt, or at n_ctx - 4)
+// synchronisation point of a caller that evaluated without sampling afterwards (a request that stops during its prompt, or at n_ctx - 4)
 extern "C" __attribute__((visibility("default"))) int bamd_synchronize(bamd_context * c) {
     HIPC(hipSetDevice(c->m->device));
     const hipError_t e = hipStreamSynchronize(c->stream);
@@ -1001,7 +1001,7 @@ extern "C" __attribute__((visibility("default"))) int bamd_set_logits_test(bamd_
     return 0;
 }
 
-// ---- sampler prefilter (SURVEY 8f-4; kernels in bamd_sampler.hip) --------------------------------------------------------
+// ---- sampler prefilter (kernels in bamd_sampler.hip) --------------------------------------------------------
 extern "C" __attribute__((visibility("default"))) int bamd_sampler_tables(bamd_context * c, const uint8_t * halve_class, const float * cutoff_of, int n_vocab) {
     bamd_model * m = c->m;
     if (n_vocab != m->V || !m->with_output) { fail("bamd_sampler_tables: needs the stage that owns the output layer, n_vocab of the model"); return 1; }
@@ -1458,7 +1458,7 @@ extern "C" __attribute__((visibility("default"))) int bamd_op_prefill_route(int 
     *most = (int) m;
     return 0;
 }
-// batched mat-mul of T activation rows against one matrix through the prefill kernels: impl 0 = integer-dot kernel, 2 = matrix-core kernel (1 and 3 were the generations removed in round 6)
+// batched mat-mul of T activation rows against one matrix through the prefill kernels: impl 0 = integer-dot kernel, 2 = matrix-core kernel (1 and 3 named kernels that are gone)
 extern "C" __attribute__((visibility("default"))) int bamd_op_mul_mat_batch(int type, const void * w_raw, int nrows, int k, const float * x, int T, const float * norm_w,
                                                                               float eps, const float * residual, float * y, int impl) {
     if (need_device()) return 1;

@@ -40,7 +40,7 @@ enum bamd_type { BAMD_F32 = 0, BAMD_F16 = 1, BAMD_Q4_K = 12, BAMD_Q5_K = 13, BAM
 BAMD_HD static inline int bamd_block_bytes(int t) { return t == BAMD_Q4_K ? 144 : t == BAMD_Q5_K ? 176 : t == BAMD_Q6_K ? 210 : 0; }
 #ifndef BAMD_XSCALES
 #define BAMD_XSCALES 0          /* 0: the file's 12 packed scale bytes per row (records of 1152 / 1408 B = 8 x the GGUF block); 1: unpacked scales and
-                                   mins, a byte each (1184 / 1440 B) — measured SLOWER on the MI355X in round 2 (gate/up 14.8 vs 13.2 us, decode 649 vs
+                                   mins, a byte each (1184 / 1440 B) — measured SLOWER on the MI355X (gate/up 14.8 vs 13.2 us, decode 649 vs
                                    666 tok/s): 9 vector instructions saved per record do not pay for +2.8 % bytes, a third request per record and
                                    records that no longer start on a 128-byte line */
 #endif

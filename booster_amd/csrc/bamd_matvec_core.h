@@ -95,8 +95,8 @@ __device__ __forceinline__ void stream_segment(const uint8_t * __restrict__ wA, 
 #pragma unroll
         for (int part = 0; part < NPARTS; ++part) {
             // after the last chunk of this row-part: the other half of the pair, the next row-group, or — at the very end of the
-            // wave's stream — D requests through the zero-record descriptor (null_rsrc: they return 0 and fetch nothing; rounds 1-5
-            // re-requested the wave's last record, one record of redundant traffic; the requests stay unconditional so that the
+            // wave's stream — D requests through the zero-record descriptor (null_rsrc: they return 0 and fetch nothing,
+            // where the wave's last record again would be one record of redundant traffic; the requests stay unconditional so that the
             // waits stay counted)
             const bool last = !(PAIR && part == 0) && r + 1 >= count;
             const bool after_b = (PAIR && part == 0) || (last && part == 1);
@@ -149,7 +149,7 @@ __device__ __forceinline__ void stream_segment(const uint8_t * __restrict__ wA, 
 
 // ---- MODE A, gate/up launch with exactly SEVEN row-group pairs per 8-wave workgroup (n_ff = 7 x 8 x 8 x CUs: Llama-3-8B / Mistral-7B, 14336 rows on
 // 256 CUs).  One pair per wave leaves wave 7 idle: SIMD 3 streams 32 records where SIMDs 0-2 stream 64, and the launch is paced by the younger
-// waves 4-6 (timeline, round 2: waves 0-3 exit at 11.4 us, waves 4-6 at 13.8, wave 7 at 3.4).  Here waves 4-6 stop three quarters into their
+// waves 4-6 (timeline: waves 0-3 exit at 11.4 us, waves 4-6 at 13.8, wave 7 at 3.4).  Here waves 4-6 stop three quarters into their
 // gate row and their up row (super-blocks 0..CUT-1, CUT = 3 nb / 4), and wave 7 computes the TERMS {d, fs, dmin, pm} of the last quarter of those six rows
 // and parks them in LDS (the split-K kernels' mechanism); waves 4-6 then replay them IN ORDER behind their own chain steps: every SIMD streams
 // 56 records, and each lane's f32 chain is still the reference's sequential chain over super-blocks 0..nb-1 (ggml-quants.c:6937-6941, :6970).
@@ -240,7 +240,7 @@ __device__ __forceinline__ void stream_pair_short(const uint8_t * __restrict__ w
 // flight while it waits.
 // COMPACT (K = 28672, the 70B ffn_down: 112 super-blocks): a parked record takes 576 bytes — {fs, pm} per lane, {d, dmin} once per row — instead of a float4 per
 // lane, so that TWO term buffers of a whole row-group fit the LDS beside the activations (2 x 63 KB + 32 KB) and the chain of row-group n overlaps the
-// streaming of row-group n + 1 (with one buffer every batch ends in barrier + 112-step chain + barrier: measured slower than one wave per row-group, round 5)
+// streaming of row-group n + 1 (with one buffer every batch ends in barrier + 112-step chain + barrier: measured slower than one wave per row-group)
 struct SplitNoPre { __device__ __forceinline__ void operator()() const { } };
 template <int TYPE, typename REC, int NBW, int M, int NBUF, int EPI, int PRO, bool SMALLK = false, bool ONEB = false, bool UNEVEN = false, typename PRE = SplitNoPre, bool COMPACT = false>
 __device__ __forceinline__ void split_stream(const uint8_t * __restrict__ w, int nb, int first, int count, int stride,

@@ -93,7 +93,7 @@ static const bool g_gateup7 = [] { const char * e = getenv("BAMD_GATEUP7"); retu
 
 // gate/up launch with FOURTEEN row-group pairs per workgroup (n_ff = 112 x grid, K = 8192: Llama-3-70B on 256 CUs).  One pair or two per wave (the generic
 // dealing: waves 0-5 two, waves 6-7 one) put four pairs on SIMDs 0 and 1 and three on SIMDs 2 and 3, and the launch ended with waves 4 and 5 alone
-// (timeline, round 6: waves 0-3 exit at 37.5 us, waves 6-7 at 30, waves 4-5 at 47).  Here every SIMD streams SEVEN rows: waves 0-3 two pairs each
+// (timeline: waves 0-3 exit at 37.5 us, waves 6-7 at 30, waves 4-5 at 47).  Here every SIMD streams SEVEN rows: waves 0-3 two pairs each
 // (pairs w, w + 4), waves 4-7 one pair (8 + w - 4) and then HALF of a pair — waves 4 / 6 the gate row of pairs 12 / 13, waves 5 / 7 the up row, the gate
 // value crossing to the up row's wave through LDS for silu(gate) * up.  Whole rows only: every chain is one wave's sequential chain, as everywhere.
 template <int TYPE, int NBP>

@@ -172,7 +172,7 @@ bool bamd_launch_fast_mixed(const bamd_mv_args & a, int pro, int epi, int grid, 
     if ((nb & 7) != 0 || nb > 8 * BAMD_ACT_BATCH || t0 == t1 || grid < 1 || (nrg0 + nrg1) % grid) return false;
     const int cnt = (nrg0 + nrg1) / grid, nbw = nb >> 3;
     if (cnt == 5 && nrg0 >= 4 * grid && nbw == 4) {                             // the Llama-3-70B shape: K = 8192, five row-groups per workgroup (four of wq | wk, the fifth wk or wv)
-        // MEASURED AND NOT USED BY DEFAULT (round 4, MI355X, a 10-layer stage at the 70B widths, ms per token): one wave per row-group (mode A) 1.260, this
+        // MEASURED AND NOT USED BY DEFAULT (MI355X, a 10-layer stage at the 70B widths, ms per token): one wave per row-group (mode A) 1.260, this
         // split-K instance on eight waves (20 records per wave in registers) 1.275, on sixteen waves (10 records, 128 VGPRs) 1.293 — the prologue, the
         // terms of a wave's records and a 32-step chain per workgroup cost more than five of eight waves streaming 32 records each.  BAMD_QKV70_WAVES=8 / 16
         // selects it for the record (tests/test_gpu_fullsize_ref.py::test_config4_70b_stage runs bit-exact through either).

@@ -121,12 +121,12 @@ __device__ __forceinline__ void batch_segment(const uint8_t * __restrict__ wA, c
     }
 }
 
-// (Rounds 2-5 kept a first generation of matrix-core mat-mul kernels here — every wave expanding its own 16 rows — and a second one in bamd_prefill2.hip;
-// round 6 measured what bounds them (profiles/r06_prefill_ceiling.txt) and kept ONE: bamd_prefill2.hip.  This file keeps the integer-dot kernel — the second
+// (A first generation of matrix-core mat-mul kernels stood here — every wave expanding its own 16 rows — and a second one in bamd_prefill2.hip;
+// what bounds them is measured in profiles/r06_prefill_ceiling.txt, and ONE was kept: bamd_prefill2.hip.  This file keeps the integer-dot kernel — the second
 // implementation the matrix-core kernels are tested against, and what a matrix without a side table runs on — and the plumbing.)
 
 // grid (token tiles, row slots): consecutive workgroups share the weights (L2) and differ in the token tile.  TT tokens per tile: BAMD_TT = 8 while their Q8_K
-// activations fit the LDS (K <= 17920), 4 beyond (K <= 35840: the 70B ffn_down at K = 28672 — round 6; before, a 70B-width model without side tables had no batched
+// activations fit the LDS (K <= 17920), 4 beyond (K <= 35840: the 70B ffn_down at K = 28672; without them a 70B-width model without side tables had no batched
 // kernel at all and evaluated prompts token by token)
 template <int EPI, int TT>
 __global__ void __launch_bounds__(512) matmul_batch_kernel(bamd_mm_args a) {

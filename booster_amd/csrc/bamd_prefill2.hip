@@ -1,11 +1,11 @@
-// bamd_prefill2.hip — round 5: the exact matrix-core prefill mat-mul with the A fragments BUILT ONCE PER WORKGROUP (Q4_K / Q5_K / Q6_K x Q8_K).
+// bamd_prefill2.hip — the exact matrix-core prefill mat-mul with the A fragments BUILT ONCE PER WORKGROUP (Q4_K / Q5_K / Q6_K x Q8_K).
 //
 // Reference: ggml_compute_forward_mul_mat with ne11 = T (ggml.c:12277-12492) over ggml_vec_dot_q{4,5,6}_K_q8_K (ggml-quants.c:6832 / :7400 / :8037);
 // the second implementation it is tested against is the integer-dot kernel of bamd_prefill.hip (matmul_batch_kernel): ONE
 // v_mfma_f32_16x16x32_f16 per SIMD lane e of the reference gives the exact integer sums isum_e of a 16-row x 16-token tile, the f32 chains
 // acc_e = fma(d_x d_y, isum_e, acc_e), the min terms and the final hsum tree follow on the VALU in the reference's order.
 //
-// What changed against bamd_prefill.hip, and why: there every wave expands the nibbles of ITS 16 rows into f16 scale x quant
+// Against kernels in which every wave builds its own fragments, and why: there every wave expands the nibbles of ITS 16 rows into f16 scale x quant
 // fragments and uses each fragment for two MFMAs — 365 issued instructions per wave and super-block, ~150 of them that expansion and the header
 // unpacking in front of it.  Here
 //   * a workgroup is 64 rows x 64 tokens and every fragment is built ONCE per workgroup, one super-block AHEAD, into an LDS ring in MFMA operand layout
@@ -16,9 +16,10 @@
 //     super-block for Q4_K / Q5_K, 72 B for Q6_K: the MI355X has the HBM for it): the builders' per-(row, sub-block pair) scale operands
 //     {s, -1024 s, s'/16, -64 s'} as packed f16 pairs, and the consumers' d, dmin as f32 plus the min-term MFMA operands {2 m_a, 2 m_b, m_a, m_b}, which
 //     travel global -> LDS by DMA with the activation records;
-//   * two layouts: sixteen waves with one 16 x 16 tile each (matmul_mfma3_q4k_kernel: Q4_K / Q5_K), eight waves with 16 x 32 each (matmul_mfma2_q6k_kernel: Q6_K).
-// Same bits as the round-2 kernels (removed in round 6), a third fewer vector instructions per MFMA — and the same time: DESIGN 4c has the measurements of what
-// bounds it, profiles/r06_prefill_ceiling.txt the timing-only ceiling builds (-DBAMD_PREFILL_CEILING).
+//   * two layouts: sixteen waves with one 16 x 16 tile each (matmul_mfma3_q4k_kernel: Q4_K / Q5_K), eight waves with 16 x 32 each (matmul_mfma2_q6k_kernel: Q6_K);
+//     up to 64 tokens, where 64-row blocks leave the chip idle, 16-row blocks of specialised waves (matmul_few_kernel).
+// Same bits as those kernels (which are gone), a third fewer vector instructions per MFMA — and the same time: profiles/r06_prefill_ceiling.txt has
+// what bounds it and the timing-only ceiling builds (-DBAMD_PREFILL_CEILING).
 #include "bamd_device.h"
 #include "bamd_mfma_common.h"
 #include <type_traits>
@@ -137,7 +138,7 @@ struct XStage {
 
 // ---- Q4_K / Q5_K: the sixteen-wave kernel further down (matmul_mfma3_q4k_kernel).  MFMA lane l = (m = l & 15, g = l >> 4): A row m, B token m, k-slots (g, i) =
 //      (sub-block 2g + (i >> 2), u = i & 3); C/D rows 4g + i, token m.  (An eight-wave layout of the same arithmetic — 16 x 32 per wave, 96 accumulators, two waves
-//      per SIMD — lived here in round 5: 27.4 vs 25.4 ms per 512-token micro-batch; removed in round 6, profiles/r06_prefill_ceiling.txt.)
+//      per SIMD — took 27.4 vs 25.4 ms per 512-token micro-batch, profiles/r06_prefill_ceiling.txt.)
 
 // ---- Q6_K: a step is HALF a super-block (four e: 16 MFMAs per wave, two per e and token tile) -----------------------------------------------
 // scale x (q - 32) reaches 4096: the scale is split sc = sa + sl (prefill_aux_q6k_kernel), both fragments come from one f16 image v = (1024 + q) - 1056
@@ -285,7 +286,7 @@ __global__ void __launch_bounds__(512) matmul_mfma2_q6k_kernel(bamd_mma2_args a)
 }
 
 // ==== sixteen waves ===========================================================================================================================
-// The eight-wave kernels above trade vector instructions for LDS traffic and end where the round-2 kernels were (two waves per SIMD: a step is a chain of
+// The eight-wave kernels above trade vector instructions for LDS traffic and end where those were (two waves per SIMD: a step is a chain of
 // dependent latencies).  This kernel — the default for Q4_K / Q5_K — puts four waves on every SIMD:
 //   * a workgroup is SIXTEEN waves: four row tiles x four token tiles, ONE 16 x 16 tile per wave (48 accumulator registers, <= 118 VGPRs);
 //     every A fragment is built once and read by four waves, every token record staged once and read by four;
@@ -297,7 +298,7 @@ __global__ void __launch_bounds__(512) matmul_mfma2_q6k_kernel(bamd_mma2_args a)
 //   * the builder's scale operands travel by DMA as well, two steps ahead, into the operand slot of the block that is being read (its previous content
 //     was consumed one step earlier), so a wave's own loads are 8 bytes of nibbles per lane and step through a buffer descriptor (scalar offset);
 //   * d_y sits inside the token record; the chain FMAs of e follow the MFMA of e + 2 (no MFMA -> VALU wait states); the epilogue stores 16 bytes per lane.
-// 112 issued instructions per wave and step (the round-2 kernel: 365 per two tiles).  What that bought and what it did not: DESIGN 4c.
+// 112 issued instructions per wave and step (one that builds its own fragments: 365 per two tiles).  What bounds it: profiles/r06_prefill_ceiling.txt.
 #define X3_BLK (X_BS_BYTES + X3_CHS + 4096 + 32)           /* records (38 KiB) | headers (3 KiB) | operands (4 KiB) | 32 bytes of zeros: 46 112 B */
 #define X3_BLK0 (2 * X_AF_BYTES)
 #define X3_LDS_BYTES (X3_BLK0 + 2 * X3_BLK)                /* 158 784 B */

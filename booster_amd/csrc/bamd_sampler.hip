@@ -1,4 +1,4 @@
-// bamd_sampler.hip — device side of the Janus sampler (SURVEY §8 f4): the penalties of sample_janus_token (cpp/janus.cpp:236-280)
+// bamd_sampler.hip — device side of the Janus sampler: the penalties of sample_janus_token (cpp/janus.cpp:236-280)
 // applied to the logits where the lm_head left them, then the shortlist { logit / top >= cutoff } (janus.cpp:285-320), so that a
 // few candidates instead of n_vocab floats cross PCIe per token.  Every float operation is the reference's: float x float for the
 // plain scale, float x double -> float where the reference multiplies by a double expression, IEEE division for the ratio test.

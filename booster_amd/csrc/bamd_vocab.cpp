@@ -59,7 +59,7 @@ bool BamdVocab::load(const GgufFile & g, std::string & err) {
     // Mistral-Nemo (tekken), Viking / Poro ... as GGUF names them); the pre-tokenisers of other architectures' families (qwen2, falcon, starcoder ...) are
     // restated and pinned as well — llm_load_vocab keys on tokenizer.ggml.pre alone
     // (the architecture check lives in the model loader, bamd_engine.cpp: the vocabulary is keyed on tokenizer.ggml.model / .pre alone, as llm_load_vocab is —
-    //  vocab-only use on files of other families keeps working; ADVICE r4)
+    //  vocab-only use on files of other families keeps working)
     std::string model;
     if (!g.get_str("tokenizer.ggml.model", model)) { err = "missing tokenizer.ggml.model"; return false; }
     if (model == "no_vocab") { type = BAMD_VOCAB_NONE; return true; }

@@ -1,4 +1,4 @@
-// bamd_vocab.h — tokenizer side of the bridge (SURVEY §8f-1): GGUF vocabulary, SPM and byte-level BPE tokenisers,
+// bamd_vocab.h — tokenizer side of the bridge: GGUF vocabulary, SPM and byte-level BPE tokenisers,
 // token -> piece, end-of-generation test.  CPU-only host code; restates the behaviour of cpp/src/llama-vocab.cpp
 // (llm_tokenizer_spm :190-330, llm_tokenizer_bpe :340-560, tokenizer_st_partition :1119-1240, llama_tokenize_internal
 // :1243-1345, llama_token_to_piece_impl :1539-1608) and the vocab loading of cpp/src/llama.cpp:5250-5760.

@@ -205,7 +205,7 @@ def random_kquant_tensor(ttype, row_len, n_rows, rng, amp=1.0):
 
 def q4_k_m_type(name, il, n_layer):
     """Tensor type under llama.cpp's Q4_K_M recipe for the tensors we use (reference: llama.cpp:15442-15444,
-    :15547-15555, :15603-15610, use_more_bits :15466-15480; SURVEY §8 header)."""
+    :15547-15555, :15603-15610, use_more_bits :15466-15480)."""
     more = il < n_layer // 8 or il >= 7 * n_layer // 8 or (il - n_layer // 8) % 3 == 2
     if name == "output":
         return Q6_K

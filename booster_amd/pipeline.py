@@ -22,7 +22,7 @@ def split_layers(n_layer, n_stage):
     return list(zip([0] + cuts[:-1], cuts))
 
 
-# decode-time model of a launch sequence on the MI355X (DESIGN section 5): weights stream at ~6.2 TB/s inside a launch, lm_head (one long launch) at
+# decode-time model of a launch sequence on the MI355X: weights stream at ~6.2 TB/s inside a launch, lm_head (one long launch) at
 # ~6.4 TB/s, and every layer pays ~21 us that no byte explains (five dependent launches: boundary, first requests, chain tail; attention latency).
 # Checked against the measured launch times: 8B 44.3 us per layer / 67 us lm_head, 70B 107 / 133.
 STREAM_BPS, HEAD_BPS, LAYER_FIXED_S, HEAD_FIXED_S = 6.2e12, 6.4e12, 21e-6, 2e-6
@@ -304,7 +304,7 @@ def _prompt_phase(stage, dist, rank, world, prompt, n_seq, pos_offset, tok, want
 
 
 def run_layer_split_bench(path, cfg, N, rank, local, prompt, n_ctx, warmup, steps, dist, torch, model_name="Llama-3-8B Q4_K_M"):
-    """bench.py's N > 1 leg.  `value` = the BASELINE metric at N GPUs: greedy batch-1 decode of ONE sequence through the N layer-split
+    """bench.py's N > 1 leg.  `value` = the headline metric at N GPUs: greedy batch-1 decode of ONE sequence through the N layer-split
     stages (the stages work one after another, so it does not grow with N — Booster's `gpus:` split buys capacity, not batch-1 speed);
     the throughput with N independent sequences in flight (Booster's pods keeping every stage busy) is reported beside it."""
     import booster_amd
@@ -385,8 +385,8 @@ def run_plumbing_check(N, rank, prompt, warmup, steps, dist, stage_cls, n_layer=
     """bench.py --backend gloo: everything of the N > 1 leg EXCEPT the GPU stage — launch, rendezvous, layer ranges, the round schedule with its
     two-phase use (warm-up, then K timed steps from the carried token), the group-size check, max-over-ranks timing, rank 0's JSON — on a deterministic
     CPU stand-in for the stage (FakeStage).  `value` is the stand-in's rate and means nothing; `config.fed_tokens` lets the test compare the pipelined
-    tokens with a sequential evaluation.  N <= 2: five layers split evenly (the round-3 test's shape); beyond: 10 layers per rank split by
-    split_layers_balanced, i.e. the 80-layer / 8-stage schedule of BASELINE config 4 at N = 8."""
+    tokens with a sequential evaluation.  N <= 2: five layers split evenly (the smallest shape that exercises both); beyond: 10 layers per rank split by
+    split_layers_balanced, i.e. the 80-layer / 8-stage schedule of Llama-3-70B at N = 8."""
     import torch
     if n_layer is None:
         n_layer = 5 if N <= 2 else 10 * N

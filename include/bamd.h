@@ -1,7 +1,7 @@
 /* bamd.h — C-ABI of libbooster_amd.so, level 1: the model-runtime calls that Booster's bridge makes.
  *
  * This is the layer the reference's cpp/bridge.cpp and cpp/janus.cpp call through cpp/include/llama.h
- * (SURVEY.md §8b "below the boundary"); every entry point names the llama.h function it replaces.  Plain C
+ * (what the application calls below its model and context objects); every entry point names the llama.h function it replaces.  Plain C
  * types only: pointers are HOST pointers unless the name says `dev`.  All functions return 0 on success or a
  * non-zero error code unless documented otherwise; bamd_last_error() gives the message.  There is NO CPU
  * fallback: without a usable MI355X-class HIP device every compute entry point fails loudly.
@@ -91,14 +91,14 @@ int bamd_kv_seq_div(bamd_context * c, int p0, int p1, int d);
 /* Greedy decode entirely on the device: n_steps single-token steps starting at position n_past; step 0 consumes
  * the arg-max of the logits left by the previous bamd_decode/bamd_generate_greedy call.  out_tokens receives
  * n_steps+1 ids: the token fed to each step, then the arg-max after the last step.  No host round trip between
- * steps: the steps are replayed as AQL packets with fence scope NONE from the library's own HSA queue (round 6; csrc/bamd_aql.h) where
+ * steps: the steps are replayed as AQL packets with fence scope NONE from the library's own HSA queue (csrc/bamd_aql.h) where
  * the step's kernels allow it, else as one hipGraph per step on the context's stream (bamd_set_aql(0) / BAMD_AQL=0 forces that).
  * *elapsed_ms (optional) = time of the n_steps steps (HIP events; host clock from submission to completion on the own queue). */
 int bamd_generate_greedy(bamd_context * c, int n_past, int n_steps, int32_t * out_tokens, float * elapsed_ms);
 void bamd_set_aql(int on);                 /* process-wide: 1 (default, also env BAMD_AQL) = own AQL queue where possible; 0 = hipGraph replays */
 int bamd_aql_runs(const bamd_context * c); /* bamd_generate_greedy calls + single-token bamd_decode steps of this context that ran on the own queue so far */
 
-/* ---- layer-split stage interface (one process per GPU; hidden state moves between stages, SURVEY §8e) ---- */
+/* ---- layer-split stage interface (one process per GPU; hidden state moves between stages) ---- */
 /* Run this stage's layers on one token.  The token id comes from `token`, or — when token_dev is non-NULL — from that
  * device int32 (no host round trip; used on the first stage).  hidden_in_dev: f32 [n_embd] device pointer (ignored on
  * the first stage, which embeds the token); hidden_out_dev: f32 [n_embd] device pointer (ignored on the last stage,
@@ -120,7 +120,7 @@ int bamd_model_device(const bamd_model * m);
 /* arg-max token of the last bamd_stage_step(want_logits=1) on the last stage; synchronises `hip_stream`. */
 int bamd_stage_argmax(bamd_context * c, void * hip_stream, int32_t * token);
 
-/* ---- sampler prefilter on the device (SURVEY §8f-4): the Janus penalties and shortlist where the lm_head left the logits ---- */
+/* ---- sampler prefilter on the device: the Janus penalties and shortlist where the lm_head left the logits ---- */
 /* one distinct penalised token: logit = (float)(logit * pre) when pre != 0 (the EOS boost, janus.cpp:236), then `count` times
  * logit *= f (kind 0: float x float, janus.cpp:263) or logit = (float)(logit * d) (kind 1: float x double, janus.cpp:255) */
 typedef struct { int32_t id, count, kind; float f; double d, pre; } bamd_logit_penalty;
@@ -145,7 +145,7 @@ int bamd_synchronize(bamd_context * c);
 /* test hook: overwrite the device logits (n_vocab floats) */
 int bamd_set_logits_test(bamd_context * c, const float * logits);
 
-/* ---- tokenizer of a GGUF, CPU only (SURVEY §8f-1): llama_tokenize / llama_token_to_piece / llama_token_is_eog ---- */
+/* ---- tokenizer of a GGUF, CPU only: llama_tokenize / llama_token_to_piece / llama_token_is_eog ---- */
 typedef struct bamd_vocab bamd_vocab;
 bamd_vocab * bamd_vocab_load(const char * gguf_path);                   /* llm_load_vocab, llama.cpp:5250 */
 void bamd_vocab_free(bamd_vocab * v);
@@ -189,7 +189,7 @@ int bamd_bridge_stage_layout(void * ctx, int32_t * out, int cap_stages);
 
 /* Prompt evaluation mode, process-wide: 1 (default, also env BAMD_PREFILL_BATCH) = bamd_decode with 2..512 tokens runs the batched
  * prefill kernels (every layer once per micro-batch, like llama_decode with n_tokens > 1); 0 = token by token through the decode
- * kernels.  Bit-identical results.  Contexts with n_ctx > 8192 use the token-by-token path regardless (round 1). */
+ * kernels.  Bit-identical results.  Contexts with n_ctx > 8192 use the token-by-token path regardless. */
 void bamd_set_prefill_batch(int on);   /* 2 = batched, but the mat-muls on the integer-dot kernel instead of the matrix-core kernels (the path of a model whose
                                         * side tables did not fit: they are built at model load, all matrices or none, BAMD_PREFILL_AUX_RESERVE_GB of the device left free) */
 

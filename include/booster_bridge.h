@@ -2,7 +2,7 @@
  *
  * Byte-compatible with the `extern "C"` block of the reference's cpp/bridge.h:132-165; the Go side
  * (pkg/server/server.go:7-36, pkg/booster/booster.go:15-21) declares exactly these prototypes in its cgo preamble.
- * Semantics follow cpp/bridge.cpp (file:line cited per symbol) with the deviations listed in INTEGRATION.md:
+ * Semantics follow cpp/bridge.cpp (file:line cited per symbol) with these deviations:
  *   - the model runs on MI355X GPUs through include/bamd.h (no CPU path: gpu1..gpu4 all zero is an error);
  *   - status() returns a pointer that stays valid and NUL-terminated while a decode appends (the reference's is racy);
  *   - stop flags are atomics.

@@ -284,7 +284,7 @@ static float vec_dot_q(int type, int n, const void * w, const bo_block_q8_K * y)
 }
 
 /* ggml.c:12277-12492: src1 rows -> Q8_K once (:12345-12372), then one vec_dot per (row, col) (:12186-12275).
- * The result does not depend on the thread count or chunking (SURVEY fact 7). */
+ * The result does not depend on the thread count or chunking. */
 void bo_mul_mat_q(int type, const void * W, int64_t nrows, int64_t K, const float * x, int64_t T, float * y, int nthreads) {
     const size_t rs = bo_row_size(type, K);
     const int64_t nb = K / BO_QK_K;
@@ -527,7 +527,7 @@ int bo_decode(bo_ctx * c, const int32_t * tokens, int T, int n_past) {
                 const int hk = h / gq;
                 const float * qh = q + (size_t) t * E + h * hd;
                 if (T == 1) {
-                    /* llamafile_sgemm F16 x F32 (SURVEY fact 9: q stays f32 when T == 1) */
+                    /* llamafile_sgemm F16 x F32 (q stays f32 when T == 1) */
                     for (int i = 0; i < n_kv; ++i)
                         kq[i] = bo_dot_f16_f32_tinyblas(c->k[il] + (size_t) i * Ekv + hk * hd, qh, hd);
                 } else {

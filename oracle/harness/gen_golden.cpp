@@ -3,7 +3,7 @@
 // oracle/Makefile.  It is run ONLY in the build container (the reference cannot travel to the GPU box);
 // its outputs are committed as data under tests/golden/.
 //
-// What it does (SURVEY.md §4 / §8c):
+// What it does:
 //   1. writes a tiny synthetic Llama GGUF with the reference's own gguf_* writer and ggml_quantize_chunk
 //      (reference: ggml.c gguf_init_empty/gguf_add_tensor/gguf_write_to_file, ggml_quantize_chunk);
 //   2. loads it with llama_load_model_from_file, runs one prefill micro-batch and N greedy decode steps
@@ -167,7 +167,7 @@ int main(int argc, char ** argv) {
 
     llama_context_params cp = llama_context_default_params();
     cp.n_ctx = 128; cp.n_batch = 512; cp.n_ubatch = 512;
-    cp.n_threads = 2; cp.n_threads_batch = 2;     // outputs are thread-count invariant (SURVEY fact 7)
+    cp.n_threads = 2; cp.n_threads_batch = 2;     // outputs are thread-count invariant
     cp.cb_eval = cb_eval; cp.cb_eval_user_data = nullptr;
     cp.flash_attn = false;
     llama_context * ctx = llama_new_context_with_model(model, cp);

@@ -26,7 +26,7 @@ int main(int argc, char ** argv) {
     if (!ctx) { fprintf(stderr, "ref_bench: cannot create context\n"); return 1; }
     const int V = llama_n_vocab(model);
     std::vector<llama_token> prompt((size_t) n_prompt);
-    for (int i = 0; i < n_prompt; ++i) prompt[(size_t) i] = (llama_token) ((7919ll * i + 13) % V);   // SURVEY 8d synthetic prompt
+    for (int i = 0; i < n_prompt; ++i) prompt[(size_t) i] = (llama_token) ((7919ll * i + 13) % V);   // the synthetic prompt
     auto t0 = std::chrono::steady_clock::now();
     if (llama_decode(ctx, llama_batch_get_one(prompt.data(), n_prompt, 0, 0))) { fprintf(stderr, "ref_bench: prefill failed\n"); return 1; }
     const double tp = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();

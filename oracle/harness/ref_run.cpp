@@ -2,7 +2,7 @@
 // GENUINE reference CPU path (ggml + llama.cpp as vendored by gotzmann/booster, compiled in place by oracle/Makefile).  Runs ONLY
 // in the build container; what it writes is committed as data under tests/golden/ (tokens, a few logits, digests — no weights).
 //
-// It evaluates the deterministic synthetic prompt tok[i] = (7919 i + 13) mod V (SURVEY.md §8d) in micro-batches of 512 exactly as
+// It evaluates the deterministic synthetic prompt tok[i] = (7919 i + 13) mod V in micro-batches of 512 exactly as
 // cpp/bridge.cpp feeds a prompt (n_batch chunks through llama_decode, bridge.cpp:560-600), then decodes greedily, and records for
 // the prompt's last token and every generated token:
 //   tokens        i32 [n_decode + 1]     arg-max of each logits vector (token fed to the next step)
