@@ -153,7 +153,7 @@ __global__ void __launch_bounds__(256) ssm_step_kernel(bamd_batch_dev b, bamd_ss
 // matrix instructions take 0.4 us of a SIMD's time; the rest is what stands between them, which is why two waves share a SIMD (four waves a block: 331 us).
 // The products meet a later token's B, C and x with a factor of zero, which hides any finite value: the sums above are the recurrence as long as the state in front is finite and every B,
 // C, x and step size of a chunk is below SSM_TAME in magnitude (then no product overflows: a token adds less than 2^90 to a state).  From the first chunk that is not so on, a block goes one
-// token after the other, so that an infinity or NaN reaches the tokens behind it and none in front.
+// token after the other, so that an infinity or NaN reaches the tokens behind it and none in front.  (The look at every value of a chunk: 258 -> 264 us on one card.)
 #define SSM_TAME 0x1p30f
 template <int NT>
 __global__ void __launch_bounds__(512) ssm_chunk_kernel(bamd_batch_dev b, bamd_ssm_args a) {
