@@ -151,16 +151,14 @@ __global__ void __launch_bounds__(256) ssm_step_kernel(bamd_batch_dev b, bamd_ss
 // (the four rows a lane holds are the four steps of a 16x16x4 product), as B^T C comes out in the order that its product with x wants.  Chunk c + 2 is requested and chunk c + 1 put
 // into LDS while c is computed.  One token after the other on the vector ALUs was a chain of 283 ns per token: 2048 tokens of 128 heads x 64 x 128 took 525 us; now 271.  A chunk's
 // matrix instructions take 0.4 us of a SIMD's time; the rest is what stands between them, which is why two waves share a SIMD (four waves a block: 331 us).
-// The products meet a later token's B, C and x with a factor of zero, which hides any finite value: the sums above are the recurrence as long as the state in front is finite and every B,
-// C, x and step size of a chunk is below SSM_TAME in magnitude (then no product overflows: a token adds less than 2^90 to a state).  From the first chunk that is not so on, a block goes one
-// token after the other, so that an infinity or NaN reaches the tokens behind it and none in front.  (The look at every value of a chunk: 258 -> 264 us on one card.)
-#define SSM_TAME 0x1p30f
+// The products meet a later token's B, C and x with a factor of zero, which hides any finite value; an infinity, a NaN or a product that overflows shows as a y that is not finite.  Then the
+// wave takes the chunk again one token after the other, from the state in front of it, so that such a token reaches those behind it and none in front.  (A look at every value on
+// its way into LDS instead cost 264 us for 258; this one, under the stores of y, nothing.)
 template <int NT>
 __global__ void __launch_bounds__(512) ssm_chunk_kernel(bamd_batch_dev b, bamd_ssm_args a) {
     constexpr int NQ = 4, NP = 16 * NQ * NT, LB = NP + 4, LX = 36, LD = 20, PF = 16 * NP / 512, KS = 512 / NP;      // row lengths in LDS: four rows on, 16 banks on
     __shared__ __align__(16) float Bs[2][16 * LB], Cs[2][16 * LB], xs[2][16 * LX], yp[2][NQ][16 * LX], dm[2][16 * LD];
     __shared__ __align__(16) float pre[2][16], fd[2][16], dts[2][16];
-    __shared__ int wild[2];                                        // a chunk of this parity was not tame
     const bamd_entry e = b.ent[blockIdx.z];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 15, q = lane >> 4, ct = wave & 1, part = wave >> 1;
     const int h = blockIdx.y, p0 = blockIdx.x * 32, pw = min(32, a.P - p0), N = a.N, inner = a.heads * a.P, ch = inner + 2 * a.groups * N, g = h / (a.heads / a.groups);
@@ -171,7 +169,6 @@ __global__ void __launch_bounds__(512) ssm_chunk_kernel(bamd_batch_dev b, bamd_s
     for (int j = 0; j < NT; ++j)
 #pragma unroll
         for (int i = 0; i < 4; ++i) { const int n = n0 + j * 16 + q * 4 + i, p = ct * 16 + col; S[j][i] = e.pos0 > 0 && n < N && p < pw ? st[(size_t) n * a.P + p] : 0.f; }
-    if (tid < 2) wild[tid] = 0;
     const float D = a.D[h];
     // Chunks on their way, by the parity of the chunk.  Every load is unconditional (a row or column clamped into range, zeroed on its way to LDS): a branch around each costs more
     // than the chunk's arithmetic.  Thread: state row kn of the tokens kt, kt + KS, .., column xc of token xt, step size and decay of token col
@@ -213,10 +210,6 @@ __global__ void __launch_bounds__(512) ssm_chunk_kernel(bamd_batch_dev b, bamd_s
         }
         xf[w] = xc < pw && xt < nt ? xf[w] : 0.f;
         xs[w][xt * LX + xc] = xf[w];
-        float most = fmaf(xf[w], xf[w], fdt[w] * fdt[w]);
-#pragma unroll
-        for (int i = 0; i < PF; ++i) most = fmaf(bf[w][i], bf[w][i], fmaf(cf[w][i], cf[w][i], most));
-        if (!(most < SSM_TAME * SSM_TAME)) wild[w] = 1;
         if (wave < 4) {                                            // row s = tid / 16: the products of the decays s + 1 .. t = col (zero above the diagonal)
             const int s = tid >> 4;
             const float v = scan_up(col > s ? fdec[w] : 1.f);
@@ -231,55 +224,50 @@ __global__ void __launch_bounds__(512) ssm_chunk_kernel(bamd_batch_dev b, bamd_s
         }
     };
     request(0, std::integral_constant<int, 0>()); request(16, std::integral_constant<int, 1>());
-    __syncthreads();                                               // (wild is cleared)
     put(e.n, std::integral_constant<int, 0>());
     __syncthreads();
-    float inf = 0.f;
-#pragma unroll
-    for (int j = 0; j < NT; ++j)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) inf = fmaf(S[j][i], 0.f, inf);
-    bool serial = __any(!(inf == 0.f));
     auto chunk = [&](int t0, auto par) {
         constexpr int w = decltype(par)::value;
         const int nt = e.n - t0;
         const float xk = xf[w], zk = zf[w];
         request(t0 + 32, par);
-        serial = __builtin_amdgcn_readfirstlane(serial || wild[w]);
-        if (!serial) {
-            bamd_v4 cr[NT], br[NT], gt = { 0, 0, 0, 0 }, g2 = { 0, 0, 0, 0 }, y = { 0, 0, 0, 0 }, y2 = { 0, 0, 0, 0 };
-            float ba[NT][4], xw[4], xd[4];
+        bamd_v4 cr[NT], br[NT], gt = { 0, 0, 0, 0 }, g2 = { 0, 0, 0, 0 }, y = { 0, 0, 0, 0 }, y2 = { 0, 0, 0, 0 };
+        bamd_v4 T[NT];                                                // the state behind the chunk
+        float ba[NT][4], xw[4], xd[4];
 #pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                cr[j] = *(const bamd_v4 *) &Cs[w][col * LB + n0 + j * 16 + q * 4]; br[j] = *(const bamd_v4 *) &Bs[w][col * LB + n0 + j * 16 + q * 4];
+        for (int j = 0; j < NT; ++j) {
+            cr[j] = *(const bamd_v4 *) &Cs[w][col * LB + n0 + j * 16 + q * 4]; br[j] = *(const bamd_v4 *) &Bs[w][col * LB + n0 + j * 16 + q * 4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) ba[j][i] = Bs[w][(q * 4 + i) * LB + n0 + j * 16 + col];
+            for (int i = 0; i < 4; ++i) ba[j][i] = Bs[w][(q * 4 + i) * LB + n0 + j * 16 + col];
+        }
+        const bamd_v4 pr = *(const bamd_v4 *) &pre[w][q * 4], dv = *(const bamd_v4 *) &dm[w][col * LD + q * 4], d4 = *(const bamd_v4 *) &dts[w][q * 4], f4 = *(const bamd_v4 *) &fd[w][q * 4];
+        const float all = pre[w][15];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { const float x = xs[w][(q * 4 + i) * LX + ct * 16 + col]; xd[i] = x * d4[i]; xw[i] = x * f4[i]; }
+        if (nt > 16) put(nt - 16, std::integral_constant<int, w ^ 1>());       // (requested a chunk ago; its place was read before the last barrier)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (i & 1) { g2 = __builtin_amdgcn_mfma_f32_16x16x4f32(br[j][i], cr[j][i], g2, 0, 0, 0); y2 = __builtin_amdgcn_mfma_f32_16x16x4f32(cr[j][i], S[j][i], y2, 0, 0, 0); }
+                else { gt = __builtin_amdgcn_mfma_f32_16x16x4f32(br[j][i], cr[j][i], gt, 0, 0, 0); y = __builtin_amdgcn_mfma_f32_16x16x4f32(cr[j][i], S[j][i], y, 0, 0, 0); }
             }
-            const bamd_v4 pr = *(const bamd_v4 *) &pre[w][q * 4], dv = *(const bamd_v4 *) &dm[w][col * LD + q * 4], d4 = *(const bamd_v4 *) &dts[w][q * 4], f4 = *(const bamd_v4 *) &fd[w][q * 4];
-            const float all = pre[w][15];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) { const float x = xs[w][(q * 4 + i) * LX + ct * 16 + col]; xd[i] = x * d4[i]; xw[i] = x * f4[i]; }
-            if (nt > 16) put(nt - 16, std::integral_constant<int, w ^ 1>());       // (requested a chunk ago; its place was read before the last barrier)
+        for (int j = 0; j < NT; ++j) T[j] = S[j] * all;
 #pragma unroll
-            for (int j = 0; j < NT; ++j)
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    if (i & 1) { g2 = __builtin_amdgcn_mfma_f32_16x16x4f32(br[j][i], cr[j][i], g2, 0, 0, 0); y2 = __builtin_amdgcn_mfma_f32_16x16x4f32(cr[j][i], S[j][i], y2, 0, 0, 0); }
-                    else { gt = __builtin_amdgcn_mfma_f32_16x16x4f32(br[j][i], cr[j][i], gt, 0, 0, 0); y = __builtin_amdgcn_mfma_f32_16x16x4f32(cr[j][i], S[j][i], y, 0, 0, 0); }
-                }
+            for (int j = 0; j < NT; ++j) T[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ba[j][i], xw[i], T[j], 0, 0, 0);
+        y = (y + y2) * pr;
 #pragma unroll
-            for (int j = 0; j < NT; ++j) S[j] = S[j] * all;
+        for (int i = 0; i < 4; ++i) y = __builtin_amdgcn_mfma_f32_16x16x4f32((gt[i] + g2[i]) * dv[i], xd[i], y, 0, 0, 0);
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 4; ++i) yp[w][part][(q * 4 + i) * LX + ct * 16 + col] = y[i];
+        const float sum = (y[0] + y[1]) + (y[2] + y[3]);          // (looked at while the stores are under way; a sum that overflows by itself costs time, nothing else)
+        if (!__any(!(fabsf(sum) < INFINITY))) {
 #pragma unroll
-                for (int j = 0; j < NT; ++j) S[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ba[j][i], xw[i], S[j], 0, 0, 0);
-            y = (y + y2) * pr;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) y = __builtin_amdgcn_mfma_f32_16x16x4f32((gt[i] + g2[i]) * dv[i], xd[i], y, 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) yp[w][part][(q * 4 + i) * LX + ct * 16 + col] = y[i];
+            for (int j = 0; j < NT; ++j) S[j] = T[j];
         } else {
-            if (nt > 16) put(nt - 16, std::integral_constant<int, w ^ 1>());
             for (int t = 0; t < min(nt, 16); ++t) {
                 const float d = t ? dm[w][t * LD + t - 1] : pre[w][0], xv = dts[w][t] * xs[w][t * LX + ct * 16 + col];
                 float y = 0.f;
