@@ -406,11 +406,11 @@ static void mv_one(const bamd_dense & w, const bamd_batch_dev & b, const bamd_pr
 }
 // Two shares of K where a matrix has too few row tiles for the CUs (more than 128 would make a second round of their blocks) and enough columns that halves are still worth a block: at K = 2048
 // they are level with 8 rows (2048 outputs: 5.7 us) and ahead with more (45 rows 8.7 -> 7.5) or longer rows (K = 4096: 7.1 -> 6.5, 11.8 -> 9.4).  A prologue that writes state stays whole.  A bfloat16
-// row built in front is built whole by either half's block, which more than 64 row tiles pay back from K = 5632 on (2048 outputs, PolyNorm: K = 4096 9.3 us whole, 9.8 in halves; 5632 11.9 and
-// 10.9; 64 row tiles: 8.7 and 8.7); the 32-bit products behind it are longer (12.5 and 11.5)
+// row built in front is built whole by either half's block, which more than 64 row tiles pay back where the whole product's waves would need a second round of eight column blocks, beyond K = 4096
+// (1536 outputs, PolyNorm: K = 4096 8.8 us whole, 9.2 in halves; 4128 9.6 and 9.2; 64 row tiles: 8.7 and 8.7); the 32-bit products behind it are longer (12.5 and 11.5)
 static int few_parts(int act, const bamd_dense & w, int pre, int most) {
     if (most < 2 || w.row_tiles > 128 || w.k_tiles < 64 || pre == BAMD_PRE_RESIDUAL || pre == BAMD_PRE_FINAL || pre == BAMD_PRE_LAYER) return 1;
-    return act == BAMD_ACT_BF16 && pre != BAMD_PRE_ROWS && w.row_tiles > 64 && w.k_tiles < 176 ? 1 : 2;
+    return act == BAMD_ACT_BF16 && pre != BAMD_PRE_ROWS && w.row_tiles > 64 && w.k_tiles <= 128 ? 1 : 2;
 }
 int bamd_dense_route(int act, const bamd_dense & w, int rows, int pre, int most, int & share) {
     if (pre < 0) return pick_tile(act, w, rows, most, share);
