@@ -312,7 +312,8 @@ def op_mul_mat_vec(ttype, w_raw, nrows, k, x, norm_w=None, eps=0.0, residual=Non
 
 
 def op_mul_mat_batch(ttype, w_raw, nrows, k, x, norm_w=None, eps=0.0, residual=None, impl=0):
-    """Y[t] = W . Q8_K(x[t]) for T rows at once through the prefill kernels: impl 0 = integer-dot kernel, 2 = matrix-core kernels."""
+    """Y[t] = W . Q8_K(x[t]) for T rows at once through the prefill kernels: impl 0 = integer-dot kernel, 2 = the matrix-core kernel a prompt takes, 4 | 5 = the one of many tokens on
+    eight | four (Q6_K) waves, whatever the size."""
     w_raw = np.ascontiguousarray(w_raw, np.uint8); x = np.ascontiguousarray(x, np.float32)
     T = x.shape[0]
     nw = None if norm_w is None else np.ascontiguousarray(norm_w, np.float32)

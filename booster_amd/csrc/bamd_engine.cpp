@@ -671,6 +671,10 @@ extern "C" int bamd_stage_step(bamd_context * c, int32_t token, const void * tok
                                int prefill_mode, void * hip_stream);
 // ---- batched prefill: a micro-batch of T > 1 tokens through the layers at once (llama_decode with n_tokens > 1) -----------
 #define BAMD_PREFILL_CAP 512            /* the reference's default n_batch / n_ubatch */
+// Prompt tokens that go through the layers together.  A position's results do not depend on the others in its micro-batch (masked positions add exact zeros), except that a
+// micro-batch of ONE token has arithmetic of its own: prefill_part cuts so that the one-token tail of a prompt stays one.  2048 tokens fill the chip where 512 leave the last round of
+// blocks half empty (14336 x 4096: 3.5 rounds; 6144 x 4096: 1.5), and take one pass over the output layer instead of four.  Attention runs in slices of BAMD_PREFILL_CAP (score rows).
+#define BAMD_PREFILL_WIDE 2048
 // pos_hi: last position of the micro-batch — its score rows (2 x padded length floats per head) must fit the LDS: 18 432 positions
 static bool prefill_batch_supported(const bamd_context * c, int pos_hi) {
     const bamd_model * m = c->m;
@@ -729,17 +733,34 @@ static void build_prefill_aux(bamd_model * m, hipStream_t s) {
     hipStreamSynchronize(s);
     m->aux_ok = true;
 }
-static int ensure_batch_buffers(bamd_context * c) {
-    if (c->bcap) return 0;
+// buffers for T tokens: of BAMD_PREFILL_CAP, of BAMD_PREFILL_WIDE once a longer prompt comes.  1: not allocated (what was there stays)
+static int ensure_batch_buffers(bamd_context * c, int tokens) {
+    if (c->bcap >= tokens) return 0;
     bamd_model * m = c->m;
-    const size_t T = BAMD_PREFILL_CAP, Ekv = (size_t) m->Hkv * m->hd;
-    if (dev_alloc(c->allocs, (void **) &c->bx, T * m->E * 4) || dev_alloc(c->allocs, (void **) &c->bx2, T * m->E * 4) ||
-        dev_alloc(c->allocs, (void **) &c->bqkv, T * (m->E + 2 * Ekv) * 4) || dev_alloc(c->allocs, (void **) &c->batt, T * m->E * 4) ||
-        dev_alloc(c->allocs, (void **) &c->bh, T * m->F * 4) ||
-        dev_alloc(c->allocs, (void **) &c->bblob, T * bamd_blob_bytes(std::max(m->E, m->F))) ||
-        dev_alloc(c->allocs, (void **) &c->bblob16, T * bamd_blob16_bytes(std::max(m->E, m->F)))) return 1;
+    const size_t T = tokens <= BAMD_PREFILL_CAP ? BAMD_PREFILL_CAP : BAMD_PREFILL_WIDE, Ekv = (size_t) m->Hkv * m->hd;
+    const int Kmax = std::max(m->E, m->F);
+    void ** const slot[] = { (void **) &c->bx, (void **) &c->bx2, (void **) &c->bqkv, (void **) &c->batt, (void **) &c->bh, (void **) &c->bblob, (void **) &c->bblob16, (void **) &c->bfrag, (void **) &c->bst };
+    const size_t bytes[] = { T * m->E * 4, T * m->E * 4, T * (m->E + 2 * Ekv) * 4, T * m->E * 4, T * m->F * 4, T * bamd_blob_bytes(Kmax), T * bamd_blob16_bytes(Kmax), bamd_tokfrag_bytes((int) T, Kmax),
+                             (BAMD_PREFILL_WIDE / BAMD_PREFILL_CAP) * sizeof(bamd_step_state) };
+    constexpr int N = sizeof bytes / sizeof *bytes;
+    std::vector<void *> got; void * p[N];
+    for (int i = 0; i < N; ++i) if (dev_alloc(got, &p[i], bytes[i])) { (void) hipGetLastError(); for (void * q : got) hipFree(q); return 1; }
+    if (c->bcap) {
+        HIPC(hipStreamSynchronize(c->stream));
+        for (void ** o : slot) { auto it = std::find(c->allocs.begin(), c->allocs.end(), *o); if (it != c->allocs.end()) c->allocs.erase(it); hipFree(*o); }
+    }
+    for (int i = 0; i < N; ++i) { *slot[i] = p[i]; c->allocs.push_back(p[i]); }
     c->bcap = (int) T;
     return 0;
+}
+// tokens of a prompt of n tokens at n_past that are evaluated as one batch, cut as llama_decode's n_ubatch cuts (llama.cpp:14615) wherever that shows
+static int prefill_part(bamd_context * c, int n, int n_past) {
+    const int wide = n > BAMD_PREFILL_WIDE ? BAMD_PREFILL_WIDE : n % BAMD_PREFILL_CAP == 1 ? n - 1 : n;
+    if (wide > BAMD_PREFILL_CAP && g_prefill_mfma && c->m->aux_ok && !c->cells.active && !c->bwide_failed && prefill_batch_supported(c, n_past + wide - 1)) {
+        if (hipSetDevice(c->m->device) == hipSuccess && !ensure_batch_buffers(c, wide)) return wide;
+        c->bwide_failed = true;                                   // (no memory for them: prompts go on in portions of BAMD_PREFILL_CAP)
+    }
+    return std::min(BAMD_PREFILL_CAP, n);
 }
 // one batched mat-mul: K-quant segments with a side table on the matrix-core kernels, the rest on the integer-dot kernel (identical bits either way).
 // aux[i]: side table of segment i (null: none)
@@ -747,6 +768,7 @@ static int batch_mm(bamd_context * c, bamd_mm_args a, int epi, int T, hipStream_
     bamd_model * m = c->m;
     auto on_mfma = [&](int i) { return g_prefill_mfma && aux[i] && (a.seg[i].type == BAMD_Q4_K || a.seg[i].type == BAMD_Q5_K || a.seg[i].type == BAMD_Q6_K); };
     auto mm_mfma = [&](const bamd_mv_seg & sg, const void * ax, int nv, float * out, const float * res, int e) {
+        if (const int waves = bamd_prefill_tokfrag(sg.type, sg.nrows, a.K, T)) return bamd_launch_matmul_wide(sg.w, sg.type, nv, sg.nrows, a.K, c->bfrag, T, out, res, e, a.ldo, waves, s);
         return bamd_launch_matmul_mfma2(sg.w, ax, sg.type, nv, sg.nrows, a.K, c->bblob16, T, out, res, e, a.ldo, s);
     };
     if (epi == BAMD_EPI_SILU_MUL) {
@@ -773,6 +795,15 @@ static int batch_mm(bamd_context * c, bamd_mm_args a, int epi, int T, hipStream_
     }
     return 0;
 }
+// the activations of a product quantised into the layouts that its segments' kernels read
+static void batch_quantize(bamd_context * c, const float * x, const float * nw, const bamd_mm_args & a, int T, hipStream_t s, const void * const * aux, bool pair = false) {
+    bool ints = false, recs = false, frags = false;
+    for (int i = 0; i < a.nseg; ++i) {
+        const bool mfma = g_prefill_mfma && aux[i] && (!pair || (aux[0] && aux[1] && a.seg[0].type == a.seg[1].type));
+        if (!mfma) ints = true; else if (bamd_prefill_tokfrag(a.seg[i].type, a.seg[i].nrows, a.K, T)) frags = true; else recs = true;
+    }
+    bamd_launch_quantize_batch(x, nw, c->m->eps, a.K, T, ints ? c->bblob : nullptr, recs ? c->bblob16 : nullptr, frags ? c->bfrag : nullptr, s);
+}
 // first stage: tokens already in c->forced; later stages: hidden_in [T][E] f32 on this device.  Last stage: leaves the hidden state of
 // the LAST token in c->x (for lm_head); other stages: writes hidden_out [T][E] (possibly on the next device: peer copy).
 static int enqueue_prefill_batch(bamd_context * c, int T, int n_past, hipStream_t s, const void * hidden_in = nullptr, void * hidden_out = nullptr) {
@@ -782,54 +813,64 @@ static int enqueue_prefill_batch(bamd_context * c, int T, int n_past, hipStream_
     h.pos_base = n_past; h.pos = n_past; h.n_ctx = c->n_ctx; h.step = T;
     h.n_kv = std::min(c->n_ctx, (n_past + T + 31) / 32 * 32);
     HIPC(hipMemcpyAsync(c->st, &h, sizeof h, hipMemcpyHostToDevice, s));
+    bamd_step_state hs[BAMD_PREFILL_WIDE / BAMD_PREFILL_CAP];            // of every slice of the attention
+    for (int i = 0; i < (T + BAMD_PREFILL_CAP - 1) / BAMD_PREFILL_CAP; ++i) { hs[i] = h; hs[i].pos = hs[i].pos_base = n_past + i * BAMD_PREFILL_CAP; }
+    HIPC(hipMemcpyAsync(c->bst, hs, sizeof h * (size_t) ((T + BAMD_PREFILL_CAP - 1) / BAMD_PREFILL_CAP), hipMemcpyHostToDevice, s));
     if (m->with_embd) bamd_launch_embed_batch(c->forced, T, m->tok_embd.raw, m->tok_embd.type, E, m->V, c->bx, s);
     else HIPC(hipMemcpyAsync(c->bx, hidden_in, (size_t) T * E * 4, hipMemcpyDeviceToDevice, s));
     for (size_t il = 0; il < m->layers.size(); ++il) {
         const DevLayer & ly = m->layers[il];
         bamd_mm_args a; memset(&a, 0, sizeof a);
         // q,k,v                                                            (llama.cpp:8810-8835)
-        bamd_launch_quantize_batch(c->bx, ly.attn_norm, m->eps, E, T, c->bblob, c->bblob16, s);
         seg_of(a.seg[0], ly.wq, c->bqkv); a.nseg = 1;
         if (ly.wk.type == ly.wq.type) { a.seg[0].nrows += ly.wk.nrows; a.seg[0].nvalid += ly.wk.nrows; }
         else { seg_of(a.seg[a.nseg], ly.wk, c->bqkv + E); a.nseg++; }
         if (ly.wv.type == ly.wk.type) { a.seg[a.nseg - 1].nrows += ly.wv.nrows; a.seg[a.nseg - 1].nvalid += ly.wv.nrows; }
         else { seg_of(a.seg[a.nseg], ly.wv, c->bqkv + E + Ekv); a.nseg++; }
         a.blob = c->bblob; a.K = E; a.T = T; a.ldo = ldq;
+        batch_quantize(c, c->bx, ly.attn_norm, a, T, s, ly.aux_qkv);
         if (batch_mm(c, a, BAMD_EPI_STORE, T, s, ly.aux_qkv)) return fail("batched mat-mul: unsupported shape");
         // RoPE, KV store, attention with the T>1 semantics                  (llama.cpp:8837-8849, :8318-8353)
         bamd_attn_args t; memset(&t, 0, sizeof t);
         t.st = c->st; t.q = c->bqkv; t.k = c->bqkv + E; t.v = c->bqkv + E + Ekv; t.kc = c->kc[il]; t.vc = c->vc[il]; t.rope = c->rope; t.out = c->batt;
         t.hd = m->hd; t.Hkv = m->Hkv; t.n_ctx = c->n_ctx_pad; t.kq_scale = 1.0f / sqrtf((float) m->hd); t.prefill_mode = 1;
-        t.batch = 1; t.ld_qkv = ldq; t.ld_out = E; t.lds_ld = attn_lds_ld(c, n_past + T - 1); t.batch_pos0p1 = n_past + 1;
-        {
-            const size_t need = m->hd == 128 ? bamd_attention_batch_mfma_scratch(m->Hkv, gq, T, t.lds_ld) : 0;
-            if (need > c->attn_bscr_bytes && !(c->attn_bscr_failed && need >= c->attn_bscr_failed)) {   // (freed with the context; replaced only while nothing of this context is in flight: stream order)
-                HIPC(hipStreamSynchronize(s));
-                if (c->attn_bscr) hipFree(c->attn_bscr);
-                c->attn_bscr = nullptr; c->attn_bscr_bytes = 0;
-                // ~ H * T * ld * 4 bytes (0.5 GB at 8 K positions on the 8B shape, 2.4 GB at 18 K on a 70B stage).  If the device cannot spare it the
-                // prompt is not lost: without a scratch block the matrix-core launcher declines and attn_batch_kernel (VALU, no scratch) runs
-                if (hipMalloc((void **) &c->attn_bscr, need) == hipSuccess) c->attn_bscr_bytes = need;
-                else { (void) hipGetLastError(); c->attn_bscr = nullptr; c->attn_bscr_failed = need; }   // not retried for this size or larger (or every layer of every micro-batch drains the stream and fails again)
-            }
-            t.batch_scratch = need && c->attn_bscr_bytes >= need ? c->attn_bscr : nullptr;
+        t.batch = 1; t.ld_qkv = ldq; t.ld_out = E;
+        const int slice = std::min(T, BAMD_PREFILL_CAP);
+        const size_t scratch = m->hd == 128 ? bamd_attention_batch_mfma_scratch(m->Hkv, gq, slice, attn_lds_ld(c, n_past + T - 1)) : 0;      // of the last slice: the longest rows
+        auto score_rows = [&](size_t need) -> int {              // (freed with the context; replaced only while nothing of this context is in flight: stream order)
+            if (need <= c->attn_bscr_bytes || (c->attn_bscr_failed && need >= c->attn_bscr_failed)) return 0;
+            HIPC(hipStreamSynchronize(s));
+            if (c->attn_bscr) hipFree(c->attn_bscr);
+            c->attn_bscr = nullptr; c->attn_bscr_bytes = 0;
+            // ~ H * slice * ld * 4 bytes (0.5 GB at 8 K positions on the 8B shape, 2.4 GB at 18 K on a 70B stage).  If the device cannot spare it the
+            // prompt is not lost: without a scratch block the matrix-core launcher declines and attn_batch_kernel (VALU, no scratch) runs
+            if (hipMalloc((void **) &c->attn_bscr, need) == hipSuccess) c->attn_bscr_bytes = need;
+            else { (void) hipGetLastError(); c->attn_bscr = nullptr; c->attn_bscr_failed = need; }   // not retried for this size or larger (or every layer of every micro-batch drains the stream and fails again)
+            return 0;
+        };
+        if (score_rows(scratch)) return 1;
+        for (int off = 0; off < T; off += slice) {
+            const int n = std::min(slice, T - off);
+            bamd_attn_args u = t;
+            u.st = c->bst + off / BAMD_PREFILL_CAP; u.batch_pos0p1 = n_past + off + 1; u.lds_ld = attn_lds_ld(c, n_past + off + n - 1);
+            u.q += (size_t) off * ldq; u.k += (size_t) off * ldq; u.v += (size_t) off * ldq; u.out += (size_t) off * E;
+            const size_t need = m->hd == 128 ? bamd_attention_batch_mfma_scratch(m->Hkv, gq, n, u.lds_ld) : 0;
+            if (score_rows(need)) return 1;                      // (a slice in front of one whose rows did not fit)
+            u.batch_scratch = need && c->attn_bscr_bytes >= need ? c->attn_bscr : nullptr;
+            if (bamd_launch_attention_batch(u, gq, n, s)) return fail("batched attention: unsupported head configuration");
         }
-        if (bamd_launch_attention_batch(t, gq, T, s)) return fail("batched attention: unsupported head configuration");
         // x2 = x + Wo . att
-        bamd_launch_quantize_batch(c->batt, nullptr, 0.f, E, T, c->bblob, c->bblob16, s);
         memset(&a, 0, sizeof a);
         seg_of(a.seg[0], ly.wo, c->bx2); a.nseg = 1; a.blob = c->bblob; a.K = E; a.T = T; a.ldo = E; a.res = c->bx;
-        { const void * ax[3] = { ly.aux_o, nullptr, nullptr }; if (batch_mm(c, a, BAMD_EPI_ADD, T, s, ax)) return fail("batched mat-mul: unsupported shape"); }
+        { const void * ax[3] = { ly.aux_o, nullptr, nullptr }; batch_quantize(c, c->batt, nullptr, a, T, s, ax); if (batch_mm(c, a, BAMD_EPI_ADD, T, s, ax)) return fail("batched mat-mul: unsupported shape"); }
         // h = silu(Wg . a) * (Wu . a)
-        bamd_launch_quantize_batch(c->bx2, ly.ffn_norm, m->eps, E, T, c->bblob, c->bblob16, s);
         memset(&a, 0, sizeof a);
         seg_of(a.seg[0], ly.wg, c->bh); seg_of(a.seg[1], ly.wu, c->bh); a.nseg = 2; a.blob = c->bblob; a.K = E; a.T = T; a.ldo = F;
-        { const void * ax[3] = { ly.aux_g, ly.aux_u, nullptr }; if (batch_mm(c, a, BAMD_EPI_SILU_MUL, T, s, ax)) return fail("batched mat-mul: unsupported shape"); }
+        { const void * ax[3] = { ly.aux_g, ly.aux_u, nullptr }; batch_quantize(c, c->bx2, ly.ffn_norm, a, T, s, ax, true); if (batch_mm(c, a, BAMD_EPI_SILU_MUL, T, s, ax)) return fail("batched mat-mul: unsupported shape"); }
         // x = x2 + Wd . h
-        bamd_launch_quantize_batch(c->bh, nullptr, 0.f, F, T, c->bblob, c->bblob16, s);
         memset(&a, 0, sizeof a);
         seg_of(a.seg[0], ly.wd, c->bx); a.nseg = 1; a.blob = c->bblob; a.K = F; a.T = T; a.ldo = E; a.res = c->bx2;
-        { const void * ax[3] = { ly.aux_d, nullptr, nullptr }; if (batch_mm(c, a, BAMD_EPI_ADD, T, s, ax)) return fail("batched mat-mul: unsupported shape"); }
+        { const void * ax[3] = { ly.aux_d, nullptr, nullptr }; batch_quantize(c, c->bh, nullptr, a, T, s, ax); if (batch_mm(c, a, BAMD_EPI_ADD, T, s, ax)) return fail("batched mat-mul: unsupported shape"); }
     }
     if (m->with_output) HIPC(hipMemcpyAsync(c->x, c->bx + (size_t) (T - 1) * E, (size_t) E * 4, hipMemcpyDeviceToDevice, s));
     else HIPC(hipMemcpyAsync(hidden_out, c->bx, (size_t) T * E * 4, hipMemcpyDeviceToDevice, s));
@@ -871,9 +912,12 @@ extern "C" __attribute__((visibility("default"))) int bamd_decode(bamd_context *
     }
     if (n_tokens > BAMD_PREFILL_CAP && g_prefill_batch) {
         // llama_decode's n_ubatch split (llama.cpp:14615): micro-batches of 512, the logits are those of the last token
-        for (int i = 0; i < n_tokens; i += BAMD_PREFILL_CAP)
-            if (bamd_decode(c, tokens + i, std::min(BAMD_PREFILL_CAP, n_tokens - i), n_past + i)) return 1;
-        return 0;
+        int part = prefill_part(c, n_tokens, n_past);
+        if (part < n_tokens) {
+            for (int i = 0; i < n_tokens; i += part, part = prefill_part(c, n_tokens - i, n_past + i))
+                if (bamd_decode(c, tokens + i, part, n_past + i)) return 1;
+            return 0;
+        }
     }
     if (n_tokens > c->forced_cap) { fail("n_tokens out of range (token by token evaluation takes at most 4096 per call)"); return 1; }
     if (hipSetDevice(m->device) != hipSuccess) { fail("hipSetDevice"); return 1; }
@@ -881,9 +925,9 @@ extern "C" __attribute__((visibility("default"))) int bamd_decode(bamd_context *
     if (c->cells.active && n_tokens > 1) { fail("after a context shift (bamd_kv_seq_add) tokens are evaluated one per call"); return 1; }
     if (!c->cells.active) c->n_cached = std::max(c->n_cached, n_past + n_tokens);
     if (hipMemcpyAsync(c->forced, tokens, (size_t) n_tokens * 4, hipMemcpyHostToDevice, s) != hipSuccess) { fail("H2D tokens"); return 1; }
-    if (n_tokens > 1 && n_tokens <= BAMD_PREFILL_CAP && prefill_batch_supported(c, n_past + n_tokens - 1)) {
+    if (n_tokens > 1 && (n_tokens <= BAMD_PREFILL_CAP || n_tokens <= c->bcap) && prefill_batch_supported(c, n_past + n_tokens - 1)) {
         // one micro-batch: every layer once for all tokens (each weight record unpacked once per 8 tokens), lm_head for the last
-        if (ensure_batch_buffers(c)) return 1;
+        if (ensure_batch_buffers(c, n_tokens)) return 1;
         if (enqueue_prefill_batch(c, n_tokens, n_past, s)) return 1;
         enqueue_lm_head(c, s, nullptr);                                  // n_outputs = 1: last token only (llama.cpp:14580-14593)
     } else if (n_tokens == 1) {
@@ -963,7 +1007,7 @@ extern "C" __attribute__((visibility("default"))) int bamd_stage_prefill(bamd_co
     if (m->with_embd) { if (!tokens) return fail("bamd_stage_prefill: tokens required on the first stage"); HIPC(hipMemcpyAsync(c->forced, tokens, (size_t) n_tokens * 4, hipMemcpyHostToDevice, s)); }
     else if (!hidden_in_dev) return fail("bamd_stage_prefill: hidden_in required");
     if (!m->with_output && !hidden_out_dev) return fail("bamd_stage_prefill: hidden_out required");
-    if (ensure_batch_buffers(c)) return 1;
+    if (ensure_batch_buffers(c, n_tokens)) return 1;
     if (enqueue_prefill_batch(c, n_tokens, n_past, s, hidden_in_dev, hidden_out_dev)) return 1;
     if (m->with_output && want_logits) enqueue_lm_head(c, s, nullptr);
     {   // a launch the runtime rejected (LDS size, grid) leaves no other trace (bamd_decode checks the same way)
@@ -1458,7 +1502,8 @@ extern "C" __attribute__((visibility("default"))) int bamd_op_prefill_route(int 
     *most = (int) m;
     return 0;
 }
-// batched mat-mul of T activation rows against one matrix through the prefill kernels: impl 0 = integer-dot kernel, 2 = matrix-core kernel (1 and 3 named kernels that are gone)
+// batched mat-mul of T activation rows against one matrix through the prefill kernels: impl 0 = integer-dot kernel, 2 = the matrix-core kernel that a prompt takes, 4 | 5 = the one of many tokens
+// on eight | four (Q6_K) waves, whatever the size (1 and 3 named kernels that are gone)
 extern "C" __attribute__((visibility("default"))) int bamd_op_mul_mat_batch(int type, const void * w_raw, int nrows, int k, const float * x, int T, const float * norm_w,
                                                                               float eps, const float * residual, float * y, int impl) {
     if (need_device()) return 1;
@@ -1468,12 +1513,15 @@ extern "C" __attribute__((visibility("default"))) int bamd_op_mul_mat_batch(int 
     void * raw = t.up(w_raw, wb), * str = t.up(nullptr, wbp);
     float * dx = (float *) t.up(x, (size_t) T * k * 4); float * dw = norm_w ? (float *) t.up(norm_w, (size_t) k * 4) : nullptr;
     float * dres = residual ? (float *) t.up(residual, (size_t) T * nrows * 4) : nullptr; float * dy = (float *) t.up(nullptr, (size_t) T * nrows * 4);
-    void * blob = t.up(nullptr, (size_t) T * bamd_blob_bytes(k)), * blob16 = t.up(nullptr, (size_t) T * bamd_blob16_bytes(k));
-    if (!raw || !str || !dx || !dy || !blob || !blob16 || (norm_w && !dw) || (residual && !dres)) return fail("device alloc/copy failed");
+    void * blob = t.up(nullptr, (size_t) T * bamd_blob_bytes(k)), * blob16 = t.up(nullptr, (size_t) T * bamd_blob16_bytes(k)), * frag = t.up(nullptr, bamd_tokfrag_bytes(T, k));
+    if (!raw || !str || !dx || !dy || !blob || !blob16 || !frag || (norm_w && !dw) || (residual && !dres)) return fail("device alloc/copy failed");
     HIPC(hipMemset(str, 0, wbp));
     bamd_launch_repack(raw, str, type, nrows, k, nullptr);
-    bamd_launch_quantize_batch(dx, dw, eps, k, T, blob, blob16, nullptr);
-    if (impl == 2) {                                                // the matrix-core kernel: side table built here, as the engine builds it at model load
+    bamd_launch_quantize_batch(dx, dw, eps, k, T, blob, blob16, frag, nullptr);
+    const int waves = impl == 4 ? 8 : impl == 5 ? 4 : impl == 2 ? bamd_prefill_tokfrag(type, nrows_pad, k, T) : 0;
+    if (waves) {
+        if (bamd_launch_matmul_wide(str, type, nrows, nrows_pad, k, frag, T, dy, dres, dres ? BAMD_EPI_ADD : BAMD_EPI_STORE, nrows, waves, nullptr)) return fail("MFMA path: unsupported type/shape");
+    } else if (impl == 2) {                                                // the matrix-core kernel: side table built here, as the engine builds it at model load
         void * aux = t.up(nullptr, bamd_prefill_aux_bytes(type, nrows_pad, k));
         if (!aux) return fail("device alloc failed");
         bamd_launch_prefill_aux(str, type, nrows_pad, k, aux, nullptr);

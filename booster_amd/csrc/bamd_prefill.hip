@@ -21,9 +21,10 @@
 // (the B operand of the Q4_K min-term MFMA), then the four i16 pairs (S_2l, S_2l+1) (Q5_K), then the block scale d_y (f32, byte 560); after the nb super-blocks, yd[nb] f32 again.
 template <bool NORM>
 __global__ void __launch_bounds__(512) quantize_batch_kernel(const float * __restrict__ x, const float * __restrict__ nw, float eps, int K,
-                                                             uint8_t * __restrict__ blob, uint8_t * __restrict__ blob16) {
+                                                             uint8_t * __restrict__ blob, uint8_t * __restrict__ blob16, uint8_t * __restrict__ frag) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    const int nb = K >> 8, t = blockIdx.x;
+    // the sixteen tokens of a tile on one XCD (workgroups go round the eight): their pieces of a line of fragments meet in its L2
+    const int nb = K >> 8, u = blockIdx.x & 127, t = (blockIdx.x | 127) < gridDim.x ? (int) (blockIdx.x & ~127u) + (u & 7) * 16 + (u >> 3) : (int) blockIdx.x;
     uint32_t * q8 = (uint32_t *) smem; int * S = (int *) (q8 + nb * 64); float * yd = (float *) (S + nb * 8);
     double * red = (double *) (smem + BAMD_ACT_RED_OFF(nb));
     const float * xt = x + (size_t) t * K;
@@ -55,6 +56,28 @@ __global__ void __launch_bounds__(512) quantize_batch_kernel(const float * __res
         }
         float * oyd = (float *) (o + (size_t) nb * BAMD_B16_REC);
         for (int i = threadIdx.x; i < nb; i += blockDim.x) { oyd[i] = yd[i]; *(float *) (o + (size_t) i * BAMD_B16_REC + 560) = yd[i]; }   // d_y also inside the record (bamd_prefill2.hip: no separate copy)
+    }
+    if (frag) {
+        // the operands of bamd_prefill_wide.hip, by tiles of 16 tokens: [tile][super-block][e][g][token] x 16 bytes (sub-blocks 2g and 2g+1 of chunk e as f16), behind them
+        // d_y [tile][super-block][token] and the block sums [tile][super-block][pair l][token] as {S_2l & ~1, S_2l+1 & ~1, S_2l & 1, S_2l+1 & 1} in f16 (|S| <= 4064)
+        const size_t ntile = (gridDim.x + 15) / 16, tile = (size_t) (t >> 4) * nb;
+        const int m = t & 15;
+        uint8_t * dy = frag + ntile * nb * 8192, * mn = dy + ntile * nb * 64;
+        for (int i = threadIdx.x; i < nb * 32; i += blockDim.x) {
+            const uint32_t w0 = q8[2 * i], w1 = q8[2 * i + 1];
+            uint4 v;
+            auto two = [](uint32_t lo, uint32_t hi) { return (uint32_t) f2h((float) (int8_t) lo) | ((uint32_t) f2h((float) (int8_t) hi) << 16); };
+            v.x = two(w0, w0 >> 16); v.y = two(w0 >> 8, w0 >> 24); v.z = two(w1, w1 >> 16); v.w = two(w1 >> 8, w1 >> 24);      // bytes 0, 2, 1, 3: as masks take them out of a dword of quants
+            *(uint4 *) (frag + tile * 8192 + (size_t) i * 256 + m * 16) = v;      // i = (super-block, e, g)
+        }
+        for (int i = threadIdx.x; i < nb * 4; i += blockDim.x) {
+            const int ci = i >> 2, l = i & 3, sa = S[ci * 8 + 2 * l], sb = S[ci * 8 + 2 * l + 1];
+            uint2 v;
+            v.x = (uint32_t) f2h((float) (sa & ~1)) | ((uint32_t) f2h((float) (sb & ~1)) << 16);
+            v.y = (uint32_t) f2h((float) (sa & 1)) | ((uint32_t) f2h((float) (sb & 1)) << 16);
+            *(uint2 *) (mn + (tile + ci) * 512 + l * 128 + m * 8) = v;
+        }
+        for (int i = threadIdx.x; i < nb; i += blockDim.x) *(float *) (dy + (tile + i) * 64 + m * 4) = yd[i];
     }
 }
 
@@ -188,9 +211,9 @@ __global__ void __launch_bounds__(256) embed_batch_kernel(const int32_t * __rest
 // ---- batched prefill launchers ------------------------------------------------------------------------------------------
 size_t bamd_blob_bytes(int K) { return BAMD_BLOB_BYTES(K >> 8); }
 size_t bamd_blob16_bytes(int K) { return BAMD_BLOB16_BYTES(K >> 8); }
-void bamd_launch_quantize_batch(const float * x, const float * nw, float eps, int K, int T, void * blob, void * blob16, hipStream_t s) {
-    if (nw) hipLaunchKernelGGL((quantize_batch_kernel<true>),  dim3(T), dim3(512), act_lds_bytes(K), s, x, nw, eps, K, (uint8_t *) blob, (uint8_t *) blob16);
-    else    hipLaunchKernelGGL((quantize_batch_kernel<false>), dim3(T), dim3(512), act_lds_bytes(K), s, x, nw, eps, K, (uint8_t *) blob, (uint8_t *) blob16);
+void bamd_launch_quantize_batch(const float * x, const float * nw, float eps, int K, int T, void * blob, void * blob16, void * frag, hipStream_t s) {
+    if (nw) hipLaunchKernelGGL((quantize_batch_kernel<true>),  dim3(T), dim3(512), act_lds_bytes(K), s, x, nw, eps, K, (uint8_t *) blob, (uint8_t *) blob16, (uint8_t *) frag);
+    else    hipLaunchKernelGGL((quantize_batch_kernel<false>), dim3(T), dim3(512), act_lds_bytes(K), s, x, nw, eps, K, (uint8_t *) blob, (uint8_t *) blob16, (uint8_t *) frag);
 }
 int bamd_launch_matmul_batch(const bamd_mm_args & a, int epi, int n_cu, hipStream_t s) {
     int nrg = 0;

@@ -16,7 +16,7 @@
 //     super-block for Q4_K / Q5_K, 72 B for Q6_K: the MI355X has the HBM for it): the builders' per-(row, sub-block pair) scale operands
 //     {s, -1024 s, s'/16, -64 s'} as packed f16 pairs, and the consumers' d, dmin as f32 plus the min-term MFMA operands {2 m_a, 2 m_b, m_a, m_b}, which
 //     travel global -> LDS by DMA with the activation records;
-//   * two layouts: sixteen waves with one 16 x 16 tile each (matmul_mfma3_q4k_kernel: Q4_K / Q5_K), eight waves with 16 x 32 each (matmul_mfma2_q6k_kernel: Q6_K);
+//   * sixteen waves with one 16 x 16 tile each (matmul_mfma3_q4k_kernel: Q4_K / Q5_K), where the products of many tokens (bamd_prefill_wide.hip) would leave CUs idle;
 //     up to 64 tokens, where 64-row blocks leave the chip idle, 16-row blocks of specialised waves (matmul_few_kernel).
 // Same bits as those kernels (which are gone), a third fewer vector instructions per MFMA — and the same time: profiles/r06_prefill_ceiling.txt has
 // what bounds it and the timing-only ceiling builds (-DBAMD_PREFILL_CEILING).
@@ -38,23 +38,15 @@ struct bamd_mma2_args {
     unsigned long long * dbg;        // -DX_TIMING builds: per-wave phase clocks of workgroup (0, 0) (tools/prefill_phase.py); else unused
 };
 
-// LDS map (byte offsets).  Both copies of every region lie within 64 KiB of the region's first copy, so one base register per region
-// serves both buffers through the 16-bit offset field of the DS instructions (the buffer in use is a compile-time parity of the step).
+// LDS map of the sixteen-wave kernel (byte offsets), each region twice
 #define X_FR 1040                                          /* bytes between fragments: 1 KiB + 16 — the builder's 16-byte stores of eight lanes (one row, e = 0..7) then fall on eight
                                                               different bank quads (260 dwords = 4 mod 64); a fragment itself stays contiguous (lane * 16) for the consumers' ds_read_b128 */
 #define X_AF_BYTES (32 * X_FR)                             /* A fragments of one super-block: 4 row tiles x 8 fragments */
 #define X_BS_BYTES (64 * BAMD_B16_REC)                     /* 64 token records of one super-block (38 912 B) */
 #define X_CH4_RT 640                                       /* Q4_K / Q5_K consumer header of a row tile: 16 x d f32 | 16 x dmin f32 | 16 x 4 x 8 B of min operands */
 #define X_CH6_RT 64                                        /* Q6_K: 16 x d f32 */
-#define X_CH_MAX (4 * X_CH4_RT)
 #define X3_CHS 3072                                        /* Q4_K / Q5_K consumer headers of a row block and super-block in the side table: 4 x 640 B, padded to three DMA instructions */
-#define X_BLK (X_BS_BYTES + X_CH_MAX + 256 + 32)           /* records | headers | 64 d_y | 32 bytes of zeros: 41 760 B */
 #define X_AF0 0
-#define X_BLK0 (2 * X_AF_BYTES)
-#define X_LDS_BYTES (X_BLK0 + 2 * X_BLK)                   /* 149 056 B */
-#define X_CH_OFF X_BS_BYTES
-#define X_YD_OFF (X_BS_BYTES + X_CH_MAX)
-#define X_Z_OFF (X_YD_OFF + 256)
 
 // ---- load-time side tables ---------------------------------------------------------------------------------------------------
 // grid (super-blocks, row tiles incl. the padding tiles of the last row block), 64 threads = the MFMA lanes (m = row of the tile, g)
@@ -108,182 +100,9 @@ __global__ void __launch_bounds__(64) prefill_aux_q6k_kernel(const uint8_t * __r
     if (g == 0) *(float *) (ch + (((size_t) (rtile >> 2) * nb + ci) * 4 + (rtile & 3)) * X_CH6_RT + m * 4) = h2f(d16);
 }
 
-// ---- the activation / header stage: global -> LDS by DMA --------------------------------------------------------------------------
-// chunk list of a step (16 B each): 2432 chunks of token records (64 tokens x 38), then the NCH chunks of the row block's consumer headers;
-// wave-instruction k = 64 consecutive chunks; round r: instruction 8 r + wave.  Rounds 0..3 (and round 4 for waves 0..5) are records; round
-// 4 of waves 6, 7 and the tail instructions are headers (NCH = 160 for Q4_K / Q5_K: a half instruction on wave 0; 16 for Q6_K: lanes 0..15 of
-// wave 6); the 64 block scales d_y go as one 4-byte instruction on wave 1.
-template <int NCH>
-struct XStage {
-    uint32_t off[5]; uint32_t offx; bool x_on;
-    __device__ __forceinline__ void plan(int tid, int wave, int lane, int t0, int T, size_t b16, int nb) {
-        auto rec_off = [&](int idx) { const int tok = idx / BAMD_B16_Q, q = idx - tok * BAMD_B16_Q; const int tg = t0 + tok < T ? t0 + tok : T - 1; return (uint32_t) ((size_t) tg * b16 + (size_t) q * 16); };
-#pragma unroll
-        for (int r = 0; r < 4; ++r) off[r] = rec_off(r * 512 + tid);
-        off[4] = wave < 6 ? rec_off(2048 + tid) : (uint32_t) (tid - 384) * 16u;
-        if (NCH > 128) { offx = wave == 0 ? (uint32_t) (128 + lane) * 16u : 0u; x_on = wave == 0 && lane < NCH - 128; } else { offx = 0u; x_on = false; }
-        if (wave == 1) { const int tg = t0 + lane < T ? t0 + lane : T - 1; offx = (uint32_t) ((size_t) tg * b16 + (size_t) nb * BAMD_B16_REC); }
-    }
-    // recs = blob16 + ci * BAMD_B16_REC, hdrs = headers of (row block, ci), yds = blob16 + ci * 4; blk = LDS byte address of the block to fill
-    __device__ __forceinline__ void issue(const uint8_t * recs, const uint8_t * hdrs, const uint8_t * yds, uint32_t blk, int wave, int lane) const {
-        const uint32_t wdst = blk + (uint32_t) wave * 1024u;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) lds_dma16_s(recs, off[r], wdst + (uint32_t) r * 8192u);
-        if (wave < 6) lds_dma16_s(recs, off[4], wdst + 32768u);
-        else if (NCH >= 128 || (wave == 6 && lane < NCH)) lds_dma16_s(hdrs, off[4], wdst + 32768u);
-        if (NCH > 128 && x_on) lds_dma16_s(hdrs, offx, blk + X_CH_OFF + 2048u);
-        if (wave == 1) lds_dma4_s(yds, offx, blk + X_YD_OFF);
-    }
-};
-
 // ---- Q4_K / Q5_K: the sixteen-wave kernel further down (matmul_mfma3_q4k_kernel).  MFMA lane l = (m = l & 15, g = l >> 4): A row m, B token m, k-slots (g, i) =
 //      (sub-block 2g + (i >> 2), u = i & 3); C/D rows 4g + i, token m.  (An eight-wave layout of the same arithmetic — 16 x 32 per wave, 96 accumulators, two waves
 //      per SIMD — took 27.4 vs 25.4 ms per 512-token micro-batch, profiles/r06_prefill_ceiling.txt.)
-
-// ---- Q6_K: a step is HALF a super-block (four e: 16 MFMAs per wave, two per e and token tile) -----------------------------------------------
-// scale x (q - 32) reaches 4096: the scale is split sc = sa + sl (prefill_aux_q6k_kernel), both fragments come from one f16 image v = (1024 + q) - 1056
-// of the quants as v x sa and v x sl (exact), and the two MFMAs of an (e, token tile) are CHAINED through the accumulator: S = A_l.B + (A_a.B + 0)
-// is the exact integer isum (|isum| < 2^24, every partial sum an integer below that bound) — the fmaf(16, S_1, S_2) of bamd_prefill.hip is gone.
-// Scales are per 16 elements: for SIMD lane e the sub-block c uses scales[2c + (e >= 4)] (ggml-quants.c:8145-8216), i.e. the builder operands of a
-// half step are those of e-half h.  Fragment ring: two half steps x 4 row tiles x 4 e x 2 fragments x 1 KiB = 2 x 32 KiB; the activation stage
-// (whole super-blocks) is refilled every second half step.
-template <int EPI>
-__global__ void __launch_bounds__(512) matmul_mfma2_q6k_kernel(bamd_mma2_args a) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = wave_id(), m = lane & 15, g = lane >> 4;
-    const int rt = wave >> 1, tp = wave & 1;
-    const int nb = a.K >> 8;
-    const int rb = blockIdx.y, t0 = blockIdx.x * 64;
-    const int rtg = rb * 4 + rt;
-    const bool live = rtg * 16 < a.nrows_pad;
-    const size_t b16 = BAMD_BLOB16_BYTES(nb);
-    const uint32_t lds0 = (uint32_t) (size_t) (bamd_lds_vp) smem;
-    XStage<16> stg; stg.plan(tid, wave, lane, t0, a.T, b16, nb);
-    const uint8_t * chb = a.ch + (size_t) rb * nb * (4 * X_CH6_RT);
-#define X_STAGE(ci_, b_) stg.issue(a.blob16 + (size_t) (ci_) * BAMD_B16_REC, chb + (size_t) (ci_) * (4 * X_CH6_RT), a.blob16 + (size_t) (ci_) * 4, lds0 + X_BLK0 + (uint32_t) (b_) * X_BLK, wave, lane)
-    // builder (as in the Q4_K kernel: the stream's own rows, one record group per wave): wave (rt, q = tp), lane (p = lane >> 5, r = (lane >> 2) & 7, el = lane & 3)
-    // takes, per half step, chunk e = 4 H + el of row 8q + r and builds the pieces of MFMA lanes (8q + r, g = 2p + j), j = 0, 1: the ql dwords 2p, 2p + 1
-    // (sub-blocks 2g / 2g+1 sit in the low (j = 0) or high (j = 1) nibbles) and the qh dword p of stream lane (r, e).  Eight consecutive lanes = two rows x
-    // four fragments: their 16-byte stores fall on eight different bank quads (fragment pairs 2 x X_FR bytes apart).
-    const int bp = lane >> 5, br = (lane >> 2) & 7, bel = lane & 3;
-    const int rgq = 2 * (live ? rtg : rb * 4) + tp;
-    const int rgc = rgq * 8 < a.nrows_pad ? rgq : rgq - 1;
-    const uint8_t * wql = a.w + (size_t) rgc * nb * 1680 + (size_t) ((br * 8 + bel) * 16 + bp * 8);
-    const uint8_t * wqh = a.w + (size_t) rgc * nb * 1680 + 1024 + (size_t) ((br * 8 + bel) * 8 + bp * 4);
-    const uint8_t * phb = a.ph + (size_t) rb * nb * 8192 + (size_t) rt * 1024 + (size_t) ((2 * bp) * 256 + (8 * tp + br) * 16);
-    uint2 ql[2]; uint32_t qh[2]; uint4 sc[2][2];
-    auto load_set = [&](int hs, auto set_tag) {                // operands of half step hs = 2 ci + h
-        constexpr int S = decltype(set_tag)::value;
-        const int ci = hs >> 1, h = hs & 1;
-        ql[S] = *(const uint2 *) (wql + (size_t) ci * 1680 + h * 64);
-        qh[S] = *(const uint32_t *) (wqh + (size_t) ci * 1680 + h * 32);
-        sc[S][0] = *(const uint4 *) (phb + (size_t) hs * 4096); sc[S][1] = *(const uint4 *) (phb + (size_t) hs * 4096 + 256);
-    };
-    const bamd_h2 k1056 = { (_Float16) -1056.f, (_Float16) -1056.f };
-    bamd_h2u v0, v1, v2, v3;
-    auto build_a = [&](const uint2 & q, uint32_t hq, int j) {
-        // the two high bits of a quant sit at bits sh, sh + 1 (sub-block 2g) / sh + 2, sh + 3 (2g + 1) of their byte of hq (sh = 4 j) and belong at bits 4, 5:
-        // a ROTATION of the dword (what wraps around lands outside the mask 0x30 of every byte), then one and-or
-        const uint32_t sh = 4u * (uint32_t) j;
-        const uint32_t uA = (__builtin_amdgcn_alignbit(hq, hq, (28u + sh) & 31u) & 0x30303030u) | ((q.x >> sh) & 0x0f0f0f0fu);
-        const uint32_t uB = (__builtin_amdgcn_alignbit(hq, hq, (30u + sh) & 31u) & 0x30303030u) | ((q.y >> sh) & 0x0f0f0f0fu);
-        bamd_h2u c;
-        c.u = __builtin_amdgcn_perm(0x64646464u, uA, 0x04010400u); v0.h = c.h + k1056;      // (1024 + q) - 1056 = q - 32, exact
-        c.u = __builtin_amdgcn_perm(0x64646464u, uA, 0x04030402u); v1.h = c.h + k1056;
-        c.u = __builtin_amdgcn_perm(0x64646464u, uB, 0x04010400u); v2.h = c.h + k1056;
-        c.u = __builtin_amdgcn_perm(0x64646464u, uB, 0x04030402u); v3.h = c.h + k1056;
-    };
-    auto build_b = [&](const uint4 & s, unsigned char * dst) {  // dst: the A_a fragment; A_l X_FR bytes behind it
-        bamd_h2u sa0, sl0, sa1, sl1, x0, x1, x2, x3; sa0.u = s.x; sl0.u = s.y; sa1.u = s.z; sl1.u = s.w;
-        x0.h = v0.h * sa0.h; x1.h = v1.h * sa0.h; x2.h = v2.h * sa1.h; x3.h = v3.h * sa1.h;
-        *(uint4 *) dst = (uint4) { x0.u, x1.u, x2.u, x3.u };
-        x0.h = v0.h * sl0.h; x1.h = v1.h * sl0.h; x2.h = v2.h * sl1.h; x3.h = v3.h * sl1.h;
-        *(uint4 *) (dst + X_FR) = (uint4) { x0.u, x1.u, x2.u, x3.u };
-    };
-    unsigned char * afw = smem + X_AF0 + (rt * 4 + bel) * (2 * X_FR) + ((2 * bp) * 16 + 8 * tp + br) * 16;     // [row tile][e' = 0..3][a | l][X_FR]: MFMA lane (8 tp + br, 2 bp + j) at + j * 256
-    const unsigned char * afr = smem + X_AF0 + rt * 8 * X_FR + lane * 16;
-    const unsigned char * bop = smem + X_BLK0 + (size_t) ((2 * tp) * 16 + m) * BAMD_B16_REC + g * 16;
-    const unsigned char * chd = smem + X_BLK0 + X_CH_OFF + rt * X_CH6_RT + g * 16;                 // d of rows 4g .. 4g+3
-    const unsigned char * ydp = smem + X_BLK0 + X_YD_OFF + ((2 * tp) * 16 + m) * 4;
-    bamd_f4 acc[2][8];
-#pragma unroll
-    for (int n = 0; n < 2; ++n) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc[n][e] = (bamd_f4) { 0.f, 0.f, 0.f, 0.f };
-    }
-    X_STAGE(0, 0);
-    load_set(0, std::integral_constant<int, 0>());
-    load_set(1, std::integral_constant<int, 1>());
-#pragma unroll
-    for (int j = 0; j < 2; ++j) { build_a(ql[0], qh[0], j); build_b(sc[0][j], afw + j * 256); }
-    lds_dma_wait();
-    __syncthreads();
-    const int nhs = 2 * nb;
-    // half step hs = 2 ci + H: fragments in ring slot H, activation block ci & 1 = BLK
-    auto step = [&](const int hs, auto h_tag, auto blk_tag) {
-        constexpr int H = decltype(h_tag)::value, BLK = decltype(blk_tag)::value, NXT = H ^ 1;
-        const int ci = hs >> 1;
-        if (H == 0) X_STAGE(ci + 1 < nb ? ci + 1 : nb - 1, BLK ^ 1);                               // the next super-block's records: a whole step ahead
-        load_set(hs + 2 < nhs ? hs + 2 : nhs - 2 + H, std::integral_constant<int, H>());
-        __builtin_amdgcn_sched_barrier(0);
-        float D[2][4];
-        {
-            const bamd_f4 dw = *(const bamd_f4 *) (chd + BLK * X_BLK);
-#pragma unroll
-            for (int n = 0; n < 2; ++n) {
-                const float ydv = *(const float *) (ydp + BLK * X_BLK + n * 64);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) D[n][i] = ydv * dw[i];
-            }
-        }
-        bamd_h8 Aa[2], Al[2], Bq[2][2];
-#define X_LDA(e_, p_) (*(const bamd_h8 *) (afr + H * X_AF_BYTES + (e_) * (2 * X_FR) + (p_) * X_FR))
-#define X_LDB(e_, n_) (*(const bamd_h8 *) (bop + BLK * X_BLK + (n_) * (16 * BAMD_B16_REC) + (4 * H + (e_)) * 64))
-        Aa[0] = X_LDA(0, 0); Al[0] = X_LDA(0, 1); Bq[0][0] = X_LDB(0, 0); Bq[0][1] = X_LDB(0, 1);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            if (e + 1 < 4) { Aa[(e + 1) & 1] = X_LDA(e + 1, 0); Al[(e + 1) & 1] = X_LDA(e + 1, 1); Bq[(e + 1) & 1][0] = X_LDB(e + 1, 0); Bq[(e + 1) & 1][1] = X_LDB(e + 1, 1); }
-            if ((e & 1) == 0) build_a(ql[NXT], qh[NXT], e >> 1);
-#pragma unroll
-            for (int n = 0; n < 2; ++n) {
-                const bamd_f4 z = { 0.f, 0.f, 0.f, 0.f };
-                const bamd_f4 s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(Aa[e & 1], Bq[e & 1][n], z, 0, 0, 0);
-                const bamd_f4 s2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(Al[e & 1], Bq[e & 1][n], s1, 0, 0, 0);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) acc[n][4 * H + e][i] = fmaf(D[n][i], s2[i], acc[n][4 * H + e][i]);
-            }
-            if (e & 1) build_b(sc[NXT][e >> 1], afw + NXT * X_AF_BYTES + (e >> 1) * 256);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-#undef X_LDA
-#undef X_LDB
-        if (H == 1) lds_dma_wait();
-        __syncthreads();
-    };
-    for (int ci = 0; ci < nb; ci += 2) {
-        step(2 * ci, std::integral_constant<int, 0>(), std::integral_constant<int, 0>());
-        step(2 * ci + 1, std::integral_constant<int, 1>(), std::integral_constant<int, 0>());
-        if (ci + 1 < nb) {
-            step(2 * ci + 2, std::integral_constant<int, 0>(), std::integral_constant<int, 1>());
-            step(2 * ci + 3, std::integral_constant<int, 1>(), std::integral_constant<int, 1>());
-        }
-    }
-#undef X_STAGE
-    if (!live) return;
-#pragma unroll
-    for (int n = 0; n < 2; ++n) {
-        const int t = t0 + (2 * tp + n) * 16 + m;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float val = ((acc[n][0][i] + acc[n][4][i]) + (acc[n][2][i] + acc[n][6][i])) + ((acc[n][1][i] + acc[n][5][i]) + (acc[n][3][i] + acc[n][7][i]));
-            const int row = rtg * 16 + 4 * g + i;
-            if (t < a.T && row < a.nrows) {
-                const size_t o = (size_t) t * a.ldo + row;
-                a.out[o] = EPI == BAMD_EPI_ADD ? val + a.res[o] : EPI == BAMD_EPI_SILU_MUL ? v_silu(a.res[o]) * val : val;
-            }
-        }
-    }
-}
 
 // ==== sixteen waves ===========================================================================================================================
 // The eight-wave kernels above trade vector instructions for LDS traffic and end where those were (two waves per SIMD: a step is a chain of
@@ -794,7 +613,7 @@ void bamd_launch_prefill_aux(const void * w_stream, int type, int nrows_pad, int
 // the most dynamic LDS any launch below takes
 static constexpr size_t x_max_lds() {
     size_t m = few_lds(BAMD_Q6_K, 4);
-    for (const size_t v : { (size_t) X3_LDS_BYTES, (size_t) X_LDS_BYTES, few_lds(BAMD_Q4_K, 4), few_lds(BAMD_Q5_K, 4) }) m = v > m ? v : m;
+    for (const size_t v : { (size_t) X3_LDS_BYTES, few_lds(BAMD_Q4_K, 4), few_lds(BAMD_Q5_K, 4) }) m = v > m ? v : m;      // (bamd_prefill_wide.hip takes no more: asserted there)
     return m;
 }
 static bool x_takes(const void * kernel, size_t lds) { return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds) == hipSuccess; }
@@ -804,7 +623,7 @@ int bamd_prefill_mfma_supported(void) {
     int dev = 0, lds = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess) { (void) hipGetLastError(); return 0; }
     if ((size_t) lds < x_max_lds()) return 0;
-    if (!x_takes((const void *) matmul_mfma3_q4k_kernel<BAMD_EPI_STORE, false>, X3_LDS_BYTES) || !x_takes((const void *) matmul_mfma2_q6k_kernel<BAMD_EPI_STORE>, X_LDS_BYTES) ||
+    if (!x_takes((const void *) matmul_mfma3_q4k_kernel<BAMD_EPI_STORE, false>, X3_LDS_BYTES) || !bamd_wide_supported() ||
         !x_takes((const void *) matmul_few_kernel<BAMD_Q6_K, BAMD_EPI_STORE, 4>, few_lds(BAMD_Q6_K, 4))) { (void) hipGetLastError(); return 0; }
     return 1;
 }
@@ -825,9 +644,12 @@ static int x_few_tiles(int type, int nrows_pad, int nb, int T) {
     const long few = c.extra + (long) ((nrows_pad + 15) / 16 + 255) / 256 * (c.start[i] + (long) (line >= 48 && line <= 80 ? c.near_half : c.other)[i] * nb);
     return few < ((long) x_row_blocks(nrows_pad) + 255) / 256 * (c.start64 + (long) c.step64 * nb) ? i + 2 : 0;
 }
+int bamd_prefill_few_tiles(int type, int nrows_pad, int K, int T) { return x_few_tiles(type, nrows_pad, K >> 8, T); }
 size_t bamd_prefill_route(int type, int nrows_pad, int K, int T, int * few_tiles, size_t * most) {
     *few_tiles = x_few_tiles(type, nrows_pad, K >> 8, T); *most = x_max_lds();
-    return *few_tiles ? few_lds(type, *few_tiles) : type == BAMD_Q6_K ? X_LDS_BYTES : X3_LDS_BYTES;
+    if (*few_tiles) return few_lds(type, *few_tiles);
+    const int waves = bamd_prefill_tokfrag(type, nrows_pad, K, T);
+    return waves ? bamd_wide_lds(type, T, waves) : X3_LDS_BYTES;
 }
 int bamd_launch_matmul_mfma2(const void * w_stream, const void * aux, int type, int nrows, int nrows_pad, int K, const void * blob16, int T, float * out, const float * res,
                              int epi, int ldo, hipStream_t s) {
@@ -838,10 +660,6 @@ int bamd_launch_matmul_mfma2(const void * w_stream, const void * aux, int type, 
     a.out = out; a.res = res; a.blob16 = (const uint8_t *) blob16; a.K = K; a.T = T; a.nrows = nrows; a.nrows_pad = nrows_pad; a.ldo = ldo;
     a.dbg = g_prefill_dbg;
     const dim3 grid((T + 63) / 64, x_row_blocks(nrows_pad));
-#define X_LAUNCH(KERNEL, ...) do { \
-        if (epi == BAMD_EPI_ADD)           hipLaunchKernelGGL((KERNEL<BAMD_EPI_ADD __VA_ARGS__>),      grid, dim3(512), X_LDS_BYTES, s, a); \
-        else if (epi == BAMD_EPI_SILU_MUL) hipLaunchKernelGGL((KERNEL<BAMD_EPI_SILU_MUL __VA_ARGS__>), grid, dim3(512), X_LDS_BYTES, s, a); \
-        else                               hipLaunchKernelGGL((KERNEL<BAMD_EPI_STORE __VA_ARGS__>),    grid, dim3(512), X_LDS_BYTES, s, a); } while (0)
     const dim3 grid3(grid.x, BAMD_PREFILL_CEILING == 2 ? (grid.y + 1) / 2 : grid.y);     // (ceiling build 2: every workgroup issues the MFMAs of two; timing only)
 #define X3_LAUNCH(KERNEL, ...) do { \
         if (epi == BAMD_EPI_ADD)           hipLaunchKernelGGL((KERNEL<BAMD_EPI_ADD __VA_ARGS__>),      grid3, dim3(1024), X3_LDS_BYTES, s, a); \
@@ -860,10 +678,9 @@ int bamd_launch_matmul_mfma2(const void * w_stream, const void * aux, int type, 
 #undef XF_LAUNCH
         return 0;
     }
-    if (type == BAMD_Q6_K)      X_LAUNCH(matmul_mfma2_q6k_kernel);
+    if (type == BAMD_Q6_K)      return 1;                         // (bamd_prefill_wide.hip)
     else if (type == BAMD_Q5_K) X3_LAUNCH(matmul_mfma3_q4k_kernel, , true);
     else                        X3_LAUNCH(matmul_mfma3_q4k_kernel, , false);
 #undef X3_LAUNCH
-#undef X_LAUNCH
     return 0;
 }

@@ -344,3 +344,33 @@ def test_pipeline_prompt_phase_on_real_kernels(bamd, tmp_path):
                 bamd.set_prefill_batch(True)
                 st.close()
             assert fed[0] == want, "%d-token prompt, %s" % (n_prompt, mode)
+
+
+def test_long_prompts_in_one_batch(tmp_path):
+    """prompts of more than 512 tokens go through the layers up to 2048 at a time: the same bits as in portions of 512 (the one-token tail of n = 513, 1025, 2049 keeps its own
+    arithmetic), as on the integer-dot kernel, on top of cached tokens, and from a context whose buffers grew"""
+    import booster_amd as bamd
+    p = str(tmp_path / "m.gguf")
+    gguf.write_synthetic_llama(p, E=1024, H=8, Hkv=2, L=3, F=2560, V=512, theta=500000.0, seed=5, type_fn=lambda n, il: gguf.q4_k_m_type(n, il, 3))
+    m = bamd.Model(p)
+    long = bamd.Context(m, 4096)
+    for n in (513, 514, 1025, 1500, 2048, 2049, 3000):
+        toks = [(31 * i + 7 * n) % 512 for i in range(n)]
+        got = long.decode(toks, 0).copy()
+        c = bamd.Context(m, 4096)
+        for i in range(0, n, 512):
+            want = c.decode(toks[i:i + 512], i).copy()
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), n
+        tail = [(5 * i + n) % 512 for i in range(700)]
+        got = long.decode(tail, n).copy()
+        for i in range(0, 700, 512):
+            want = c.decode(tail[i:i + 512], n + i).copy()
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (n, "on top")
+        c.close()
+    bamd.set_prefill_batch(2)
+    try:
+        c = bamd.Context(m, 4096); want = c.decode(toks, 0).copy(); c.close()
+    finally:
+        bamd.set_prefill_batch(1)
+    assert np.array_equal(long.decode(toks, 0).view(np.uint32), want.view(np.uint32))
+    long.close(); m.close()

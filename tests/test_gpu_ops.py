@@ -266,6 +266,25 @@ def test_mul_mat_batch_few_tokens(bamd, po, t, nb, rows):
             assert_bits(got[i], ref + res[i] if res is not None else ref, "type %d nb %d rows %d T %d token %d" % (t, nb, rows, T, i))
 
 
+@pytest.mark.parametrize("t,impl", [(12, 4), (13, 4), (14, 4), (14, 5)])
+@pytest.mark.parametrize("nb,rows", [(1, 8), (2, 136), (3, 24), (8, 72), (9, 1000), (17, 40)])
+def test_mul_mat_batch_many_tokens(bamd, po, t, impl, nb, rows):
+    """16 rows and up to 64 tokens per wave, on eight and on four waves: fewer super-blocks than are copied ahead, whole and part octets of them (the min pass), a last tile of
+    eight rows, row tiles past the end, every edge of the token tiles; against the integer-dot kernel, the first and last token against the oracle"""
+    K = nb * 256
+    rng = np.random.default_rng(1700 * t + nb)
+    W = random_kquant_tensor(t, K, rows, rng)
+    for T in (1, 16, 17, 33, 48, 49, 64, 65, 97, 130):
+        X = (rng.standard_normal((T, K)) * 3).astype(np.float32)
+        res = rng.standard_normal((T, rows)).astype(np.float32) if T % 2 else None
+        got = bamd.op_mul_mat_batch(t, W, rows, K, X, residual=res, impl=impl)
+        want = bamd.op_mul_mat_batch(t, W, rows, K, X, residual=res, impl=0)
+        assert_bits(got, want, "type %d impl %d nb %d rows %d T %d" % (t, impl, nb, rows, T))
+        for i in {0, T - 1}:
+            ref = po.mul_mat_q(t, W, rows, K, X[i], nthreads=8)[0]
+            assert_bits(got[i], ref + res[i] if res is not None else ref, "type %d nb %d rows %d T %d token %d" % (t, nb, rows, T, i))
+
+
 def test_attention_long_context_eight_heads_per_kv_head(bamd, po):
     """the 70B head layout at a long context: gq = 8 -> four query heads per workgroup of the softmax + P.V launch (128 KB of probability rows in
     LDS at n_ctx 8192), the V^T ring over 125 blocks, a half block at the end (n_kv % 64 == 32)"""
