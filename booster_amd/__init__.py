@@ -55,6 +55,8 @@ def lib():
         L.bamd_n_ctx.argtypes = [vp]
         L.bamd_kv_cache_clear.argtypes = [vp]
         L.bamd_decode.argtypes = [vp, vp, ci, ci]
+        L.bamd_decode_logits.argtypes = [vp, vp, ci, ci, vp]
+        L.bamd_set_logits_readback.restype = None; L.bamd_set_logits_readback.argtypes = [vp, ci]
         L.bamd_get_logits.restype = C.POINTER(C.c_float); L.bamd_get_logits.argtypes = [vp]
         L.bamd_generate_greedy.argtypes = [vp, ci, ci, vp, C.POINTER(C.c_float)]
         L.bamd_kv_seq_rm.argtypes = [vp, ci, ci]; L.bamd_kv_seq_add.argtypes = [vp, ci, ci, ci]; L.bamd_kv_seq_div.argtypes = [vp, ci, ci, ci]
@@ -173,9 +175,10 @@ class Context:
     def decode(self, tokens, n_past):
         """llama_decode(llama_batch_get_one(tokens, n, n_past, 0)); returns the last token's logits."""
         t = np.ascontiguousarray(tokens, np.int32)
-        if lib().bamd_decode(self.h, _p(t), t.size, n_past) != 0:
+        out = np.empty(self.model.n_vocab, np.float32)
+        if lib().bamd_decode_logits(self.h, _p(t), t.size, n_past, _p(out)) != 0:
             raise BamdError(lib().bamd_last_error().decode())
-        return np.ctypeslib.as_array(lib().bamd_get_logits(self.h), shape=(self.model.n_vocab,)).copy()
+        return out
 
     def decode_batch(self, entries):
         """one batch: entries = [(sequence, tokens, wanted places)]; returns the wanted logits in order, [n, n_vocab]"""
@@ -185,7 +188,7 @@ class Context:
             t, w = np.ascontiguousarray(tokens, np.int32), np.ascontiguousarray(want, np.int32)
             keep += [t, w]
             a.seq, a.n_tokens, a.tokens, a.n_want, a.want = seq, t.size, t.ctypes.data, w.size, w.ctypes.data
-        out = np.zeros((n_want, self.model.n_vocab), np.float32)
+        out = np.empty((n_want, self.model.n_vocab), np.float32)
         _chk(lib().bamd_decode_batch(self.h, arr, len(entries), _p(out) if n_want else None))
         return out
 

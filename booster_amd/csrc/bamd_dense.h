@@ -40,6 +40,16 @@ struct bamd_residual_args {
     const float * gi;
     float * xo; void * h; int E, ldh;              // xo [rows][E]; h [rows][ldh], zero beyond E (null: not wanted)
 };
+// A decoding step between host and device without the copy engine.  The host leaves the step's descriptors in pinned memory (`in`); the step's first kernel embeds the tokens straight
+// from there and leaves the descriptors where the others read them, its last one writes the logits to pinned memory and then `done`
+#define BAMD_STEP_ROWS 64
+struct bamd_step_box {
+    struct { bamd_entry ent[BAMD_STEP_ROWS]; int32_t tok[BAMD_STEP_ROWS]; uint32_t serial; } in;
+    alignas(64) uint32_t done;
+};
+struct bamd_step_dev { bamd_entry * ent; int32_t * row_entry, * tokens, * want; uint32_t * count_serial; };      // count_serial: blocks that are done (0 between steps), serial of the step
+void bamd_launch_step_open(const bamd_step_box * box, int rows, const bamd_step_dev & d, const uint16_t * embd, const uint16_t * pos, float scale, int E, int V, float * x, hipStream_t s);
+void bamd_launch_step_close(const float * logits, size_t n, float * host, bamd_step_box * box, uint32_t * count_serial, hipStream_t s);      // n floats (0: only `done`)
 void bamd_launch_embed_rows(const bamd_batch_dev & b, const uint16_t * embd, const uint16_t * pos, float scale, int E, int V, float * x, hipStream_t s);
 void bamd_launch_residual_rows(int act, const bamd_batch_dev & b, const bamd_residual_args & a, hipStream_t s);
 int bamd_norm_threads(int n, int rows);            // threads of a block that norms one of so many rows of n

@@ -312,7 +312,7 @@ static int context_init(bamd_context * c, bamd_model * m, int n_ctx, int n_seq) 
         const size_t rows = BAMD_LOGIT_ROWS;
         if (dev_alloc(c->allocs, (void **) &c->logits, rows * m->V * 4) || dev_alloc(c->allocs, (void **) &c->co_err, 64)) return 1;
         HIPC(hipMemset(c->logits, 0, rows * m->V * 4)); HIPC(hipMemset(c->co_err, 0, 64));
-        HIPC(hipHostMalloc((void **) &c->logits_host, rows * m->V * 4 + 64));
+        HIPC(hipHostMalloc((void **) &c->logits_host, rows * m->V * 4 + 64, hipHostMallocCoherent));      // (written by a step's last kernel)
         memset(c->logits_host + m->V, 0, 64);
         if (m->rt->context_init(c)) return 1;
         HIPC(hipDeviceSynchronize());
@@ -346,7 +346,7 @@ static int context_init(bamd_context * c, bamd_model * m, int n_ctx, int n_seq) 
     HIPC(hipMemsetAsync(c->co_gran, 0, (size_t) m->H * m->hd * 8 + 64, c->stream));
     c->co_err = (uint32_t *) (c->co_gran + (size_t) m->H * m->hd);
     HIPC(hipMemsetAsync(c->logits, 0, (size_t) m->V * 4, c->stream));
-    HIPC(hipHostMalloc((void **) &c->logits_host, (size_t) m->V * 4 + 64));     // + the give-up words of the co-launch / engine kernels, read back with the logits
+    HIPC(hipHostMalloc((void **) &c->logits_host, (size_t) m->V * 4 + 64, hipHostMallocCoherent));     // + the give-up words of the co-launch / engine kernels, read back with the logits
     memset(c->logits_host + m->V, 0, 64);
     c->forced_cap = 4096; c->out_cap = n_ctx + 8;
     if (dev_alloc(c->allocs, (void **) &c->forced, (size_t) c->forced_cap * 4) || dev_alloc(c->allocs, (void **) &c->out_tokens, (size_t) c->out_cap * 4)) return 1;
@@ -891,7 +891,8 @@ static int co_gave_up(bamd_context * c) {
     memset(c->logits_host + c->m->V, 0, 32);
     return fail("co-launched attention + wo: a workgroup gave up waiting for the attention role (results invalid)");
 }
-extern "C" __attribute__((visibility("default"))) int bamd_decode(bamd_context * c, const int32_t * tokens, int n_tokens, int n_past) {
+// out: where the caller wants the logits (null: left for bamd_get_logits)
+static int decode_to(bamd_context * c, const int32_t * tokens, int n_tokens, int n_past, float * out) {
     bamd_model * m = c->m;
     if (!m->with_embd || !m->with_output) { fail("bamd_decode needs a stage that owns embedding and output"); return 1; }
     if (!tokens || n_tokens < 1) { fail("n_tokens out of range"); return 1; }
@@ -902,12 +903,11 @@ extern "C" __attribute__((visibility("default"))) int bamd_decode(bamd_context *
         const int32_t last = n_tokens - 1;
         const bamd_batch_entry e = { 0, n_tokens, tokens, 1, &last };
         c->logits_host_valid = false;
-        try { if (m->rt->decode_batch(c, &e, 1, nullptr, false)) return 1; }
+        float * to = !c->logits_readback ? nullptr : out ? out : c->logits_host;
+        try { if (m->rt->decode_batch(c, &e, 1, to, false)) return 1; }
         catch (const std::exception & ex) { return fail(std::string("decode: ") + ex.what()); }
-        if (!c->logits_readback) { c->status_pending = true; return 0; }
-        HIPC(hipMemcpyAsync(c->logits_host, c->logits, (size_t) m->V * 4, hipMemcpyDeviceToHost, c->stream));
-        HIPC(hipStreamSynchronize(c->stream));
-        c->logits_host_valid = true;
+        if (!to) c->status_pending = true;
+        else c->logits_host_valid = true;                           // (they pass through logits_host)
         return 0;
     }
     if (n_tokens > BAMD_PREFILL_CAP && g_prefill_batch) {
@@ -915,7 +915,7 @@ extern "C" __attribute__((visibility("default"))) int bamd_decode(bamd_context *
         int part = prefill_part(c, n_tokens, n_past);
         if (part < n_tokens) {
             for (int i = 0; i < n_tokens; i += part, part = prefill_part(c, n_tokens - i, n_past + i))
-                if (bamd_decode(c, tokens + i, part, n_past + i)) return 1;
+                if (decode_to(c, tokens + i, part, n_past + i, i + part < n_tokens ? nullptr : out)) return 1;
             return 0;
         }
     }
@@ -931,6 +931,7 @@ extern "C" __attribute__((visibility("default"))) int bamd_decode(bamd_context *
         if (enqueue_prefill_batch(c, n_tokens, n_past, s)) return 1;
         enqueue_lm_head(c, s, nullptr);                                  // n_outputs = 1: last token only (llama.cpp:14580-14593)
     } else if (n_tokens == 1) {
+        c->aql_gave = false;
         // single token: the captured stage-step graph (state and token are two small host copies, then one graph launch)
         if (bamd_stage_step(c, tokens[0], nullptr, n_past, nullptr, nullptr, 1, 0, s)) return 1;
     } else {
@@ -947,6 +948,12 @@ extern "C" __attribute__((visibility("default"))) int bamd_decode(bamd_context *
         if (le != hipSuccess) { fail(std::string("kernel launch failed: ") + hipGetErrorString(le)); return 1; }
     }
     c->logits_host_valid = c->logits_readback;
+    if (c->aql_gave) {                                              // a step of the own queue whose last kernel wrote the logits and the status words to the host
+        c->aql_gave = false;
+        if (co_gave_up(c)) return 1;
+        if (out) memcpy(out, c->logits_host, (size_t) m->V * 4);
+        return 0;
+    }
     if (c->logits_readback && hipMemcpyAsync(c->logits_host, c->logits, (size_t) m->V * 4, hipMemcpyDeviceToHost, s) != hipSuccess) { fail("D2H logits"); return 1; }
     if (status_readback(c, s) != hipSuccess) { fail("D2H co-launch status"); return 1; }
     if (!c->logits_readback) {
@@ -956,9 +963,18 @@ extern "C" __attribute__((visibility("default"))) int bamd_decode(bamd_context *
         c->status_pending = true;
         return 0;
     }
+    if (out) bamd_touch(out, (size_t) m->V);                        // while the device is at work
     hipError_t e = hipStreamSynchronize(s);
     if (e != hipSuccess) { fail(std::string("decode failed: ") + hipGetErrorString(e)); return 1; }
     if (co_gave_up(c)) return 1;
+    if (out) memcpy(out, c->logits_host, (size_t) m->V * 4);
+    return 0;
+}
+extern "C" __attribute__((visibility("default"))) int bamd_decode(bamd_context * c, const int32_t * tokens, int n_tokens, int n_past) { return decode_to(c, tokens, n_tokens, n_past, nullptr); }
+extern "C" __attribute__((visibility("default"))) int bamd_decode_logits(bamd_context * c, const int32_t * tokens, int n_tokens, int n_past, float * logits) {
+    if (!logits) return fail("bamd_decode_logits: no place for the logits");
+    if (decode_to(c, tokens, n_tokens, n_past, logits)) return 1;
+    if (!c->logits_readback) { const float * l = bamd_get_logits(c); if (!l) return 1; memcpy(logits, l, (size_t) c->m->V * 4); }
     return 0;
 }
 extern "C" __attribute__((visibility("default"))) int bamd_decode_batch(bamd_context * c, const bamd_batch_entry * entries, int n_entries, float * logits) {
@@ -1206,23 +1222,24 @@ extern "C" __attribute__((visibility("default"))) int bamd_stage_step(bamd_conte
     //      the bridge's token loop); layer-split stages, device-side tokens, shifted cells and prefill-mode steps keep the stage graphs below ----
     if (g_aql && !c->aql_failed && m->with_embd && m->with_output && !token_dev && !hidden_in_dev && !hidden_out_dev && want_logits && !prefill_mode &&
         !c->cells.active && s == c->stream && s != nullptr) {
-        const int fused = attn_fused_for(c, pos) ? 1 : 0;
+        const int fused = attn_fused_for(c, pos) ? 1 : 0, key = fused * 2 + (c->logits_readback ? 1 : 0);
         bool ok = fused == 1;
         if (!ok) { bamd_attn_args t; memset(&t, 0, sizeof t); t.hd = m->hd; t.Hkv = m->Hkv; t.n_ctx = c->n_ctx_pad; ok = bamd_attention_split_is_ik_clean(t, m->H / m->Hkv) != 0; }
         if (ok && !c->inbox && hipHostMalloc((void **) &c->inbox, sizeof(bamd_step_state)) != hipSuccess) { (void) hipGetLastError(); c->inbox = nullptr; ok = false; }
         if (ok) {
-            if (c->aql_step && c->aql_step_key != fused) { bamd_aql_free(c->aql_step); c->aql_step = nullptr; }
+            if (c->aql_step && c->aql_step_key != key) { bamd_aql_free(c->aql_step); c->aql_step = nullptr; }
             if (!c->aql_step) {
                 bamd_aql_recording rec;
                 bamd_aql_rec = &rec;
                 bamd_launch_step_begin(c->st, c->forced, 1, c->out_tokens, m->tok_embd.raw, m->tok_embd.type, m->E, m->V, c->x, 1, s, nullptr, nullptr, c->rope, c->rope_cur, m->hd, c->inbox);
                 const int rc = enqueue_layers(c, 0, s, nullptr, pos);
                 enqueue_lm_head(c, s, nullptr);
+                if (c->logits_readback) bamd_launch_logits_out(c->logits, c->logits_host, m->V, c->co_err, s);
                 bamd_aql_rec = nullptr;
                 const char * why = "recording failed";
                 if (!rc) c->aql_step = bamd_aql_build(m->device, rec, &why);
                 if (!c->aql_step) { c->aql_failed = true; if (getenv("BAMD_AQL_VERBOSE")) fprintf(stderr, "bamd: own AQL queue not used: %s\n", why ? why : "?"); }
-                c->aql_step_key = fused;
+                c->aql_step_key = key;
             }
         }
         if (ok && c->aql_step) {
@@ -1235,6 +1252,7 @@ extern "C" __attribute__((visibility("default"))) int bamd_stage_step(bamd_conte
             const char * why = nullptr;
             if (bamd_aql_run(c->aql_step, 1, nullptr, &why)) return fail(std::string("own AQL queue: ") + (why ? why : "?"));
             c->aql_steps += 1;
+            c->aql_gave = c->logits_readback;
             return 0;
         }
     }

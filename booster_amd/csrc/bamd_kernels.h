@@ -77,6 +77,7 @@ void bamd_launch_matvec(const bamd_mv_args & a, int pro, int epi, int n_cu, hipS
 void bamd_launch_step_begin(bamd_step_state * st, const int32_t * forced, int n_forced, int32_t * out_tokens, const void * embd,
                             int embd_type, int E, int V, float * x, int do_embed, hipStream_t s, const int32_t * slots = nullptr, int32_t * cellpos = nullptr,
                             const float * rope = nullptr, float * rope_cur = nullptr, int hd = 0, const bamd_step_state * inbox = nullptr);
+void bamd_launch_logits_out(const float * logits, float * host, int V, const uint32_t * status, hipStream_t s);      // V logits and the eight status words behind them to pinned memory
 int  bamd_launch_attention(const bamd_attn_args & a, int gq, int max_tiles, hipStream_t s);
 int  bamd_attention_split_is_ik_clean(const bamd_attn_args & a, int gq);      // the long-sequence path of this shape keeps the inter-kernel rules (bamd_device.h): own-queue replay allowed
 // single-launch attention and the wo projection (+ residual) behind it in ONE launch (bamd_colaunch.hip); gran: [H * hd] zero-initialised 8-byte

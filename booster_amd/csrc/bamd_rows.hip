@@ -5,16 +5,44 @@
 #include <algorithm>
 
 // block (1024 columns, row)
-__global__ void __launch_bounds__(256) embed_rows_kernel(bamd_batch_dev b, const uint16_t * __restrict__ embd, const uint16_t * __restrict__ pos, float scale, int E, int V, float * __restrict__ x) {
-    const int row = blockIdx.y, i0 = blockIdx.x * 1024 + threadIdx.x * 4;
-    int t = b.tokens[row]; t = t < 0 ? 0 : t >= V ? V - 1 : t;
-    const bamd_entry e = b.ent[b.row_entry[row]];
-    const int p = e.pos0 + (row - e.row0);
+__device__ __forceinline__ void embed_piece(int row, int t, int p, const uint16_t * __restrict__ embd, const uint16_t * __restrict__ pos, float scale, int E, int V, float * __restrict__ x) {
+    const int i0 = blockIdx.x * 1024 + threadIdx.x * 4;
+    t = t < 0 ? 0 : t >= V ? V - 1 : t;
     const uint16_t * er = embd + (size_t) t * E, * pr = pos ? pos + (size_t) p * E : nullptr;
     if (i0 + 3 < E && (E & 3) == 0) {
         const uint2 u = *(const uint2 *) (er + i0), w = pr ? *(const uint2 *) (pr + i0) : uint2{ 0, 0 };
         *(bamd_v4 *) (x + (size_t) row * E + i0) = bamd_v4{ bf_lo(u.x) * scale + bf_lo(w.x), bf_hi(u.x) * scale + bf_hi(w.x), bf_lo(u.y) * scale + bf_lo(w.y), bf_hi(u.y) * scale + bf_hi(w.y) };
     } else for (int i = i0; i < min(i0 + 4, E); ++i) x[(size_t) row * E + i] = bf_f(er[i]) * scale + (pr ? bf_f(pr[i]) : 0.f);
+}
+__global__ void __launch_bounds__(256) embed_rows_kernel(bamd_batch_dev b, const uint16_t * __restrict__ embd, const uint16_t * __restrict__ pos, float scale, int E, int V, float * __restrict__ x) {
+    const int row = blockIdx.y;
+    const bamd_entry e = b.ent[b.row_entry[row]];
+    embed_piece(row, b.tokens[row], e.pos0 + (row - e.row0), embd, pos, scale, E, V, x);
+}
+__device__ __forceinline__ int32_t box_ld(const int32_t * p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
+// The step's descriptors and tokens come out of host memory here: a copy engine in front of the step, and one behind it, were 40 us of a token's 465 (width 2048).  Every block reads
+// its own token (two independent reads over the bus), the first one the descriptors of all rows
+__global__ void __launch_bounds__(256) step_open_kernel(const bamd_step_box * box, bamd_step_dev d, const uint16_t * __restrict__ embd, const uint16_t * __restrict__ pos, float scale, int E, int V, float * __restrict__ x) {
+    const int row = blockIdx.y, tid = threadIdx.x;
+    embed_piece(row, box_ld(&box->in.tok[row]), pos ? box_ld(&box->in.ent[row].pos0) : 0, embd, pos, scale, E, V, x);
+    if (blockIdx.x || row) return;
+    const int n = gridDim.y, words = n * (int) (sizeof(bamd_entry) / 4);
+    for (int i = tid; i < words; i += 256) ((int32_t *) d.ent)[i] = box_ld((const int32_t *) box->in.ent + i);
+    for (int i = tid; i < n; i += 256) { d.tokens[i] = box_ld(&box->in.tok[i]); d.row_entry[i] = i; d.want[i] = i; }
+    if (tid == 0) d.count_serial[1] = (uint32_t) box_ld((const int32_t *) &box->in.serial);
+}
+// n floats to host memory; the block that ends last tells the host.  Every thread's stores are out before its block counts
+__global__ void __launch_bounds__(256) step_close_kernel(const float * __restrict__ logits, size_t n, float * __restrict__ host, uint32_t * done, uint32_t * count_serial) {
+    const size_t stride = (size_t) gridDim.x * 256, i0 = (size_t) blockIdx.x * 256 + threadIdx.x;
+    for (size_t i = i0; i < n / 4; i += stride) *(bamd_v4 *) (host + i * 4) = *(const bamd_v4 *) (logits + i * 4);
+    for (size_t i = n / 4 * 4 + i0; i < n; i += stride) host[i] = logits[i];
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x) return;
+    if (__hip_atomic_fetch_add(count_serial, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1 < gridDim.x) return;
+    count_serial[0] = 0;
+    __threadfence_system();
+    __hip_atomic_store(done, count_serial[1], __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 template <typename T> __global__ void __launch_bounds__(1024) residual_rows_kernel(bamd_batch_dev b, bamd_residual_args a) {
     __shared__ float red[64];
@@ -80,6 +108,14 @@ int bamd_norm_threads(int n, int rows) { return (n & 3) && rows <= 512 ? (int) r
 static dim3 sum_block(int n, int rows) { return dim3(bamd_norm_threads(n, rows)); }
 void bamd_launch_embed_rows(const bamd_batch_dev & b, const uint16_t * embd, const uint16_t * pos, float scale, int E, int V, float * x, hipStream_t s) {
     hipLaunchKernelGGL(embed_rows_kernel, dim3((E + 1023) / 1024, b.rows), dim3(256), 0, s, b, embd, pos, scale, E, V, x);
+}
+void bamd_launch_step_open(const bamd_step_box * box, int rows, const bamd_step_dev & d, const uint16_t * embd, const uint16_t * pos, float scale, int E, int V, float * x, hipStream_t s) {
+    hipLaunchKernelGGL(step_open_kernel, dim3((E + 1023) / 1024, rows), dim3(256), 0, s, box, d, embd, pos, scale, E, V, x);
+}
+// a block per 4096 floats, up to 128: a row of 32 000 goes out at the bus's rate
+void bamd_launch_step_close(const float * logits, size_t n, float * host, bamd_step_box * box, uint32_t * count_serial, hipStream_t s) {
+    const size_t blocks = (n + 4095) / 4096;
+    hipLaunchKernelGGL(step_close_kernel, dim3((unsigned) (blocks < 1 ? 1 : blocks > 128 ? 128 : blocks)), dim3(256), 0, s, logits, n, host, &box->done, count_serial);
 }
 void bamd_launch_residual_rows(int act, const bamd_batch_dev & b, const bamd_residual_args & a, hipStream_t s) {
     if (a.norm == BAMD_NORM_LAYER) {

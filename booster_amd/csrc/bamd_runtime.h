@@ -94,7 +94,7 @@ struct bamd_context {
     hipStream_t stream = nullptr;
     hipGraphExec_t graph = nullptr; int graph_fused = -1;
     bamd_aql_graph * aql = nullptr; int aql_key = -1; bool aql_failed = false; int aql_runs = 0;    // the same step as AQL packets for the own queue (bamd_aql.h)
-    bamd_aql_graph * aql_step = nullptr; int aql_step_key = -1; int aql_steps = 0;                 // bamd_stage_step's single-token step on the own queue
+    bamd_aql_graph * aql_step = nullptr; int aql_step_key = -1; int aql_steps = 0; bool aql_gave = false;                // bamd_stage_step's single-token step on the own queue
     bamd_step_state * inbox = nullptr;           // pinned host memory: the state of that step, read by step_begin_kernel itself (no copy in front of the step)
     unsigned long long * co_gran = nullptr;   // co-launch granules [H * hd] {value, tag} + give-up counter behind them (bamd_colaunch.hip), zero-initialised
     uint32_t * co_err = nullptr;
@@ -118,6 +118,8 @@ struct bamd_context {
     std::vector<void *> allocs;
 };
 
+// fresh memory is given its pages here (a fault per 4 KiB: 130 us for sixteen rows of 32 000 logits), in time that the host would wait for the device
+static inline void bamd_touch(float * p, size_t n) { for (size_t i = 0; i < n; i += 1024) ((volatile float *) p)[i] = 0.f; if (n) ((volatile float *) p)[n - 1] = 0.f; }
 static inline int dev_alloc(std::vector<void *> & keep, void ** p, size_t bytes) {
     HIPC(hipMalloc(p, bytes + 4096));           // + 4 KiB: the sixteen-wave prefill kernel's nibble loads of the two super-blocks behind the end of K run past
                                                 // the last record group (bamd_prefill2.hip)

@@ -12,6 +12,7 @@
 #include "bamd_stack.h"
 
 #include <algorithm>
+#include <chrono>
 #include <fstream>
 #include <iterator>
 #include <map>
@@ -173,6 +174,7 @@ struct Stack : bamd_arch_runtime {
     const char * vocab_path() override { return vocab.c_str(); }
 };
 
+static_assert(BAMD_STEP_ROWS <= BAMD_LOGIT_ROWS, "a step's rows fit the logit rows");
 struct Seq { int len = 0, par = 0; std::vector<int32_t> pages; };
 struct Timer {                                     // per-launch HIP events (profile_kinds)
     std::vector<hipEvent_t> ev; std::vector<int> kind; std::vector<double> bytes;
@@ -201,7 +203,8 @@ struct Ctx {
     unsigned char * dev = nullptr; int32_t * pages = nullptr;
     static constexpr int RING = 4;
     unsigned char * host[RING] = {}; int32_t * pages_host[RING] = {}; hipEvent_t ev[RING] = {}; int ring = 0;
-    std::map<int, hipGraphExec_t> graphs;          // rows * 2 + greedy
+    std::map<int, hipGraphExec_t> graphs;          // rows * 4 + what is in front and behind (STEP_*)
+    bamd_step_box * box = nullptr; uint32_t * count_serial = nullptr; uint32_t serial = 0;      // decoding steps by way of pinned memory; serial: of the last one
 };
 struct Pass {                                      // one pass through the layers
     Ctx & c; Stack & st; hipStream_t s; bamd_batch_dev b; bool decode = false;
@@ -600,12 +603,17 @@ int Stack::context_init(bamd_context * bc) {
         HIPC(hipHostMalloc((void **) &c.host[i], y.total)); HIPC(hipHostMalloc((void **) &c.pages_host[i], (size_t) S * c.max_pages * 4));
         HIPC(hipEventCreateWithFlags(&c.ev[i], hipEventDisableTiming));
     }
+    HIPC(hipHostMalloc((void **) &c.box, sizeof(bamd_step_box), hipHostMallocCoherent));
+    memset(c.box, 0, sizeof(bamd_step_box));
+    if (dev_alloc(bc->allocs, (void **) &c.count_serial, 8)) return 1;
+    HIPC(hipMemset(c.count_serial, 0, 8));
     return 0;
 }
 void Stack::context_free(bamd_context * bc) {
     Ctx * c = (Ctx *) bc->arch_state;
     if (!c) return;
     for (auto & g : c->graphs) hipGraphExecDestroy(g.second);
+    if (c->box) hipHostFree(c->box);
     for (int i = 0; i < Ctx::RING; ++i) { if (c->host[i]) hipHostFree(c->host[i]); if (c->pages_host[i]) hipHostFree(c->pages_host[i]); if (c->ev[i]) hipEventDestroy(c->ev[i]); }
     for (void * p : { c->kc, c->kk, c->kv, (void *) c->filtered, (void *) c->steps, (void *) c->alpha, (void *) c->seg_state, (void *) c->seg_decay }) if (p) hipFree(p);
     delete c;
@@ -775,6 +783,12 @@ int Pass::head(const int32_t * want, int n, float * logits) {
 // a piece of a batch entry in one pass
 struct Piece { int seq, n; const int32_t * tokens; };
 
+int send_pages(Ctx & c, int r, hipStream_t s) {
+    for (size_t i = 0; i < c.seqs.size(); ++i) std::copy(c.seqs[i].pages.begin(), c.seqs[i].pages.end(), c.pages_host[r] + i * c.max_pages);
+    HIPC(hipMemcpyAsync(c.pages, c.pages_host[r], c.seqs.size() * (size_t) c.max_pages * 4, hipMemcpyHostToDevice, s));
+    c.pages_dirty = false;
+    return 0;
+}
 // fills the step descriptors of a pass and sends them; want: rows of the pass
 int send(Pass & p, const std::vector<Piece> & pc, const std::vector<int32_t> & want) {
     Ctx & c = p.c;
@@ -819,11 +833,7 @@ int send(Pass & p, const std::vector<Piece> & pc, const std::vector<int32_t> & w
     }
     memcpy(h + c.lay.want, want.data(), want.size() * 4);
     HIPC(hipMemcpyAsync(c.dev, h, c.lay.total, hipMemcpyHostToDevice, p.s));
-    if (c.pages_dirty) {
-        for (size_t i = 0; i < c.seqs.size(); ++i) std::copy(c.seqs[i].pages.begin(), c.seqs[i].pages.end(), c.pages_host[r] + i * c.max_pages);
-        HIPC(hipMemcpyAsync(c.pages, c.pages_host[r], c.seqs.size() * (size_t) c.max_pages * 4, hipMemcpyHostToDevice, p.s));
-        c.pages_dirty = false;
-    }
+    if (c.pages_dirty && send_pages(c, r, p.s)) return 1;
     HIPC(hipEventRecord(c.ev[r], p.s));
     p.b = { (bamd_entry *) (c.dev + c.lay.ent), (int32_t *) (c.dev + c.lay.row), (int32_t *) (c.dev + c.lay.tok), (int) pc.size(), rows, c.c->n_seq, c.pages, c.max_pages };
     p.k_rows = kb * BAMD_PAGE; p.n_tiles = nt; p.n_segs = ns;
@@ -832,18 +842,59 @@ int send(Pass & p, const std::vector<Piece> & pc, const std::vector<int32_t> & w
 }
 int embed(Pass & p) { bamd_launch_embed_rows(p.b, p.st.embd, p.st.pos, p.st.scale, p.st.E, p.st.V, p.x, p.s); return 0; }
 
-// decoding rows -> logits of every row, as a graph (greedy: the loop's token hand-over in front, the arg-max behind)
-int decode_rows(Pass & p, bool greedy) {
+// waits until a step has written its logits and no longer reads its descriptors; a wait that gets long goes on in the runtime.  must: a step that never ran is an error
+int step_done(Ctx & c, uint32_t serial, bool must) {
+    auto there = [&] { return (int32_t) (__atomic_load_n(&c.box->done, __ATOMIC_ACQUIRE) - serial) >= 0; };
+    const auto t0 = std::chrono::steady_clock::now();
+    for (int i = 0; !there(); ++i) {
+        __builtin_ia32_pause();
+        if ((i & 255) == 255 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(5)) {
+            HIPC(hipStreamSynchronize(c.c->stream));
+            return there() || !must ? 0 : fail("decoding step: the device did not finish it");
+        }
+    }
+    return 0;
+}
+// the descriptors of a decoding step (rows of one token each, every row's logits wanted) left for step_open_kernel
+int leave(Pass & p, const std::vector<Piece> & pc) {
+    Ctx & c = p.c;
+    if (step_done(c, c.serial, false)) return 1;                   // (a step that nobody waited for may still read the last ones)
+    for (size_t e = 0; e < pc.size(); ++e) {
+        Seq & q = c.seqs[(size_t) pc[e].seq];
+        c.box->in.ent[e] = { pc[e].seq, (int32_t) e, 1, q.len, q.par, 0 };
+        c.box->in.tok[e] = pc[e].tokens[0];
+    }
+    c.box->in.serial = ++c.serial;
+    __atomic_thread_fence(__ATOMIC_RELEASE);
+    p.max_n = 1;
+    if (c.pages_dirty) {
+        const int r = c.ring; c.ring = (c.ring + 1) % Ctx::RING;
+        HIPC(hipEventSynchronize(c.ev[r]));
+        if (send_pages(c, r, p.s)) return 1;
+        HIPC(hipEventRecord(c.ev[r], p.s));
+    }
+    p.b = { (bamd_entry *) (c.dev + c.lay.ent), (int32_t *) (c.dev + c.lay.row), (int32_t *) (c.dev + c.lay.tok), (int) pc.size(), (int) pc.size(), c.c->n_seq, c.pages, c.max_pages };
+    p.x = c.xa; p.xo = c.xb; p.pend = nullptr; p.ldp = 0; p.pend_g = nullptr; p.pend_parts = 1;
+    return 0;
+}
+// decoding rows -> logits of every row, as a graph.  STEP_GREEDY: the loop's token hand-over in front, the arg-max behind; STEP_HOST: descriptors from the box, logits to the host;
+// STEP_DEVICE: descriptors from the box, logits where they are
+enum { STEP_HOST = 0, STEP_DEVICE = 1, STEP_GREEDY = 2 };
+int decode_rows(Pass & p, int kind) {
     Ctx & c = p.c;
     const int n = p.b.rows;
+    const bool greedy = kind == STEP_GREEDY;
     auto enqueue = [&]() -> int {
         if (greedy) bamd_launch_advance((bamd_entry *) p.b.ent, (int32_t *) p.b.tokens, c.keys, n, c.gen_out, c.gen_cap, c.step, 1, p.st.V, p.s);
-        if (embed(p) || p.layers() || p.head((const int32_t *) (c.dev + c.lay.want), n, c.c->logits)) return 1;
+        if (greedy) embed(p);
+        else bamd_launch_step_open(c.box, n, { (bamd_entry *) p.b.ent, (int32_t *) p.b.row_entry, (int32_t *) p.b.tokens, (int32_t *) (c.dev + c.lay.want), c.count_serial }, p.st.embd, p.st.pos, p.st.scale, p.st.E, p.st.V, p.x, p.s);
+        if (p.layers() || p.head((const int32_t *) (c.dev + c.lay.want), n, c.c->logits)) return 1;
         if (greedy) bamd_launch_argmax_rows(c.c->logits, n, p.st.V, c.keys, false, p.s);
+        else bamd_launch_step_close(c.c->logits, kind == STEP_HOST ? (size_t) n * p.st.V : 0, c.c->logits_host, c.box, c.count_serial, p.s);
         return 0;
     };
     if (!g_graph) return enqueue();
-    const int key = n * 2 + (greedy ? 1 : 0);
+    const int key = n * 4 + kind;
     auto it = c.graphs.find(key);
     if (it == c.graphs.end()) {
         hipGraph_t g = nullptr; hipGraphExec_t ex = nullptr;
@@ -905,27 +956,32 @@ int Stack::decode_batch(bamd_context * bc, const bamd_batch_entry * e, int n, fl
             add(i, from, cnt, false);
             from += cnt;
         }
+    bool idle = false, touched = false;                             // everything enqueued has been waited for; the caller's rows are backed by memory
     for (Plan & pl : plans) {
         Pass p{ c, *this, bc->stream, {}, pl.decode };
-        const bool graph = pl.decode && pl.rows <= BAMD_LOGIT_ROWS && !pl.want.empty();
-        std::vector<int32_t> rows = pl.want;
-        if (graph) { rows.resize((size_t) pl.rows); for (int i = 0; i < pl.rows; ++i) rows[(size_t) i] = i; }
-        if (send(p, pl.pc, rows)) return 1;
-        if (graph) { if (decode_rows(p, false)) return 1; }
+        const bool graph = pl.decode && pl.rows <= BAMD_STEP_ROWS && !pl.want.empty();
+        if (graph ? leave(p, pl.pc) : send(p, pl.pc, pl.want)) return 1;
+        if (graph) { if (decode_rows(p, logits ? STEP_HOST : STEP_DEVICE)) return 1; }
         else if (embed(p) || p.layers()) return 1;
+        idle = false;
         moved(c, pl.pc);
         for (size_t w = 0; w < pl.want.size(); w += BAMD_LOGIT_ROWS) {
             const int k = (int) std::min<size_t>(BAMD_LOGIT_ROWS, pl.want.size() - w);
             if (!graph && p.head((const int32_t *) (c.dev + c.lay.want) + w, k, bc->logits)) return 1;
             if (!logits) continue;                                  // the last rows stay in c->logits
-            const int back = graph ? pl.rows : k;
-            HIPC(hipMemcpyAsync(bc->logits_host, bc->logits, (size_t) back * V * 4, hipMemcpyDeviceToHost, bc->stream));
-            HIPC(hipStreamSynchronize(bc->stream));
-            for (int i = 0; i < k; ++i) memcpy(logits + pl.dst[w + (size_t) i] * V, bc->logits_host + (size_t) (graph ? pl.want[w + (size_t) i] : i) * V, (size_t) V * 4);
+            if (!graph) HIPC(hipMemcpyAsync(bc->logits_host, bc->logits, (size_t) k * V * 4, hipMemcpyDeviceToHost, bc->stream));
+            if (!touched && logits != bc->logits_host) bamd_touch(logits, n_want * V);      // while the device is at work
+            touched = true;
+            if (graph) { if (step_done(c, c.serial, true)) return 1; } else HIPC(hipStreamSynchronize(bc->stream));
+            idle = true;
+            for (int i = 0; i < k; ++i) {
+                float * to = logits + pl.dst[w + (size_t) i] * V; const float * from = bc->logits_host + (size_t) (graph ? pl.want[w + (size_t) i] : i) * V;
+                if (to != from) memcpy(to, from, (size_t) V * 4);
+            }
         }
         HIPC(hipGetLastError());
     }
-    if (wait) HIPC(hipStreamSynchronize(bc->stream));
+    if (wait && !idle) HIPC(hipStreamSynchronize(bc->stream));
     return 0;
 }
 
@@ -962,7 +1018,7 @@ int Stack::generate(bamd_context * bc, const int32_t * seqs, int n, int n_steps,
     if (hipEventCreate(&b) != hipSuccess) { hipEventDestroy(a); return fail("hipEventCreate"); }
     int rc = 0;
     hipEventRecord(a, s);
-    for (int t = 0; t < n_steps && !rc; ++t) rc = decode_rows(p, true);
+    for (int t = 0; t < n_steps && !rc; ++t) rc = decode_rows(p, STEP_GREEDY);
     hipEventRecord(b, s);
     if (!rc) {
         for (const Piece & q : pc) { c.seqs[(size_t) q.seq].len += n_steps; c.seqs[(size_t) q.seq].par ^= n_steps & 1; }

@@ -61,6 +61,8 @@ void           bamd_kv_cache_clear(bamd_context * c);                   /* llama
  * Returns 0, or 1 on failure like llama_decode. */
 int           bamd_decode(bamd_context * c, const int32_t * tokens, int n_tokens, int n_past);
 const float * bamd_get_logits(bamd_context * c);                        /* llama_get_logits: host, n_vocab floats */
+/* bamd_decode + a copy of bamd_get_logits into n_vocab floats of the caller's (their pages are touched while the device is at work) */
+int           bamd_decode_logits(bamd_context * c, const int32_t * tokens, int n_tokens, int n_past, float * logits);
 
 /* llama_decode on a llama_batch of several sequences: every entry's tokens run behind what its sequence already holds (none: from position 0), all entries as
  * one batch.  want: ascending places among the entry's tokens whose logits are asked for; `logits` (host, may be NULL) receives them in order, n_vocab floats each. */

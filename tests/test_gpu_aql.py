@@ -81,6 +81,23 @@ def test_single_token_decode_steps_on_the_own_queue(bamd):
     assert np.array_equal(bits(res[True][0]), bits(res[False][0]))
 
 
+@pytest.mark.parametrize("name", ["tiny_a", "tiny_b"])
+def test_steps_on_the_own_queue_read_or_not(bamd, name):
+    """the step that writes its logits to the host itself, and the one that leaves them on the device, in turn: the same bits"""
+    m = bamd.Model(os.path.join(GOLDEN, name + ".gguf")); ctx = bamd.Context(m, 128)
+    prompt = [5, 9, 2, 77, 31, 8, 1, 40]
+    ctx.decode(prompt, 0)
+    want = [ctx.decode([3 + i], 8 + i) for i in range(12)]
+    ctx.decode(prompt, 0)
+    try:
+        for i in range(12):
+            bamd.lib().bamd_set_logits_readback(ctx.h, int(i % 3 == 0))
+            got = ctx.decode([3 + i], 8 + i)
+            assert np.array_equal(bits(got), bits(want[i])) and np.array_equal(bits(ctx.last_logits()), bits(want[i])), i
+    finally:
+        bamd.lib().bamd_set_logits_readback(ctx.h, 1)
+
+
 def test_many_replays_across_the_ring_wrap(bamd):
     """the queue's ring holds 16384 packets: 400 greedy calls of 20 steps on the tiny model write ~ 5 x that, one doorbell never spanning the wrap (bamd_aql.cpp)"""
     path = os.path.join(GOLDEN, "tiny_a.gguf")

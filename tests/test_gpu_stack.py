@@ -32,6 +32,11 @@ def near(a, b, dtype, f=1.0):
     assert np.isfinite(a).all() and e.max() < f * TOL[dtype], "worst row %s: %.3g" % (np.unravel_index(e.argmax(), e.shape), e.max())
 
 
+def bamd_lib():
+    import booster_amd
+    return booster_amd.lib()
+
+
 # ---- mechanisms alone --------------------------------------------------------------------------------------------------------------------------------------
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("n,k,rows", [(1, 1, 1), (17, 31, 3), (130, 33, 64), (300, 75, 16), (48, 600, 17), (513, 96, 33), (260, 288, 65), (1100, 320, 500), (2050, 160, 1500)])
@@ -492,6 +497,33 @@ def test_decode_interface(run):
         c.kv_seq_rm(10, -1)
     c.kv_seq_rm(0, -1)
     assert c.seq_len(0) == 0
+
+
+@pytest.mark.parametrize("read_every", [1, 2, 5])
+def test_decoding_steps_read_or_not(run, read_every):
+    """decoding steps whose logits go to the host, and steps that nobody waits for in between (descriptors by way of pinned memory): the same bits, whoever reads when"""
+    case, c, dtype = run
+    t = tokens(case.cfg, 100, 1)
+    L = bamd_lib()
+    rows = []
+    c.decode(t[:60], 0)
+    want = {k: c.decode(t[k:k + 1], k) for k in range(60, 80)}
+    c.decode(t[:60], 0)
+    try:
+        for n_past in range(60, 80):
+            L.bamd_set_logits_readback(c.h, 0)
+            tok = np.ascontiguousarray(t[n_past:n_past + 1], np.int32)
+            if (n_past + 1) % read_every:
+                assert L.bamd_decode(c.h, tok.ctypes.data, 1, n_past) == 0
+                continue
+            L.bamd_set_logits_readback(c.h, n_past % 2)
+            rows.append((n_past, c.decode(tok, n_past), c.last_logits()))
+    finally:
+        L.bamd_set_logits_readback(c.h, 1)
+    for k, a, b in rows:
+        assert np.array_equal(a.view(np.uint32), want[k].view(np.uint32)) and np.array_equal(a.view(np.uint32), b.view(np.uint32)), k
+    near(rows[-1][1], case.logits(t)[rows[-1][0]], dtype)
+    c.seq_free(0)
 
 
 def test_greedy_generation(run):
