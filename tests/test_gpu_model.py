@@ -374,3 +374,22 @@ def test_long_prompts_in_one_batch(tmp_path):
         bamd.set_prefill_batch(1)
     assert np.array_equal(long.decode(toks, 0).view(np.uint32), want.view(np.uint32))
     long.close(); m.close()
+
+
+@pytest.mark.parametrize("n", [2, 63, 64, 65, 511, 832, 895, 896, 897, 960, 1029, 1811])
+def test_attention_of_a_prompt_around_the_rows_that_stay_on_chip(tmp_path, n):
+    """the score rows of the first 896 positions stay in LDS, those beyond go through a scratch block: the same bits as token by token, for one to eight query heads per KV head"""
+    import booster_amd as bamd
+    for Hkv in (8, 2, 1):
+        p = str(tmp_path / ("m%d.gguf" % Hkv))
+        gguf.write_synthetic_llama(p, E=1024, H=8, Hkv=Hkv, L=2, F=1024, V=512, theta=500000.0, seed=7, type_fn=lambda n, il: gguf.q4_k_m_type(n, il, 2))
+        m = bamd.Model(p)
+        toks = [(29 * i + 3 * n) % 512 for i in range(n)]
+        c = bamd.Context(m, 2048); got = c.decode(toks, 0).copy(); c.close()
+        bamd.set_prefill_batch(False)
+        try:
+            c = bamd.Context(m, 2048); want = c.decode(toks, 0).copy(); c.close()
+        finally:
+            bamd.set_prefill_batch(True)
+        m.close()
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), Hkv
