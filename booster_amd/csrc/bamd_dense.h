@@ -163,6 +163,7 @@ struct bamd_segment { int32_t entry, t0, n, first, last; };       // first, last
 int bamd_launch_gla(const bamd_batch_dev & b, const bamd_gla_args & a, int max_n, const bamd_segment * segs, int n_segs, hipStream_t s);
 void bamd_launch_gla_norm(int act, const bamd_gla_args & a, int rows, hipStream_t s);
 int bamd_gla_blocks(int heads, int Pp);            // blocks of one segment
+int bamd_gla_step_columns(const bamd_gla_args & a, int rows);      // value columns per block of a decoding step
 bool bamd_gla_valid(const bamd_gla_args & a);
 
 // ---- both at once ------------------------------------------------------------------------------------------------------------------------------------

@@ -91,15 +91,18 @@ template <int MODE> static int scan_pick(int pt, const bamd_batch_dev & b, const
     return pt == 16 ? scan_go<16, MODE>(b, a, segs, n_segs, many, s) : pt == 32 ? scan_go<32, MODE>(b, a, segs, n_segs, many, s) : scan_go<64, MODE>(b, a, segs, n_segs, many, s);
 }
 int bamd_gla_blocks(int heads, int Pp) { return (Pp + 63) / 64 * heads; }
+// value columns of a decoding block: enough blocks for the chip, narrower ones only as far as they are filled
+int bamd_gla_step_columns(const bamd_gla_args & a, int rows) {
+    const long wide = (long) bamd_gla_blocks(a.heads, a.Pp) * rows;
+    return a.Pp <= 16 || wide * 2 < 256 ? 16 : a.Pp <= 32 || wide < 256 ? 32 : 64;
+}
 bool bamd_gla_valid(const bamd_gla_args & a) {
     return a.Np >= 4 && a.Np <= 256 && !(a.Np & 3) && a.Pp >= 4 && !(a.Pp & 3) && a.heads >= 1 && a.rank >= 1 && a.rank <= 1024 && !((a.ld | a.q_off | a.k_off | a.v_off) & 3) && (a.g_off < 0 || !(a.g_off & 3)) && !((a.ldo | a.out_off) & 3);
 }
 int bamd_launch_gla(const bamd_batch_dev & b, const bamd_gla_args & a, int max_n, const bamd_segment * segs, int n_segs, hipStream_t s) {
     if (!bamd_gla_valid(a) || max_n < 1) return 1;
-    // enough blocks for the chip; narrower blocks only as far as they are filled
-    const long wide = (long) bamd_gla_blocks(a.heads, a.Pp) * (max_n == 1 ? b.n_entries : n_segs);
-    const int pt = a.Pp <= 16 || (max_n == 1 && wide * 2 < 256) ? 16 : a.Pp <= 32 || wide < 256 ? 32 : 64;
-    if (max_n == 1) return scan_pick<GLA_STEP>(pt, b, a, nullptr, b.n_entries, false, s);
+    if (max_n == 1) return scan_pick<GLA_STEP>(bamd_gla_step_columns(a, b.n_entries), b, a, nullptr, b.n_entries, false, s);
+    const int pt = a.Pp <= 32 || (long) bamd_gla_blocks(a.heads, a.Pp) * n_segs < 256 ? a.Pp <= 16 ? 16 : 32 : 64;
     if (!a.alpha) return 1;
     const bool many = n_segs > b.n_entries;
     if (many && (!segs || !a.seg_state || !a.seg_decay)) return 1;

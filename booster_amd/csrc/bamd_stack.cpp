@@ -184,7 +184,9 @@ struct Timer {                                     // per-launch HIP events (pro
 #define STACK_ROWS 2048                            /* token rows of one pass */
 #define Y2_PLANES 2                                /* shares of K of an output or down projection: there is room for them whatever the rows, so that whether K is halved goes by the shape alone */
 #define SEG_MIN 64                                 /* tokens of the shortest scan segment */
-#define PAIR_ROWS 4                                /* decoding rows up to which two branches share their launches */
+// Decoding rows up to which two branches share their launches.  us per step, two launches against four: width 2048, 8 layers, 5 rows 654 and 723, 16 rows 875 and 941, 64 rows 1748 and 1904;
+// width 4096, 5 rows 1327 and 1407, 16 rows 1686 and 1739, 32 rows 2341 and 2380, 64 rows 3307 and 3292
+#define PAIR_ROWS 64
 #define SEG_BLOCKS 768                             /* blocks a scan wants */
 struct Ctx {
     bamd_context * c = nullptr; Stack * st = nullptr;

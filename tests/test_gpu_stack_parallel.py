@@ -6,7 +6,9 @@ import numpy as np
 import pytest
 
 from oracle import stack_oracle as so
-from test_gpu_stack import DTYPES, near, rel
+import stack_cases
+from stack_cases import tokens
+from test_gpu_stack import Case, DTYPES, near, rel
 
 pytestmark = pytest.mark.gpu
 
@@ -256,3 +258,22 @@ def test_head_norm_and_gate(bamd, dtype):
     near(go.reshape(20, -1), -0.6 * out.reshape(20, -1), dtype)
     gy, go, _ = bamd.op_gated_linear(pos0=0, state=np.zeros((3, 12, 37)), dtype=dtype, **dict(a, gate=None))
     near(go, np.stack([[so.rms(y, 1e-5) * a["norm"] for y in row] for row in gy.astype(np.float64)]), dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H,d,dv,steps", [(3, 130, 70, (2, 21, 22, 42, 43, 64, 65)), (6, 64, 65, (5, 11, 22)), (7, 20, 30, (19, 37)), (2, 100, 9, (6, 64))])
+def test_decoding_rows_that_share_launches(bamd, dtype, H, d, dv, steps, tmp_path):
+    """a step of that many sequences, whose recurrence takes 16, 32 or 64 columns a block; beyond 64 rows the branches have their own launches"""
+    cfg = stack_cases.mafurax(64, 97, [stack_cases.parallel(stack_cases.attend(4, 2, 24, 20, 0.4, 6.0, 50, 19, 3), 0.7, (H, d, dv, 8.0), 1.3, ff=80, limit=0.8)])
+    case = Case(str(tmp_path / "m"), cfg, 3, dict(rel=8, rank=5))
+    m = bamd.Model(case.folder, dtype=dtype)
+    c = bamd.Context(m, 64 * max(steps), max(steps))
+    t = [tokens(cfg, 7 + len(steps), 30 + i) for i in range(3)]
+    want = [case.logits(x) for x in t]
+    c.decode_batch([(s, t[s % 3][:5 + s % 3], [4 + s % 3]) for s in range(max(steps))])
+    at = [5 + s % 3 for s in range(max(steps))]
+    for n in steps:
+        got = c.decode_batch([(s, [t[s % 3][at[s]]], [0]) for s in range(n)])
+        near(got, np.stack([want[s % 3][at[s]] for s in range(n)]), dtype)
+        for s in range(n): at[s] += 1
+    c.close(); m.close()
