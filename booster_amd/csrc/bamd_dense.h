@@ -81,6 +81,9 @@ enum { BAMD_PRE_ROWS = 0, BAMD_PRE_RESIDUAL = 1, BAMD_PRE_POLY = 2, BAMD_PRE_GRO
 struct bamd_pre_args { bamd_residual_args res; bamd_poly_args poly; bamd_group_norm_args grp; bamd_glu_args glu; const float * gf; const int32_t * want; };
 #define BAMD_MV_ROWS 64
 int bamd_launch_dense_mv(int act, const bamd_dense & w, int pre, const bamd_batch_dev & b, const bamd_pre_args * p, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s, int * parts = nullptr);
+// a few rows of the product with gate and up rows in turn, and the gated unit of its results, operands of the product behind, to h.  bamd_dense_few_glu: it is covered
+bool bamd_dense_few_glu(int act, const bamd_dense & w, int rows);
+int bamd_launch_dense_few_glu(const bamd_dense & w, const void * x, int ldx, int rows, void * h, int ldh, float limit, hipStream_t s);
 int bamd_dense_route(int act, const bamd_dense & w, int rows, int pre, int most, int & share);      // many rows (pre < 0): the tile; few rows: -1; share: shares of K, of at most `most`
 size_t bamd_dense_mv_lds(int act, int K);         // operand bytes of a built row: must stay within BAMD_MV_LDS
 #define BAMD_MV_LDS (96 * 1024)

@@ -296,8 +296,9 @@ __global__ void __launch_bounds__(64 * NW) dense_mv_kernel(bamd_dense w, bamd_ba
 // wave streams its share of K — RT KiB of weights and NT of the rows per step — by DMA through a ring of NS steps of its own: 64 consecutive bytes of a row per four lanes, read
 // back in fragment order (dense_tile_kernel's layout), no barrier between steps, and while the sums of a group of tiles meet, the next group's first steps are under way.  LDS holds
 // one block of eight waves per CU.  16 x 14336 x 4096: 32.3 -> 27.1 us (4.3 TB/s of weights), 16 x 32000 x 4096: 62 -> 50 (5.3), 45 x 4096 x 14336: 57 -> 48 us.
-template <int NT, int RT, int NS>
-__global__ void __launch_bounds__(512) dense_few_kernel(bamd_dense w, const bamd_bf * x, int ldx, int rows, float * out, int ldo) {
+// GLU (an even RT): gate and up tiles in turn; out is the gated unit's bfloat16 row.
+template <int NT, int RT, int NS, bool GLU>
+__global__ void __launch_bounds__(512) dense_few_kernel(bamd_dense w, const bamd_bf * x, int ldx, int rows, float * out, int ldo, float limit) {
     constexpr int NW = 8, STEP = (NT + RT) * 1024, RING = NS * STEP;
     extern __shared__ __align__(16) unsigned char lds[];
     float * red = (float *) (lds + NW * RING);                    // [wave][RT][NT][64 lanes][4]
@@ -357,22 +358,28 @@ __global__ void __launch_bounds__(512) dense_few_kernel(bamd_dense w, const bamd
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        for (int i = tid; i < RT * NT * 256; i += 64 * NW) {
-            const int c = i >> 8, l = (i >> 2) & 63, k = i & 3, r = (c % NT) * 16 + (l & 15), o = (grp * RT + c / NT) * 16 + (l >> 4) * 4 + k;
-            if (r < rows && o < w.rows) {
-                float v = 0.f;
+        auto sum = [&](int c, int l, int k) {
+            float v = 0.f;
 #pragma unroll
-                for (int q = 0; q < NW; ++q) v += red[((q * RT * NT + c) * 64 + l) * 4 + k];
-                out[(size_t) r * ldo + o] = v;
+            for (int q = 0; q < NW; ++q) v += red[((q * RT * NT + c) * 64 + l) * 4 + k];
+            return v;
+        };
+        if constexpr (GLU) {
+            for (int i = tid; i < RT / 2 * NT * 256; i += 64 * NW) {
+                const int c = i >> 8, t = c / NT * 2, l = (i >> 2) & 63, k = i & 3, r = (c % NT) * 16 + (l & 15), o = (grp * RT + t) * 8 + (l >> 4) * 4 + k;
+                if (r < rows && o < w.rows / 2) ((bamd_bf *) out)[(size_t) r * ldo + o] = (bamd_bf) clamped_glu(sum(t * NT + c % NT, l, k), sum((t + 1) * NT + c % NT, l, k), limit);
             }
+        } else for (int i = tid; i < RT * NT * 256; i += 64 * NW) {
+            const int c = i >> 8, l = (i >> 2) & 63, k = i & 3, r = (c % NT) * 16 + (l & 15), o = (grp * RT + c / NT) * 16 + (l >> 4) * 4 + k;
+            if (r < rows && o < w.rows) out[(size_t) r * ldo + o] = sum(c, l, k);
         }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");              // (no copy outlives the block)
 }
-template <int NT, int RT, int NS>
-static void few_go(const bamd_dense & w, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s, int parts = 1) {
+template <int NT, int RT, int NS, bool GLU = false>
+static void few_go(const bamd_dense & w, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s, int parts = 1, float limit = 0.f) {
     const int groups = (w.row_tiles + RT - 1) / RT;
-    hipLaunchKernelGGL((dense_few_kernel<NT, RT, NS>), dim3(groups < 256 ? groups : 256, parts), dim3(512), (size_t) 8 * (NS * (NT + RT) + NT * RT) * 1024, s, w, (const bamd_bf *) x, ldx, rows, out, ldo);
+    hipLaunchKernelGGL((dense_few_kernel<NT, RT, NS, GLU>), dim3(groups < 256 ? groups : 256, parts), dim3(512), (size_t) 8 * (NS * (NT + RT) + NT * RT) * 1024, s, w, (const bamd_bf *) x, ldx, rows, out, ldo, limit);
 }
 // RT by the rounds over the CUs; a round of 1, 2 or 3 tiles at K = 4096 takes 7.1, 12.7 and 16 us with up to 16 rows, one of 1 or 2 tiles 9.0 and 15.1 us with up to 32.
 // With more rows the 64 x 64 tiles of prompts are ahead once they fill the CUs (45 x 22672 x 4096: 49 against 74 us) and behind before (45 x 4096 x 14336: 136 against 48)
@@ -438,6 +445,17 @@ static int mv_pick(const bamd_dense & w, int pre, const bamd_batch_dev & b, cons
     else if (rows <= 16) mv_one<T, BAMD_PRE_ROWS>(w, b, p, x, ldx, rows, out, ldo, s, n);
     else if (rows <= 32) mv_go<T, 2, 8, BAMD_PRE_ROWS>(w, b, p, x, ldx, rows, out, ldo, s, n);
     else mv_go<T, 4, 8, BAMD_PRE_ROWS>(w, b, p, x, ldx, rows, out, ldo, s, n);
+    return 0;
+}
+// The gated unit as a part of the product in front of it costs the launch behind that (4 us) and 32-bit results on their way through memory; it asks for pairs of row tiles, which a block of
+// up to 32 rows has where it takes two.  A decoding step of 8 layers, before and after: 2048 x 16384 6 rows 675 -> 657 us, 16 866 -> 848, 17 931 -> 897; 4096 x 28672 (three tiles a block were ahead
+// without) 6 rows 1368 -> 1350, 16 1683 -> 1660.  Four tiles a block: 666, 848; 1394, 1684.  More rows: where few_pick takes the tiles of prompts, they have the unit as well
+// (64 rows 3181 -> 3141)
+bool bamd_dense_few_glu(int act, const bamd_dense & w, int rows) { return act == BAMD_ACT_BF16 && !(w.row_tiles & 1) && rows > 1 && (rows <= 32 || (rows <= BAMD_MV_ROWS && w.row_tiles > 768)); }
+int bamd_launch_dense_few_glu(const bamd_dense & w, const void * x, int ldx, int rows, void * h, int ldh, float limit, hipStream_t s) {
+    if (!bamd_dense_few_glu(BAMD_ACT_BF16, w, rows) || ldx < w.k_tiles * 32 || (ldx & 7) || ldh < w.row_tiles * 8 || (ldh & 3)) return 1;
+    if (rows > 32) return gemm_tiles<bamd_bf, BAMD_OUT_GLU>(w, x, ldx, rows, h, ldh, limit, s);
+    if (rows > 16) few_go<2, 2, 4, true>(w, x, ldx, rows, (float *) h, ldh, s, 1, limit); else few_go<1, 2, 5, true>(w, x, ldx, rows, (float *) h, ldh, s, 1, limit);
     return 0;
 }
 int bamd_launch_dense_mv(int act, const bamd_dense & w, int pre, const bamd_batch_dev & b, const bamd_pre_args * p, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s, int * parts) {

@@ -748,10 +748,12 @@ int Pass::layers() {
         parts = Y2_PLANES;
         pa.res = residual(nullptr, nullptr, ly.pre2);
         const bool glu = st.d.mlp_act == STACK_ACT_CLAMPED_GLU;
-        if (glu && b.rows > BAMD_MV_ROWS) {                        // the product's tiles write the down-projection's operand
+        const bool few = glu && bamd_dense_few_glu(st.act, ly.up, b.rows);
+        if (few || (glu && b.rows > BAMD_MV_ROWS)) {                // the product writes the down-projection's operand
             begin(2, 0); bamd_launch_residual_rows(st.act, b, pa.res, s); end();
             begin(4, (double) ly.up.bytes);
-            const int rc = bamd_launch_dense_gemm(st.act, ly.up, c.h, pa.res.ldh, b.rows, c.y, ly.down.K, BAMD_OUT_GLU, s, ly.limit);
+            const int rc = few ? bamd_launch_dense_few_glu(ly.up, c.h, pa.res.ldh, b.rows, c.y, ly.down.K, ly.limit, s)
+                               : bamd_launch_dense_gemm(st.act, ly.up, c.h, pa.res.ldh, b.rows, c.y, ly.down.K, BAMD_OUT_GLU, s, ly.limit);
             end();
             if (rc) return fail("dense product: unsupported shape");
             if (product(ly.down, c.y, ly.down.K, c.y2, c.ldy2, 5, &parts)) return 1;
@@ -1202,7 +1204,7 @@ BAMD_OP bamd_op_dense_glu(int act, const uint16_t * gate, const uint16_t * upw, 
     if (s.l.alloc(d, 2 * ldo, k) || s.act_rows(x, rows, k, d.K, &dx) || s.alloc((void **) &dy, (size_t) rows * ldo * 4)) return 1;
     uint16_t * w = const_cast<uint16_t *>(d.w);
     if (s.l.pack(&tg, at, Loader::steps(k, 1), w, 2) || s.l.pack(&tu, at, Loader::steps(k, 1), w + (size_t) 16 * d.K, 2)) return 1;
-    if (bamd_launch_dense_gemm(act, d, dx, d.K, rows, dy, ldo, BAMD_OUT_GLU, s.l.s, limit)) return fail("bamd_op_dense_glu: unsupported shape");
+    if (bamd_dense_few_glu(act, d, rows) ? bamd_launch_dense_few_glu(d, dx, d.K, rows, dy, ldo, limit, s.l.s) : bamd_launch_dense_gemm(act, d, dx, d.K, rows, dy, ldo, BAMD_OUT_GLU, s.l.s, limit)) return fail("bamd_op_dense_glu: unsupported shape");
     HIPC(hipGetLastError());
     return s.rows_back(dy, rows, F, ldo, y, act == BAMD_ACT_F32);
 }

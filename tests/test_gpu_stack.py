@@ -84,6 +84,17 @@ def test_dense_tiles(bamd, dtype, n, rows, k):
 @pytest.mark.parametrize("k", [1, 70, 300])
 def test_dense_gated_tiles(bamd, dtype, F, rows, tile, k):
     assert bamd.op_dense_route(2 * ((F + 31) // 32 * 32), k, rows, dtype, most=1) == (tile, 1)
+    gated(bamd, dtype, F, rows, k)
+
+
+# a unit alone, a remainder of a round of units, rows at the edges of their groups, and beyond 32 the tiles of prompts (7000: enough row tiles; 200: not enough, in the engine the unit has its own launch)
+@pytest.mark.parametrize("F,rows", [(1, 2), (16, 16), (40, 17), (8210, 5), (8210, 32), (7000, 33), (200, 64)])
+@pytest.mark.parametrize("k", [1, 230, 2050])
+def test_dense_gated_few_rows(bamd, F, rows, k):
+    gated(bamd, "bfloat16", F, rows, k)
+
+
+def gated(bamd, dtype, F, rows, k):
     r = np.random.default_rng(F + k + rows)
     gate, up = (so.f32_to_bf16(r.standard_normal((F, k)).astype(np.float32)) for _ in range(2))
     x, limit = r.standard_normal((rows, k)).astype(np.float32), 7.0
