@@ -219,6 +219,22 @@ def test_ssm(bamd, H, P, N, G, taps):
         pos += n
 
 
+@pytest.mark.parametrize("H,P,N,G", [(2, 40, 128, 1), (130, 33, 24, 2), (256, 64, 12, 1), (257, 20, 3, 1), (1, 64, 256, 1), (128, 64, 256, 1), (256, 64, 256, 4)])
+def test_ssm_tokens_of_four_taps(bamd, H, P, N, G):
+    """one token after the other, from a fresh state on: blocks of 16, 32 and 64 columns, with one, two and three channels per thread"""
+    r = np.random.default_rng(H + P + N)
+    inner, ch = H * P, H * P + 2 * G * N
+    f = lambda a: np.asarray(a, np.float32)
+    conv, cb, dtb, A, D = map(f, (r.standard_normal((ch, 4)), r.standard_normal(ch) * 0.3, r.uniform(-6, 1, H), r.uniform(-4, 3, H), r.standard_normal(H)))
+    rows = f(r.standard_normal((6, inner + ch + H)))
+    hist, S = np.zeros((3, ch)), np.zeros((H, N, P))
+    gh, gs = f(hist) + 7, f(S) + 7
+    for pos in range(6):
+        want, hist, S = plain_ssm(rows[pos:pos + 1].astype(np.float64), H, P, N, G, conv, cb, dtb, A, D, hist, S)
+        got, gh, gs = bamd.op_ssm(rows[pos:pos + 1], pos, H, P, N, G, conv, cb, dtb, A, D, gh, gs)
+        assert rel(got, want) < 2e-5 and rel(gs, S) < 2e-5 and np.array_equal(gh, f(hist)), pos
+
+
 @pytest.mark.parametrize("H,P,N,G", [(2, 32, 64, 1), (1, 33, 65, 1), (3, 64, 128, 3), (1, 31, 129, 1), (2, 100, 200, 2), (1, 16, 256, 1)])
 def test_ssm_chunks(bamd, H, P, N, G):
     """prompts through every number of state tiles, around the width of a block and the sixteen tokens of a chunk, with decays down to zero and up to one; portions continue one another"""
