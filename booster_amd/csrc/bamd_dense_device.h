@@ -69,9 +69,15 @@ __device__ __forceinline__ float row_max16(float v) {
     v = fmaxf(v, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x140, 0xf, 0xf, true)));
     return v;
 }
+__device__ __forceinline__ float wave_max(float v) {
+    const int i = __float_as_int(row_max16(v));
+    return fmaxf(fmaxf(__int_as_float(__builtin_amdgcn_readlane(i, 0)), __int_as_float(__builtin_amdgcn_readlane(i, 16))), fmaxf(__int_as_float(__builtin_amdgcn_readlane(i, 32)), __int_as_float(__builtin_amdgcn_readlane(i, 48))));
+}
 __device__ __forceinline__ void wave_lds_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier(); }
 
-// sums of NV values over the block; red: NV * 16 floats of LDS.  Every thread gets the result
+// sums of NV values over the block; red: NV * 16 floats of LDS.  Every thread gets the result.  The waves' sums are read by sixteen lanes at once: a loop over them is a chain of up to
+// 16 NV reads of LDS, in front of every product of one row and in every row kernel
+// (131 tokens read and 24 chatted at width 2048: 11.73 -> 11.57 ms; sixteen sequences served at 4096: 34.89 -> 34.62)
 template <int NV> __device__ __forceinline__ void block_sum(float (&v)[NV], float * red) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
 #pragma unroll
@@ -82,7 +88,7 @@ template <int NV> __device__ __forceinline__ void block_sum(float (&v)[NV], floa
         for (int i = 0; i < NV; ++i) red[i * 16 + wave] = v[i];
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < NV; ++i) { float t = 0.f; for (int w = 0; w < nw; ++w) t += red[i * 16 + w]; v[i] = t; }
+    for (int i = 0; i < NV; ++i) v[i] = row_sum16((lane & 15) < nw ? red[i * 16 + (lane & 15)] : 0.f);
 }
 
 // A row of n floats spread over the block four at a time, kept in registers between the passes over it: `fits` rows (n a multiple of four, at most RC pieces per
@@ -142,11 +148,11 @@ template <int RC> __device__ __forceinline__ void row_moments(const RowRegs<RC> 
     __syncthreads();
     if (lane == 0) { red[wave] = m; red[16 + wave] = q; red[32 + wave] = c; }
     __syncthreads();
-    mean = 0.f; var = 0.f;
-    for (int w = 0; w < nw; ++w) mean += red[w] * red[32 + w];
-    mean /= (float) n;
-    for (int w = 0; w < nw; ++w) { const float d = red[w] - mean; var += red[16 + w] + red[32 + w] * d * d; }
-    var /= (float) n;
+    const int w = lane & 15;
+    const float mw = w < nw ? red[w] : 0.f, qw = w < nw ? red[16 + w] : 0.f, cw = w < nw ? red[32 + w] : 0.f;
+    mean = row_sum16(mw * cw) / (float) n;
+    const float d = mw - mean;
+    var = row_sum16(qw + cw * d * d) / (float) n;
 }
 // residual sum with the layer norm of the sublayer's output, and the layer norm (gain gi, null: none) the next sublayer reads, of one row by the whole block
 template <typename T>
@@ -371,13 +377,11 @@ __device__ __forceinline__ void group_norm_row(const bamd_group_norm_args & a, i
 #pragma unroll
             for (int k = 0; k < 4; ++k) t += v[c][k] * v[c][k];
         }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o);
+        t = wave_sum(t);
         __syncthreads();
         if (lane == 0) inv[wave] = t;
         __syncthreads();
-        float sum = 0.f;
-        for (int w = 0; w < wp; ++w) sum += inv[g * wp + w];
+        const float sum = row_sum16((lane & 15) < wp ? inv[g * wp + (lane & 15)] : 0.f);
         const float r = 1.0f / sqrtf(sum / (float) per + a.eps);
 #pragma unroll
         for (int c = 0; c < RC; ++c) { const int i = at0 + c * by; if (i < per) store4<T>(h + base + i, v[c] * r * *(const bamd_v4 *) (a.w + base + i)); }

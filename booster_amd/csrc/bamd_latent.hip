@@ -253,7 +253,7 @@ __global__ void __launch_bounds__(256) latent_decode_kernel(bamd_batch_dev b, ba
             const float m_old = m;
 #pragma unroll
             for (int i = 0; i < KEYS / 16; ++i) { v[i] = sc[hd][k + 16 * i]; m = fmaxf(m, v[i]); }
-            m = fmaxf(m, __shfl_xor(m, 1)); m = fmaxf(m, __shfl_xor(m, 2)); m = fmaxf(m, __shfl_xor(m, 4)); m = fmaxf(m, __shfl_xor(m, 8));
+            m = row_max16(m);
             float sum = 0.f;
 #pragma unroll
             for (int i = 0; i < KEYS / 16; ++i) {
@@ -263,7 +263,7 @@ __global__ void __launch_bounds__(256) latent_decode_kernel(bamd_batch_dev b, ba
                 Ps[hd * PS + k + 16 * i] = hi;
                 if constexpr (NP == 2) Ps[(16 + hd) * PS + k + 16 * i] = to_act<T>(p - (float) hi);
             }
-            sum += __shfl_xor(sum, 1); sum += __shfl_xor(sum, 2); sum += __shfl_xor(sum, 4); sum += __shfl_xor(sum, 8);
+            sum = row_sum16(sum);
             if (k == 0) { const float f = __expf(m_old - m); al[hd] = f; ls[hd] = ls[hd] * f + sum; mx[hd] = m; }
         }
         __syncthreads();
@@ -321,14 +321,9 @@ template <typename T> __global__ void __launch_bounds__(512) latent_combine_kern
     if (wave == 0) {
         const float snk = a.sink ? a.sink[h] : -INFINITY;
         const float ms = lane < live ? part_ml[((base + lane) * 16 + hh) * 2] : -INFINITY, ls = lane < live ? part_ml[((base + lane) * 16 + hh) * 2 + 1] : 0.f;
-        float m = fmaxf(snk, ms);
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-        const float w = lane < live ? expf(ms - m) : 0.f;
-        float sum = w * ls;
+        const float m = wave_max(fmaxf(snk, ms)), w = lane < live ? expf(ms - m) : 0.f;
         wsp[lane] = w;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+        float sum = wave_sum(w * ls);
         if (a.sink) sum += expf(snk - m);
         if (lane == 0) inv = (a.gated ? sigmoid_f(a.in[(size_t) row * a.ld + a.g_off + h]) : 1.f) / sum;
     }
@@ -342,7 +337,12 @@ template <typename T> __global__ void __launch_bounds__(512) latent_combine_kern
         *(bamd_v4 *) (cl + a.Rp * (1 + grp) + q4) = v;
     }
     __syncthreads();
-    for (int r = tid; r < a.Rp; r += 512) { float v = 0.f; for (int g = 0; g < ng; ++g) v += cl[a.Rp * (1 + g) + r]; cl[r] = v; }
+    for (int r = tid; r < a.Rp; r += 512) {
+        float v = 0.f;
+#pragma unroll 8
+        for (int g = 0; g < ng; ++g) v += cl[a.Rp * (1 + g) + r];
+        cl[r] = v;
+    }
     __syncthreads();
     const int kt_n = a.Rp / 32, vt_n = a.D / 16;
     for (int t = wave; t < vt_n; t += 8) {
