@@ -69,6 +69,12 @@ __device__ __forceinline__ float row_max16(float v) {
     v = fmaxf(v, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x140, 0xf, 0xf, true)));
     return v;
 }
+// The tile of a flash kernel's block.  Tiles come with the longest key ranges first; where every CU gets a second block and none a third one, the second ones are taken the other way round,
+// so that the longest range shares its CU with the shortest.
+__device__ __forceinline__ int paired_tile(int heads) {
+    const int at = blockIdx.x / heads, n = gridDim.x / heads, half = 256 / heads;
+    return at >= half && n <= 2 * half ? n - 1 - (at - half) : at;
+}
 __device__ __forceinline__ float wave_max(float v) {
     const int i = __float_as_int(row_max16(v));
     return fmaxf(fmaxf(__int_as_float(__builtin_amdgcn_readlane(i, 0)), __int_as_float(__builtin_amdgcn_readlane(i, 16))), fmaxf(__int_as_float(__builtin_amdgcn_readlane(i, 32)), __int_as_float(__builtin_amdgcn_readlane(i, 48))));

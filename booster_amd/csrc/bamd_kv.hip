@@ -64,9 +64,10 @@ template <typename T> __global__ void __launch_bounds__(256) kv_store_kernel(bam
     }
 }
 
-// ND: head size in 32s; RT: 16-row query tiles per wave; four waves
+// ND: head size in 32s; RT: 16-row query tiles per wave; four waves.  Two blocks fit a CU's LDS with bfloat16 heads of up to 128, and registers are held to the half that lets both be there: a wave's
+// pass is a chain that only other waves fill.  2048 tokens x 32 heads x 128, window 1024: 219 us with one block per CU, 135 with two, 129 paired.  (Rescaling only in passes that move a maximum: 228 for 219)
 template <typename T, int ND, int RT>
-__global__ void __launch_bounds__(256) kv_prompt_kernel(bamd_batch_dev b, bamd_kv_args a, const bamd_qtile * tiles) {
+__global__ void __launch_bounds__(256, sizeof(T) == 2 && ND <= 4 ? 2 : 1) kv_prompt_kernel(bamd_batch_dev b, bamd_kv_args a, const bamd_qtile * tiles) {
     constexpr int D = ND * 32, NV = ND * 2, KS = D + 16 / sizeof(T), VS = 64 + 16 / sizeof(T), NP = sizeof(T) == 2 ? 2 : 1;     // NP: terms of a weight
     constexpr int PIECES = 64 * D * (int) sizeof(T) / 16, PER = PIECES / 256 > 0 ? PIECES / 256 : 1, NB = 64 * RT + 63;         // NB: distances of a pass
     extern __shared__ __align__(16) unsigned char lds[];
@@ -74,7 +75,7 @@ __global__ void __launch_bounds__(256) kv_prompt_kernel(bamd_batch_dev b, bamd_k
     __shared__ float bs[NB + 1];
     // blocks of one kv head stay on one XCD (every eighth block) as far as the head counts allow
     const int rep = a.heads / a.kv_heads, hb = blockIdx.x % a.heads, g = hb % a.kv_heads, h = g * rep + hb / a.kv_heads;
-    const bamd_qtile qt = tiles[blockIdx.x / a.heads];
+    const bamd_qtile qt = tiles[paired_tile(a.heads)];
     const bamd_entry e = b.ent[qt.entry];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lr = lane & 15, lq = lane >> 4;
     T * P = Ps + (size_t) wave * NP * 16 * RT * VS;

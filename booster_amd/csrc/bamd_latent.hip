@@ -34,15 +34,17 @@ template <typename T> __global__ void __launch_bounds__(256) latent_gather_kerne
 }
 
 // ---- prompts ----------------------------------------------------------------------------------------------------------------------------------------
-// ND: head size in 32s (queries, keys and values); RT: 16-row query tiles per wave; four waves
+// ND: head size in 32s (queries, keys and values); RT: 16-row query tiles per wave; four waves.  A wave's pass is a chain — keys, scores, maxima, weights through LDS, values — which only other
+// waves fill: two blocks fit a CU's LDS with bfloat16 heads of up to 128, and registers are held to the half that lets both be there.  Maxima of sixteen lanes by data-parallel moves, sums added
+// up once at the end, sums rescaled only in passes that move a maximum.  2048 tokens x 32 heads x 128: 211 us; moves for permutes of LDS and fewer rescales 158; two blocks per CU 146; paired 141
 template <typename T, int ND, int RT>
-__global__ void __launch_bounds__(256) latent_prompt_kernel(bamd_batch_dev b, bamd_latent_args a, const bamd_qtile * tiles, int n_heads, const T * kmat, const T * vt, int ldv) {
+__global__ void __launch_bounds__(256, sizeof(T) == 2 && ND <= 4 ? 2 : 1) latent_prompt_kernel(bamd_batch_dev b, bamd_latent_args a, const bamd_qtile * tiles, int n_heads, const T * kmat, const T * vt, int ldv) {
     constexpr int D = ND * 32, NV = ND * 2, KS = D + 16 / sizeof(T), VS = 64 + 16 / sizeof(T), NP = sizeof(T) == 2 ? 2 : 1;     // NP: terms of a weight
     constexpr int PIECES = 64 * D * (int) sizeof(T) / 16;
     extern __shared__ __align__(16) unsigned char lds[];
     T * Ks = (T *) lds, * Vs = Ks + 64 * KS, * Ps = Vs + D * VS;                 // Ps: per wave [NP][16 RT][VS]
     const int h = blockIdx.x % n_heads;
-    const bamd_qtile qt = tiles[blockIdx.x / n_heads];
+    const bamd_qtile qt = tiles[paired_tile(n_heads)];
     const bamd_entry e = b.ent[qt.entry];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lr = lane & 15, lq = lane >> 4;
     T * P = Ps + (size_t) wave * NP * 16 * RT * VS;
@@ -60,11 +62,11 @@ __global__ void __launch_bounds__(256) latent_prompt_kernel(bamd_batch_dev b, ba
         }
     }
     bamd_v4 o[RT][NV]; float m[RT][4], l[RT][4];
-    const float snk = a.sink ? a.sink[h] : -INFINITY;
+    const float l2e = 1.4426950408889634f, scale = a.scale * l2e, snk = a.sink ? a.sink[h] * l2e : -INFINITY;      // scores, maxima and the sink times log2(e)
 #pragma unroll
     for (int i = 0; i < RT; ++i) {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) { m[i][k] = snk; l[i][k] = a.sink ? 1.f : 0.f; }
+        for (int k = 0; k < 4; ++k) { m[i][k] = snk; l[i][k] = a.sink && lr == 0 ? 1.f : 0.f; }
 #pragma unroll
         for (int j = 0; j < NV; ++j) o[i][j] = bamd_v4{ 0, 0, 0, 0 };
     }
@@ -114,6 +116,9 @@ __global__ void __launch_bounds__(256) latent_prompt_kernel(bamd_batch_dev b, ba
 #pragma unroll
                 for (int i = 0; i < RT; ++i) sc[i][t] = mma(q[i][k], kf, sc[i][t]);
             }
+        const bool all = k0 + 63 <= e.pos0 + r0;                   // every key of the pass is seen by every row
+        float al[RT][4];
+        bool moved = false;
 #pragma unroll
         for (int i = 0; i < RT; ++i) {
 #pragma unroll
@@ -122,28 +127,34 @@ __global__ void __launch_bounds__(256) latent_prompt_kernel(bamd_batch_dev b, ba
                 float mx = m[i][r];
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
-                    float v = sc[i][t][r] * a.scale;
-                    if (k0 + t * 16 + lr > pos) v = -INFINITY;
+                    float v = sc[i][t][r] * scale;
+                    if (!all && k0 + t * 16 + lr > pos) v = -INFINITY;
                     sc[i][t][r] = v; mx = fmaxf(mx, v);
                 }
-                mx = fmaxf(mx, __shfl_xor(mx, 1)); mx = fmaxf(mx, __shfl_xor(mx, 2)); mx = fmaxf(mx, __shfl_xor(mx, 4)); mx = fmaxf(mx, __shfl_xor(mx, 8));
-                const float al = mx == -INFINITY ? 1.f : __expf(m[i][r] - mx), ref = mx == -INFINITY ? 0.f : mx;
+                mx = row_max16(mx);
+                al[i][r] = mx == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m[i][r] - mx);
+                const float ref = mx == -INFINITY ? 0.f : mx;
+                moved |= mx != m[i][r];
                 float sum = 0.f;
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
-                    const float pe = __expf(sc[i][t][r] - ref);
+                    const float pe = __builtin_amdgcn_exp2f(sc[i][t][r] - ref);
                     sum += pe;
                     T * d = P + (i * 16 + lq * 4 + r) * VS + t * 16 + lr;
                     const T hi = to_act<T>(pe);
                     *d = hi;
                     if constexpr (NP == 2) d[16 * RT * VS] = to_act<T>(pe - (float) hi);
                 }
-                sum += __shfl_xor(sum, 1); sum += __shfl_xor(sum, 2); sum += __shfl_xor(sum, 4); sum += __shfl_xor(sum, 8);
-                l[i][r] = l[i][r] * al + sum; m[i][r] = mx;
-#pragma unroll
-                for (int j = 0; j < NV; ++j) o[i][j][r] *= al;
+                l[i][r] = l[i][r] * al[i][r] + sum; m[i][r] = mx;  // (sums of this lane's columns; added up at the end)
             }
         }
+        if (__any(moved))                                          // (no maximum of the wave's rows has moved in most passes)
+#pragma unroll
+            for (int i = 0; i < RT; ++i)
+#pragma unroll
+                for (int j = 0; j < NV; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) o[i][j][r] *= al[i][r];
         wave_lds_fence();
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
@@ -168,8 +179,9 @@ __global__ void __launch_bounds__(256) latent_prompt_kernel(bamd_batch_dev b, ba
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int row = r0 + i * 16 + lq * 4 + r;
+            const float sum = row_sum16(l[i][r]);
             if (row >= e.n) continue;
-            float f = 1.0f / l[i][r];
+            float f = 1.0f / sum;
             if (a.gated) f *= sigmoid_f(a.in[(size_t) (e.row0 + row) * a.ld + a.g_off + h]);
             T * d = (T *) a.out + (size_t) (e.row0 + row) * a.ldo + h * D;
 #pragma unroll

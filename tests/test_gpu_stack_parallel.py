@@ -112,6 +112,22 @@ def test_window_attention(bamd, dtype, H, G, d, dv, T, pos0, window, keep):
         near(bamd.op_kv_attention(dtype=dtype, splits=splits, **a).reshape(T, -1), want, dtype)
 
 
+@pytest.mark.parametrize("H,G,d,T,window", [(128, 8, 24, 257, 100), (128, 32, 24, 512, 1000), (128, 4, 24, 513, 70), (85, 5, 40, 700, 130)])
+def test_window_attention_in_paired_blocks(bamd, H, G, d, T, window):
+    """tiles of 128 queries: one block per CU and a part of a second, two, two and a part of a third, and heads that do not divide the CUs"""
+    a = case("bfloat16", H, G, d, d, T, 0, window, 3)
+    unit = lambda x: x / np.sqrt((x.astype(np.float64) ** 2).mean(-1, keepdims=True) + a["eps"])
+    q, k, i, j = unit(a["q"]), unit(a["k"]), np.arange(T)[:, None], np.arange(T)[None]
+    bucket = np.array([so.distance_bucket(x, len(a["rel"]), a["bias_max"]) for x in range(T)])[np.maximum(i - j, 0)]
+    want = np.zeros((T, H, d))
+    for h in range(H):
+        s = so.softcap(q[:, h] @ k[:, h // (H // G)].T * a["scale"], a["cap"]) + a["rel"][bucket, h]
+        s = np.where((j > i) | ((i - j >= window) & (j >= 3)), -np.inf, s)
+        w = np.exp(s - s.max(-1, keepdims=True))
+        want[:, h] = w / w.sum(-1, keepdims=True) @ a["v"][:, h // (H // G)] * so.sigmoid(a["gate"][:, h])[:, None]
+    near(bamd.op_kv_attention(dtype="bfloat16", splits=0, **a).reshape(T, -1), want.reshape(T, -1), "bfloat16")
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("splits", [0, 3])
 def test_every_part_may_be_absent(bamd, dtype, splits):
