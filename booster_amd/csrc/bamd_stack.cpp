@@ -204,7 +204,7 @@ struct Ctx {
     struct Layout { size_t ent, row, tok, want, tile, kblk, seg, total; int tiles, kblks, segs; } lay;
     unsigned char * dev = nullptr; int32_t * pages = nullptr;
     static constexpr int RING = 4;
-    unsigned char * host[RING] = {}; int32_t * pages_host[RING] = {}; hipEvent_t ev[RING] = {}; int ring = 0;
+    unsigned char * pinned = nullptr, * host[RING] = {}; int32_t * pages_host[RING] = {}; hipEvent_t ev[RING] = {}; int ring = 0;
     std::map<int, hipGraphExec_t> graphs;          // rows * 4 + what is in front and behind (STEP_*)
     bamd_step_box * box = nullptr; uint32_t * count_serial = nullptr; uint32_t serial = 0;      // decoding steps by way of pinned memory; serial: of the last one
 };
@@ -601,12 +601,18 @@ int Stack::context_init(bamd_context * bc) {
     y.ent = put(sizeof(bamd_entry) * (size_t) max_e); y.row = put(R * 4); y.tok = put(R * 4); y.want = put(R * 4); y.tile = put(sizeof(bamd_qtile) * (size_t) y.tiles); y.kblk = put((size_t) y.kblks * 4); y.seg = put(sizeof(bamd_segment) * (size_t) y.segs);
     y.total = at;
     if (dev_alloc(bc->allocs, (void **) &c.dev, y.total) || dev_alloc(bc->allocs, (void **) &c.pages, (size_t) S * c.max_pages * 4)) return 1;
+    // one pinned block: nine allocations were a fifth to a third of what a context costs to make (width 2048, one sequence: 523 -> 335 us, width 4096: 831 -> 672)
+    at = 0;
+    const size_t box = put(sizeof(bamd_step_box)), pages = (size_t) S * c.max_pages * 4, ring = at;
+    for (int i = 0; i < Ctx::RING; ++i) { put(y.total); put(pages); }
+    HIPC(hipHostMalloc((void **) &c.pinned, at, hipHostMallocCoherent));
+    c.box = (bamd_step_box *) (c.pinned + box);
+    memset(c.box, 0, sizeof(bamd_step_box));
+    at = ring;
     for (int i = 0; i < Ctx::RING; ++i) {
-        HIPC(hipHostMalloc((void **) &c.host[i], y.total)); HIPC(hipHostMalloc((void **) &c.pages_host[i], (size_t) S * c.max_pages * 4));
+        c.host[i] = c.pinned + put(y.total); c.pages_host[i] = (int32_t *) (c.pinned + put(pages));
         HIPC(hipEventCreateWithFlags(&c.ev[i], hipEventDisableTiming));
     }
-    HIPC(hipHostMalloc((void **) &c.box, sizeof(bamd_step_box), hipHostMallocCoherent));
-    memset(c.box, 0, sizeof(bamd_step_box));
     if (dev_alloc(bc->allocs, (void **) &c.count_serial, 8)) return 1;
     HIPC(hipMemset(c.count_serial, 0, 8));
     return 0;
@@ -615,8 +621,8 @@ void Stack::context_free(bamd_context * bc) {
     Ctx * c = (Ctx *) bc->arch_state;
     if (!c) return;
     for (auto & g : c->graphs) hipGraphExecDestroy(g.second);
-    if (c->box) hipHostFree(c->box);
-    for (int i = 0; i < Ctx::RING; ++i) { if (c->host[i]) hipHostFree(c->host[i]); if (c->pages_host[i]) hipHostFree(c->pages_host[i]); if (c->ev[i]) hipEventDestroy(c->ev[i]); }
+    if (c->pinned) hipHostFree(c->pinned);
+    for (int i = 0; i < Ctx::RING; ++i) if (c->ev[i]) hipEventDestroy(c->ev[i]);
     for (void * p : { c->kc, c->kk, c->kv, (void *) c->filtered, (void *) c->steps, (void *) c->alpha, (void *) c->seg_state, (void *) c->seg_decay }) if (p) hipFree(p);
     delete c;
     bc->arch_state = nullptr;
