@@ -667,8 +667,7 @@ static int kv_find_slot(bamd_context * c, int pos, int * cell, int * n_kv) {
     return 0;
 }
 
-extern "C" int bamd_stage_step(bamd_context * c, int32_t token, const void * token_dev, int pos, const void * hidden_in_dev, void * hidden_out_dev, int want_logits,
-                               int prefill_mode, void * hip_stream);
+static int stage_step(bamd_context * c, int32_t token, const void * token_dev, int pos, const void * hidden_in_dev, void * hidden_out_dev, int want_logits, int prefill_mode, hipStream_t s, bool * gave);
 // ---- batched prefill: a micro-batch of T > 1 tokens through the layers at once (llama_decode with n_tokens > 1) -----------
 #define BAMD_PREFILL_CAP 512            /* the reference's default n_batch / n_ubatch */
 // Prompt tokens that go through the layers together.  A position's results do not depend on the others in its micro-batch (masked positions add exact zeros), except that a
@@ -922,6 +921,7 @@ static int decode_to(bamd_context * c, const int32_t * tokens, int n_tokens, int
     if (n_tokens > c->forced_cap) { fail("n_tokens out of range (token by token evaluation takes at most 4096 per call)"); return 1; }
     if (hipSetDevice(m->device) != hipSuccess) { fail("hipSetDevice"); return 1; }
     hipStream_t s = c->stream;
+    bool gave = false;                                              // the step wrote the logits and the status words to the host itself
     if (c->cells.active && n_tokens > 1) { fail("after a context shift (bamd_kv_seq_add) tokens are evaluated one per call"); return 1; }
     if (!c->cells.active) c->n_cached = std::max(c->n_cached, n_past + n_tokens);
     if (hipMemcpyAsync(c->forced, tokens, (size_t) n_tokens * 4, hipMemcpyHostToDevice, s) != hipSuccess) { fail("H2D tokens"); return 1; }
@@ -931,9 +931,8 @@ static int decode_to(bamd_context * c, const int32_t * tokens, int n_tokens, int
         if (enqueue_prefill_batch(c, n_tokens, n_past, s)) return 1;
         enqueue_lm_head(c, s, nullptr);                                  // n_outputs = 1: last token only (llama.cpp:14580-14593)
     } else if (n_tokens == 1) {
-        c->aql_gave = false;
         // single token: the captured stage-step graph (state and token are two small host copies, then one graph launch)
-        if (bamd_stage_step(c, tokens[0], nullptr, n_past, nullptr, nullptr, 1, 0, s)) return 1;
+        if (stage_step(c, tokens[0], nullptr, n_past, nullptr, nullptr, 1, 0, s, c->logits_readback ? &gave : nullptr)) return 1;
     } else {
         if (set_state(c, n_past, s, false)) return 1;
         const int prefill_mode = n_tokens > 1;
@@ -948,8 +947,7 @@ static int decode_to(bamd_context * c, const int32_t * tokens, int n_tokens, int
         if (le != hipSuccess) { fail(std::string("kernel launch failed: ") + hipGetErrorString(le)); return 1; }
     }
     c->logits_host_valid = c->logits_readback;
-    if (c->aql_gave) {                                              // a step of the own queue whose last kernel wrote the logits and the status words to the host
-        c->aql_gave = false;
+    if (gave) {
         if (co_gave_up(c)) return 1;
         if (out) memcpy(out, c->logits_host, (size_t) m->V * 4);
         return 0;
@@ -1210,19 +1208,16 @@ extern "C" __attribute__((visibility("default"))) int bamd_generate_greedy(bamd_
 extern "C" __attribute__((visibility("default"))) int bamd_aql_runs(const bamd_context * c) { return c->aql_runs + c->aql_steps; }
 
 // ---- layer-split stage ---------------------------------------------------------------------------------
-extern "C" __attribute__((visibility("default"))) int bamd_stage_step(bamd_context * c, int32_t token, const void * token_dev, int pos, const void * hidden_in_dev,
-                               void * hidden_out_dev, int want_logits, int prefill_mode, void * hip_stream) {
+// gave (null: the caller does not ask): true once the step has run to its end and left its logits and status words in logits_host
+static int stage_step(bamd_context * c, int32_t token, const void * token_dev, int pos, const void * hidden_in_dev, void * hidden_out_dev, int want_logits, int prefill_mode, hipStream_t s, bool * gave) {
     bamd_model * m = c->m;
-    HIPC(hipSetDevice(m->device));
-    hipStream_t s = (hipStream_t) hip_stream;            // NULL = the HIP default (null) stream, as for any HIP API
-    if (m->rt) return m->rt->stage(c, token_dev ? nullptr : &token, token_dev, 1, pos, hidden_in_dev, hidden_out_dev, want_logits != 0, s);
     if (pos < 0 || pos >= c->n_ctx) return fail("position out of range");
     // ---- own AQL queue (bamd_aql.h): the whole single-stage step — state from a pinned host inbox, layers, lm_head — as packets with fence scope NONE, one host
     //      wait at its end.  For the caller that owns embedding and output, feeds host tokens on the context's own stream and wants the logits (bamd_decode from
     //      the bridge's token loop); layer-split stages, device-side tokens, shifted cells and prefill-mode steps keep the stage graphs below ----
     if (g_aql && !c->aql_failed && m->with_embd && m->with_output && !token_dev && !hidden_in_dev && !hidden_out_dev && want_logits && !prefill_mode &&
         !c->cells.active && s == c->stream && s != nullptr) {
-        const int fused = attn_fused_for(c, pos) ? 1 : 0, key = fused * 2 + (c->logits_readback ? 1 : 0);
+        const int fused = attn_fused_for(c, pos) ? 1 : 0, key = fused * 2 + (gave ? 1 : 0);
         bool ok = fused == 1;
         if (!ok) { bamd_attn_args t; memset(&t, 0, sizeof t); t.hd = m->hd; t.Hkv = m->Hkv; t.n_ctx = c->n_ctx_pad; ok = bamd_attention_split_is_ik_clean(t, m->H / m->Hkv) != 0; }
         if (ok && !c->inbox && hipHostMalloc((void **) &c->inbox, sizeof(bamd_step_state)) != hipSuccess) { (void) hipGetLastError(); c->inbox = nullptr; ok = false; }
@@ -1234,7 +1229,7 @@ extern "C" __attribute__((visibility("default"))) int bamd_stage_step(bamd_conte
                 bamd_launch_step_begin(c->st, c->forced, 1, c->out_tokens, m->tok_embd.raw, m->tok_embd.type, m->E, m->V, c->x, 1, s, nullptr, nullptr, c->rope, c->rope_cur, m->hd, c->inbox);
                 const int rc = enqueue_layers(c, 0, s, nullptr, pos);
                 enqueue_lm_head(c, s, nullptr);
-                if (c->logits_readback) bamd_launch_logits_out(c->logits, c->logits_host, m->V, c->co_err, s);
+                if (gave) bamd_launch_logits_out(c->logits, c->logits_host, m->V, c->co_err, s);
                 bamd_aql_rec = nullptr;
                 const char * why = "recording failed";
                 if (!rc) c->aql_step = bamd_aql_build(m->device, rec, &why);
@@ -1252,7 +1247,7 @@ extern "C" __attribute__((visibility("default"))) int bamd_stage_step(bamd_conte
             const char * why = nullptr;
             if (bamd_aql_run(c->aql_step, 1, nullptr, &why)) return fail(std::string("own AQL queue: ") + (why ? why : "?"));
             c->aql_steps += 1;
-            c->aql_gave = c->logits_readback;
+            if (gave) *gave = true;
             return 0;
         }
     }
@@ -1308,6 +1303,13 @@ extern "C" __attribute__((visibility("default"))) int bamd_stage_step(bamd_conte
     }
     HIPC(hipGraphLaunch(sg.exec, s));
     return 0;
+}
+extern "C" __attribute__((visibility("default"))) int bamd_stage_step(bamd_context * c, int32_t token, const void * token_dev, int pos, const void * hidden_in_dev,
+                               void * hidden_out_dev, int want_logits, int prefill_mode, void * hip_stream) {
+    HIPC(hipSetDevice(c->m->device));
+    hipStream_t s = (hipStream_t) hip_stream;            // NULL = the HIP default (null) stream, as for any HIP API
+    if (c->m->rt) return c->m->rt->stage(c, token_dev ? nullptr : &token, token_dev, 1, pos, hidden_in_dev, hidden_out_dev, want_logits != 0, s);
+    return stage_step(c, token, token_dev, pos, hidden_in_dev, hidden_out_dev, want_logits, prefill_mode, s, nullptr);
 }
 // write the arg-max token of the last lm_head of this (last) stage into a device int32 — no host round trip
 extern "C" __attribute__((visibility("default"))) int bamd_stage_token_to(bamd_context * c, void * token_dev, void * hip_stream) {

@@ -3,6 +3,7 @@
   * single-token bamd_decode steps (the bridge's token loop: state from the pinned host inbox);
   * more packets than the queue's ring holds (the wrap), many short replays.
 BAMD_AQL=0 in the environment (tools/switch_matrix.sh) turns the assertions about which path ran around."""
+import ctypes
 import os
 
 import numpy as np
@@ -96,6 +97,37 @@ def test_steps_on_the_own_queue_read_or_not(bamd, name):
             assert np.array_equal(bits(got), bits(want[i])) and np.array_equal(bits(ctx.last_logits()), bits(want[i])), i
     finally:
         bamd.lib().bamd_set_logits_readback(ctx.h, 1)
+
+
+@pytest.mark.parametrize("read", [1, 0])
+@pytest.mark.parametrize("name", ["tiny_a", "tiny_b"])
+def test_a_prompt_behind_a_stage_step_on_the_contexts_own_stream(bamd, name, read):
+    """bamd_stage_step on the stream that lets it take the own queue, then a prompt: the prompt's own logits, in a fresh context's bits, and the step's own where they are asked for"""
+    m = bamd.Model(os.path.join(GOLDEN, name + ".gguf")); ctx, fresh = bamd.Context(m, 128), bamd.Context(m, 128)
+    L = bamd.lib()
+    L.bamd_context_stream.restype = ctypes.c_void_p; L.bamd_context_stream.argtypes = [ctypes.c_void_p]
+    s = L.bamd_context_stream(ctx.h)
+    prompt, more = [5, 9, 2, 77, 31, 8, 1, 40], [12, 6, 60]
+    try:
+        for at in (len(prompt), 0):                               # behind the step, and from the beginning
+            before = ctx.decode(prompt, 0)
+            ctx.stage_step(3, len(prompt), None, None, True, False, s)
+            kept = ctx.last_logits()
+            L.bamd_set_logits_readback(ctx.h, read)
+            got = ctx.decode(more, at + (at > 0))
+            left = ctx.last_logits()
+            L.bamd_set_logits_readback(ctx.h, 1)
+            fresh.decode(prompt, 0)
+            step = fresh.decode([3], len(prompt))
+            want = fresh.decode(more, at + (at > 0))
+            assert np.array_equal(bits(got), bits(want)) and np.array_equal(bits(left), bits(want)), at
+            assert np.array_equal(bits(kept), bits(before)), at               # the step is no decode: what that left on the host stays
+            ctx.decode(prompt, 0)
+            ctx.stage_step(3, len(prompt), None, None, True, False, s)
+            assert np.array_equal(bits(ctx.stage_logits(s)), bits(step))
+    finally:
+        L.bamd_set_logits_readback(ctx.h, 1)
+    ctx.close(); fresh.close(); m.close()
 
 
 def test_many_replays_across_the_ring_wrap(bamd):
