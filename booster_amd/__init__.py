@@ -87,7 +87,7 @@ def lib():
         L.bamd_op_kv_attention.argtypes = [ci, vp, vp, vp, vp, ci, vp, vp, ci, ci, ci, ci, ci, cf, cf, cf, ci, vp, ci, ci, ci, ci, cf, ci, vp]
         L.bamd_op_gated_linear.argtypes = [ci, vp, vp, vp, vp, vp, vp, vp, vp, ci, ci, ci, ci, ci, ci, cf, cf, cf, cf, ci, vp, vp, vp]
         L.bamd_set_aql.argtypes = [ci]; L.bamd_set_aql.restype = None
-        L.bamd_aql_runs.argtypes = [vp]
+        L.bamd_aql_runs.argtypes = [vp]; L.bamd_aql_recorded.argtypes = [vp]
         _lib = L
     return _lib
 

@@ -368,7 +368,7 @@ extern "C" __attribute__((visibility("default"))) void bamd_context_free(bamd_co
     if (c->m) hipSetDevice(c->m->device);
     if (c->m && c->m->rt && c->arch_state) { if (c->stream) hipStreamSynchronize(c->stream); c->m->rt->context_free(c); }
     if (c->graph) hipGraphExecDestroy(c->graph);
-    bamd_aql_free(c->aql); bamd_aql_free(c->aql_step);
+    bamd_aql_free(c->aql); for (bamd_aql_graph * g : c->aql_step) bamd_aql_free(g);
     if (c->inbox) hipHostFree(c->inbox);
     for (auto & row : c->sgraph) for (auto & g : row) if (g.exec) hipGraphExecDestroy(g.exec);
     for (void * p : c->allocs) hipFree(p);
@@ -1206,6 +1206,8 @@ extern "C" __attribute__((visibility("default"))) int bamd_generate_greedy(bamd_
 }
 // how many bamd_generate_greedy calls of this context ran on the own AQL queue so far (tests, bench: which path produced the number)
 extern "C" __attribute__((visibility("default"))) int bamd_aql_runs(const bamd_context * c) { return c->aql_runs + c->aql_steps; }
+// how many single-token steps have been recorded for that queue (tests: switching the read-back records nothing again)
+extern "C" __attribute__((visibility("default"))) int bamd_aql_recorded(const bamd_context * c) { return c->aql_recorded; }
 
 // ---- layer-split stage ---------------------------------------------------------------------------------
 // gave (null: the caller does not ask): true once the step has run to its end and left its logits and status words in logits_host
@@ -1217,13 +1219,13 @@ static int stage_step(bamd_context * c, int32_t token, const void * token_dev, i
     //      the bridge's token loop); layer-split stages, device-side tokens, shifted cells and prefill-mode steps keep the stage graphs below ----
     if (g_aql && !c->aql_failed && m->with_embd && m->with_output && !token_dev && !hidden_in_dev && !hidden_out_dev && want_logits && !prefill_mode &&
         !c->cells.active && s == c->stream && s != nullptr) {
-        const int fused = attn_fused_for(c, pos) ? 1 : 0, key = fused * 2 + (gave ? 1 : 0);
+        const int fused = attn_fused_for(c, pos) ? 1 : 0;
+        bamd_aql_graph *& step = c->aql_step[fused * 2 + (gave ? 1 : 0)];
         bool ok = fused == 1;
         if (!ok) { bamd_attn_args t; memset(&t, 0, sizeof t); t.hd = m->hd; t.Hkv = m->Hkv; t.n_ctx = c->n_ctx_pad; ok = bamd_attention_split_is_ik_clean(t, m->H / m->Hkv) != 0; }
         if (ok && !c->inbox && hipHostMalloc((void **) &c->inbox, sizeof(bamd_step_state)) != hipSuccess) { (void) hipGetLastError(); c->inbox = nullptr; ok = false; }
         if (ok) {
-            if (c->aql_step && c->aql_step_key != key) { bamd_aql_free(c->aql_step); c->aql_step = nullptr; }
-            if (!c->aql_step) {
+            if (!step) {
                 bamd_aql_recording rec;
                 bamd_aql_rec = &rec;
                 bamd_launch_step_begin(c->st, c->forced, 1, c->out_tokens, m->tok_embd.raw, m->tok_embd.type, m->E, m->V, c->x, 1, s, nullptr, nullptr, c->rope, c->rope_cur, m->hd, c->inbox);
@@ -1232,12 +1234,12 @@ static int stage_step(bamd_context * c, int32_t token, const void * token_dev, i
                 if (gave) bamd_launch_logits_out(c->logits, c->logits_host, m->V, c->co_err, s);
                 bamd_aql_rec = nullptr;
                 const char * why = "recording failed";
-                if (!rc) c->aql_step = bamd_aql_build(m->device, rec, &why);
-                if (!c->aql_step) { c->aql_failed = true; if (getenv("BAMD_AQL_VERBOSE")) fprintf(stderr, "bamd: own AQL queue not used: %s\n", why ? why : "?"); }
-                c->aql_step_key = key;
+                if (!rc) step = bamd_aql_build(m->device, rec, &why);
+                c->aql_recorded += 1;
+                if (!step) { c->aql_failed = true; if (getenv("BAMD_AQL_VERBOSE")) fprintf(stderr, "bamd: own AQL queue not used: %s\n", why ? why : "?"); }
             }
         }
-        if (ok && c->aql_step) {
+        if (ok && step) {
             if (next_serial(c, s)) return 1;
             c->n_cached = std::max(c->n_cached, pos + 1);
             HIPC(hipStreamSynchronize(s));                               // whatever this context enqueued before (a prompt micro-batch nobody waited for) is done
@@ -1245,7 +1247,7 @@ static int stage_step(bamd_context * c, int32_t token, const void * token_dev, i
             memset(in, 0, sizeof *in);
             in->pos_base = pos; in->n_ctx = c->n_ctx; in->serial = c->host_serial; in->token = token;
             const char * why = nullptr;
-            if (bamd_aql_run(c->aql_step, 1, nullptr, &why)) return fail(std::string("own AQL queue: ") + (why ? why : "?"));
+            if (bamd_aql_run(step, 1, nullptr, &why)) return fail(std::string("own AQL queue: ") + (why ? why : "?"));
             c->aql_steps += 1;
             if (gave) *gave = true;
             return 0;

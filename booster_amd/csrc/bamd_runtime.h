@@ -94,7 +94,7 @@ struct bamd_context {
     hipStream_t stream = nullptr;
     hipGraphExec_t graph = nullptr; int graph_fused = -1;
     bamd_aql_graph * aql = nullptr; int aql_key = -1; bool aql_failed = false; int aql_runs = 0;    // the same step as AQL packets for the own queue (bamd_aql.h)
-    bamd_aql_graph * aql_step = nullptr; int aql_step_key = -1; int aql_steps = 0;                 // stage_step's single-token step on the own queue; key: fused attention x logits to the host
+    bamd_aql_graph * aql_step[4] = {}; int aql_steps = 0, aql_recorded = 0;                        // stage_step's single-token steps on the own queue: fused attention x logits to the host
     bamd_step_state * inbox = nullptr;           // pinned host memory: the state of that step, read by step_begin_kernel itself (no copy in front of the step)
     unsigned long long * co_gran = nullptr;   // co-launch granules [H * hd] {value, tag} + give-up counter behind them (bamd_colaunch.hip), zero-initialised
     uint32_t * co_err = nullptr;

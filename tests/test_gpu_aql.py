@@ -97,6 +97,8 @@ def test_steps_on_the_own_queue_read_or_not(bamd, name):
             assert np.array_equal(bits(got), bits(want[i])) and np.array_equal(bits(ctx.last_logits()), bits(want[i])), i
     finally:
         bamd.lib().bamd_set_logits_readback(ctx.h, 1)
+    # a step that gives its logits and one that does not: each is recorded once, however often they take turns
+    assert bamd.lib().bamd_aql_recorded(ctx.h) == (2 if OWN_QUEUE else 0) and (ctx.aql_runs() == 24) == OWN_QUEUE
 
 
 @pytest.mark.parametrize("read", [1, 0])
