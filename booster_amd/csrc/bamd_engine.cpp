@@ -732,15 +732,13 @@ static void build_prefill_aux(bamd_model * m, hipStream_t s) {
     hipStreamSynchronize(s);
     m->aux_ok = true;
 }
-// buffers for T tokens: of BAMD_PREFILL_CAP, of BAMD_PREFILL_WIDE once a longer prompt comes.  1: not allocated (what was there stays)
+// buffers for T tokens: of BAMD_PREFILL_CAP, of BAMD_PREFILL_WIDE once a longer prompt comes (the layouts of quantised activations: ensure_layout).  1: not allocated (what was there stays)
 static int ensure_batch_buffers(bamd_context * c, int tokens) {
     if (c->bcap >= tokens) return 0;
     bamd_model * m = c->m;
     const size_t T = tokens <= BAMD_PREFILL_CAP ? BAMD_PREFILL_CAP : BAMD_PREFILL_WIDE, Ekv = (size_t) m->Hkv * m->hd;
-    const int Kmax = std::max(m->E, m->F);
-    void ** const slot[] = { (void **) &c->bx, (void **) &c->bx2, (void **) &c->bqkv, (void **) &c->batt, (void **) &c->bh, (void **) &c->bblob, (void **) &c->bblob16, (void **) &c->bfrag, (void **) &c->bst };
-    const size_t bytes[] = { T * m->E * 4, T * m->E * 4, T * (m->E + 2 * Ekv) * 4, T * m->E * 4, T * m->F * 4, T * bamd_blob_bytes(Kmax), T * bamd_blob16_bytes(Kmax), bamd_tokfrag_bytes((int) T, Kmax),
-                             (BAMD_PREFILL_WIDE / BAMD_PREFILL_CAP) * sizeof(bamd_step_state) };
+    void ** const slot[] = { (void **) &c->bx, (void **) &c->bx2, (void **) &c->bqkv, (void **) &c->batt, (void **) &c->bh, (void **) &c->bst };
+    const size_t bytes[] = { T * m->E * 4, T * m->E * 4, T * (m->E + 2 * Ekv) * 4, T * m->E * 4, T * m->F * 4, (BAMD_PREFILL_WIDE / BAMD_PREFILL_CAP) * sizeof(bamd_step_state) };
     constexpr int N = sizeof bytes / sizeof *bytes;
     std::vector<void *> got; void * p[N];
     for (int i = 0; i < N; ++i) if (dev_alloc(got, &p[i], bytes[i])) { (void) hipGetLastError(); for (void * q : got) hipFree(q); return 1; }
@@ -750,6 +748,17 @@ static int ensure_batch_buffers(bamd_context * c, int tokens) {
     }
     for (int i = 0; i < N; ++i) { *slot[i] = p[i]; c->allocs.push_back(p[i]); }
     c->bcap = (int) T;
+    return 0;
+}
+// Layout k of T quantised activations (0 rows of bytes, 1 f16 records, 2 f16 fragments), allocated when a product first reads it, by steps of BAMD_PREFILL_CAP tokens: most models read one or
+// two (of 2048 tokens at a feed-forward of 14336 all three would be 170 MB, the fragments are 64).  1: not allocated (what was there stays)
+static int ensure_layout(bamd_context * c, int k, int T) {
+    if (c->blay_tokens[k] >= T) return 0;
+    const int cap = (T + BAMD_PREFILL_CAP - 1) / BAMD_PREFILL_CAP * BAMD_PREFILL_CAP, Kmax = std::max(c->m->E, c->m->F);
+    void *& o = c->blay[k], * p = nullptr; std::vector<void *> got;
+    if (dev_alloc(got, &p, k == 2 ? bamd_tokfrag_bytes(cap, Kmax) : cap * (k ? bamd_blob16_bytes(Kmax) : bamd_blob_bytes(Kmax)))) { (void) hipGetLastError(); return 1; }
+    if (o) { hipDeviceSynchronize(); c->allocs.erase(std::find(c->allocs.begin(), c->allocs.end(), o)); hipFree(o); }
+    o = p; c->allocs.push_back(p); c->blay_tokens[k] = cap;
     return 0;
 }
 // tokens of a prompt of n tokens at n_past that are evaluated as one batch, cut as llama_decode's n_ubatch cuts (llama.cpp:14615) wherever that shows
@@ -767,8 +776,8 @@ static int batch_mm(bamd_context * c, bamd_mm_args a, int epi, int T, hipStream_
     bamd_model * m = c->m;
     auto on_mfma = [&](int i) { return g_prefill_mfma && aux[i] && (a.seg[i].type == BAMD_Q4_K || a.seg[i].type == BAMD_Q5_K || a.seg[i].type == BAMD_Q6_K); };
     auto mm_mfma = [&](const bamd_mv_seg & sg, const void * ax, int nv, float * out, const float * res, int e) {
-        if (const int waves = bamd_prefill_tokfrag(sg.type, sg.nrows, a.K, T)) return bamd_launch_matmul_wide(sg.w, sg.type, nv, sg.nrows, a.K, c->bfrag, T, out, res, e, a.ldo, waves, s);
-        return bamd_launch_matmul_mfma2(sg.w, ax, sg.type, nv, sg.nrows, a.K, c->bblob16, T, out, res, e, a.ldo, s);
+        if (const int waves = bamd_prefill_tokfrag(sg.type, sg.nrows, a.K, T)) return bamd_launch_matmul_wide(sg.w, sg.type, nv, sg.nrows, a.K, c->blay[2], T, out, res, e, a.ldo, waves, s);
+        return bamd_launch_matmul_mfma2(sg.w, ax, sg.type, nv, sg.nrows, a.K, c->blay[1], T, out, res, e, a.ldo, s);
     };
     if (epi == BAMD_EPI_SILU_MUL) {
         if (on_mfma(0) && on_mfma(1) && a.seg[1].type == a.seg[0].type) {
@@ -794,17 +803,20 @@ static int batch_mm(bamd_context * c, bamd_mm_args a, int epi, int T, hipStream_
     }
     return 0;
 }
-// the activations of a product quantised into the layouts that its segments' kernels read
-static void batch_quantize(bamd_context * c, const float * x, const float * nw, const bamd_mm_args & a, int T, hipStream_t s, const void * const * aux, bool pair = false) {
+// the activations of a product quantised into the layouts that its segments' kernels read; a.blob is set.  1: no memory for one of them
+static int batch_quantize(bamd_context * c, const float * x, const float * nw, bamd_mm_args & a, int T, hipStream_t s, const void * const * aux, bool pair = false) {
     bool ints = false, recs = false, frags = false;
     for (int i = 0; i < a.nseg; ++i) {
         const bool mfma = g_prefill_mfma && aux[i] && (!pair || (aux[0] && aux[1] && a.seg[0].type == a.seg[1].type));
         if (!mfma) ints = true; else if (bamd_prefill_tokfrag(a.seg[i].type, a.seg[i].nrows, a.K, T)) frags = true; else recs = true;
     }
-    bamd_launch_quantize_batch(x, nw, c->m->eps, a.K, T, ints ? c->bblob : nullptr, recs ? c->bblob16 : nullptr, frags ? c->bfrag : nullptr, s);
+    if ((ints && ensure_layout(c, 0, T)) || (recs && ensure_layout(c, 1, T)) || (frags && ensure_layout(c, 2, T))) return 1;
+    a.blob = (const uint8_t *) c->blay[0];
+    bamd_launch_quantize_batch(x, nw, c->m->eps, a.K, T, ints ? c->blay[0] : nullptr, recs ? c->blay[1] : nullptr, frags ? c->blay[2] : nullptr, s);
+    return 0;
 }
 // first stage: tokens already in c->forced; later stages: hidden_in [T][E] f32 on this device.  Last stage: leaves the hidden state of
-// the LAST token in c->x (for lm_head); other stages: writes hidden_out [T][E] (possibly on the next device: peer copy).
+// the LAST token in c->x (for lm_head); other stages: writes hidden_out [T][E] (possibly on the next device: peer copy).  2: no memory for a layout of activations
 static int enqueue_prefill_batch(bamd_context * c, int T, int n_past, hipStream_t s, const void * hidden_in = nullptr, void * hidden_out = nullptr) {
     bamd_model * m = c->m;
     const int E = m->E, F = m->F, Ekv = m->Hkv * m->hd, ldq = E + 2 * Ekv, gq = m->H / m->Hkv;
@@ -826,8 +838,8 @@ static int enqueue_prefill_batch(bamd_context * c, int T, int n_past, hipStream_
         else { seg_of(a.seg[a.nseg], ly.wk, c->bqkv + E); a.nseg++; }
         if (ly.wv.type == ly.wk.type) { a.seg[a.nseg - 1].nrows += ly.wv.nrows; a.seg[a.nseg - 1].nvalid += ly.wv.nrows; }
         else { seg_of(a.seg[a.nseg], ly.wv, c->bqkv + E + Ekv); a.nseg++; }
-        a.blob = c->bblob; a.K = E; a.T = T; a.ldo = ldq;
-        batch_quantize(c, c->bx, ly.attn_norm, a, T, s, ly.aux_qkv);
+        a.K = E; a.T = T; a.ldo = ldq;
+        if (batch_quantize(c, c->bx, ly.attn_norm, a, T, s, ly.aux_qkv)) return 2;
         if (batch_mm(c, a, BAMD_EPI_STORE, T, s, ly.aux_qkv)) return fail("batched mat-mul: unsupported shape");
         // RoPE, KV store, attention with the T>1 semantics                  (llama.cpp:8837-8849, :8318-8353)
         bamd_attn_args t; memset(&t, 0, sizeof t);
@@ -860,16 +872,16 @@ static int enqueue_prefill_batch(bamd_context * c, int T, int n_past, hipStream_
         }
         // x2 = x + Wo . att
         memset(&a, 0, sizeof a);
-        seg_of(a.seg[0], ly.wo, c->bx2); a.nseg = 1; a.blob = c->bblob; a.K = E; a.T = T; a.ldo = E; a.res = c->bx;
-        { const void * ax[3] = { ly.aux_o, nullptr, nullptr }; batch_quantize(c, c->batt, nullptr, a, T, s, ax); if (batch_mm(c, a, BAMD_EPI_ADD, T, s, ax)) return fail("batched mat-mul: unsupported shape"); }
+        seg_of(a.seg[0], ly.wo, c->bx2); a.nseg = 1; a.K = E; a.T = T; a.ldo = E; a.res = c->bx;
+        { const void * ax[3] = { ly.aux_o, nullptr, nullptr }; if (batch_quantize(c, c->batt, nullptr, a, T, s, ax)) return 2; if (batch_mm(c, a, BAMD_EPI_ADD, T, s, ax)) return fail("batched mat-mul: unsupported shape"); }
         // h = silu(Wg . a) * (Wu . a)
         memset(&a, 0, sizeof a);
-        seg_of(a.seg[0], ly.wg, c->bh); seg_of(a.seg[1], ly.wu, c->bh); a.nseg = 2; a.blob = c->bblob; a.K = E; a.T = T; a.ldo = F;
-        { const void * ax[3] = { ly.aux_g, ly.aux_u, nullptr }; batch_quantize(c, c->bx2, ly.ffn_norm, a, T, s, ax, true); if (batch_mm(c, a, BAMD_EPI_SILU_MUL, T, s, ax)) return fail("batched mat-mul: unsupported shape"); }
+        seg_of(a.seg[0], ly.wg, c->bh); seg_of(a.seg[1], ly.wu, c->bh); a.nseg = 2; a.K = E; a.T = T; a.ldo = F;
+        { const void * ax[3] = { ly.aux_g, ly.aux_u, nullptr }; if (batch_quantize(c, c->bx2, ly.ffn_norm, a, T, s, ax, true)) return 2; if (batch_mm(c, a, BAMD_EPI_SILU_MUL, T, s, ax)) return fail("batched mat-mul: unsupported shape"); }
         // x = x2 + Wd . h
         memset(&a, 0, sizeof a);
-        seg_of(a.seg[0], ly.wd, c->bx); a.nseg = 1; a.blob = c->bblob; a.K = F; a.T = T; a.ldo = E; a.res = c->bx2;
-        { const void * ax[3] = { ly.aux_d, nullptr, nullptr }; batch_quantize(c, c->bh, nullptr, a, T, s, ax); if (batch_mm(c, a, BAMD_EPI_ADD, T, s, ax)) return fail("batched mat-mul: unsupported shape"); }
+        seg_of(a.seg[0], ly.wd, c->bx); a.nseg = 1; a.K = F; a.T = T; a.ldo = E; a.res = c->bx2;
+        { const void * ax[3] = { ly.aux_d, nullptr, nullptr }; if (batch_quantize(c, c->bh, nullptr, a, T, s, ax)) return 2; if (batch_mm(c, a, BAMD_EPI_ADD, T, s, ax)) return fail("batched mat-mul: unsupported shape"); }
     }
     if (m->with_output) HIPC(hipMemcpyAsync(c->x, c->bx + (size_t) (T - 1) * E, (size_t) E * 4, hipMemcpyDeviceToDevice, s));
     else HIPC(hipMemcpyAsync(hidden_out, c->bx, (size_t) T * E * 4, hipMemcpyDeviceToDevice, s));
@@ -928,7 +940,9 @@ static int decode_to(bamd_context * c, const int32_t * tokens, int n_tokens, int
     if (n_tokens > 1 && (n_tokens <= BAMD_PREFILL_CAP || n_tokens <= c->bcap) && prefill_batch_supported(c, n_past + n_tokens - 1)) {
         // one micro-batch: every layer once for all tokens (each weight record unpacked once per 8 tokens), lm_head for the last
         if (ensure_batch_buffers(c, n_tokens)) return 1;
-        if (enqueue_prefill_batch(c, n_tokens, n_past, s)) return 1;
+        const int rc = enqueue_prefill_batch(c, n_tokens, n_past, s);
+        if (rc == 2 && n_tokens > BAMD_PREFILL_CAP) { c->bwide_failed = true; return decode_to(c, tokens, n_tokens, n_past, out); }      // (in portions, from the beginning)
+        if (rc) return 1;
         enqueue_lm_head(c, s, nullptr);                                  // n_outputs = 1: last token only (llama.cpp:14580-14593)
     } else if (n_tokens == 1) {
         // single token: the captured stage-step graph (state and token are two small host copies, then one graph launch)

@@ -376,6 +376,26 @@ def test_long_prompts_in_one_batch(tmp_path):
     long.close(); m.close()
 
 
+def test_a_long_prompt_takes_the_activation_layout_that_it_reads(tmp_path):
+    """2048 tokens at once: rows of the layers' vectors, the score rows beyond 896 positions, and of the three layouts of quantised activations the one that every product of this size reads"""
+    import booster_amd as bamd
+    import torch
+    E, F, Hkv, T = 1024, 8192, 2, 2048
+    p = str(tmp_path / "m.gguf")
+    gguf.write_synthetic_llama(p, E=E, H=8, Hkv=Hkv, L=1, F=F, V=512, theta=500000.0, seed=9, type_fn=lambda n, il: gguf.Q4_K)
+    m = bamd.Model(p)
+    toks = [(31 * i) % 512 for i in range(T)]
+    warm = bamd.Context(m, T); want = warm.decode(toks, 0).copy(); warm.close()
+    c = bamd.Context(m, T)
+    before = torch.cuda.mem_get_info()[0]
+    got = c.decode(toks, 0)
+    took = before - torch.cuda.mem_get_info()[0]
+    rows, scores, fragments = T * 4 * (3 * E + E + 2 * Hkv * 128 + F), Hkv * 128 * 16 * (T - 896) * 4, T // 16 * F // 256 * (8192 + 64 + 512)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    assert took <= rows + scores + fragments + 9 * (2 << 20), took      # nine allocations, each rounded up to at most 2 MB; the other two layouts would be 60 MB
+    c.close(); m.close()
+
+
 @pytest.mark.parametrize("n", [2, 63, 64, 65, 511, 832, 895, 896, 897, 960, 1029, 1811])
 def test_attention_of_a_prompt_around_the_rows_that_stay_on_chip(tmp_path, n):
     """the score rows of the first 896 positions stay in LDS, those beyond go through a scratch block: the same bits as token by token, for one to eight query heads per KV head"""
