@@ -318,6 +318,14 @@ def test_latent_attention(bamd, dtype, H, d, dv, R, T, pos0):
         near(got.reshape(T, -1), want.reshape(T, -1), dtype)
 
 
+@pytest.mark.parametrize("H,d,R,T,pos0", [(128, 24, 20, 257, 0), (128, 24, 20, 512, 70), (128, 24, 20, 513, 0), (85, 40, 36, 700, 130)])
+def test_latent_attention_in_paired_blocks(bamd, H, d, R, T, pos0):
+    """tiles of 128 queries: one block per CU and a part of a second, two (taken the other way round), two and a part of a third (plain order), and heads that do not divide the CUs"""
+    a = attention_case(H, d, d, R, T, pos0, H + T, "bfloat16")
+    want = plain_attention(H=H, **a)
+    near(bamd.op_latent_attention(dtype="bfloat16", **a).reshape(T, -1), want.reshape(T, -1), "bfloat16")
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("pos0", [0, 127, 250])
 def test_one_key_stands_out(bamd, dtype, pos0):
