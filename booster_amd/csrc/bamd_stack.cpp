@@ -184,9 +184,11 @@ struct Timer {                                     // per-launch HIP events (pro
 #define STACK_ROWS 2048                            /* token rows of one pass */
 #define Y2_PLANES 2                                /* shares of K of an output or down projection: there is room for them whatever the rows, so that whether K is halved goes by the shape alone */
 #define SEG_MIN 64                                 /* tokens of the shortest scan segment */
-// Decoding rows up to which two branches share their launches.  us per step, two launches against four: width 2048, 8 layers, 5 rows 654 and 723, 16 rows 875 and 941, 64 rows 1748 and 1904;
-// width 4096, 5 rows 1327 and 1407, 16 rows 1686 and 1739, 32 rows 2341 and 2380, 64 rows 3307 and 3292
+// Decoding rows up to which two branches share their launches (bfloat16, 32-bit).  us per step of 4 layers behind 1000 tokens, two launches against four, bfloat16: width 512, 5 rows 194 and 228, 64 rows
+// 660 and 703; width 2048, 342 and 368, 1061 and 1141; width 4096, 718 and 744, 1891 and 1935.  32-bit: width 1024, 48 rows 881 and 913, 64 rows 1130 and 1092; width 4096, 24 rows 1983 and
+// 2013, 32 rows 2327 and 2316, 48 rows 3618 and 3639, 64 rows 4114 and 4041
 #define PAIR_ROWS 64
+#define PAIR_ROWS_F32 48
 #define SEG_BLOCKS 768                             /* blocks a scan wants */
 struct Ctx {
     bamd_context * c = nullptr; Stack * st = nullptr;
@@ -730,7 +732,7 @@ int Parallel::run(Pass & p, MixState & st, Operand & o) {
     o.x = p.c.h; o.ldx = out.K;
     p.begin(1, p.tm ? step_bytes(p.c.seqs[0].len + 1) : 0);
     auto * kv = dynamic_cast<KvAttention *>(br[0].get()); auto * gl = dynamic_cast<GatedLinear *>(br[1].get());
-    if (p.decode && p.b.rows <= PAIR_ROWS && kv && gl) {           // few rows: the branches' blocks share their launches
+    if (p.decode && p.b.rows <= (p.st.act == BAMD_ACT_F32 ? PAIR_ROWS_F32 : PAIR_ROWS) && kv && gl) {           // few rows: the branches' blocks share their launches
         const bamd_kv_args k = kv->args(p, st.sub[0], ld_of(in), out.K);
         if (bamd_launch_kv_gla_decode(p.st.act, p.b, k, gl->args(p, st.sub[1], ld_of(in), out.K), p.c.part_o, p.c.part_ml, kv_splits(k, p.b.rows, p.c.max_pages), p.s)) return fail("attention beside gated linear attention: unsupported shape");
     } else for (size_t i = 0; i < br.size(); ++i) if (br[i]->run(p, st.sub[i], ld_of(in), out.K)) return 1;

@@ -279,7 +279,7 @@ def test_head_norm_and_gate(bamd, dtype):
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("H,d,dv,steps", [(3, 130, 70, (2, 21, 22, 42, 43, 64, 65)), (6, 64, 65, (5, 11, 22)), (7, 20, 30, (19, 37)), (2, 100, 9, (6, 64))])
 def test_decoding_rows_that_share_launches(bamd, dtype, H, d, dv, steps, tmp_path):
-    """a step of that many sequences, whose recurrence takes 16, 32 or 64 columns a block; beyond 64 rows the branches have their own launches"""
+    """a step of that many sequences, whose recurrence takes 16, 32 or 64 columns a block; beyond 64 rows (48 in 32-bit) the branches have their own launches"""
     cfg = stack_cases.mafurax(64, 97, [stack_cases.parallel(stack_cases.attend(4, 2, 24, 20, 0.4, 6.0, 50, 19, 3), 0.7, (H, d, dv, 8.0), 1.3, ff=80, limit=0.8)])
     case = Case(str(tmp_path / "m"), cfg, 3, dict(rel=8, rank=5))
     m = bamd.Model(case.folder, dtype=dtype)
