@@ -922,7 +922,7 @@ static int decode_to(bamd_context * c, const int32_t * tokens, int n_tokens, int
         return 0;
     }
     if (n_tokens > BAMD_PREFILL_CAP && g_prefill_batch) {
-        // llama_decode's n_ubatch split (llama.cpp:14615): micro-batches of 512, the logits are those of the last token
+        // llama_decode's n_ubatch split (llama.cpp:14615) as prefill_part makes it: parts of up to 2048, or micro-batches of 512; the logits are those of the last token
         int part = prefill_part(c, n_tokens, n_past);
         if (part < n_tokens) {
             for (int i = 0; i < n_tokens; i += part, part = prefill_part(c, n_tokens - i, n_past + i))
@@ -938,7 +938,7 @@ static int decode_to(bamd_context * c, const int32_t * tokens, int n_tokens, int
     if (!c->cells.active) c->n_cached = std::max(c->n_cached, n_past + n_tokens);
     if (hipMemcpyAsync(c->forced, tokens, (size_t) n_tokens * 4, hipMemcpyHostToDevice, s) != hipSuccess) { fail("H2D tokens"); return 1; }
     if (n_tokens > 1 && (n_tokens <= BAMD_PREFILL_CAP || n_tokens <= c->bcap) && prefill_batch_supported(c, n_past + n_tokens - 1)) {
-        // one micro-batch: every layer once for all tokens (each weight record unpacked once per 8 tokens), lm_head for the last
+        // one part: every layer once for all tokens, lm_head for the last
         if (ensure_batch_buffers(c, n_tokens)) return 1;
         const int rc = enqueue_prefill_batch(c, n_tokens, n_past, s);
         if (rc == 2 && n_tokens > BAMD_PREFILL_CAP) { c->bwide_failed = true; return decode_to(c, tokens, n_tokens, n_past, out); }      // (in portions, from the beginning)

@@ -1,4 +1,4 @@
-// bamd_prefill2.hip — the exact matrix-core prefill mat-mul with the A fragments BUILT ONCE PER WORKGROUP (Q4_K / Q5_K / Q6_K x Q8_K).
+// bamd_prefill2.hip — the exact matrix-core prefill mat-mul with the A fragments BUILT ONCE PER WORKGROUP (Q4_K / Q5_K x Q8_K; up to 64 tokens Q6_K x Q8_K as well).
 //
 // Reference: ggml_compute_forward_mul_mat with ne11 = T (ggml.c:12277-12492) over ggml_vec_dot_q{4,5,6}_K_q8_K (ggml-quants.c:6832 / :7400 / :8037);
 // the second implementation it is tested against is the integer-dot kernel of bamd_prefill.hip (matmul_batch_kernel): ONE
@@ -31,7 +31,7 @@ union bamd_h2u { uint32_t u; bamd_h2 h; };
 struct bamd_mma2_args {
     const uint8_t * w;               // wave-stream records of the matrix (bamd_formats.h)
     const uint8_t * ph;              // prefill aux, builder part:  [row block of 64][super-block]([e-half], Q6_K)[4 row tiles][64 MFMA lanes][16 B]
-    const uint8_t * ch;              // prefill aux, consumer part: [row block of 64][super-block][4 row tiles][X_CH_RT B]
+    const uint8_t * ch;              // prefill aux, consumer part: [row block of 64][super-block][4 row tiles][X_CH4_RT or X_CH6_RT B]
     float * out; const float * res;  // [T][ldo]
     const uint8_t * blob16;          // f16 activation records (quantize_batch_kernel)
     int K, T, nrows, nrows_pad, ldo;
@@ -105,8 +105,8 @@ __global__ void __launch_bounds__(64) prefill_aux_q6k_kernel(const uint8_t * __r
 //      per SIMD — took 27.4 vs 25.4 ms per 512-token micro-batch, profiles/r06_prefill_ceiling.txt.)
 
 // ==== sixteen waves ===========================================================================================================================
-// The eight-wave kernels above trade vector instructions for LDS traffic and end where those were (two waves per SIMD: a step is a chain of
-// dependent latencies).  This kernel — the default for Q4_K / Q5_K — puts four waves on every SIMD:
+// Eight waves with two tiles each trade vector instructions for LDS traffic and gain nothing (two waves per SIMD: a step is a chain of dependent
+// latencies).  This kernel puts four waves on every SIMD:
 //   * a workgroup is SIXTEEN waves: four row tiles x four token tiles, ONE 16 x 16 tile per wave (48 accumulator registers, <= 118 VGPRs);
 //     every A fragment is built once and read by four waves, every token record staged once and read by four;
 //   * staging is three full-wave DMA instructions per wave and step, the same straight-line code on every wave: sources are fixed per-wave scalar pointers

@@ -12,9 +12,10 @@
 //   * rows are the N side: the lane that holds an accumulator holds its row's header too, so d comes out of the header that the scales come from;
 //   * the min terms are a second pass over K with 64 accumulators of their own (they need 24 bytes per row and 36 per token and super-block): together they would spill;
 //   * the only thing waves share is the token fragments, which lie in memory as the lanes read them (quantize_batch_kernel) and are copied to LDS a super-block ahead, one barrier
-//     per super-block.  Quants and headers come through LDS too (private to the wave, two super-blocks ahead), which keeps every request of the loop a counted copy.
-// 2048 tokens, K = 4096, Q4_K, in a running prompt: 14336 rows 708 -> 523 us (343 -> 460 TFLOP/s), 6144 rows 312 -> 222, 4096 rows 216 -> 152; Q6_K, K = 14336, 4096 rows 880 -> 524.
-// Per super-block of 128 rows x 64 tokens 2.3 us: chains 1.5, copies and barrier 0.25, min pass 0.55.  Tried: the eight e on two waves (four waves per SIMD, half the registers): 3.0
+//     per super-block.  Quants and headers come through LDS too (private to the wave, two super-blocks ahead), which makes every request of the loop a counted copy; except with Q6_K on
+//     eight waves, where two registers are kept in scratch memory and the compiler's wait for the one it reads back at the top of a super-block waits for the copies in flight as well.
+// 2048 tokens, K = 4096, Q4_K, in a running prompt: 14336 rows 708 -> 523 us (343 -> 460 TFLOP/s), 6144 rows 312 -> 222, 4096 rows 216 -> 152; Q6_K, K = 14336, 4096 rows 880 -> 510.
+// Per super-block of 128 rows x 64 tokens 2.3 us; by itself the 14336-row launch takes 553 us (2.5 per super-block), 427 without the min pass, in Q5_K 528 and 453.  Tried: the eight e on two waves (four waves per SIMD, half the registers): 3.0
 // us; matrix instructions and chains pinned in turn: no faster; a loop without a seam between super-blocks: 2.5 us, 3.4 for Q6_K.
 #include "bamd_device.h"
 #include "bamd_mfma_common.h"
@@ -384,7 +385,8 @@ static int wide_rounds(int nrows_pad, int T, int waves) { return (((T + 15) / 16
 int bamd_prefill_tokfrag(int type, int nrows_pad, int K, int T) {
     if (bamd_prefill_few_tiles(type, nrows_pad, K, T)) return 0;
     // Both sides by their rounds of 256 blocks, one block per CU, and a round's time at K = 4096 in us (it grows with K alike): 64 x 64 on sixteen waves 26; here 26 | 32 | 38 with two,
-    // three, four token tiles.  Measured, 4096-row model: 14336 rows 96 tokens 50 | 35, 128 tokens 52 | 41, 200 tokens 97 | 77; 6144 rows 128 tokens 27 | 36, 200 tokens 50 | 38; 4096
+    // three, four token tiles.  Q5_K and other K go by the same line: of 143 sizes each of Q4_K and Q5_K (65 to 2048 tokens, 1024 to 14336 rows, K from 2048 to 14336) it takes the slower
+    // kernel by more than a hundredth nowhere.  Measured, 4096-row model: 14336 rows 96 tokens 50 | 35, 128 tokens 52 | 41, 200 tokens 97 | 77; 6144 rows 128 tokens 27 | 36, 200 tokens 50 | 38; 4096
     // rows 256 tokens 29 | 37, 512 tokens 54 | 41.  Q6_K, four waves against eight: 1024 rows 512 tokens 31 | 39, K = 14336 4096 rows 256 tokens 101 | 121, 512 tokens 198 | 136
     if (type == BAMD_Q6_K) return wide_rounds(nrows_pad, T, 8) * 100 <= wide_rounds(nrows_pad, T, 4) * 77 ? 8 : 4;
     static const int round[3] = { 26, 32, 38 };

@@ -113,7 +113,7 @@ struct bamd_context {
     // phase-stamp blocks (bamd_timeline_step, BAMD_TIMING builds): one block of BAMD_TL_SLOT_WORDS u64 per launch
     unsigned long long * tl_base = nullptr; int tl_slot = 0, tl_cap = 0;
     int bcap = 0; bool bwide_failed = false;
-    float * attn_bscr = nullptr; size_t attn_bscr_bytes = 0, attn_bscr_failed = 0;   // score rows of the matrix-core prefill attention beyond BAMD_AM_MAXPOS = 512 positions (grow-only; absent = the VALU kernel runs)
+    float * attn_bscr = nullptr; size_t attn_bscr_bytes = 0, attn_bscr_failed = 0;   // score rows of the matrix-core prefill attention beyond BAMD_AM_MAXPOS = 896 positions (grow-only; absent = the VALU kernel runs)
     float * bx = nullptr, * bx2 = nullptr, * bqkv = nullptr, * batt = nullptr, * bh = nullptr; bamd_step_state * bst = nullptr;
     void * blay[3] = {}; int blay_tokens[3] = {};                   // activations quantised: rows of bytes, f16 records, f16 fragments (each allocated when a product first reads it)
     std::vector<void *> allocs;

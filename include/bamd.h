@@ -57,15 +57,16 @@ void           bamd_kv_cache_clear(bamd_context * c);                   /* llama
 /* llama_decode(ctx, llama_batch_get_one(tokens, n_tokens, n_past, 0)) (llama.cpp:18517, :14537).
  * Processes the tokens at positions n_past.. with the reference's semantics for a micro-batch of n_tokens
  * (n_tokens > 1: attention scores use the f16-rounded q of the reference's T>1 path) and leaves the logits of
- * the LAST token for bamd_get_logits.  More than 512 tokens are evaluated in micro-batches of 512 (n_ubatch, llama.cpp:14615).
+ * the LAST token for bamd_get_logits.  More than 512 tokens are cut as n_ubatch = 512 cuts (llama.cpp:14615) wherever that shows
+ * in the results; up to 2048 go through the layers together where there is memory for them.
  * Returns 0, or 1 on failure like llama_decode. */
 int           bamd_decode(bamd_context * c, const int32_t * tokens, int n_tokens, int n_past);
 const float * bamd_get_logits(bamd_context * c);                        /* llama_get_logits: host, n_vocab floats */
-/* bamd_decode + a copy of bamd_get_logits into n_vocab floats of the caller's (their pages are touched while the device is at work) */
+/* bamd_decode + a copy of bamd_get_logits into n_vocab floats of the caller's (their pages are touched while the device is at work; undefined behind a failure) */
 int           bamd_decode_logits(bamd_context * c, const int32_t * tokens, int n_tokens, int n_past, float * logits);
 
 /* llama_decode on a llama_batch of several sequences: every entry's tokens run behind what its sequence already holds (none: from position 0), all entries as
- * one batch.  want: ascending places among the entry's tokens whose logits are asked for; `logits` (host, may be NULL) receives them in order, n_vocab floats each. */
+ * one batch.  want: ascending places among the entry's tokens whose logits are asked for; `logits` (host, may be NULL) receives them in order, n_vocab floats each (undefined behind a failure). */
 typedef struct { int32_t seq, n_tokens; const int32_t * tokens; int32_t n_want; const int32_t * want; } bamd_batch_entry;
 int bamd_decode_batch(bamd_context * c, const bamd_batch_entry * entries, int n_entries, float * logits);
 int bamd_seq_len(bamd_context * c, int seq);                            /* tokens the sequence holds, -1 = no such sequence */
