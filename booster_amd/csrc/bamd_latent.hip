@@ -62,11 +62,14 @@ __global__ void __launch_bounds__(256, sizeof(T) == 2 && ND <= 4 ? 2 : 1) latent
         }
     }
     bamd_v4 o[RT][NV]; float m[RT][4], l[RT][4];
-    const float l2e = 1.4426950408889634f, scale = a.scale * l2e, snk = a.sink ? a.sink[h] * l2e : -INFINITY;      // scores, maxima and the sink times log2(e)
+    // Maxima and the sink are kept times log2(e).  An exponent is one fused product and difference with the maximum: the product of a score is not rounded, and what the maximum was rounded
+    // by is common to the keys and the sink
+    const float l2e = 1.4426950408889634f, scale = a.scale * l2e, snk = a.sink ? a.sink[h] * l2e : -INFINITY;
+    const float one = !a.sink ? 0.f : fabsf(snk) < INFINITY ? __builtin_amdgcn_exp2f(fmaf(a.sink[h], l2e, -snk)) : 1.f;
 #pragma unroll
     for (int i = 0; i < RT; ++i) {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) { m[i][k] = snk; l[i][k] = a.sink && lr == 0 ? 1.f : 0.f; }
+        for (int k = 0; k < 4; ++k) { m[i][k] = snk; l[i][k] = lr == 0 ? one : 0.f; }
 #pragma unroll
         for (int j = 0; j < NV; ++j) o[i][j] = bamd_v4{ 0, 0, 0, 0 };
     }
@@ -129,7 +132,7 @@ __global__ void __launch_bounds__(256, sizeof(T) == 2 && ND <= 4 ? 2 : 1) latent
                 for (int t = 0; t < 4; ++t) {
                     float v = sc[i][t][r] * scale;
                     if (!all && k0 + t * 16 + lr > pos) v = -INFINITY;
-                    sc[i][t][r] = v; mx = fmaxf(mx, v);
+                    mx = fmaxf(mx, v);
                 }
                 mx = row_max16(mx);
                 al[i][r] = mx == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m[i][r] - mx);
@@ -138,7 +141,8 @@ __global__ void __launch_bounds__(256, sizeof(T) == 2 && ND <= 4 ? 2 : 1) latent
                 float sum = 0.f;
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
-                    const float pe = __builtin_amdgcn_exp2f(sc[i][t][r] - ref);
+                    float pe = __builtin_amdgcn_exp2f(fmaf(sc[i][t][r], scale, -ref));
+                    if (!all && k0 + t * 16 + lr > pos) pe = 0.f;
                     sum += pe;
                     T * d = P + (i * 16 + lq * 4 + r) * VS + t * 16 + lr;
                     const T hi = to_act<T>(pe);

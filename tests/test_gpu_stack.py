@@ -349,6 +349,27 @@ def test_one_key_stands_out(bamd, dtype, pos0):
         near(bamd.op_latent_attention(dtype=dtype, decode=True, **case).reshape(1, -1), want.reshape(1, -1), dtype, 3)
 
 
+@pytest.mark.parametrize("scale", [0.125, 0.13])
+def test_scores_far_from_zero(bamd, scale):
+    """whole numbers that 32 bits hold exactly, thousands from zero and a few from one another, beside a sink among them and one far below: what a score or a maximum is rounded by (2^-13 of the
+    exponent here, 1e-4 of a weight) must not show in the weights"""
+    H, d, R, n, T = 2, 64, 32, 200, 70
+    a = attention_case(H, d, 16, R, T, n, 3, "float32")
+    r = np.random.default_rng(4)
+    past = r.integers(-3, 4, (n, R)).astype(np.float32)
+    past[:, 0] = 200
+    q = np.zeros((T, H, d), np.float32)
+    q[:, :, 1:R] = r.integers(-2, 3, (T, H, R - 1))
+    q[:, :, 0] = 160
+    uk = np.zeros((H, d, R), np.float32)
+    uk[:, np.arange(R), np.arange(R)] = 1
+    uv = a["uv"].copy()
+    uv[:, 0] = 0
+    a = dict(a, q=q, past=past, uk=so.f32_to_bf16(uk.reshape(H * d, R)), uv=uv, sink=np.array([32005 * scale, -5], np.float32), scale=scale)
+    want = plain_attention(H=H, **dict(a, scale=float(np.float32(scale))))
+    near(bamd.op_latent_attention(dtype="float32", **a).reshape(T, -1), want.reshape(T, -1), "float32")
+
+
 @pytest.mark.parametrize("decode", [False, True])
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_sinks_and_gates(bamd, dtype, decode):
