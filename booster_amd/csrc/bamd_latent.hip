@@ -36,7 +36,7 @@ template <typename T> __global__ void __launch_bounds__(256) latent_gather_kerne
 // ---- prompts ----------------------------------------------------------------------------------------------------------------------------------------
 // ND: head size in 32s (queries, keys and values); RT: 16-row query tiles per wave; four waves.  A wave's pass is a chain — keys, scores, maxima, weights through LDS, values — which only other
 // waves fill: two blocks fit a CU's LDS with bfloat16 heads of up to 128, and registers are held to the half that lets both be there.  Maxima of sixteen lanes by data-parallel moves, sums added
-// up once at the end, sums rescaled only in passes that move a maximum.  2048 tokens x 32 heads x 128: 211 us; moves for permutes of LDS and fewer rescales 158; two blocks per CU 146; paired 141
+// up once at the end, sums rescaled only in passes that move a maximum.  2048 tokens x 32 heads x 128: 211 us; moves for permutes of LDS and fewer rescales 158; two blocks per CU 146; paired 141; (on another card) exponents as fused products 133 -> 129
 template <typename T, int ND, int RT>
 __global__ void __launch_bounds__(256, sizeof(T) == 2 && ND <= 4 ? 2 : 1) latent_prompt_kernel(bamd_batch_dev b, bamd_latent_args a, const bamd_qtile * tiles, int n_heads, const T * kmat, const T * vt, int ldv) {
     constexpr int D = ND * 32, NV = ND * 2, KS = D + 16 / sizeof(T), VS = 64 + 16 / sizeof(T), NP = sizeof(T) == 2 ? 2 : 1;     // NP: terms of a weight
