@@ -75,7 +75,9 @@ void bamd_launch_advance(bamd_entry * ent, int32_t * tokens, unsigned long long 
 // f32 [rows][ldo] | activation type [rows][ldo] | activation type, transposed [n][ldo] | activation type, the clamped gated unit of alternating 16-row tiles [rows][ldo]
 enum { BAMD_OUT_F32 = 0, BAMD_OUT_ACT = 1, BAMD_OUT_ACT_T = 2, BAMD_OUT_GLU = 3 };
 // parts: in, how many shares of K the caller can take (f32 results only; share i goes to out + i * rows * ldo); out, how many there are: one or two
+// x: rows of operands; 32-bit: what bamd_launch_split_rows made of them (6 bytes per value, ldx = 96 k_tiles)
 int bamd_launch_dense_gemm(int act, const bamd_dense & w, const void * x, int ldx, int rows, void * out, int ldo, int out_kind, hipStream_t s, float limit = 0.f, int * parts = nullptr);
+void bamd_launch_split_rows(const float * x, int ldx, int rows, int k_tiles, void * planes, hipStream_t s);
 // few rows (<= BAMD_MV_ROWS): the weights stream once; out f32 [rows][ldo].  pre: how the operand comes about —
 enum { BAMD_PRE_ROWS = 0, BAMD_PRE_RESIDUAL = 1, BAMD_PRE_POLY = 2, BAMD_PRE_GROUP = 3, BAMD_PRE_FINAL = 4, BAMD_PRE_GLU = 5, BAMD_PRE_LAYER = 6 };     // (LAYER: RESIDUAL and FINAL with layer norms, chosen by res.norm); x given | one row, built in front of the product from the argument block
 struct bamd_pre_args { bamd_residual_args res; bamd_poly_args poly; bamd_group_norm_args grp; bamd_glu_args glu; const float * gf; const int32_t * want; };

@@ -52,6 +52,38 @@ __device__ __forceinline__ void store_tile(const bamd_v4 (&a)[NI], int j, int mb
         }
     }
 }
+// A 32-bit activation is the sum of three bfloat16 numbers, eight bits of its significand each (cut off, not rounded: parts of one sign, and what is left is exact), and products of bfloat16
+// numbers are exact in 32 bits: three bfloat16 matrix instructions do what eight of 16x16x4_f32 did, with three roundings of a sum per 32 columns for thirty-two.
+template <typename T> constexpr int bamd_planes = sizeof(T) == 4 ? 3 : 1;
+// rows [rows][ldx] of 32 k_tiles floats -> [rows][k_tiles][3 planes][32].  A value that is not finite is its first plane alone
+__global__ void __launch_bounds__(256) split_rows_kernel(const float * __restrict__ x, int ldx, int k_tiles, uint16_t * __restrict__ planes) {
+    const int i = (blockIdx.x * 256 + threadIdx.x) * 8;
+    if (i >= k_tiles * 32) return;
+    const float * p = x + (size_t) blockIdx.y * ldx + i;
+    const bamd_v4 a = *(const bamd_v4 *) p, b = *(const bamd_v4 *) (p + 4);
+    uint32_t h[3][4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        uint32_t part[2][3];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const float v = c < 2 ? a[c * 2 + e] : b[c * 2 - 4 + e];
+            const uint32_t u = __float_as_uint(v);
+            const bool finite = (u & 0x7f800000u) != 0x7f800000u;
+            const float m = finite ? v - __uint_as_float(u & 0xffff0000u) : 0.f, l = m - __uint_as_float(__float_as_uint(m) & 0xffff0000u);
+            part[e][0] = finite || !(u & 0x007fffffu) ? u : u | 0x00400000u;
+            part[e][1] = __float_as_uint(m); part[e][2] = __float_as_uint(l);
+        }
+#pragma unroll
+        for (int n = 0; n < 3; ++n) h[n][c] = (part[0][n] >> 16) | (part[1][n] & 0xffff0000u);
+    }
+    uint16_t * d = planes + (size_t) blockIdx.y * k_tiles * 96 + (i >> 5) * 96 + (i & 31);
+#pragma unroll
+    for (int n = 0; n < 3; ++n) *(bamd_u4 *) (d + n * 32) = bamd_u4{ h[n][0], h[n][1], h[n][2], h[n][3] };
+}
+void bamd_launch_split_rows(const float * x, int ldx, int rows, int k_tiles, void * planes, hipStream_t s) {
+    hipLaunchKernelGGL(split_rows_kernel, dim3((k_tiles * 4 + 255) / 256, rows), dim3(256), 0, s, x, ldx, k_tiles, (uint16_t *) planes);
+}
 // TM activation rows x TN matrix rows per block of WM x WN waves.  Both operands travel global -> LDS by DMA (a kilobyte per instruction: 16 rows x 32 columns), NS stages
 // of 32 columns deep: while the matrix instructions of column block k run from registers, the fragments of k + 1 are read from LDS and the copies of the NS - 2 blocks
 // behind it are under way; one barrier per column block, which waits for copies issued NS - 2 blocks ago.  What bounded the kernel before it (128 x 128, staged through registers) was LDS
@@ -59,12 +91,15 @@ __device__ __forceinline__ void store_tile(const bamd_v4 (&a)[NI], int j, int mb
 // all of them in front of the first costs 15 %.
 // Activations lie in LDS as they come from memory, four lanes on 64 consecutive bytes of a row (one 16-byte piece of 16 rows per four lanes costs the vector memory path
 // four times the lookups: 446 -> 409 us below), the pieces of a row turned by half its number: sixteen rows of one piece then fall on different banks.
+// 32-bit (three planes of activations): the sums of a column block start at zero and are added to the accumulators by the vector units, a row of tiles behind.  The matrix instructions cut off
+// where the vector units round: kept in them from one column block to the next, a sum of 14336 positive products was off by 6.3e-6 (1.8e-6 with the f32 instructions), so it is 3.2e-7 (and
+// 4.1e-7 for 2.2e-6 with random signs).  500 x 8192 x 2048 118 -> 46 us, 500 x 12608 x 2048 178 -> 75, 500 x 2048 x 8192 122 -> 63.
 // 2048 x 28672 x 4096: 676 -> 409 us (1176 TFLOP/s); 2048 x 4096 x 14336: 284 -> 185 us (1303); 2048 x 2048 x 2048: 41 -> 22 us; 131 x 8192 x 2048: 23 -> 16 us.
 template <typename T, int TM, int TN, int WM, int WN, int NS, int OUT>
-__global__ void __launch_bounds__(64 * WM * WN) dense_tile_kernel(bamd_dense w, const T * x, int ldx, int rows, void * out, int ldo, int n_mt, int n_nt, float limit) {
+__global__ void __launch_bounds__(64 * WM * WN) dense_tile_kernel(bamd_dense w, const bamd_bf * x, int ldx, int rows, void * out, int ldo, int n_mt, int n_nt, float limit) {
     const int kb = (int) ((long) w.k_tiles * blockIdx.y / gridDim.y), nk = (int) ((long) w.k_tiles * (blockIdx.y + 1) / gridDim.y) - kb;      // this block's share of K
-    constexpr int XT = TM / 16, WT = TN / 16, NW = WM * WN, MI = XT / WM, NI = WT / WN, XK = sizeof(T) / 2, PX = XT * XK / NW, PW = WT / NW, PER = PX + PW, STAGE = (XT * XK + WT) * 1024;       // XK: KiB of an activation block
-    static_assert(XT * XK % NW == 0 && WT % NW == 0 && MI * WM == XT && NI * WN == WT && NS >= 4 && (NS & (NS - 1)) == 0, "");
+    constexpr int XT = TM / 16, WT = TN / 16, NW = WM * WN, MI = XT / WM, NI = WT / WN, XP = bamd_planes<T>, PX = XT * XP / NW, PW = WT / NW, PER = PX + PW, STAGE = (XT * XP + WT) * 1024;
+    static_assert(XT * XP % NW == 0 && (XP == 1 || MI % 2 == 0) && WT % NW == 0 && MI * WM == XT && NI * WN == WT && NS >= 4 && (NS & (NS - 1)) == 0, "");
     extern __shared__ __align__(16) unsigned char lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int total = n_mt * n_nt;
@@ -72,41 +107,43 @@ __global__ void __launch_bounds__(64 * WM * WN) dense_tile_kernel(bamd_dense w, 
     { const int per = (total + 7) / 8, xcd = id & 7, k = id >> 3; id = xcd * per + k; if (k >= per || id >= total) return; }
     const int mt = id % n_mt, nt = id / n_mt, m0 = mt * TM, n0t = nt * WT;
     // this wave's share of a stage: PX operand blocks of activations, PW of weights
-    const unsigned char * xbase = (const unsigned char *) (x + (size_t) m0 * ldx + (size_t) kb * 32), * wbase = (const unsigned char *) (w.w + ((size_t) n0t * w.k_tiles + kb) * 512);
+    const unsigned char * xbase = (const unsigned char *) (x + (size_t) m0 * ldx + (size_t) kb * (32 * XP)), * wbase = (const unsigned char *) (w.w + ((size_t) n0t * w.k_tiles + kb) * 512);
     uint32_t xo[PX], wo[PW];
 #pragma unroll
-    for (int i = 0; i < PX; ++i) {                                // bfloat16: 16 rows of four 16-byte pieces; 32-bit: 8 rows of eight
-        int row = XK == 1 ? (wave * PX + i) * 16 + (lane >> 2) : (wave * PX + i) * 8 + (lane >> 3);
+    for (int i = 0; i < PX; ++i) {                                // 16 rows of four 16-byte pieces, of one plane
+        const int u = wave * PX + i;
+        int row = u / XP * 16 + (lane >> 2);
         row = m0 + row < rows ? row : rows - 1 - m0;
-        xo[i] = (uint32_t) row * (uint32_t) ldx * (uint32_t) sizeof(T) + (uint32_t) (XK == 1 ? (lane & 3) ^ ((lane >> 3) & 3) : (lane & 7) ^ (lane >> 3)) * 16u;
+        xo[i] = (uint32_t) row * (uint32_t) ldx * 2u + (uint32_t) (u % XP) * 64u + (uint32_t) ((lane & 3) ^ ((lane >> 3) & 3)) * 16u;
     }
 #pragma unroll
     for (int i = 0; i < PW; ++i) { int tile = wave * PW + i; tile = n0t + tile < w.row_tiles ? tile : w.row_tiles - 1 - n0t; wo[i] = (uint32_t) tile * (uint32_t) w.k_tiles * 1024u + (uint32_t) lane * 16u; }
-    const uint32_t xd = (uint32_t) (size_t) (bamd_lds_vp) lds + (uint32_t) wave * PX * 1024u, wd = (uint32_t) (size_t) (bamd_lds_vp) lds + (uint32_t) (XT * XK + wave * PW) * 1024u;
+    const uint32_t xd = (uint32_t) (size_t) (bamd_lds_vp) lds + (uint32_t) wave * PX * 1024u, wd = (uint32_t) (size_t) (bamd_lds_vp) lds + (uint32_t) (XT * XP + wave * PW) * 1024u;
     // copy i of PER of stage k (behind the last column block: the last one again, into a stage nobody reads)
     auto copy = [&](int k, int i) {
         const int kk = k < nk ? k : nk - 1;
         const uint32_t st = (uint32_t) (k & (NS - 1)) * STAGE;
-        if (i < PX) lds_dma16_s(xbase + (size_t) kk * (32 * sizeof(T)), xo[i], xd + st + i * 1024u);
+        if (i < PX) lds_dma16_s(xbase + (size_t) kk * (64 * XP), xo[i], xd + st + i * 1024u);
         else lds_dma16_s(wbase + (size_t) kk * 1024, wo[i - PX], wd + st + (i - PX) * 1024u);
     };
     const int wm = wave % WM, wn = wave / WM;
     const int r = lane & 15, q = lane >> 4;                       // the lane's row of a block and its eight columns
-    const unsigned char * xb = lds + (size_t) wm * MI * XK * 1024 + (XK == 1 ? (r * 4 + (q ^ ((r >> 1) & 3))) * 16 : (r * 8 + ((2 * q) ^ (r & 7))) * 16), * wb = lds + (size_t) (XT * XK + wn * NI) * 1024 + lane * 16;
-    const int xb2 = XK == 1 ? 0 : (((2 * q + 1) ^ (r & 7)) - ((2 * q) ^ (r & 7))) * 16;      // 32-bit: from the first four columns to the other four
+    const unsigned char * xb = lds + (size_t) wm * MI * XP * 1024 + (r * 4 + (q ^ ((r >> 1) & 3))) * 16, * wb = lds + (size_t) (XT * XP + wn * NI) * 1024 + lane * 16;
     bamd_v4 acc[MI][NI];
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < NI; ++j) acc[i][j] = bamd_v4{ 0, 0, 0, 0 };
-    Frag<T> xf[2][MI];
-    bamd_u4 wr[2][NI];                                            // as packed; 32-bit operands are widened where they are used
-    auto read_x = [&](int k, int p, int i) {
-        const unsigned char * at = xb + (k & (NS - 1)) * STAGE + i * (XK * 1024);
-        if constexpr (XK == 1) xf[p][i].load((const T *) at);
-        else { xf[p][i].a = *(const bamd_v4 *) at; xf[p][i].b = *(const bamd_v4 *) (at + xb2); }
+    bamd_v4 part[2][NI];                                          // 32-bit: the sums of a column block, of this row of tiles and the one in front
+#pragma unroll
+    for (int j = 0; j < NI; ++j) part[(MI - 1) & 1][j] = bamd_v4{ 0, 0, 0, 0 };
+    auto add = [&](int i) {
+#pragma unroll
+        for (int j = 0; j < NI; ++j) acc[i][j] = acc[i][j] + part[i & 1][j];
     };
-    auto read_w = [&](int k, int p, int j) { wr[p][j] = *(const bamd_u4 *) (wb + (k & (NS - 1)) * STAGE + j * 1024); };
+    bamd_bf8 xf[2][MI][XP], wf[2][NI];
+    auto read_x = [&](int k, int p, int i, int c) { xf[p][i][c] = *(const bamd_bf8 *) (xb + (k & (NS - 1)) * STAGE + (i * XP + c) * 1024); };
+    auto read_w = [&](int k, int p, int j) { wf[p][j] = *(const bamd_bf8 *) (wb + (k & (NS - 1)) * STAGE + j * 1024); };
     auto wait = [&] {                                             // in block k: leaves NS - 3 stages of this wave's copies under way, so that stage k + 1 is whole; then every wave's
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"((NS - 3) * PER) : "memory");
         __builtin_amdgcn_s_barrier();
@@ -115,9 +152,6 @@ __global__ void __launch_bounds__(64 * WM * WN) dense_tile_kernel(bamd_dense w, 
     auto block = [&](int k, auto par) {
         constexpr int P = decltype(par)::value;
         wait();                                                   // stage k + 1 is whole; stage k - 1 is free
-        Frag<T> wf[NI];
-#pragma unroll
-        for (int j = 0; j < NI; ++j) wf[j].weight(wr[P][j]);
         // MI groups: a row of matrix instructions, and spread over them the copies of stage k + NS - 1 and the reads of stage k + 1
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
@@ -125,12 +159,18 @@ __global__ void __launch_bounds__(64 * WM * WN) dense_tile_kernel(bamd_dense w, 
             for (int c = i * PER / MI; c < (i + 1) * PER / MI; ++c) copy(k + NS - 1, c);
 #pragma unroll
             for (int j = i * NI / MI; j < (i + 1) * NI / MI; ++j) read_w(k + 1, P ^ 1, j);
-            read_x(k + 1, P ^ 1, i);
 #pragma unroll
-            for (int j = 0; j < NI; ++j) {
-                if constexpr (OUT == BAMD_OUT_ACT_T) acc[i][j] = mma(xf[P][i], wf[j], acc[i][j]);      // lane: four activation rows of one matrix row
-                else acc[i][j] = mma(wf[j], xf[P][i], acc[i][j]);                                       // lane: four matrix rows of one activation row
-            }
+            for (int c = 0; c < XP; ++c) read_x(k + 1, P ^ 1, i, c);
+#pragma unroll
+            for (int c = XP - 1; c >= 0; --c)                     // the smallest parts first
+#pragma unroll
+                for (int j = 0; j < NI; ++j) {
+                    const bamd_v4 from = XP == 1 ? acc[i][j] : c == XP - 1 ? bamd_v4{ 0, 0, 0, 0 } : part[i & 1][j];
+                    bamd_v4 & to = XP == 1 ? acc[i][j] : part[i & 1][j];
+                    if constexpr (OUT == BAMD_OUT_ACT_T) to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf[P][i][c], wf[P][j], from, 0, 0, 0);      // lane: four activation rows of one matrix row
+                    else to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[P][j], xf[P][i][c], from, 0, 0, 0);                                       // lane: four matrix rows of one activation row
+                }
+            if constexpr (XP > 1) add(i ? i - 1 : MI - 1);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -142,12 +182,15 @@ __global__ void __launch_bounds__(64 * WM * WN) dense_tile_kernel(bamd_dense w, 
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 #pragma unroll
-    for (int i = 0; i < MI; ++i) read_x(0, 0, i);
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int c = 0; c < XP; ++c) read_x(0, 0, i, c);
 #pragma unroll
     for (int j = 0; j < NI; ++j) read_w(0, 0, j);
     int k = 0;
     for (; k + 2 <= nk; k += 2) { block(k, std::integral_constant<int, 0>()); block(k + 1, std::integral_constant<int, 1>()); }
     if (k < nk) block(k, std::integral_constant<int, 0>());
+    if constexpr (XP > 1) add(MI - 1);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");              // (no copy outlives the block)
     const int n_lim = w.row_tiles * 16;
     if constexpr (OUT == BAMD_OUT_F32) out = (float *) out + (size_t) blockIdx.y * rows * ldo;
@@ -159,7 +202,7 @@ __global__ void __launch_bounds__(64 * WM * WN) dense_tile_kernel(bamd_dense w, 
 template <typename T, int TM, int TN, int WM, int WN, int NS, int OUT>
 static int tile_go(const bamd_dense & w, const void * x, int ldx, int rows, void * out, int ldo, float limit, int parts, hipStream_t s) {
     const int n_mt = (rows + TM - 1) / TM, n_nt = (w.row_tiles + TN / 16 - 1) / (TN / 16), per = (n_mt * n_nt + 7) / 8;
-    hipLaunchKernelGGL((dense_tile_kernel<T, TM, TN, WM, WN, NS, OUT>), dim3(per * 8, parts), dim3(64 * WM * WN), (size_t) NS * (TM / 16 * sizeof(T) / 2 + TN / 16) * 1024, s, w, (const T *) x, ldx, rows, out, ldo, n_mt, n_nt, limit);
+    hipLaunchKernelGGL((dense_tile_kernel<T, TM, TN, WM, WN, NS, OUT>), dim3(per * 8, parts), dim3(64 * WM * WN), (size_t) NS * (TM / 16 * bamd_planes<T> + TN / 16) * 1024, s, w, (const bamd_bf *) x, ldx, rows, out, ldo, n_mt, n_nt, limit);
     return 0;
 }
 // The tile whose rounds over the 256 CUs end first.  Measured per block of 32 columns, all CUs busy (ns): 256 x 256 700, 128 x 256 450, 128 x 128 250, all three one block per CU,
@@ -168,17 +211,26 @@ static int tile_go(const bamd_dense & w, const void * x, int ldx, int rows, void
 // start and end once more (4 us).  131 x 2048 x 8192: 38 -> 22 us, 412 x 4096 x 8192: 85 -> 39; four shares were no faster (24 and 43 us).  Halves of 64 x 64 tiles that put a second block on
 // a CU take 300 where each half is longer than 2048 columns: 131 x 4096 x 14336 whole 70 us, in halves of such tiles 74, of 128 x 128 58 (8192 columns: 41, 43, 36); at K = 4096 they are
 // level or ahead (131 x 3072: 24.0 and 24.4, 300 x 2048: 24.4 and 19.9).  Of 187 halved sizes (K 1056 to 14336) nine are slower than whole by more than 2 %, at most 7 % (17 and 11 % without).
-// 32-bit: bound by the f32 matrix instructions: small tiles, several blocks per CU.  Halves take half as long up to 128 tiles (K = 4096: 76 -> 41 us), from there to 192 they share CUs and
-// take 0 to 8 % less (K = 1024: 24.4 and 24.7, K = 4096: 76.9 -> 72.5)
+// 32-bit, three planes of activations: a block of 128 x 256 takes 800 ns where few CUs are busy and 1280 where all are (their copies out of L2), 128 x 128 430 and 690, 64 x 128 370 and 460, two of them
+// on a CU 700 to 800, 64 x 64 250 and 300, four on a CU 1000.  Halves: only what the reader of the second plane pays.  Of 94 choices (512 to 12608 outputs, K 512 to 14336, 70 to 2048 rows) the mean is
+// 0.5 % behind the best and the worst 10 %
 enum { TILE_256_256 = 0, TILE_128_256 = 1, TILE_128_128 = 2, TILE_64_128 = 3, TILE_64_64 = 4, TILE_64_64_DEEP = 5 };
 static int pick_tile(int act, const bamd_dense & w, int rows, int most, int & share) {
     share = 1;
-    if (act == BAMD_ACT_F32) {
-        if (most > 1 && (long) ((rows + 63) / 64) * ((w.row_tiles + 3) / 4) <= 192 && w.k_tiles >= 32) share = 2;
-        return TILE_64_64;
-    }
     auto tiles = [&](int tm, int tn) { return (long) ((rows + tm - 1) / tm) * ((w.row_tiles * 16 + tn - 1) / tn); };
     long best = 0; int pick = 0;
+    if (act == BAMD_ACT_F32) {
+        static const int kind[4] = { TILE_128_256, TILE_128_128, TILE_64_128, TILE_64_64 };
+        for (int p = 1; p <= most && p <= 2 && (p == 1 || w.k_tiles >= 32); ++p) {
+            auto rounds = [](long b, long lo, long by) { return b / 256 * (lo + by) + (b % 256 ? lo + by * (b % 256) / 256 : 0); };
+            const long b1 = tiles(64, 128) * p, b0 = tiles(64, 64) * p;
+            const long t[4] = { rounds(tiles(128, 256) * p, 800, 480), rounds(tiles(128, 128) * p, 430, 260), std::max(b1 > 256 ? 700 : 370 + 90 * b1 / 256, 400 * b1 / 256), std::max(250 + 50 * b0 / 256, 250 * b0 / 256) };
+            const int i = (int) (std::min_element(t, t + 4) - t);
+            const long ns = t[i] * ((w.k_tiles + p - 1) / p) + (p > 1 ? (long) rows * w.row_tiles * 16 / 1000 : 0);
+            if (p == 1 || ns < best) { best = ns; pick = kind[i]; share = p; }
+        }
+        return pick;
+    }
     for (int p = 1; p <= most && p <= 2 && (p == 1 || w.k_tiles >= 32); ++p) {
         auto rounds = [&](int tm, int tn, long cost) { return (tiles(tm, tn) * p + 255) / 256 * cost; };
         const long pairs = p == 2 && w.k_tiles > 128 && tiles(64, 64) * 2 > 256 ? 300 : 160;
@@ -202,6 +254,11 @@ static int gemm_tiles(const bamd_dense & w, const void * x, int ldx, int rows, v
         case TILE_64_128: return tile_go<T, 64, 128, 2, 2, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
         case TILE_64_64_DEEP: return tile_go<T, 64, 64, 2, 2, 8, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
     }
+    else switch (tile) {                                          // three planes of activations: waves as tall as wide would read twice as much of them
+        case TILE_128_256: return tile_go<T, 128, 256, 2, 4, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
+        case TILE_128_128: return tile_go<T, 128, 128, 4, 2, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
+        case TILE_64_128: return tile_go<T, 64, 128, 2, 2, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
+    }
     return tile_go<T, 64, 64, 2, 2, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
 }
 // f32 rows are stored four matrix rows at a time: ldo % 4 == 0; x rows start on 16 bytes and hold k_tiles * 32 columns
@@ -217,7 +274,7 @@ static int gemm_out(const bamd_dense & w, const void * x, int ldx, int rows, voi
     return 1;
 }
 int bamd_launch_dense_gemm(int act, const bamd_dense & w, const void * x, int ldx, int rows, void * out, int ldo, int kind, hipStream_t s, float limit, int * parts) {
-    if (rows < 1 || w.row_tiles < 1 || w.k_tiles < 1 || ldx < w.k_tiles * 32 || (ldx & 7) || (ldo & 3)) return 1;
+    if (rows < 1 || w.row_tiles < 1 || w.k_tiles < 1 || ldx < w.k_tiles * (act == BAMD_ACT_F32 ? 96 : 32) || (ldx & 7) || (ldo & 3)) return 1;
     return act == BAMD_ACT_F32 ? gemm_out<float>(w, x, ldx, rows, out, ldo, kind, limit, s, parts) : gemm_out<bamd_bf>(w, x, ldx, rows, out, ldo, kind, limit, s, parts);
 }
 

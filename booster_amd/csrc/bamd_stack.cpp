@@ -199,6 +199,7 @@ struct Ctx {
     int ldy = 0, ldy2 = 0, ldy3 = 0, ldh = 0;
     void * qp = nullptr; float * part_o = nullptr, * part_ml = nullptr;
     void * kc = nullptr, * kk = nullptr, * kv = nullptr; size_t kc_n = 0, kk_n = 0, kv_n = 0;      // unpacked latents / keys / values of a prompt pass
+    void * planes = nullptr; size_t planes_n = 0;                                                  // 32-bit operand rows of a prompt's product, split
     float * filtered = nullptr, * steps = nullptr; size_t filtered_n = 0, steps_n = 0;             // filtered channels, step sizes and decays of a prompt pass
     float * alpha = nullptr, * seg_state = nullptr, * seg_decay = nullptr; size_t alpha_n = 0, seg_state_n = 0, seg_decay_n = 0;      // decays and segment states of a prompt pass
     unsigned long long * keys = nullptr; int32_t * step = nullptr, * gen_out = nullptr; int gen_cap = 0;
@@ -224,10 +225,12 @@ struct Pass {                                      // one pass through the layer
         return a;
     }
     void advanced(const float * y, int ld, const float * g, int parts) { std::swap(x, xo); pend = y; ldp = ld; pend_g = g; pend_parts = parts; }
+    int split(const bamd_dense & w, const void * & x, int & ldx, int rows);      // 32-bit operand rows as bamd_launch_dense_gemm takes them; bfloat16 rows are left alone
     // a product whose operand rows exist; small row counts stream the weights once
     // parts: in, shares of K the result's buffer can hold; out, shares there are (the rows' residual sum adds them)
     int product(const bamd_dense & w, const void * in, int ldx, float * out, int ldo, int kind, int * parts = nullptr) {
         begin(kind, (double) w.bytes);
+        if (b.rows > BAMD_MV_ROWS && split(w, in, ldx, b.rows)) return 1;
         const int rc = b.rows <= BAMD_MV_ROWS ? bamd_launch_dense_mv(st.act, w, BAMD_PRE_ROWS, b, nullptr, in, ldx, b.rows, out, ldo, s, parts)
                                               : bamd_launch_dense_gemm(st.act, w, in, ldx, b.rows, out, ldo, BAMD_OUT_F32, s, 0.f, parts);
         end();
@@ -625,7 +628,7 @@ void Stack::context_free(bamd_context * bc) {
     for (auto & g : c->graphs) hipGraphExecDestroy(g.second);
     if (c->pinned) hipHostFree(c->pinned);
     for (int i = 0; i < Ctx::RING; ++i) if (c->ev[i]) hipEventDestroy(c->ev[i]);
-    for (void * p : { c->kc, c->kk, c->kv, (void *) c->filtered, (void *) c->steps, (void *) c->alpha, (void *) c->seg_state, (void *) c->seg_decay }) if (p) hipFree(p);
+    for (void * p : { c->kc, c->kk, c->kv, c->planes, (void *) c->filtered, (void *) c->steps, (void *) c->alpha, (void *) c->seg_state, (void *) c->seg_decay }) if (p) hipFree(p);
     delete c;
     bc->arch_state = nullptr;
 }
@@ -655,6 +658,13 @@ int grow(Ctx & c, void ** p, size_t * have, size_t need, hipStream_t s) {
     if (*p) HIPC(hipFree(*p));
     *p = nullptr; *have = 0;
     HIPC(hipMalloc(p, need + 4096)); *have = need;
+    return 0;
+}
+int Pass::split(const bamd_dense & w, const void * & x, int & ldx, int rows) {
+    if (st.act != BAMD_ACT_F32) return 0;
+    if (grow(c, &c.planes, &c.planes_n, (size_t) rows * std::max(c.ldh, w.K) * 6, s)) return 1;
+    bamd_launch_split_rows((const float *) x, ldx, rows, w.k_tiles, c.planes, s);
+    x = c.planes; ldx = 96 * w.k_tiles;
     return 0;
 }
 int Mamba2::run(Pass & p, MixState & st, Operand & o) {
@@ -687,7 +697,9 @@ int LatentAttention::run(Pass & p, MixState & st, Operand & o) {
         if (grow(c, &c.kc, &c.kc_n, kr * Rp * el, p.s) || grow(c, &c.kk, &c.kk_n, kr * H * D * el, p.s) || grow(c, &c.kv, &c.kv_n, kr * H * D * el, p.s)) return 1;
         bamd_launch_latent_store(act, p.b, a, p.s);
         bamd_launch_latent_gather(act, p.b, a, (const int32_t *) (c.dev + c.lay.kblk), p.k_rows, c.kc, p.s);
-        rc = bamd_launch_dense_gemm(act, uk, c.kc, Rp, p.k_rows, c.kk, H * D, BAMD_OUT_ACT, p.s) || bamd_launch_dense_gemm(act, uv, c.kc, Rp, p.k_rows, c.kv, p.k_rows, BAMD_OUT_ACT_T, p.s) ||
+        const void * lat = c.kc; int ldl = Rp;
+        if (p.split(uk, lat, ldl, p.k_rows)) return 1;
+        rc = bamd_launch_dense_gemm(act, uk, lat, ldl, p.k_rows, c.kk, H * D, BAMD_OUT_ACT, p.s) || bamd_launch_dense_gemm(act, uv, lat, ldl, p.k_rows, c.kv, p.k_rows, BAMD_OUT_ACT_T, p.s) ||
              bamd_launch_latent_prompt(act, p.b, a, (const bamd_qtile *) (c.dev + c.lay.tile), p.n_tiles, c.kk, c.kv, p.k_rows, p.s);
     }
     p.end();
@@ -760,8 +772,10 @@ int Pass::layers() {
         if (few || (glu && b.rows > BAMD_MV_ROWS)) {                // the product writes the down-projection's operand
             begin(2, 0); bamd_launch_residual_rows(st.act, b, pa.res, s); end();
             begin(4, (double) ly.up.bytes);
-            const int rc = few ? bamd_launch_dense_few_glu(ly.up, c.h, pa.res.ldh, b.rows, c.y, ly.down.K, ly.limit, s)
-                               : bamd_launch_dense_gemm(st.act, ly.up, c.h, pa.res.ldh, b.rows, c.y, ly.down.K, BAMD_OUT_GLU, s, ly.limit);
+            const void * in = c.h; int ldx = pa.res.ldh;
+            if (!few && split(ly.up, in, ldx, b.rows)) return 1;
+            const int rc = few ? bamd_launch_dense_few_glu(ly.up, in, ldx, b.rows, c.y, ly.down.K, ly.limit, s)
+                               : bamd_launch_dense_gemm(st.act, ly.up, in, ldx, b.rows, c.y, ly.down.K, BAMD_OUT_GLU, s, ly.limit);
             end();
             if (rc) return fail("dense product: unsupported shape");
             if (product(ly.down, c.y, ly.down.K, c.y2, c.ldy2, 5, &parts)) return 1;
@@ -1153,6 +1167,15 @@ struct OpScratch {                                 // device copies of one call
         }
         return 0;
     }
+    // operand rows of a product of many rows
+    int split(const bamd_dense & d, const void * & x, int & ldx, int rows) {
+        if (l.act != BAMD_ACT_F32) return 0;
+        void * p;
+        if (alloc(&p, (size_t) rows * d.K * 6)) return 1;
+        bamd_launch_split_rows((const float *) x, ldx, rows, d.k_tiles, p, l.s);
+        x = p; ldx = 96 * d.k_tiles;
+        return 0;
+    }
     int one_entry(int rows, int pos0, bamd_batch_dev & b) {
         const bamd_entry e = { 0, 0, rows, pos0, 0, 0 };
         bamd_entry * de; int32_t * re, * tk, * pg;
@@ -1184,11 +1207,12 @@ BAMD_OP bamd_op_dense(int act, const uint16_t * w, int nrows, int k, const float
     int parts = impl == 4 || impl == 5 ? 2 : 1;
     if (s.alloc((void **) &dy, (size_t) (impl == 3 ? ld_of(d) : rows) * ldo * 4 * parts)) return 1;
     bamd_batch_dev b; memset((void *) &b, 0, sizeof b);
-    int rc;
-    if (impl == 4) rc = bamd_launch_dense_gemm(act, d, dx, d.K, rows, dy, ldo, BAMD_OUT_F32, s.l.s, 0.f, &parts);
+    int rc, ldx = d.K; const void * px = dx;
+    if (impl != 1 && impl != 5 && s.split(d, px, ldx, rows)) return 1;
+    if (impl == 4) rc = bamd_launch_dense_gemm(act, d, px, ldx, rows, dy, ldo, BAMD_OUT_F32, s.l.s, 0.f, &parts);
     else if (impl == 5) rc = bamd_launch_dense_mv(act, d, BAMD_PRE_ROWS, b, nullptr, dx, d.K, rows, dy, ldo, s.l.s, &parts);
     else if (impl == 1) rc = bamd_launch_dense_mv(act, d, BAMD_PRE_ROWS, b, nullptr, dx, d.K, rows, dy, ldo, s.l.s);
-    else rc = bamd_launch_dense_gemm(act, d, dx, d.K, rows, dy, ldo, impl == 0 ? BAMD_OUT_F32 : impl == 2 ? BAMD_OUT_ACT : BAMD_OUT_ACT_T, s.l.s);
+    else rc = bamd_launch_dense_gemm(act, d, px, ldx, rows, dy, ldo, impl == 0 ? BAMD_OUT_F32 : impl == 2 ? BAMD_OUT_ACT : BAMD_OUT_ACT_T, s.l.s);
     if (rc) return fail("bamd_op_dense: unsupported shape");
     HIPC(hipGetLastError());
     if (impl >= 4) {                                              // the shares, added as their reader adds them
@@ -1212,7 +1236,9 @@ BAMD_OP bamd_op_dense_glu(int act, const uint16_t * gate, const uint16_t * upw, 
     if (s.l.alloc(d, 2 * ldo, k) || s.act_rows(x, rows, k, d.K, &dx) || s.alloc((void **) &dy, (size_t) rows * ldo * 4)) return 1;
     uint16_t * w = const_cast<uint16_t *>(d.w);
     if (s.l.pack(&tg, at, Loader::steps(k, 1), w, 2) || s.l.pack(&tu, at, Loader::steps(k, 1), w + (size_t) 16 * d.K, 2)) return 1;
-    if (bamd_dense_few_glu(act, d, rows) ? bamd_launch_dense_few_glu(d, dx, d.K, rows, dy, ldo, limit, s.l.s) : bamd_launch_dense_gemm(act, d, dx, d.K, rows, dy, ldo, BAMD_OUT_GLU, s.l.s, limit)) return fail("bamd_op_dense_glu: unsupported shape");
+    const bool few = bamd_dense_few_glu(act, d, rows); const void * px = dx; int ldx = d.K;
+    if (!few && s.split(d, px, ldx, rows)) return 1;
+    if (few ? bamd_launch_dense_few_glu(d, dx, d.K, rows, dy, ldo, limit, s.l.s) : bamd_launch_dense_gemm(act, d, px, ldx, rows, dy, ldo, BAMD_OUT_GLU, s.l.s, limit)) return fail("bamd_op_dense_glu: unsupported shape");
     HIPC(hipGetLastError());
     return s.rows_back(dy, rows, F, ldo, y, act == BAMD_ACT_F32);
 }
@@ -1301,7 +1327,9 @@ BAMD_OP bamd_op_latent_attention(int act, const float * q, const float * c, cons
     else {
         bamd_launch_latent_store(act, b, a, s.l.s);
         bamd_launch_latent_gather(act, b, a, kblk, kr, kc, s.l.s);
-        rc = bamd_launch_dense_gemm(act, a.uk, kc, Rp, kr, kk, HD, BAMD_OUT_ACT, s.l.s) || bamd_launch_dense_gemm(act, a.uv, kc, Rp, kr, kv, kr, BAMD_OUT_ACT_T, s.l.s) ||
+        const void * lat = kc; int ldl = Rp;
+        if (s.split(a.uk, lat, ldl, kr)) return 1;
+        rc = bamd_launch_dense_gemm(act, a.uk, lat, ldl, kr, kk, HD, BAMD_OUT_ACT, s.l.s) || bamd_launch_dense_gemm(act, a.uv, lat, ldl, kr, kv, kr, BAMD_OUT_ACT_T, s.l.s) ||
              bamd_launch_latent_prompt(act, b, a, tiles, (int) t.size(), kk, kv, kr, s.l.s);
     }
     if (rc) return fail("bamd_op_latent_attention: unsupported shape");

@@ -78,6 +78,38 @@ def test_dense_tiles(bamd, dtype, n, rows, k):
         assert (e <= tol * (scale if impl == 0 else np.abs(want) + 0.01 * scale)).all(), impl
 
 
+# 32-bit: one size per tile (128 x 256, 128 x 128, 64 x 128, 64 x 64), ragged, and halves of three of them.  Bound: a rounding per column block and share, and what a column block's three matrix
+# instructions cut off (2^-23 each of sums that grow to it)
+@pytest.mark.parametrize("n,rows,k,route", [(8180, 1000, 1, (1, 1)), (8180, 1000, 300, (1, 1)), (8170, 500, 70, (2, 1)), (12600, 250, 300, (2, 1)), (8170, 250, 70, (3, 1)), (2040, 1000, 300, (3, 1)), (2040, 131, 1, (4, 1)),
+                                            (2040, 131, 230, (4, 1)), (4090, 500, 2100, (2, 2)), (2040, 500, 2100, (3, 2)), (500, 131, 2100, (4, 2))])
+def test_dense_split(bamd, n, rows, k, route):
+    assert bamd.op_dense_route(n, k, rows, "float32") == route
+    r = np.random.default_rng(n + k + rows)
+    w = so.f32_to_bf16(r.standard_normal((n, k), np.float32) + np.float32(0.5))
+    x = r.standard_normal((rows, k), np.float32) * np.exp(2 * r.standard_normal((rows, 1), np.float32)) + np.float32(0.5)
+    wf = so.bf16_to_f32(w).astype(np.float64)
+    want, size = x.astype(np.float64) @ wf.T, np.abs(x).astype(np.float64) @ np.abs(wf).T
+    for impl in (4,) if route[1] == 2 else (0, 2, 3):
+        assert (np.abs(bamd.op_dense(w, x, "float32", impl) - want) <= (k / 32 + 8) * 2.0 ** -24 * size).all(), impl
+
+
+# 32-bit numbers at the ends of their range: the parts a product is made of stay what they are together
+def test_dense_split_values(bamd):
+    k, r = 96, np.random.default_rng(5)
+    w = so.f32_to_bf16(np.abs(r.standard_normal((40, k), np.float32)) * np.float32(1e-3) + np.float32(1e-4))
+    x = np.abs(r.standard_normal((70, k), np.float32))
+    nan_low = np.array([0x7f800001], np.uint32).view(np.float32)[0]
+    for row, v in ((1, np.inf), (2, -np.inf), (3, nan_low), (4, np.nan), (5, np.finfo(np.float32).max), (6, -np.finfo(np.float32).max), (7, np.float32(1e-30)), (8, 0.0)):
+        x[row, 10] = v
+    x[9] = np.finfo(np.float32).max                                    # sums beyond the range
+    with np.errstate(over="ignore", invalid="ignore"):
+        want = (x.astype(np.float64) @ so.bf16_to_f32(w).T.astype(np.float64)).astype(np.float32)
+    got = bamd.op_dense(w, x, "float32", 0)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want))
+    ok = np.isfinite(want)
+    assert not np.isnan(got[1]).any() and np.isnan(got[3:5]).all() and np.allclose(got[ok], want[ok], rtol=2e-6, atol=0)
+
+
 # the same tiles where they write the clamped gated unit of their gate and up tiles in turn: widths that end inside a pair of tiles, on its edge and inside a group of four
 @pytest.mark.parametrize("dtype,F,rows,tile", [("bfloat16", 4085, 2045, 0), ("bfloat16", 4085, 1000, 1), ("bfloat16", 2032, 1000, 2), ("bfloat16", 2046, 1100, 3), ("bfloat16", 4090, 131, 4), ("bfloat16", 1001, 131, 5), ("bfloat16", 35, 70, 5),
                                                 ("float32", 1001, 131, 4)])
