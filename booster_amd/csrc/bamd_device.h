@@ -380,7 +380,9 @@ struct ActPro {
     // mid: called once behind the first workgroup barrier (NORM) / at the start (plain).  The mode-A kernels request the second half of their
     // weight ring there: a CU's texture path takes ~1.5 us to accept the requests of eight full rings, every wave sits in its issue stage
     // for that long, and the barrier behind the sum of squares waited for the last of them
-    template <bool SMALLK = false, typename MID = NoMid, int NB = BAMD_ACT_BATCH>
+    // STAGED (prompts): the sum taken again comes out of LDS, a quarter of the vector at a time (where the quants go afterwards).  Element by element out of memory it took 400 us, and of the 130 000
+    // norms of a 2048-token prompt of 32 layers a few take it: 8B, 81.6 -> 80.6 ms
+    template <bool SMALLK = false, typename MID = NoMid, int NB = BAMD_ACT_BATCH, bool STAGED = false>
     __device__ __forceinline__ void finish(const float * __restrict__ x, const float * __restrict__ nw, float eps, int K,
                                            uint32_t * q8, int * S, float * yd, double * red, MID mid = MID()) {
         const int lane = threadIdx.x & 63, wave = wave_id(), nwaves = blockDim.x >> 6, nb = K >> 8;
@@ -416,7 +418,24 @@ struct ActPro {
             float mean = (float) md;
             if (!f32_rounding_safe(md, BAMD_F64_GUARD_ULPS(K))) {     // workgroup-uniform (every thread holds the same tot); rare
                 __syncthreads();                                            // everybody has read red[]
-                if (threadIdx.x == 0) {                                     // the reference's order, one lane (ggml.c:11874-11877)
+                if constexpr (STAGED) {
+                    float * sqs = (float *) q8;
+                    double sq = 0.0;
+                    for (int c0 = 0; c0 < K; c0 += K / 4) {
+                        for (int i = threadIdx.x; i < K / 4; i += blockDim.x) { const float xv = ik_ld(x + c0 + i); sqs[i] = xv * xv; }
+                        __syncthreads();
+                        if (threadIdx.x == 0)
+                            for (int i = 0; i < K / 4; i += 16) {           // (K is a multiple of 256)
+                                float4 f[4];
+#pragma unroll
+                                for (int j = 0; j < 4; ++j) f[j] = *(const float4 *) (sqs + i + 4 * j);
+#pragma unroll
+                                for (int j = 0; j < 4; ++j) { sq += (double) f[j].x; sq += (double) f[j].y; sq += (double) f[j].z; sq += (double) f[j].w; }
+                            }
+                        __syncthreads();
+                    }
+                    if (threadIdx.x == 0) red[0] = sq;
+                } else if (threadIdx.x == 0) {                              // the reference's order, one lane (ggml.c:11874-11877)
                     double sq = 0.0;
                     for (int i = 0; i < K; ++i) { const float xv = ik_ld(x + i); sq += (double) (xv * xv); }
                     red[0] = sq;

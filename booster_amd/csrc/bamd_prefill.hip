@@ -28,7 +28,7 @@ __global__ void __launch_bounds__(512) quantize_batch_kernel(const float * __res
     uint32_t * q8 = (uint32_t *) smem; int * S = (int *) (q8 + nb * 64); float * yd = (float *) (S + nb * 8);
     double * red = (double *) (smem + BAMD_ACT_RED_OFF(nb));
     const float * xt = x + (size_t) t * K;
-    ActPro<NORM> ap; ap.issue(xt, nw, K, wave_id()); ap.finish(xt, nw, eps, K, q8, S, yd, red);
+    ActPro<NORM> ap; ap.issue(xt, nw, K, wave_id()); ap.template finish<false, typename ActPro<NORM>::NoMid, BAMD_ACT_BATCH, true>(xt, nw, eps, K, q8, S, yd, red);
     const size_t bb = BAMD_BLOB_BYTES(nb);
     if (blob) {
         const uint4 * src = (const uint4 *) smem; uint4 * dst = (uint4 *) (blob + (size_t) t * bb);

@@ -76,6 +76,23 @@ def test_gpu_equals_the_reference_on_the_constructed_vector(kat, bamd):
     assert not np.array_equal(got, kat["q8k_tree"])
 
 
+@pytest.mark.gpu
+def test_gpu_prompts_equal_the_single_token_on_the_constructed_vector(kat, bamd):
+    """the prompt's quantiser takes the sum again out of LDS, beside tokens that need no second look"""
+    from booster_amd import gguf
+    r = np.random.default_rng(3)
+    k, n = kat["x"].size, 64
+    w = r.integers(0, 256, (n * k // 256, 144), dtype=np.uint8)
+    w[:, 0:4] = np.array([0x00, 0x1c, 0x00, 0x18], np.uint8)            # d, dmin: small f16 numbers
+    w = w.reshape(-1)
+    nw, eps = np.ones(k, np.float32), float(kat["eps"])
+    x = np.stack([kat["x"], r.standard_normal(k).astype(np.float32), kat["x"][::-1].copy(), kat["x"]])
+    want = np.stack([bamd.op_mul_mat_vec(gguf.Q4_K, w, n, k, row, norm_w=nw, eps=eps) for row in x])
+    for impl in (0, 2):
+        got = bamd.op_mul_mat_batch(gguf.Q4_K, w, n, k, x, norm_w=nw, eps=eps, impl=impl)
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), impl
+
+
 # ---- the softmax denominator (ggml.c:2619-2671): a constructed row of 64 scores (tests/golden/f64_softmax_kat.npz, tools/f64_softmax_search.py)
 #      whose reciprocal sits on an f32 rounding boundary — the sequential order and a tree order of the same eight partial sums round to
 #      DIFFERENT f32 (one ulp apart), so every probability of the row depends on the order ----
