@@ -13,6 +13,9 @@
 
 enum { BAMD_ACT_BF16 = 0, BAMD_ACT_F32 = 1 };
 
+// Operand rows of products.  By rows: row r at r * ld.  By blocks (cb > 0: elements from one block of 32 columns to the next): column block, row, column — row r of block k at k * cb + r * 32.  A block's rows lie behind one another, so that a copy of sixteen of them is one kilobyte; by rows it is sixteen pieces of 64 bytes whose distance, the length of a row, is a
+// multiple of 256 bytes in most models: all sixteen come out of one channel of an L2, while every CU asks for the same ones
+inline int bamd_row_blocks(int rows) { const int by = rows > 16 ? 16 : 2; return 32 * ((rows + by - 1) / by * by); }      // groups of sixteen rows start on a kilobyte, fewer on a cache line
 struct bamd_dense { const uint16_t * w = nullptr; int rows = 0, K = 0; int row_tiles = 0, k_tiles = 0; size_t bytes = 0; };   // rows: outputs (stored: 16 row_tiles); K: stored, 32 k_tiles
 
 // one entry of a batch: n tokens of a sequence.  Row r of the step's token matrix belongs to entry row_entry[r]; its position is pos0 + (r - row0)
@@ -39,6 +42,7 @@ struct bamd_residual_args {
     const float * mu; float * prev;                // prev: [2][n_seq][E]
     const float * gi;
     float * xo; void * h; int E, ldh;              // xo [rows][E]; h [rows][ldh], zero beyond E (null: not wanted)
+    int cb;                                        // of h: 0 by rows
 };
 // A decoding step between host and device without the copy engine.  The host leaves the step's descriptors in pinned memory (`in`); the step's first kernel embeds the tokens straight
 // from there and leaves the descriptors where the others read them, its last one writes the logits to pinned memory and then `done`
@@ -54,14 +58,14 @@ void bamd_launch_embed_rows(const bamd_batch_dev & b, const uint16_t * embd, con
 void bamd_launch_residual_rows(int act, const bamd_batch_dev & b, const bamd_residual_args & a, hipStream_t s);
 int bamd_norm_threads(int n, int rows);            // threads of a block that norms one of so many rows of n
 // a N(z) + b N(z^2) + c N(z^3) + e with coef = {a, b, c, e}, N = division by the root mean square over the F values
-struct bamd_poly_args { const float * z; int ldz; const float * coef; float eps; void * h; int F, ldh; };
+struct bamd_poly_args { const float * z; int ldz; const float * coef; float eps; void * h; int F, ldh, cb; };
 void bamd_launch_poly_rows(int act, int rows, const bamd_poly_args & a, hipStream_t s);
 // clamped gated unit: g sigmoid(1.702 g) (u + 1) with g = min(gate, limit), u = clamp(up, +-limit).  z rows: 16 gate columns and 16 up columns in turn, 2 ldh in all
-struct bamd_glu_args { const float * z; int ldz; float limit; void * h; int ldh; };
+struct bamd_glu_args { const float * z; int ldz; float limit; void * h; int ldh, cb; };
 void bamd_launch_glu_rows(int act, int rows, const bamd_glu_args & a, hipStream_t s);
 #define BAMD_MAX_NORM_GROUPS 512
 // root-mean-square norm in `groups` equal parts, times w
-struct bamd_group_norm_args { const float * y; int ldy; const float * w; int groups; float eps; void * h; int n, ldh; };
+struct bamd_group_norm_args { const float * y; int ldy; const float * w; int groups; float eps; void * h; int n, ldh, cb; };
 void bamd_launch_group_norm_rows(int act, int rows, const bamd_group_norm_args & a, hipStream_t s);
 // h[i] = norm(x' of row want[i]) * gf with x' as above (the model's last norm, of the kind a.norm); xo null
 void bamd_launch_final_rows(int act, const bamd_residual_args & a, const int32_t * want, int n_want, const float * gf, hipStream_t s);
@@ -75,17 +79,17 @@ void bamd_launch_advance(bamd_entry * ent, int32_t * tokens, unsigned long long 
 // f32 [rows][ldo] | activation type [rows][ldo] | activation type, transposed [n][ldo] | activation type, the clamped gated unit of alternating 16-row tiles [rows][ldo]
 enum { BAMD_OUT_F32 = 0, BAMD_OUT_ACT = 1, BAMD_OUT_ACT_T = 2, BAMD_OUT_GLU = 3 };
 // parts: in, how many shares of K the caller can take (f32 results only; share i goes to out + i * rows * ldo); out, how many there are: one or two
-// x: rows of operands; 32-bit: what bamd_launch_split_rows made of them (6 bytes per value, ldx = 96 k_tiles)
-int bamd_launch_dense_gemm(int act, const bamd_dense & w, const void * x, int ldx, int rows, void * out, int ldo, int out_kind, hipStream_t s, float limit = 0.f, int * parts = nullptr);
-void bamd_launch_split_rows(const float * x, int ldx, int rows, int k_tiles, void * planes, hipStream_t s);
+// x: rows of operands; 32-bit: what bamd_launch_split_rows made of them.  cb: of x; GLU: cbo of the result
+int bamd_launch_dense_gemm(int act, const bamd_dense & w, const void * x, int ldx, int cb, int rows, void * out, int ldo, int out_kind, hipStream_t s, float limit = 0.f, int * parts = nullptr, int cbo = 0);
+void bamd_launch_split_rows(const float * x, int ldx, int rows, int k_tiles, void * planes, int cb, hipStream_t s);      // by blocks of three planes: [k_tiles][cb], row r at r * 96
 // few rows (<= BAMD_MV_ROWS): the weights stream once; out f32 [rows][ldo].  pre: how the operand comes about —
 enum { BAMD_PRE_ROWS = 0, BAMD_PRE_RESIDUAL = 1, BAMD_PRE_POLY = 2, BAMD_PRE_GROUP = 3, BAMD_PRE_FINAL = 4, BAMD_PRE_GLU = 5, BAMD_PRE_LAYER = 6 };     // (LAYER: RESIDUAL and FINAL with layer norms, chosen by res.norm); x given | one row, built in front of the product from the argument block
 struct bamd_pre_args { bamd_residual_args res; bamd_poly_args poly; bamd_group_norm_args grp; bamd_glu_args glu; const float * gf; const int32_t * want; };
 #define BAMD_MV_ROWS 64
-int bamd_launch_dense_mv(int act, const bamd_dense & w, int pre, const bamd_batch_dev & b, const bamd_pre_args * p, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s, int * parts = nullptr);
+int bamd_launch_dense_mv(int act, const bamd_dense & w, int pre, const bamd_batch_dev & b, const bamd_pre_args * p, const void * x, int ldx, int cb, int rows, float * out, int ldo, hipStream_t s, int * parts = nullptr);
 // a few rows of the product with gate and up rows in turn, and the gated unit of its results, operands of the product behind, to h.  bamd_dense_few_glu: it is covered
 bool bamd_dense_few_glu(int act, const bamd_dense & w, int rows);
-int bamd_launch_dense_few_glu(const bamd_dense & w, const void * x, int ldx, int rows, void * h, int ldh, float limit, hipStream_t s);
+int bamd_launch_dense_few_glu(const bamd_dense & w, const void * x, int ldx, int cb, int rows, void * h, int ldh, int cbo, float limit, hipStream_t s);
 int bamd_dense_route(int act, const bamd_dense & w, int rows, int pre, int most, int & share);      // many rows (pre < 0): the tile; few rows: -1; share: shares of K, of at most `most`
 size_t bamd_dense_mv_lds(int act, int K);         // operand bytes of a built row: must stay within BAMD_MV_LDS
 #define BAMD_MV_LDS (96 * 1024)
@@ -112,7 +116,7 @@ struct bamd_latent_args {
     void * cache;                                  // [pages][BAMD_PAGE][Rp]
     const uint16_t * ukT;                          // decode: per head the packed transpose of the key up-projection [Rp][D]
     bamd_dense uk, uv;
-    void * out; int ldo;                           // [rows][ldo], heads x D
+    void * out; int ldo, cb;                       // [rows][ldo] or by blocks, heads x D
 };
 struct bamd_qtile { int32_t entry, q0; };
 void bamd_launch_latent_store(int act, const bamd_batch_dev & b, const bamd_latent_args & a, hipStream_t s);
@@ -135,7 +139,7 @@ struct bamd_kv_args {
     const float * bias; int bias_top;              // [heads][bias_top + 1] by distance, the last for everything farther; null: none
     int window, keep;
     void * kc, * vc;                               // [pages][kv_heads][BAMD_PAGE][D] and, transposed, [pages][kv_heads][D][BAMD_PAGE]
-    float out_scale; void * out; int ldo, out_off; // [rows][ldo], heads x D from column out_off on
+    float out_scale; void * out; int ldo, out_off, cb; // [rows][ldo] or by blocks, heads x D from column out_off on
 };
 void bamd_launch_kv_store(int act, const bamd_batch_dev & b, const bamd_kv_args & a, const int32_t * k_entry, int k_rows, hipStream_t s);
 int bamd_launch_kv_prompt(int act, const bamd_batch_dev & b, const bamd_kv_args & a, const bamd_qtile * tiles, int n_tiles, hipStream_t s);
@@ -160,7 +164,7 @@ struct bamd_gla_args {
     int heads, Np, Pp;                             // channels and columns per head, padded to a multiple of four
     // what reads y: per head y / sqrt(mean(y^2) + eps) * norm, times silu of the gate
     int g_off, P; const float * norm; float eps;   // heads x Pp of the projection (-1: no gate); columns the mean counts; [Pp], zero beyond P
-    void * out; int ldo, out_off, out_cols;        // [rows][ldo], heads x Pp from column out_off on, zero up to out_cols
+    void * out; int ldo, out_off, out_cols, cb;    // [rows][ldo] or by blocks, heads x Pp from column out_off on, zero up to out_cols
 };
 // a prompt portion is scanned in segments: the states at their starts come from a first scan of every segment alone
 struct bamd_segment { int32_t entry, t0, n, first, last; };       // first, last: of the entry's segments

@@ -24,7 +24,7 @@ void bamd_launch_pack(const uint16_t * src, const int32_t * row_off, const int32
 // ---- many rows --------------------------------------------------------------------------------------------------------------------------------------
 // one 16 x 16 result tile of a wave: activation rows from mb, matrix rows from nb; a: the tiles of the same activation rows, j: which one
 template <typename T, int OUT, int NI>
-__device__ __forceinline__ void store_tile(const bamd_v4 (&a)[NI], int j, int mb, int nb, int n_lim, int n_rows, int rows, void * out, int ldo, float limit, int lane) {
+__device__ __forceinline__ void store_tile(const bamd_v4 (&a)[NI], int j, int mb, int nb, int n_lim, int n_rows, int rows, void * out, int ldo, int cbo, float limit, int lane) {
     if (nb >= n_lim) return;
     if constexpr (OUT == BAMD_OUT_ACT_T) {
         const int n = nb + (lane & 15), m = mb + (lane >> 4) * 4;
@@ -37,7 +37,7 @@ __device__ __forceinline__ void store_tile(const bamd_v4 (&a)[NI], int j, int mb
         bamd_v4 o;
 #pragma unroll
         for (int k = 0; k < 4; ++k) o[k] = clamped_glu(a[j][k], a[j | 1][k], limit);
-        store4<T>((T *) out + (size_t) m * ldo + n, o);
+        store4<T>(row_out<T>(out, m, ldo, cbo).at(n), o);
     } else {
         const int n = nb + (lane >> 4) * 4, m = mb + (lane & 15);
         if (m >= rows) return;
@@ -55,8 +55,8 @@ __device__ __forceinline__ void store_tile(const bamd_v4 (&a)[NI], int j, int mb
 // A 32-bit activation is the sum of three bfloat16 numbers, eight bits of its significand each (cut off, not rounded: parts of one sign, and what is left is exact), and products of bfloat16
 // numbers are exact in 32 bits: three bfloat16 matrix instructions do what eight of 16x16x4_f32 did, with three roundings of a sum per 32 columns for thirty-two.
 template <typename T> constexpr int bamd_planes = sizeof(T) == 4 ? 3 : 1;
-// rows [rows][ldx] of 32 k_tiles floats -> [rows][k_tiles][3 planes][32].  A value that is not finite is its first plane alone
-__global__ void __launch_bounds__(256) split_rows_kernel(const float * __restrict__ x, int ldx, int k_tiles, uint16_t * __restrict__ planes) {
+// rows [rows][ldx] of 32 k_tiles floats -> blocks of 32 columns: [k_tiles][cb], in them [rows][3 planes][32].  A value that is not finite is its first plane alone
+__global__ void __launch_bounds__(256) split_rows_kernel(const float * __restrict__ x, int ldx, int k_tiles, uint16_t * __restrict__ planes, int cb) {
     const int i = (blockIdx.x * 256 + threadIdx.x) * 8;
     if (i >= k_tiles * 32) return;
     const float * p = x + (size_t) blockIdx.y * ldx + i;
@@ -77,12 +77,12 @@ __global__ void __launch_bounds__(256) split_rows_kernel(const float * __restric
 #pragma unroll
         for (int n = 0; n < 3; ++n) h[n][c] = (part[0][n] >> 16) | (part[1][n] & 0xffff0000u);
     }
-    uint16_t * d = planes + (size_t) blockIdx.y * k_tiles * 96 + (i >> 5) * 96 + (i & 31);
+    uint16_t * d = planes + (size_t) (i >> 5) * cb + blockIdx.y * 96 + (i & 31);
 #pragma unroll
     for (int n = 0; n < 3; ++n) *(bamd_u4 *) (d + n * 32) = bamd_u4{ h[n][0], h[n][1], h[n][2], h[n][3] };
 }
-void bamd_launch_split_rows(const float * x, int ldx, int rows, int k_tiles, void * planes, hipStream_t s) {
-    hipLaunchKernelGGL(split_rows_kernel, dim3((k_tiles * 4 + 255) / 256, rows), dim3(256), 0, s, x, ldx, k_tiles, (uint16_t *) planes);
+void bamd_launch_split_rows(const float * x, int ldx, int rows, int k_tiles, void * planes, int cb, hipStream_t s) {
+    hipLaunchKernelGGL(split_rows_kernel, dim3((k_tiles * 4 + 255) / 256, rows), dim3(256), 0, s, x, ldx, k_tiles, (uint16_t *) planes, cb);
 }
 // TM activation rows x TN matrix rows per block of WM x WN waves.  Both operands travel global -> LDS by DMA (a kilobyte per instruction: 16 rows x 32 columns), NS stages
 // of 32 columns deep: while the matrix instructions of column block k run from registers, the fragments of k + 1 are read from LDS and the copies of the NS - 2 blocks
@@ -91,12 +91,13 @@ void bamd_launch_split_rows(const float * x, int ldx, int rows, int k_tiles, voi
 // all of them in front of the first costs 15 %.
 // Activations lie in LDS as they come from memory, four lanes on 64 consecutive bytes of a row (one 16-byte piece of 16 rows per four lanes costs the vector memory path
 // four times the lookups: 446 -> 409 us below), the pieces of a row turned by half its number: sixteen rows of one piece then fall on different banks.
+// Rows by blocks (bamd_dense.h), 2048 of them: 256 x 256 tiles 0 to 4 % (8448 outputs 319 -> 305 us), 128 x 256 6 to 7 % (149 -> 138).
 // 32-bit (three planes of activations): the sums of a column block start at zero and are added to the accumulators by the vector units, a row of tiles behind.  The matrix instructions cut off
 // where the vector units round: kept in them from one column block to the next, a sum of 14336 positive products was off by 6.3e-6 (1.8e-6 with the f32 instructions), so it is 3.2e-7 (and
 // 4.1e-7 for 2.2e-6 with random signs).  500 x 8192 x 2048 118 -> 46 us, 500 x 12608 x 2048 178 -> 75, 500 x 2048 x 8192 122 -> 63.
 // 2048 x 28672 x 4096: 676 -> 409 us (1176 TFLOP/s); 2048 x 4096 x 14336: 284 -> 185 us (1303); 2048 x 2048 x 2048: 41 -> 22 us; 131 x 8192 x 2048: 23 -> 16 us.
 template <typename T, int TM, int TN, int WM, int WN, int NS, int OUT>
-__global__ void __launch_bounds__(64 * WM * WN) dense_tile_kernel(bamd_dense w, const bamd_bf * x, int ldx, int rows, void * out, int ldo, int n_mt, int n_nt, float limit) {
+__global__ void __launch_bounds__(64 * WM * WN) dense_tile_kernel(bamd_dense w, const bamd_bf * x, int ldx, int cb, int rows, void * out, int ldo, int cbo, int n_mt, int n_nt, float limit) {
     const int kb = (int) ((long) w.k_tiles * blockIdx.y / gridDim.y), nk = (int) ((long) w.k_tiles * (blockIdx.y + 1) / gridDim.y) - kb;      // this block's share of K
     constexpr int XT = TM / 16, WT = TN / 16, NW = WM * WN, MI = XT / WM, NI = WT / WN, XP = bamd_planes<T>, PX = XT * XP / NW, PW = WT / NW, PER = PX + PW, STAGE = (XT * XP + WT) * 1024;
     static_assert(XT * XP % NW == 0 && (XP == 1 || MI % 2 == 0) && WT % NW == 0 && MI * WM == XT && NI * WN == WT && NS >= 4 && (NS & (NS - 1)) == 0, "");
@@ -107,7 +108,7 @@ __global__ void __launch_bounds__(64 * WM * WN) dense_tile_kernel(bamd_dense w, 
     { const int per = (total + 7) / 8, xcd = id & 7, k = id >> 3; id = xcd * per + k; if (k >= per || id >= total) return; }
     const int mt = id % n_mt, nt = id / n_mt, m0 = mt * TM, n0t = nt * WT;
     // this wave's share of a stage: PX operand blocks of activations, PW of weights
-    const unsigned char * xbase = (const unsigned char *) (x + (size_t) m0 * ldx + (size_t) kb * (32 * XP)), * wbase = (const unsigned char *) (w.w + ((size_t) n0t * w.k_tiles + kb) * 512);
+    const unsigned char * xbase = (const unsigned char *) (x + (size_t) m0 * ldx + (size_t) kb * cb), * wbase = (const unsigned char *) (w.w + ((size_t) n0t * w.k_tiles + kb) * 512);
     uint32_t xo[PX], wo[PW];
 #pragma unroll
     for (int i = 0; i < PX; ++i) {                                // 16 rows of four 16-byte pieces, of one plane
@@ -123,7 +124,7 @@ __global__ void __launch_bounds__(64 * WM * WN) dense_tile_kernel(bamd_dense w, 
     auto copy = [&](int k, int i) {
         const int kk = k < nk ? k : nk - 1;
         const uint32_t st = (uint32_t) (k & (NS - 1)) * STAGE;
-        if (i < PX) lds_dma16_s(xbase + (size_t) kk * (64 * XP), xo[i], xd + st + i * 1024u);
+        if (i < PX) lds_dma16_s(xbase + (size_t) kk * cb * 2, xo[i], xd + st + i * 1024u);
         else lds_dma16_s(wbase + (size_t) kk * 1024, wo[i - PX], wd + st + (i - PX) * 1024u);
     };
     const int wm = wave % WM, wn = wave / WM;
@@ -197,12 +198,12 @@ __global__ void __launch_bounds__(64 * WM * WN) dense_tile_kernel(bamd_dense w, 
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < NI; ++j) store_tile<T, OUT>(acc[i], j, m0 + (wm * MI + i) * 16, (n0t + wn * NI + j) * 16, n_lim, w.rows, rows, out, ldo, limit, lane);
+        for (int j = 0; j < NI; ++j) store_tile<T, OUT>(acc[i], j, m0 + (wm * MI + i) * 16, (n0t + wn * NI + j) * 16, n_lim, w.rows, rows, out, ldo, cbo, limit, lane);
 }
 template <typename T, int TM, int TN, int WM, int WN, int NS, int OUT>
-static int tile_go(const bamd_dense & w, const void * x, int ldx, int rows, void * out, int ldo, float limit, int parts, hipStream_t s) {
+static int tile_go(const bamd_dense & w, const void * x, int ldx, int cb, int rows, void * out, int ldo, int cbo, float limit, int parts, hipStream_t s) {
     const int n_mt = (rows + TM - 1) / TM, n_nt = (w.row_tiles + TN / 16 - 1) / (TN / 16), per = (n_mt * n_nt + 7) / 8;
-    hipLaunchKernelGGL((dense_tile_kernel<T, TM, TN, WM, WN, NS, OUT>), dim3(per * 8, parts), dim3(64 * WM * WN), (size_t) NS * (TM / 16 * bamd_planes<T> + TN / 16) * 1024, s, w, (const bamd_bf *) x, ldx, rows, out, ldo, n_mt, n_nt, limit);
+    hipLaunchKernelGGL((dense_tile_kernel<T, TM, TN, WM, WN, NS, OUT>), dim3(per * 8, parts), dim3(64 * WM * WN), (size_t) NS * (TM / 16 * bamd_planes<T> + TN / 16) * 1024, s, w, (const bamd_bf *) x, ldx, cb, rows, out, ldo, cbo, n_mt, n_nt, limit);
     return 0;
 }
 // The tile whose rounds over the 256 CUs end first.  Measured per block of 32 columns, all CUs busy (ns): 256 x 256 700, 128 x 256 450, 128 x 128 250, all three one block per CU,
@@ -243,39 +244,43 @@ static int pick_tile(int act, const bamd_dense & w, int rows, int most, int & sh
     return pick == TILE_64_64 && tiles(64, 64) * share <= 256 ? TILE_64_64_DEEP : pick;
 }
 template <typename T, int OUT>
-static int gemm_tiles(const bamd_dense & w, const void * x, int ldx, int rows, void * out, int ldo, float limit, hipStream_t s, int * parts = nullptr) {
+static int gemm_tiles(const bamd_dense & w, const void * x, int ldx, int cb, int rows, void * out, int ldo, int cbo, float limit, hipStream_t s, int * parts = nullptr) {
     int share;
     const int tile = pick_tile(sizeof(T) == 4 ? BAMD_ACT_F32 : BAMD_ACT_BF16, w, rows, OUT == BAMD_OUT_F32 && parts ? *parts : 1, share);
     if (parts) *parts = share;
     if constexpr (sizeof(T) == 2) switch (tile) {
-        case TILE_256_256: return tile_go<T, 256, 256, 2, 4, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
-        case TILE_128_256: return tile_go<T, 128, 256, 2, 4, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
-        case TILE_128_128: return tile_go<T, 128, 128, 2, 4, 8, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
-        case TILE_64_128: return tile_go<T, 64, 128, 2, 2, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
-        case TILE_64_64_DEEP: return tile_go<T, 64, 64, 2, 2, 8, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
+        case TILE_256_256: return tile_go<T, 256, 256, 2, 4, 4, OUT>(w, x, ldx, cb, rows, out, ldo, cbo, limit, share, s);
+        case TILE_128_256: return tile_go<T, 128, 256, 2, 4, 4, OUT>(w, x, ldx, cb, rows, out, ldo, cbo, limit, share, s);
+        case TILE_128_128: return tile_go<T, 128, 128, 2, 4, 8, OUT>(w, x, ldx, cb, rows, out, ldo, cbo, limit, share, s);
+        case TILE_64_128: return tile_go<T, 64, 128, 2, 2, 4, OUT>(w, x, ldx, cb, rows, out, ldo, cbo, limit, share, s);
+        case TILE_64_64_DEEP: return tile_go<T, 64, 64, 2, 2, 8, OUT>(w, x, ldx, cb, rows, out, ldo, cbo, limit, share, s);
     }
     else switch (tile) {                                          // three planes of activations: waves as tall as wide would read twice as much of them
-        case TILE_128_256: return tile_go<T, 128, 256, 2, 4, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
-        case TILE_128_128: return tile_go<T, 128, 128, 4, 2, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
-        case TILE_64_128: return tile_go<T, 64, 128, 2, 2, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
+        case TILE_128_256: return tile_go<T, 128, 256, 2, 4, 4, OUT>(w, x, ldx, cb, rows, out, ldo, cbo, limit, share, s);
+        case TILE_128_128: return tile_go<T, 128, 128, 4, 2, 4, OUT>(w, x, ldx, cb, rows, out, ldo, cbo, limit, share, s);
+        case TILE_64_128: return tile_go<T, 64, 128, 2, 2, 4, OUT>(w, x, ldx, cb, rows, out, ldo, cbo, limit, share, s);
     }
-    return tile_go<T, 64, 64, 2, 2, 4, OUT>(w, x, ldx, rows, out, ldo, limit, share, s);
+    return tile_go<T, 64, 64, 2, 2, 4, OUT>(w, x, ldx, cb, rows, out, ldo, cbo, limit, share, s);
 }
-// f32 rows are stored four matrix rows at a time: ldo % 4 == 0; x rows start on 16 bytes and hold k_tiles * 32 columns
+// operand rows start on 16 bytes and hold k_tiles * 32 columns, or lie by blocks
+static bool rows_fit(const bamd_dense & w, int ldx, int cb, int rows, int in_block) { return cb ? cb >= in_block * rows && !(cb & 7) : ldx >= w.k_tiles * in_block && !(ldx & 7); }
+// f32 rows are stored four matrix rows at a time: ldo % 4 == 0
 template <typename T>
-static int gemm_out(const bamd_dense & w, const void * x, int ldx, int rows, void * out, int ldo, int kind, float limit, hipStream_t s, int * parts) {
+static int gemm_out(const bamd_dense & w, const void * x, int ldx, int cb, int rows, void * out, int ldo, int cbo, int kind, float limit, hipStream_t s, int * parts) {
     if (kind != BAMD_OUT_F32 && parts) *parts = 1;
     switch (kind) {
-        case BAMD_OUT_F32: return gemm_tiles<T, BAMD_OUT_F32>(w, x, ldx, rows, out, ldo, limit, s, parts);
-        case BAMD_OUT_ACT: return gemm_tiles<T, BAMD_OUT_ACT>(w, x, ldx, rows, out, ldo, limit, s);
-        case BAMD_OUT_ACT_T: return gemm_tiles<T, BAMD_OUT_ACT_T>(w, x, ldx, rows, out, ldo, limit, s);
-        case BAMD_OUT_GLU: return (w.row_tiles & 1) || ldo < w.row_tiles * 8 ? 1 : gemm_tiles<T, BAMD_OUT_GLU>(w, x, ldx, rows, out, ldo, limit, s);
+        case BAMD_OUT_F32: return gemm_tiles<T, BAMD_OUT_F32>(w, x, ldx, cb, rows, out, ldo, 0, limit, s, parts);
+        case BAMD_OUT_ACT: return gemm_tiles<T, BAMD_OUT_ACT>(w, x, ldx, cb, rows, out, ldo, 0, limit, s);
+        case BAMD_OUT_ACT_T: return gemm_tiles<T, BAMD_OUT_ACT_T>(w, x, ldx, cb, rows, out, ldo, 0, limit, s);
+        case BAMD_OUT_GLU: return (w.row_tiles & 1) || ldo < w.row_tiles * 8 ? 1 : gemm_tiles<T, BAMD_OUT_GLU>(w, x, ldx, cb, rows, out, ldo, cbo, limit, s);
     }
     return 1;
 }
-int bamd_launch_dense_gemm(int act, const bamd_dense & w, const void * x, int ldx, int rows, void * out, int ldo, int kind, hipStream_t s, float limit, int * parts) {
-    if (rows < 1 || w.row_tiles < 1 || w.k_tiles < 1 || ldx < w.k_tiles * (act == BAMD_ACT_F32 ? 96 : 32) || (ldx & 7) || (ldo & 3)) return 1;
-    return act == BAMD_ACT_F32 ? gemm_out<float>(w, x, ldx, rows, out, ldo, kind, limit, s, parts) : gemm_out<bamd_bf>(w, x, ldx, rows, out, ldo, kind, limit, s, parts);
+int bamd_launch_dense_gemm(int act, const bamd_dense & w, const void * x, int ldx, int cb, int rows, void * out, int ldo, int kind, hipStream_t s, float limit, int * parts, int cbo) {
+    const int in_block = act == BAMD_ACT_F32 ? 96 : 32;
+    if (rows < 1 || w.row_tiles < 1 || w.k_tiles < 1 || (ldo & 3) || !rows_fit(w, ldx, cb, rows, in_block)) return 1;
+    if (cb) ldx = in_block; else cb = in_block;
+    return act == BAMD_ACT_F32 ? gemm_out<float>(w, x, ldx, cb, rows, out, ldo, cbo, kind, limit, s, parts) : gemm_out<bamd_bf>(w, x, ldx, cb, rows, out, ldo, cbo, kind, limit, s, parts);
 }
 
 // ---- few rows ---------------------------------------------------------------------------------------------------------------------------------------
@@ -298,7 +303,7 @@ __global__ void __launch_bounds__(64 * NW) dense_mv_kernel(bamd_dense w, bamd_ba
     int tile = blockIdx.x;
     request(tile, 0, cur);                                        // on their way while the operand row is built
     if constexpr (PRE != BAMD_PRE_ROWS) {
-        T * h = (T *) lds;
+        const RowOut<T> h = { (T *) lds, 32 };
         if constexpr (PRE == BAMD_PRE_RESIDUAL) residual_row<T, true>(b, p.res, 0, h, blockIdx.x == 0, red);
         if constexpr (PRE == BAMD_PRE_POLY) poly_row<T>(p.poly, 0, h, red);
         if constexpr (PRE == BAMD_PRE_GROUP) group_norm_row<T>(p.grp, 0, h, red);
@@ -353,9 +358,11 @@ __global__ void __launch_bounds__(64 * NW) dense_mv_kernel(bamd_dense w, bamd_ba
 // wave streams its share of K — RT KiB of weights and NT of the rows per step — by DMA through a ring of NS steps of its own: 64 consecutive bytes of a row per four lanes, read
 // back in fragment order (dense_tile_kernel's layout), no barrier between steps, and while the sums of a group of tiles meet, the next group's first steps are under way.  LDS holds
 // one block of eight waves per CU.  16 x 14336 x 4096: 32.3 -> 27.1 us (4.3 TB/s of weights), 16 x 32000 x 4096: 62 -> 50 (5.3), 45 x 4096 x 14336: 57 -> 48 us.
+// Rows by blocks (bamd_dense.h): a step of eight layers, sixteen rows 1390 -> 1318 us (width 4096), 835 -> 817 (2048), 32 rows 1918 -> 1737 and 1226 -> 1143, 64 rows 2772 -> 2493 and 1716 -> 1573; up to six
+// rows, where the few there are cost little, level.
 // GLU (an even RT): gate and up tiles in turn; out is the gated unit's bfloat16 row.
 template <int NT, int RT, int NS, bool GLU>
-__global__ void __launch_bounds__(512) dense_few_kernel(bamd_dense w, const bamd_bf * x, int ldx, int rows, float * out, int ldo, float limit) {
+__global__ void __launch_bounds__(512) dense_few_kernel(bamd_dense w, const bamd_bf * x, int ldx, int cb, int rows, float * out, int ldo, int cbo, float limit) {
     constexpr int NW = 8, STEP = (NT + RT) * 1024, RING = NS * STEP;
     extern __shared__ __align__(16) unsigned char lds[];
     float * red = (float *) (lds + NW * RING);                    // [wave][RT][NT][64 lanes][4]
@@ -377,7 +384,7 @@ __global__ void __launch_bounds__(512) dense_few_kernel(bamd_dense w, const bamd
             lds_dma16_s(w.w + ((size_t) tile * w.k_tiles + k) * 512, (uint32_t) lane * 16u, ring + (uint32_t) cs * STEP + 1024u * t);
         }
 #pragma unroll
-        for (int g = 0; g < NT; ++g) lds_dma16_s((const unsigned char *) x + k * 64, xo[g], ring + (uint32_t) cs * STEP + 1024u * (g + RT));
+        for (int g = 0; g < NT; ++g) lds_dma16_s((const unsigned char *) x + k * cb * 2, xo[g], ring + (uint32_t) cs * STEP + 1024u * (g + RT));
         cs = cs + 1 < NS ? cs + 1 : 0;
         if (ck + 1 < n) ++ck; else if (ct + (int) gridDim.x < groups) { ck = 0; ct += gridDim.x; }
     };
@@ -424,7 +431,7 @@ __global__ void __launch_bounds__(512) dense_few_kernel(bamd_dense w, const bamd
         if constexpr (GLU) {
             for (int i = tid; i < RT / 2 * NT * 256; i += 64 * NW) {
                 const int c = i >> 8, t = c / NT * 2, l = (i >> 2) & 63, k = i & 3, r = (c % NT) * 16 + (l & 15), o = (grp * RT + t) * 8 + (l >> 4) * 4 + k;
-                if (r < rows && o < w.rows / 2) ((bamd_bf *) out)[(size_t) r * ldo + o] = (bamd_bf) clamped_glu(sum(t * NT + c % NT, l, k), sum((t + 1) * NT + c % NT, l, k), limit);
+                if (r < rows && o < w.rows / 2) *row_out<bamd_bf>(out, r, ldo, cbo).at(o) = (bamd_bf) clamped_glu(sum(t * NT + c % NT, l, k), sum((t + 1) * NT + c % NT, l, k), limit);
             }
         } else for (int i = tid; i < RT * NT * 256; i += 64 * NW) {
             const int c = i >> 8, l = (i >> 2) & 63, k = i & 3, r = (c % NT) * 16 + (l & 15), o = (grp * RT + c / NT) * 16 + (l >> 4) * 4 + k;
@@ -434,24 +441,24 @@ __global__ void __launch_bounds__(512) dense_few_kernel(bamd_dense w, const bamd
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");              // (no copy outlives the block)
 }
 template <int NT, int RT, int NS, bool GLU = false>
-static void few_go(const bamd_dense & w, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s, int parts = 1, float limit = 0.f) {
+static void few_go(const bamd_dense & w, const void * x, int ldx, int cb, int rows, float * out, int ldo, hipStream_t s, int parts = 1, int cbo = 0, float limit = 0.f) {
     const int groups = (w.row_tiles + RT - 1) / RT;
-    hipLaunchKernelGGL((dense_few_kernel<NT, RT, NS, GLU>), dim3(groups < 256 ? groups : 256, parts), dim3(512), (size_t) 8 * (NS * (NT + RT) + NT * RT) * 1024, s, w, (const bamd_bf *) x, ldx, rows, out, ldo, limit);
+    hipLaunchKernelGGL((dense_few_kernel<NT, RT, NS, GLU>), dim3(groups < 256 ? groups : 256, parts), dim3(512), (size_t) 8 * (NS * (NT + RT) + NT * RT) * 1024, s, w, (const bamd_bf *) x, ldx, cb, rows, out, ldo, cbo, limit);
 }
 // RT by the rounds over the CUs; a round of 1, 2 or 3 tiles at K = 4096 takes 7.1, 12.7 and 16 us with up to 16 rows, one of 1 or 2 tiles 9.0 and 15.1 us with up to 32.
 // With more rows the 64 x 64 tiles of prompts are ahead once they fill the CUs (45 x 22672 x 4096: 49 against 74 us) and behind before (45 x 4096 x 14336: 136 against 48)
-static int few_pick(const bamd_dense & w, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s, int parts) {
+static int few_pick(const bamd_dense & w, const void * x, int ldx, int cb, int rows, float * out, int ldo, hipStream_t s, int parts) {
     const long rounds[3] = { (w.row_tiles + 255) / 256, (w.row_tiles + 511) / 512, (w.row_tiles + 767) / 768 };
     if (rows > 32) {
-        if (w.row_tiles > 768 && (ldo & 3) == 0) return gemm_tiles<bamd_bf, BAMD_OUT_F32>(w, x, ldx, rows, out, ldo, 0.f, s);
-        few_go<4, 1, 3>(w, x, ldx, rows, out, ldo, s, parts);
+        if (w.row_tiles > 768 && (ldo & 3) == 0) return gemm_tiles<bamd_bf, BAMD_OUT_F32>(w, x, ldx, cb, rows, out, ldo, 0, 0.f, s);
+        few_go<4, 1, 3>(w, x, ldx, cb, rows, out, ldo, s, parts);
     } else if (rows > 16) {
-        if (rounds[0] * 90 <= rounds[1] * 151) few_go<2, 1, 5>(w, x, ldx, rows, out, ldo, s, parts); else few_go<2, 2, 4>(w, x, ldx, rows, out, ldo, s);
+        if (rounds[0] * 90 <= rounds[1] * 151) few_go<2, 1, 5>(w, x, ldx, cb, rows, out, ldo, s, parts); else few_go<2, 2, 4>(w, x, ldx, cb, rows, out, ldo, s);
     } else {
         const long t1 = rounds[0] * 71, t2 = rounds[1] * 127, t3 = rounds[2] * 160;
-        if (t1 <= t2 && t1 <= t3) few_go<1, 1, 5>(w, x, ldx, rows, out, ldo, s, parts);
-        else if (t2 <= t3) few_go<1, 2, 5>(w, x, ldx, rows, out, ldo, s);
-        else few_go<1, 3, 4>(w, x, ldx, rows, out, ldo, s);
+        if (t1 <= t2 && t1 <= t3) few_go<1, 1, 5>(w, x, ldx, cb, rows, out, ldo, s, parts);
+        else if (t2 <= t3) few_go<1, 2, 5>(w, x, ldx, cb, rows, out, ldo, s);
+        else few_go<1, 3, 4>(w, x, ldx, cb, rows, out, ldo, s);
     }
     return 0;
 }
@@ -482,7 +489,7 @@ int bamd_dense_route(int act, const bamd_dense & w, int rows, int pre, int most,
     return -1;
 }
 template <typename T>
-static int mv_pick(const bamd_dense & w, int pre, const bamd_batch_dev & b, const bamd_pre_args & p, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s, int * parts) {
+static int mv_pick(const bamd_dense & w, int pre, const bamd_batch_dev & b, const bamd_pre_args & p, const void * x, int ldx, int cb, int rows, float * out, int ldo, hipStream_t s, int * parts) {
     const int n = few_parts(sizeof(T) == 4 ? BAMD_ACT_F32 : BAMD_ACT_BF16, w, pre, parts ? *parts : 1);
     if (parts) *parts = n;
     if (pre != BAMD_PRE_ROWS) {
@@ -497,8 +504,8 @@ static int mv_pick(const bamd_dense & w, int pre, const bamd_batch_dev & b, cons
         else mv_one<T, BAMD_PRE_FINAL>(w, b, p, x, ldx, rows, out, ldo, s);
         return 0;
     }
-    if (rows < 1 || rows > BAMD_MV_ROWS || ldx < w.k_tiles * 32 || (ldx & 7)) return 1;
-    if constexpr (sizeof(T) == 2) return few_pick(w, x, ldx, rows, out, ldo, s, n);
+    if (rows < 1 || rows > BAMD_MV_ROWS || (sizeof(T) == 4 && cb) || !rows_fit(w, ldx, cb, rows, 32)) return 1;
+    if constexpr (sizeof(T) == 2) return few_pick(w, x, cb ? 32 : ldx, cb ? cb : 32, rows, out, ldo, s, n);
     else if (rows <= 16) mv_one<T, BAMD_PRE_ROWS>(w, b, p, x, ldx, rows, out, ldo, s, n);
     else if (rows <= 32) mv_go<T, 2, 8, BAMD_PRE_ROWS>(w, b, p, x, ldx, rows, out, ldo, s, n);
     else mv_go<T, 4, 8, BAMD_PRE_ROWS>(w, b, p, x, ldx, rows, out, ldo, s, n);
@@ -509,13 +516,14 @@ static int mv_pick(const bamd_dense & w, int pre, const bamd_batch_dev & b, cons
 // without) 6 rows 1368 -> 1350, 16 1683 -> 1660.  Four tiles a block: 666, 848; 1394, 1684.  More rows: where few_pick takes the tiles of prompts, they have the unit as well
 // (64 rows 3181 -> 3141)
 bool bamd_dense_few_glu(int act, const bamd_dense & w, int rows) { return act == BAMD_ACT_BF16 && !(w.row_tiles & 1) && rows > 1 && (rows <= 32 || (rows <= BAMD_MV_ROWS && w.row_tiles > 768)); }
-int bamd_launch_dense_few_glu(const bamd_dense & w, const void * x, int ldx, int rows, void * h, int ldh, float limit, hipStream_t s) {
-    if (!bamd_dense_few_glu(BAMD_ACT_BF16, w, rows) || ldx < w.k_tiles * 32 || (ldx & 7) || ldh < w.row_tiles * 8 || (ldh & 3)) return 1;
-    if (rows > 32) return gemm_tiles<bamd_bf, BAMD_OUT_GLU>(w, x, ldx, rows, h, ldh, limit, s);
-    if (rows > 16) few_go<2, 2, 4, true>(w, x, ldx, rows, (float *) h, ldh, s, 1, limit); else few_go<1, 2, 5, true>(w, x, ldx, rows, (float *) h, ldh, s, 1, limit);
+int bamd_launch_dense_few_glu(const bamd_dense & w, const void * x, int ldx, int cb, int rows, void * h, int ldh, int cbo, float limit, hipStream_t s) {
+    if (!bamd_dense_few_glu(BAMD_ACT_BF16, w, rows) || !rows_fit(w, ldx, cb, rows, 32) || ldh < w.row_tiles * 8 || (ldh & 3)) return 1;
+    if (cb) ldx = 32; else cb = 32;
+    if (rows > 32) return gemm_tiles<bamd_bf, BAMD_OUT_GLU>(w, x, ldx, cb, rows, h, ldh, cbo, limit, s);
+    if (rows > 16) few_go<2, 2, 4, true>(w, x, ldx, cb, rows, (float *) h, ldh, s, 1, cbo, limit); else few_go<1, 2, 5, true>(w, x, ldx, cb, rows, (float *) h, ldh, s, 1, cbo, limit);
     return 0;
 }
-int bamd_launch_dense_mv(int act, const bamd_dense & w, int pre, const bamd_batch_dev & b, const bamd_pre_args * p, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s, int * parts) {
+int bamd_launch_dense_mv(int act, const bamd_dense & w, int pre, const bamd_batch_dev & b, const bamd_pre_args * p, const void * x, int ldx, int cb, int rows, float * out, int ldo, hipStream_t s, int * parts) {
     static const bamd_pre_args none = {};
-    return act == BAMD_ACT_F32 ? mv_pick<float>(w, pre, b, p ? *p : none, x, ldx, rows, out, ldo, s, parts) : mv_pick<bamd_bf>(w, pre, b, p ? *p : none, x, ldx, rows, out, ldo, s, parts);
+    return act == BAMD_ACT_F32 ? mv_pick<float>(w, pre, b, p ? *p : none, x, ldx, cb, rows, out, ldo, s, parts) : mv_pick<bamd_bf>(w, pre, b, p ? *p : none, x, ldx, cb, rows, out, ldo, s, parts);
 }

@@ -134,7 +134,14 @@ template <> __device__ __forceinline__ void store4<bamd_bf>(bamd_bf * h, bamd_v4
     typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
     *(bf4 *) h = bf4{ (bamd_bf) v[0], (bamd_bf) v[1], (bamd_bf) v[2], (bamd_bf) v[3] };
 }
-template <typename T> __device__ __forceinline__ void zero_tail(T * h, int n, int ld) { for (int i = n + threadIdx.x; i < ld; i += blockDim.x) h[i] = to_act<T>(0.f); }
+// a row of operands being written (null: not wanted)
+template <typename T> struct RowOut {
+    T * p; int cb;
+    __device__ __forceinline__ explicit operator bool() const { return p != nullptr; }
+    __device__ __forceinline__ T * at(int i) const { return p + (i >> 5) * cb + (i & 31); }
+};
+template <typename T> __device__ __forceinline__ RowOut<T> row_out(void * h, int row, int ld, int cb) { return { h ? (T *) h + (size_t) row * (cb ? 32 : ld) : nullptr, cb ? cb : 32 }; }
+template <typename T> __device__ __forceinline__ void zero_tail(RowOut<T> h, int n, int ld) { for (int i = n + threadIdx.x; i < ld; i += blockDim.x) *h.at(i) = to_act<T>(0.f); }
 
 __device__ __forceinline__ float parts_sum(const float * p, int parts, size_t plane) { return parts > 1 ? p[0] + p[plane] : p[0]; }
 
@@ -162,7 +169,7 @@ template <int RC> __device__ __forceinline__ void row_moments(const RowRegs<RC> 
 }
 // residual sum with the layer norm of the sublayer's output, and the layer norm (gain gi, null: none) the next sublayer reads, of one row by the whole block
 template <typename T>
-__device__ __forceinline__ void layer_row(const bamd_residual_args & a, int row, const float * gi, T * h, bool write, float * red) {
+__device__ __forceinline__ void layer_row(const bamd_residual_args & a, int row, const float * gi, RowOut<T> h, bool write, float * red) {
     constexpr int RC = 2;
     const int E = a.E;
     const float * x = a.x + (size_t) row * E, * y = a.y ? a.y + (size_t) row * a.ldy : nullptr;
@@ -193,7 +200,7 @@ __device__ __forceinline__ void layer_row(const bamd_residual_args & a, int row,
         mean = 0.f;
         if (gi) { row_moments<RC>(xr, E, red, mean, var); r = 1.0f / sqrtf(var + a.eps); }
 #pragma unroll
-        for (int c = 0; c < RC; ++c) { const int i = RowRegs<RC>::at(c); if (i < E) store4<T>(h + i, gi ? (xr.v[c] - mean) * r * w[c] : xr.v[c]); }
+        for (int c = 0; c < RC; ++c) { const int i = RowRegs<RC>::at(c); if (i < E) store4<T>(h.at(i), gi ? (xr.v[c] - mean) * r * w[c] : xr.v[c]); }
         zero_tail(h, E, a.ldh);
         return;
     }
@@ -221,7 +228,7 @@ __device__ __forceinline__ void layer_row(const bamd_residual_args & a, int row,
     for (int i = threadIdx.x; i < E; i += blockDim.x) {
         const float xn = at(i);
         if (write) xo[i] = xn;
-        if (h) h[i] = to_act<T>(gi ? (xn - mx) * rx * gi[i] : xn);
+        if (h) *h.at(i) = to_act<T>(gi ? (xn - mx) * rx * gi[i] : xn);
     }
     if (h) zero_tail(h, E, a.ldh);
 }
@@ -231,18 +238,18 @@ __device__ __forceinline__ float clamped_glu(float gate, float up, float limit) 
 }
 // columns [from, to) of a row
 template <typename T>
-__device__ __forceinline__ void glu_row(const bamd_glu_args & a, int row, T * h, int from, int to) {
+__device__ __forceinline__ void glu_row(const bamd_glu_args & a, int row, RowOut<T> h, int from, int to) {
     const float * z = a.z + (size_t) row * a.ldz;
     for (int i = from + threadIdx.x * 4; i < to; i += blockDim.x * 4) {
         const bamd_v4 g = *(const bamd_v4 *) (z + (i >> 4) * 32 + (i & 15)), u = *(const bamd_v4 *) (z + (i >> 4) * 32 + 16 + (i & 15));
-        store4<T>(h + i, bamd_v4{ clamped_glu(g[0], u[0], a.limit), clamped_glu(g[1], u[1], a.limit), clamped_glu(g[2], u[2], a.limit), clamped_glu(g[3], u[3], a.limit) });
+        store4<T>(h.at(i), bamd_v4{ clamped_glu(g[0], u[0], a.limit), clamped_glu(g[1], u[1], a.limit), clamped_glu(g[2], u[2], a.limit), clamped_glu(g[3], u[3], a.limit) });
     }
 }
 
 // residual sum, norm of the sublayer's output and token shift of one row by the whole block.  h: LDS or global row (null: none).  write: this block also stores x' and the
 // state.  SINGLE: the step has one row
 template <typename T, bool SINGLE>
-__device__ __forceinline__ void residual_row(const bamd_batch_dev & b, const bamd_residual_args & a, int row, T * h, bool write, float * red) {
+__device__ __forceinline__ void residual_row(const bamd_batch_dev & b, const bamd_residual_args & a, int row, RowOut<T> h, bool write, float * red) {
     constexpr int RC = 2;
     const bool shifted = a.mu != nullptr;
     const int E = a.E;
@@ -276,7 +283,7 @@ __device__ __forceinline__ void residual_row(const bamd_batch_dev & b, const bam
             hn = xn;
             if (shifted) { bamd_v4 pv = pr.v[c]; if (yp) pv = pv + qr.v[c] * rp; hn = xn + (pv - xn) * mu.v[c]; }
             if (write) { *(bamd_v4 *) (a.xo + (size_t) row * E + i) = xn; if (so) *(bamd_v4 *) (so + i) = xn; }
-            if (h) store4<T>(h + i, hn);
+            if (h) store4<T>(h.at(i), hn);
         }
         if (h) zero_tail(h, E, a.ldh);
         return;
@@ -297,12 +304,12 @@ __device__ __forceinline__ void residual_row(const bamd_batch_dev & b, const bam
             hn = xn + (pv - xn) * a.mu[i];
         }
         if (write) { a.xo[(size_t) row * E + i] = xn; if (so) so[i] = xn; }
-        if (h) h[i] = to_act<T>(hn);
+        if (h) *h.at(i) = to_act<T>(hn);
     }
     if (h) zero_tail(h, E, a.ldh);
 }
 template <typename T>
-__device__ __forceinline__ void final_row(const bamd_residual_args & a, int row, const float * gf, T * h, float * red) {
+__device__ __forceinline__ void final_row(const bamd_residual_args & a, int row, const float * gf, RowOut<T> h, float * red) {
     constexpr int RC = 4;
     const int E = a.E;
     const float * x = a.x + (size_t) row * E, * y = a.y ? a.y + (size_t) row * a.ldy : nullptr;
@@ -322,7 +329,7 @@ __device__ __forceinline__ void final_row(const bamd_residual_args & a, int row,
         block_sum<1>(w, red);
         const float rf = gf[0] / sqrtf(w[0] / (float) E + a.eps);
 #pragma unroll
-        for (int c = 0; c < RC; ++c) { const int i = RowRegs<RC>::at(c); if (i < E) store4<T>(h + i, xr.v[c] * rf); }
+        for (int c = 0; c < RC; ++c) { const int i = RowRegs<RC>::at(c); if (i < E) store4<T>(h.at(i), xr.v[c] * rf); }
         zero_tail(h, E, a.ldh);
         return;
     }
@@ -335,11 +342,11 @@ __device__ __forceinline__ void final_row(const bamd_residual_args & a, int row,
     for (int i = threadIdx.x; i < E; i += blockDim.x) { const float xn = y ? x[i] + parts_sum(y + i, a.parts, a.plane) * r : x[i]; w[0] += xn * xn; }
     block_sum<1>(w, red);
     const float rf = gf[0] / sqrtf(w[0] / (float) E + a.eps);
-    for (int i = threadIdx.x; i < E; i += blockDim.x) h[i] = to_act<T>((y ? x[i] + parts_sum(y + i, a.parts, a.plane) * r : x[i]) * rf);
+    for (int i = threadIdx.x; i < E; i += blockDim.x) *h.at(i) = to_act<T>((y ? x[i] + parts_sum(y + i, a.parts, a.plane) * r : x[i]) * rf);
     zero_tail(h, E, a.ldh);
 }
 template <typename T>
-__device__ __forceinline__ void poly_row(const bamd_poly_args & a, int row, T * h, float * red) {
+__device__ __forceinline__ void poly_row(const bamd_poly_args & a, int row, RowOut<T> h, float * red) {
     constexpr int RC = 8;
     const float * z = a.z + (size_t) row * a.ldz;
     const bool fits = RowRegs<RC>::fits(a.F);
@@ -363,14 +370,14 @@ __device__ __forceinline__ void poly_row(const bamd_poly_args & a, int row, T * 
             bamd_v4 o;
 #pragma unroll
             for (int k = 0; k < 4; ++k) { const float t = zr.v[c][k], t2 = t * t; o[k] = c1 * t + c2 * t2 + c3 * (t2 * t) + c0; }
-            store4<T>(h + i, o);
+            store4<T>(h.at(i), o);
         }
-    } else for (int i = threadIdx.x; i < a.F; i += blockDim.x) { const float t = z[i], t2 = t * t; h[i] = to_act<T>(c1 * t + c2 * t2 + c3 * (t2 * t) + c0); }
+    } else for (int i = threadIdx.x; i < a.F; i += blockDim.x) { const float t = z[i], t2 = t * t; *h.at(i) = to_act<T>(c1 * t + c2 * t2 + c3 * (t2 * t) + c0); }
     zero_tail(h, a.F, a.ldh);
 }
 // inv: LDS, one float per part and 16 more
 template <typename T>
-__device__ __forceinline__ void group_norm_row(const bamd_group_norm_args & a, int row, T * h, float * inv) {
+__device__ __forceinline__ void group_norm_row(const bamd_group_norm_args & a, int row, RowOut<T> h, float * inv) {
     constexpr int RC = 4;
     const float * y = a.y + (size_t) row * a.ldy;
     const int per = a.n / a.groups, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6, wp = nw / a.groups;      // wp: waves per part
@@ -390,7 +397,7 @@ __device__ __forceinline__ void group_norm_row(const bamd_group_norm_args & a, i
         const float sum = row_sum16((lane & 15) < wp ? inv[g * wp + (lane & 15)] : 0.f);
         const float r = 1.0f / sqrtf(sum / (float) per + a.eps);
 #pragma unroll
-        for (int c = 0; c < RC; ++c) { const int i = at0 + c * by; if (i < per) store4<T>(h + base + i, v[c] * r * *(const bamd_v4 *) (a.w + base + i)); }
+        for (int c = 0; c < RC; ++c) { const int i = at0 + c * by; if (i < per) store4<T>(h.at(base + i), v[c] * r * *(const bamd_v4 *) (a.w + base + i)); }
         zero_tail(h, a.n, a.ldh);
         return;
     }
@@ -412,6 +419,6 @@ __device__ __forceinline__ void group_norm_row(const bamd_group_norm_args & a, i
         }
         __syncthreads();
     }
-    for (int i = threadIdx.x; i < a.n; i += blockDim.x) h[i] = to_act<T>(y[i] * inv[i / per] * a.w[i]);
+    for (int i = threadIdx.x; i < a.n; i += blockDim.x) *h.at(i) = to_act<T>(y[i] * inv[i / per] * a.w[i]);
     zero_tail(h, a.n, a.ldh);
 }

@@ -46,26 +46,26 @@ __global__ void __launch_bounds__(256) step_close_kernel(const float * __restric
 }
 template <typename T> __global__ void __launch_bounds__(1024) residual_rows_kernel(bamd_batch_dev b, bamd_residual_args a) {
     __shared__ float red[64];
-    residual_row<T, false>(b, a, blockIdx.x, a.h ? (T *) a.h + (size_t) blockIdx.x * a.ldh : nullptr, true, red);
+    residual_row<T, false>(b, a, blockIdx.x, row_out<T>(a.h, blockIdx.x, a.ldh, a.cb), true, red);
 }
 template <typename T> __global__ void __launch_bounds__(1024) final_rows_kernel(bamd_residual_args a, const int32_t * want, const float * gf) {
     __shared__ float red[64];
-    final_row<T>(a, want[blockIdx.x], gf, (T *) a.h + (size_t) blockIdx.x * a.ldh, red);
+    final_row<T>(a, want[blockIdx.x], gf, row_out<T>(a.h, blockIdx.x, a.ldh, a.cb), red);
 }
 template <typename T> __global__ void __launch_bounds__(1024) layer_rows_kernel(bamd_residual_args a, const int32_t * want, const float * gi) {
     __shared__ float red[64];
     const int row = want ? want[blockIdx.x] : blockIdx.x;
-    layer_row<T>(a, row, gi, a.h ? (T *) a.h + (size_t) blockIdx.x * a.ldh : nullptr, !want, red);
+    layer_row<T>(a, row, gi, row_out<T>(a.h, blockIdx.x, a.ldh, a.cb), !want, red);
 }
 // block (1024 columns, row)
-template <typename T> __global__ void __launch_bounds__(256) glu_rows_kernel(bamd_glu_args a) { glu_row<T>(a, blockIdx.y, (T *) a.h + (size_t) blockIdx.y * a.ldh, blockIdx.x * 1024, min(a.ldh, (int) blockIdx.x * 1024 + 1024)); }
+template <typename T> __global__ void __launch_bounds__(256) glu_rows_kernel(bamd_glu_args a) { glu_row<T>(a, blockIdx.y, row_out<T>(a.h, blockIdx.y, a.ldh, a.cb), blockIdx.x * 1024, min(a.ldh, (int) blockIdx.x * 1024 + 1024)); }
 template <typename T> __global__ void __launch_bounds__(1024) poly_rows_kernel(bamd_poly_args a) {
     __shared__ float red[64];
-    poly_row<T>(a, blockIdx.x, (T *) a.h + (size_t) blockIdx.x * a.ldh, red);
+    poly_row<T>(a, blockIdx.x, row_out<T>(a.h, blockIdx.x, a.ldh, a.cb), red);
 }
 template <typename T> __global__ void __launch_bounds__(1024) group_norm_rows_kernel(bamd_group_norm_args a) {
     __shared__ float inv[BAMD_MAX_NORM_GROUPS + 16];
-    group_norm_row<T>(a, blockIdx.x, (T *) a.h + (size_t) blockIdx.x * a.ldh, inv);
+    group_norm_row<T>(a, blockIdx.x, row_out<T>(a.h, blockIdx.x, a.ldh, a.cb), inv);
 }
 // block (part, row); keys must be zero
 __global__ void __launch_bounds__(256) argmax_rows_kernel(const float * __restrict__ logits, int V, unsigned long long * keys) {

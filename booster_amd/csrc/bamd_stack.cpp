@@ -218,21 +218,23 @@ struct Pass {                                      // one pass through the layer
     void begin(int kind, double bytes) { if (!tm) return; hipEvent_t e; hipEventCreate(&e); hipEventRecord(e, s); tm->ev.push_back(e); tm->kind.push_back(kind); tm->bytes.push_back(bytes); }
     void end() { if (!tm) return; hipEvent_t e; hipEventCreate(&e); hipEventRecord(e, s); tm->ev.push_back(e); }
 
+    int cb() const { return st.act == BAMD_ACT_BF16 && b.rows > 1 ? bamd_row_blocks(b.rows) : 0; }      // how the operand rows of this pass's products lie (bamd_dense.h): one row, and 32-bit rows, by rows
     bamd_residual_args residual(const float * mu, float * prev, const float * gi) {
         bamd_residual_args a; memset(&a, 0, sizeof a);
         a.norm = st.d.norm == STACK_NORM_SANDWICH ? BAMD_NORM_LAYER : BAMD_NORM_RMS; a.gi = gi;
-        a.x = x; a.y = pend; a.ldy = ldp; a.parts = pend_parts; a.plane = (size_t) b.rows * ldp; a.g = pend_g; a.eps = st.eps; a.mu = mu; a.prev = prev; a.xo = xo; a.h = c.h; a.E = st.E; a.ldh = up(st.E, 32);
+        a.x = x; a.y = pend; a.ldy = ldp; a.parts = pend_parts; a.plane = (size_t) b.rows * ldp; a.g = pend_g; a.eps = st.eps; a.mu = mu; a.prev = prev; a.xo = xo; a.h = c.h; a.E = st.E; a.ldh = up(st.E, 32); a.cb = cb();
         return a;
     }
     void advanced(const float * y, int ld, const float * g, int parts) { std::swap(x, xo); pend = y; ldp = ld; pend_g = g; pend_parts = parts; }
-    int split(const bamd_dense & w, const void * & x, int & ldx, int rows);      // 32-bit operand rows as bamd_launch_dense_gemm takes them; bfloat16 rows are left alone
+    int split(const bamd_dense & w, const void * & x, int & ldx, int & cb, int rows);      // 32-bit operand rows as bamd_launch_dense_gemm takes them; bfloat16 rows are left alone
     // a product whose operand rows exist; small row counts stream the weights once
     // parts: in, shares of K the result's buffer can hold; out, shares there are (the rows' residual sum adds them)
     int product(const bamd_dense & w, const void * in, int ldx, float * out, int ldo, int kind, int * parts = nullptr) {
         begin(kind, (double) w.bytes);
-        if (b.rows > BAMD_MV_ROWS && split(w, in, ldx, b.rows)) return 1;
-        const int rc = b.rows <= BAMD_MV_ROWS ? bamd_launch_dense_mv(st.act, w, BAMD_PRE_ROWS, b, nullptr, in, ldx, b.rows, out, ldo, s, parts)
-                                              : bamd_launch_dense_gemm(st.act, w, in, ldx, b.rows, out, ldo, BAMD_OUT_F32, s, 0.f, parts);
+        int blocks = cb();
+        if (b.rows > BAMD_MV_ROWS && split(w, in, ldx, blocks, b.rows)) return 1;
+        const int rc = b.rows <= BAMD_MV_ROWS ? bamd_launch_dense_mv(st.act, w, BAMD_PRE_ROWS, b, nullptr, in, ldx, blocks, b.rows, out, ldo, s, parts)
+                                              : bamd_launch_dense_gemm(st.act, w, in, ldx, blocks, b.rows, out, ldo, BAMD_OUT_F32, s, 0.f, parts);
         end();
         return rc ? fail("dense product: unsupported shape") : 0;
     }
@@ -240,7 +242,7 @@ struct Pass {                                      // one pass through the layer
     int product_pre(const bamd_dense & w, int pre, const bamd_pre_args & p, float * out, int ldo, int kind, int * parts = nullptr) {
         if (fused(w)) {
             begin(kind, (double) w.bytes);
-            const int rc = bamd_launch_dense_mv(st.act, w, pre, b, &p, nullptr, 0, 1, out, ldo, s, parts);
+            const int rc = bamd_launch_dense_mv(st.act, w, pre, b, &p, nullptr, 0, 0, 1, out, ldo, s, parts);
             end();
             return rc ? fail("dense product: unsupported shape") : 0;
         }
@@ -585,7 +587,7 @@ int Stack::context_init(bamd_context * bc) {
         }
         mx.partials(brows, po, pm);
     }
-    const size_t R = (size_t) c.rows_cap;
+    const size_t R = (size_t) up(c.rows_cap, 16);                  // (as bamd_row_blocks rounds)
     if (dev_alloc(bc->allocs, (void **) &c.xa, R * E * 4) || dev_alloc(bc->allocs, (void **) &c.xb, R * E * 4) || dev_alloc(bc->allocs, (void **) &c.y, R * std::max(c.ldy, 16) * 4) ||
         dev_alloc(bc->allocs, (void **) &c.y2, R * c.ldy2 * 4 * Y2_PLANES) || dev_alloc(bc->allocs, (void **) &c.y3, R * std::max(c.ldy3, 16) * 4) || dev_alloc(bc->allocs, &c.h, R * c.ldh * el())) return 1;
     if (qp && dev_alloc(bc->allocs, &c.qp, qp * el())) return 1;
@@ -660,11 +662,12 @@ int grow(Ctx & c, void ** p, size_t * have, size_t need, hipStream_t s) {
     HIPC(hipMalloc(p, need + 4096)); *have = need;
     return 0;
 }
-int Pass::split(const bamd_dense & w, const void * & x, int & ldx, int rows) {
+int Pass::split(const bamd_dense & w, const void * & x, int & ldx, int & cb, int rows) {
     if (st.act != BAMD_ACT_F32) return 0;
-    if (grow(c, &c.planes, &c.planes_n, (size_t) rows * std::max(c.ldh, w.K) * 6, s)) return 1;
-    bamd_launch_split_rows((const float *) x, ldx, rows, w.k_tiles, c.planes, s);
-    x = c.planes; ldx = 96 * w.k_tiles;
+    cb = 3 * bamd_row_blocks(rows);
+    if (grow(c, &c.planes, &c.planes_n, (size_t) cb * std::max(c.ldh, w.K) / 32 * 2, s)) return 1;
+    bamd_launch_split_rows((const float *) x, ldx, rows, w.k_tiles, c.planes, cb, s);
+    x = c.planes;
     return 0;
 }
 int Mamba2::run(Pass & p, MixState & st, Operand & o) {
@@ -678,7 +681,7 @@ int Mamba2::run(Pass & p, MixState & st, Operand & o) {
     p.end();
     if (rc) return fail("state-space kernel: unsupported shape");
     o.pre = BAMD_PRE_GROUP;
-    o.grp = { p.c.y3, inner, norm, ng, eps, p.c.h, inner, out.K };
+    o.grp = { p.c.y3, inner, norm, ng, eps, p.c.h, inner, out.K, p.cb() };
     return 0;
 }
 int splits_for(const Ctx & c, int rows, int hgroups) { return std::max(1, std::min({ 512 / std::max(1, rows * hgroups), c.max_pages, 64 })); }
@@ -687,7 +690,7 @@ int LatentAttention::run(Pass & p, MixState & st, Operand & o) {
     const int act = p.st.act;
     bamd_latent_args a; memset((void *) &a, 0, sizeof a);
     a.in = c.y; a.ld = ld_of(in); a.q_off = 0; a.c_off = H * D; a.g_off = g_off; a.c_norm = c_norm; a.eps = eps; a.scale = scale; a.sink = sink; a.gated = gated ? 1 : 0;
-    a.heads = H; a.D = D; a.R = R; a.Rp = Rp; a.cache = st.cache; a.ukT = ukT; a.uk = uk; a.uv = uv; a.out = c.h; a.ldo = out.K;
+    a.heads = H; a.D = D; a.R = R; a.Rp = Rp; a.cache = st.cache; a.ukT = ukT; a.uk = uk; a.uv = uv; a.out = c.h; a.ldo = out.K; a.cb = p.cb();
     o.x = c.h; o.ldx = out.K;
     p.begin(1, p.tm ? step_bytes(c.seqs[0].len + 1) + (double) uk.bytes + (double) uv.bytes : 0);
     int rc = 0;
@@ -697,9 +700,9 @@ int LatentAttention::run(Pass & p, MixState & st, Operand & o) {
         if (grow(c, &c.kc, &c.kc_n, kr * Rp * el, p.s) || grow(c, &c.kk, &c.kk_n, kr * H * D * el, p.s) || grow(c, &c.kv, &c.kv_n, kr * H * D * el, p.s)) return 1;
         bamd_launch_latent_store(act, p.b, a, p.s);
         bamd_launch_latent_gather(act, p.b, a, (const int32_t *) (c.dev + c.lay.kblk), p.k_rows, c.kc, p.s);
-        const void * lat = c.kc; int ldl = Rp;
-        if (p.split(uk, lat, ldl, p.k_rows)) return 1;
-        rc = bamd_launch_dense_gemm(act, uk, lat, ldl, p.k_rows, c.kk, H * D, BAMD_OUT_ACT, p.s) || bamd_launch_dense_gemm(act, uv, lat, ldl, p.k_rows, c.kv, p.k_rows, BAMD_OUT_ACT_T, p.s) ||
+        const void * lat = c.kc; int ldl = Rp, cbl = 0;
+        if (p.split(uk, lat, ldl, cbl, p.k_rows)) return 1;
+        rc = bamd_launch_dense_gemm(act, uk, lat, ldl, cbl, p.k_rows, c.kk, H * D, BAMD_OUT_ACT, p.s) || bamd_launch_dense_gemm(act, uv, lat, ldl, cbl, p.k_rows, c.kv, p.k_rows, BAMD_OUT_ACT_T, p.s) ||
              bamd_launch_latent_prompt(act, p.b, a, (const bamd_qtile *) (c.dev + c.lay.tile), p.n_tiles, c.kk, c.kv, p.k_rows, p.s);
     }
     p.end();
@@ -707,7 +710,7 @@ int LatentAttention::run(Pass & p, MixState & st, Operand & o) {
 }
 bamd_kv_args KvAttention::args(Pass & p, MixState & st, int ld, int ldo) const {
     bamd_kv_args k = a;
-    k.in = p.c.y; k.ld = ld; k.kc = st.cache; k.vc = st.cache2; k.out = p.c.h; k.ldo = ldo;
+    k.in = p.c.y; k.ld = ld; k.kc = st.cache; k.vc = st.cache2; k.out = p.c.h; k.ldo = ldo; k.cb = p.cb();
     return k;
 }
 int KvAttention::run(Pass & p, MixState & st, int ld, int ldo) {
@@ -724,7 +727,7 @@ int KvAttention::run(Pass & p, MixState & st, int ld, int ldo) {
 }
 bamd_gla_args GatedLinear::args(Pass & p, MixState & st, int ld, int ldo) const {
     bamd_gla_args g = a;
-    g.in = p.c.y; g.ld = ld; g.state = st.b; g.y = p.c.y3; g.ldy = a.heads * a.Pp; g.out = p.c.h; g.ldo = ldo;
+    g.in = p.c.y; g.ld = ld; g.state = st.b; g.y = p.c.y3; g.ldy = a.heads * a.Pp; g.out = p.c.h; g.ldo = ldo; g.cb = p.cb();
     return g;
 }
 int GatedLinear::run(Pass & p, MixState & st, int ld, int ldo) {
@@ -772,17 +775,17 @@ int Pass::layers() {
         if (few || (glu && b.rows > BAMD_MV_ROWS)) {                // the product writes the down-projection's operand
             begin(2, 0); bamd_launch_residual_rows(st.act, b, pa.res, s); end();
             begin(4, (double) ly.up.bytes);
-            const void * in = c.h; int ldx = pa.res.ldh;
-            if (!few && split(ly.up, in, ldx, b.rows)) return 1;
-            const int rc = few ? bamd_launch_dense_few_glu(ly.up, in, ldx, b.rows, c.y, ly.down.K, ly.limit, s)
-                               : bamd_launch_dense_gemm(st.act, ly.up, in, ldx, b.rows, c.y, ly.down.K, BAMD_OUT_GLU, s, ly.limit);
+            const void * in = c.h; int ldx = pa.res.ldh, blocks = cb();
+            if (!few && split(ly.up, in, ldx, blocks, b.rows)) return 1;
+            const int rc = few ? bamd_launch_dense_few_glu(ly.up, in, ldx, blocks, b.rows, c.y, ly.down.K, cb(), ly.limit, s)
+                               : bamd_launch_dense_gemm(st.act, ly.up, in, ldx, blocks, b.rows, c.y, ly.down.K, BAMD_OUT_GLU, s, ly.limit, nullptr, cb());
             end();
             if (rc) return fail("dense product: unsupported shape");
             if (product(ly.down, c.y, ly.down.K, c.y2, c.ldy2, 5, &parts)) return 1;
         } else {
             if (product_pre(ly.up, BAMD_PRE_RESIDUAL, pa, c.y, ld_of(ly.up), 4)) return 1;
-            if (glu) pa.glu = { c.y, ld_of(ly.up), ly.limit, c.h, ly.down.K };
-            else pa.poly = { c.y, ld_of(ly.up), ly.act, st.eps, c.h, ly.F, ly.down.K };
+            if (glu) pa.glu = { c.y, ld_of(ly.up), ly.limit, c.h, ly.down.K, cb() };
+            else pa.poly = { c.y, ld_of(ly.up), ly.act, st.eps, c.h, ly.F, ly.down.K, cb() };
             if (product_pre(ly.down, glu ? BAMD_PRE_GLU : BAMD_PRE_POLY, pa, c.y2, c.ldy2, 5, &parts)) return 1;
         }
         advanced(c.y2, c.ldy2, ly.norm2, parts);
@@ -795,13 +798,14 @@ int Pass::head(const int32_t * want, int n, float * logits) {
         bamd_pre_args pa; memset((void *) &pa, 0, sizeof pa);
         pa.res = a; pa.gf = st.norm_f; pa.want = want;
         begin(6, (double) st.head.bytes);
-        const int rc = bamd_launch_dense_mv(st.act, st.head, BAMD_PRE_FINAL, b, &pa, nullptr, 0, 1, logits, st.V, s);
+        const int rc = bamd_launch_dense_mv(st.act, st.head, BAMD_PRE_FINAL, b, &pa, nullptr, 0, 0, 1, logits, st.V, s);
         end();
         return rc ? fail("dense product: unsupported shape") : 0;
     }
+    a.cb = st.act == BAMD_ACT_BF16 ? bamd_row_blocks(n) : 0;
     bamd_launch_final_rows(st.act, a, want, n, st.norm_f, s);
     begin(6, (double) st.head.bytes);
-    const int rc = bamd_launch_dense_mv(st.act, st.head, BAMD_PRE_ROWS, b, nullptr, c.h, a.ldh, n, logits, st.V, s);
+    const int rc = bamd_launch_dense_mv(st.act, st.head, BAMD_PRE_ROWS, b, nullptr, c.h, a.ldh, a.cb, n, logits, st.V, s);
     end();
     return rc ? fail("dense product: unsupported shape") : 0;
 }
@@ -1145,13 +1149,15 @@ struct OpScratch {                                 // device copies of one call
     int alloc(void ** p, size_t bytes) { if (dev_alloc(keep, p, std::max<size_t>(bytes, 16))) return 1; HIPC(hipMemset(*p, 0, std::max<size_t>(bytes, 16))); return 0; }
     template <typename U> int up_(const U * h, size_t n, U ** d) { if (alloc((void **) d, n * sizeof(U))) return 1; if (n) HIPC(hipMemcpy(*d, h, n * sizeof(U), hipMemcpyHostToDevice)); return 0; }
     // f32 host rows [rows][n] -> activation rows [rows][ld]
-    int act_rows(const float * h, int rows, int n, int ld, void ** d) {
+    int act_rows(const float * h, int rows, int n, int ld, void ** d, bool blocks = false) {
         const bool f = l.act == BAMD_ACT_F32;
-        std::vector<unsigned char> b((size_t) rows * ld * (f ? 4 : 2), 0);
+        const int cb = bamd_row_blocks(rows);
+        std::vector<unsigned char> b((blocks ? (size_t) cb * (ld / 32) : (size_t) rows * ld) * (f ? 4 : 2), 0);
         for (int r = 0; r < rows; ++r) for (int i = 0; i < n; ++i) {
             const float v = h[(size_t) r * n + i];
-            if (f) memcpy(&b[((size_t) r * ld + i) * 4], &v, 4);
-            else { uint32_t u; memcpy(&u, &v, 4); u += 0x7fff + ((u >> 16) & 1); const uint16_t o = (uint16_t) (u >> 16); memcpy(&b[((size_t) r * ld + i) * 2], &o, 2); }
+            const size_t at = blocks ? (size_t) (i >> 5) * cb + r * 32 + (i & 31) : (size_t) r * ld + i;
+            if (f) memcpy(&b[at * 4], &v, 4);
+            else { uint32_t u; memcpy(&u, &v, 4); u += 0x7fff + ((u >> 16) & 1); const uint16_t o = (uint16_t) (u >> 16); memcpy(&b[at * 2], &o, 2); }
         }
         if (alloc(d, b.size())) return 1;
         HIPC(hipMemcpy(*d, b.data(), b.size(), hipMemcpyHostToDevice));
@@ -1168,12 +1174,13 @@ struct OpScratch {                                 // device copies of one call
         return 0;
     }
     // operand rows of a product of many rows
-    int split(const bamd_dense & d, const void * & x, int & ldx, int rows) {
+    int split(const bamd_dense & d, const void * & x, int & ldx, int & cb, int rows) {
         if (l.act != BAMD_ACT_F32) return 0;
         void * p;
-        if (alloc(&p, (size_t) rows * d.K * 6)) return 1;
-        bamd_launch_split_rows((const float *) x, ldx, rows, d.k_tiles, p, l.s);
-        x = p; ldx = 96 * d.k_tiles;
+        cb = 3 * bamd_row_blocks(rows);
+        if (alloc(&p, (size_t) cb * d.k_tiles * 2)) return 1;
+        bamd_launch_split_rows((const float *) x, ldx, rows, d.k_tiles, p, cb, l.s);
+        x = p;
         return 0;
     }
     int one_entry(int rows, int pos0, bamd_batch_dev & b) {
@@ -1200,19 +1207,21 @@ BAMD_OP bamd_op_dense_route(int act, int nrows, int k, int rows, int pre, int mo
 }
 BAMD_OP bamd_op_dense(int act, const uint16_t * w, int nrows, int k, const float * x, int rows, int impl, float * y) {
     OpScratch s; bamd_dense d; void * dx; float * dy = nullptr;
-    if (!w || !x || !y || nrows < 1 || k < 1 || rows < 1 || s.init(act)) return fail("bamd_op_dense: bad arguments");
+    const bool blocks = impl == 6 || impl == 7;                   // as impl 0 and 1, the operand rows by blocks
+    if (!w || !x || !y || nrows < 1 || k < 1 || rows < 1 || s.init(act) || (blocks && act != BAMD_ACT_BF16)) return fail("bamd_op_dense: bad arguments");
+    if (blocks) impl -= 6;
     const SafeTensor t = bf16_tensor(w, { nrows, k });
-    if (s.l.alloc(d, nrows, k) || s.l.pack(&t, Loader::steps(nrows, k), Loader::steps(k, 1), const_cast<uint16_t *>(d.w)) || s.act_rows(x, rows, k, d.K, &dx)) return 1;
+    if (s.l.alloc(d, nrows, k) || s.l.pack(&t, Loader::steps(nrows, k), Loader::steps(k, 1), const_cast<uint16_t *>(d.w)) || s.act_rows(x, rows, k, d.K, &dx, blocks)) return 1;
     const int ldo = impl == 3 ? up(rows, 64) : ld_of(d);
     int parts = impl == 4 || impl == 5 ? 2 : 1;
     if (s.alloc((void **) &dy, (size_t) (impl == 3 ? ld_of(d) : rows) * ldo * 4 * parts)) return 1;
     bamd_batch_dev b; memset((void *) &b, 0, sizeof b);
-    int rc, ldx = d.K; const void * px = dx;
-    if (impl != 1 && impl != 5 && s.split(d, px, ldx, rows)) return 1;
-    if (impl == 4) rc = bamd_launch_dense_gemm(act, d, px, ldx, rows, dy, ldo, BAMD_OUT_F32, s.l.s, 0.f, &parts);
-    else if (impl == 5) rc = bamd_launch_dense_mv(act, d, BAMD_PRE_ROWS, b, nullptr, dx, d.K, rows, dy, ldo, s.l.s, &parts);
-    else if (impl == 1) rc = bamd_launch_dense_mv(act, d, BAMD_PRE_ROWS, b, nullptr, dx, d.K, rows, dy, ldo, s.l.s);
-    else rc = bamd_launch_dense_gemm(act, d, px, ldx, rows, dy, ldo, impl == 0 ? BAMD_OUT_F32 : impl == 2 ? BAMD_OUT_ACT : BAMD_OUT_ACT_T, s.l.s);
+    int rc, ldx = d.K, cb = blocks ? bamd_row_blocks(rows) : 0; const void * px = dx;
+    if (impl != 1 && impl != 5 && s.split(d, px, ldx, cb, rows)) return 1;
+    if (impl == 4) rc = bamd_launch_dense_gemm(act, d, px, ldx, cb, rows, dy, ldo, BAMD_OUT_F32, s.l.s, 0.f, &parts);
+    else if (impl == 5) rc = bamd_launch_dense_mv(act, d, BAMD_PRE_ROWS, b, nullptr, dx, d.K, 0, rows, dy, ldo, s.l.s, &parts);
+    else if (impl == 1) rc = bamd_launch_dense_mv(act, d, BAMD_PRE_ROWS, b, nullptr, dx, d.K, cb, rows, dy, ldo, s.l.s);
+    else rc = bamd_launch_dense_gemm(act, d, px, ldx, cb, rows, dy, ldo, impl == 0 ? BAMD_OUT_F32 : impl == 2 ? BAMD_OUT_ACT : BAMD_OUT_ACT_T, s.l.s);
     if (rc) return fail("bamd_op_dense: unsupported shape");
     HIPC(hipGetLastError());
     if (impl >= 4) {                                              // the shares, added as their reader adds them
@@ -1236,9 +1245,9 @@ BAMD_OP bamd_op_dense_glu(int act, const uint16_t * gate, const uint16_t * upw, 
     if (s.l.alloc(d, 2 * ldo, k) || s.act_rows(x, rows, k, d.K, &dx) || s.alloc((void **) &dy, (size_t) rows * ldo * 4)) return 1;
     uint16_t * w = const_cast<uint16_t *>(d.w);
     if (s.l.pack(&tg, at, Loader::steps(k, 1), w, 2) || s.l.pack(&tu, at, Loader::steps(k, 1), w + (size_t) 16 * d.K, 2)) return 1;
-    const bool few = bamd_dense_few_glu(act, d, rows); const void * px = dx; int ldx = d.K;
-    if (!few && s.split(d, px, ldx, rows)) return 1;
-    if (few ? bamd_launch_dense_few_glu(d, dx, d.K, rows, dy, ldo, limit, s.l.s) : bamd_launch_dense_gemm(act, d, px, ldx, rows, dy, ldo, BAMD_OUT_GLU, s.l.s, limit)) return fail("bamd_op_dense_glu: unsupported shape");
+    const bool few = bamd_dense_few_glu(act, d, rows); const void * px = dx; int ldx = d.K, cb = 0;
+    if (!few && s.split(d, px, ldx, cb, rows)) return 1;
+    if (few ? bamd_launch_dense_few_glu(d, dx, d.K, 0, rows, dy, ldo, 0, limit, s.l.s) : bamd_launch_dense_gemm(act, d, px, ldx, cb, rows, dy, ldo, BAMD_OUT_GLU, s.l.s, limit)) return fail("bamd_op_dense_glu: unsupported shape");
     HIPC(hipGetLastError());
     return s.rows_back(dy, rows, F, ldo, y, act == BAMD_ACT_F32);
 }
@@ -1327,9 +1336,9 @@ BAMD_OP bamd_op_latent_attention(int act, const float * q, const float * c, cons
     else {
         bamd_launch_latent_store(act, b, a, s.l.s);
         bamd_launch_latent_gather(act, b, a, kblk, kr, kc, s.l.s);
-        const void * lat = kc; int ldl = Rp;
-        if (s.split(a.uk, lat, ldl, kr)) return 1;
-        rc = bamd_launch_dense_gemm(act, a.uk, lat, ldl, kr, kk, HD, BAMD_OUT_ACT, s.l.s) || bamd_launch_dense_gemm(act, a.uv, lat, ldl, kr, kv, kr, BAMD_OUT_ACT_T, s.l.s) ||
+        const void * lat = kc; int ldl = Rp, cbl = 0;
+        if (s.split(a.uk, lat, ldl, cbl, kr)) return 1;
+        rc = bamd_launch_dense_gemm(act, a.uk, lat, ldl, cbl, kr, kk, HD, BAMD_OUT_ACT, s.l.s) || bamd_launch_dense_gemm(act, a.uv, lat, ldl, cbl, kr, kv, kr, BAMD_OUT_ACT_T, s.l.s) ||
              bamd_launch_latent_prompt(act, b, a, tiles, (int) t.size(), kk, kv, kr, s.l.s);
     }
     if (rc) return fail("bamd_op_latent_attention: unsupported shape");

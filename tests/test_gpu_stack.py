@@ -110,6 +110,17 @@ def test_dense_split_values(bamd):
     assert not np.isnan(got[1]).any() and np.isnan(got[3:5]).all() and np.allclose(got[ok], want[ok], rtol=2e-6, atol=0)
 
 
+# operand rows by blocks of 32 columns, as the passes have them, against the same rows by rows: every tile of many rows and every group of few, ragged
+@pytest.mark.parametrize("n,rows,impl", [(8170, 2045, 0), (8170, 1000, 0), (4090, 1000, 0), (4090, 1100, 0), (8190, 131, 0), (2047, 131, 0), (2030, 1, 1), (2030, 16, 1), (4620, 3, 1), (11000, 15, 1), (4100, 17, 1), (4620, 32, 1), (4620, 33, 1),
+                                         (12400, 33, 1), (520, 64, 1)])
+@pytest.mark.parametrize("k", [1, 300, 2050])
+def test_dense_rows_by_blocks(bamd, n, rows, impl, k):
+    r = np.random.default_rng(n + k + rows)
+    w = so.f32_to_bf16(r.standard_normal((n, k), np.float32))
+    x = so.round_bf16(r.standard_normal((rows, k), np.float32))
+    assert np.array_equal(bamd.op_dense(w, x, "bfloat16", impl + 6).view(np.uint32), bamd.op_dense(w, x, "bfloat16", impl).view(np.uint32))
+
+
 # the same tiles where they write the clamped gated unit of their gate and up tiles in turn: widths that end inside a pair of tiles, on its edge and inside a group of four
 @pytest.mark.parametrize("dtype,F,rows,tile", [("bfloat16", 4085, 2045, 0), ("bfloat16", 4085, 1000, 1), ("bfloat16", 2032, 1000, 2), ("bfloat16", 2046, 1100, 3), ("bfloat16", 4090, 131, 4), ("bfloat16", 1001, 131, 5), ("bfloat16", 35, 70, 5),
                                                 ("float32", 1001, 131, 4)])
