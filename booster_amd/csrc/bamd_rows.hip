@@ -4,9 +4,8 @@
 #include "bamd_dense_device.h"
 #include <algorithm>
 
-// block (1024 columns, row)
-__device__ __forceinline__ void embed_piece(int row, int t, int p, const uint16_t * __restrict__ embd, const uint16_t * __restrict__ pos, float scale, int E, int V, float * __restrict__ x) {
-    const int i0 = blockIdx.x * 1024 + threadIdx.x * 4;
+// columns i0 .. i0 + 3
+__device__ __forceinline__ void embed_piece(int i0, int row, int t, int p, const uint16_t * __restrict__ embd, const uint16_t * __restrict__ pos, float scale, int E, int V, float * __restrict__ x) {
     t = t < 0 ? 0 : t >= V ? V - 1 : t;
     const uint16_t * er = embd + (size_t) t * E, * pr = pos ? pos + (size_t) p * E : nullptr;
     if (i0 + 3 < E && (E & 3) == 0) {
@@ -17,19 +16,24 @@ __device__ __forceinline__ void embed_piece(int row, int t, int p, const uint16_
 __global__ void __launch_bounds__(256) embed_rows_kernel(bamd_batch_dev b, const uint16_t * __restrict__ embd, const uint16_t * __restrict__ pos, float scale, int E, int V, float * __restrict__ x) {
     const int row = blockIdx.y;
     const bamd_entry e = b.ent[b.row_entry[row]];
-    embed_piece(row, b.tokens[row], e.pos0 + (row - e.row0), embd, pos, scale, E, V, x);
+    embed_piece(blockIdx.x * 1024 + threadIdx.x * 4, row, b.tokens[row], e.pos0 + (row - e.row0), embd, pos, scale, E, V, x);
 }
 __device__ __forceinline__ int32_t box_ld(const int32_t * p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
-// The step's descriptors and tokens come out of host memory here: a copy engine in front of the step, and one behind it, were 40 us of a token's 465 (width 2048).  Every block reads
-// its own token (two independent reads over the bus), the first one the descriptors of all rows
-__global__ void __launch_bounds__(256) step_open_kernel(const bamd_step_box * box, bamd_step_dev d, const uint16_t * __restrict__ embd, const uint16_t * __restrict__ pos, float scale, int E, int V, float * __restrict__ x) {
-    const int row = blockIdx.y, tid = threadIdx.x;
-    embed_piece(row, box_ld(&box->in.tok[row]), pos ? box_ld(&box->in.ent[row].pos0) : 0, embd, pos, scale, E, V, x);
-    if (blockIdx.x || row) return;
-    const int n = gridDim.y, words = n * (int) (sizeof(bamd_entry) / 4);
-    for (int i = tid; i < words; i += 256) ((int32_t *) d.ent)[i] = box_ld((const int32_t *) box->in.ent + i);
-    for (int i = tid; i < n; i += 256) { d.tokens[i] = box_ld(&box->in.tok[i]); d.row_entry[i] = i; d.want[i] = i; }
-    if (tid == 0) d.count_serial[1] = (uint32_t) box_ld((const int32_t *) &box->in.serial);
+// The step's descriptors and tokens come out of host memory here: a copy engine in front of the step, and one behind it, were 40 us of a token's 465 (width 2048).  A block per row, one lane of
+// which reads its token and position (two independent reads over the bus), the first block the descriptors of all rows.  Every wave of a block per 1024 columns reading them by itself, they were
+// 512 reads for sixteen rows of 4096: 27 us, now 7; one row of 2048 9.6, now 6.5
+__global__ void __launch_bounds__(1024) step_open_kernel(const bamd_step_box * box, bamd_step_dev d, const uint16_t * __restrict__ embd, const uint16_t * __restrict__ pos, float scale, int E, int V, float * __restrict__ x) {
+    __shared__ int32_t at[2];
+    const int row = blockIdx.x, tid = threadIdx.x;
+    if (tid == 0) { const int32_t t = box_ld(&box->in.tok[row]), p = pos ? box_ld(&box->in.ent[row].pos0) : 0; at[0] = t; at[1] = p; }
+    if (row == 0) {
+        const int n = gridDim.x, words = n * (int) (sizeof(bamd_entry) / 4), by = blockDim.x;
+        for (int i = tid; i < words; i += by) ((int32_t *) d.ent)[i] = box_ld((const int32_t *) box->in.ent + i);
+        for (int i = tid; i < n; i += by) { d.tokens[i] = box_ld(&box->in.tok[i]); d.row_entry[i] = i; d.want[i] = i; }
+        if (tid == by - 1) d.count_serial[1] = (uint32_t) box_ld((const int32_t *) &box->in.serial);
+    }
+    __syncthreads();
+    for (int i0 = tid * 4; i0 < E; i0 += blockDim.x * 4) embed_piece(i0, row, at[0], at[1], embd, pos, scale, E, V, x);
 }
 // n floats to host memory; the block that ends last tells the host.  Every thread's stores are out before its block counts
 __global__ void __launch_bounds__(256) step_close_kernel(const float * __restrict__ logits, size_t n, float * __restrict__ host, uint32_t * done, uint32_t * count_serial) {
@@ -110,7 +114,7 @@ void bamd_launch_embed_rows(const bamd_batch_dev & b, const uint16_t * embd, con
     hipLaunchKernelGGL(embed_rows_kernel, dim3((E + 1023) / 1024, b.rows), dim3(256), 0, s, b, embd, pos, scale, E, V, x);
 }
 void bamd_launch_step_open(const bamd_step_box * box, int rows, const bamd_step_dev & d, const uint16_t * embd, const uint16_t * pos, float scale, int E, int V, float * x, hipStream_t s) {
-    hipLaunchKernelGGL(step_open_kernel, dim3((E + 1023) / 1024, rows), dim3(256), 0, s, box, d, embd, pos, scale, E, V, x);
+    hipLaunchKernelGGL(step_open_kernel, dim3(rows), dim3(std::min(1024, std::max(128, ((E + 3) / 4 + 63) / 64 * 64))), 0, s, box, d, embd, pos, scale, E, V, x);
 }
 // a block per 4096 floats, up to 128: a row of 32 000 goes out at the bus's rate
 void bamd_launch_step_close(const float * logits, size_t n, float * host, bamd_step_box * box, uint32_t * count_serial, hipStream_t s) {
