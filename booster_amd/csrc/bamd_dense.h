@@ -84,11 +84,14 @@ int bamd_launch_dense_gemm(int act, const bamd_dense & w, const void * x, int ld
 void bamd_launch_split_rows(const float * x, int ldx, int rows, int k_tiles, void * planes, int cb, hipStream_t s);      // by blocks of three planes: [k_tiles][cb], row r at r * 96
 // few rows (<= BAMD_MV_ROWS): the weights stream once; out f32 [rows][ldo].  pre: how the operand comes about —
 enum { BAMD_PRE_ROWS = 0, BAMD_PRE_RESIDUAL = 1, BAMD_PRE_POLY = 2, BAMD_PRE_GROUP = 3, BAMD_PRE_FINAL = 4, BAMD_PRE_GLU = 5, BAMD_PRE_LAYER = 6 };     // (LAYER: RESIDUAL and FINAL with layer norms, chosen by res.norm); x given | one row, built in front of the product from the argument block
-struct bamd_pre_args { bamd_residual_args res; bamd_poly_args poly; bamd_group_norm_args grp; bamd_glu_args glu; const float * gf; const int32_t * want; };
+// results of a step's last product, on their way to the host as well (host null: not); `done` behind them (count_serial null: not)
+struct bamd_step_out { float * host = nullptr; uint32_t * done = nullptr, * count_serial = nullptr; };
+struct bamd_pre_args { bamd_residual_args res; bamd_poly_args poly; bamd_group_norm_args grp; bamd_glu_args glu; const float * gf; const int32_t * want; bamd_step_out close; };
 #define BAMD_MV_ROWS 64
 int bamd_launch_dense_mv(int act, const bamd_dense & w, int pre, const bamd_batch_dev & b, const bamd_pre_args * p, const void * x, int ldx, int cb, int rows, float * out, int ldo, hipStream_t s, int * parts = nullptr);
 // a few rows of the product with gate and up rows in turn, and the gated unit of its results, operands of the product behind, to h.  bamd_dense_few_glu: it is covered
 bool bamd_dense_few_glu(int act, const bamd_dense & w, int rows);
+bool bamd_dense_closes(int act, const bamd_dense & w, int rows, int ldo);      // bamd_launch_dense_mv covers `close` (the tiles of prompts, which it takes for more rows, do not)
 int bamd_launch_dense_few_glu(const bamd_dense & w, const void * x, int ldx, int cb, int rows, void * h, int ldh, int cbo, float limit, hipStream_t s);
 int bamd_dense_route(int act, const bamd_dense & w, int rows, int pre, int most, int & share);      // many rows (pre < 0): the tile; few rows: -1; share: shares of K, of at most `most`
 size_t bamd_dense_mv_lds(int act, int K);         // operand bytes of a built row: must stay within BAMD_MV_LDS

@@ -285,6 +285,22 @@ int bamd_launch_dense_gemm(int act, const bamd_dense & w, const void * x, int ld
 
 // ---- few rows ---------------------------------------------------------------------------------------------------------------------------------------
 // NT: groups of 16 rows; NW: waves; U: 32-column blocks per request batch of a wave
+// where a lane's four sums lie among a wave's 256: sixteen lanes that read four outputs each, of four rows, find them in different banks
+__device__ __forceinline__ int sum_slot(int l) { return ((l & 48) | ((l ^ (l >> 2 & 12)) & 15)) * 4; }
+// The last product of a decoding step brings its results to the host as it goes (stores that write through, 64 bytes of a row per instruction: in pieces of eight a row of 32 000 takes 1.3 ms)
+// and says when they are there: every wave waits for its own, the block that is done last tells the host.  The count itself orders nothing (acquire and release at every block's end are
+// write-backs of the L2: 10 us of a step).  A launch behind the product took 50 us for sixteen rows of 32 000, 6.5 for one; a step of eight layers, width 2048, one row 437 -> 430 us, six rows 649 ->
+// 632, width 4096, sixteen rows 1333 -> 1304, 32-bit, eight rows 808 -> 776
+__device__ __forceinline__ void to_host(const bamd_step_out & c, size_t at, float v) { if (c.host) __hip_atomic_store(c.host + at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
+__device__ __forceinline__ void close_step(const bamd_step_out & c) {
+    if (!c.count_serial) return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x || __hip_atomic_fetch_add(c.count_serial, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 < gridDim.x * gridDim.y) return;
+    c.count_serial[0] = 0;
+    __threadfence_system();
+    __hip_atomic_store(c.done, c.count_serial[1], __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 template <typename T, int NT, int NW, int PRE>
 __global__ void __launch_bounds__(64 * NW) dense_mv_kernel(bamd_dense w, bamd_batch_dev b, bamd_pre_args p, const T * x, int ldx, int rows, float * out, int ldo) {
     constexpr int U = sizeof(T) == 2 ? 8 : 4;
@@ -340,18 +356,20 @@ __global__ void __launch_bounds__(64 * NW) dense_mv_kernel(bamd_dense w, bamd_ba
         }
         __syncthreads();                                          // (the sums of the tile before are read)
 #pragma unroll
-        for (int n = 0; n < NT; ++n) *(bamd_v4 *) (red + ((wave * NT + n) * 64 + lane) * 4) = acc[n];
+        for (int n = 0; n < NT; ++n) *(bamd_v4 *) (red + (wave * NT + n) * 256 + sum_slot(lane)) = acc[n];
         __syncthreads();
-        for (int i = tid; i < NT * 256; i += 64 * NW) {
-            const int n = i >> 8, l = (i >> 2) & 63, k = i & 3, r = n * 16 + (l & 15), o = tile * 16 + (l >> 4) * 4 + k;
+        for (int i = tid; i < NT * 256; i += 64 * NW) {           // sixteen outputs of a row per sixteen lanes: four each, on a quarter of the lanes, are 1 to 2 % of a step slower
+            const int n = i >> 8, c = i & 15, rl = (i >> 4) & 15, r = n * 16 + rl, o = tile * 16 + c;
             if (r < rows && o < w.rows) {
                 float v = 0.f;
 #pragma unroll
-                for (int q = 0; q < NW; ++q) v += red[((q * NT + n) * 64 + l) * 4 + k];
+                for (int q = 0; q < NW; ++q) v += red[(q * NT + n) * 256 + sum_slot((c >> 2) * 16 + rl) + (c & 3)];
                 out[(size_t) r * ldo + o] = v;
+                to_host(p.close, (size_t) r * ldo + o, v);
             }
         }
     }
+    close_step(p.close);
 }
 // Up to 64 rows, bfloat16: NT groups of 16 rows, RT row tiles of the matrix.  Every block reads all the rows: bytes out of L2 (NT per RT of weights) and, read by the lanes of a
 // fragment as above, four times the lookups of the same bytes in one piece, were what the product took (16 rows x 14336 x 4096: 32 us, of which the weights are 19).  Here every
@@ -362,7 +380,7 @@ __global__ void __launch_bounds__(64 * NW) dense_mv_kernel(bamd_dense w, bamd_ba
 // rows, where the few there are cost little, level.
 // GLU (an even RT): gate and up tiles in turn; out is the gated unit's bfloat16 row.
 template <int NT, int RT, int NS, bool GLU>
-__global__ void __launch_bounds__(512) dense_few_kernel(bamd_dense w, const bamd_bf * x, int ldx, int cb, int rows, float * out, int ldo, int cbo, float limit) {
+__global__ void __launch_bounds__(512) dense_few_kernel(bamd_dense w, const bamd_bf * x, int ldx, int cb, int rows, float * out, int ldo, int cbo, float limit, bamd_step_out close) {
     constexpr int NW = 8, STEP = (NT + RT) * 1024, RING = NS * STEP;
     extern __shared__ __align__(16) unsigned char lds[];
     float * red = (float *) (lds + NW * RING);                    // [wave][RT][NT][64 lanes][4]
@@ -418,47 +436,57 @@ __global__ void __launch_bounds__(512) dense_few_kernel(bamd_dense w, const bamd
 #pragma unroll
         for (int t = 0; t < RT; ++t)
 #pragma unroll
-            for (int g = 0; g < NT; ++g) *(bamd_v4 *) (red + (((wave * RT + t) * NT + g) * 64 + lane) * 4) = acc[t][g];
+            for (int g = 0; g < NT; ++g) *(bamd_v4 *) (red + ((wave * RT + t) * NT + g) * 256 + sum_slot(lane)) = acc[t][g];
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        auto sum = [&](int c, int l, int k) {
-            float v = 0.f;
-#pragma unroll
-            for (int q = 0; q < NW; ++q) v += red[((q * RT * NT + c) * 64 + l) * 4 + k];
-            return v;
-        };
         if constexpr (GLU) {
-            for (int i = tid; i < RT / 2 * NT * 256; i += 64 * NW) {
-                const int c = i >> 8, t = c / NT * 2, l = (i >> 2) & 63, k = i & 3, r = (c % NT) * 16 + (l & 15), o = (grp * RT + t) * 8 + (l >> 4) * 4 + k;
-                if (r < rows && o < w.rows / 2) *row_out<bamd_bf>(out, r, ldo, cbo).at(o) = (bamd_bf) clamped_glu(sum(t * NT + c % NT, l, k), sum((t + 1) * NT + c % NT, l, k), limit);
+            auto sum = [&](int c, int rl, int o4) {               // of four columns, row rl of cell c
+                bamd_v4 v = { 0, 0, 0, 0 };
+#pragma unroll
+                for (int q = 0; q < NW; ++q) v = v + *(const bamd_v4 *) (red + (q * RT * NT + c) * 256 + sum_slot(o4 * 16 + rl));
+                return v;
+            };
+            for (int i = tid; i < RT / 2 * NT * 64; i += 64 * NW) {
+                const int c = i >> 6, t = c / NT * 2, rl = (i >> 2) & 15, r = (c % NT) * 16 + rl, o = (grp * RT + t) * 8 + (i & 3) * 4;      // (pairs of tiles: w.rows / 2 is a multiple of sixteen)
+                if (r >= rows || o >= w.rows / 2) continue;
+                const bamd_v4 g = sum(t * NT + c % NT, rl, i & 3), u = sum((t + 1) * NT + c % NT, rl, i & 3);
+                store4<bamd_bf>(row_out<bamd_bf>(out, r, ldo, cbo).at(o), bamd_v4{ clamped_glu(g[0], u[0], limit), clamped_glu(g[1], u[1], limit), clamped_glu(g[2], u[2], limit), clamped_glu(g[3], u[3], limit) });
             }
         } else for (int i = tid; i < RT * NT * 256; i += 64 * NW) {
-            const int c = i >> 8, l = (i >> 2) & 63, k = i & 3, r = (c % NT) * 16 + (l & 15), o = (grp * RT + c / NT) * 16 + (l >> 4) * 4 + k;
-            if (r < rows && o < w.rows) out[(size_t) r * ldo + o] = sum(c, l, k);
+            const int c = i >> 8, oc = i & 15, rl = (i >> 4) & 15, r = (c % NT) * 16 + rl, o = (grp * RT + c / NT) * 16 + oc;
+            if (r < rows && o < w.rows) {
+                float v = 0.f;
+#pragma unroll
+                for (int q = 0; q < NW; ++q) v += red[(q * RT * NT + c) * 256 + sum_slot((oc >> 2) * 16 + rl) + (oc & 3)];
+                out[(size_t) r * ldo + o] = v;
+                to_host(close, (size_t) r * ldo + o, v);
+            }
         }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");              // (no copy outlives the block)
+    close_step(close);
 }
 template <int NT, int RT, int NS, bool GLU = false>
-static void few_go(const bamd_dense & w, const void * x, int ldx, int cb, int rows, float * out, int ldo, hipStream_t s, int parts = 1, int cbo = 0, float limit = 0.f) {
+static void few_go(const bamd_dense & w, const void * x, int ldx, int cb, int rows, float * out, int ldo, hipStream_t s, int parts, const bamd_step_out & close, int cbo = 0, float limit = 0.f) {
     const int groups = (w.row_tiles + RT - 1) / RT;
-    hipLaunchKernelGGL((dense_few_kernel<NT, RT, NS, GLU>), dim3(groups < 256 ? groups : 256, parts), dim3(512), (size_t) 8 * (NS * (NT + RT) + NT * RT) * 1024, s, w, (const bamd_bf *) x, ldx, cb, rows, out, ldo, cbo, limit);
+    hipLaunchKernelGGL((dense_few_kernel<NT, RT, NS, GLU>), dim3(groups < 256 ? groups : 256, parts), dim3(512), (size_t) 8 * (NS * (NT + RT) + NT * RT) * 1024, s, w, (const bamd_bf *) x, ldx, cb, rows, out, ldo, cbo, limit, close);
 }
+bool bamd_dense_closes(int act, const bamd_dense & w, int rows, int ldo) { return act == BAMD_ACT_F32 || rows <= 32 || w.row_tiles <= 768 || (ldo & 3); }
 // RT by the rounds over the CUs; a round of 1, 2 or 3 tiles at K = 4096 takes 7.1, 12.7 and 16 us with up to 16 rows, one of 1 or 2 tiles 9.0 and 15.1 us with up to 32.
 // With more rows the 64 x 64 tiles of prompts are ahead once they fill the CUs (45 x 22672 x 4096: 49 against 74 us) and behind before (45 x 4096 x 14336: 136 against 48)
-static int few_pick(const bamd_dense & w, const void * x, int ldx, int cb, int rows, float * out, int ldo, hipStream_t s, int parts) {
+static int few_pick(const bamd_dense & w, const void * x, int ldx, int cb, int rows, float * out, int ldo, hipStream_t s, int parts, const bamd_step_out & close) {
     const long rounds[3] = { (w.row_tiles + 255) / 256, (w.row_tiles + 511) / 512, (w.row_tiles + 767) / 768 };
     if (rows > 32) {
-        if (w.row_tiles > 768 && (ldo & 3) == 0) return gemm_tiles<bamd_bf, BAMD_OUT_F32>(w, x, ldx, cb, rows, out, ldo, 0, 0.f, s);
-        few_go<4, 1, 3>(w, x, ldx, cb, rows, out, ldo, s, parts);
+        if (!bamd_dense_closes(BAMD_ACT_BF16, w, rows, ldo)) return gemm_tiles<bamd_bf, BAMD_OUT_F32>(w, x, ldx, cb, rows, out, ldo, 0, 0.f, s);
+        few_go<4, 1, 3>(w, x, ldx, cb, rows, out, ldo, s, parts, close);
     } else if (rows > 16) {
-        if (rounds[0] * 90 <= rounds[1] * 151) few_go<2, 1, 5>(w, x, ldx, cb, rows, out, ldo, s, parts); else few_go<2, 2, 4>(w, x, ldx, cb, rows, out, ldo, s);
+        if (rounds[0] * 90 <= rounds[1] * 151) few_go<2, 1, 5>(w, x, ldx, cb, rows, out, ldo, s, parts, close); else few_go<2, 2, 4>(w, x, ldx, cb, rows, out, ldo, s, 1, close);
     } else {
         const long t1 = rounds[0] * 71, t2 = rounds[1] * 127, t3 = rounds[2] * 160;
-        if (t1 <= t2 && t1 <= t3) few_go<1, 1, 5>(w, x, ldx, cb, rows, out, ldo, s, parts);
-        else if (t2 <= t3) few_go<1, 2, 5>(w, x, ldx, cb, rows, out, ldo, s);
-        else few_go<1, 3, 4>(w, x, ldx, cb, rows, out, ldo, s);
+        if (t1 <= t2 && t1 <= t3) few_go<1, 1, 5>(w, x, ldx, cb, rows, out, ldo, s, parts, close);
+        else if (t2 <= t3) few_go<1, 2, 5>(w, x, ldx, cb, rows, out, ldo, s, 1, close);
+        else few_go<1, 3, 4>(w, x, ldx, cb, rows, out, ldo, s, 1, close);
     }
     return 0;
 }
@@ -505,7 +533,7 @@ static int mv_pick(const bamd_dense & w, int pre, const bamd_batch_dev & b, cons
         return 0;
     }
     if (rows < 1 || rows > BAMD_MV_ROWS || (sizeof(T) == 4 && cb) || !rows_fit(w, ldx, cb, rows, 32)) return 1;
-    if constexpr (sizeof(T) == 2) return few_pick(w, x, cb ? 32 : ldx, cb ? cb : 32, rows, out, ldo, s, n);
+    if constexpr (sizeof(T) == 2) return few_pick(w, x, cb ? 32 : ldx, cb ? cb : 32, rows, out, ldo, s, n, p.close);
     else if (rows <= 16) mv_one<T, BAMD_PRE_ROWS>(w, b, p, x, ldx, rows, out, ldo, s, n);
     else if (rows <= 32) mv_go<T, 2, 8, BAMD_PRE_ROWS>(w, b, p, x, ldx, rows, out, ldo, s, n);
     else mv_go<T, 4, 8, BAMD_PRE_ROWS>(w, b, p, x, ldx, rows, out, ldo, s, n);
@@ -520,7 +548,7 @@ int bamd_launch_dense_few_glu(const bamd_dense & w, const void * x, int ldx, int
     if (!bamd_dense_few_glu(BAMD_ACT_BF16, w, rows) || !rows_fit(w, ldx, cb, rows, 32) || ldh < w.row_tiles * 8 || (ldh & 3)) return 1;
     if (cb) ldx = 32; else cb = 32;
     if (rows > 32) return gemm_tiles<bamd_bf, BAMD_OUT_GLU>(w, x, ldx, cb, rows, h, ldh, cbo, limit, s);
-    if (rows > 16) few_go<2, 2, 4, true>(w, x, ldx, cb, rows, (float *) h, ldh, s, 1, cbo, limit); else few_go<1, 2, 5, true>(w, x, ldx, cb, rows, (float *) h, ldh, s, 1, cbo, limit);
+    if (rows > 16) few_go<2, 2, 4, true>(w, x, ldx, cb, rows, (float *) h, ldh, s, 1, {}, cbo, limit); else few_go<1, 2, 5, true>(w, x, ldx, cb, rows, (float *) h, ldh, s, 1, {}, cbo, limit);
     return 0;
 }
 int bamd_launch_dense_mv(int act, const bamd_dense & w, int pre, const bamd_batch_dev & b, const bamd_pre_args * p, const void * x, int ldx, int cb, int rows, float * out, int ldo, hipStream_t s, int * parts) {

@@ -256,7 +256,7 @@ struct Pass {                                      // one pass through the layer
         return product(w, c.h, ldx, out, ldo, kind, parts);
     }
     int layers();
-    int head(const int32_t * want, int n, float * logits);
+    int head(const int32_t * want, int n, float * logits, const bamd_step_out & close = {});
 };
 
 // ---- mixers -------------------------------------------------------------------------------------------------------------------------------------------
@@ -792,10 +792,11 @@ int Pass::layers() {
     }
     return 0;
 }
-int Pass::head(const int32_t * want, int n, float * logits) {
+int Pass::head(const int32_t * want, int n, float * logits, const bamd_step_out & close) {
+    bamd_pre_args pa; memset((void *) &pa, 0, sizeof pa);
+    pa.close = close;
     bamd_residual_args a = residual(nullptr, nullptr, nullptr);
     if (fused(st.head) && n == 1) {
-        bamd_pre_args pa; memset((void *) &pa, 0, sizeof pa);
         pa.res = a; pa.gf = st.norm_f; pa.want = want;
         begin(6, (double) st.head.bytes);
         const int rc = bamd_launch_dense_mv(st.act, st.head, BAMD_PRE_FINAL, b, &pa, nullptr, 0, 0, 1, logits, st.V, s);
@@ -805,7 +806,7 @@ int Pass::head(const int32_t * want, int n, float * logits) {
     a.cb = st.act == BAMD_ACT_BF16 ? bamd_row_blocks(n) : 0;
     bamd_launch_final_rows(st.act, a, want, n, st.norm_f, s);
     begin(6, (double) st.head.bytes);
-    const int rc = bamd_launch_dense_mv(st.act, st.head, BAMD_PRE_ROWS, b, nullptr, c.h, a.ldh, a.cb, n, logits, st.V, s);
+    const int rc = bamd_launch_dense_mv(st.act, st.head, BAMD_PRE_ROWS, b, &pa, c.h, a.ldh, a.cb, n, logits, st.V, s);
     end();
     return rc ? fail("dense product: unsupported shape") : 0;
 }
@@ -918,9 +919,12 @@ int decode_rows(Pass & p, int kind) {
         if (greedy) bamd_launch_advance((bamd_entry *) p.b.ent, (int32_t *) p.b.tokens, c.keys, n, c.gen_out, c.gen_cap, c.step, 1, p.st.V, p.s);
         if (greedy) embed(p);
         else bamd_launch_step_open(c.box, n, { (bamd_entry *) p.b.ent, (int32_t *) p.b.row_entry, (int32_t *) p.b.tokens, (int32_t *) (c.dev + c.lay.want), c.count_serial }, p.st.embd, p.st.pos, p.st.scale, p.st.E, p.st.V, p.x, p.s);
-        if (p.layers() || p.head((const int32_t *) (c.dev + c.lay.want), n, c.c->logits)) return 1;
+        bamd_step_out out;
+        const bool closes = !greedy && bamd_dense_closes(p.st.act, p.st.head, n, p.st.V);
+        if (closes) out = { kind == STEP_HOST ? c.c->logits_host : nullptr, &c.box->done, c.count_serial };
+        if (p.layers() || p.head((const int32_t *) (c.dev + c.lay.want), n, c.c->logits, out)) return 1;
         if (greedy) bamd_launch_argmax_rows(c.c->logits, n, p.st.V, c.keys, false, p.s);
-        else bamd_launch_step_close(c.c->logits, kind == STEP_HOST ? (size_t) n * p.st.V : 0, c.c->logits_host, c.box, c.count_serial, p.s);
+        else if (!closes) bamd_launch_step_close(c.c->logits, kind == STEP_HOST ? (size_t) n * p.st.V : 0, c.c->logits_host, c.box, c.count_serial, p.s);
         return 0;
     };
     if (!g_graph) return enqueue();
