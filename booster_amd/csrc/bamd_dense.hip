@@ -7,6 +7,7 @@
 #include "bamd_dense_device.h"
 #include "bamd_mfma_common.h"
 #include <algorithm>
+#include <limits.h>
 #include <type_traits>
 
 // ---- packing at load: value (row, col) of the packed matrix = src[row_off[row] + col_off[col]], zero where either is negative; row tiles go to every step-th row tile of
@@ -96,36 +97,42 @@ void bamd_launch_split_rows(const float * x, int ldx, int rows, int k_tiles, voi
 // where the vector units round: kept in them from one column block to the next, a sum of 14336 positive products was off by 6.3e-6 (1.8e-6 with the f32 instructions), so it is 3.2e-7 (and
 // 4.1e-7 for 2.2e-6 with random signs).  500 x 8192 x 2048 118 -> 46 us, 500 x 12608 x 2048 178 -> 75, 500 x 2048 x 8192 122 -> 63.
 // 2048 x 28672 x 4096: 676 -> 409 us (1176 TFLOP/s); 2048 x 4096 x 14336: 284 -> 185 us (1303); 2048 x 2048 x 2048: 41 -> 22 us; 131 x 8192 x 2048: 23 -> 16 us.
+__device__ __forceinline__ const unsigned char * uniform_at(const unsigned char * p) {
+    return (const unsigned char *) ((uint64_t) (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (uint64_t) p) | (uint64_t) (uint32_t) __builtin_amdgcn_readfirstlane((int) ((uint64_t) p >> 32)) << 32);
+}
 template <typename T, int TM, int TN, int WM, int WN, int NS, int OUT>
 __global__ void __launch_bounds__(64 * WM * WN) dense_tile_kernel(bamd_dense w, const bamd_bf * x, int ldx, int cb, int rows, void * out, int ldo, int cbo, int n_mt, int n_nt, float limit) {
     const int kb = (int) ((long) w.k_tiles * blockIdx.y / gridDim.y), nk = (int) ((long) w.k_tiles * (blockIdx.y + 1) / gridDim.y) - kb;      // this block's share of K
-    constexpr int XT = TM / 16, WT = TN / 16, NW = WM * WN, MI = XT / WM, NI = WT / WN, XP = bamd_planes<T>, PX = XT * XP / NW, PW = WT / NW, PER = PX + PW, STAGE = (XT * XP + WT) * 1024;
-    static_assert(XT * XP % NW == 0 && (XP == 1 || MI % 2 == 0) && WT % NW == 0 && MI * WM == XT && NI * WN == WT && NS >= 4 && (NS & (NS - 1)) == 0, "");
+    constexpr int XT = TM / 16, WT = TN / 16, NW = WM * WN, MI = XT / WM, NI = WT / WN, XP = bamd_planes<T>, UNITS = XT * XP + WT, PER = (UNITS + NW - 1) / NW, STAGE = UNITS * 1024;
+    static_assert((XP == 1 || MI % 2 == 0) && MI * WM == XT && NI * WN == WT && NS >= 4 && (NS & (NS - 1)) == 0 && (OUT != BAMD_OUT_GLU || NI % 2 == 0), "");
     extern __shared__ __align__(16) unsigned char lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int total = n_mt * n_nt;
     int id = blockIdx.x;
     { const int per = (total + 7) / 8, xcd = id & 7, k = id >> 3; id = xcd * per + k; if (k >= per || id >= total) return; }
     const int mt = id % n_mt, nt = id / n_mt, m0 = mt * TM, n0t = nt * WT;
-    // this wave's share of a stage: PX operand blocks of activations, PW of weights
-    const unsigned char * xbase = (const unsigned char *) (x + (size_t) m0 * ldx + (size_t) kb * cb), * wbase = (const unsigned char *) (w.w + ((size_t) n0t * w.k_tiles + kb) * 512);
-    uint32_t xo[PX], wo[PW];
+    // this wave's share of a stage: PER of its kilobytes, of activations and then of weights (past the last one: that one again)
+    const unsigned char * src[PER]; uint32_t off[PER], step[PER], dst[PER];
 #pragma unroll
-    for (int i = 0; i < PX; ++i) {                                // 16 rows of four 16-byte pieces, of one plane
-        const int u = wave * PX + i;
-        int row = u / XP * 16 + (lane >> 2);
-        row = m0 + row < rows ? row : rows - 1 - m0;
-        xo[i] = (uint32_t) row * (uint32_t) ldx * 2u + (uint32_t) (u % XP) * 64u + (uint32_t) ((lane & 3) ^ ((lane >> 3) & 3)) * 16u;
+    for (int i = 0; i < PER; ++i) {
+        const int u = i * NW + wave < UNITS ? i * NW + wave : UNITS - 1;
+        dst[i] = (uint32_t) (size_t) (bamd_lds_vp) lds + (uint32_t) u * 1024u;
+        if (u < XT * XP) {                                        // 16 rows of four 16-byte pieces, of one plane
+            int row = u / XP * 16 + (lane >> 2);
+            row = m0 + row < rows ? row : rows - 1 - m0;
+            src[i] = uniform_at((const unsigned char *) (x + (size_t) m0 * ldx + (size_t) kb * cb)); step[i] = (uint32_t) cb * 2u;
+            off[i] = (uint32_t) row * (uint32_t) ldx * 2u + (uint32_t) (u % XP) * 64u + (uint32_t) ((lane & 3) ^ ((lane >> 3) & 3)) * 16u;
+        } else {
+            int tile = u - XT * XP;
+            tile = n0t + tile < w.row_tiles ? tile : w.row_tiles - 1 - n0t;
+            src[i] = uniform_at((const unsigned char *) (w.w + ((size_t) n0t * w.k_tiles + kb) * 512)); step[i] = 1024u;
+            off[i] = (uint32_t) tile * (uint32_t) w.k_tiles * 1024u + (uint32_t) lane * 16u;
+        }
     }
-#pragma unroll
-    for (int i = 0; i < PW; ++i) { int tile = wave * PW + i; tile = n0t + tile < w.row_tiles ? tile : w.row_tiles - 1 - n0t; wo[i] = (uint32_t) tile * (uint32_t) w.k_tiles * 1024u + (uint32_t) lane * 16u; }
-    const uint32_t xd = (uint32_t) (size_t) (bamd_lds_vp) lds + (uint32_t) wave * PX * 1024u, wd = (uint32_t) (size_t) (bamd_lds_vp) lds + (uint32_t) (XT * XP + wave * PW) * 1024u;
     // copy i of PER of stage k (behind the last column block: the last one again, into a stage nobody reads)
     auto copy = [&](int k, int i) {
         const int kk = k < nk ? k : nk - 1;
-        const uint32_t st = (uint32_t) (k & (NS - 1)) * STAGE;
-        if (i < PX) lds_dma16_s(xbase + (size_t) kk * cb * 2, xo[i], xd + st + i * 1024u);
-        else lds_dma16_s(wbase + (size_t) kk * 1024, wo[i - PX], wd + st + (i - PX) * 1024u);
+        lds_dma16_s(src[i] + (size_t) kk * step[i], off[i], dst[i] + (uint32_t) (k & (NS - 1)) * STAGE);
     };
     const int wm = wave % WM, wn = wave / WM;
     const int r = lane & 15, q = lane >> 4;                       // the lane's row of a block and its eight columns
@@ -206,8 +213,10 @@ static int tile_go(const bamd_dense & w, const void * x, int ldx, int cb, int ro
     hipLaunchKernelGGL((dense_tile_kernel<T, TM, TN, WM, WN, NS, OUT>), dim3(per * 8, parts), dim3(64 * WM * WN), (size_t) NS * (TM / 16 * bamd_planes<T> + TN / 16) * 1024, s, w, (const bamd_bf *) x, ldx, cb, rows, out, ldo, cbo, n_mt, n_nt, limit);
     return 0;
 }
-// The tile whose rounds over the 256 CUs end first.  Measured per block of 32 columns, all CUs busy (ns): 256 x 256 700, 128 x 256 450, 128 x 128 250, all three one block per CU,
-// so that a round started is a round paid; 64 x 128 190 and 64 x 64 160 share a CU with two to four others and never take less than 250 and 160.  Where even the small tiles leave
+// The tile whose rounds over the 256 CUs end first.  Measured per block of 32 columns (ns), half of the CUs busy and all: 256 x 256 650 to 785, 256 x 224 630 to 740, 256 x 192 565 to 655, 256 x 160
+// 512 to 572, 128 x 256 432 to 490, 128 x 128 250 to 280, all of them one block per CU, so that a round started is a round paid: the widths between are there for what 256 leaves over.  2048 x 16896 x
+// 4096 (66 tiles of 256 in two rows of rounds and a bit) 289 -> 258 us on 192, 2048 x 4736 x 4096 94 -> 74 on 160, 1485 x 14336 x 4096 192 -> 164 on 192, 2048 x 14336 x 4096 206 -> 198 on 224; over 23
+// sizes the choice is 0.3 % behind the best on average (7 % without them).  64 x 128 195 and 64 x 64 160 share a CU with two to four others and never take less than 250 and 160.  Where even the small tiles leave
 // CUs idle and the reader of the result can add planes, K is halved: two planes cost their bytes twice (at 4 TB/s) and blocks their
 // start and end once more (4 us).  131 x 2048 x 8192: 38 -> 22 us, 412 x 4096 x 8192: 85 -> 39; four shares were no faster (24 and 43 us).  Halves of 64 x 64 tiles that put a second block on
 // a CU take 300 where each half is longer than 2048 columns: 131 x 4096 x 14336 whole 70 us, in halves of such tiles 74, of 128 x 128 58 (8192 columns: 41, 43, 36); at K = 4096 they are
@@ -215,8 +224,8 @@ static int tile_go(const bamd_dense & w, const void * x, int ldx, int cb, int ro
 // 32-bit, three planes of activations: a block of 128 x 256 takes 800 ns where few CUs are busy and 1280 where all are (their copies out of L2), 128 x 128 430 and 690, 64 x 128 370 and 460, two of them
 // on a CU 700 to 800, 64 x 64 250 and 300, four on a CU 1000.  Halves: only what the reader of the second plane pays.  Of 94 choices (512 to 12608 outputs, K 512 to 14336, 70 to 2048 rows) the mean is
 // 0.5 % behind the best and the worst 10 %
-enum { TILE_256_256 = 0, TILE_128_256 = 1, TILE_128_128 = 2, TILE_64_128 = 3, TILE_64_64 = 4, TILE_64_64_DEEP = 5 };
-static int pick_tile(int act, const bamd_dense & w, int rows, int most, int & share) {
+enum { TILE_256_256 = 0, TILE_128_256 = 1, TILE_128_128 = 2, TILE_64_128 = 3, TILE_64_64 = 4, TILE_64_64_DEEP = 5, TILE_256_224 = 6, TILE_256_192 = 7, TILE_256_160 = 8 };
+static int pick_tile(int act, const bamd_dense & w, int rows, int most, int & share, int out) {
     share = 1;
     auto tiles = [&](int tm, int tn) { return (long) ((rows + tm - 1) / tm) * ((w.row_tiles * 16 + tn - 1) / tn); };
     long best = 0; int pick = 0;
@@ -233,12 +242,15 @@ static int pick_tile(int act, const bamd_dense & w, int rows, int most, int & sh
         return pick;
     }
     for (int p = 1; p <= most && p <= 2 && (p == 1 || w.k_tiles >= 32); ++p) {
-        auto rounds = [&](int tm, int tn, long cost) { return (tiles(tm, tn) * p + 255) / 256 * cost; };
+        auto rounds = [&](int tm, int tn, long lo, long by) { const long b = tiles(tm, tn) * p; return b / 256 * (lo + by) + (b % 256 ? lo + by * std::max(0l, b % 256 - 128) / 128 : 0); };
         const long pairs = p == 2 && w.k_tiles > 128 && tiles(64, 64) * 2 > 256 ? 300 : 160;
-        const long t[5] = { rounds(256, 256, 700), rounds(128, 256, 450), rounds(128, 128, 250), std::max(tiles(64, 128) * p * 190 / 256, 250l), std::max(tiles(64, 64) * p * 160 / 256, pairs) };
-        const int i = (int) (std::min_element(t, t + 5) - t);
+        const bool odd = p == 1 && out != BAMD_OUT_GLU;           // gate and up tiles lie in turn: a wave holds an even number
+        const long t[8] = { rounds(256, 256, 650, 135), rounds(128, 256, 432, 58), rounds(128, 128, 250, 30), std::max(tiles(64, 128) * p * 195 / 256, 250l), std::max(tiles(64, 64) * p * 160 / 256, pairs),
+                            odd ? rounds(256, 224, 630, 110) : LONG_MAX, p == 1 ? rounds(256, 192, 565, 90) : LONG_MAX, odd ? rounds(256, 160, 512, 60) : LONG_MAX };
+        static const int kind[8] = { TILE_256_256, TILE_128_256, TILE_128_128, TILE_64_128, TILE_64_64, TILE_256_224, TILE_256_192, TILE_256_160 };
+        const int i = (int) (std::min_element(t, t + 8) - t);
         const long ns = t[i] * ((w.k_tiles + p - 1) / p) + (p > 1 ? 4000 + (long) p * rows * w.row_tiles * 16 / 500 : 0);
-        if (p == 1 || ns < best) { best = ns; pick = i; share = p; }
+        if (p == 1 || ns < best) { best = ns; pick = kind[i]; share = p; }
     }
     // one tile per CU at most: twice the stages hide more of the memory's latency (131 x 2048 x 8192: 49 -> 38 us); with more, blocks hide each other's
     return pick == TILE_64_64 && tiles(64, 64) * share <= 256 ? TILE_64_64_DEEP : pick;
@@ -246,10 +258,13 @@ static int pick_tile(int act, const bamd_dense & w, int rows, int most, int & sh
 template <typename T, int OUT>
 static int gemm_tiles(const bamd_dense & w, const void * x, int ldx, int cb, int rows, void * out, int ldo, int cbo, float limit, hipStream_t s, int * parts = nullptr) {
     int share;
-    const int tile = pick_tile(sizeof(T) == 4 ? BAMD_ACT_F32 : BAMD_ACT_BF16, w, rows, OUT == BAMD_OUT_F32 && parts ? *parts : 1, share);
+    const int tile = pick_tile(sizeof(T) == 4 ? BAMD_ACT_F32 : BAMD_ACT_BF16, w, rows, OUT == BAMD_OUT_F32 && parts ? *parts : 1, share, OUT);
     if (parts) *parts = share;
     if constexpr (sizeof(T) == 2) switch (tile) {
         case TILE_256_256: return tile_go<T, 256, 256, 2, 4, 4, OUT>(w, x, ldx, cb, rows, out, ldo, cbo, limit, share, s);
+        case TILE_256_224: if constexpr (OUT != BAMD_OUT_GLU) return tile_go<T, 256, 224, 4, 2, 4, OUT>(w, x, ldx, cb, rows, out, ldo, cbo, limit, share, s); else return 1;
+        case TILE_256_192: return tile_go<T, 256, 192, 4, 2, 4, OUT>(w, x, ldx, cb, rows, out, ldo, cbo, limit, share, s);
+        case TILE_256_160: if constexpr (OUT != BAMD_OUT_GLU) return tile_go<T, 256, 160, 4, 2, 4, OUT>(w, x, ldx, cb, rows, out, ldo, cbo, limit, share, s); else return 1;
         case TILE_128_256: return tile_go<T, 128, 256, 2, 4, 4, OUT>(w, x, ldx, cb, rows, out, ldo, cbo, limit, share, s);
         case TILE_128_128: return tile_go<T, 128, 128, 2, 4, 8, OUT>(w, x, ldx, cb, rows, out, ldo, cbo, limit, share, s);
         case TILE_64_128: return tile_go<T, 64, 128, 2, 2, 4, OUT>(w, x, ldx, cb, rows, out, ldo, cbo, limit, share, s);
@@ -512,7 +527,7 @@ static int few_parts(int act, const bamd_dense & w, int pre, int most) {
     return act == BAMD_ACT_BF16 && pre != BAMD_PRE_ROWS && w.row_tiles > 64 && w.k_tiles <= 128 ? 1 : 2;
 }
 int bamd_dense_route(int act, const bamd_dense & w, int rows, int pre, int most, int & share) {
-    if (pre < 0) return pick_tile(act, w, rows, most, share);
+    if (pre < 0) return pick_tile(act, w, rows, most, share, BAMD_OUT_F32);
     share = few_parts(act, w, pre, most);
     return -1;
 }

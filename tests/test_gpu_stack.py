@@ -110,6 +110,26 @@ def test_dense_split_values(bamd):
     assert not np.isnan(got[1]).any() and np.isnan(got[3:5]).all() and np.allclose(got[ok], want[ok], rtol=2e-6, atol=0)
 
 
+# the widths between: 256 x 224, 256 x 192 and 256 x 160, ragged in every dimension; the gated unit on 256 x 192
+@pytest.mark.parametrize("n,rows,tile", [(14330, 1000, 6), (11000, 900, 7), (12600, 1485, 8)])
+@pytest.mark.parametrize("k", [1, 70, 300])
+def test_dense_tiles_between(bamd, n, rows, tile, k):
+    assert bamd.op_dense_route(n, k, rows, "bfloat16", most=1) == (tile, 1)
+    r = np.random.default_rng(n + k + rows)
+    w = so.f32_to_bf16(r.standard_normal((n, k), np.float32))
+    x = so.round_bf16(r.standard_normal((rows, k), np.float32))
+    wf = so.bf16_to_f32(w)
+    want, scale = x.astype(np.float64) @ wf.T.astype(np.float64), np.sqrt((x * x) @ (wf * wf).T) + 1e-30
+    for impl, tol in ((0, 8e-6), (6, 8e-6), (2, 2.0 ** -8), (3, 2.0 ** -8)):         # as test_dense_tiles
+        e = np.abs(bamd.op_dense(w, x, "bfloat16", impl) - want)
+        assert (e <= tol * (scale if impl in (0, 6) else np.abs(want) + 0.01 * scale)).all(), impl
+
+
+@pytest.mark.parametrize("k", [1, 300])
+def test_dense_gated_tile_between(bamd, k):
+    gated(bamd, "bfloat16", 5490, 900, k)
+
+
 # operand rows by blocks of 32 columns, as the passes have them, against the same rows by rows: every tile of many rows and every group of few, ragged
 @pytest.mark.parametrize("n,rows,impl", [(8170, 2045, 0), (8170, 1000, 0), (4090, 1000, 0), (4090, 1100, 0), (8190, 131, 0), (2047, 131, 0), (2030, 1, 1), (2030, 16, 1), (4620, 3, 1), (11000, 15, 1), (4100, 17, 1), (4620, 32, 1), (4620, 33, 1),
                                          (12400, 33, 1), (520, 64, 1)])
