@@ -225,7 +225,7 @@ static int tile_go(const bamd_dense & w, const void * x, int ldx, int cb, int ro
 // on a CU 700 to 800, 64 x 64 250 and 300, four on a CU 1000.  Halves: only what the reader of the second plane pays.  Of 94 choices (512 to 12608 outputs, K 512 to 14336, 70 to 2048 rows) the mean is
 // 0.5 % behind the best and the worst 10 %
 enum { TILE_256_256 = 0, TILE_128_256 = 1, TILE_128_128 = 2, TILE_64_128 = 3, TILE_64_64 = 4, TILE_64_64_DEEP = 5, TILE_256_224 = 6, TILE_256_192 = 7, TILE_256_160 = 8 };
-static int pick_tile(int act, const bamd_dense & w, int rows, int most, int & share, int out) {
+static int pick_tile(int act, const bamd_dense & w, int rows, int most, int & share, int out, long * cost = nullptr) {
     share = 1;
     auto tiles = [&](int tm, int tn) { return (long) ((rows + tm - 1) / tm) * ((w.row_tiles * 16 + tn - 1) / tn); };
     long best = 0; int pick = 0;
@@ -252,14 +252,36 @@ static int pick_tile(int act, const bamd_dense & w, int rows, int most, int & sh
         const long ns = t[i] * ((w.k_tiles + p - 1) / p) + (p > 1 ? 4000 + (long) p * rows * w.row_tiles * 16 / 500 : 0);
         if (p == 1 || ns < best) { best = ns; pick = kind[i]; share = p; }
     }
+    if (cost) *cost = best;
     // one tile per CU at most: twice the stages hide more of the memory's latency (131 x 2048 x 8192: 49 -> 38 us); with more, blocks hide each other's
     return pick == TILE_64_64 && tiles(64, 64) * share <= 256 ? TILE_64_64_DEEP : pick;
+}
+// Row tiles of the matrix that whole rounds of 256 x 256 take, the rest going to a product of its own, where that is ahead by more than 3 % (of one product; halves are not cut): 0 none.  The launch
+// between them is 4 us.  2048 x 28672 x 4096 with the gated unit (3.5 rounds) 377 -> 352 us; 2048 x 16896 x 4096 249 -> 239
+static int whole_rounds(const bamd_dense & w, int rows, int out) {
+    const int n_mt = (rows + 255) / 256;
+    if (256 % n_mt) return 0;
+    const int per = 256 / n_mt * 16, full = w.row_tiles / per * per;      // row tiles of a round
+    if (!full || full == w.row_tiles) return 0;
+    bamd_dense a = w, b = w; int share; long whole, ca, cb;
+    a.row_tiles = full; b.row_tiles = w.row_tiles - full;
+    pick_tile(BAMD_ACT_BF16, w, rows, 1, share, out, &whole);
+    const int ta = pick_tile(BAMD_ACT_BF16, a, rows, 1, share, out, &ca);
+    pick_tile(BAMD_ACT_BF16, b, rows, 1, share, out, &cb);
+    return ta == TILE_256_256 && (ca + cb + 4000) * 103 < whole * 100 ? full : 0;
 }
 template <typename T, int OUT>
 static int gemm_tiles(const bamd_dense & w, const void * x, int ldx, int cb, int rows, void * out, int ldo, int cbo, float limit, hipStream_t s, int * parts = nullptr) {
     int share;
     const int tile = pick_tile(sizeof(T) == 4 ? BAMD_ACT_F32 : BAMD_ACT_BF16, w, rows, OUT == BAMD_OUT_F32 && parts ? *parts : 1, share, OUT);
     if (parts) *parts = share;
+    if constexpr (sizeof(T) == 2 && (OUT == BAMD_OUT_F32 || OUT == BAMD_OUT_GLU)) if (const int n = share == 1 ? whole_rounds(w, rows, OUT) : 0) {
+        bamd_dense a = w, b = w;
+        a.row_tiles = n; a.rows = std::min(w.rows, n * 16);
+        b.row_tiles = w.row_tiles - n; b.rows = w.rows - n * 16; b.w = w.w + (size_t) n * w.k_tiles * 512;
+        void * rest = OUT == BAMD_OUT_F32 ? (void *) ((float *) out + n * 16) : (T *) out + (cbo ? (size_t) (n / 4) * cbo : (size_t) n * 8);
+        return gemm_tiles<T, OUT>(a, x, ldx, cb, rows, out, ldo, cbo, limit, s) || gemm_tiles<T, OUT>(b, x, ldx, cb, rows, rest, ldo, cbo, limit, s);
+    }
     if constexpr (sizeof(T) == 2) switch (tile) {
         case TILE_256_256: return tile_go<T, 256, 256, 2, 4, 4, OUT>(w, x, ldx, cb, rows, out, ldo, cbo, limit, share, s);
         case TILE_256_224: if constexpr (OUT != BAMD_OUT_GLU) return tile_go<T, 256, 224, 4, 2, 4, OUT>(w, x, ldx, cb, rows, out, ldo, cbo, limit, share, s); else return 1;

@@ -130,6 +130,27 @@ def test_dense_gated_tile_between(bamd, k):
     gated(bamd, "bfloat16", 5490, 900, k)
 
 
+# whole rounds of 256 x 256 and the rest apart: the same bits as the parts by themselves (a sum's order does not hang on the tile)
+@pytest.mark.parametrize("n,rows,k,cut", [(16890, 2045, 1500, 16384), (16890, 1030, 1500, 0)])
+def test_dense_whole_rounds(bamd, n, rows, k, cut):
+    r = np.random.default_rng(n + k + rows)
+    w = so.f32_to_bf16(r.standard_normal((n, k), np.float32))
+    x = so.round_bf16(r.standard_normal((rows, k), np.float32))
+    parts = [w[:cut], w[cut:]] if cut else [w[:8192], w[8192:]]
+    want = np.concatenate([bamd.op_dense(p, x, "bfloat16", 0) for p in parts], 1)
+    for impl in (0, 6):
+        assert np.array_equal(bamd.op_dense(w, x, "bfloat16", impl).view(np.uint32), want.view(np.uint32)), impl
+
+
+def test_dense_gated_whole_rounds(bamd):
+    F, rows, k, cut = 14330, 2045, 1500, 12288
+    r = np.random.default_rng(F + k + rows)
+    gate, up = (so.f32_to_bf16(r.standard_normal((F, k), np.float32) * np.float32(0.03)) for _ in range(2))
+    x = so.round_bf16(r.standard_normal((rows, k), np.float32))
+    want = np.concatenate([bamd.op_dense_glu(gate[i:j], up[i:j], x, 7.0, "bfloat16") for i, j in ((0, cut), (cut, F))], 1)
+    assert np.array_equal(bamd.op_dense_glu(gate, up, x, 7.0, "bfloat16").view(np.uint32), want.view(np.uint32))
+
+
 # operand rows by blocks of 32 columns, as the passes have them, against the same rows by rows: every tile of many rows and every group of few, ragged
 @pytest.mark.parametrize("n,rows,impl", [(8170, 2045, 0), (8170, 1000, 0), (4090, 1000, 0), (4090, 1100, 0), (8190, 131, 0), (2047, 131, 0), (2030, 1, 1), (2030, 16, 1), (4620, 3, 1), (11000, 15, 1), (4100, 17, 1), (4620, 32, 1), (4620, 33, 1),
                                          (12400, 33, 1), (520, 64, 1)])
