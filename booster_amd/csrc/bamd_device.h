@@ -250,7 +250,9 @@ __device__ __forceinline__ double seq_expsum8(const float * vals, int n) {
                                         barrier + sequential chain replay: what the reference's arithmetic costs per launch (profiles/r05_ceiling.txt) */
 #endif
 #define BAMD_ACT_RED_OFF(nb) ((((size_t) (nb) * (256 + 32 + 4)) + 15) & ~(size_t) 15)
-template <bool NORM>
+// NORM: 0 the vector as it is, 1 its RMSNorm with weights nw, 2 the vector times silu(nw), the feed-forward's gate (prompts)
+__device__ __forceinline__ float v_silu(float x);
+template <int NORM>
 struct ActPro {
     float4 v[BAMD_ACT_BATCH], w[BAMD_ACT_BATCH];
     int okmask;                                          // bit b: batch slot b holds a block of the vector (wave-uniform)
@@ -310,7 +312,8 @@ struct ActPro {
         uint32_t amaxb[NB];
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
-            if (NORM) {                                  // y = (x*scale)*w : ggml_vec_scale_f32 then ggml_mul (llama.cpp:7940-7950)
+            if (NORM == 2) { v[b].x = v_silu(w[b].x) * v[b].x; v[b].y = v_silu(w[b].y) * v[b].y; v[b].z = v_silu(w[b].z) * v[b].z; v[b].w = v_silu(w[b].w) * v[b].w; }
+            if (NORM == 1) {                             // y = (x*scale)*w : ggml_vec_scale_f32 then ggml_mul (llama.cpp:7940-7950)
                 v[b].x = (v[b].x * scale) * w[b].x; v[b].y = (v[b].y * scale) * w[b].y;
                 v[b].z = (v[b].z * scale) * w[b].z; v[b].w = (v[b].w * scale) * w[b].w;
             }
@@ -389,9 +392,9 @@ struct ActPro {
         const int step = nwaves * BAMD_ACT_BATCH;
         float scale = 1.0f;
 #if BAMD_CEILING & 1
-        if (NORM) { mid(); } else
+        if (NORM == 1) { mid(); } else
 #endif
-        if (NORM) {
+        if (NORM == 1) {
             // sum of squares in double (ggml.c:11874-11877), fixed tree order; f32_rounding_safe() below decides whether the order can matter
             double s = 0.0;
 #pragma unroll

@@ -90,7 +90,7 @@ void bamd_launch_k_shift(unsigned short * kc, int n_cells, int Hkv, int hd, cons
 size_t bamd_blob_bytes(int K);
 size_t bamd_blob16_bytes(int K);
 // blob: int8 activations for matmul_batch_kernel; blob16: f16 records for bamd_prefill2.hip; frag: f16 fragments for bamd_prefill_wide.hip (each may be null)
-void bamd_launch_quantize_batch(const float * x, const float * nw, float eps, int K, int T, void * blob, void * blob16, void * frag, hipStream_t s);
+void bamd_launch_quantize_batch(const float * x, const float * nw, float eps, int K, int T, void * blob, void * blob16, void * frag, hipStream_t s, const float * gate = nullptr);      // gate [T][K]: silu(gate) x is quantised (nw null)
 size_t bamd_tokfrag_bytes(int T, int K);       // token fragments of T rows of K activations (frag of bamd_launch_quantize_batch)
 // K-quant matrices on the matrix cores, exact (bamd_prefill2.hip): y[t][row] = W[row,:] . Q8_K(a_t); epi BAMD_EPI_STORE: out = y; BAMD_EPI_ADD: out = y + res;
 // BAMD_EPI_SILU_MUL: out = silu(res) * y (res = the gate projection, may alias out).  The A fragments are built once per 64-row x 64-token workgroup from the
@@ -106,7 +106,7 @@ int  bamd_prefill_few_tiles(int type, int nrows_pad, int K, int T);       // tok
 int  bamd_prefill_tokfrag(int type, int nrows_pad, int K, int T);
 size_t bamd_wide_lds(int type, int T, int waves);       // dynamic LDS of that launch
 bool bamd_wide_supported(void);                          // the current device takes it
-int  bamd_launch_matmul_wide(const void * w_stream, int type, int nrows, int nrows_pad, int K, const void * frag, int T, float * out, const float * res, int epi, int ldo, int waves, hipStream_t s);
+int  bamd_launch_matmul_wide(const void * w_stream, int type, int nrows, int nrows_pad, int K, const void * frag, int T, float * out, const float * res, int epi, int ldo, int waves, hipStream_t s, const void * w2 = nullptr, float * out2 = nullptr);      // w2, out2: a second matrix of the same shape (BAMD_EPI_STORE)
 int  bamd_launch_matmul_batch(const bamd_mm_args & a, int epi, int n_cu, hipStream_t s);      // 1 = shape not supported
 void bamd_launch_embed_batch(const int32_t * tokens, int T, const void * embd, int embd_type, int E, int V, float * x, hipStream_t s);
 int  bamd_launch_attention_batch(const bamd_attn_args & a, int gq, int T, hipStream_t s);     // 1 = shape not supported

@@ -19,7 +19,7 @@
 // (e, g) = the int8 of sub-blocks 2g and 2g+1, chunk e, as exact f16: one 16-byte B operand of v_mfma_f32_16x16x32_f16 per lane —
 // then, per pair l of sub-blocks, the four halves {S_h(2l), S_h(2l+1), S_l(2l), S_l(2l+1)} of the block sums split as S = 2 S_h + S_l
 // (the B operand of the Q4_K min-term MFMA), then the four i16 pairs (S_2l, S_2l+1) (Q5_K), then the block scale d_y (f32, byte 560); after the nb super-blocks, yd[nb] f32 again.
-template <bool NORM>
+template <int NORM>
 __global__ void __launch_bounds__(512) quantize_batch_kernel(const float * __restrict__ x, const float * __restrict__ nw, float eps, int K,
                                                              uint8_t * __restrict__ blob, uint8_t * __restrict__ blob16, uint8_t * __restrict__ frag) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -28,6 +28,7 @@ __global__ void __launch_bounds__(512) quantize_batch_kernel(const float * __res
     uint32_t * q8 = (uint32_t *) smem; int * S = (int *) (q8 + nb * 64); float * yd = (float *) (S + nb * 8);
     double * red = (double *) (smem + BAMD_ACT_RED_OFF(nb));
     const float * xt = x + (size_t) t * K;
+    if (NORM == 2) nw += (size_t) t * K;
     ActPro<NORM> ap; ap.issue(xt, nw, K, wave_id()); ap.template finish<false, typename ActPro<NORM>::NoMid, BAMD_ACT_BATCH, true>(xt, nw, eps, K, q8, S, yd, red);
     const size_t bb = BAMD_BLOB_BYTES(nb);
     if (blob) {
@@ -211,9 +212,10 @@ __global__ void __launch_bounds__(256) embed_batch_kernel(const int32_t * __rest
 // ---- batched prefill launchers ------------------------------------------------------------------------------------------
 size_t bamd_blob_bytes(int K) { return BAMD_BLOB_BYTES(K >> 8); }
 size_t bamd_blob16_bytes(int K) { return BAMD_BLOB16_BYTES(K >> 8); }
-void bamd_launch_quantize_batch(const float * x, const float * nw, float eps, int K, int T, void * blob, void * blob16, void * frag, hipStream_t s) {
-    if (nw) hipLaunchKernelGGL((quantize_batch_kernel<true>),  dim3(T), dim3(512), act_lds_bytes(K), s, x, nw, eps, K, (uint8_t *) blob, (uint8_t *) blob16, (uint8_t *) frag);
-    else    hipLaunchKernelGGL((quantize_batch_kernel<false>), dim3(T), dim3(512), act_lds_bytes(K), s, x, nw, eps, K, (uint8_t *) blob, (uint8_t *) blob16, (uint8_t *) frag);
+void bamd_launch_quantize_batch(const float * x, const float * nw, float eps, int K, int T, void * blob, void * blob16, void * frag, hipStream_t s, const float * gate) {
+    if (gate) hipLaunchKernelGGL((quantize_batch_kernel<2>),   dim3(T), dim3(512), act_lds_bytes(K), s, x, gate, eps, K, (uint8_t *) blob, (uint8_t *) blob16, (uint8_t *) frag);
+    else if (nw) hipLaunchKernelGGL((quantize_batch_kernel<1>),  dim3(T), dim3(512), act_lds_bytes(K), s, x, nw, eps, K, (uint8_t *) blob, (uint8_t *) blob16, (uint8_t *) frag);
+    else    hipLaunchKernelGGL((quantize_batch_kernel<0>), dim3(T), dim3(512), act_lds_bytes(K), s, x, nw, eps, K, (uint8_t *) blob, (uint8_t *) blob16, (uint8_t *) frag);
 }
 int bamd_launch_matmul_batch(const bamd_mm_args & a, int epi, int n_cu, hipStream_t s) {
     int nrg = 0;

@@ -30,6 +30,7 @@ struct bamd_wide_args {
     const uint8_t * w;               // wave-stream records of the matrix (bamd_formats.h)
     const uint8_t * frag;            // token fragments (quantize_batch_kernel)
     float * out; const float * res;  // [T][ldo]
+    const uint8_t * w2; float * out2;       // of the blocks z = 1
     int K, T, nrows, nrows_pad, ldo, epi;
 };
 
@@ -65,6 +66,7 @@ __global__ void __launch_bounds__(64 * WV) matmul_wide_kernel(bamd_wide_args a) 
     constexpr bool Q4 = TYPE == BAMD_Q4_K, Q5 = TYPE == BAMD_Q5_K, Q6 = TYPE == BAMD_Q6_K;
     constexpr int RECB = WideW<TYPE>::RECB, WS = WideW<TYPE>::SLOT, HDR = WideW<TYPE>::HDR, TS = wide_tslot(NTT), NW = WideW<TYPE>::COPIES;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    if (blockIdx.z) { a.w = a.w2; a.out = a.out2; }
     const int lane = threadIdx.x & 63, wave = wave_id(), m = lane & 15, g = lane >> 4;
     const int nb = a.K >> 8, ntile = (a.T + 15) >> 4, tile0 = blockIdx.x * NTT;
     const int nrt = (a.nrows_pad + 15) >> 4, rt0 = blockIdx.y * WV + wave, rt = rt0 < nrt ? rt0 : nrt - 1;
@@ -400,13 +402,13 @@ bool bamd_wide_supported(void) {
     auto takes = [](const void * k, size_t lds) { return hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds) == hipSuccess; };
     return takes((const void *) matmul_wide_kernel<BAMD_Q4_K, 4, 8>, wide_lds<BAMD_Q4_K>(4, 8)) && takes((const void *) matmul_wide_kernel<BAMD_Q6_K, 4, 8>, wide_lds<BAMD_Q6_K>(4, 8));
 }
-int bamd_launch_matmul_wide(const void * w_stream, int type, int nrows, int nrows_pad, int K, const void * frag, int T, float * out, const float * res, int epi, int ldo, int waves, hipStream_t s) {
+int bamd_launch_matmul_wide(const void * w_stream, int type, int nrows, int nrows_pad, int K, const void * frag, int T, float * out, const float * res, int epi, int ldo, int waves, hipStream_t s, const void * w2, float * out2) {
     if ((type != BAMD_Q4_K && type != BAMD_Q5_K && type != BAMD_Q6_K) || (nrows_pad & 7) || (K & 255) || K <= 0 || T <= 0 || nrows <= 0) return 1;
     if (epi != BAMD_EPI_STORE && epi != BAMD_EPI_ADD && epi != BAMD_EPI_SILU_MUL) return 1;
-    if ((epi != BAMD_EPI_STORE) != (res != nullptr) || (waves != 8 && (waves != 4 || type != BAMD_Q6_K))) return 1;
-    const bamd_wide_args a = { (const uint8_t *) w_stream, (const uint8_t *) frag, out, res, K, T, nrows, nrows_pad, ldo, epi };
+    if ((epi != BAMD_EPI_STORE) != (res != nullptr) || (w2 != nullptr) != (out2 != nullptr) || (w2 && epi != BAMD_EPI_STORE) || (waves != 8 && (waves != 4 || type != BAMD_Q6_K))) return 1;
+    const bamd_wide_args a = { (const uint8_t *) w_stream, (const uint8_t *) frag, out, res, (const uint8_t *) w2, out2, K, T, nrows, nrows_pad, ldo, epi };
     const int n = wide_tiles(T);
-    const dim3 grid(((T + 15) / 16 + n - 1) / n, ((nrows_pad + 15) / 16 + waves - 1) / waves);
+    const dim3 grid(((T + 15) / 16 + n - 1) / n, ((nrows_pad + 15) / 16 + waves - 1) / waves, w2 ? 2 : 1);
 #define XW_W(TYPE_, N_, WV_) hipLaunchKernelGGL((matmul_wide_kernel<TYPE_, N_, WV_>), grid, dim3(64 * WV_), wide_lds<TYPE_>(N_, WV_), s, a)
 #define XW_N(TYPE_, WV_) do { if (n == 2) XW_W(TYPE_, 2, WV_); else if (n == 3) XW_W(TYPE_, 3, WV_); else XW_W(TYPE_, 4, WV_); } while (0)
     if (type == BAMD_Q4_K) XW_N(BAMD_Q4_K, 8); else if (type == BAMD_Q5_K) XW_N(BAMD_Q5_K, 8); else if (waves == 8) XW_N(BAMD_Q6_K, 8); else XW_N(BAMD_Q6_K, 4);

@@ -376,6 +376,20 @@ def test_long_prompts_in_one_batch(tmp_path):
     long.close(); m.close()
 
 
+@pytest.mark.parametrize("quant", ["Q4_K", "Q5_K", "Q6_K"])
+def test_gate_and_up_of_a_prompt_in_one_launch(bamd, po, tmp_path, quant):
+    """every count of token tiles per block, edges of tiles and of the rule (256 | 257 tokens), a feed-forward of ten super-blocks"""
+    t = getattr(gguf, quant)
+    p = str(tmp_path / "m.gguf")
+    gguf.write_synthetic_llama(p, E=512, H=4, Hkv=2, L=2, F=1280, V=512, seed=5, type_fn=lambda n, il: t)
+    om = po.OracleModel(gguf.GGUFReader(p)); oc = po.OracleContext(om, 320, nthreads=8)
+    m = bamd.Model(p); ctx = bamd.Context(m, 320)
+    for T in (2, 16, 17, 33, 49, 65, 129, 256, 257):
+        toks = [(7919 * i + 13 * T) % 512 for i in range(T)]
+        assert np.array_equal(bits(ctx.decode(toks, 0)), bits(oc.decode(toks, 0))), T
+    oc.close(); ctx.close(); m.close()
+
+
 def test_a_long_prompt_takes_the_activation_layout_that_it_reads(tmp_path):
     """2048 tokens at once: rows of the layers' vectors, the score rows beyond 896 positions, and of the three layouts of quantised activations the one that every product of this size reads"""
     import booster_amd as bamd
