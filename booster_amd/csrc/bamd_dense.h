@@ -13,8 +13,9 @@
 
 enum { BAMD_ACT_BF16 = 0, BAMD_ACT_F32 = 1 };
 
-// Operand rows of products.  By rows: row r at r * ld.  By blocks (cb > 0: elements from one block of 32 columns to the next): column block, row, column — row r of block k at k * cb + r * 32.  A block's rows lie behind one another, so that a copy of sixteen of them is one kilobyte; by rows it is sixteen pieces of 64 bytes whose distance, the length of a row, is a
+// Operand rows of products: bfloat16, or (32-bit) three bfloat16 planes of 32 columns in turn, whose sum is the number: six bytes per value, and every distance below is three times as long.  By rows: row r at r * ld.  By blocks (cb > 0: elements from one block of 32 columns to the next): column block, row, column — row r of block k at k * cb + r * 32.  A block's rows lie behind one another, so that a copy of sixteen of them is one kilobyte; by rows it is sixteen pieces of 64 bytes whose distance, the length of a row, is a
 // multiple of 256 bytes in most models: all sixteen come out of one channel of an L2, while every CU asks for the same ones
+inline int bamd_row_planes(int act) { return act == BAMD_ACT_F32 ? 3 : 1; }
 inline int bamd_row_blocks(int rows) { const int by = rows > 16 ? 16 : 2; return 32 * ((rows + by - 1) / by * by); }      // groups of sixteen rows start on a kilobyte, fewer on a cache line
 struct bamd_dense { const uint16_t * w = nullptr; int rows = 0, K = 0; int row_tiles = 0, k_tiles = 0; size_t bytes = 0; };   // rows: outputs (stored: 16 row_tiles); K: stored, 32 k_tiles
 
@@ -79,9 +80,9 @@ void bamd_launch_advance(bamd_entry * ent, int32_t * tokens, unsigned long long 
 // f32 [rows][ldo] | activation type [rows][ldo] | activation type, transposed [n][ldo] | activation type, the clamped gated unit of alternating 16-row tiles [rows][ldo]
 enum { BAMD_OUT_F32 = 0, BAMD_OUT_ACT = 1, BAMD_OUT_ACT_T = 2, BAMD_OUT_GLU = 3 };
 // parts: in, how many shares of K the caller can take (f32 results only; share i goes to out + i * rows * ldo); out, how many there are: one or two
-// x: rows of operands; 32-bit: what bamd_launch_split_rows made of them.  cb: of x; GLU: cbo of the result
+// cb: of x; GLU: cbo of the result
 int bamd_launch_dense_gemm(int act, const bamd_dense & w, const void * x, int ldx, int cb, int rows, void * out, int ldo, int out_kind, hipStream_t s, float limit = 0.f, int * parts = nullptr, int cbo = 0);
-void bamd_launch_split_rows(const float * x, int ldx, int rows, int k_tiles, void * planes, int cb, hipStream_t s);      // by blocks of three planes: [k_tiles][cb], row r at r * 96
+void bamd_launch_split_rows(const float * x, int ldx, int rows, int k_tiles, void * planes, int cb, hipStream_t s);      // 32-bit rows as operand rows by blocks
 // few rows (<= BAMD_MV_ROWS): the weights stream once; out f32 [rows][ldo].  pre: how the operand comes about —
 enum { BAMD_PRE_ROWS = 0, BAMD_PRE_RESIDUAL = 1, BAMD_PRE_POLY = 2, BAMD_PRE_GROUP = 3, BAMD_PRE_FINAL = 4, BAMD_PRE_GLU = 5, BAMD_PRE_LAYER = 6 };     // (LAYER: RESIDUAL and FINAL with layer norms, chosen by res.norm); x given | one row, built in front of the product from the argument block
 // results of a step's last product, on their way to the host as well (host null: not); `done` behind them (count_serial null: not)
@@ -95,7 +96,7 @@ bool bamd_dense_closes(int act, const bamd_dense & w, int rows, int ldo);      /
 int bamd_launch_dense_few_glu(const bamd_dense & w, const void * x, int ldx, int cb, int rows, void * h, int ldh, int cbo, float limit, hipStream_t s);
 int bamd_dense_route(int act, const bamd_dense & w, int rows, int pre, int most, int & share);      // many rows (pre < 0): the tile; few rows: -1; share: shares of K, of at most `most`
 size_t bamd_dense_mv_lds(int act, int K);         // operand bytes of a built row: must stay within BAMD_MV_LDS
-#define BAMD_MV_LDS (96 * 1024)
+#define BAMD_MV_LDS(act) ((act) == BAMD_ACT_F32 ? 128 * 1024 : 96 * 1024)
 
 // ---- state-space recurrence ------------------------------------------------------------------------------------------------------------------------
 struct bamd_ssm_args {

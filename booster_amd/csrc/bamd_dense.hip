@@ -38,7 +38,7 @@ __device__ __forceinline__ void store_tile(const bamd_v4 (&a)[NI], int j, int mb
         bamd_v4 o;
 #pragma unroll
         for (int k = 0; k < 4; ++k) o[k] = clamped_glu(a[j][k], a[j | 1][k], limit);
-        store4<T>(row_out<T>(out, m, ldo, cbo).at(n), o);
+        store4<Operand<T>>(row_out<Operand<T>>(out, m, ldo, cbo).at(n), o);
     } else {
         const int n = nb + (lane >> 4) * 4, m = mb + (lane & 15);
         if (m >= rows) return;
@@ -53,37 +53,15 @@ __device__ __forceinline__ void store_tile(const bamd_v4 (&a)[NI], int j, int mb
         }
     }
 }
-// A 32-bit activation is the sum of three bfloat16 numbers, eight bits of its significand each (cut off, not rounded: parts of one sign, and what is left is exact), and products of bfloat16
-// numbers are exact in 32 bits: three bfloat16 matrix instructions do what eight of 16x16x4_f32 did, with three roundings of a sum per 32 columns for thirty-two.
-template <typename T> constexpr int bamd_planes = sizeof(T) == 4 ? 3 : 1;
-// rows [rows][ldx] of 32 k_tiles floats -> blocks of 32 columns: [k_tiles][cb], in them [rows][3 planes][32].  A value that is not finite is its first plane alone
-__global__ void __launch_bounds__(256) split_rows_kernel(const float * __restrict__ x, int ldx, int k_tiles, uint16_t * __restrict__ planes, int cb) {
-    const int i = (blockIdx.x * 256 + threadIdx.x) * 8;
-    if (i >= k_tiles * 32) return;
-    const float * p = x + (size_t) blockIdx.y * ldx + i;
-    const bamd_v4 a = *(const bamd_v4 *) p, b = *(const bamd_v4 *) (p + 4);
-    uint32_t h[3][4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        uint32_t part[2][3];
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            const float v = c < 2 ? a[c * 2 + e] : b[c * 2 - 4 + e];
-            const uint32_t u = __float_as_uint(v);
-            const bool finite = (u & 0x7f800000u) != 0x7f800000u;
-            const float m = finite ? v - __uint_as_float(u & 0xffff0000u) : 0.f, l = m - __uint_as_float(__float_as_uint(m) & 0xffff0000u);
-            part[e][0] = finite || !(u & 0x007fffffu) ? u : u | 0x00400000u;
-            part[e][1] = __float_as_uint(m); part[e][2] = __float_as_uint(l);
-        }
-#pragma unroll
-        for (int n = 0; n < 3; ++n) h[n][c] = (part[0][n] >> 16) | (part[1][n] & 0xffff0000u);
-    }
-    uint16_t * d = planes + (size_t) (i >> 5) * cb + blockIdx.y * 96 + (i & 31);
-#pragma unroll
-    for (int n = 0; n < 3; ++n) *(bamd_u4 *) (d + n * 32) = bamd_u4{ h[n][0], h[n][1], h[n][2], h[n][3] };
+// 32-bit: weights are bfloat16, activations three planes of it (bamd_dense_device.h), and products of bfloat16 numbers are exact in 32 bits: three bfloat16 matrix instructions do what eight of
+// 16x16x4_f32 did, with three roundings of a sum per 32 columns for thirty-two.
+// rows [rows][ldx] of 32 k_tiles floats -> operand rows by blocks (rows that no kernel writes as operands: cached latents)
+__global__ void __launch_bounds__(256) split_rows_kernel(const float * __restrict__ x, int ldx, int k_tiles, void * planes, int cb) {
+    const int i = (blockIdx.x * 256 + threadIdx.x) * 4;
+    if (i < k_tiles * 32) store4<bamd_s3>(row_out<bamd_s3>(planes, blockIdx.y, 0, cb).at(i), *(const bamd_v4 *) (x + (size_t) blockIdx.y * ldx + i));
 }
 void bamd_launch_split_rows(const float * x, int ldx, int rows, int k_tiles, void * planes, int cb, hipStream_t s) {
-    hipLaunchKernelGGL(split_rows_kernel, dim3((k_tiles * 4 + 255) / 256, rows), dim3(256), 0, s, x, ldx, k_tiles, (uint16_t *) planes, cb);
+    hipLaunchKernelGGL(split_rows_kernel, dim3((k_tiles * 8 + 255) / 256, rows), dim3(256), 0, s, x, ldx, k_tiles, planes, cb);
 }
 // TM activation rows x TN matrix rows per block of WM x WN waves.  Both operands travel global -> LDS by DMA (a kilobyte per instruction: 16 rows x 32 columns), NS stages
 // of 32 columns deep: while the matrix instructions of column block k run from registers, the fragments of k + 1 are read from LDS and the copies of the NS - 2 blocks
@@ -314,7 +292,7 @@ static int gemm_out(const bamd_dense & w, const void * x, int ldx, int cb, int r
     return 1;
 }
 int bamd_launch_dense_gemm(int act, const bamd_dense & w, const void * x, int ldx, int cb, int rows, void * out, int ldo, int kind, hipStream_t s, float limit, int * parts, int cbo) {
-    const int in_block = act == BAMD_ACT_F32 ? 96 : 32;
+    const int in_block = 32 * bamd_row_planes(act);
     if (rows < 1 || w.row_tiles < 1 || w.k_tiles < 1 || (ldo & 3) || !rows_fit(w, ldx, cb, rows, in_block)) return 1;
     if (cb) ldx = in_block; else cb = in_block;
     return act == BAMD_ACT_F32 ? gemm_out<float>(w, x, ldx, cb, rows, out, ldo, cbo, kind, limit, s, parts) : gemm_out<bamd_bf>(w, x, ldx, cb, rows, out, ldo, cbo, kind, limit, s, parts);
@@ -339,8 +317,9 @@ __device__ __forceinline__ void close_step(const bamd_step_out & c) {
     __hip_atomic_store(c.done, c.count_serial[1], __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 template <typename T, int NT, int NW, int PRE>
-__global__ void __launch_bounds__(64 * NW) dense_mv_kernel(bamd_dense w, bamd_batch_dev b, bamd_pre_args p, const T * x, int ldx, int rows, float * out, int ldo) {
-    constexpr int U = sizeof(T) == 2 ? 8 : 4;
+__global__ void __launch_bounds__(64 * NW) dense_mv_kernel(bamd_dense w, bamd_batch_dev b, bamd_pre_args p, const bamd_bf * x, int ldx, int cb, int rows, float * out, int ldo) {
+    constexpr int U = 8, P = bamd_planes<T>;
+    typedef Operand<T> O;
     extern __shared__ __align__(16) unsigned char lds[];
     __shared__ float red[NW * NT * 256];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -356,13 +335,13 @@ __global__ void __launch_bounds__(64 * NW) dense_mv_kernel(bamd_dense w, bamd_ba
     int tile = blockIdx.x;
     request(tile, 0, cur);                                        // on their way while the operand row is built
     if constexpr (PRE != BAMD_PRE_ROWS) {
-        const RowOut<T> h = { (T *) lds, 32 };
-        if constexpr (PRE == BAMD_PRE_RESIDUAL) residual_row<T, true>(b, p.res, 0, h, blockIdx.x == 0, red);
-        if constexpr (PRE == BAMD_PRE_POLY) poly_row<T>(p.poly, 0, h, red);
-        if constexpr (PRE == BAMD_PRE_GROUP) group_norm_row<T>(p.grp, 0, h, red);
-        if constexpr (PRE == BAMD_PRE_GLU) glu_row<T>(p.glu, 0, h, 0, p.glu.ldh);
-        if constexpr (PRE == BAMD_PRE_LAYER) layer_row<T>(p.res, p.want ? p.want[0] : 0, p.want ? p.gf : p.res.gi, h, !p.want && blockIdx.x == 0, red);
-        if constexpr (PRE == BAMD_PRE_FINAL) final_row<T>(p.res, p.want[0], p.gf, h, red);
+        const RowOut<O> h = { (O *) lds, 32 * P };
+        if constexpr (PRE == BAMD_PRE_RESIDUAL) residual_row<O, true>(b, p.res, 0, h, blockIdx.x == 0, red);
+        if constexpr (PRE == BAMD_PRE_POLY) poly_row<O>(p.poly, 0, h, red);
+        if constexpr (PRE == BAMD_PRE_GROUP) group_norm_row<O>(p.grp, 0, h, red);
+        if constexpr (PRE == BAMD_PRE_GLU) glu_row<O>(p.glu, 0, h, 0, p.glu.ldh);
+        if constexpr (PRE == BAMD_PRE_LAYER) layer_row<O>(p.res, p.want ? p.want[0] : 0, p.want ? p.gf : p.res.gi, h, !p.want && blockIdx.x == 0, red);
+        if constexpr (PRE == BAMD_PRE_FINAL) final_row<O>(p.res, p.want[0], p.gf, h, red);
         __syncthreads();
     }
     const int col = lane & 15, kq = (lane >> 4) * 8;
@@ -378,13 +357,19 @@ __global__ void __launch_bounds__(64 * NW) dense_mv_kernel(bamd_dense w, bamd_ba
             for (int u = 0; u < U; ++u) {
                 const int kt = k0 + c * U + u;
                 if (kt < k1) {
-                    Frag<T> wf; wf.weight(cur[u]);
+                    const bamd_bf8 wf = __builtin_bit_cast(bamd_bf8, cur[u]);
 #pragma unroll
                     for (int n = 0; n < NT; ++n) {
-                        Frag<T> xf;
-                        if constexpr (PRE != BAMD_PRE_ROWS) xf.load((const T *) lds + kt * 32 + kq);
-                        else { int r = n * 16 + col; r = r < rows ? r : rows - 1; xf.load(x + (size_t) r * ldx + kt * 32 + kq); }
-                        acc[n] = mma(wf, xf, acc[n]);
+                        const bamd_bf * at;
+                        if constexpr (PRE != BAMD_PRE_ROWS) at = (const bamd_bf *) lds + kt * (32 * P) + kq;
+                        else { int r = n * 16 + col; r = r < rows ? r : rows - 1; at = x + (size_t) r * ldx + (size_t) kt * cb + kq; }
+                        if constexpr (P == 1) acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, *(const bamd_bf8 *) at, acc[n], 0, 0, 0);
+                        else {                                    // (from zero, and added by the vector units: dense_tile_kernel)
+                            bamd_v4 s = { 0, 0, 0, 0 };
+#pragma unroll
+                            for (int i = P - 1; i >= 0; --i) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, *(const bamd_bf8 *) (at + i * 32), s, 0, 0, 0);
+                            acc[n] = acc[n] + s;
+                        }
                     }
                 }
             }
@@ -527,18 +512,18 @@ static int few_pick(const bamd_dense & w, const void * x, int ldx, int cb, int r
     }
     return 0;
 }
-size_t bamd_dense_mv_lds(int act, int K) { return (size_t) (K + 31) / 32 * 32 * (act == BAMD_ACT_F32 ? 4 : 2); }
+size_t bamd_dense_mv_lds(int act, int K) { return (size_t) (K + 31) / 32 * 64 * bamd_row_planes(act); }
 template <typename T, int NT, int NW, int PRE>
-static void mv_go(const bamd_dense & w, const bamd_batch_dev & b, const bamd_pre_args & p, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s, int parts = 1) {
+static void mv_go(const bamd_dense & w, const bamd_batch_dev & b, const bamd_pre_args & p, const void * x, int ldx, int cb, int rows, float * out, int ldo, hipStream_t s, int parts = 1) {
     const int grid = w.row_tiles < 4096 / NW ? w.row_tiles : 4096 / NW;       // what is resident at once; blocks walk the tiles
     const size_t lds = PRE == BAMD_PRE_ROWS ? 0 : bamd_dense_mv_lds(sizeof(T) == 4 ? BAMD_ACT_F32 : BAMD_ACT_BF16, w.k_tiles * 32);
-    hipLaunchKernelGGL((dense_mv_kernel<T, NT, NW, PRE>), dim3(grid, parts), dim3(64 * NW), lds, s, w, b, p, (const T *) x, ldx, rows, out, ldo);
+    hipLaunchKernelGGL((dense_mv_kernel<T, NT, NW, PRE>), dim3(grid, parts), dim3(64 * NW), lds, s, w, b, p, (const bamd_bf *) x, ldx, cb, rows, out, ldo);
 }
 // sixteen waves where the tiles alone would leave the chip half empty
 template <typename T, int PRE>
-static void mv_one(const bamd_dense & w, const bamd_batch_dev & b, const bamd_pre_args & p, const void * x, int ldx, int rows, float * out, int ldo, hipStream_t s, int parts = 1) {
-    if (w.row_tiles <= 256) mv_go<T, 1, 16, PRE>(w, b, p, x, ldx, rows, out, ldo, s, parts);
-    else mv_go<T, 1, 8, PRE>(w, b, p, x, ldx, rows, out, ldo, s);
+static void mv_one(const bamd_dense & w, const bamd_batch_dev & b, const bamd_pre_args & p, const void * x, int ldx, int cb, int rows, float * out, int ldo, hipStream_t s, int parts = 1) {
+    if (w.row_tiles <= 256) mv_go<T, 1, 16, PRE>(w, b, p, x, ldx, cb, rows, out, ldo, s, parts);
+    else mv_go<T, 1, 8, PRE>(w, b, p, x, ldx, cb, rows, out, ldo, s);
 }
 // Two shares of K where a matrix has too few row tiles for the CUs (more than 128 would make a second round of their blocks) and enough columns that halves are still worth a block: at K = 2048
 // they are level with 8 rows (2048 outputs: 5.7 us) and ahead with more (45 rows 8.7 -> 7.5) or longer rows (K = 4096: 7.1 -> 6.5, 11.8 -> 9.4).  A prologue that writes state stays whole.  A bfloat16
@@ -558,22 +543,24 @@ static int mv_pick(const bamd_dense & w, int pre, const bamd_batch_dev & b, cons
     const int n = few_parts(sizeof(T) == 4 ? BAMD_ACT_F32 : BAMD_ACT_BF16, w, pre, parts ? *parts : 1);
     if (parts) *parts = n;
     if (pre != BAMD_PRE_ROWS) {
-        if (rows != 1 || bamd_dense_mv_lds(sizeof(T) == 4 ? BAMD_ACT_F32 : BAMD_ACT_BF16, w.k_tiles * 32) > BAMD_MV_LDS) return 1;
+        if (rows != 1 || bamd_dense_mv_lds(sizeof(T) == 4 ? BAMD_ACT_F32 : BAMD_ACT_BF16, w.k_tiles * 32) > BAMD_MV_LDS(sizeof(T) == 4 ? BAMD_ACT_F32 : BAMD_ACT_BF16)) return 1;
         const int ldh = pre == BAMD_PRE_POLY ? p.poly.ldh : pre == BAMD_PRE_GROUP ? p.grp.ldh : pre == BAMD_PRE_GLU ? p.glu.ldh : p.res.ldh;
         if (ldh != w.k_tiles * 32) return 1;
-        if (pre == BAMD_PRE_RESIDUAL && p.res.norm != BAMD_NORM_LAYER) mv_one<T, BAMD_PRE_RESIDUAL>(w, b, p, x, ldx, rows, out, ldo, s);
-        else if (pre == BAMD_PRE_POLY) mv_one<T, BAMD_PRE_POLY>(w, b, p, x, ldx, rows, out, ldo, s, n);
-        else if (pre == BAMD_PRE_GROUP) mv_one<T, BAMD_PRE_GROUP>(w, b, p, x, ldx, rows, out, ldo, s, n);
-        else if (pre == BAMD_PRE_GLU) mv_one<T, BAMD_PRE_GLU>(w, b, p, x, ldx, rows, out, ldo, s, n);
-        else if (p.res.norm == BAMD_NORM_LAYER) mv_one<T, BAMD_PRE_LAYER>(w, b, p, x, ldx, rows, out, ldo, s);
-        else mv_one<T, BAMD_PRE_FINAL>(w, b, p, x, ldx, rows, out, ldo, s);
+        if (pre == BAMD_PRE_RESIDUAL && p.res.norm != BAMD_NORM_LAYER) mv_one<T, BAMD_PRE_RESIDUAL>(w, b, p, x, ldx, cb, rows, out, ldo, s);
+        else if (pre == BAMD_PRE_POLY) mv_one<T, BAMD_PRE_POLY>(w, b, p, x, ldx, cb, rows, out, ldo, s, n);
+        else if (pre == BAMD_PRE_GROUP) mv_one<T, BAMD_PRE_GROUP>(w, b, p, x, ldx, cb, rows, out, ldo, s, n);
+        else if (pre == BAMD_PRE_GLU) mv_one<T, BAMD_PRE_GLU>(w, b, p, x, ldx, cb, rows, out, ldo, s, n);
+        else if (p.res.norm == BAMD_NORM_LAYER) mv_one<T, BAMD_PRE_LAYER>(w, b, p, x, ldx, cb, rows, out, ldo, s);
+        else mv_one<T, BAMD_PRE_FINAL>(w, b, p, x, ldx, cb, rows, out, ldo, s);
         return 0;
     }
-    if (rows < 1 || rows > BAMD_MV_ROWS || (sizeof(T) == 4 && cb) || !rows_fit(w, ldx, cb, rows, 32)) return 1;
-    if constexpr (sizeof(T) == 2) return few_pick(w, x, cb ? 32 : ldx, cb ? cb : 32, rows, out, ldo, s, n, p.close);
-    else if (rows <= 16) mv_one<T, BAMD_PRE_ROWS>(w, b, p, x, ldx, rows, out, ldo, s, n);
-    else if (rows <= 32) mv_go<T, 2, 8, BAMD_PRE_ROWS>(w, b, p, x, ldx, rows, out, ldo, s, n);
-    else mv_go<T, 4, 8, BAMD_PRE_ROWS>(w, b, p, x, ldx, rows, out, ldo, s, n);
+    const int in_block = 32 * bamd_planes<T>;
+    if (rows < 1 || rows > BAMD_MV_ROWS || !rows_fit(w, ldx, cb, rows, in_block)) return 1;
+    if (cb) ldx = in_block; else cb = in_block;
+    if constexpr (sizeof(T) == 2) return few_pick(w, x, ldx, cb, rows, out, ldo, s, n, p.close);
+    else if (rows <= 16) mv_one<T, BAMD_PRE_ROWS>(w, b, p, x, ldx, cb, rows, out, ldo, s, n);
+    else if (rows <= 32) mv_go<T, 2, 8, BAMD_PRE_ROWS>(w, b, p, x, ldx, cb, rows, out, ldo, s, n);
+    else mv_go<T, 4, 8, BAMD_PRE_ROWS>(w, b, p, x, ldx, cb, rows, out, ldo, s, n);
     return 0;
 }
 // The gated unit as a part of the product in front of it costs the launch behind that (4 us) and 32-bit results on their way through memory; it asks for pairs of row tiles, which a block of

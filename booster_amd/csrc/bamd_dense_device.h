@@ -2,6 +2,7 @@
 // activation types, block reductions, and the row mechanisms in the form that both the row kernels and the prologues of the few-row product use.
 #pragma once
 #include "bamd_dense.h"
+#include <type_traits>
 
 typedef __bf16 bamd_bf;
 typedef __bf16 bamd_bf8 __attribute__((ext_vector_type(8)));
@@ -134,14 +135,43 @@ template <> __device__ __forceinline__ void store4<bamd_bf>(bamd_bf * h, bamd_v4
     typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
     *(bf4 *) h = bf4{ (bamd_bf) v[0], (bamd_bf) v[1], (bamd_bf) v[2], (bamd_bf) v[3] };
 }
-// a row of operands being written (null: not wanted)
-template <typename T> struct RowOut {
-    T * p; int cb;
-    __device__ __forceinline__ explicit operator bool() const { return p != nullptr; }
-    __device__ __forceinline__ T * at(int i) const { return p + (i >> 5) * cb + (i & 31); }
+// A 32-bit operand is the sum of three bfloat16 numbers, eight bits of its significand each (cut off, not rounded: parts of one sign, and what is left is exact), in planes 32 elements apart.  A value
+// that is not finite is its first plane alone
+struct Split { uint32_t p[3]; };                                   // in the upper sixteen bits
+__device__ __forceinline__ Split split_f(float v) {
+    const uint32_t u = __float_as_uint(v);
+    const bool finite = (u & 0x7f800000u) != 0x7f800000u;
+    const float m = finite ? v - __uint_as_float(u & 0xffff0000u) : 0.f, l = m - __uint_as_float(__float_as_uint(m) & 0xffff0000u);
+    return { { finite || !(u & 0x007fffffu) ? u : u | 0x00400000u, __float_as_uint(m), __float_as_uint(l) } };
+}
+struct bamd_s3 {
+    uint16_t v;
+    __device__ __forceinline__ void operator=(Split s) { (&v)[0] = (uint16_t) (s.p[0] >> 16); (&v)[32] = (uint16_t) (s.p[1] >> 16); (&v)[64] = (uint16_t) (s.p[2] >> 16); }
 };
-template <typename T> __device__ __forceinline__ RowOut<T> row_out(void * h, int row, int ld, int cb) { return { h ? (T *) h + (size_t) row * (cb ? 32 : ld) : nullptr, cb ? cb : 32 }; }
-template <typename T> __device__ __forceinline__ void zero_tail(RowOut<T> h, int n, int ld) { for (int i = n + threadIdx.x; i < ld; i += blockDim.x) *h.at(i) = to_act<T>(0.f); }
+template <typename T> struct OperandOf { typedef T type; };
+template <> struct OperandOf<float> { typedef bamd_s3 type; };
+template <typename T> using Operand = typename OperandOf<T>::type;      // what the operand rows of products in compute type T are made of
+template <typename T> constexpr int bamd_planes = sizeof(T) == 4 ? 3 : 1;
+template <typename O> __device__ __forceinline__ auto to_operand(float f) { if constexpr (std::is_same<O, bamd_s3>::value) return split_f(f); else return (O) f; }
+template <> __device__ __forceinline__ void store4<bamd_s3>(bamd_s3 * h, bamd_v4 v) {
+    Split s[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s[i] = split_f(v[i]);
+#pragma unroll
+    for (int n = 0; n < 3; ++n) *(uint2 *) ((uint16_t *) h + n * 32) = uint2{ (s[0].p[n] >> 16) | (s[1].p[n] & 0xffff0000u), (s[2].p[n] >> 16) | (s[3].p[n] & 0xffff0000u) };
+}
+// a row of operands (O) being written (null: not wanted)
+template <typename O> struct RowOut {
+    static constexpr int P = std::is_same<O, bamd_s3>::value ? 3 : 1;
+    O * p; int cb;
+    __device__ __forceinline__ explicit operator bool() const { return p != nullptr; }
+    __device__ __forceinline__ O * at(int i) const { return p + (i >> 5) * cb + (i & 31); }
+};
+template <typename O> __device__ __forceinline__ RowOut<O> row_out(void * h, int row, int ld, int cb) {
+    constexpr int P = RowOut<O>::P;
+    return { h ? (O *) h + (size_t) row * (cb ? 32 * P : ld * P) : nullptr, cb ? cb : 32 * P };
+}
+template <typename O> __device__ __forceinline__ void zero_tail(RowOut<O> h, int n, int ld) { for (int i = n + threadIdx.x; i < ld; i += blockDim.x) *h.at(i) = to_operand<O>(0.f); }
 
 __device__ __forceinline__ float parts_sum(const float * p, int parts, size_t plane) { return parts > 1 ? p[0] + p[plane] : p[0]; }
 
@@ -228,7 +258,7 @@ __device__ __forceinline__ void layer_row(const bamd_residual_args & a, int row,
     for (int i = threadIdx.x; i < E; i += blockDim.x) {
         const float xn = at(i);
         if (write) xo[i] = xn;
-        if (h) *h.at(i) = to_act<T>(gi ? (xn - mx) * rx * gi[i] : xn);
+        if (h) *h.at(i) = to_operand<T>(gi ? (xn - mx) * rx * gi[i] : xn);
     }
     if (h) zero_tail(h, E, a.ldh);
 }
@@ -304,7 +334,7 @@ __device__ __forceinline__ void residual_row(const bamd_batch_dev & b, const bam
             hn = xn + (pv - xn) * a.mu[i];
         }
         if (write) { a.xo[(size_t) row * E + i] = xn; if (so) so[i] = xn; }
-        if (h) *h.at(i) = to_act<T>(hn);
+        if (h) *h.at(i) = to_operand<T>(hn);
     }
     if (h) zero_tail(h, E, a.ldh);
 }
@@ -342,7 +372,7 @@ __device__ __forceinline__ void final_row(const bamd_residual_args & a, int row,
     for (int i = threadIdx.x; i < E; i += blockDim.x) { const float xn = y ? x[i] + parts_sum(y + i, a.parts, a.plane) * r : x[i]; w[0] += xn * xn; }
     block_sum<1>(w, red);
     const float rf = gf[0] / sqrtf(w[0] / (float) E + a.eps);
-    for (int i = threadIdx.x; i < E; i += blockDim.x) *h.at(i) = to_act<T>((y ? x[i] + parts_sum(y + i, a.parts, a.plane) * r : x[i]) * rf);
+    for (int i = threadIdx.x; i < E; i += blockDim.x) *h.at(i) = to_operand<T>((y ? x[i] + parts_sum(y + i, a.parts, a.plane) * r : x[i]) * rf);
     zero_tail(h, E, a.ldh);
 }
 template <typename T>
@@ -372,7 +402,7 @@ __device__ __forceinline__ void poly_row(const bamd_poly_args & a, int row, RowO
             for (int k = 0; k < 4; ++k) { const float t = zr.v[c][k], t2 = t * t; o[k] = c1 * t + c2 * t2 + c3 * (t2 * t) + c0; }
             store4<T>(h.at(i), o);
         }
-    } else for (int i = threadIdx.x; i < a.F; i += blockDim.x) { const float t = z[i], t2 = t * t; *h.at(i) = to_act<T>(c1 * t + c2 * t2 + c3 * (t2 * t) + c0); }
+    } else for (int i = threadIdx.x; i < a.F; i += blockDim.x) { const float t = z[i], t2 = t * t; *h.at(i) = to_operand<T>(c1 * t + c2 * t2 + c3 * (t2 * t) + c0); }
     zero_tail(h, a.F, a.ldh);
 }
 // inv: LDS, one float per part and 16 more
@@ -419,6 +449,6 @@ __device__ __forceinline__ void group_norm_row(const bamd_group_norm_args & a, i
         }
         __syncthreads();
     }
-    for (int i = threadIdx.x; i < a.n; i += blockDim.x) *h.at(i) = to_act<T>(y[i] * inv[i / per] * a.w[i]);
+    for (int i = threadIdx.x; i < a.n; i += blockDim.x) *h.at(i) = to_operand<T>(y[i] * inv[i / per] * a.w[i]);
     zero_tail(h, a.n, a.ldh);
 }

@@ -132,7 +132,7 @@ __device__ __forceinline__ void gla_scan_block(const bamd_gla_args & a, int h, i
 template <typename T> __device__ __forceinline__ void gla_norm_block(const bamd_gla_args & a, int h0, int row) {
     constexpr int RC = 4;
     const int h = h0 + (threadIdx.x >> 4), l = (threadIdx.x & 15) * 4;
-    const RowOut<T> out = row_out<T>(a.out, row, a.ldo, a.cb);
+    const RowOut<Operand<T>> out = row_out<Operand<T>>(a.out, row, a.ldo, a.cb);
     if (h < a.heads) {
         const float * y = a.y + (size_t) row * a.ldy + h * a.Pp, * g = a.g_off >= 0 ? a.in + (size_t) row * a.ld + a.g_off + h * a.Pp : nullptr;
         bamd_v4 v[RC], gv[RC];
@@ -152,11 +152,11 @@ template <typename T> __device__ __forceinline__ void gla_norm_block(const bamd_
             if (g)
 #pragma unroll
                 for (int k = 0; k < 4; ++k) t[k] *= gate[k] / (1.0f + __expf(-gate[k]));
-            store4<T>(out.at(a.out_off + h * a.Pp + i), t);
+            store4<Operand<T>>(out.at(a.out_off + h * a.Pp + i), t);
         };
 #pragma unroll
         for (int c = 0; c < RC; ++c) if (l + c * 64 < a.Pp) put(l + c * 64, v[c], gv[c]);
         for (int i = l + RC * 64; i < a.Pp; i += 64) put(i, *(const bamd_v4 *) (y + i), g ? *(const bamd_v4 *) (g + i) : bamd_v4{ 0, 0, 0, 0 });
     }
-    if (h0 + 16 >= a.heads) for (int c = a.heads * a.Pp + threadIdx.x; c < a.out_cols; c += 256) *out.at(a.out_off + c) = to_act<T>(0.f);
+    if (h0 + 16 >= a.heads) for (int c = a.heads * a.Pp + threadIdx.x; c < a.out_cols; c += 256) *out.at(a.out_off + c) = to_operand<Operand<T>>(0.f);
 }

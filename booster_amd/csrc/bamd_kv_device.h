@@ -259,6 +259,6 @@ __device__ __forceinline__ void kv_combine_block(const bamd_kv_args & a, int h, 
         const float * src = part_o + (base * 16 + hh % 16) * a.D + d;
         float t = 0.f;
         for (int s = 0; s < splits; ++s) t += wt[s] * src[(size_t) s * 16 * a.D];
-        *row_out<T>(a.out, row, a.ldo, a.cb).at(a.out_off + h * a.D + d) = to_act<T>(t * f);
+        *row_out<Operand<T>>(a.out, row, a.ldo, a.cb).at(a.out_off + h * a.D + d) = to_operand<Operand<T>>(t * f);
     }
 }

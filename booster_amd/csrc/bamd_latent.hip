@@ -187,9 +187,9 @@ __global__ void __launch_bounds__(256, sizeof(T) == 2 && ND <= 4 ? 2 : 1) latent
             if (row >= e.n) continue;
             float f = 1.0f / sum;
             if (a.gated) f *= sigmoid_f(a.in[(size_t) (e.row0 + row) * a.ld + a.g_off + h]);
-            const RowOut<T> d = row_out<T>(a.out, e.row0 + row, a.ldo, a.cb);
+            const RowOut<Operand<T>> d = row_out<Operand<T>>(a.out, e.row0 + row, a.ldo, a.cb);
 #pragma unroll
-            for (int j = 0; j < NV; ++j) *d.at(h * D + j * 16 + lr) = to_act<T>(o[i][j][r] * f);
+            for (int j = 0; j < NV; ++j) *d.at(h * D + j * 16 + lr) = to_operand<Operand<T>>(o[i][j][r] * f);
         }
 }
 
@@ -371,7 +371,7 @@ template <typename T> __global__ void __launch_bounds__(512) latent_combine_kern
             v += bf_lo(w.x) * x[0] + bf_hi(w.x) * x[1] + bf_lo(w.y) * x[2] + bf_hi(w.y) * x[3] + bf_lo(w.z) * x[4] + bf_hi(w.z) * x[5] + bf_lo(w.w) * x[6] + bf_hi(w.w) * x[7];
         }
         v += __shfl_xor(v, 16); v += __shfl_xor(v, 32);
-        if (lane < 16) *row_out<T>(a.out, row, a.ldo, a.cb).at(h * a.D + t * 16 + lane) = to_act<T>(v * inv);
+        if (lane < 16) *row_out<Operand<T>>(a.out, row, a.ldo, a.cb).at(h * a.D + t * 16 + lane) = to_operand<Operand<T>>(v * inv);
     }
 }
 

@@ -123,28 +123,28 @@ void bamd_launch_step_close(const float * logits, size_t n, float * host, bamd_s
 }
 void bamd_launch_residual_rows(int act, const bamd_batch_dev & b, const bamd_residual_args & a, hipStream_t s) {
     if (a.norm == BAMD_NORM_LAYER) {
-        if (act == BAMD_ACT_F32) hipLaunchKernelGGL(layer_rows_kernel<float>, dim3(b.rows), sum_block(a.E, b.rows), 0, s, a, nullptr, a.gi);
+        if (act == BAMD_ACT_F32) hipLaunchKernelGGL(layer_rows_kernel<bamd_s3>, dim3(b.rows), sum_block(a.E, b.rows), 0, s, a, nullptr, a.gi);
         else hipLaunchKernelGGL(layer_rows_kernel<bamd_bf>, dim3(b.rows), sum_block(a.E, b.rows), 0, s, a, nullptr, a.gi);
-    } else if (act == BAMD_ACT_F32) hipLaunchKernelGGL(residual_rows_kernel<float>, dim3(b.rows), sum_block(a.E, b.rows), 0, s, b, a);
+    } else if (act == BAMD_ACT_F32) hipLaunchKernelGGL(residual_rows_kernel<bamd_s3>, dim3(b.rows), sum_block(a.E, b.rows), 0, s, b, a);
     else hipLaunchKernelGGL(residual_rows_kernel<bamd_bf>, dim3(b.rows), sum_block(a.E, b.rows), 0, s, b, a);
 }
 void bamd_launch_final_rows(int act, const bamd_residual_args & a, const int32_t * want, int n_want, const float * gf, hipStream_t s) {
     if (a.norm == BAMD_NORM_LAYER) {
-        if (act == BAMD_ACT_F32) hipLaunchKernelGGL(layer_rows_kernel<float>, dim3(n_want), sum_block(a.E, n_want), 0, s, a, want, gf);
+        if (act == BAMD_ACT_F32) hipLaunchKernelGGL(layer_rows_kernel<bamd_s3>, dim3(n_want), sum_block(a.E, n_want), 0, s, a, want, gf);
         else hipLaunchKernelGGL(layer_rows_kernel<bamd_bf>, dim3(n_want), sum_block(a.E, n_want), 0, s, a, want, gf);
-    } else if (act == BAMD_ACT_F32) hipLaunchKernelGGL(final_rows_kernel<float>, dim3(n_want), sum_block(a.E, n_want), 0, s, a, want, gf);
+    } else if (act == BAMD_ACT_F32) hipLaunchKernelGGL(final_rows_kernel<bamd_s3>, dim3(n_want), sum_block(a.E, n_want), 0, s, a, want, gf);
     else hipLaunchKernelGGL(final_rows_kernel<bamd_bf>, dim3(n_want), sum_block(a.E, n_want), 0, s, a, want, gf);
 }
 void bamd_launch_poly_rows(int act, int rows, const bamd_poly_args & a, hipStream_t s) {
-    if (act == BAMD_ACT_F32) hipLaunchKernelGGL(poly_rows_kernel<float>, dim3(rows), row_block(a.F), 0, s, a);
+    if (act == BAMD_ACT_F32) hipLaunchKernelGGL(poly_rows_kernel<bamd_s3>, dim3(rows), row_block(a.F), 0, s, a);
     else hipLaunchKernelGGL(poly_rows_kernel<bamd_bf>, dim3(rows), row_block(a.F), 0, s, a);
 }
 void bamd_launch_glu_rows(int act, int rows, const bamd_glu_args & a, hipStream_t s) {
-    if (act == BAMD_ACT_F32) hipLaunchKernelGGL(glu_rows_kernel<float>, dim3((a.ldh + 1023) / 1024, rows), dim3(256), 0, s, a);
+    if (act == BAMD_ACT_F32) hipLaunchKernelGGL(glu_rows_kernel<bamd_s3>, dim3((a.ldh + 1023) / 1024, rows), dim3(256), 0, s, a);
     else hipLaunchKernelGGL(glu_rows_kernel<bamd_bf>, dim3((a.ldh + 1023) / 1024, rows), dim3(256), 0, s, a);
 }
 void bamd_launch_group_norm_rows(int act, int rows, const bamd_group_norm_args & a, hipStream_t s) {
-    if (act == BAMD_ACT_F32) hipLaunchKernelGGL(group_norm_rows_kernel<float>, dim3(rows), row_block(a.n), 0, s, a);
+    if (act == BAMD_ACT_F32) hipLaunchKernelGGL(group_norm_rows_kernel<bamd_s3>, dim3(rows), row_block(a.n), 0, s, a);
     else hipLaunchKernelGGL(group_norm_rows_kernel<bamd_bf>, dim3(rows), row_block(a.n), 0, s, a);
 }
 void bamd_launch_argmax_rows(const float * logits, int n, int V, unsigned long long * keys, bool clear, hipStream_t s) {

@@ -199,7 +199,7 @@ struct Ctx {
     int ldy = 0, ldy2 = 0, ldy3 = 0, ldh = 0;
     void * qp = nullptr; float * part_o = nullptr, * part_ml = nullptr;
     void * kc = nullptr, * kk = nullptr, * kv = nullptr; size_t kc_n = 0, kk_n = 0, kv_n = 0;      // unpacked latents / keys / values of a prompt pass
-    void * planes = nullptr; size_t planes_n = 0;                                                  // 32-bit operand rows of a prompt's product, split
+    void * planes = nullptr; size_t planes_n = 0;                                                  // 32-bit latents of a prompt pass as operand rows
     float * filtered = nullptr, * steps = nullptr; size_t filtered_n = 0, steps_n = 0;             // filtered channels, step sizes and decays of a prompt pass
     float * alpha = nullptr, * seg_state = nullptr, * seg_decay = nullptr; size_t alpha_n = 0, seg_state_n = 0, seg_decay_n = 0;      // decays and segment states of a prompt pass
     unsigned long long * keys = nullptr; int32_t * step = nullptr, * gen_out = nullptr; int gen_cap = 0;
@@ -218,7 +218,7 @@ struct Pass {                                      // one pass through the layer
     void begin(int kind, double bytes) { if (!tm) return; hipEvent_t e; hipEventCreate(&e); hipEventRecord(e, s); tm->ev.push_back(e); tm->kind.push_back(kind); tm->bytes.push_back(bytes); }
     void end() { if (!tm) return; hipEvent_t e; hipEventCreate(&e); hipEventRecord(e, s); tm->ev.push_back(e); }
 
-    int cb() const { return st.act == BAMD_ACT_BF16 && b.rows > 1 ? bamd_row_blocks(b.rows) : 0; }      // how the operand rows of this pass's products lie (bamd_dense.h): one row, and 32-bit rows, by rows
+    int cb() const { return b.rows > 1 ? bamd_row_planes(st.act) * bamd_row_blocks(b.rows) : 0; }      // how the operand rows of this pass's products lie (bamd_dense.h): one row by rows
     bamd_residual_args residual(const float * mu, float * prev, const float * gi) {
         bamd_residual_args a; memset(&a, 0, sizeof a);
         a.norm = st.d.norm == STACK_NORM_SANDWICH ? BAMD_NORM_LAYER : BAMD_NORM_RMS; a.gi = gi;
@@ -226,19 +226,19 @@ struct Pass {                                      // one pass through the layer
         return a;
     }
     void advanced(const float * y, int ld, const float * g, int parts) { std::swap(x, xo); pend = y; ldp = ld; pend_g = g; pend_parts = parts; }
-    int split(const bamd_dense & w, const void * & x, int & ldx, int & cb, int rows);      // 32-bit operand rows as bamd_launch_dense_gemm takes them; bfloat16 rows are left alone
+    int split(const bamd_dense & w, const void * & x, int & ldx, int & cb, int rows);      // rows in the compute type as operand rows
     // a product whose operand rows exist; small row counts stream the weights once
     // parts: in, shares of K the result's buffer can hold; out, shares there are (the rows' residual sum adds them)
     int product(const bamd_dense & w, const void * in, int ldx, float * out, int ldo, int kind, int * parts = nullptr) {
         begin(kind, (double) w.bytes);
-        int blocks = cb();
-        if (b.rows > BAMD_MV_ROWS && split(w, in, ldx, blocks, b.rows)) return 1;
+        const int blocks = cb();
+        ldx *= bamd_row_planes(st.act);
         const int rc = b.rows <= BAMD_MV_ROWS ? bamd_launch_dense_mv(st.act, w, BAMD_PRE_ROWS, b, nullptr, in, ldx, blocks, b.rows, out, ldo, s, parts)
                                               : bamd_launch_dense_gemm(st.act, w, in, ldx, blocks, b.rows, out, ldo, BAMD_OUT_F32, s, 0.f, parts);
         end();
         return rc ? fail("dense product: unsupported shape") : 0;
     }
-    bool fused(const bamd_dense & w) const { return b.rows == 1 && decode && bamd_dense_mv_lds(st.act, w.K) <= BAMD_MV_LDS; }
+    bool fused(const bamd_dense & w) const { return b.rows == 1 && decode && bamd_dense_mv_lds(st.act, w.K) <= BAMD_MV_LDS(st.act); }
     int product_pre(const bamd_dense & w, int pre, const bamd_pre_args & p, float * out, int ldo, int kind, int * parts = nullptr) {
         if (fused(w)) {
             begin(kind, (double) w.bytes);
@@ -589,7 +589,7 @@ int Stack::context_init(bamd_context * bc) {
     }
     const size_t R = (size_t) up(c.rows_cap, 16);                  // (as bamd_row_blocks rounds)
     if (dev_alloc(bc->allocs, (void **) &c.xa, R * E * 4) || dev_alloc(bc->allocs, (void **) &c.xb, R * E * 4) || dev_alloc(bc->allocs, (void **) &c.y, R * std::max(c.ldy, 16) * 4) ||
-        dev_alloc(bc->allocs, (void **) &c.y2, R * c.ldy2 * 4 * Y2_PLANES) || dev_alloc(bc->allocs, (void **) &c.y3, R * std::max(c.ldy3, 16) * 4) || dev_alloc(bc->allocs, &c.h, R * c.ldh * el())) return 1;
+        dev_alloc(bc->allocs, (void **) &c.y2, R * c.ldy2 * 4 * Y2_PLANES) || dev_alloc(bc->allocs, (void **) &c.y3, R * std::max(c.ldy3, 16) * 4) || dev_alloc(bc->allocs, &c.h, R * c.ldh * 2 * bamd_row_planes(act))) return 1;
     if (qp && dev_alloc(bc->allocs, &c.qp, qp * el())) return 1;
     if (po && (dev_alloc(bc->allocs, (void **) &c.part_o, po * 4) || dev_alloc(bc->allocs, (void **) &c.part_ml, pm * 4))) return 1;
     if (qp) HIPC(hipMemset(c.qp, 0, qp * el()));                  // rows of absent heads stay zero
@@ -665,7 +665,7 @@ int grow(Ctx & c, void ** p, size_t * have, size_t need, hipStream_t s) {
 int Pass::split(const bamd_dense & w, const void * & x, int & ldx, int & cb, int rows) {
     if (st.act != BAMD_ACT_F32) return 0;
     cb = 3 * bamd_row_blocks(rows);
-    if (grow(c, &c.planes, &c.planes_n, (size_t) cb * std::max(c.ldh, w.K) / 32 * 2, s)) return 1;
+    if (grow(c, &c.planes, &c.planes_n, (size_t) cb * w.k_tiles * 2, s)) return 1;
     bamd_launch_split_rows((const float *) x, ldx, rows, w.k_tiles, c.planes, cb, s);
     x = c.planes;
     return 0;
@@ -775,10 +775,9 @@ int Pass::layers() {
         if (few || (glu && b.rows > BAMD_MV_ROWS)) {                // the product writes the down-projection's operand
             begin(2, 0); bamd_launch_residual_rows(st.act, b, pa.res, s); end();
             begin(4, (double) ly.up.bytes);
-            const void * in = c.h; int ldx = pa.res.ldh, blocks = cb();
-            if (!few && split(ly.up, in, ldx, blocks, b.rows)) return 1;
-            const int rc = few ? bamd_launch_dense_few_glu(ly.up, in, ldx, blocks, b.rows, c.y, ly.down.K, cb(), ly.limit, s)
-                               : bamd_launch_dense_gemm(st.act, ly.up, in, ldx, blocks, b.rows, c.y, ly.down.K, BAMD_OUT_GLU, s, ly.limit, nullptr, cb());
+            const int ldx = pa.res.ldh * bamd_row_planes(st.act), blocks = cb();
+            const int rc = few ? bamd_launch_dense_few_glu(ly.up, c.h, ldx, blocks, b.rows, c.y, ly.down.K, blocks, ly.limit, s)
+                               : bamd_launch_dense_gemm(st.act, ly.up, c.h, ldx, blocks, b.rows, c.y, ly.down.K, BAMD_OUT_GLU, s, ly.limit, nullptr, blocks);
             end();
             if (rc) return fail("dense product: unsupported shape");
             if (product(ly.down, c.y, ly.down.K, c.y2, c.ldy2, 5, &parts)) return 1;
@@ -803,7 +802,7 @@ int Pass::head(const int32_t * want, int n, float * logits, const bamd_step_out 
         end();
         return rc ? fail("dense product: unsupported shape") : 0;
     }
-    a.cb = st.act == BAMD_ACT_BF16 ? bamd_row_blocks(n) : 0;
+    a.cb = bamd_row_planes(st.act) * bamd_row_blocks(n);
     bamd_launch_final_rows(st.act, a, want, n, st.norm_f, s);
     begin(6, (double) st.head.bytes);
     const int rc = bamd_launch_dense_mv(st.act, st.head, BAMD_PRE_ROWS, b, &pa, c.h, a.ldh, a.cb, n, logits, st.V, s);
@@ -1152,28 +1151,46 @@ struct OpScratch {                                 // device copies of one call
     }
     int alloc(void ** p, size_t bytes) { if (dev_alloc(keep, p, std::max<size_t>(bytes, 16))) return 1; HIPC(hipMemset(*p, 0, std::max<size_t>(bytes, 16))); return 0; }
     template <typename U> int up_(const U * h, size_t n, U ** d) { if (alloc((void **) d, n * sizeof(U))) return 1; if (n) HIPC(hipMemcpy(*d, h, n * sizeof(U), hipMemcpyHostToDevice)); return 0; }
-    // f32 host rows [rows][n] -> activation rows [rows][ld]
-    int act_rows(const float * h, int rows, int n, int ld, void ** d, bool blocks = false) {
-        const bool f = l.act == BAMD_ACT_F32;
-        const int cb = bamd_row_blocks(rows);
-        std::vector<unsigned char> b((blocks ? (size_t) cb * (ld / 32) : (size_t) rows * ld) * (f ? 4 : 2), 0);
+    // f32 host rows [rows][n] -> rows [rows][ld] in the compute type, or operand rows
+    int act_rows(const float * h, int rows, int n, int ld, void ** d) { return rows_to(h, rows, n, ld, d, l.act == BAMD_ACT_F32, 0); }
+    int operand_rows(const float * h, int rows, int n, int ld, void ** d, int cb = 0) { return rows_to(h, rows, n, ld, d, false, bamd_row_planes(l.act), cb); }
+    // place of value (r, i) of operand rows
+    static size_t operand_at(int r, int i, int ld, int planes, int cb) { return cb ? (size_t) (i >> 5) * cb + (size_t) r * 32 * planes + (i & 31) : (size_t) r * ld * planes + (size_t) (i >> 5) * 32 * planes + (i & 31); }
+    int rows_to(const float * h, int rows, int n, int ld, void ** d, bool f, int planes, int cb = 0) {
+        std::vector<unsigned char> b(f ? (size_t) rows * ld * 4 : (cb ? (size_t) cb * (ld / 32) : (size_t) rows * ld * std::max(planes, 1)) * 2, 0);
         for (int r = 0; r < rows; ++r) for (int i = 0; i < n; ++i) {
-            const float v = h[(size_t) r * n + i];
-            const size_t at = blocks ? (size_t) (i >> 5) * cb + r * 32 + (i & 31) : (size_t) r * ld + i;
-            if (f) memcpy(&b[at * 4], &v, 4);
-            else { uint32_t u; memcpy(&u, &v, 4); u += 0x7fff + ((u >> 16) & 1); const uint16_t o = (uint16_t) (u >> 16); memcpy(&b[at * 2], &o, 2); }
+            float v = h[(size_t) r * n + i];
+            uint32_t u; memcpy(&u, &v, 4);
+            if (f) { memcpy(&b[((size_t) r * ld + i) * 4], &v, 4); continue; }
+            const size_t at = operand_at(r, i, ld, std::max(planes, 1), cb) * 2;
+            if (planes < 3) { u += 0x7fff + ((u >> 16) & 1); const uint16_t o = (uint16_t) (u >> 16); memcpy(&b[at], &o, 2); continue; }
+            const bool finite = (u & 0x7f800000u) != 0x7f800000u;
+            if (!finite && (u & 0x007fffffu)) u |= 0x00400000u;
+            for (int k = 0; k < 3; ++k) {
+                const uint16_t o = (uint16_t) (u >> 16); memcpy(&b[at + 64 * k], &o, 2);
+                const uint32_t top = u & 0xffff0000u; float t; memcpy(&t, &top, 4);
+                v = finite ? v - t : 0.f; memcpy(&u, &v, 4);
+            }
         }
         if (alloc(d, b.size())) return 1;
         HIPC(hipMemcpy(*d, b.data(), b.size(), hipMemcpyHostToDevice));
         return 0;
     }
-    int rows_back(const void * d, int rows, int n, int ld, float * h, bool f) {
-        std::vector<unsigned char> b((size_t) rows * ld * (f ? 4 : 2));
+    int rows_back(const void * d, int rows, int n, int ld, float * h, bool f) { return rows_from(d, rows, n, ld, h, f, 1); }
+    int operand_back(const void * d, int rows, int n, int ld, float * h) { return rows_from(d, rows, n, ld, h, false, bamd_row_planes(l.act)); }
+    int rows_from(const void * d, int rows, int n, int ld, float * h, bool f, int planes) {
+        std::vector<unsigned char> b((size_t) rows * ld * (f ? 4 : 2 * planes));
         HIPC(hipStreamSynchronize(l.s));
         HIPC(hipMemcpy(b.data(), d, b.size(), hipMemcpyDeviceToHost));
         for (int r = 0; r < rows; ++r) for (int i = 0; i < n; ++i) {
-            if (f) memcpy(&h[(size_t) r * n + i], &b[((size_t) r * ld + i) * 4], 4);
-            else { uint16_t o; memcpy(&o, &b[((size_t) r * ld + i) * 2], 2); const uint32_t u = (uint32_t) o << 16; memcpy(&h[(size_t) r * n + i], &u, 4); }
+            float & o = h[(size_t) r * n + i];
+            if (f) { memcpy(&o, &b[((size_t) r * ld + i) * 4], 4); continue; }
+            o = 0.f;
+            for (int k = planes - 1; k >= 0; --k) {               // (the smallest first: each sum is exact)
+                uint16_t v; memcpy(&v, &b[operand_at(r, i, ld, planes, 0) * 2 + 64 * k], 2);
+                const uint32_t u = (uint32_t) v << 16; float t; memcpy(&t, &u, 4);
+                o = k == planes - 1 ? t : t + o;
+            }
         }
         return 0;
     }
@@ -1211,20 +1228,19 @@ BAMD_OP bamd_op_dense_route(int act, int nrows, int k, int rows, int pre, int mo
 }
 BAMD_OP bamd_op_dense(int act, const uint16_t * w, int nrows, int k, const float * x, int rows, int impl, float * y) {
     OpScratch s; bamd_dense d; void * dx; float * dy = nullptr;
-    const bool blocks = impl == 6 || impl == 7;                   // as impl 0 and 1, the operand rows by blocks
-    if (!w || !x || !y || nrows < 1 || k < 1 || rows < 1 || s.init(act) || (blocks && act != BAMD_ACT_BF16)) return fail("bamd_op_dense: bad arguments");
-    if (blocks) impl -= 6;
+    const int planes = bamd_row_planes(act), cb = impl == 6 || impl == 7 ? planes * bamd_row_blocks(rows) : 0;                   // 6, 7: as impl 0 and 1, the operand rows by blocks
+    if (!w || !x || !y || nrows < 1 || k < 1 || rows < 1 || s.init(act)) return fail("bamd_op_dense: bad arguments");
+    if (cb) impl -= 6;
     const SafeTensor t = bf16_tensor(w, { nrows, k });
-    if (s.l.alloc(d, nrows, k) || s.l.pack(&t, Loader::steps(nrows, k), Loader::steps(k, 1), const_cast<uint16_t *>(d.w)) || s.act_rows(x, rows, k, d.K, &dx, blocks)) return 1;
+    if (s.l.alloc(d, nrows, k) || s.l.pack(&t, Loader::steps(nrows, k), Loader::steps(k, 1), const_cast<uint16_t *>(d.w)) || s.operand_rows(x, rows, k, d.K, &dx, cb)) return 1;
     const int ldo = impl == 3 ? up(rows, 64) : ld_of(d);
     int parts = impl == 4 || impl == 5 ? 2 : 1;
     if (s.alloc((void **) &dy, (size_t) (impl == 3 ? ld_of(d) : rows) * ldo * 4 * parts)) return 1;
     bamd_batch_dev b; memset((void *) &b, 0, sizeof b);
-    int rc, ldx = d.K, cb = blocks ? bamd_row_blocks(rows) : 0; const void * px = dx;
-    if (impl != 1 && impl != 5 && s.split(d, px, ldx, cb, rows)) return 1;
+    int rc; const int ldx = d.K * planes; const void * px = dx;
     if (impl == 4) rc = bamd_launch_dense_gemm(act, d, px, ldx, cb, rows, dy, ldo, BAMD_OUT_F32, s.l.s, 0.f, &parts);
-    else if (impl == 5) rc = bamd_launch_dense_mv(act, d, BAMD_PRE_ROWS, b, nullptr, dx, d.K, 0, rows, dy, ldo, s.l.s, &parts);
-    else if (impl == 1) rc = bamd_launch_dense_mv(act, d, BAMD_PRE_ROWS, b, nullptr, dx, d.K, cb, rows, dy, ldo, s.l.s);
+    else if (impl == 5) rc = bamd_launch_dense_mv(act, d, BAMD_PRE_ROWS, b, nullptr, dx, ldx, cb, rows, dy, ldo, s.l.s, &parts);
+    else if (impl == 1) rc = bamd_launch_dense_mv(act, d, BAMD_PRE_ROWS, b, nullptr, dx, ldx, cb, rows, dy, ldo, s.l.s);
     else rc = bamd_launch_dense_gemm(act, d, px, ldx, cb, rows, dy, ldo, impl == 0 ? BAMD_OUT_F32 : impl == 2 ? BAMD_OUT_ACT : BAMD_OUT_ACT_T, s.l.s);
     if (rc) return fail("bamd_op_dense: unsupported shape");
     HIPC(hipGetLastError());
@@ -1246,42 +1262,41 @@ BAMD_OP bamd_op_dense_glu(int act, const uint16_t * gate, const uint16_t * upw, 
     const int ldo = up(F, 32);
     const SafeTensor tg = bf16_tensor(gate, { F, k }), tu = bf16_tensor(upw, { F, k });
     std::vector<int32_t> at = Loader::steps(F, k); at.resize((size_t) ldo, -1);
-    if (s.l.alloc(d, 2 * ldo, k) || s.act_rows(x, rows, k, d.K, &dx) || s.alloc((void **) &dy, (size_t) rows * ldo * 4)) return 1;
+    if (s.l.alloc(d, 2 * ldo, k) || s.operand_rows(x, rows, k, d.K, &dx) || s.alloc((void **) &dy, (size_t) rows * ldo * 6)) return 1;
     uint16_t * w = const_cast<uint16_t *>(d.w);
     if (s.l.pack(&tg, at, Loader::steps(k, 1), w, 2) || s.l.pack(&tu, at, Loader::steps(k, 1), w + (size_t) 16 * d.K, 2)) return 1;
-    const bool few = bamd_dense_few_glu(act, d, rows); const void * px = dx; int ldx = d.K, cb = 0;
-    if (!few && s.split(d, px, ldx, cb, rows)) return 1;
-    if (few ? bamd_launch_dense_few_glu(d, dx, d.K, 0, rows, dy, ldo, 0, limit, s.l.s) : bamd_launch_dense_gemm(act, d, px, ldx, cb, rows, dy, ldo, BAMD_OUT_GLU, s.l.s, limit)) return fail("bamd_op_dense_glu: unsupported shape");
+    const bool few = bamd_dense_few_glu(act, d, rows); const int ldx = d.K * bamd_row_planes(act);
+    if (few ? bamd_launch_dense_few_glu(d, dx, ldx, 0, rows, dy, ldo, 0, limit, s.l.s) : bamd_launch_dense_gemm(act, d, dx, ldx, 0, rows, dy, ldo, BAMD_OUT_GLU, s.l.s, limit)) return fail("bamd_op_dense_glu: unsupported shape");
     HIPC(hipGetLastError());
-    return s.rows_back(dy, rows, F, ldo, y, act == BAMD_ACT_F32);
+    return s.operand_back(dy, rows, F, ldo, y);
 }
 BAMD_OP bamd_op_residual_rows(int act, const float * x, const float * y, float g, float eps, const float * mu, float * prev, int pos0, int rows, int E, float * xo, float * h) {
     OpScratch s; bamd_batch_dev b; bamd_residual_args a; memset((void *) &a, 0, sizeof a);
     if (!x || !xo || !h || rows < 1 || E < 1 || (mu && !prev) || s.init(act) || s.one_entry(rows, pos0, b)) return fail("bamd_op_residual_rows: bad arguments");
     const size_t n = (size_t) rows * E;
     float * dx, * dy = nullptr, * dg, * dmu = nullptr, * dp = nullptr, * dxo; void * dh;
-    if (s.up_(x, n, &dx) || (y && s.up_(y, n, &dy)) || s.up_(&g, 1, &dg) || (mu && (s.up_(mu, (size_t) E, &dmu) || s.alloc((void **) &dp, (size_t) 8 * E))) || s.alloc((void **) &dxo, n * 4) || s.alloc(&dh, (size_t) rows * up(E, 32) * 4)) return 1;
+    if (s.up_(x, n, &dx) || (y && s.up_(y, n, &dy)) || s.up_(&g, 1, &dg) || (mu && (s.up_(mu, (size_t) E, &dmu) || s.alloc((void **) &dp, (size_t) 8 * E))) || s.alloc((void **) &dxo, n * 4) || s.alloc(&dh, (size_t) rows * up(E, 32) * 6)) return 1;
     if (mu) HIPC(hipMemcpy(dp, prev, (size_t) E * 4, hipMemcpyHostToDevice));
     a.x = dx; a.y = dy; a.ldy = E; a.g = dg; a.eps = eps; a.mu = dmu; a.prev = dp; a.xo = dxo; a.h = dh; a.E = E; a.ldh = up(E, 32);
     bamd_launch_residual_rows(act, b, a, s.l.s);
     HIPC(hipGetLastError());
-    if (s.rows_back(dxo, rows, E, E, xo, true) || s.rows_back(dh, rows, E, a.ldh, h, act == BAMD_ACT_F32)) return 1;
+    if (s.rows_back(dxo, rows, E, E, xo, true) || s.operand_back(dh, rows, E, a.ldh, h)) return 1;
     if (mu) HIPC(hipMemcpy(prev, dp + E, (size_t) E * 4, hipMemcpyDeviceToHost));
     return 0;
 }
 BAMD_OP bamd_op_poly_norm(int act, const float * z, const float * coef, float eps, int rows, int F, float * out) {
     OpScratch s; float * dz, * dc; void * dh;
-    if (!z || !coef || !out || rows < 1 || F < 1 || s.init(act) || s.up_(z, (size_t) rows * F, &dz) || s.up_(coef, 4, &dc) || s.alloc(&dh, (size_t) rows * up(F, 32) * 4)) return fail("bamd_op_poly_norm: bad arguments");
+    if (!z || !coef || !out || rows < 1 || F < 1 || s.init(act) || s.up_(z, (size_t) rows * F, &dz) || s.up_(coef, 4, &dc) || s.alloc(&dh, (size_t) rows * up(F, 32) * 6)) return fail("bamd_op_poly_norm: bad arguments");
     bamd_launch_poly_rows(act, rows, { dz, F, dc, eps, dh, F, up(F, 32) }, s.l.s);
     HIPC(hipGetLastError());
-    return s.rows_back(dh, rows, F, up(F, 32), out, act == BAMD_ACT_F32);
+    return s.operand_back(dh, rows, F, up(F, 32), out);
 }
 BAMD_OP bamd_op_group_norm(int act, const float * y, const float * w, int groups, float eps, int rows, int n, float * out) {
     OpScratch s; float * dy, * dw; void * dh;
-    if (!y || !w || !out || rows < 1 || n < 1 || groups < 1 || groups > BAMD_MAX_NORM_GROUPS || n % groups || s.init(act) || s.up_(y, (size_t) rows * n, &dy) || s.up_(w, (size_t) n, &dw) || s.alloc(&dh, (size_t) rows * up(n, 32) * 4)) return fail("bamd_op_group_norm: bad arguments");
+    if (!y || !w || !out || rows < 1 || n < 1 || groups < 1 || groups > BAMD_MAX_NORM_GROUPS || n % groups || s.init(act) || s.up_(y, (size_t) rows * n, &dy) || s.up_(w, (size_t) n, &dw) || s.alloc(&dh, (size_t) rows * up(n, 32) * 6)) return fail("bamd_op_group_norm: bad arguments");
     bamd_launch_group_norm_rows(act, rows, { dy, n, dw, groups, eps, dh, n, up(n, 32) }, s.l.s);
     HIPC(hipGetLastError());
-    return s.rows_back(dh, rows, n, up(n, 32), out, act == BAMD_ACT_F32);
+    return s.operand_back(dh, rows, n, up(n, 32), out);
 }
 BAMD_OP bamd_op_ssm(const float * in, int rows, int pos0, int heads, int P, int N, int groups, int taps, const float * conv, const float * conv_b, const float * dt_bias, const float * A_log, const float * D,
                     float * hist, float * state, float * out) {
@@ -1317,7 +1332,7 @@ BAMD_OP bamd_op_latent_attention(int act, const float * q, const float * c, cons
     const SafeTensor tk = bf16_tensor(uk, { heads * dim, rank }), tv = bf16_tensor(uv, { heads * vdim, rank });
     float * din, * dn, * dsink = nullptr, * po, * pm; void * cache, * qp, * o, * kc, * kk, * kv; uint16_t * ukT; bamd_qtile * tiles; int32_t * kblk;
     const int n_pg = kr / BAMD_PAGE, splits = std::min(n_pg, 3), tq = bamd_latent_prompt_rows(act, D);
-    if (s.up_(in.data(), in.size(), &din) || s.up_(c_norm, (size_t) rank, &dn) || (sink && s.up_(sink, (size_t) heads, &dsink)) || s.alloc(&o, (size_t) rows * HD * 4) || s.alloc(&qp, (size_t) hp * Rp * 4) ||
+    if (s.up_(in.data(), in.size(), &din) || s.up_(c_norm, (size_t) rank, &dn) || (sink && s.up_(sink, (size_t) heads, &dsink)) || s.alloc(&o, (size_t) rows * HD * 6) || s.alloc(&qp, (size_t) hp * Rp * 4) ||
         s.alloc((void **) &po, (size_t) hp * splits * Rp * 4) || s.alloc((void **) &pm, (size_t) hp * splits * 8) || s.alloc(&kc, (size_t) kr * Rp * 4) || s.alloc(&kk, (size_t) kr * HD * 4) || s.alloc(&kv, (size_t) kr * HD * 4)) return 1;
     // the cache in front: page i of the sequence lies at place n_pg - 1 - i
     std::vector<float> flat((size_t) n_pg * BAMD_PAGE * rank, 0.f);
@@ -1348,7 +1363,7 @@ BAMD_OP bamd_op_latent_attention(int act, const float * q, const float * c, cons
     if (rc) return fail("bamd_op_latent_attention: unsupported shape");
     HIPC(hipGetLastError());
     std::vector<float> wide((size_t) rows * HD);
-    if (s.rows_back(o, rows, HD, HD, wide.data(), act == BAMD_ACT_F32)) return 1;
+    if (s.operand_back(o, rows, HD, HD, wide.data())) return 1;
     for (int r = 0; r < rows; ++r) for (int h = 0; h < heads; ++h) memcpy(out + ((size_t) r * heads + h) * vdim, &wide[(size_t) r * HD + h * D], (size_t) vdim * 4);
     return 0;
 }
@@ -1357,11 +1372,11 @@ BAMD_OP bamd_op_layer_rows(int act, const float * x, const float * y, const floa
     if (!x || !xo || !h || (y && !g) || rows < 1 || E < 1 || s.init(act) || s.one_entry(rows, 0, b)) return fail("bamd_op_layer_rows: bad arguments");
     const size_t n = (size_t) rows * E;
     float * dx, * dy = nullptr, * dg = nullptr, * di = nullptr, * dxo; void * dh;
-    if (s.up_(x, n, &dx) || (y && (s.up_(y, n, &dy) || s.up_(g, (size_t) E, &dg))) || (gi && s.up_(gi, (size_t) E, &di)) || s.alloc((void **) &dxo, n * 4) || s.alloc(&dh, (size_t) rows * up(E, 32) * 4)) return 1;
+    if (s.up_(x, n, &dx) || (y && (s.up_(y, n, &dy) || s.up_(g, (size_t) E, &dg))) || (gi && s.up_(gi, (size_t) E, &di)) || s.alloc((void **) &dxo, n * 4) || s.alloc(&dh, (size_t) rows * up(E, 32) * 6)) return 1;
     a.norm = BAMD_NORM_LAYER; a.x = dx; a.y = dy; a.ldy = E; a.g = dg; a.gi = di; a.eps = eps; a.xo = dxo; a.h = dh; a.E = E; a.ldh = up(E, 32);
     bamd_launch_residual_rows(act, b, a, s.l.s);
     HIPC(hipGetLastError());
-    return s.rows_back(dxo, rows, E, E, xo, true) || s.rows_back(dh, rows, E, a.ldh, h, act == BAMD_ACT_F32);
+    return s.rows_back(dxo, rows, E, E, xo, true) || s.operand_back(dh, rows, E, a.ldh, h);
 }
 BAMD_OP bamd_op_clamped_glu(int act, const float * gate, const float * upv, float limit, int rows, int F, float * out) {
     OpScratch s; float * dz; void * dh;
@@ -1369,10 +1384,10 @@ BAMD_OP bamd_op_clamped_glu(int act, const float * gate, const float * upv, floa
     const int ldh = up(F, 32);
     std::vector<float> z((size_t) rows * 2 * ldh, 0.f);
     for (int r = 0; r < rows; ++r) for (int i = 0; i < F; ++i) { float * p = &z[(size_t) r * 2 * ldh + (i / 16) * 32 + i % 16]; p[0] = gate[(size_t) r * F + i]; p[16] = upv[(size_t) r * F + i]; }
-    if (s.up_(z.data(), z.size(), &dz) || s.alloc(&dh, (size_t) rows * ldh * 4)) return 1;
+    if (s.up_(z.data(), z.size(), &dz) || s.alloc(&dh, (size_t) rows * ldh * 6)) return 1;
     bamd_launch_glu_rows(act, rows, { dz, 2 * ldh, limit, dh, ldh }, s.l.s);
     HIPC(hipGetLastError());
-    return s.rows_back(dh, rows, F, ldh, out, act == BAMD_ACT_F32);
+    return s.operand_back(dh, rows, F, ldh, out);
 }
 // past_k, past_v: what the cache holds in front of the rows (keys as they are cached), [pos0][kv_heads][dim / vdim]; rel: [rel_rows][heads] or null; splits: shares of a decoded row
 BAMD_OP bamd_op_kv_attention(int act, const float * q, const float * k, const float * v, const float * gate, int rows, const float * past_k, const float * past_v, int pos0, int heads, int kv_heads, int dim, int vdim,
@@ -1402,7 +1417,7 @@ BAMD_OP bamd_op_kv_attention(int act, const float * q, const float * k, const fl
     if (rel) { a.bias_top = bias_max; const std::vector<float> e = expand_bias(std::vector<float>(rel, rel + (size_t) rel_rows * H), rel_rows, H, bias_max); if (s.up_(e.data(), e.size(), &db)) return 1; }
     const size_t cells = (size_t) bamd_kv_groups(a) * std::max(splits, 1);
     if (s.up_(in.data(), in.size(), &din) || s.act_rows(fk.data(), kr, G * D, G * D, &a.kc) || s.act_rows(fv.data(), kr, G * D, G * D, &a.vc) || s.up_(t.data(), t.size(), &tiles) || s.up_(kb.data(), kb.size(), &kblk) ||
-        s.alloc(&o, (size_t) rows * H * D * 4) || s.alloc((void **) &po, cells * 16 * D * 4) || s.alloc((void **) &pm, cells * 128)) return 1;
+        s.alloc(&o, (size_t) rows * H * D * 6) || s.alloc((void **) &po, cells * 16 * D * 4) || s.alloc((void **) &pm, cells * 128)) return 1;
     a.in = din; a.bias = db; a.out = o;
     int rc;
     if (splits) rc = bamd_launch_kv_decode(act, b, a, po, pm, splits, s.l.s);
@@ -1410,7 +1425,7 @@ BAMD_OP bamd_op_kv_attention(int act, const float * q, const float * k, const fl
     if (rc) return fail("bamd_op_kv_attention: unsupported shape");
     HIPC(hipGetLastError());
     std::vector<float> wide((size_t) rows * H * D);
-    if (s.rows_back(o, rows, H * D, H * D, wide.data(), act == BAMD_ACT_F32)) return 1;
+    if (s.operand_back(o, rows, H * D, H * D, wide.data())) return 1;
     for (int r = 0; r < rows; ++r) for (int h = 0; h < H; ++h) memcpy(out + ((size_t) r * H + h) * vdim, &wide[((size_t) r * H + h) * D], (size_t) vdim * 4);
     return 0;
 }
@@ -1447,14 +1462,14 @@ BAMD_OP bamd_op_gated_linear(int act, const float * q, const float * k, const fl
     for (bamd_segment & g : seg) g.last = (int) seg.size() - 1;
     float * din, * ds, * db, * dn, * dy; uint16_t * dw; bamd_segment * dseg; void * o;
     if (s.up_(in.data(), in.size(), &din) || s.up_(st.data(), st.size(), &ds) || s.up_(bias.data(), bias.size(), &db) || s.up_(nm.data(), nm.size(), &dn) || s.up_(w.data(), w.size(), &dw) || s.up_(seg.data(), seg.size(), &dseg) ||
-        s.alloc((void **) &dy, (size_t) rows * H * Pp * 4) || s.alloc(&o, (size_t) rows * a.ldo * 4) || s.alloc((void **) &a.alpha, (size_t) rows * ch * 4) || s.alloc((void **) &a.seg_state, seg.size() * ch * Pp * 4) ||
+        s.alloc((void **) &dy, (size_t) rows * H * Pp * 4) || s.alloc(&o, (size_t) rows * a.ldo * 6) || s.alloc((void **) &a.alpha, (size_t) rows * ch * 4) || s.alloc((void **) &a.seg_state, seg.size() * ch * Pp * 4) ||
         s.alloc((void **) &a.seg_decay, seg.size() * ch * 4)) return 1;
     a.in = din; a.a2 = dw; a.a2b = db; a.norm = dn; a.state = ds; a.y = dy; a.out = o;
     if (bamd_launch_gla(b, a, rows, dseg, (int) seg.size(), s.l.s)) return fail("bamd_op_gated_linear: unsupported shape");
     bamd_launch_gla_norm(act, a, rows, s.l.s);
     HIPC(hipGetLastError());
     std::vector<float> wy((size_t) rows * H * Pp), wo(wy.size());
-    if (s.rows_back(dy, rows, H * Pp, H * Pp, wy.data(), true) || s.rows_back(o, rows, H * Pp, a.ldo, wo.data(), act == BAMD_ACT_F32)) return 1;
+    if (s.rows_back(dy, rows, H * Pp, H * Pp, wy.data(), true) || s.operand_back(o, rows, H * Pp, a.ldo, wo.data())) return 1;
     HIPC(hipMemcpy(st.data(), ds, st.size() * 4, hipMemcpyDeviceToHost));
     for (int r = 0; r < rows; ++r) for (int h = 0; h < H; ++h) {
         memcpy(y + ((size_t) r * H + h) * vdim, &wy[((size_t) r * H + h) * Pp], (size_t) vdim * 4);
