@@ -192,9 +192,9 @@ static int tile_go(const bamd_dense & w, const void * x, int ldx, int cb, int ro
     return 0;
 }
 // The tile whose rounds over the 256 CUs end first.  Measured per block of 32 columns (ns), half of the CUs busy and all: 256 x 256 650 to 785, 256 x 224 630 to 740, 256 x 192 565 to 655, 256 x 160
-// 512 to 572, 128 x 256 432 to 490, 128 x 128 250 to 280, all of them one block per CU, so that a round started is a round paid: the widths between are there for what 256 leaves over.  2048 x 16896 x
+// 512 to 572, 128 x 256 432 to 490, 128 x 128 250 (280 in several rounds), all of them one block per CU, so that a round started is a round paid: the widths between are there for what 256 leaves over.  2048 x 16896 x
 // 4096 (66 tiles of 256 in two rows of rounds and a bit) 289 -> 258 us on 192, 2048 x 4736 x 4096 94 -> 74 on 160, 1485 x 14336 x 4096 192 -> 164 on 192, 2048 x 14336 x 4096 206 -> 198 on 224; over 23
-// sizes the choice is 0.3 % behind the best on average (7 % without them).  64 x 128 195 and 64 x 64 160 share a CU with two to four others and never take less than 250 and 160.  Where even the small tiles leave
+// sizes the choice is 0.3 % behind the best on average (7 % without them); of 53 others where they change it, it is 16 % ahead on average and 3 % behind at worst.  64 x 128 195 and 64 x 64 160 share a CU with two to four others and never take less than 250 and 160.  Where even the small tiles leave
 // CUs idle and the reader of the result can add planes, K is halved: two planes cost their bytes twice (at 4 TB/s) and blocks their
 // start and end once more (4 us).  131 x 2048 x 8192: 38 -> 22 us, 412 x 4096 x 8192: 85 -> 39; four shares were no faster (24 and 43 us).  Halves of 64 x 64 tiles that put a second block on
 // a CU take 300 where each half is longer than 2048 columns: 131 x 4096 x 14336 whole 70 us, in halves of such tiles 74, of 128 x 128 58 (8192 columns: 41, 43, 36); at K = 4096 they are
@@ -223,7 +223,7 @@ static int pick_tile(int act, const bamd_dense & w, int rows, int most, int & sh
         auto rounds = [&](int tm, int tn, long lo, long by) { const long b = tiles(tm, tn) * p; return b / 256 * (lo + by) + (b % 256 ? lo + by * std::max(0l, b % 256 - 128) / 128 : 0); };
         const long pairs = p == 2 && w.k_tiles > 128 && tiles(64, 64) * 2 > 256 ? 300 : 160;
         const bool odd = p == 1 && out != BAMD_OUT_GLU;           // gate and up tiles lie in turn: a wave holds an even number
-        const long t[8] = { rounds(256, 256, 650, 135), rounds(128, 256, 432, 58), rounds(128, 128, 250, 30), std::max(tiles(64, 128) * p * 195 / 256, 250l), std::max(tiles(64, 64) * p * 160 / 256, pairs),
+        const long t[8] = { rounds(256, 256, 650, 135), rounds(128, 256, 432, 58), tiles(128, 128) * p <= 256 ? 250 : rounds(128, 128, 250, 30), std::max(tiles(64, 128) * p * 195 / 256, 250l), std::max(tiles(64, 64) * p * 160 / 256, pairs),
                             odd ? rounds(256, 224, 630, 110) : LONG_MAX, p == 1 ? rounds(256, 192, 565, 90) : LONG_MAX, odd ? rounds(256, 160, 512, 60) : LONG_MAX };
         static const int kind[8] = { TILE_256_256, TILE_128_256, TILE_128_128, TILE_64_128, TILE_64_64, TILE_256_224, TILE_256_192, TILE_256_160 };
         const int i = (int) (std::min_element(t, t + 8) - t);
