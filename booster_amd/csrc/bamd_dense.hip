@@ -316,7 +316,7 @@ __device__ __forceinline__ void close_step(const bamd_step_out & c) {
     __threadfence_system();
     __hip_atomic_store(c.done, c.count_serial[1], __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
-template <typename T, int NT, int NW, int PRE>
+template <typename T, int NT, int NW, int PRE, bool ONE>
 __global__ void __launch_bounds__(64 * NW) dense_mv_kernel(bamd_dense w, bamd_batch_dev b, bamd_pre_args p, const bamd_bf * x, int ldx, int cb, int rows, float * out, int ldo) {
     constexpr int U = 8, P = bamd_planes<T>;
     typedef Operand<T> O;
@@ -336,12 +336,12 @@ __global__ void __launch_bounds__(64 * NW) dense_mv_kernel(bamd_dense w, bamd_ba
     request(tile, 0, cur);                                        // on their way while the operand row is built
     if constexpr (PRE != BAMD_PRE_ROWS) {
         const RowOut<O> h = { (O *) lds, 32 * P };
-        if constexpr (PRE == BAMD_PRE_RESIDUAL) residual_row<O, true>(b, p.res, 0, h, blockIdx.x == 0, red);
-        if constexpr (PRE == BAMD_PRE_POLY) poly_row<O>(p.poly, 0, h, red);
+        if constexpr (PRE == BAMD_PRE_RESIDUAL) residual_row<O, true, ONE>(b, p.res, 0, h, blockIdx.x == 0, red);
+        if constexpr (PRE == BAMD_PRE_POLY) poly_row<O, ONE>(p.poly, 0, h, red);
         if constexpr (PRE == BAMD_PRE_GROUP) group_norm_row<O>(p.grp, 0, h, red);
         if constexpr (PRE == BAMD_PRE_GLU) glu_row<O>(p.glu, 0, h, 0, p.glu.ldh);
-        if constexpr (PRE == BAMD_PRE_LAYER) layer_row<O>(p.res, p.want ? p.want[0] : 0, p.want ? p.gf : p.res.gi, h, !p.want && blockIdx.x == 0, red);
-        if constexpr (PRE == BAMD_PRE_FINAL) final_row<O>(p.res, p.want[0], p.gf, h, red);
+        if constexpr (PRE == BAMD_PRE_LAYER) layer_row<O, ONE>(p.res, p.want ? p.want[0] : 0, p.want ? p.gf : p.res.gi, h, !p.want && blockIdx.x == 0, red);
+        if constexpr (PRE == BAMD_PRE_FINAL) final_row<O, ONE>(p.res, p.want[0], p.gf, h, red);
         __syncthreads();
     }
     const int col = lane & 15, kq = (lane >> 4) * 8;
@@ -462,25 +462,21 @@ __global__ void __launch_bounds__(512) dense_few_kernel(bamd_dense w, const bamd
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        if constexpr (GLU) {
-            auto sum = [&](int c, int rl, int o4) {               // of four columns, row rl of cell c
-                bamd_v4 v = { 0, 0, 0, 0 };
+        auto sum = [&](int c, int rl, int o) {                    // of column o, row rl of cell c
+            float v = 0.f;
 #pragma unroll
-                for (int q = 0; q < NW; ++q) v = v + *(const bamd_v4 *) (red + (q * RT * NT + c) * 256 + sum_slot(o4 * 16 + rl));
-                return v;
-            };
-            for (int i = tid; i < RT / 2 * NT * 64; i += 64 * NW) {
-                const int c = i >> 6, t = c / NT * 2, rl = (i >> 2) & 15, r = (c % NT) * 16 + rl, o = (grp * RT + t) * 8 + (i & 3) * 4;      // (pairs of tiles: w.rows / 2 is a multiple of sixteen)
-                if (r >= rows || o >= w.rows / 2) continue;
-                const bamd_v4 g = sum(t * NT + c % NT, rl, i & 3), u = sum((t + 1) * NT + c % NT, rl, i & 3);
-                store4<bamd_bf>(row_out<bamd_bf>(out, r, ldo, cbo).at(o), bamd_v4{ clamped_glu(g[0], u[0], limit), clamped_glu(g[1], u[1], limit), clamped_glu(g[2], u[2], limit), clamped_glu(g[3], u[3], limit) });
+            for (int q = 0; q < NW; ++q) v += red[(q * RT * NT + c) * 256 + sum_slot((o >> 2) * 16 + rl) + (o & 3)];
+            return v;
+        };
+        if constexpr (GLU) {
+            for (int i = tid; i < RT / 2 * NT * 256; i += 64 * NW) {
+                const int c = i >> 8, t = c / NT * 2, oc = i & 15, rl = (i >> 4) & 15, r = (c % NT) * 16 + rl, o = (grp * RT + t) * 8 + oc;
+                if (r < rows && o < w.rows / 2) *row_out<bamd_bf>(out, r, ldo, cbo).at(o) = (bamd_bf) clamped_glu(sum(t * NT + c % NT, rl, oc), sum((t + 1) * NT + c % NT, rl, oc), limit);
             }
         } else for (int i = tid; i < RT * NT * 256; i += 64 * NW) {
             const int c = i >> 8, oc = i & 15, rl = (i >> 4) & 15, r = (c % NT) * 16 + rl, o = (grp * RT + c / NT) * 16 + oc;
             if (r < rows && o < w.rows) {
-                float v = 0.f;
-#pragma unroll
-                for (int q = 0; q < NW; ++q) v += red[(q * RT * NT + c) * 256 + sum_slot((oc >> 2) * 16 + rl) + (oc & 3)];
+                const float v = sum(c, rl, oc);
                 out[(size_t) r * ldo + o] = v;
                 to_host(close, (size_t) r * ldo + o, v);
             }
@@ -514,10 +510,13 @@ static int few_pick(const bamd_dense & w, const void * x, int ldx, int cb, int r
 }
 size_t bamd_dense_mv_lds(int act, int K) { return (size_t) (K + 31) / 32 * 64 * bamd_row_planes(act); }
 template <typename T, int NT, int NW, int PRE>
-static void mv_go(const bamd_dense & w, const bamd_batch_dev & b, const bamd_pre_args & p, const void * x, int ldx, int cb, int rows, float * out, int ldo, hipStream_t s, int parts = 1) {
+static void mv_go(const bamd_dense & w, const bamd_batch_dev & b, const bamd_pre_args & p, const void * x, int ldx, int cb, int n, float * out, int ldo, hipStream_t s, int parts = 1) {
     const int grid = w.row_tiles < 4096 / NW ? w.row_tiles : 4096 / NW;       // what is resident at once; blocks walk the tiles
     const size_t lds = PRE == BAMD_PRE_ROWS ? 0 : bamd_dense_mv_lds(sizeof(T) == 4 ? BAMD_ACT_F32 : BAMD_ACT_BF16, w.k_tiles * 32);
-    hipLaunchKernelGGL((dense_mv_kernel<T, NT, NW, PRE>), dim3(grid, parts), dim3(64 * NW), lds, s, w, b, p, (const bamd_bf *) x, ldx, cb, rows, out, ldo);
+    constexpr bool rows = PRE == BAMD_PRE_RESIDUAL || PRE == BAMD_PRE_LAYER || PRE == BAMD_PRE_FINAL;
+    if constexpr (rows || PRE == BAMD_PRE_POLY)
+        if ((rows ? p.res.E : p.poly.F) & 3) { hipLaunchKernelGGL((dense_mv_kernel<T, NT, NW, PRE, true>), dim3(grid, parts), dim3(64 * NW), lds, s, w, b, p, (const bamd_bf *) x, ldx, cb, n, out, ldo); return; }
+    hipLaunchKernelGGL((dense_mv_kernel<T, NT, NW, PRE, false>), dim3(grid, parts), dim3(64 * NW), lds, s, w, b, p, (const bamd_bf *) x, ldx, cb, n, out, ldo);
 }
 // sixteen waves where the tiles alone would leave the chip half empty
 template <typename T, int PRE>

@@ -98,37 +98,6 @@ template <int NV> __device__ __forceinline__ void block_sum(float (&v)[NV], floa
     for (int i = 0; i < NV; ++i) v[i] = row_sum16((lane & 15) < nw ? red[i * 16 + (lane & 15)] : 0.f);
 }
 
-// A row of n floats spread over the block four at a time, kept in registers between the passes over it: `fits` rows (n a multiple of four, at most RC pieces per
-// thread) take this path, others re-read memory.
-template <int RC> struct RowRegs {
-    bamd_v4 v[RC];
-    static __device__ __forceinline__ bool fits(int n) { return (n & 3) == 0 && n <= (int) blockDim.x * 4 * RC; }
-    static __device__ __forceinline__ int at(int c) { return ((int) threadIdx.x + c * (int) blockDim.x) * 4; }
-    __device__ __forceinline__ void load(const float * p, int n) {
-#pragma unroll
-        for (int c = 0; c < RC; ++c) v[c] = at(c) < n ? *(const bamd_v4 *) (p + at(c)) : bamd_v4{ 0, 0, 0, 0 };
-    }
-    // the sum of one or two planes
-    __device__ __forceinline__ void load(const float * p, int n, int parts, size_t plane) {
-        load(p, n);
-        if (parts <= 1) return;
-        RowRegs b; b.load(p + plane, n);
-#pragma unroll
-        for (int i = 0; i < RC; ++i) v[i] = v[i] + b.v[i];
-    }
-    __device__ __forceinline__ void clear() {
-#pragma unroll
-        for (int c = 0; c < RC; ++c) v[c] = bamd_v4{ 0, 0, 0, 0 };
-    }
-    __device__ __forceinline__ float squares() const {
-        float t = 0.f;
-#pragma unroll
-        for (int c = 0; c < RC; ++c)
-#pragma unroll
-            for (int k = 0; k < 4; ++k) t += v[c][k] * v[c][k];
-        return t;
-    }
-};
 template <typename T> __device__ __forceinline__ void store4(T * h, bamd_v4 v);
 template <> __device__ __forceinline__ void store4<float>(float * h, bamd_v4 v) { *(bamd_v4 *) h = v; }
 template <> __device__ __forceinline__ void store4<bamd_bf>(bamd_bf * h, bamd_v4 v) {
@@ -166,6 +135,7 @@ template <typename O> struct RowOut {
     O * p; int cb;
     __device__ __forceinline__ explicit operator bool() const { return p != nullptr; }
     __device__ __forceinline__ O * at(int i) const { return p + (i >> 5) * cb + (i & 31); }
+    __device__ __forceinline__ O * at(int base, int j, int lane) const { return p + ((base >> 5) + (j >> 1)) * cb + ((j & 1) * 16 + lane); }      // column base + 16 j + lane of a base that is a multiple of 32
 };
 template <typename O> __device__ __forceinline__ RowOut<O> row_out(void * h, int row, int ld, int cb) {
     constexpr int P = RowOut<O>::P;
@@ -173,20 +143,80 @@ template <typename O> __device__ __forceinline__ RowOut<O> row_out(void * h, int
 }
 template <typename O> __device__ __forceinline__ void zero_tail(RowOut<O> h, int n, int ld) { for (int i = n + threadIdx.x; i < ld; i += blockDim.x) *h.at(i) = to_operand<O>(0.f); }
 
+// A row of n floats spread over the block, kept in registers between the passes over it: four at a time, or (ONE) one at a time, a block's width apart, where n is no multiple of four and rows start
+// anywhere.  `fits`: at most RC pieces of four per thread; longer rows are read again for every sum.  Odd widths on registers, before and after, us: a token of four layers of 3098 371 -> 327 (Mafurax), 1998 208 -> 188 (Tupitar), eight sequences of 587 190 -> 165
+template <int RC, bool ONE> struct RowRegs {
+    bamd_v4 v[RC];
+    static __device__ __forceinline__ bool fits(int n) { return (ONE || (n & 3) == 0) && n <= (int) blockDim.x * 4 * RC; }
+    static __device__ __forceinline__ int at(int c, int k) { return ONE ? (int) threadIdx.x + (c * 4 + k) * (int) blockDim.x : ((int) threadIdx.x + c * (int) blockDim.x) * 4 + k; }
+    __device__ __forceinline__ void load(const float * p, int n) {
+#pragma unroll
+        for (int c = 0; c < RC; ++c) {
+            if constexpr (ONE)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) v[c][k] = at(c, k) < n ? p[at(c, k)] : 0.f;
+            else v[c] = at(c, 0) < n ? *(const bamd_v4 *) (p + at(c, 0)) : bamd_v4{ 0, 0, 0, 0 };
+        }
+    }
+    // the sum of one or two planes
+    __device__ __forceinline__ void load(const float * p, int n, int parts, size_t plane) {
+        load(p, n);
+        if (parts <= 1) return;
+        RowRegs b; b.load(p + plane, n);
+#pragma unroll
+        for (int i = 0; i < RC; ++i) v[i] = v[i] + b.v[i];
+    }
+    __device__ __forceinline__ void store(float * p, int n) const {
+#pragma unroll
+        for (int c = 0; c < RC; ++c) {
+            if constexpr (ONE) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) if (at(c, k) < n) p[at(c, k)] = v[c][k];
+            } else if (at(c, 0) < n) *(bamd_v4 *) (p + at(c, 0)) = v[c];
+        }
+    }
+    template <typename O> __device__ __forceinline__ void put(RowOut<O> h, int n, int from = 0) const {      // from: pieces in front of these
+#pragma unroll
+        for (int c = 0; c < RC; ++c) {
+            if constexpr (ONE) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) if (at(from + c, k) < n) *h.at(at(from + c, k)) = to_operand<O>(v[c][k]);
+            } else if (at(from + c, 0) < n) store4<O>(h.at(at(from + c, 0)), v[c]);
+        }
+    }
+    __device__ __forceinline__ void clear() {
+#pragma unroll
+        for (int c = 0; c < RC; ++c) v[c] = bamd_v4{ 0, 0, 0, 0 };
+    }
+    __device__ __forceinline__ float squares() const {
+        float t = 0.f;
+#pragma unroll
+        for (int c = 0; c < RC; ++c)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) t += v[c][k] * v[c][k];
+        return t;
+    }
+};
+
 __device__ __forceinline__ float parts_sum(const float * p, int parts, size_t plane) { return parts > 1 ? p[0] + p[plane] : p[0]; }
 
 // mean and variance (mean of the squared deviations) of a row in registers: per wave around its own mean, then over the waves.  red: 48 floats of LDS
-template <int RC> __device__ __forceinline__ void row_moments(const RowRegs<RC> & r, int n, float * red, float & mean, float & var) {
+template <int RC, bool ONE> __device__ __forceinline__ void row_moments(const RowRegs<RC, ONE> & r, int n, float * red, float & mean, float & var) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
     float s = 0.f, c = 0.f, q = 0.f;
 #pragma unroll
-    for (int i = 0; i < RC; ++i) if (RowRegs<RC>::at(i) < n) { s += (r.v[i][0] + r.v[i][1]) + (r.v[i][2] + r.v[i][3]); c += 4.f; }
+    for (int i = 0; i < RC; ++i) {
+        if constexpr (ONE) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) { s += r.v[i][k]; c += r.at(i, k) < n ? 1.f : 0.f; }      // (zero behind the row)
+        } else if (r.at(i, 0) < n) { s += (r.v[i][0] + r.v[i][1]) + (r.v[i][2] + r.v[i][3]); c += 4.f; }
+    }
     s = wave_sum(s); c = wave_sum(c);
     const float m = c > 0.f ? s / c : 0.f;
 #pragma unroll
-    for (int i = 0; i < RC; ++i) if (RowRegs<RC>::at(i) < n)
+    for (int i = 0; i < RC; ++i)
 #pragma unroll
-        for (int k = 0; k < 4; ++k) { const float d = r.v[i][k] - m; q += d * d; }
+        for (int k = 0; k < 4; ++k) { const float d = r.v[i][k] - m; if (r.at(i, k) < n) q += d * d; }
     q = wave_sum(q);
     __syncthreads();
     if (lane == 0) { red[wave] = m; red[16 + wave] = q; red[32 + wave] = c; }
@@ -198,39 +228,38 @@ template <int RC> __device__ __forceinline__ void row_moments(const RowRegs<RC> 
     var = row_sum16(qw + cw * d * d) / (float) n;
 }
 // residual sum with the layer norm of the sublayer's output, and the layer norm (gain gi, null: none) the next sublayer reads, of one row by the whole block
-template <typename T>
+template <typename T, bool ONE>
 __device__ __forceinline__ void layer_row(const bamd_residual_args & a, int row, const float * gi, RowOut<T> h, bool write, float * red) {
     constexpr int RC = 2;
     const int E = a.E;
     const float * x = a.x + (size_t) row * E, * y = a.y ? a.y + (size_t) row * a.ldy : nullptr;
     float * xo = a.xo + (size_t) row * E;
-    if (RowRegs<RC>::fits(E)) {
-        RowRegs<RC> xr, yr;
-        bamd_v4 g[RC], w[RC];
+    if (RowRegs<RC, ONE>::fits(E)) {
+        RowRegs<RC, ONE> xr, yr, g, w;
         xr.load(x, E);
-        if (y) yr.load(y, E, a.parts, a.plane);
-#pragma unroll
-        for (int c = 0; c < RC; ++c) {
-            const int i = RowRegs<RC>::at(c);
-            if (y) g[c] = i < E ? *(const bamd_v4 *) (a.g + i) : bamd_v4{ 0, 0, 0, 0 };
-            if (gi) w[c] = i < E ? *(const bamd_v4 *) (gi + i) : bamd_v4{ 0, 0, 0, 0 };
-        }
+        if (y) { yr.load(y, E, a.parts, a.plane); g.load(a.g, E); }
+        if (gi) w.load(gi, E);
         float mean, var;
         if (y) {
-            row_moments<RC>(yr, E, red, mean, var);
+            row_moments(yr, E, red, mean, var);
             const float r = 1.0f / sqrtf(var + a.eps);
 #pragma unroll
-            for (int c = 0; c < RC; ++c) xr.v[c] = xr.v[c] + (yr.v[c] - mean) * r * g[c];
+            for (int c = 0; c < RC; ++c) xr.v[c] = xr.v[c] + (yr.v[c] - mean) * r * g.v[c];
         }
-        if (write)
-#pragma unroll
-            for (int c = 0; c < RC; ++c) { const int i = RowRegs<RC>::at(c); if (i < E) *(bamd_v4 *) (xo + i) = xr.v[c]; }
+        if (write) xr.store(xo, E);
         if (!h) return;
-        float r = 1.f;
-        mean = 0.f;
-        if (gi) { row_moments<RC>(xr, E, red, mean, var); r = 1.0f / sqrtf(var + a.eps); }
+        if (gi) {
+            if constexpr (ONE)                                    // (what lies behind the row is not zero any more)
 #pragma unroll
-        for (int c = 0; c < RC; ++c) { const int i = RowRegs<RC>::at(c); if (i < E) store4<T>(h.at(i), gi ? (xr.v[c] - mean) * r * w[c] : xr.v[c]); }
+                for (int c = 0; c < RC; ++c)
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) if (xr.at(c, k) >= E) xr.v[c][k] = 0.f;
+            row_moments(xr, E, red, mean, var);
+            const float r = 1.0f / sqrtf(var + a.eps);
+#pragma unroll
+            for (int c = 0; c < RC; ++c) xr.v[c] = (xr.v[c] - mean) * r * w.v[c];
+        }
+        xr.put(h, E);
         zero_tail(h, E, a.ldh);
         return;
     }
@@ -278,7 +307,7 @@ __device__ __forceinline__ void glu_row(const bamd_glu_args & a, int row, RowOut
 
 // residual sum, norm of the sublayer's output and token shift of one row by the whole block.  h: LDS or global row (null: none).  write: this block also stores x' and the
 // state.  SINGLE: the step has one row
-template <typename T, bool SINGLE>
+template <typename T, bool SINGLE, bool ONE>
 __device__ __forceinline__ void residual_row(const bamd_batch_dev & b, const bamd_residual_args & a, int row, RowOut<T> h, bool write, float * red) {
     constexpr int RC = 2;
     const bool shifted = a.mu != nullptr;
@@ -293,8 +322,8 @@ __device__ __forceinline__ void residual_row(const bamd_batch_dev & b, const bam
     const float * xp = before ? x - E : nullptr, * yp = before && y ? y - a.ldy : nullptr;
     const float * sp = shifted && first && e.pos0 > 0 ? a.prev + ((size_t) e.par * b.n_seq + e.seq) * E : nullptr;
     float * so = shifted && last && write ? a.prev + ((size_t) (e.par ^ 1) * b.n_seq + e.seq) * E : nullptr;
-    if (RowRegs<RC>::fits(E)) {
-        RowRegs<RC> xr, yr, pr, qr, mu;
+    if (RowRegs<RC, ONE>::fits(E)) {
+        RowRegs<RC, ONE> xr, yr, pr, qr, mu;
         xr.load(x, E);
         if (y) yr.load(y, E, a.parts, a.plane);
         if (shifted) { mu.load(a.mu, E); if (before) { pr.load(xp, E); if (yp) qr.load(yp, E, a.parts, a.plane); } else if (sp) pr.load(sp, E); else pr.clear(); }
@@ -303,19 +332,16 @@ __device__ __forceinline__ void residual_row(const bamd_batch_dev & b, const bam
             const float g = a.g[0];
             if constexpr (SINGLE) { float v[1] = { yr.squares() }; block_sum<1>(v, red); r = g / sqrtf(v[0] / (float) E + a.eps); }
             else { float v[2] = { yr.squares(), yp ? qr.squares() : 0.f }; block_sum<2>(v, red); r = g / sqrtf(v[0] / (float) E + a.eps); rp = g / sqrtf(v[1] / (float) E + a.eps); }
-        }
 #pragma unroll
-        for (int c = 0; c < RC; ++c) {
-            const int i = RowRegs<RC>::at(c);
-            if (i >= E) continue;
-            bamd_v4 xn = xr.v[c], hn;
-            if (y) xn = xn + yr.v[c] * r;
-            hn = xn;
-            if (shifted) { bamd_v4 pv = pr.v[c]; if (yp) pv = pv + qr.v[c] * rp; hn = xn + (pv - xn) * mu.v[c]; }
-            if (write) { *(bamd_v4 *) (a.xo + (size_t) row * E + i) = xn; if (so) *(bamd_v4 *) (so + i) = xn; }
-            if (h) store4<T>(h.at(i), hn);
+            for (int c = 0; c < RC; ++c) xr.v[c] = xr.v[c] + yr.v[c] * r;
         }
-        if (h) zero_tail(h, E, a.ldh);
+        if (write) { xr.store(a.xo + (size_t) row * E, E); if (so) xr.store(so, E); }
+        if (!h) return;
+        if (shifted)
+#pragma unroll
+            for (int c = 0; c < RC; ++c) { bamd_v4 pv = pr.v[c]; if (yp) pv = pv + qr.v[c] * rp; xr.v[c] = xr.v[c] + (pv - xr.v[c]) * mu.v[c]; }
+        xr.put(h, E);
+        zero_tail(h, E, a.ldh);
         return;
     }
     float r = 0.f, rp = 0.f;
@@ -338,14 +364,14 @@ __device__ __forceinline__ void residual_row(const bamd_batch_dev & b, const bam
     }
     if (h) zero_tail(h, E, a.ldh);
 }
-template <typename T>
+template <typename T, bool ONE>
 __device__ __forceinline__ void final_row(const bamd_residual_args & a, int row, const float * gf, RowOut<T> h, float * red) {
     constexpr int RC = 4;
     const int E = a.E;
     const float * x = a.x + (size_t) row * E, * y = a.y ? a.y + (size_t) row * a.ldy : nullptr;
     float v[1] = { 0.f }, w[1] = { 0.f };
-    if (RowRegs<RC>::fits(E)) {
-        RowRegs<RC> xr, yr;
+    if (RowRegs<RC, ONE>::fits(E)) {
+        RowRegs<RC, ONE> xr, yr;
         xr.load(x, E);
         if (y) {
             yr.load(y, E, a.parts, a.plane);
@@ -359,7 +385,8 @@ __device__ __forceinline__ void final_row(const bamd_residual_args & a, int row,
         block_sum<1>(w, red);
         const float rf = gf[0] / sqrtf(w[0] / (float) E + a.eps);
 #pragma unroll
-        for (int c = 0; c < RC; ++c) { const int i = RowRegs<RC>::at(c); if (i < E) store4<T>(h.at(i), xr.v[c] * rf); }
+        for (int c = 0; c < RC; ++c) xr.v[c] = xr.v[c] * rf;
+        xr.put(h, E);
         zero_tail(h, E, a.ldh);
         return;
     }
@@ -375,34 +402,41 @@ __device__ __forceinline__ void final_row(const bamd_residual_args & a, int row,
     for (int i = threadIdx.x; i < E; i += blockDim.x) *h.at(i) = to_operand<T>((y ? x[i] + parts_sum(y + i, a.parts, a.plane) * r : x[i]) * rf);
     zero_tail(h, E, a.ldh);
 }
-template <typename T>
+template <typename T, bool ONE>
 __device__ __forceinline__ void poly_row(const bamd_poly_args & a, int row, RowOut<T> h, float * red) {
     constexpr int RC = 8;
     const float * z = a.z + (size_t) row * a.ldz;
-    const bool fits = RowRegs<RC>::fits(a.F);
-    RowRegs<RC> zr;
-    float v[3] = { 0.f, 0.f, 0.f };
-    if (fits) {
+    float v[3] = { 0.f, 0.f, 0.f }, c0, c1, c2, c3;
+    auto sums = [&](float t) { const float t2 = t * t, t3 = t2 * t; v[0] += t2; v[1] += t2 * t2; v[2] += t3 * t3; };
+    auto coefficients = [&] {
+        block_sum<3>(v, red);
+        const float n = (float) a.F;
+        c1 = a.coef[0] / sqrtf(v[0] / n + a.eps); c2 = a.coef[1] / sqrtf(v[1] / n + a.eps); c3 = a.coef[2] / sqrtf(v[2] / n + a.eps); c0 = a.coef[3];
+    };
+    auto value = [&](float t) { const float t2 = t * t; return c1 * t + c2 * t2 + c3 * (t2 * t) + c0; };
+    if (RowRegs<RC, ONE>::fits(a.F)) {
+        RowRegs<RC, ONE> zr;
         zr.load(z, a.F);
+        // pieces that no thread has are passed over: two of eight are there for 8192 values on 1024 threads
 #pragma unroll
         for (int c = 0; c < RC; ++c)
+            if (c * 4 * (int) blockDim.x < a.F)
 #pragma unroll
-            for (int k = 0; k < 4; ++k) { const float t = zr.v[c][k], t2 = t * t, t3 = t2 * t; v[0] += t2; v[1] += t2 * t2; v[2] += t3 * t3; }
-    } else for (int i = threadIdx.x; i < a.F; i += blockDim.x) { const float t = z[i], t2 = t * t, t3 = t2 * t; v[0] += t2; v[1] += t2 * t2; v[2] += t3 * t3; }
-    block_sum<3>(v, red);
-    const float n = (float) a.F;
-    const float c1 = a.coef[0] / sqrtf(v[0] / n + a.eps), c2 = a.coef[1] / sqrtf(v[1] / n + a.eps), c3 = a.coef[2] / sqrtf(v[2] / n + a.eps), c0 = a.coef[3];
-    if (fits) {
+                for (int k = 0; k < 4; ++k) sums(zr.v[c][k]);
+        coefficients();
 #pragma unroll
         for (int c = 0; c < RC; ++c) {
-            const int i = RowRegs<RC>::at(c);
-            if (i >= a.F) continue;
-            bamd_v4 o;
+            if (c * 4 * (int) blockDim.x >= a.F) break;
+            RowRegs<1, ONE> o;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) { const float t = zr.v[c][k], t2 = t * t; o[k] = c1 * t + c2 * t2 + c3 * (t2 * t) + c0; }
-            store4<T>(h.at(i), o);
+            for (int k = 0; k < 4; ++k) o.v[0][k] = value(zr.v[c][k]);
+            o.put(h, a.F, c);
         }
-    } else for (int i = threadIdx.x; i < a.F; i += blockDim.x) { const float t = z[i], t2 = t * t; *h.at(i) = to_operand<T>(c1 * t + c2 * t2 + c3 * (t2 * t) + c0); }
+    } else {
+        for (int i = threadIdx.x; i < a.F; i += blockDim.x) sums(z[i]);
+        coefficients();
+        for (int i = threadIdx.x; i < a.F; i += blockDim.x) *h.at(i) = to_operand<T>(value(z[i]));
+    }
     zero_tail(h, a.F, a.ldh);
 }
 // inv: LDS, one float per part and 16 more

@@ -201,7 +201,7 @@ __global__ void __launch_bounds__(256, sizeof(T) == 2 && ND <= 4 ? 2 : 1) kv_pro
             if (a.gated) f *= sigmoid_f(a.in[(size_t) (e.row0 + row) * a.ld + a.g_off + h]);
             const RowOut<Operand<T>> d = row_out<Operand<T>>(a.out, e.row0 + row, a.ldo, a.cb);
 #pragma unroll
-            for (int j = 0; j < NV; ++j) *d.at(a.out_off + h * D + j * 16 + lr) = to_operand<Operand<T>>(o[i][j][r] * f);
+            for (int j = 0; j < NV; ++j) *d.at(a.out_off + h * D, j, lr) = to_operand<Operand<T>>(o[i][j][r] * f);
         }
 }
 

@@ -48,24 +48,24 @@ __global__ void __launch_bounds__(256) step_close_kernel(const float * __restric
     __threadfence_system();
     __hip_atomic_store(done, count_serial[1], __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
-template <typename T> __global__ void __launch_bounds__(1024) residual_rows_kernel(bamd_batch_dev b, bamd_residual_args a) {
+template <typename T, bool ONE> __global__ void __launch_bounds__(1024) residual_rows_kernel(bamd_batch_dev b, bamd_residual_args a) {
     __shared__ float red[64];
-    residual_row<T, false>(b, a, blockIdx.x, row_out<T>(a.h, blockIdx.x, a.ldh, a.cb), true, red);
+    residual_row<T, false, ONE>(b, a, blockIdx.x, row_out<T>(a.h, blockIdx.x, a.ldh, a.cb), true, red);
 }
-template <typename T> __global__ void __launch_bounds__(1024) final_rows_kernel(bamd_residual_args a, const int32_t * want, const float * gf) {
+template <typename T, bool ONE> __global__ void __launch_bounds__(1024) final_rows_kernel(bamd_residual_args a, const int32_t * want, const float * gf) {
     __shared__ float red[64];
-    final_row<T>(a, want[blockIdx.x], gf, row_out<T>(a.h, blockIdx.x, a.ldh, a.cb), red);
+    final_row<T, ONE>(a, want[blockIdx.x], gf, row_out<T>(a.h, blockIdx.x, a.ldh, a.cb), red);
 }
-template <typename T> __global__ void __launch_bounds__(1024) layer_rows_kernel(bamd_residual_args a, const int32_t * want, const float * gi) {
+template <typename T, bool ONE> __global__ void __launch_bounds__(1024) layer_rows_kernel(bamd_residual_args a, const int32_t * want, const float * gi) {
     __shared__ float red[64];
     const int row = want ? want[blockIdx.x] : blockIdx.x;
-    layer_row<T>(a, row, gi, row_out<T>(a.h, blockIdx.x, a.ldh, a.cb), !want, red);
+    layer_row<T, ONE>(a, row, gi, row_out<T>(a.h, blockIdx.x, a.ldh, a.cb), !want, red);
 }
 // block (1024 columns, row)
 template <typename T> __global__ void __launch_bounds__(256) glu_rows_kernel(bamd_glu_args a) { glu_row<T>(a, blockIdx.y, row_out<T>(a.h, blockIdx.y, a.ldh, a.cb), blockIdx.x * 1024, min(a.ldh, (int) blockIdx.x * 1024 + 1024)); }
-template <typename T> __global__ void __launch_bounds__(1024) poly_rows_kernel(bamd_poly_args a) {
+template <typename T, bool ONE> __global__ void __launch_bounds__(1024) poly_rows_kernel(bamd_poly_args a) {
     __shared__ float red[64];
-    poly_row<T>(a, blockIdx.x, row_out<T>(a.h, blockIdx.x, a.ldh, a.cb), red);
+    poly_row<T, ONE>(a, blockIdx.x, row_out<T>(a.h, blockIdx.x, a.ldh, a.cb), red);
 }
 template <typename T> __global__ void __launch_bounds__(1024) group_norm_rows_kernel(bamd_group_norm_args a) {
     __shared__ float inv[BAMD_MAX_NORM_GROUPS + 16];
@@ -121,23 +121,20 @@ void bamd_launch_step_close(const float * logits, size_t n, float * host, bamd_s
     const size_t blocks = (n + 4095) / 4096;
     hipLaunchKernelGGL(step_close_kernel, dim3((unsigned) (blocks < 1 ? 1 : blocks > 128 ? 128 : blocks)), dim3(256), 0, s, logits, n, host, &box->done, count_serial);
 }
+// by the compile-time kinds: operands, and whether a row's length is a multiple of four
+#define ROWS_GO(KERNEL_, N_, ROWS_, BLOCK_, ...) do { \
+        if (act == BAMD_ACT_F32) { if ((N_) & 3) hipLaunchKernelGGL((KERNEL_<bamd_s3, true>), dim3(ROWS_), BLOCK_, 0, s, __VA_ARGS__); else hipLaunchKernelGGL((KERNEL_<bamd_s3, false>), dim3(ROWS_), BLOCK_, 0, s, __VA_ARGS__); } \
+        else if ((N_) & 3) hipLaunchKernelGGL((KERNEL_<bamd_bf, true>), dim3(ROWS_), BLOCK_, 0, s, __VA_ARGS__); else hipLaunchKernelGGL((KERNEL_<bamd_bf, false>), dim3(ROWS_), BLOCK_, 0, s, __VA_ARGS__); } while (0)
 void bamd_launch_residual_rows(int act, const bamd_batch_dev & b, const bamd_residual_args & a, hipStream_t s) {
-    if (a.norm == BAMD_NORM_LAYER) {
-        if (act == BAMD_ACT_F32) hipLaunchKernelGGL(layer_rows_kernel<bamd_s3>, dim3(b.rows), sum_block(a.E, b.rows), 0, s, a, nullptr, a.gi);
-        else hipLaunchKernelGGL(layer_rows_kernel<bamd_bf>, dim3(b.rows), sum_block(a.E, b.rows), 0, s, a, nullptr, a.gi);
-    } else if (act == BAMD_ACT_F32) hipLaunchKernelGGL(residual_rows_kernel<bamd_s3>, dim3(b.rows), sum_block(a.E, b.rows), 0, s, b, a);
-    else hipLaunchKernelGGL(residual_rows_kernel<bamd_bf>, dim3(b.rows), sum_block(a.E, b.rows), 0, s, b, a);
+    if (a.norm == BAMD_NORM_LAYER) ROWS_GO(layer_rows_kernel, a.E, b.rows, sum_block(a.E, b.rows), a, nullptr, a.gi);
+    else ROWS_GO(residual_rows_kernel, a.E, b.rows, sum_block(a.E, b.rows), b, a);
 }
 void bamd_launch_final_rows(int act, const bamd_residual_args & a, const int32_t * want, int n_want, const float * gf, hipStream_t s) {
-    if (a.norm == BAMD_NORM_LAYER) {
-        if (act == BAMD_ACT_F32) hipLaunchKernelGGL(layer_rows_kernel<bamd_s3>, dim3(n_want), sum_block(a.E, n_want), 0, s, a, want, gf);
-        else hipLaunchKernelGGL(layer_rows_kernel<bamd_bf>, dim3(n_want), sum_block(a.E, n_want), 0, s, a, want, gf);
-    } else if (act == BAMD_ACT_F32) hipLaunchKernelGGL(final_rows_kernel<bamd_s3>, dim3(n_want), sum_block(a.E, n_want), 0, s, a, want, gf);
-    else hipLaunchKernelGGL(final_rows_kernel<bamd_bf>, dim3(n_want), sum_block(a.E, n_want), 0, s, a, want, gf);
+    if (a.norm == BAMD_NORM_LAYER) ROWS_GO(layer_rows_kernel, a.E, n_want, sum_block(a.E, n_want), a, want, gf);
+    else ROWS_GO(final_rows_kernel, a.E, n_want, sum_block(a.E, n_want), a, want, gf);
 }
 void bamd_launch_poly_rows(int act, int rows, const bamd_poly_args & a, hipStream_t s) {
-    if (act == BAMD_ACT_F32) hipLaunchKernelGGL(poly_rows_kernel<bamd_s3>, dim3(rows), row_block(a.F), 0, s, a);
-    else hipLaunchKernelGGL(poly_rows_kernel<bamd_bf>, dim3(rows), row_block(a.F), 0, s, a);
+    ROWS_GO(poly_rows_kernel, a.F, rows, row_block(a.F), a);
 }
 void bamd_launch_glu_rows(int act, int rows, const bamd_glu_args & a, hipStream_t s) {
     if (act == BAMD_ACT_F32) hipLaunchKernelGGL(glu_rows_kernel<bamd_s3>, dim3((a.ldh + 1023) / 1024, rows), dim3(256), 0, s, a);

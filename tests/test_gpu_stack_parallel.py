@@ -9,6 +9,7 @@ from oracle import stack_oracle as so
 import stack_cases
 from stack_cases import tokens
 from test_gpu_stack import Case, DTYPES, near, rel
+from test_gpu_stack import test_poly_norm as poly_norm_case
 
 pytestmark = pytest.mark.gpu
 
@@ -50,6 +51,38 @@ def test_norms_of_rows_at_the_edge_of_a_block(bamd, dtype, E):
     near(xo, ref, "float32")
     near(h, np.stack([so.token_shift(a, b, mu) for a, b in zip(ref, np.concatenate([prev[None], ref[:-1]]))]), dtype)
     near(last, ref[-1], "float32")
+
+
+# odd lengths, which lie in registers one by one: the longest that a block holds, and one more
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("E,F", [(1023, 2047), (4095, 8191), (8191, 32767), (8193, 32769)])
+def test_norms_of_rows_of_odd_lengths(bamd, dtype, E, F):
+    test_norms_of_rows_at_the_edge_of_a_block(bamd, dtype, E)
+    poly_norm_case(bamd, dtype, F)
+
+
+# and in front of the product of one row: blocks of 512 threads hold 4095 and not 4097, whatever the kind of norm; token by token against the prompt
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("kind,E", [("tupitar", 2047), ("tupitar", 4097), ("mafurax", 4095), ("mafurax", 4097)])
+def test_odd_widths_token_by_token(bamd, tmp_path, dtype, kind, E):
+    from booster_amd import synthetic
+    mlp = {"kind": "dense", "ff": 3001}
+    if kind == "tupitar":
+        layers = [{"type": "latent_attention", "mixer": dict(heads=2, dim=32, vdim=32, kv_rank=40, scale=32 ** -0.5), "mlp": mlp},
+                  {"type": "mamba2", "mixer": dict(heads=3, vdim=32, state=32, groups=1, norm_groups=1, conv=4), "mlp": mlp}]
+        cfg = {"architecture": "Tupitar", "vocab": 80, "width": E, "max_positions": 64, "embedding": {"scale": 1.0}, "norm": {"eps": 1e-6}, "layers": layers}
+    else:
+        left = dict(heads=2, kv_heads=1, dim=32, vdim=32, scale=32 ** -0.5, softcap=30.0, bias_max=512, mask=dict(size=16, keep_first=2))
+        layers = [{"type": "parallel", "mixer": dict(left=left, left_scale=0.5, right=dict(heads=2, dim=32, vdim=32, tau=16.0), right_scale=0.8), "mlp": dict(mlp, limit=7.0)}] * 2
+        cfg = {"architecture": "Mafurax", "vocab": 80, "width": E, "logit_scale": E ** -0.5, "norm": {"eps": 1e-6}, "layers": layers}
+    synthetic.write_synthetic_stack(str(tmp_path / "m"), cfg)
+    m = bamd.Model(str(tmp_path / "m"), dtype=dtype)
+    a, b = bamd.Context(m, 64, 1), bamd.Context(m, 64, 1)
+    t = np.random.default_rng(E).integers(0, 80, 9).astype(np.int32)
+    whole = a.decode_batch([(0, t, list(range(9)))])
+    each = np.concatenate([b.decode_batch([(0, t[i:i + 1], [0])]) for i in range(9)])
+    near(each, whole, dtype, 2.0)                                  # (either is off by its own rounding)
+    a.close(); b.close(); m.close()
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
