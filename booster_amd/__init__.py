@@ -370,7 +370,8 @@ def _act(dtype):
 
 
 def op_dense(w, x, dtype, impl=0):
-    """impl 0: many-row kernel, 1: few-row kernel, 2 / 3: many-row kernel with an activation-typed / transposed result, 4 / 5: as 0 / 1 with K halved where that is faster"""
+    """impl 0: many-row kernel, 1: few-row kernel, 2 / 3: many-row kernel with an activation-typed / transposed result, 4 / 5: as 0 / 1 with K halved where that is faster,
+    6 / 7: as 0 / 1 with the operand rows by blocks"""
     w, x = np.ascontiguousarray(w, np.uint16), _f32(x)
     y = np.zeros((x.shape[0], w.shape[0]), np.float32)
     _chk(lib().bamd_op_dense(_act(dtype), _p(w), w.shape[0], w.shape[1], _p(x), x.shape[0], impl, _p(y)))

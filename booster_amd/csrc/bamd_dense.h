@@ -2,8 +2,10 @@
 // (bamd_dense.hip), row-wise mechanisms (bamd_rows.hip), the state-space recurrence (bamd_ssm.hip), latent attention (bamd_latent.hip), attention over cached keys and
 // values (bamd_kv.hip), gated linear attention (bamd_gla.hip).
 //
-// Every kernel exists for two activation types: bfloat16 (matrix operands in bfloat16, 32-bit accumulation) and float (operands in 32-bit as well; weights are
-// widened).  Residual stream, norms, scores, decays and states are 32-bit in both.
+// Every kernel exists for two activation types: bfloat16 (matrix operands in bfloat16, 32-bit accumulation) and float.  There a product's rows are kept as three bfloat16
+// parts each, which together are the number: three exact products with the bfloat16 weights, summed in 32-bit, on the fast matrix instructions; attention and recurrences
+// take 32-bit operands.  Since a part may be zero, a weight that is not finite gives NaN there where it could give infinity.  Residual stream, norms, scores, decays and
+// states are 32-bit in both.
 //
 // Packed matrix [rows][K]: 16-row tiles; per tile the K / 32 blocks follow one another, 1 KiB each: lane l of a wave holds row l % 16, columns (l / 16) * 8 .. + 8 —
 // the operand layout of v_mfma_f32_16x16x32_bf16, so that one 16-byte load per lane is one contiguous kilobyte and needs no shuffling, in prompts and in decoding.

@@ -1,7 +1,7 @@
 // bamd_dense.hip — products with dense bfloat16 matrices in the packed layout of bamd_dense.h.
 //   dense_tile_kernel: many rows (prompts).  Weight and activation tiles global -> LDS by DMA, four or eight stages deep, under the matrix instructions.
-//   dense_few_kernel: up to 64 rows (decoding several sequences, short prompts), bfloat16.  The waves of a block split K, each with a DMA ring of weights and rows.
-//   dense_mv_kernel: a row (decoding), and up to 64 in 32-bit.  The eight or sixteen waves of a block split K; every wave streams its share of a 16-row tile straight from HBM into matrix operands.  With
+//   dense_few_kernel: up to 64 rows (decoding several sequences, short prompts), bfloat16; its rows may lie by blocks.  The waves of a block split K, each with a DMA ring of weights and rows.
+//   dense_mv_kernel: a row (decoding), and up to 64 in three parts (32-bit).  The eight or sixteen waves of a block split K; every wave streams its share of a 16-row tile straight from HBM into matrix operands.  With
 //     a single row the mechanism in front of the product (residual + norm + token shift or layer norms, PolyNorm, clamped gated unit, grouped norm, last norm) runs as its prologue, its weights
 //     already requested.
 #include "bamd_dense_device.h"

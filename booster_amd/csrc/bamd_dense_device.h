@@ -19,7 +19,6 @@ template <> struct Frag<bamd_bf> {
     bamd_bf8 v;
     __device__ __forceinline__ void zero() { v = __builtin_bit_cast(bamd_bf8, bamd_u4{ 0, 0, 0, 0 }); }
     __device__ __forceinline__ void load(const bamd_bf * p) { v = *(const bamd_bf8 *) p; }
-    __device__ __forceinline__ void weight(bamd_u4 w) { v = __builtin_bit_cast(bamd_bf8, w); }
     __device__ __forceinline__ void set(int i, float f) { v[i] = (bamd_bf) f; }
     __device__ __forceinline__ void store(bamd_bf * p) const { *(bamd_bf8 *) p = v; }
 };
@@ -27,7 +26,6 @@ template <> struct Frag<float> {
     bamd_v4 a, b;
     __device__ __forceinline__ void zero() { a = bamd_v4{ 0, 0, 0, 0 }; b = a; }
     __device__ __forceinline__ void load(const float * p) { a = *(const bamd_v4 *) p; b = *(const bamd_v4 *) (p + 4); }
-    __device__ __forceinline__ void weight(bamd_u4 w) { a = bamd_v4{ bf_lo(w.x), bf_hi(w.x), bf_lo(w.y), bf_hi(w.y) }; b = bamd_v4{ bf_lo(w.z), bf_hi(w.z), bf_lo(w.w), bf_hi(w.w) }; }
     __device__ __forceinline__ void set(int i, float f) { if (i < 4) a[i] = f; else b[i - 4] = f; }
     __device__ __forceinline__ void store(float * p) const { *(bamd_v4 *) p = a; *(bamd_v4 *) (p + 4) = b; }
 };

@@ -105,9 +105,8 @@ __global__ void __launch_bounds__(64) advance_kernel(bamd_entry * ent, int32_t *
 
 static dim3 row_block(int n) { return dim3(n > 1024 ? 1024 : 256); }
 // Rows that two pieces of four floats per thread hold (RowRegs<2>): no more waves than that takes, since every sum over the row waits for all of them
-// (layer norms of six rows of 2048: 6.6 -> 5.5 us, of 2048 rows of 4096: 32 -> 23 us; up to 1024 threads before; six rows of 2052: 5.3 -> 4.8 us, 14.1 on the 256 threads that fall four floats short).  Rows that are not held (no multiple of four) are read again for every
-// sum, one float per thread and step: all the threads there are (six rows of 2050 on 256 threads: 13.9 us, on 1024: 7.8), unless there are rows for more blocks than are resident at once
-// (a prompt of 2048 tokens of width 1030 on 1024 threads: 855 us, on 256: 815)
+// (layer norms of six rows of 2048: 6.6 -> 5.5 us, of 2048 rows of 4096: 32 -> 23 us; up to 1024 threads before; six rows of 2052: 5.3 -> 4.8 us, 14.1 on the 256 threads that fall four floats short).  Other lengths are held one float
+// at a time, on 1024 threads while that many blocks are resident at once (six rows of 4098: 6.4 us, 6.8 on 576 threads; of 2050 6.2, 5.7 on 320; read again for every sum they took 9.8 and 7.4)
 int bamd_norm_threads(int n, int rows) { return (n & 3) && rows <= 512 ? (int) row_block(n).x : std::min(1024, std::max(256, ((n + 7) / 8 + 63) / 64 * 64)); }
 static dim3 sum_block(int n, int rows) { return dim3(bamd_norm_threads(n, rows)); }
 void bamd_launch_embed_rows(const bamd_batch_dev & b, const uint16_t * embd, const uint16_t * pos, float scale, int E, int V, float * x, hipStream_t s) {

@@ -249,7 +249,8 @@ int bamd_op_latent_attention(int act, const float * q, const float * c, const fl
                              const float * c_norm, const uint16_t * uk, const uint16_t * uv, const float * sink, int decode, float * out);
 /* which form of a kernel a size takes (host arithmetic, no device needed).  Threads of a block that norms one of so many rows of n floats */
 int bamd_op_norm_threads(int n, int rows);
-/* a product of the layer stacks, K in at most `most` shares: pre -1: many rows, returns the tile (0..5: 256 x 256, 128 x 256, 128 x 128, 64 x 128, 64 x 64 with four and with eight stages);
+/* a product of the layer stacks, K in at most `most` shares: pre -1: many rows, returns the tile (0..8: 256 x 256, 128 x 256, 128 x 128, 64 x 128, 64 x 64 with four and with
+ * eight stages, 256 x 224, 256 x 192, 256 x 160);
  * pre 0: up to 64 rows, 2 / 3 / 5: one row built in front (PolyNorm, grouped norm, clamped gated unit), returns -1; -2: bad arguments */
 int bamd_op_dense_route(int act, int nrows, int k, int rows, int pre, int most, int * shares);
 /* the matrix-core product of T tokens with a K-quant matrix: token tiles per block of the few-token kernel (0: 64-row blocks), the launch's dynamic LDS, and the most any such launch takes */
