@@ -801,6 +801,10 @@ static int batch_mm(bamd_context * c, bamd_mm_args a, int epi, int T, hipStream_
         return bamd_launch_matmul_batch(a, epi, m->n_cu, s);
     }
     bamd_mm_args rest = a; rest.nseg = 0;
+    // queries, keys | values of other bits, few tokens: one launch (declined otherwise)
+    const int six = a.nseg == 2 && epi == BAMD_EPI_STORE && on_mfma(0) && on_mfma(1) && a.seg[0].type != a.seg[1].type ? (a.seg[1].type == BAMD_Q6_K ? 1 : 0) : -1;
+    auto side = [&](int i) { return bamd_few_side{ a.seg[i].w, aux[i], a.seg[i].type, a.seg[i].nvalid > 0 ? a.seg[i].nvalid : a.seg[i].nrows, a.seg[i].nrows }; };
+    if (six >= 0 && !bamd_launch_matmul_few_two(side(six), a.seg[six].out, side(1 - six), a.seg[1 - six].out, a.K, c->blay[1], T, a.ldo, s)) return 0;
     for (int i = 0; i < a.nseg; ++i) {
         if (on_mfma(i)) {
             const int nv = a.seg[i].nvalid > 0 ? a.seg[i].nvalid : a.seg[i].nrows;

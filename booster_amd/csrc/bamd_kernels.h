@@ -101,6 +101,9 @@ size_t bamd_prefill_aux_bytes(int type, int nrows_pad, int K);
 void bamd_launch_prefill_aux(const void * w_stream, int type, int nrows_pad, int K, void * aux, hipStream_t s);
 int  bamd_launch_matmul_mfma2(const void * w_stream, const void * aux, int type, int nrows, int nrows_pad, int K, const void * blob16, int T, float * out, const float * res,
                               int epi, int ldo, hipStream_t s);
+// two of them in one launch, a Q6_K one and a Q4_K or Q5_K one, where both go by the few-token kernel (1: they don't)
+struct bamd_few_side { const void * stream, * aux; int type, nrows, nrows_pad; };
+int  bamd_launch_matmul_few_two(const bamd_few_side & six, float * out6, const bamd_few_side & w, float * out, int K, const void * blob16, int T, int ldo, hipStream_t s);
 // the same from token fragments, for many tokens (bamd_prefill_wide.hip).  bamd_prefill_tokfrag: the waves per block such a product takes there, 0: it takes bamd_launch_matmul_mfma2
 int  bamd_prefill_few_tiles(int type, int nrows_pad, int K, int T);       // token tiles per block of the few-token kernel, 0: another kernel
 int  bamd_prefill_tokfrag(int type, int nrows_pad, int K, int T);

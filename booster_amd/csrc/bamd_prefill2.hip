@@ -381,14 +381,14 @@ constexpr size_t few_lds(int type, int ntt) {
     return (size_t) 16 * X_FR + (size_t) XF_RING * few_records(ntt) * 1024 + (size_t) XF_WRING * (type == BAMD_Q6_K ? FewW<BAMD_Q6_K>::SLOT : type == BAMD_Q5_K ? FewW<BAMD_Q5_K>::SLOT : FewW<BAMD_Q4_K>::SLOT) + 32;
 }
 template <int TYPE, int EPI, int NTT>
-__global__ void __launch_bounds__(768) matmul_few_kernel(bamd_mma2_args a) {
+__device__ __forceinline__ void few_block(const bamd_mma2_args & a, int rtg) {
     constexpr bool Q5 = TYPE == BAMD_Q5_K, Q6 = TYPE == BAMD_Q6_K;
     constexpr uint32_t RECB = Q6 ? 1680u : Q5 ? BAMD_RECB_Q5K : BAMD_RECB_Q4K;
     constexpr int RI = few_records(NTT), RS = RI * 1024, NR = (RI + 3) / 4, NW = FewW<TYPE>::COPIES, WS = FewW<TYPE>::SLOT;
     constexpr int REC0 = 16 * X_FR, W0 = REC0 + XF_RING * RS, Z0 = W0 + XF_WRING * WS;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_id(), tt = wave, bw = wave & 3, m = lane & 15, g = lane >> 4;
-    const int nb = a.K >> 8, rtg = blockIdx.y, rb = rtg >> 2, rtl = rtg & 3, t0 = blockIdx.x * (16 * NTT);
+    const int nb = a.K >> 8, rb = rtg >> 2, rtl = rtg & 3, t0 = blockIdx.x * (16 * NTT);
     const size_t b16 = BAMD_BLOB16_BYTES(nb);
     const uint32_t lds0 = (uint32_t) (size_t) (bamd_lds_vp) smem;
     const bool active = tt < NTT && t0 + tt * 16 < a.T, builder = (wave >> 2) == 1, copier = wave >= 8;
@@ -590,6 +590,17 @@ __global__ void __launch_bounds__(768) matmul_few_kernel(bamd_mma2_args a) {
     }
 }
 
+template <int TYPE, int EPI, int NTT>
+__global__ void __launch_bounds__(768) matmul_few_kernel(bamd_mma2_args a) { few_block<TYPE, EPI, NTT>(a, blockIdx.y); }
+// Two products of the same tokens in one launch: the Q6_K one (`first` row tiles) in front, since its blocks take longer, then a Q4_K or Q5_K one.  By themselves queries and keys of the 8B shape
+// are a round of 256 blocks and a quarter, values another quarter of one:
+// a prompt of 37 tokens 5033 -> 4786 us (16 of 32 layers have such values)
+template <int TYPE, int NTT>
+__global__ void __launch_bounds__(768) matmul_few_two_kernel(bamd_mma2_args six, bamd_mma2_args a, int first) {
+    if ((int) blockIdx.y < first) few_block<BAMD_Q6_K, BAMD_EPI_STORE, NTT>(six, blockIdx.y);
+    else few_block<TYPE, BAMD_EPI_STORE, NTT>(a, blockIdx.y - first);
+}
+
 // ---- host side -----------------------------------------------------------------------------------------------------------------------------
 static inline int x_row_blocks(int nrows_pad) { return (nrows_pad + 63) / 64; }
 static unsigned long long * g_prefill_dbg = nullptr;      // -DX_TIMING builds: where the kernels of the next launches leave their phase clocks (bamd_prefill_dbg)
@@ -651,14 +662,30 @@ size_t bamd_prefill_route(int type, int nrows_pad, int K, int T, int * few_tiles
     const int waves = bamd_prefill_tokfrag(type, nrows_pad, K, T);
     return waves ? bamd_wide_lds(type, T, waves) : X3_LDS_BYTES;
 }
+static bamd_mma2_args x_args(const bamd_few_side & w, int K, const void * blob16, int T, float * out, const float * res, int ldo) {
+    const uint8_t * aux = (const uint8_t *) w.aux;
+    return { (const uint8_t *) w.stream, aux, aux + x_ph_bytes(w.type, w.nrows_pad, K), out, res, (const uint8_t *) blob16, K, T, w.nrows, w.nrows_pad, ldo, g_prefill_dbg };
+}
+int bamd_launch_matmul_few_two(const bamd_few_side & six, float * out6, const bamd_few_side & w, float * out, int K, const void * blob16, int T, int ldo, hipStream_t s) {
+    if (six.type != BAMD_Q6_K || (w.type != BAMD_Q4_K && w.type != BAMD_Q5_K) || ((six.nrows_pad | w.nrows_pad) & 7) || (K & 255) || !six.aux || !w.aux) return 1;
+    const int ntt = x_few_tiles(w.type, w.nrows_pad, K >> 8, T);
+    if (!ntt || x_few_tiles(six.type, six.nrows_pad, K >> 8, T) != ntt) return 1;
+    const bamd_mma2_args a6 = x_args(six, K, blob16, T, out6, nullptr, ldo), a = x_args(w, K, blob16, T, out, nullptr, ldo);
+    const int first = (six.nrows_pad + 15) / 16;
+    const dim3 grid((T + 16 * ntt - 1) / (16 * ntt), first + (w.nrows_pad + 15) / 16);
+#define XF2_LAUNCH(TYPE_, NTT_) hipLaunchKernelGGL((matmul_few_two_kernel<TYPE_, NTT_>), grid, dim3(768), std::max(few_lds(BAMD_Q6_K, NTT_), few_lds(TYPE_, NTT_)), s, a6, a, first)
+#define XF2_TYPE(TYPE_) do { if (ntt == 2) XF2_LAUNCH(TYPE_, 2); else if (ntt == 3) XF2_LAUNCH(TYPE_, 3); else XF2_LAUNCH(TYPE_, 4); } while (0)
+    if (w.type == BAMD_Q5_K) XF2_TYPE(BAMD_Q5_K); else XF2_TYPE(BAMD_Q4_K);
+#undef XF2_TYPE
+#undef XF2_LAUNCH
+    return 0;
+}
 int bamd_launch_matmul_mfma2(const void * w_stream, const void * aux, int type, int nrows, int nrows_pad, int K, const void * blob16, int T, float * out, const float * res,
                              int epi, int ldo, hipStream_t s) {
     if ((type != BAMD_Q4_K && type != BAMD_Q5_K && type != BAMD_Q6_K) || (nrows_pad & 7) || (K & 255) || !aux) return 1;
     if (epi != BAMD_EPI_STORE && epi != BAMD_EPI_ADD && epi != BAMD_EPI_SILU_MUL) return 1;
     if ((epi != BAMD_EPI_STORE) != (res != nullptr)) return 1;
-    bamd_mma2_args a; a.w = (const uint8_t *) w_stream; a.ph = (const uint8_t *) aux; a.ch = a.ph + x_ph_bytes(type, nrows_pad, K);
-    a.out = out; a.res = res; a.blob16 = (const uint8_t *) blob16; a.K = K; a.T = T; a.nrows = nrows; a.nrows_pad = nrows_pad; a.ldo = ldo;
-    a.dbg = g_prefill_dbg;
+    const bamd_mma2_args a = x_args({ w_stream, aux, type, nrows, nrows_pad }, K, blob16, T, out, res, ldo);
     const dim3 grid((T + 63) / 64, x_row_blocks(nrows_pad));
     const dim3 grid3(grid.x, BAMD_PREFILL_CEILING == 2 ? (grid.y + 1) / 2 : grid.y);     // (ceiling build 2: every workgroup issues the MFMAs of two; timing only)
 #define X3_LAUNCH(KERNEL, ...) do { \

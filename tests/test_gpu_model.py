@@ -390,6 +390,19 @@ def test_gate_and_up_of_a_prompt_in_one_launch(bamd, po, tmp_path, quant):
     oc.close(); ctx.close(); m.close()
 
 
+@pytest.mark.parametrize("rest,values", [("Q4_K", "Q6_K"), ("Q5_K", "Q6_K"), ("Q6_K", "Q4_K"), ("Q4_K", "Q5_K")])
+def test_queries_keys_and_values_of_a_prompt_in_one_launch(bamd, po, tmp_path, rest, values):
+    """values of other bits than queries and keys: every count of token tiles, edges of tiles and of the few-token kernel; the last pair takes two launches"""
+    p = str(tmp_path / "m.gguf")
+    gguf.write_synthetic_llama(p, E=768, H=6, Hkv=3, L=2, F=1024, V=512, seed=6, type_fn=lambda n, il: getattr(gguf, values if "attn_v" in n else rest))
+    om = po.OracleModel(gguf.GGUFReader(p)); oc = po.OracleContext(om, 96, nthreads=8)
+    m = bamd.Model(p); ctx = bamd.Context(m, 96)
+    for T in (2, 15, 16, 17, 32, 33, 48, 49, 64, 65):
+        toks = [(7919 * i + 13 * T) % 512 for i in range(T)]
+        assert np.array_equal(bits(ctx.decode(toks, 0)), bits(oc.decode(toks, 0))), T
+    oc.close(); ctx.close(); m.close()
+
+
 def test_a_long_prompt_takes_the_activation_layout_that_it_reads(tmp_path):
     """2048 tokens at once: rows of the layers' vectors, the score rows beyond 896 positions, and of the three layouts of quantised activations the one that every product of this size reads"""
     import booster_amd as bamd
