@@ -61,6 +61,26 @@ def test_norms_of_rows_of_odd_lengths(bamd, dtype, E, F):
     poly_norm_case(bamd, dtype, F)
 
 
+# a step's logits, which the head brings to the host itself or leaves to a kernel behind it (33 to 64 bfloat16 rows of more than 768 row tiles and of whole pieces of four): vocabularies around the
+# tiles and the rule, every form of the few-row product, a step after the other; against the prompt
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("V", [83, 4100, 12288, 12290, 12292])
+def test_logits_of_steps(bamd, tmp_path, dtype, V):
+    from booster_amd import synthetic
+    layer = {"type": "mamba2", "mixer": dict(heads=2, vdim=32, state=32, groups=1, norm_groups=1, conv=4), "mlp": {"kind": "dense", "ff": 96}}
+    cfg = {"architecture": "Tupitar", "vocab": V, "width": 64, "max_positions": 64, "embedding": {"scale": 1.0}, "norm": {"eps": 1e-6}, "layers": [layer]}
+    synthetic.write_synthetic_stack(str(tmp_path / "m"), cfg)
+    m = bamd.Model(str(tmp_path / "m"), dtype=dtype)
+    for n in (1, 2, 16, 17, 32, 33, 64):
+        a, b = bamd.Context(m, 64, n), bamd.Context(m, 64, n)
+        t = np.random.default_rng(n).integers(0, V, (n, 3)).astype(np.int32)
+        whole = a.decode_batch([(i, t[i], [0, 1, 2]) for i in range(n)]).reshape(n, 3, V)
+        for k in range(3):
+            near(b.decode_batch([(i, t[i, k:k + 1], [0]) for i in range(n)]), np.ascontiguousarray(whole[:, k]), dtype, 2.0)
+        a.close(); b.close()
+    m.close()
+
+
 # and in front of the product of one row: blocks of 512 threads hold 4095 and not 4097, whatever the kind of norm; token by token against the prompt
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("kind,E", [("tupitar", 2047), ("tupitar", 4097), ("mafurax", 4095), ("mafurax", 4097)])
