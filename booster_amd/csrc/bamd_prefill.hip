@@ -1,5 +1,6 @@
 // bamd_prefill.hip — batched prefill: per-token Q8_K quantisation into global blobs, the exact MFMA mat-mul kernels (Q4_K, Q6_K),
 // the integer-dot batched mat-mul (any K-quant), batched embedding, silu*up.  Helpers: bamd_device.h.
+#include <algorithm>
 #include "bamd_device.h"
 #include "bamd_mfma_common.h"
 #include <type_traits>
@@ -24,19 +25,21 @@ __global__ void __launch_bounds__(512) quantize_batch_kernel(const float * __res
                                                              uint8_t * __restrict__ blob, uint8_t * __restrict__ blob16, uint8_t * __restrict__ frag) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     // the sixteen tokens of a tile on one XCD (workgroups go round the eight): their pieces of a line of fragments meet in its L2
-    const int nb = K >> 8, u = blockIdx.x & 127, t = (blockIdx.x | 127) < gridDim.x ? (int) (blockIdx.x & ~127u) + (u & 7) * 16 + (u >> 3) : (int) blockIdx.x;
+    const int u = blockIdx.x & 127, t = (blockIdx.x | 127) < gridDim.x ? (int) (blockIdx.x & ~127u) + (u & 7) * 16 + (u >> 3) : (int) blockIdx.x;
+    // without a norm a row's super-blocks have nothing to do with one another: gridDim.y blocks share them (nb from b0 of nbt)
+    const int nbt = K >> 8, b0 = NORM == 1 ? 0 : nbt * (int) blockIdx.y / (int) gridDim.y, nb = NORM == 1 ? nbt : nbt * ((int) blockIdx.y + 1) / (int) gridDim.y - b0;
     uint32_t * q8 = (uint32_t *) smem; int * S = (int *) (q8 + nb * 64); float * yd = (float *) (S + nb * 8);
     double * red = (double *) (smem + BAMD_ACT_RED_OFF(nb));
-    const float * xt = x + (size_t) t * K;
-    if (NORM == 2) nw += (size_t) t * K;
-    ActPro<NORM> ap; ap.issue(xt, nw, K, wave_id()); ap.template finish<false, typename ActPro<NORM>::NoMid, BAMD_ACT_BATCH, true>(xt, nw, eps, K, q8, S, yd, red);
+    const float * xt = x + (size_t) t * K + b0 * 256;
+    if (NORM == 2) nw += (size_t) t * K + b0 * 256;
+    ActPro<NORM> ap; ap.issue(xt, nw, nb * 256, wave_id()); ap.template finish<false, typename ActPro<NORM>::NoMid, BAMD_ACT_BATCH, true>(xt, nw, eps, nb * 256, q8, S, yd, red);
     const size_t bb = BAMD_BLOB_BYTES(nb);
-    if (blob) {
+    if (blob) {                                                       // (an image of the whole row: gridDim.y is 1)
         const uint4 * src = (const uint4 *) smem; uint4 * dst = (uint4 *) (blob + (size_t) t * bb);
         for (int i = threadIdx.x; i < (int) (bb / 16); i += blockDim.x) dst[i] = src[i];
     }
     if (blob16) {
-        uint8_t * o = blob16 + (size_t) t * BAMD_BLOB16_BYTES(nb);
+        uint8_t * o = blob16 + (size_t) t * BAMD_BLOB16_BYTES(nbt) + (size_t) b0 * BAMD_B16_REC;
         for (int i = threadIdx.x; i < nb * 64; i += blockDim.x) {          // q8[ci*64 + e*8 + c] = sub-block c, chunk e, 4 int8
             const int ci = i >> 6, e = (i >> 3) & 7, c = i & 7;
             const uint32_t w = q8[i];
@@ -55,15 +58,15 @@ __global__ void __launch_bounds__(512) quantize_batch_kernel(const float * __res
             // (S_2l, S_2l+1) as i16 pairs (Q5_K: v_dot2_i32_i16)
             *(uint32_t *) (o + (size_t) ci * BAMD_B16_REC + 544 + l * 4) = ((uint32_t) sa & 0xffffu) | ((uint32_t) sb << 16);
         }
-        float * oyd = (float *) (o + (size_t) nb * BAMD_B16_REC);
+        float * oyd = (float *) (o + (size_t) (nbt - b0) * BAMD_B16_REC) + b0;
         for (int i = threadIdx.x; i < nb; i += blockDim.x) { oyd[i] = yd[i]; *(float *) (o + (size_t) i * BAMD_B16_REC + 560) = yd[i]; }   // d_y also inside the record (bamd_prefill2.hip: no separate copy)
     }
     if (frag) {
         // the operands of bamd_prefill_wide.hip, by tiles of 16 tokens: [tile][super-block][e][g][token] x 16 bytes (sub-blocks 2g and 2g+1 of chunk e as f16), behind them
         // d_y [tile][super-block][token] and the block sums [tile][super-block][pair l][token] as {S_2l & ~1, S_2l+1 & ~1, S_2l & 1, S_2l+1 & 1} in f16 (|S| <= 4064)
-        const size_t ntile = (gridDim.x + 15) / 16, tile = (size_t) (t >> 4) * nb;
+        const size_t ntile = (gridDim.x + 15) / 16, tile = (size_t) (t >> 4) * nbt + b0;
         const int m = t & 15;
-        uint8_t * dy = frag + ntile * nb * 8192, * mn = dy + ntile * nb * 64;
+        uint8_t * dy = frag + ntile * nbt * 8192, * mn = dy + ntile * nbt * 64;
         for (int i = threadIdx.x; i < nb * 32; i += blockDim.x) {
             const uint32_t w0 = q8[2 * i], w1 = q8[2 * i + 1];
             uint4 v;
@@ -213,9 +216,14 @@ __global__ void __launch_bounds__(256) embed_batch_kernel(const int32_t * __rest
 size_t bamd_blob_bytes(int K) { return BAMD_BLOB_BYTES(K >> 8); }
 size_t bamd_blob16_bytes(int K) { return BAMD_BLOB16_BYTES(K >> 8); }
 void bamd_launch_quantize_batch(const float * x, const float * nw, float eps, int K, int T, void * blob, void * blob16, void * frag, hipStream_t s, const float * gate) {
-    if (gate) hipLaunchKernelGGL((quantize_batch_kernel<2>),   dim3(T), dim3(512), act_lds_bytes(K), s, x, gate, eps, K, (uint8_t *) blob, (uint8_t *) blob16, (uint8_t *) frag);
-    else if (nw) hipLaunchKernelGGL((quantize_batch_kernel<1>),  dim3(T), dim3(512), act_lds_bytes(K), s, x, nw, eps, K, (uint8_t *) blob, (uint8_t *) blob16, (uint8_t *) frag);
-    else    hipLaunchKernelGGL((quantize_batch_kernel<0>), dim3(T), dim3(512), act_lds_bytes(K), s, x, nw, eps, K, (uint8_t *) blob, (uint8_t *) blob16, (uint8_t *) frag);
+    // Few tokens: as many blocks to a row as the CUs have room for, each with a super-block per wave or more.  37 tokens of a feed-forward of 14 336 were 37 blocks
+    // that went over their row twice, 8.4 us of which 4 are the launch; a prompt of 8B 4795 -> 4677 us
+    const int nb = K >> 8, parts = blob || (nw && !gate) ? 1 : std::max(1, std::min(nb / 8, 256 / T));
+    const dim3 grid(T, parts);
+    const size_t lds = act_lds_bytes((nb + parts - 1) / parts * 256);
+    if (gate) hipLaunchKernelGGL((quantize_batch_kernel<2>),   grid, dim3(512), lds, s, x, gate, eps, K, (uint8_t *) blob, (uint8_t *) blob16, (uint8_t *) frag);
+    else if (nw) hipLaunchKernelGGL((quantize_batch_kernel<1>),  grid, dim3(512), lds, s, x, nw, eps, K, (uint8_t *) blob, (uint8_t *) blob16, (uint8_t *) frag);
+    else    hipLaunchKernelGGL((quantize_batch_kernel<0>), grid, dim3(512), lds, s, x, nw, eps, K, (uint8_t *) blob, (uint8_t *) blob16, (uint8_t *) frag);
 }
 int bamd_launch_matmul_batch(const bamd_mm_args & a, int epi, int n_cu, hipStream_t s) {
     int nrg = 0;

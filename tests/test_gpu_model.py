@@ -390,6 +390,20 @@ def test_gate_and_up_of_a_prompt_in_one_launch(bamd, po, tmp_path, quant):
     oc.close(); ctx.close(); m.close()
 
 
+@pytest.mark.parametrize("quant,E,F", [("Q4_K", 768, 4352), ("Q6_K", 2048, 6144)])
+def test_quantised_rows_of_few_tokens_in_parts(bamd, po, tmp_path, quant, E, F):
+    """17 super-blocks in two parts, 24 in one to three, by the tokens (256 | 128, 129 | 85, 86): rows as they are, and of silu(gate) up"""
+    t = getattr(gguf, quant)
+    p = str(tmp_path / "m.gguf")
+    gguf.write_synthetic_llama(p, E=E, H=E // 128, Hkv=E // 256, L=1, F=F, V=512, seed=8, type_fn=lambda n, il: t)
+    om = po.OracleModel(gguf.GGUFReader(p)); oc = po.OracleContext(om, 160, nthreads=8)
+    m = bamd.Model(p); ctx = bamd.Context(m, 160)
+    for T in (2, 17, 64, 85, 86, 128, 129):
+        toks = [(7919 * i + 13 * T) % 512 for i in range(T)]
+        assert np.array_equal(bits(ctx.decode(toks, 0)), bits(oc.decode(toks, 0))), T
+    oc.close(); ctx.close(); m.close()
+
+
 @pytest.mark.parametrize("rest,values", [("Q4_K", "Q6_K"), ("Q5_K", "Q6_K"), ("Q6_K", "Q4_K"), ("Q4_K", "Q5_K")])
 def test_queries_keys_and_values_of_a_prompt_in_one_launch(bamd, po, tmp_path, rest, values):
     """values of other bits than queries and keys: every count of token tiles, edges of tiles and of the few-token kernel; the last pair takes two launches"""
