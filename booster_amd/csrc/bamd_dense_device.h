@@ -191,30 +191,45 @@ template <int RC, bool ONE> struct RowRegs {
 #pragma unroll
         for (int c = 0; c < RC; ++c)
 #pragma unroll
-            for (int k = 0; k < 4; ++k) t += v[c][k] * v[c][k];
+            for (int k = 0; k < 4; ++k) { if constexpr (ONE) t = fmaf(v[c][k], v[c][k], t); else t += v[c][k] * v[c][k]; }      // (ONE: as rows that are read again are summed)
         return t;
     }
 };
 
 __device__ __forceinline__ float parts_sum(const float * p, int parts, size_t plane) { return parts > 1 ? p[0] + p[plane] : p[0]; }
 
-// mean and variance (mean of the squared deviations) of a row in registers: per wave around its own mean, then over the waves.  red: 48 floats of LDS
+// mean and variance (mean of the squared deviations) of a row in registers: per wave around its own mean, then over the waves; ONE: around the row's mean, as rows that are read again.  red: 48
+// floats of LDS.  Which square of a sum is rounded by itself is written out: left to the compiler, it changes with the code around it, and a last place of a variance moves every result behind it
 template <int RC, bool ONE> __device__ __forceinline__ void row_moments(const RowRegs<RC, ONE> & r, int n, float * red, float & mean, float & var) {
+    if constexpr (ONE) {
+        float v[1] = { 0.f };
+#pragma unroll
+        for (int i = 0; i < RC; ++i)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[0] += r.v[i][k];        // (zero behind the row)
+        block_sum<1>(v, red);
+        mean = v[0] / (float) n; v[0] = 0.f;
+#pragma unroll
+        for (int i = 0; i < RC; ++i)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) { const float d = r.v[i][k] - mean; if (r.at(i, k) < n) v[0] = fmaf(d, d, v[0]); }
+        block_sum<1>(v, red);
+        var = v[0] / (float) n;
+        return;
+    }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
     float s = 0.f, c = 0.f, q = 0.f;
 #pragma unroll
-    for (int i = 0; i < RC; ++i) {
-        if constexpr (ONE) {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) { s += r.v[i][k]; c += r.at(i, k) < n ? 1.f : 0.f; }      // (zero behind the row)
-        } else if (r.at(i, 0) < n) { s += (r.v[i][0] + r.v[i][1]) + (r.v[i][2] + r.v[i][3]); c += 4.f; }
-    }
+    for (int i = 0; i < RC; ++i) if (r.at(i, 0) < n) { s += (r.v[i][0] + r.v[i][1]) + (r.v[i][2] + r.v[i][3]); c += 4.f; }
     s = wave_sum(s); c = wave_sum(c);
     const float m = c > 0.f ? s / c : 0.f;
 #pragma unroll
-    for (int i = 0; i < RC; ++i)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) { const float d = r.v[i][k] - m; if (r.at(i, k) < n) q += d * d; }
+    for (int i = 0; i < RC; ++i) if (r.at(i, 0) < n) {
+        const bamd_v4 d = r.v[i] - m;
+        if (i == 0) q = fmaf(d[0], d[0], d[1] * d[1]);
+        else { q = fmaf(d[0], d[0], q); q = fmaf(d[1], d[1], q); }
+        q = fmaf(d[2], d[2], q); q = fmaf(d[3], d[3], q);
+    }
     q = wave_sum(q);
     __syncthreads();
     if (lane == 0) { red[wave] = m; red[16 + wave] = q; red[32 + wave] = c; }
@@ -420,7 +435,10 @@ __device__ __forceinline__ void poly_row(const bamd_poly_args & a, int row, RowO
         for (int c = 0; c < RC; ++c)
             if (c * 4 * (int) blockDim.x < a.F)
 #pragma unroll
-                for (int k = 0; k < 4; ++k) sums(zr.v[c][k]);
+                for (int k = 0; k < 4; ++k) {
+                    const float t = zr.v[c][k], t2 = t * t, t3 = t2 * t;
+                    if constexpr (ONE) { v[0] = fmaf(t, t, v[0]); v[1] = fmaf(t2, t2, v[1]); v[2] = fmaf(t3, t3, v[2]); } else sums(t);
+                }
         coefficients();
 #pragma unroll
         for (int c = 0; c < RC; ++c) {

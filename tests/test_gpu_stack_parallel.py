@@ -35,6 +35,51 @@ def test_layer_norms_around_a_sublayer(bamd, dtype, E, rows, with_y, with_pre):
     near(h, np.stack([so.layer_norm(a, gi, 1e-4) for a in ref]) if with_pre else ref, dtype)
 
 
+# The order of a layer norm's sums is fixed, to the bit: rows of whole pieces of four, and odd ones, which lie in registers one by one and are summed as longer ones are.  Lengths whose waves hold a
+# power of two of the row, so that a wave's mean times its count is exact
+@pytest.mark.parametrize("E", [4, 8, 256, 1024, 2048, 4096, 3, 587, 1023, 2050, 4095])
+def test_sums_of_a_layer_norm_keep_their_order(bamd, E):
+    f, rows = np.float32, 64
+    t = bamd.lib().bamd_op_norm_threads(E, rows)
+    def tree(a):                                                           # neighbours first; 64 lanes of a wave, sixteen waves
+        while a.shape[-1] > 1:
+            a = a[..., 0::2] + a[..., 1::2]
+        return a[..., 0]
+    def fma(a, b, c):
+        return (a.astype(np.longdouble) * b + c).astype(f)
+    def over_waves(a):
+        return tree(np.concatenate([a, np.zeros((16 - a.shape[0]), f)]))
+    def sum_of(a):
+        return over_waves(tree(a.reshape(-1, 64)))
+    def norm(y):
+        if E % 4:                                                          # thread i: y[i], y[i + t], ...
+            v = np.zeros(-(-E // t) * t, f); v[:E] = y
+            v, there = v.reshape(-1, t), (np.arange(v.size) < E).reshape(-1, t)
+            s = q = np.zeros(t, f)
+            for a in v: s = s + a
+            mean = sum_of(s) / f(E)
+            for a, b in zip(v, there): q = np.where(b, fma(a - mean, a - mean, q), q)
+            return mean, sum_of(q) / f(E)
+        n = -(-E // (4 * t))                                               # thread i: pieces i, i + t, ...
+        v = np.zeros(n * 4 * t, f); v[:E] = y
+        v, there = v.reshape(n, t, 4), np.arange(n * t).reshape(n, t) < E // 4
+        s = q = c = np.zeros(t, f)
+        for a, b in zip(v, there): s, c = s + ((a[:, 0] + a[:, 1]) + (a[:, 2] + a[:, 3])), c + f(4) * b
+        s, c = tree(s.reshape(-1, 64)), tree(c.reshape(-1, 64))
+        m = np.where(c > 0, s / np.maximum(c, f(1)), f(0))
+        for i, (a, b) in enumerate(zip(v, there)):
+            d = a - np.repeat(m, 64)[:, None]
+            p = fma(d[:, 0], d[:, 0], d[:, 1] * d[:, 1]) if i == 0 else fma(d[:, 1], d[:, 1], fma(d[:, 0], d[:, 0], q))
+            q = np.where(b, fma(d[:, 3], d[:, 3], fma(d[:, 2], d[:, 2], p)), q)
+        mean = over_waves(m * c) / f(E)
+        return mean, over_waves(fma(c * (m - mean), m - mean, tree(q.reshape(-1, 64)))) / f(E)
+    r = np.random.default_rng(E)
+    x, y, g = (r.standard_normal(s, f) for s in ((rows, E), (rows, E), (E,)))
+    y = y + f(0.3)
+    want = np.stack([fma((b - mean) * (f(1) / np.sqrt(var + f(1e-6))), g, a) for a, b in zip(x, y) for mean, var in (norm(b),)])
+    assert np.array_equal(bamd.op_layer_rows(x, y, g, None, 1e-6, "float32")[0].view(np.uint32), want.view(np.uint32))
+
+
 # widths just inside and outside of what a block of four or five waves keeps in registers, and widths that no block keeps
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("E", [1030, 2044, 2048, 2050, 2052, 2560, 2564, 4100])
