@@ -103,9 +103,11 @@ template <> __device__ __forceinline__ void store4<bamd_bf>(bamd_bf * h, bamd_v4
     *(bf4 *) h = bf4{ (bamd_bf) v[0], (bamd_bf) v[1], (bamd_bf) v[2], (bamd_bf) v[3] };
 }
 // A 32-bit operand is the sum of three bfloat16 numbers, eight bits of its significand each (cut off, not rounded: parts of one sign, and what is left is exact), in planes 32 elements apart.  A value
-// that is not finite is its first plane alone
+// that is not finite is its first plane alone.  The number is fixed before it is taken apart: where it is a product, the compiler would fuse that into the subtraction, and the parts were those of
+// the product without its rounding, cut off at the third
 struct Split { uint32_t p[3]; };                                   // in the upper sixteen bits
 __device__ __forceinline__ Split split_f(float v) {
+    asm("" : "+v"(v));
     const uint32_t u = __float_as_uint(v);
     const bool finite = (u & 0x7f800000u) != 0x7f800000u;
     const float m = finite ? v - __uint_as_float(u & 0xffff0000u) : 0.f, l = m - __uint_as_float(__float_as_uint(m) & 0xffff0000u);

@@ -80,6 +80,24 @@ def test_sums_of_a_layer_norm_keep_their_order(bamd, E):
     assert np.array_equal(bamd.op_layer_rows(x, y, g, None, 1e-6, "float32")[0].view(np.uint32), want.view(np.uint32))
 
 
+# What a 32-bit row of operands holds is the rounded number, also where the last step in front of it is a product: factors that are known to the bit (means of zero, a root of 2^40, a single key)
+@pytest.mark.parametrize("n", [64, 96, 5000, 301])
+def test_operand_rows_hold_rounded_products(bamd, n):
+    f = np.float32
+    r = np.random.default_rng(n)
+    y, w = r.standard_normal((3, n), f), r.standard_normal(n, f)
+    same = lambda got, want: np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    assert same(bamd.op_group_norm(y, w, 1, 2.0 ** 40, "float32"), y * f(2.0 ** -20) * w)
+    x = np.zeros((3, n), f)
+    x[:, 0:n - 1:2], x[:, 1:n:2] = y[:, :n // 2], -y[:, :n // 2]                  # sums of zero, whatever their order
+    xo, h = bamd.op_layer_rows(x, None, None, w, 2.0 ** 40, "float32")
+    assert same(xo, x) and np.array_equal(h, x * f(2.0 ** -20) * w)
+    q, k, v = (r.standard_normal((1, h, 64), f) for h in (6, 2, 2))
+    for splits in (0, 1):
+        got = bamd.op_kv_attention(q, k, v, None, None, None, 0.125, 30.0, 1e-6, False, None, 0, 100, 0, "float32", out_scale=0.7, splits=splits)
+        assert same(got, np.repeat(v, 3, 1) * f(0.7)), splits
+
+
 # widths just inside and outside of what a block of four or five waves keeps in registers, and widths that no block keeps
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("E", [1030, 2044, 2048, 2050, 2052, 2560, 2564, 4100])
