@@ -102,16 +102,16 @@ template <> __device__ __forceinline__ void store4<bamd_bf>(bamd_bf * h, bamd_v4
     typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
     *(bf4 *) h = bf4{ (bamd_bf) v[0], (bamd_bf) v[1], (bamd_bf) v[2], (bamd_bf) v[3] };
 }
-// A 32-bit operand is the sum of three bfloat16 numbers, eight bits of its significand each (cut off, not rounded: parts of one sign, and what is left is exact), in planes 32 elements apart.  A value
-// that is not finite is its first plane alone.  The number is fixed before it is taken apart: where it is a product, the compiler would fuse that into the subtraction, and the parts were those of
-// the product without its rounding, cut off at the third
+// A 32-bit operand is the sum of three bfloat16 numbers in planes 32 elements apart: the largest one below it, the largest below what is left, and the rest, which has eight bits.  All three are
+// exact and have the number's sign, and none is zero (from 1e-28 on) or infinite unless the number is: so a product with a weight that is not finite is what it would be in 32 bits.  A
+// zero, an infinity, a NaN: itself three times.
+// The number is fixed before it is taken apart: where it is a product, the compiler would fuse that into the subtraction, and the parts were those of the product without its rounding, cut off at the third
 struct Split { uint32_t p[3]; };                                   // in the upper sixteen bits
 __device__ __forceinline__ Split split_f(float v) {
     asm("" : "+v"(v));
-    const uint32_t u = __float_as_uint(v);
-    const bool finite = (u & 0x7f800000u) != 0x7f800000u;
-    const float m = finite ? v - __uint_as_float(u & 0xffff0000u) : 0.f, l = m - __uint_as_float(__float_as_uint(m) & 0xffff0000u);
-    return { { finite || !(u & 0x007fffffu) ? u : u | 0x00400000u, __float_as_uint(m), __float_as_uint(l) } };
+    const uint32_t u = __float_as_uint(v), abs = u & 0x7fffffffu, same = abs > 0x7f800000u ? u | 0x00400000u : u;
+    const float m = v - __uint_as_float((u - 1) & 0xffff0000u), l = m - __uint_as_float((__float_as_uint(m) - 1) & 0xffff0000u);
+    return abs - 1 < 0x7f7fffffu ? Split{ { u - 1, __float_as_uint(m) - 1, __float_as_uint(l) } } : Split{ { same, same, same } };
 }
 struct bamd_s3 {
     uint16_t v;

@@ -1164,12 +1164,14 @@ struct OpScratch {                                 // device copies of one call
             if (f) { memcpy(&b[((size_t) r * ld + i) * 4], &v, 4); continue; }
             const size_t at = operand_at(r, i, ld, std::max(planes, 1), cb) * 2;
             if (planes < 3) { u += 0x7fff + ((u >> 16) & 1); const uint16_t o = (uint16_t) (u >> 16); memcpy(&b[at], &o, 2); continue; }
-            const bool finite = (u & 0x7f800000u) != 0x7f800000u;
-            if (!finite && (u & 0x007fffffu)) u |= 0x00400000u;
+            const uint32_t abs = u & 0x7fffffffu;                     // (split_f)
+            const bool apart = abs - 1 < 0x7f7fffffu;
+            if (abs > 0x7f800000u) u |= 0x00400000u;
             for (int k = 0; k < 3; ++k) {
-                const uint16_t o = (uint16_t) (u >> 16); memcpy(&b[at + 64 * k], &o, 2);
-                const uint32_t top = u & 0xffff0000u; float t; memcpy(&t, &top, 4);
-                v = finite ? v - t : 0.f; memcpy(&u, &v, 4);
+                const uint32_t top = apart && k < 2 ? (u - 1) & 0xffff0000u : u;
+                const uint16_t o = (uint16_t) (top >> 16); memcpy(&b[at + 64 * k], &o, 2);
+                if (!apart) continue;
+                float t; memcpy(&t, &top, 4); v -= t; memcpy(&u, &v, 4);
             }
         }
         if (alloc(d, b.size())) return 1;

@@ -110,6 +110,26 @@ def test_dense_split_values(bamd):
     assert not np.isnan(got[1]).any() and np.isnan(got[3:5]).all() and np.allclose(got[ok], want[ok], rtol=2e-6, atol=0)
 
 
+# and weights that are not finite: what 32-bit products give, whatever parts an activation has (numbers of eight bits, powers of two, zeros and infinities among them)
+@pytest.mark.parametrize("rows,impl", [(70, 0), (70, 2), (70, 6), (5, 1), (17, 1), (64, 7)])
+def test_dense_weights_that_are_not_finite(bamd, rows, impl):
+    k, r = 160, np.random.default_rng(rows)
+    x = r.standard_normal((rows, k), np.float32) + np.float32(5)
+    x[:, 10:14] = [1, -2, 0.375, 1 + 2.0 ** -16]
+    x[0, 20:24], x[1, 20], x[2, 21], x[3, 22] = [0, -0.0, 1e-28, -1e-28], np.inf, -np.inf, np.nan
+    x[4] = so.round_bf16(x[4])
+    w = r.standard_normal((60, k)).astype(np.float32)
+    for row, col, v in ((0, 10, np.inf), (1, 11, np.inf), (2, 12, -np.inf), (3, 13, np.nan), (4, 10, np.inf), (4, 12, np.inf), (5, 10, np.inf), (5, 11, np.inf), (6, 20, np.inf), (7, 21, -np.inf), (8, 22, np.inf), (9, 23, np.inf), (10, 50, -np.inf)):
+        w[row, col] = v
+    w = so.f32_to_bf16(w)
+    with np.errstate(invalid="ignore"):
+        want = sum(x[:, i:i + 1].astype(np.float64) * so.bf16_to_f32(w[:, i]).astype(np.float64) for i in range(k)).astype(np.float32)      # (one by one: a matrix product may leave zeros out)
+    got = bamd.op_dense(w, x, "float32", impl)
+    assert np.isinf(want).sum() > 8 * rows and np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want))
+    ok = np.isfinite(want)
+    assert np.allclose(got[ok], want[ok], rtol=0, atol=160 * 2.0 ** -24 * 40)
+
+
 # the widths between: 256 x 224, 256 x 192 and 256 x 160, ragged in every dimension; the gated unit on 256 x 192
 @pytest.mark.parametrize("n,rows,tile", [(14330, 1000, 6), (11000, 900, 7), (12600, 1485, 8)])
 @pytest.mark.parametrize("k", [1, 70, 300])
