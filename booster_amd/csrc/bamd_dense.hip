@@ -55,13 +55,13 @@ __device__ __forceinline__ void store_tile(const bamd_v4 (&a)[NI], int j, int mb
 }
 // 32-bit: weights are bfloat16, activations three planes of it (bamd_dense_device.h), and products of bfloat16 numbers are exact in 32 bits: three bfloat16 matrix instructions do what eight of
 // 16x16x4_f32 did, with three roundings of a sum per 32 columns for thirty-two.
-// rows [rows][ldx] of 32 k_tiles floats -> operand rows by blocks (rows that no kernel writes as operands: cached latents)
+// rows [rows][ldx] of 32 k_tiles floats -> operand rows by blocks (rows that no kernel writes as operands: cached latents, of which a pass may have more than a grid's y axis takes)
 __global__ void __launch_bounds__(256) split_rows_kernel(const float * __restrict__ x, int ldx, int k_tiles, void * planes, int cb) {
-    const int i = (blockIdx.x * 256 + threadIdx.x) * 4;
-    if (i < k_tiles * 32) store4<bamd_s3>(row_out<bamd_s3>(planes, blockIdx.y, 0, cb).at(i), *(const bamd_v4 *) (x + (size_t) blockIdx.y * ldx + i));
+    const int i = (blockIdx.y * 256 + threadIdx.x) * 4;
+    if (i < k_tiles * 32) store4<bamd_s3>(row_out<bamd_s3>(planes, blockIdx.x, 0, cb).at(i), *(const bamd_v4 *) (x + (size_t) blockIdx.x * ldx + i));
 }
 void bamd_launch_split_rows(const float * x, int ldx, int rows, int k_tiles, void * planes, int cb, hipStream_t s) {
-    hipLaunchKernelGGL(split_rows_kernel, dim3((k_tiles * 8 + 255) / 256, rows), dim3(256), 0, s, x, ldx, k_tiles, planes, cb);
+    hipLaunchKernelGGL(split_rows_kernel, dim3(rows, (k_tiles * 8 + 255) / 256), dim3(256), 0, s, x, ldx, k_tiles, planes, cb);
 }
 // TM activation rows x TN matrix rows per block of WM x WN waves.  Both operands travel global -> LDS by DMA (a kilobyte per instruction: 16 rows x 32 columns), NS stages
 // of 32 columns deep: while the matrix instructions of column block k run from registers, the fragments of k + 1 are read from LDS and the copies of the NS - 2 blocks

@@ -431,6 +431,15 @@ def test_latent_attention_in_paired_blocks(bamd, H, d, R, T, pos0):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("T,pos0", [(3, 65600), (70, 65470)])
+def test_latent_attention_behind_many_positions(bamd, dtype, T, pos0):
+    """more cached rows than a grid's y axis may have blocks"""
+    a = attention_case(2, 24, 40, 36, T, pos0, T, dtype)
+    want = plain_attention(H=2, **a)
+    near(bamd.op_latent_attention(dtype=dtype, **a).reshape(T, -1), want.reshape(T, -1), dtype, 3)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("pos0", [0, 127, 250])
 def test_one_key_stands_out(bamd, dtype, pos0):
     """one score far above hundreds of others, at the first positions, on both sides of every page border, at the query itself, and just behind it (never seen)"""
