@@ -774,20 +774,20 @@ static int prefill_part(bamd_context * c, int n, int n_past) {
 // the CUs by themselves, so are both of up to 48 tokens.  Prompts, apart and together, us: 8B 16 tokens 5107 and 4393, 37 5547 and 5050, 64 5950 and 5520, 180 11 323 and 10 215; 7B in Q6_K, 6 layers, 37 1168
 // and 1062; width 3072 x 11 008, 8 layers, 32 1156 and 1025, 256 2543 and 2329.  Of 100 such (2 to 256 tokens, widths 1024 to 4096, Q4_K and Q6_K) it is never slower by more than the runs differ (1 %)
 #define BAMD_PAIR_TOKENS 256
-static bool one_launch(bamd_context * c, const bamd_mm_args & a, int T, const void * const * aux) {
+static bool one_launch(bamd_context * c, const bamd_mm_args & a, int T, const void * const * aux) {      // (without memory for its layout of the activations: two launches, by the one there is)
     if (!g_prefill_mfma || !aux[0] || !aux[1] || a.seg[0].type != a.seg[1].type || a.seg[0].nrows != a.seg[1].nrows || T > BAMD_PAIR_TOKENS || 2 * T > c->bcap) return false;
-    return a.seg[0].type == BAMD_Q4_K || a.seg[0].type == BAMD_Q5_K || a.seg[0].type == BAMD_Q6_K;
+    return (a.seg[0].type == BAMD_Q4_K || a.seg[0].type == BAMD_Q5_K || a.seg[0].type == BAMD_Q6_K) && !ensure_layout(c, 2, T);
 }
 // one batched mat-mul: K-quant segments with a side table on the matrix-core kernels, the rest on the integer-dot kernel (identical bits either way).
-// aux[i]: side table of segment i (null: none)
-static int batch_mm(bamd_context * c, bamd_mm_args a, int epi, int T, hipStream_t s, const void * const * aux) {
+// aux[i]: side table of segment i (null: none).  both: gate and up as one_launch said
+static int batch_mm(bamd_context * c, bamd_mm_args a, int epi, int T, hipStream_t s, const void * const * aux, bool both = false) {
     bamd_model * m = c->m;
     auto on_mfma = [&](int i) { return g_prefill_mfma && aux[i] && (a.seg[i].type == BAMD_Q4_K || a.seg[i].type == BAMD_Q5_K || a.seg[i].type == BAMD_Q6_K); };
     auto mm_mfma = [&](const bamd_mv_seg & sg, const void * ax, int nv, float * out, const float * res, int e) {
         if (const int waves = bamd_prefill_tokfrag(sg.type, sg.nrows, a.K, T)) return bamd_launch_matmul_wide(sg.w, sg.type, nv, sg.nrows, a.K, c->blay[2], T, out, res, e, a.ldo, waves, s);
         return bamd_launch_matmul_mfma2(sg.w, ax, sg.type, nv, sg.nrows, a.K, c->blay[1], T, out, res, e, a.ldo, s);
     };
-    if (epi == BAMD_EPI_SILU_MUL && one_launch(c, a, T, aux))
+    if (both)
         return bamd_launch_matmul_wide(a.seg[0].w, a.seg[0].type, a.seg[0].nvalid > 0 ? a.seg[0].nvalid : a.seg[0].nrows, a.seg[0].nrows, a.K, c->blay[2], T, a.seg[0].out, nullptr, BAMD_EPI_STORE, a.ldo, 8, s,
                                        a.seg[1].w, a.seg[0].out + (size_t) T * a.ldo);
     if (epi == BAMD_EPI_SILU_MUL) {
@@ -819,8 +819,7 @@ static int batch_mm(bamd_context * c, bamd_mm_args a, int epi, int T, hipStream_
     return 0;
 }
 // the activations of a product quantised into the layouts that its segments' kernels read; a.blob is set.  1: no memory for one of them
-static int batch_quantize(bamd_context * c, const float * x, const float * nw, bamd_mm_args & a, int T, hipStream_t s, const void * const * aux, bool pair = false, const float * gate = nullptr) {
-    const bool both = pair && one_launch(c, a, T, aux);
+static int batch_quantize(bamd_context * c, const float * x, const float * nw, bamd_mm_args & a, int T, hipStream_t s, const void * const * aux, bool pair = false, bool both = false, const float * gate = nullptr) {
     bool ints = false, recs = false, frags = both;
     for (int i = 0; i < a.nseg && !both; ++i) {
         const bool mfma = g_prefill_mfma && aux[i] && (!pair || (aux[0] && aux[1] && a.seg[0].type == a.seg[1].type));
@@ -893,13 +892,14 @@ static int enqueue_prefill_batch(bamd_context * c, int T, int n_past, hipStream_
         // h = silu(Wg . a) * (Wu . a)
         memset(&a, 0, sizeof a);
         seg_of(a.seg[0], ly.wg, c->bh); seg_of(a.seg[1], ly.wu, c->bh); a.nseg = 2; a.K = E; a.T = T; a.ldo = F;
-        bool apart = false;                                       // gate and up, not their product
-        { const void * ax[3] = { ly.aux_g, ly.aux_u, nullptr }; apart = one_launch(c, a, T, ax); }
-        { const void * ax[3] = { ly.aux_g, ly.aux_u, nullptr }; if (batch_quantize(c, c->bx2, ly.ffn_norm, a, T, s, ax, true)) return 2; if (batch_mm(c, a, BAMD_EPI_SILU_MUL, T, s, ax)) return fail("batched mat-mul: unsupported shape"); }
+        const void * gu[3] = { ly.aux_g, ly.aux_u, nullptr };
+        const bool apart = one_launch(c, a, T, gu);               // gate and up, not their product
+        if (batch_quantize(c, c->bx2, ly.ffn_norm, a, T, s, gu, true, apart)) return 2;
+        if (batch_mm(c, a, BAMD_EPI_SILU_MUL, T, s, gu, apart)) return fail("batched mat-mul: unsupported shape");
         // x = x2 + Wd . h
         memset(&a, 0, sizeof a);
         seg_of(a.seg[0], ly.wd, c->bx); a.nseg = 1; a.K = F; a.T = T; a.ldo = E; a.res = c->bx2;
-        { const void * ax[3] = { ly.aux_d, nullptr, nullptr }; if (batch_quantize(c, apart ? c->bh + (size_t) T * F : c->bh, nullptr, a, T, s, ax, false, apart ? c->bh : nullptr)) return 2; if (batch_mm(c, a, BAMD_EPI_ADD, T, s, ax)) return fail("batched mat-mul: unsupported shape"); }
+        { const void * ax[3] = { ly.aux_d, nullptr, nullptr }; if (batch_quantize(c, apart ? c->bh + (size_t) T * F : c->bh, nullptr, a, T, s, ax, false, false, apart ? c->bh : nullptr)) return 2; if (batch_mm(c, a, BAMD_EPI_ADD, T, s, ax)) return fail("batched mat-mul: unsupported shape"); }
     }
     if (m->with_output) HIPC(hipMemcpyAsync(c->x, c->bx + (size_t) (T - 1) * E, (size_t) E * 4, hipMemcpyDeviceToDevice, s));
     else HIPC(hipMemcpyAsync(hidden_out, c->bx, (size_t) T * E * 4, hipMemcpyDeviceToDevice, s));
