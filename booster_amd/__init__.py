@@ -80,7 +80,7 @@ def lib():
         L.bamd_op_poly_norm.argtypes = [ci, vp, vp, cf, ci, ci, vp]
         L.bamd_op_group_norm.argtypes = [ci, vp, vp, ci, cf, ci, ci, vp]
         L.bamd_op_ssm.argtypes = [vp, ci, ci, ci, ci, ci, ci, ci, vp, vp, vp, vp, vp, vp, vp, vp]
-        L.bamd_op_dense_glu.argtypes = [ci, vp, vp, ci, ci, vp, ci, cf, vp]; L.bamd_op_dense_route.argtypes = [ci, ci, ci, ci, ci, ci, vp]
+        L.bamd_op_dense_glu.argtypes = L.bamd_op_dense_glu_blocks.argtypes = [ci, vp, vp, ci, ci, vp, ci, cf, vp]; L.bamd_op_dense_route.argtypes = [ci, ci, ci, ci, ci, ci, vp]
         L.bamd_op_latent_attention.argtypes = [ci, vp, vp, vp, ci, vp, ci, ci, ci, ci, ci, cf, cf, vp, vp, vp, vp, ci, vp]
         L.bamd_op_layer_rows.argtypes = [ci, vp, vp, vp, vp, cf, ci, ci, vp, vp]
         L.bamd_op_clamped_glu.argtypes = [ci, vp, vp, cf, ci, ci, vp]
@@ -378,11 +378,11 @@ def op_dense(w, x, dtype, impl=0):
     return y
 
 
-def op_dense_glu(gate, up, x, limit, dtype):
-    """the clamped gated unit of x . gate^T and x . up^T, written by the many-row product"""
+def op_dense_glu(gate, up, x, limit, dtype, blocks=False):
+    """the clamped gated unit of x . gate^T and x . up^T, written by the many-row product; blocks: operand rows and results by blocks"""
     gate, up, x = np.ascontiguousarray(gate, np.uint16), np.ascontiguousarray(up, np.uint16), _f32(x)
     y = np.zeros((x.shape[0], gate.shape[0]), np.float32)
-    _chk(lib().bamd_op_dense_glu(_act(dtype), _p(gate), _p(up), gate.shape[0], gate.shape[1], _p(x), x.shape[0], limit, _p(y)))
+    _chk((lib().bamd_op_dense_glu_blocks if blocks else lib().bamd_op_dense_glu)(_act(dtype), _p(gate), _p(up), gate.shape[0], gate.shape[1], _p(x), x.shape[0], limit, _p(y)))
     return y
 
 

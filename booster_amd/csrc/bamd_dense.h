@@ -97,6 +97,7 @@ bool bamd_dense_few_glu(int act, const bamd_dense & w, int rows);
 bool bamd_dense_closes(int act, const bamd_dense & w, int rows, int ldo);      // bamd_launch_dense_mv covers `close` (the tiles of prompts, which it takes for more rows, do not)
 int bamd_launch_dense_few_glu(const bamd_dense & w, const void * x, int ldx, int cb, int rows, void * h, int ldh, int cbo, float limit, hipStream_t s);
 int bamd_dense_route(int act, const bamd_dense & w, int rows, int pre, int most, int & share);      // many rows (pre < 0): the tile; few rows: -1; share: shares of K, of at most `most`
+int bamd_dense_cut(const bamd_dense & w, int rows, int out);      // many bfloat16 rows, K whole, BAMD_OUT_F32 or _GLU: row tiles of the first of two launches, 0: one
 size_t bamd_dense_mv_lds(int act, int K);         // operand bytes of a built row: must stay within BAMD_MV_LDS
 #define BAMD_MV_LDS(act) ((act) == BAMD_ACT_F32 ? 128 * 1024 : 96 * 1024)
 

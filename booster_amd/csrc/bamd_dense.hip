@@ -236,7 +236,7 @@ static int pick_tile(int act, const bamd_dense & w, int rows, int most, int & sh
 }
 // Row tiles of the matrix that whole rounds of 256 x 256 take, the rest going to a product of its own, where that is ahead by more than 3 % (of one product; halves are not cut): 0 none.  The launch
 // between them is 4 us.  2048 x 28672 x 4096 with the gated unit (3.5 rounds) 377 -> 352 us; 2048 x 16896 x 4096 249 -> 239
-static int whole_rounds(const bamd_dense & w, int rows, int out) {
+int bamd_dense_cut(const bamd_dense & w, int rows, int out) {
     const int n_mt = (rows + 255) / 256;
     if (256 % n_mt) return 0;
     const int per = 256 / n_mt * 16, full = w.row_tiles / per * per;      // row tiles of a round
@@ -253,7 +253,7 @@ static int gemm_tiles(const bamd_dense & w, const void * x, int ldx, int cb, int
     int share;
     const int tile = pick_tile(sizeof(T) == 4 ? BAMD_ACT_F32 : BAMD_ACT_BF16, w, rows, OUT == BAMD_OUT_F32 && parts ? *parts : 1, share, OUT);
     if (parts) *parts = share;
-    if constexpr (sizeof(T) == 2 && (OUT == BAMD_OUT_F32 || OUT == BAMD_OUT_GLU)) if (const int n = share == 1 ? whole_rounds(w, rows, OUT) : 0) {
+    if constexpr (sizeof(T) == 2 && (OUT == BAMD_OUT_F32 || OUT == BAMD_OUT_GLU)) if (const int n = share == 1 ? bamd_dense_cut(w, rows, OUT) : 0) {
         bamd_dense a = w, b = w;
         a.row_tiles = n; a.rows = std::min(w.rows, n * 16);
         b.row_tiles = w.row_tiles - n; b.rows = w.rows - n * 16; b.w = w.w + (size_t) n * w.k_tiles * 512;

@@ -1179,9 +1179,9 @@ struct OpScratch {                                 // device copies of one call
         return 0;
     }
     int rows_back(const void * d, int rows, int n, int ld, float * h, bool f) { return rows_from(d, rows, n, ld, h, f, 1); }
-    int operand_back(const void * d, int rows, int n, int ld, float * h) { return rows_from(d, rows, n, ld, h, false, bamd_row_planes(l.act)); }
-    int rows_from(const void * d, int rows, int n, int ld, float * h, bool f, int planes) {
-        std::vector<unsigned char> b((size_t) rows * ld * (f ? 4 : 2 * planes));
+    int operand_back(const void * d, int rows, int n, int ld, float * h, int cb = 0) { return rows_from(d, rows, n, ld, h, false, bamd_row_planes(l.act), cb); }
+    int rows_from(const void * d, int rows, int n, int ld, float * h, bool f, int planes, int cb = 0) {
+        std::vector<unsigned char> b(cb ? (size_t) cb * (ld / 32) * 2 : (size_t) rows * ld * (f ? 4 : 2 * planes));
         HIPC(hipStreamSynchronize(l.s));
         HIPC(hipMemcpy(b.data(), d, b.size(), hipMemcpyDeviceToHost));
         for (int r = 0; r < rows; ++r) for (int i = 0; i < n; ++i) {
@@ -1189,7 +1189,7 @@ struct OpScratch {                                 // device copies of one call
             if (f) { memcpy(&o, &b[((size_t) r * ld + i) * 4], 4); continue; }
             o = 0.f;
             for (int k = planes - 1; k >= 0; --k) {               // (the smallest first: each sum is exact)
-                uint16_t v; memcpy(&v, &b[operand_at(r, i, ld, planes, 0) * 2 + 64 * k], 2);
+                uint16_t v; memcpy(&v, &b[operand_at(r, i, ld, planes, cb) * 2 + 64 * k], 2);
                 const uint32_t u = (uint32_t) v << 16; float t; memcpy(&t, &u, 4);
                 o = k == planes - 1 ? t : t + o;
             }
@@ -1228,6 +1228,12 @@ BAMD_OP bamd_op_dense_route(int act, int nrows, int k, int rows, int pre, int mo
     d.rows = nrows; d.K = up(k, 32); d.row_tiles = up(nrows, 16) / 16; d.k_tiles = d.K / 32;
     return bamd_dense_route(act, d, rows, pre, most, *shares);
 }
+BAMD_OP bamd_op_dense_cut(int nrows, int k, int rows, int gated) {
+    if (nrows < 1 || k < 1 || rows < 1) { fail("bamd_op_dense_cut: bad arguments"); return -1; }
+    bamd_dense d;
+    d.rows = nrows; d.K = up(k, 32); d.row_tiles = up(nrows, 16) / 16; d.k_tiles = d.K / 32;
+    return bamd_dense_cut(d, rows, gated ? BAMD_OUT_GLU : BAMD_OUT_F32) * 16;
+}
 BAMD_OP bamd_op_dense(int act, const uint16_t * w, int nrows, int k, const float * x, int rows, int impl, float * y) {
     OpScratch s; bamd_dense d; void * dx; float * dy = nullptr;
     const int planes = bamd_row_planes(act), cb = impl == 6 || impl == 7 ? planes * bamd_row_blocks(rows) : 0;                   // 6, 7: as impl 0 and 1, the operand rows by blocks
@@ -1258,20 +1264,22 @@ BAMD_OP bamd_op_dense(int act, const uint16_t * w, int nrows, int k, const float
     for (int n = 0; n < nrows; ++n) for (int r = 0; r < rows; ++r) y[(size_t) r * nrows + n] = tr[(size_t) n * rows + r];
     return 0;
 }
-BAMD_OP bamd_op_dense_glu(int act, const uint16_t * gate, const uint16_t * upw, int F, int k, const float * x, int rows, float limit, float * y) {
+static int op_dense_glu(int act, const uint16_t * gate, const uint16_t * upw, int F, int k, const float * x, int rows, float limit, bool blocks, float * y) {
     OpScratch s; bamd_dense d; void * dx; float * dy = nullptr;
     if (!gate || !upw || !x || !y || F < 1 || k < 1 || rows < 1 || s.init(act)) return fail("bamd_op_dense_glu: bad arguments");
-    const int ldo = up(F, 32);
+    const int ldo = up(F, 32), cb = blocks ? bamd_row_planes(act) * bamd_row_blocks(rows) : 0;
     const SafeTensor tg = bf16_tensor(gate, { F, k }), tu = bf16_tensor(upw, { F, k });
     std::vector<int32_t> at = Loader::steps(F, k); at.resize((size_t) ldo, -1);
-    if (s.l.alloc(d, 2 * ldo, k) || s.operand_rows(x, rows, k, d.K, &dx) || s.alloc((void **) &dy, (size_t) rows * ldo * 6)) return 1;
+    if (s.l.alloc(d, 2 * ldo, k) || s.operand_rows(x, rows, k, d.K, &dx, cb) || s.alloc((void **) &dy, (size_t) up(rows, 16) * ldo * 6)) return 1;
     uint16_t * w = const_cast<uint16_t *>(d.w);
     if (s.l.pack(&tg, at, Loader::steps(k, 1), w, 2) || s.l.pack(&tu, at, Loader::steps(k, 1), w + (size_t) 16 * d.K, 2)) return 1;
     const bool few = bamd_dense_few_glu(act, d, rows); const int ldx = d.K * bamd_row_planes(act);
-    if (few ? bamd_launch_dense_few_glu(d, dx, ldx, 0, rows, dy, ldo, 0, limit, s.l.s) : bamd_launch_dense_gemm(act, d, dx, ldx, 0, rows, dy, ldo, BAMD_OUT_GLU, s.l.s, limit)) return fail("bamd_op_dense_glu: unsupported shape");
+    if (few ? bamd_launch_dense_few_glu(d, dx, ldx, cb, rows, dy, ldo, cb, limit, s.l.s) : bamd_launch_dense_gemm(act, d, dx, ldx, cb, rows, dy, ldo, BAMD_OUT_GLU, s.l.s, limit, nullptr, cb)) return fail("bamd_op_dense_glu: unsupported shape");
     HIPC(hipGetLastError());
-    return s.operand_back(dy, rows, F, ldo, y);
+    return s.operand_back(dy, rows, F, ldo, y, cb);
 }
+BAMD_OP bamd_op_dense_glu(int act, const uint16_t * gate, const uint16_t * upw, int F, int k, const float * x, int rows, float limit, float * y) { return op_dense_glu(act, gate, upw, F, k, x, rows, limit, false, y); }
+BAMD_OP bamd_op_dense_glu_blocks(int act, const uint16_t * gate, const uint16_t * upw, int F, int k, const float * x, int rows, float limit, float * y) { return op_dense_glu(act, gate, upw, F, k, x, rows, limit, true, y); }
 BAMD_OP bamd_op_residual_rows(int act, const float * x, const float * y, float g, float eps, const float * mu, float * prev, int pos0, int rows, int E, float * xo, float * h) {
     OpScratch s; bamd_batch_dev b; bamd_residual_args a; memset((void *) &a, 0, sizeof a);
     if (!x || !xo || !h || rows < 1 || E < 1 || (mu && !prev) || s.init(act) || s.one_entry(rows, pos0, b)) return fail("bamd_op_residual_rows: bad arguments");

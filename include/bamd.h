@@ -237,6 +237,7 @@ int bamd_op_attention(const float * q, const float * k, const float * v, uint16_
 int bamd_op_dense(int act, const uint16_t * w, int nrows, int k, const float * x, int rows, int impl, float * y);
 /* y[rows][F] = the clamped gated unit of x . gate^T and x . up^T (bfloat16 [F][k]), by the many-row kernel that writes it itself, in the activation type */
 int bamd_op_dense_glu(int act, const uint16_t * gate, const uint16_t * up, int F, int k, const float * x, int rows, float limit, float * y);
+int bamd_op_dense_glu_blocks(int act, const uint16_t * gate, const uint16_t * up, int F, int k, const float * x, int rows, float limit, float * y);      /* the same, operands and results by blocks of 32 columns */
 /* xo = x + rms_norm(y) * g (y NULL: x), h = xo + (xo of the row in front - xo) * mu (mu NULL: xo); prev [E]: the row in front of the first (used when pos0 > 0), replaced by the last */
 int bamd_op_residual_rows(int act, const float * x, const float * y, float g, float eps, const float * mu, float * prev, int pos0, int rows, int E, float * xo, float * h);
 int bamd_op_poly_norm(int act, const float * z, const float * coef, float eps, int rows, int F, float * out);
@@ -253,6 +254,8 @@ int bamd_op_norm_threads(int n, int rows);
  * eight stages, 256 x 224, 256 x 192, 256 x 160);
  * pre 0: up to 64 rows, 2 / 3 / 5: one row built in front (PolyNorm, grouped norm, clamped gated unit), returns -1; -2: bad arguments */
 int bamd_op_dense_route(int act, int nrows, int k, int rows, int pre, int most, int * shares);
+/* many bfloat16 rows, K whole (gated: gate and up rows in turn): outputs of the first of two launches, 0: one launch; -1: bad arguments */
+int bamd_op_dense_cut(int nrows, int k, int rows, int gated);
 /* the matrix-core product of T tokens with a K-quant matrix: token tiles per block of the few-token kernel (0: 64-row blocks), the launch's dynamic LDS, and the most any such launch takes */
 int bamd_op_prefill_route(int type, int nrows, int k, int T, int * few_tiles, int * lds, int * most);
 /* RoPE (cos,sin) table row as built on the host for position pos (ggml_rope_cache_init, ggml.c:14017) */

@@ -156,6 +156,7 @@ def test_dense_whole_rounds(bamd, n, rows, k, cut):
     r = np.random.default_rng(n + k + rows)
     w = so.f32_to_bf16(r.standard_normal((n, k), np.float32))
     x = so.round_bf16(r.standard_normal((rows, k), np.float32))
+    assert bamd.lib().bamd_op_dense_cut(n, k, rows, 0) == cut and not bamd.lib().bamd_op_dense_cut(cut or n, k, rows, 0)
     parts = [w[:cut], w[cut:]] if cut else [w[:8192], w[8192:]]
     want = np.concatenate([bamd.op_dense(p, x, "bfloat16", 0) for p in parts], 1)
     for impl in (0, 6):
@@ -163,12 +164,14 @@ def test_dense_whole_rounds(bamd, n, rows, k, cut):
 
 
 def test_dense_gated_whole_rounds(bamd):
-    F, rows, k, cut = 14330, 2045, 1500, 12288
+    F, rows, k, cut = 14330, 2045, 2050, 12288                          # (rows of 1500 columns are not worth a second launch)
     r = np.random.default_rng(F + k + rows)
     gate, up = (so.f32_to_bf16(r.standard_normal((F, k), np.float32) * np.float32(0.03)) for _ in range(2))
     x = so.round_bf16(r.standard_normal((rows, k), np.float32))
+    assert bamd.lib().bamd_op_dense_cut(2 * ((F + 31) // 32 * 32), k, rows, 1) == 2 * cut
     want = np.concatenate([bamd.op_dense_glu(gate[i:j], up[i:j], x, 7.0, "bfloat16") for i, j in ((0, cut), (cut, F))], 1)
-    assert np.array_equal(bamd.op_dense_glu(gate, up, x, 7.0, "bfloat16").view(np.uint32), want.view(np.uint32))
+    for blocks in (False, True):
+        assert np.array_equal(bamd.op_dense_glu(gate, up, x, 7.0, "bfloat16", blocks).view(np.uint32), want.view(np.uint32)), blocks
 
 
 # operand rows by blocks of 32 columns, as the passes have them, against the same rows by rows: every tile of many rows and every group of few, ragged
@@ -180,6 +183,29 @@ def test_dense_rows_by_blocks(bamd, n, rows, impl, k):
     w = so.f32_to_bf16(r.standard_normal((n, k), np.float32))
     x = so.round_bf16(r.standard_normal((rows, k), np.float32))
     assert np.array_equal(bamd.op_dense(w, x, "bfloat16", impl + 6).view(np.uint32), bamd.op_dense(w, x, "bfloat16", impl).view(np.uint32))
+
+
+# and in 32-bit, three planes to a block: 128 x 256, 128 x 128, 64 x 128 and 64 x 64, and groups of 16, 32 and 64 rows
+@pytest.mark.parametrize("n,rows,impl", [(8180, 1000, 0), (8170, 500, 0), (8170, 250, 0), (2040, 131, 0), (2030, 1, 1), (4620, 2, 1), (2030, 16, 1), (4100, 17, 1), (4100, 32, 1), (4620, 33, 1), (520, 64, 1)])
+@pytest.mark.parametrize("k", [1, 300, 2050])
+def test_dense_rows_by_blocks_in_32_bit(bamd, n, rows, impl, k):
+    if impl == 0:
+        assert bamd.op_dense_route(n, k, rows, "float32", most=1)[0] == {1000: 1, 500: 2, 250: 3, 131: 4}[rows]
+    r = np.random.default_rng(n + k + rows)
+    w = so.f32_to_bf16(r.standard_normal((n, k), np.float32))
+    x = r.standard_normal((rows, k), np.float32)
+    assert np.array_equal(bamd.op_dense(w, x, "float32", impl + 6).view(np.uint32), bamd.op_dense(w, x, "float32", impl).view(np.uint32))
+
+
+# the gated unit from operands by blocks to results by blocks, against rows: few rows, the tiles of many, and 32-bit results of three planes
+@pytest.mark.parametrize("dtype,F,rows", [("bfloat16", 1001, 3), ("bfloat16", 1001, 17), ("bfloat16", 8210, 32), ("bfloat16", 7000, 33), ("bfloat16", 4085, 1000), ("bfloat16", 5490, 900), ("bfloat16", 1001, 131),
+                                          ("float32", 4085, 1000), ("float32", 4085, 500), ("float32", 1001, 131)])
+@pytest.mark.parametrize("k", [1, 300])
+def test_dense_gated_by_blocks(bamd, dtype, F, rows, k):
+    r = np.random.default_rng(F + k + rows)
+    gate, up = (so.f32_to_bf16(r.standard_normal((F, k), np.float32)) for _ in range(2))
+    x = r.standard_normal((rows, k), np.float32)
+    assert np.array_equal(bamd.op_dense_glu(gate, up, x, 7.0, dtype, True).view(np.uint32), bamd.op_dense_glu(gate, up, x, 7.0, dtype).view(np.uint32))
 
 
 # the same tiles where they write the clamped gated unit of their gate and up tiles in turn: widths that end inside a pair of tiles, on its edge and inside a group of four

@@ -12,7 +12,7 @@ def L():
 
 def test_norm_blocks_hold_the_rows_they_can(L):
     """a thread holds two pieces of four floats: every row of up to 8192 floats that is a multiple of four fits its block, and no block has a wave more than that takes (or fewer than four); rows
-    that are no multiple of four, which are read again for every sum, get all the threads unless there are blocks enough without"""
+    that are no multiple of four, which lie in registers one by one, get all the threads unless there are blocks enough without"""
     for n in range(4, 8196, 4):
         t = L.bamd_op_norm_threads(n, 1)
         assert t == L.bamd_op_norm_threads(n, 4096)
