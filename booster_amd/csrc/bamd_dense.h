@@ -15,8 +15,8 @@
 
 enum { BAMD_ACT_BF16 = 0, BAMD_ACT_F32 = 1 };
 
-// Operand rows of products: bfloat16, or (32-bit) three bfloat16 planes of 32 columns in turn, whose sum is the number: six bytes per value, and every distance below is three times as long.  By rows: row r at r * ld.  By blocks (cb > 0: elements from one block of 32 columns to the next): column block, row, column — row r of block k at k * cb + r * 32.  A block's rows lie behind one another, so that a copy of sixteen of them is one kilobyte; by rows it is sixteen pieces of 64 bytes whose distance, the length of a row, is a
-// multiple of 256 bytes in most models: all sixteen come out of one channel of an L2, while every CU asks for the same ones
+// Operand rows of products: bfloat16, or (32-bit) three bfloat16 planes of 32 columns in turn, whose sum is the number: six bytes per value, and every distance below is three times as long.  By rows: row r at r * ld.  By blocks (cb > 0: elements from one block of 32 columns to the next): column block, row, column — row r of block k at k * cb + r * 32.  A block's rows lie behind one another, so that a copy of sixteen of them is one kilobyte (32-bit, where a row's three planes of the block follow one another: sixteen pieces of 64 bytes, 192 apart); by rows it is sixteen
+// pieces of 64 bytes whose distance, the length of a row, is a multiple of 256 bytes in most models: all sixteen come out of one channel of an L2, while every CU asks for the same ones
 inline int bamd_row_planes(int act) { return act == BAMD_ACT_F32 ? 3 : 1; }
 inline int bamd_row_blocks(int rows) { const int by = rows > 16 ? 16 : 2; return 32 * ((rows + by - 1) / by * by); }      // groups of sixteen rows start on a kilobyte, fewer on a cache line
 struct bamd_dense { const uint16_t * w = nullptr; int rows = 0, K = 0; int row_tiles = 0, k_tiles = 0; size_t bytes = 0; };   // rows: outputs (stored: 16 row_tiles); K: stored, 32 k_tiles
@@ -87,7 +87,9 @@ int bamd_launch_dense_gemm(int act, const bamd_dense & w, const void * x, int ld
 void bamd_launch_split_rows(const float * x, int ldx, int rows, int k_tiles, void * planes, int cb, hipStream_t s);      // 32-bit rows as operand rows by blocks
 // few rows (<= BAMD_MV_ROWS): the weights stream once; out f32 [rows][ldo].  pre: how the operand comes about —
 enum { BAMD_PRE_ROWS = 0, BAMD_PRE_RESIDUAL = 1, BAMD_PRE_POLY = 2, BAMD_PRE_GROUP = 3, BAMD_PRE_FINAL = 4, BAMD_PRE_GLU = 5, BAMD_PRE_LAYER = 6 };     // (LAYER: RESIDUAL and FINAL with layer norms, chosen by res.norm); x given | one row, built in front of the product from the argument block
-// results of a step's last product, on their way to the host as well (host null: not); `done` behind them (count_serial null: not)
+// results of a step's last product, on their way to the host as well (host null: not); `done` behind them (count_serial null: not).  Two things hold this up.  A system-scope store to host memory is
+// past every cache once s_waitcnt vmcnt(0) lets its wave go on (gfx950; the language's memory model would ask for a release in every block, which was measured at 17 us of a step), so the block
+// that counts last may tell the host.  And `done` comes before the kernel's end: the results on the device are read behind it on the same stream only
 struct bamd_step_out { float * host = nullptr; uint32_t * done = nullptr, * count_serial = nullptr; };
 struct bamd_pre_args { bamd_residual_args res; bamd_poly_args poly; bamd_group_norm_args grp; bamd_glu_args glu; const float * gf; const int32_t * want; bamd_step_out close; };
 #define BAMD_MV_ROWS 64

@@ -235,7 +235,8 @@ static int pick_tile(int act, const bamd_dense & w, int rows, int most, int & sh
     return pick == TILE_64_64 && tiles(64, 64) * share <= 256 ? TILE_64_64_DEEP : pick;
 }
 // Row tiles of the matrix that whole rounds of 256 x 256 take, the rest going to a product of its own, where that is ahead by more than 3 % (of one product; halves are not cut): 0 none.  The launch
-// between them is 4 us.  2048 x 28672 x 4096 with the gated unit (3.5 rounds) 377 -> 352 us; 2048 x 16896 x 4096 249 -> 239
+// between them is 4 us.  2048 x 28672 x 4096 with the gated unit (3.5 rounds) 377 -> 352 us; 2048 x 16896 x 4096 249 -> 239.  Only for numbers of row tiles that divide the CUs: a round of others leaves
+// some idle, and what a cut gives there has not been measured
 int bamd_dense_cut(const bamd_dense & w, int rows, int out) {
     const int n_mt = (rows + 255) / 256;
     if (256 % n_mt) return 0;
