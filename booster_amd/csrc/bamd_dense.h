@@ -4,7 +4,7 @@
 //
 // Every kernel exists for two activation types: bfloat16 (matrix operands in bfloat16, 32-bit accumulation) and float.  There a product's rows are kept as three bfloat16
 // parts each, which together are the number: three exact products with the bfloat16 weights, summed in 32-bit, on the fast matrix instructions; attention and recurrences
-// take 32-bit operands.  No part is zero or infinite unless the number is, so that weights which are not finite come out as in 32 bits.  Residual stream, norms, scores, decays and
+// take 32-bit operands.  No part is zero unless the number is, so that weights which are not finite come out as in 32 bits.  Residual stream, norms, scores, decays and
 // states are 32-bit in both.
 //
 // Packed matrix [rows][K]: 16-row tiles; per tile the K / 32 blocks follow one another, 1 KiB each: lane l of a wave holds row l % 16, columns (l / 16) * 8 .. + 8 —

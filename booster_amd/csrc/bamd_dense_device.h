@@ -103,15 +103,16 @@ template <> __device__ __forceinline__ void store4<bamd_bf>(bamd_bf * h, bamd_v4
     *(bf4 *) h = bf4{ (bamd_bf) v[0], (bamd_bf) v[1], (bamd_bf) v[2], (bamd_bf) v[3] };
 }
 // A 32-bit operand is the sum of three bfloat16 numbers in planes 32 elements apart: the largest one below it, the largest below what is left, and the rest, which has eight bits.  All three are
-// exact and have the number's sign, and none is zero (from 1e-28 on) or infinite unless the number is: so a product with a weight that is not finite is what it would be in 32 bits.  A
-// zero, an infinity, a NaN: itself three times.
+// exact and have the number's sign, none is zero (from 1e-28 on) unless the number is, and an infinity or NaN is what is left of itself: so a product with a number or a weight that is not
+// finite is what it would be in 32 bits, without a test for it.
 // The number is fixed before it is taken apart: where it is a product, the compiler would fuse that into the subtraction, and the parts were those of the product without its rounding, cut off at the third
 struct Split { uint32_t p[3]; };                                   // in the upper sixteen bits
 __device__ __forceinline__ Split split_f(float v) {
     asm("" : "+v"(v));
-    const uint32_t u = __float_as_uint(v), abs = u & 0x7fffffffu, same = abs > 0x7f800000u ? u | 0x00400000u : u;
-    const float m = v - __uint_as_float((u - 1) & 0xffff0000u), l = m - __uint_as_float((__float_as_uint(m) - 1) & 0xffff0000u);
-    return abs - 1 < 0x7f7fffffu ? Split{ { u - 1, __float_as_uint(m) - 1, __float_as_uint(l) } } : Split{ { same, same, same } };
+    const uint32_t some = v != 0.f, h = __float_as_uint(v) - some;
+    const float m = v - __uint_as_float(h & 0xffff0000u);
+    const uint32_t g = __float_as_uint(m) - some;
+    return { { h, g, __float_as_uint(m - __uint_as_float(g & 0xffff0000u)) } };
 }
 struct bamd_s3 {
     uint16_t v;

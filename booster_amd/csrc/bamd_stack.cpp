@@ -1164,13 +1164,10 @@ struct OpScratch {                                 // device copies of one call
             if (f) { memcpy(&b[((size_t) r * ld + i) * 4], &v, 4); continue; }
             const size_t at = operand_at(r, i, ld, std::max(planes, 1), cb) * 2;
             if (planes < 3) { u += 0x7fff + ((u >> 16) & 1); const uint16_t o = (uint16_t) (u >> 16); memcpy(&b[at], &o, 2); continue; }
-            const uint32_t abs = u & 0x7fffffffu;                     // (split_f)
-            const bool apart = abs - 1 < 0x7f7fffffu;
-            if (abs > 0x7f800000u) u |= 0x00400000u;
+            const uint32_t some = v != 0.f;                           // (split_f)
             for (int k = 0; k < 3; ++k) {
-                const uint32_t top = apart && k < 2 ? (u - 1) & 0xffff0000u : u;
+                const uint32_t top = (k < 2 ? u - some : u) & 0xffff0000u;
                 const uint16_t o = (uint16_t) (top >> 16); memcpy(&b[at + 64 * k], &o, 2);
-                if (!apart) continue;
                 float t; memcpy(&t, &top, 4); v -= t; memcpy(&u, &v, 4);
             }
         }
