@@ -153,11 +153,21 @@ template <int RC, bool ONE> struct RowRegs {
     __device__ __forceinline__ void load(const float * p, int n) {
 #pragma unroll
         for (int c = 0; c < RC; ++c) {
-            if constexpr (ONE)
+            if constexpr (ONE && RC > 4) {                        // long rows (PolyNorm's): a branch for four values of the block, none for a thread's.  32 tests of a thread's were 1.5 us of a kernel's 8
+                v[c] = bamd_v4{ 0, 0, 0, 0 };
+                if (c * 4 * (int) blockDim.x < n)
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) v[c][k] = p[at(c, k) < n ? at(c, k) : n - 1];
+            } else if constexpr (ONE)
 #pragma unroll
                 for (int k = 0; k < 4; ++k) v[c][k] = at(c, k) < n ? p[at(c, k)] : 0.f;
             else v[c] = at(c, 0) < n ? *(const bamd_v4 *) (p + at(c, 0)) : bamd_v4{ 0, 0, 0, 0 };
         }
+        if constexpr (ONE && RC > 4)                              // (once all of them are asked for)
+#pragma unroll
+            for (int c = 0; c < RC; ++c) if (c * 4 * (int) blockDim.x < n && (c + 1) * 4 * (int) blockDim.x > n)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) v[c][k] = at(c, k) < n ? v[c][k] : 0.f;
     }
     // the sum of one or two planes
     __device__ __forceinline__ void load(const float * p, int n, int parts, size_t plane) {
