@@ -964,4 +964,8 @@ static inline size_t act_lds_bytes(int K) {
                                             ds_read_b128 lane groups of gfx950 ({0-3,12-15,20-27}, ...: MI355X_MICROARCH.md, LDS) see 16 distinct banks-of-4 (560 B: 2-way conflicts, SQ_LDS_BANK_CONFLICT 17.9M -> 9.1M per launch) */
 #endif
 #define BAMD_B16_Q (BAMD_B16_REC / 16)
-#define BAMD_BLOB16_BYTES(nb) ((((size_t) (nb) * (BAMD_B16_REC + 4)) + 15) & ~(size_t) 15)   /* per-token stride: records + d_y floats, 16-byte multiple */
+// In memory the records of a super-block lie together, token by token, 704 B apart: half a 128-byte line more than whole ones.  matmul_few_kernel's copies, 48 tokens of an 8B model: 4706 us a
+// prompt; 608, 640 and 672 B apart 4904 to 4912
+#define BAMD_B16_MEM 704
+#define BAMD_B16_STEP(T) (((uint32_t) (T) * BAMD_B16_MEM + 127u) & ~127u)    /* the records of a super-block of T tokens: whole lines */
+#define BAMD_BLOB16_BYTES(nb) (((size_t) (nb) + 1) * (BAMD_B16_MEM + 128))   /* per token; the sixteen-wave kernel's last copies read one super-block past the end */

@@ -19,7 +19,8 @@
 // f16 copy of a token's Q8_K row for the MFMA path.  Per super-block BAMD_B16_REC = 608 B (560 used): 8 (e) x 4 (g) groups of 8 halves — group
 // (e, g) = the int8 of sub-blocks 2g and 2g+1, chunk e, as exact f16: one 16-byte B operand of v_mfma_f32_16x16x32_f16 per lane —
 // then, per pair l of sub-blocks, the four halves {S_h(2l), S_h(2l+1), S_l(2l), S_l(2l+1)} of the block sums split as S = 2 S_h + S_l
-// (the B operand of the Q4_K min-term MFMA), then the four i16 pairs (S_2l, S_2l+1) (Q5_K), then the block scale d_y (f32, byte 560); after the nb super-blocks, yd[nb] f32 again.
+// (the B operand of the Q4_K min-term MFMA), then the four i16 pairs (S_2l, S_2l+1) (Q5_K), then the block scale d_y (f32, byte 560).  Records lie by super-block, then token:
+// what a step copies is one run of memory.
 template <int NORM>
 __global__ void __launch_bounds__(512) quantize_batch_kernel(const float * __restrict__ x, const float * __restrict__ nw, float eps, int K,
                                                              uint8_t * __restrict__ blob, uint8_t * __restrict__ blob16, uint8_t * __restrict__ frag) {
@@ -39,13 +40,14 @@ __global__ void __launch_bounds__(512) quantize_batch_kernel(const float * __res
         for (int i = threadIdx.x; i < (int) (bb / 16); i += blockDim.x) dst[i] = src[i];
     }
     if (blob16) {
-        uint8_t * o = blob16 + (size_t) t * BAMD_BLOB16_BYTES(nbt) + (size_t) b0 * BAMD_B16_REC;
+        const size_t rstep = BAMD_B16_STEP(gridDim.x);
+        uint8_t * o = blob16 + (size_t) b0 * rstep + (size_t) t * BAMD_B16_MEM;
         for (int i = threadIdx.x; i < nb * 64; i += blockDim.x) {          // q8[ci*64 + e*8 + c] = sub-block c, chunk e, 4 int8
             const int ci = i >> 6, e = (i >> 3) & 7, c = i & 7;
             const uint32_t w = q8[i];
             const unsigned short h0 = f2h((float) (int8_t) (w)), h1 = f2h((float) (int8_t) (w >> 8)), h2 = f2h((float) (int8_t) (w >> 16)), h3 = f2h((float) (int8_t) (w >> 24));
             uint2 v; v.x = (uint32_t) h0 | ((uint32_t) h1 << 16); v.y = (uint32_t) h2 | ((uint32_t) h3 << 16);
-            *(uint2 *) (o + (size_t) ci * BAMD_B16_REC + (size_t) (e * 4 + (c >> 1)) * 16 + (c & 1) * 8) = v;
+            *(uint2 *) (o + (size_t) ci * rstep + (size_t) (e * 4 + (c >> 1)) * 16 + (c & 1) * 8) = v;
         }
         for (int i = threadIdx.x; i < nb * 4; i += blockDim.x) {
             const int ci = i >> 2, l = i & 3;
@@ -54,12 +56,11 @@ __global__ void __launch_bounds__(512) quantize_batch_kernel(const float * __res
             uint2 mf;
             mf.x = (uint32_t) f2h((float) (sa >> 1)) | ((uint32_t) f2h((float) (sb >> 1)) << 16);
             mf.y = (uint32_t) f2h((float) (sa & 1)) | ((uint32_t) f2h((float) (sb & 1)) << 16);
-            *(uint2 *) (o + (size_t) ci * BAMD_B16_REC + 512 + l * 8) = mf;
+            *(uint2 *) (o + (size_t) ci * rstep + 512 + l * 8) = mf;
             // (S_2l, S_2l+1) as i16 pairs (Q5_K: v_dot2_i32_i16)
-            *(uint32_t *) (o + (size_t) ci * BAMD_B16_REC + 544 + l * 4) = ((uint32_t) sa & 0xffffu) | ((uint32_t) sb << 16);
+            *(uint32_t *) (o + (size_t) ci * rstep + 544 + l * 4) = ((uint32_t) sa & 0xffffu) | ((uint32_t) sb << 16);
         }
-        float * oyd = (float *) (o + (size_t) (nbt - b0) * BAMD_B16_REC) + b0;
-        for (int i = threadIdx.x; i < nb; i += blockDim.x) { oyd[i] = yd[i]; *(float *) (o + (size_t) i * BAMD_B16_REC + 560) = yd[i]; }   // d_y also inside the record (bamd_prefill2.hip: no separate copy)
+        for (int i = threadIdx.x; i < nb; i += blockDim.x) *(float *) (o + (size_t) i * rstep + 560) = yd[i];
     }
     if (frag) {
         // the operands of bamd_prefill_wide.hip, by tiles of 16 tokens: [tile][super-block][e][g][token] x 16 bytes (sub-blocks 2g and 2g+1 of chunk e as f16), behind them

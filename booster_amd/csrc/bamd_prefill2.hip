@@ -147,11 +147,11 @@ __global__ void __launch_bounds__(1024) matmul_mfma3_q4k_kernel(bamd_mma2_args a
     const int rb = blockIdx.y, t0 = blockIdx.x * 64;
     const int rtg = rb * 4 + rt;
     const bool live = rtg * 16 < a.nrows_pad;
-    const size_t b16 = BAMD_BLOB16_BYTES(nb);
+    const uint32_t rstep = BAMD_B16_STEP(a.T);             // records of a super-block: all tokens' one behind the other
     const uint32_t lds0 = (uint32_t) (size_t) (bamd_lds_vp) smem;
     // ---- stage plan.  A block = 45 KiB-instructions: k = 0..37 records (chunk 64 k + lane of 64 tokens x 38), 38..40 consumer headers, 41..44 builder
     //      operands.  Wave w issues k = w, 16 + w and k2 = 32 + w (w <= 12; waves 13..15 repeat the operand copies 41..43: same bytes, same place).
-    auto rec_off = [&](int idx) { const int tok = idx / BAMD_B16_Q, q = idx - tok * BAMD_B16_Q; const int tg = t0 + tok < a.T ? t0 + tok : a.T - 1; return (uint32_t) ((size_t) tg * b16 + (size_t) q * 16); };
+    auto rec_off = [&](int idx) { const int tok = idx / BAMD_B16_Q, q = idx - tok * BAMD_B16_Q; const int tg = t0 + tok < a.T ? t0 + tok : a.T - 1; return (uint32_t) tg * BAMD_B16_MEM + (uint32_t) q * 16u; };
     const int k2 = wave <= 12 ? 32 + wave : 28 + wave;
     const bool rec2 = k2 <= 37, hdr2 = k2 >= 38 && k2 <= 40;
     uint32_t so0 = rec_off(tid), so1 = rec_off(1024 + tid);          // advance by one super-block per step (sources stay fixed scalar pointers)
@@ -159,13 +159,13 @@ __global__ void __launch_bounds__(1024) matmul_mfma3_q4k_kernel(bamd_mma2_args a
     // sources of the NEXT stage call (the first call stages super-block 0 and the operands of super-block 1)
     const uint8_t * p01 = a.blob16;
     const uint8_t * p2 = rec2 ? a.blob16 : hdr2 ? a.ch + (size_t) rb * nb * X3_CHS : a.ph + (size_t) rb * nb * 4096 + 4096;
-    const uint32_t st2 = rec2 ? (uint32_t) BAMD_B16_REC : hdr2 ? (uint32_t) X3_CHS : 4096u;
+    const uint32_t st2 = rec2 ? rstep : hdr2 ? (uint32_t) X3_CHS : 4096u;
     // destinations by the parity of the step that issues the copies: records / headers of ci + 1 -> the OTHER block, operands of ci + 2 -> the block in use
     const uint32_t blk_a = lds0 + X3_BLK0, blk_b = blk_a + X3_BLK;
     const uint32_t d0_even = blk_b + (uint32_t) wave * 1024u, d0_odd = blk_a + (uint32_t) wave * 1024u;
     const uint32_t d2_even = (k2 <= 40 ? blk_b : blk_a) + (uint32_t) k2 * 1024u, d2_odd = (k2 <= 40 ? blk_a : blk_b) + (uint32_t) k2 * 1024u;
 #define X3_STAGE(PAR) do { x3_dma(p01, so0, (PAR) ? d0_odd : d0_even); x3_dma(p01, so1, ((PAR) ? d0_odd : d0_even) + 16384u); x3_dma(p2, so2, (PAR) ? d2_odd : d2_even); \
-                           so0 += BAMD_B16_REC; so1 += BAMD_B16_REC; so2 += st2; } while (0)
+                           so0 += rstep; so1 += rstep; so2 += st2; } while (0)
     // ---- builder: wave (rt, tt) = record group q = tt & 1 of the row tile, pieces g = 2 gh + j (gh = tt >> 1, j = 0, 1): lane (r, e) holds dwords 2 gh, 2 gh + 1
     //      of stream lane (r, e) = the halves of MFMA lanes (8 q + r, 2 gh + j) of fragment e
     const int br = lane >> 3, be = lane & 7, bq = tt & 1, gh = tt >> 1;
@@ -266,7 +266,7 @@ __global__ void __launch_bounds__(1024) matmul_mfma3_q4k_kernel(bamd_mma2_args a
 #endif
                 if (e == 0) x3_dma(p01, so0, CUR ? d0_odd : d0_even);
                 if (e == 1) x3_dma(p01, so1, (CUR ? d0_odd : d0_even) + 16384u);
-                if (e == 2) { x3_dma(p2, so2, CUR ? d2_odd : d2_even); so0 += BAMD_B16_REC; so1 += BAMD_B16_REC; so2 += st2; }
+                if (e == 2) { x3_dma(p2, so2, CUR ? d2_odd : d2_even); so0 += rstep; so1 += rstep; so2 += st2; }
                 if (e == 3) load_set(ci + 2, std::integral_constant<int, CUR>());
 #if !BAMD_PREFILL_CEILING
                 if (e > 1) {
@@ -369,8 +369,9 @@ __global__ void __launch_bounds__(1024) matmul_mfma3_q4k_kernel(bamd_mma2_args a
 // each, four copy (all of it one after the other on four waves: 1230 ns a super-block at 37 tokens; copies spread over consumers and builders: 930 — a copy holds its wave until
 // the vector memory path takes it); the arithmetic, its order and the layouts are those above.  Everything a step reads travels global -> LDS by DMA — token records two
 // super-blocks ahead, the row tile's quants, scales and headers four — and the wait at the end of a step leaves what was issued in it (and the weights issued in the one before)
-// in flight, so that a step is not as long as the memory's latency.  37 tokens, 4096 rows: K = 4096 25.0 -> 12.9 us, K = 14336 77 -> 38 us (Q6_K 105 -> 46 us); the copies of
-// the token records, the same to every block, are 24 us of the 38.
+// in flight, so that a step is not as long as the memory's latency.  37 tokens, 4096 rows: K = 4096 25.0 -> 12.9 us, K = 14336 77 -> 38 us (Q6_K 105 -> 46 us).  The copies of
+// the token records, the same to every block, were 24 us of the 38: of the tokens that there are and half a line out of step (BAMD_B16_MEM), 38 -> 34.6 us, a prompt 4681 -> 4511 (48 tokens,
+// no fewer copies, level).
 //   W slot of a super-block   Q4_K / Q5_K: 2 x 1 KiB quants of the two record groups | 1 KiB builder operands | 1 KiB consumer header | Q5_K: 2 x 256 B fifth bits
 //                             Q6_K: 2 x 1 KiB low bits | 2 x 512 B high bits | 2 x 1 KiB builder operands of the e-halves | 64 B of d
 template <int TYPE> struct FewW { static constexpr int SLOT = TYPE == BAMD_Q6_K ? 5184 : TYPE == BAMD_Q5_K ? 4608 : 4096, COPIES = TYPE == BAMD_Q4_K ? 1 : 2; };
@@ -384,27 +385,13 @@ template <int TYPE, int EPI, int NTT>
 __device__ __forceinline__ void few_block(const bamd_mma2_args & a, int rtg) {
     constexpr bool Q5 = TYPE == BAMD_Q5_K, Q6 = TYPE == BAMD_Q6_K;
     constexpr uint32_t RECB = Q6 ? 1680u : Q5 ? BAMD_RECB_Q5K : BAMD_RECB_Q4K;
-    constexpr int RI = few_records(NTT), RS = RI * 1024, NR = (RI + 3) / 4, NW = FewW<TYPE>::COPIES, WS = FewW<TYPE>::SLOT;
+    constexpr int RS = few_records(NTT) * 1024, NW = FewW<TYPE>::COPIES, WS = FewW<TYPE>::SLOT;
     constexpr int REC0 = 16 * X_FR, W0 = REC0 + XF_RING * RS, Z0 = W0 + XF_WRING * WS;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_id(), tt = wave, bw = wave & 3, m = lane & 15, g = lane >> 4;
     const int nb = a.K >> 8, rb = rtg >> 2, rtl = rtg & 3, t0 = blockIdx.x * (16 * NTT);
-    const size_t b16 = BAMD_BLOB16_BYTES(nb);
     const uint32_t lds0 = (uint32_t) (size_t) (bamd_lds_vp) smem;
     const bool active = tt < NTT && t0 + tt * 16 < a.T, builder = (wave >> 2) == 1, copier = wave >= 8;
-    // ---- copies.  Token records: RI instructions of 64 16-byte pieces, copier w issues w, w + 4, ... (one short of an instruction repeats its last)
-    uint32_t ro[NR], rd[NR];
-#pragma unroll
-    for (int r = 0; r < NR; ++r) {
-        int k = r * 4 + bw; if (k >= RI) k -= 4;
-        const int idx = k * 64 + lane, tok = idx / BAMD_B16_Q, q = idx - tok * BAMD_B16_Q, tg = t0 + tok < a.T ? t0 + tok : a.T - 1;
-        ro[r] = (uint32_t) ((size_t) tg * b16 + (size_t) q * 16); rd[r] = lds0 + REC0 + (uint32_t) k * 1024u;
-    }
-    auto copy_records = [&](int ci, int slot) {
-        const void * src = uniform_ptr(a.blob16 + (size_t) (ci < nb ? ci : nb - 1) * BAMD_B16_REC);
-#pragma unroll
-        for (int r = 0; r < NR; ++r) lds_dma16_s(src, ro[r], rd[r] + (uint32_t) slot * RS);
-    };
     // the row tile's operands: a kilobyte per copier, and the fifth bits / high bits and d of Q5_K / Q6_K.  A last tile of 8 (padded) rows takes its first record group twice
     // (rows 8..15 are never stored)
     const int rgq = 2 * rtg + (bw & 1), rgc = rgq * 8 < a.nrows_pad ? rgq : rgq - 1;
@@ -533,25 +520,48 @@ __device__ __forceinline__ void few_block(const bamd_mma2_args & a, int rtg) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) acc[4 * H + e][i] = fmaf(D[i], s[e][i], acc[4 * H + e][i]);
     };
-    // records of 0 and the operands of 0 and 1 have landed when all but the last NR + 2 NW copies have; so it stays: at the end of step ci the records of ci + 1 (issued in ci - 1) and
-    // the operands of ci + 2 (issued in ci - 2) have landed
-    auto publish = [&] { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(NR + 2 * NW) : "memory"); __builtin_amdgcn_s_barrier(); asm volatile("" ::: "memory"); };
     auto barrier = [&] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); __builtin_amdgcn_s_barrier(); asm volatile("" ::: "memory"); };
     if (tid < 8) *(uint32_t *) (smem + Z0 + tid * 4) = 0u;
     // a loop per kind of wave, barrier for barrier alike (one loop with branches inside moves the 48 accumulators through every join)
     auto after = [](int s, int by, int ring) { s += by; return s < ring ? s : s - ring; };
-    if (copier) { copy_records(0, 0); copy_weights(0, 0); copy_weights(1, 1); copy_records(1, 1); copy_weights(2, 2); copy_weights(3, 3); }
-    publish();
     if (copier) {
-        barrier();
-        for (int ci = 0, rs = 0, ws = 0; ci < nb; ++ci, rs = after(rs, 1, XF_RING), ws = after(ws, 1, XF_WRING)) {
-            copy_records(ci + 2, after(rs, 2, XF_RING)); copy_weights(ci + 4, after(ws, 4, XF_WRING));
-            if (Q6) barrier();
-            publish();
-        }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");          // (no copy outlives the block)
+        // Token records lie one token behind the other (quantize_batch_kernel): the kilobytes of those that there are, copier w issues w, w + 4, ... (one too many is the last again;
+        // behind it the LDS holds anything: columns of tokens that are never stored).  The wait leaves the copies of the last step in flight, so their number is a constant of the loop.
+        const int pieces = (a.T - t0 < 16 * NTT ? a.T - t0 : 16 * NTT) * BAMD_B16_Q, ri = (pieces + 63) / 64, need = (ri + 3) / 4;
+        auto copies = [&](auto nr_tag) {
+            constexpr int NR = decltype(nr_tag)::value;
+            uint32_t ro[NR], rd[NR];
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                const int k = r * 4 + bw < ri ? r * 4 + bw : ri - 1, idx = k * 64 + lane, pi = idx < pieces ? idx : pieces - 1, tok = pi / BAMD_B16_Q;
+                ro[r] = (uint32_t) (t0 + tok) * BAMD_B16_MEM + (uint32_t) (pi - tok * BAMD_B16_Q) * 16u; rd[r] = lds0 + REC0 + (uint32_t) k * 1024u;
+            }
+            auto copy_records = [&](int ci, int slot) {
+                const void * src = uniform_ptr(a.blob16 + (size_t) (ci < nb ? ci : nb - 1) * BAMD_B16_STEP(a.T));
+#pragma unroll
+                for (int r = 0; r < NR; ++r) lds_dma16_s(src, ro[r], rd[r] + (uint32_t) slot * RS);
+            };
+            // records of 0 and the operands of 0 and 1 have landed when all but the last NR + 2 NW copies have; so it stays: at the end of step ci the records of ci + 1 (issued in
+            // ci - 1) and the operands of ci + 2 (issued in ci - 2) have landed
+            auto landed = [&] { asm volatile("s_waitcnt vmcnt(%0)" :: "n"(NR + 2 * NW) : "memory"); barrier(); };
+            copy_records(0, 0); copy_weights(0, 0); copy_weights(1, 1); copy_records(1, 1); copy_weights(2, 2); copy_weights(3, 3);
+            landed();
+            barrier();
+            for (int ci = 0, rs = 0, ws = 0; ci < nb; ++ci, rs = after(rs, 1, XF_RING), ws = after(ws, 1, XF_WRING)) {
+                copy_records(ci + 2, after(rs, 2, XF_RING)); copy_weights(ci + 4, after(ws, 4, XF_WRING));
+                if (Q6) barrier();
+                landed();
+            }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // (no copy outlives the block)
+        };
+#define XF_NEED(N_) if (need <= N_) { copies(std::integral_constant<int, N_>()); return; }
+        if constexpr (NTT == 2) { XF_NEED(1) XF_NEED(2) XF_NEED(3) XF_NEED(4) copies(std::integral_constant<int, 5>()); }       // up to 32 tokens
+        else if constexpr (NTT == 3) { XF_NEED(5) XF_NEED(6) XF_NEED(7) copies(std::integral_constant<int, 8>()); }              // 33 to 48
+        else { XF_NEED(8) XF_NEED(9) copies(std::integral_constant<int, 10>()); }                                              // 49 to 64
+#undef XF_NEED
         return;
     }
+    barrier();
     if (builder) {
         if constexpr (Q6) build6(smem + W0, 0, fr0); else build45(smem + W0, fr0);
         barrier();
@@ -639,20 +649,19 @@ int bamd_prefill_mfma_supported(void) {
     return 1;
 }
 // Token tiles (of 16) per block of the few-token kernel for this product, 0: one of the kernels with 64-row blocks.
-// Up to 64 tokens: whichever ends first.  Both take a start and a time per super-block, for every round of 256 blocks.  The few-token kernel's goes by its token tiles, and with three (33 to
-// 48 tokens) by how the records of neighbouring tokens lie to the 128-byte lines that they are copied in: a stride of about half a line more or less is the fast one.  Constants in ns,
-// fitted to 1323 sizes (three types, 8 to 64 tokens, 1024 to 24576 rows, K 1024 to 14336), of which this rule takes the slower kernel for 23 by more than 1.5 %, at most 4 %.
+// Up to 64 tokens: whichever ends first.  Both take a start and a time per super-block, for every round of 256 blocks; the few-token kernel's goes by its token tiles.  Constants in ns,
+// fitted to 1323 sizes (three types, 8 to 64 tokens, 1024 to 24576 rows, K 1024 to 14336) with all records of the tiles copied: with fewer tokens the few-token kernel is faster than they say.
 // Where the two part, K = 4096, 64-row blocks against 16-row ones in us: 8192 rows Q4_K 32 tokens 24.1 | 18.4, 48 tokens 24.0 | 22.7, 64 tokens 24.1 | 25.5; 12288 rows 32 tokens 25.2 | 27.9;
-// Q6_K 8192 rows 64 tokens 34.7 | 31.2; and by the lines, Q4_K, 6144 rows, 36 tokens: K = 4096 23.9 | 22.8, K = 3840 22.7 | 25.2
-struct x_cost { int start64, step64, extra, start[3], near_half[3], other[3]; };      // extra: what the few-token kernel's launch takes more, whatever its rounds
+// Q6_K 8192 rows 64 tokens 34.7 | 31.2
+struct x_cost { int start64, step64, extra, start[3], step[3]; };      // extra: what the few-token kernel's launch takes more, whatever its rounds
 static int x_few_tiles(int type, int nrows_pad, int nb, int T) {
-    static const x_cost costs[3] = { { 3010, 1300, 1150, { 1790, 2140, 2400 }, { 410, 530, 590 }, { 420, 640, 600 } },         // Q4_K
-                                     { 3410, 1240, 1800, { 1900, 2180, 2600 }, { 416, 520, 580 }, { 420, 563, 590 } },         // Q5_K
-                                     { 3590, 1815, 1150, { 2040, 2400, 2740 }, { 680, 710, 750 }, { 685, 740, 783 } } };       // Q6_K
+    static const x_cost costs[3] = { { 3010, 1300, 1150, { 1790, 2140, 2400 }, { 410, 530, 590 } },         // Q4_K
+                                     { 3410, 1240, 1800, { 1900, 2180, 2600 }, { 416, 520, 580 } },         // Q5_K
+                                     { 3590, 1815, 1150, { 2040, 2400, 2740 }, { 680, 710, 750 } } };       // Q6_K
     if (T > 64) return 0;
     const x_cost & c = costs[type == BAMD_Q6_K ? 2 : type == BAMD_Q5_K ? 1 : 0];
-    const int i = T <= 32 ? 0 : T <= 48 ? 1 : 2, line = (int) (BAMD_BLOB16_BYTES(nb) & 127);
-    const long few = c.extra + (long) ((nrows_pad + 15) / 16 + 255) / 256 * (c.start[i] + (long) (line >= 48 && line <= 80 ? c.near_half : c.other)[i] * nb);
+    const int i = T <= 32 ? 0 : T <= 48 ? 1 : 2;
+    const long few = c.extra + (long) ((nrows_pad + 15) / 16 + 255) / 256 * (c.start[i] + (long) c.step[i] * nb);
     return few < ((long) x_row_blocks(nrows_pad) + 255) / 256 * (c.start64 + (long) c.step64 * nb) ? i + 2 : 0;
 }
 int bamd_prefill_few_tiles(int type, int nrows_pad, int K, int T) { return x_few_tiles(type, nrows_pad, K >> 8, T); }

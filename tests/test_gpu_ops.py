@@ -266,6 +266,17 @@ def test_mul_mat_batch_few_tokens(bamd, po, t, nb, rows):
             assert_bits(got[i], ref + res[i] if res is not None else ref, "type %d nb %d rows %d T %d token %d" % (t, nb, rows, T, i))
 
 
+@pytest.mark.parametrize("t", [12, 13, 14])
+@pytest.mark.parametrize("T", [3, 6, 7, 13, 14, 20, 21, 26, 27, 34, 40, 41, 47, 53, 54, 60, 61])
+def test_mul_mat_batch_few_tokens_record_copies(bamd, t, T):
+    """token records are copied by the kilobyte, as many as there are tokens: every count of them per copying wave, and its edges"""
+    nb, rows = 6, 72
+    rng = np.random.default_rng(100 * t + T)
+    W = random_kquant_tensor(t, nb * 256, rows, rng)
+    X = (rng.standard_normal((T, nb * 256)) * 3).astype(np.float32)
+    assert_bits(bamd.op_mul_mat_batch(t, W, rows, nb * 256, X, impl=2), bamd.op_mul_mat_batch(t, W, rows, nb * 256, X, impl=0), "type %d T %d" % (t, T))
+
+
 @pytest.mark.parametrize("t,impl", [(12, 4), (13, 4), (14, 4), (14, 5)])
 @pytest.mark.parametrize("nb,rows", [(1, 8), (2, 136), (3, 24), (8, 72), (9, 1000), (17, 40)])
 def test_mul_mat_batch_many_tokens(bamd, po, t, impl, nb, rows):
