@@ -143,7 +143,11 @@ __global__ void __launch_bounds__(64 * WV) matmul_wide_kernel(bamd_wide_args a) 
     const bamd_f4 z = { 0.f, 0.f, 0.f, 0.f };
     const bamd_h2 k1024 = { (_Float16) -1024.f, (_Float16) -1024.f }, k1056 = { (_Float16) -1056.f, (_Float16) -1056.f }, k1152 = { (_Float16) -1152.f, (_Float16) -1152.f };
     auto pair_of = [](uint32_t bytes, uint32_t sel) { bamd_h2u c; c.u = __builtin_amdgcn_perm(0x64646464u, bytes, sel); return c.h; };       // two bytes as 1024 + byte, f16
-    auto plus1024 = [](uint32_t v, uint32_t mask) { bamd_h2u c; c.u = (v & mask) | 0x64006400u; return c.h; };
+    // (constants in registers, unknown to the compiler: one v_and_or_b32, which takes no literals, for v_and_b32 and v_or_b32 with literals; 32 of 265 vector instructions a super-block,
+    // the product's loop 3290 -> 3134 cycles, 14336 rows x 2048 tokens x 4096 499 -> 484 us)
+    uint32_t k6400 = 0x64006400u, low = 0x000f000fu, high = 0x00f000f0u;
+    if constexpr (Q4) { asm volatile("" : "+v"(k6400)); asm volatile("" : "+s"(low), "+s"(high)); }
+    auto plus1024 = [&](uint32_t v, uint32_t mask) { bamd_h2u c; c.u = (v & mask) | k6400; return c.h; };
     union Frag { bamd_h2 h[4]; bamd_h8 v; };
     const uint32_t upper = 0u - (uint32_t) (g >> 1);              // (a mask, no branch)
     bamd_h2 s0, n0, s1, n1, sl0, sl1; uint32_t sc6[2];
@@ -197,8 +201,8 @@ __global__ void __launch_bounds__(64 * WV) matmul_wide_kernel(bamd_wide_args a) 
                 f.h[2] = __builtin_elementwise_fma(pair_of(hi, 0x04020400u), s1, n1); f.h[3] = __builtin_elementwise_fma(pair_of(hi, 0x04030401u), s1, n1);
             } else {
                 const uint32_t w8 = r.q >> 8;
-                f.h[0] = __builtin_elementwise_fma(plus1024(r.q, 0x000f000fu), s0, n0); f.h[1] = __builtin_elementwise_fma(plus1024(w8, 0x000f000fu), s0, n0);
-                f.h[2] = __builtin_elementwise_fma(plus1024(r.q, 0x00f000f0u), s1, n1); f.h[3] = __builtin_elementwise_fma(plus1024(w8, 0x00f000f0u), s1, n1);
+                f.h[0] = __builtin_elementwise_fma(plus1024(r.q, low), s0, n0); f.h[1] = __builtin_elementwise_fma(plus1024(w8, low), s0, n0);
+                f.h[2] = __builtin_elementwise_fma(plus1024(r.q, high), s1, n1); f.h[3] = __builtin_elementwise_fma(plus1024(w8, high), s1, n1);
             }
         }
     };
