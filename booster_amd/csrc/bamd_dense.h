@@ -136,6 +136,10 @@ int bamd_latent_prompt_rows(int act, int D);       // query rows per tile
 int bamd_latent_max_rank(int act);
 // decoding: one row per entry.  qp: absorbed queries [rows][heads padded to 16][Rp]; part_o [rows][hgroups][splits][16][Rp], part_ml [..][16][2]
 int bamd_launch_latent_decode(int act, const bamd_batch_dev & b, const bamd_latent_args & a, void * qp, float * part_o, float * part_ml, int splits, hipStream_t s);
+// the same in one launch (bamd_latent_step_valid), which is the faster one for rows of up to `most` positions where bamd_latent_one_launch says so; what is faster for some length is for all shorter ones
+bool bamd_latent_step_valid(int D, int Rp);
+bool bamd_latent_one_launch(int act, int D, int Rp, int rows, int heads, int most);
+void bamd_launch_latent_step(int act, const bamd_batch_dev & b, const bamd_latent_args & a, hipStream_t s);
 
 // ---- attention over cached keys and values -----------------------------------------------------------------------------------------------------------
 // Grouped heads over 64-position pages; position i sees j <= i with i - j < window or j < keep.  Optional: unit-RMS queries and keys, a cap on the scores (cap tanh(s / cap)),

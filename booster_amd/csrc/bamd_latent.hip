@@ -5,6 +5,7 @@
 //     parts, partial sums combined, then the value up-projection per head.
 // A sink enters as the first key's place in the running maximum and sum (weight exp(sink), no value); a gate multiplies each head by sigmoid of its own projection.
 #include "bamd_dense_device.h"
+#include <algorithm>
 #include <math.h>
 
 // ---- the cache --------------------------------------------------------------------------------------------------------------------------------------
@@ -375,6 +376,183 @@ template <typename T> __global__ void __launch_bounds__(512) latent_combine_kern
     }
 }
 
+// A decoded token of one head in one launch: block (head, row) of sixteen waves.  The query goes into the latent space (qp = W_uk^T q), the sequence's latents pass by in registers — a wave
+// holds whole rows, takes their scores, and adds them up with their weights, all by itself — and the sixteen waves' sums, the token's own latent and the sink meet in front of the value
+// up-projection.  The three launches above become one; the pass over the cache that sixteen heads share there is every head's own here, out of the L2.  W_uk and the first latents are requested
+// before the token's row arrives.  Scores, weights and sums are 32-bit on the vector units: a head is one row of the matrix cores.
+// KT: D / 32; NRT: sixteen-row tiles of W_uk per wave (Rp <= 256 NRT); NP: pieces of sixteen bytes of a latent per lane
+template <typename T> __device__ __forceinline__ void piece_of(const bamd_u4 & w, float * x) {
+    if constexpr (sizeof(T) == 2) { x[0] = bf_lo(w.x); x[1] = bf_hi(w.x); x[2] = bf_lo(w.y); x[3] = bf_hi(w.y); x[4] = bf_lo(w.z); x[5] = bf_hi(w.z); x[6] = bf_lo(w.w); x[7] = bf_hi(w.w); }
+    else { x[0] = __uint_as_float(w.x); x[1] = __uint_as_float(w.y); x[2] = __uint_as_float(w.z); x[3] = __uint_as_float(w.w); }
+}
+template <typename T, int KT, int NRT, int NP> __global__ void __launch_bounds__(1024) latent_step_kernel(bamd_batch_dev b, bamd_latent_args a) {
+    constexpr int VPP = 16 / (int) sizeof(T), D = 32 * KT, VT = D / 16, KP = 16 / VT, NKT = (8 * NRT + KP - 1) / KP, PF = NP == 2 ? 2 : NRT == 2 ? 3 : 4, RM = 256 * NRT;      // KP: shares of K per value tile
+    extern __shared__ __align__(16) unsigned char lds[];
+    __shared__ float q[D], qp[RM], own[RM], red[32], ms[257], ls[257], part[16][16];
+    const int h = blockIdx.x, row = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int rt_n = a.Rp / 16, kt_n = a.Rp / 32, pr = a.Rp / VPP;
+    bamd_u4 wk[NRT][KT];
+#pragma unroll
+    for (int j = 0; j < NRT; ++j)
+#pragma unroll
+        for (int k = 0; k < KT; ++k) wk[j][k] = wave + 16 * j < rt_n ? *(const bamd_u4 *) (a.ukT + ((((size_t) h * rt_n + wave + 16 * j) * KT + k) * 64 + lane) * 8) : bamd_u4{ 0, 0, 0, 0 };
+    const bamd_entry e = b.ent[row];
+    const int past = e.pos0;
+    const int32_t * const pages = b.pages + (size_t) e.seq * b.max_pages;
+    const float * in = a.in + (size_t) row * a.ld;
+    float qv = 0.f, cv = 0.f, cn = 0.f;
+    static_assert(D <= 1024 && RM <= 1024, "a thread per value of the query and of the latent");
+    if (tid < D) qv = in[a.q_off + h * D + tid];
+    if (tid < a.R) { cv = in[a.c_off + tid]; cn = a.c_norm[tid]; }
+    // rows of the cache: 2^lg lanes hold one (NP > 1: every lane NP pieces of one), a wave `rows` at a time, PF times in a batch; row (i * 16 + wave) * rows + lane >> lg.  A batch's rows never
+    // straddle a page: `rows` is a power of two
+    int lg = 0; while (lg < 6 && (1 << lg) < pr) ++lg;
+    const int rows = 64 >> lg, sub = lane >> lg, px = lane & ((1 << lg) - 1);
+    bamd_u4 pc[2][PF][NP];
+    auto request = [&](int batch, auto to) {
+#pragma unroll
+        for (int i = 0; i < PF; ++i) {
+            const int r0 = ((batch * PF + i) * 16 + wave) * rows, r = r0 + sub;
+            const T * src = (const T *) a.cache + ((size_t) (r0 < past ? pages[r0 / BAMD_PAGE] : 0) * BAMD_PAGE + r % BAMD_PAGE) * a.Rp;
+#pragma unroll
+            for (int p = 0; p < NP; ++p) pc[decltype(to)::value][i][p] = r < past && px + 64 * p < pr ? *(const bamd_u4 *) (src + (px + 64 * p) * VPP) : bamd_u4{ 0, 0, 0, 0 };
+        }
+    };
+    const int batches = (past + PF * 16 * rows - 1) / (PF * 16 * rows);
+    const std::integral_constant<int, 0> even; const std::integral_constant<int, 1> odd;
+    request(0, even); request(1, odd);
+    float sq[1] = { cv * cv };
+    if (tid < D) q[tid] = qv;
+    block_sum<1>(sq, red);                                         // (its barriers publish q as well)
+    if (tid < a.Rp) {                                              // as it is cached
+        const T v = to_act<T>(tid < a.R ? cv * (1.0f / sqrtf(sq[0] / (float) a.R + a.eps)) * cn : 0.f);
+        own[tid] = (float) v;
+        if (h == 0) ((T *) a.cache)[((size_t) pages[past / BAMD_PAGE] * BAMD_PAGE + past % BAMD_PAGE) * a.Rp + tid] = v;
+    }
+#pragma unroll
+    for (int j = 0; j < NRT; ++j) {
+        float v = 0.f;
+#pragma unroll
+        for (int k = 0; k < KT; ++k) {
+            const float * x = q + k * 32 + (lane >> 4) * 8;
+            const bamd_u4 w = wk[j][k];
+            v += bf_lo(w.x) * x[0] + bf_hi(w.x) * x[1] + bf_lo(w.y) * x[2] + bf_hi(w.y) * x[3] + bf_lo(w.z) * x[4] + bf_hi(w.z) * x[5] + bf_lo(w.w) * x[6] + bf_hi(w.w) * x[7];
+        }
+        v += __shfl_xor(v, 16); v += __shfl_xor(v, 32);
+        if (lane < 16 && wave + 16 * j < rt_n) qp[(wave + 16 * j) * 16 + lane] = v;
+    }
+    bamd_u4 wv[NKT];                                               // of this wave's value tile and share of K
+    const int vt = wave % VT, kp = wave / VT;
+#pragma unroll
+    for (int k = 0; k < NKT; ++k) wv[k] = k * KP + kp < kt_n ? *(const bamd_u4 *) (a.uv.w + ((((size_t) h * VT + vt) * kt_n + k * KP + kp) * 64 + lane) * 8) : bamd_u4{ 0, 0, 0, 0 };
+    __syncthreads();
+    float qx[NP][VPP], o[NP][VPP], m = -INFINITY, l = 0.f;
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+        for (int i = 0; i < VPP; ++i) { qx[p][i] = px + 64 * p < pr ? qp[(px + 64 * p) * VPP + i] : 0.f; o[p][i] = 0.f; }
+    auto take = [&](int batch, auto from) {
+        float s[PF], mx = m;
+#pragma unroll
+        for (int i = 0; i < PF; ++i) {
+            float v = 0.f;
+#pragma unroll
+            for (int p = 0; p < NP; ++p) {
+                float x[VPP];
+                piece_of<T>(pc[decltype(from)::value][i][p], x);
+#pragma unroll
+                for (int k = 0; k < VPP; ++k) v += qx[p][k] * x[k];
+            }
+            s[i] = v;
+        }
+        if (lg >= 4) {
+#pragma unroll
+            for (int i = 0; i < PF; ++i) s[i] = row_sum16(s[i]);
+        } else for (int d = 1; d < (1 << lg); d *= 2)
+#pragma unroll
+            for (int i = 0; i < PF; ++i) s[i] += __shfl_xor(s[i], d);
+        if (lg >= 5)
+#pragma unroll
+            for (int i = 0; i < PF; ++i) s[i] += __shfl_xor(s[i], 16);
+        if (lg >= 6)
+#pragma unroll
+            for (int i = 0; i < PF; ++i) s[i] += __shfl_xor(s[i], 32);
+#pragma unroll
+        for (int i = 0; i < PF; ++i) { s[i] = ((batch * PF + i) * 16 + wave) * rows + sub < past ? s[i] * a.scale : -INFINITY; mx = fmaxf(mx, s[i]); }
+        const float ref = mx == -INFINITY ? 0.f : mx, f = __expf(m - ref);          // (no rows yet: nothing to rescale)
+        l *= f; m = mx;
+#pragma unroll
+        for (int p = 0; p < NP; ++p)
+#pragma unroll
+            for (int k = 0; k < VPP; ++k) o[p][k] *= f;
+#pragma unroll
+        for (int i = 0; i < PF; ++i) {
+            const float w = __expf(s[i] - ref);
+            l += w;
+#pragma unroll
+            for (int p = 0; p < NP; ++p) {
+                float x[VPP];
+                piece_of<T>(pc[decltype(from)::value][i][p], x);
+#pragma unroll
+                for (int k = 0; k < VPP; ++k) o[p][k] += w * x[k];
+            }
+        }
+    };
+    for (int t = 0; t < batches; t += 2) {
+        take(t, even); request(t + 2, even);
+        if (t + 1 < batches) { take(t + 1, odd); request(t + 3, odd); }
+    }
+    // sixteen waves x `rows` sums, the own latent behind them
+    float * const ps = (float *) lds;                              // [16 rows][Rp]
+    const int n = 16 * rows, at = wave * rows + sub;
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+        if (px + 64 * p < pr)
+#pragma unroll
+            for (int k = 0; k < VPP; ++k) ps[at * a.Rp + (px + 64 * p) * VPP + k] = o[p][k];
+    if (px == 0) { ms[at] = m; ls[at] = l; }
+    if (wave == 0) {
+        float v = 0.f;
+        for (int r = lane; r < a.Rp; r += 64) v += qp[r] * own[r];
+        v = wave_sum(v) * a.scale;
+        if (lane == 0) { ms[n] = v; ls[n] = 1.f; }
+    }
+    __syncthreads();
+    const float snk = a.sink ? a.sink[h] : -INFINITY;
+    float mx = fmaxf(snk, ms[n]);
+    for (int i = lane; i < n; i += 64) mx = fmaxf(mx, ms[i]);
+    mx = wave_max(mx);
+    float sum = 0.f;
+    for (int i = lane; i <= n; i += 64) sum += __expf(ms[i] - mx) * ls[i];
+    sum = wave_sum(sum);
+    if (a.sink) sum += expf(snk - mx);
+    const int th = a.Rp <= 256 ? 4 : 2, r = tid / th, g = tid % th;          // th threads per value of the latent: neighbours
+    float v = 0.f;
+    if (r < a.Rp) {
+        for (int i = g; i < n; i += th) v += __expf(ms[i] - mx) * ps[i * a.Rp + r];
+        if (g == 0) v += __expf(ms[n] - mx) * own[r];
+    }
+    v += __shfl_xor(v, 1); if (th == 4) v += __shfl_xor(v, 2);
+    if (r < a.Rp && g == 0) qp[r] = v;                             // (the scores are behind a barrier)
+    __syncthreads();
+    v = 0.f;
+#pragma unroll
+    for (int k = 0; k < NKT; ++k)
+        if (k * KP + kp < kt_n) {
+            const float * x = qp + (k * KP + kp) * 32 + (lane >> 4) * 8;
+            const bamd_u4 w = wv[k];
+            v += bf_lo(w.x) * x[0] + bf_hi(w.x) * x[1] + bf_lo(w.y) * x[2] + bf_hi(w.y) * x[3] + bf_lo(w.z) * x[4] + bf_hi(w.z) * x[5] + bf_lo(w.w) * x[6] + bf_hi(w.w) * x[7];
+        }
+    v += __shfl_xor(v, 16); v += __shfl_xor(v, 32);
+    if (lane < 16) part[wave][lane] = v;
+    __syncthreads();
+    if (tid >= D) return;
+    v = 0.f;
+#pragma unroll
+    for (int k = 0; k < KP; ++k) v += part[k * VT + tid / 16][tid % 16];
+    *row_out<Operand<T>>(a.out, row, a.ldo, a.cb).at(h * D + tid) = to_operand<Operand<T>>(v * ((a.gated ? sigmoid_f(in[a.g_off + h]) : 1.f) / sum));
+}
+
 // ---- launches ---------------------------------------------------------------------------------------------------------------------------------------
 void bamd_launch_latent_store(int act, const bamd_batch_dev & b, const bamd_latent_args & a, hipStream_t s) {
     if (act == BAMD_ACT_F32) hipLaunchKernelGGL(latent_store_kernel<float>, dim3(b.rows), dim3(256), 0, s, b, a);
@@ -434,6 +612,28 @@ static int decode_go(const bamd_batch_dev & b, const bamd_latent_args & a, void 
     else decode_pick<T, 32>(b, a, (const T *) qp, part_o, part_ml, splits, s);
     hipLaunchKernelGGL(latent_combine_kernel<T>, dim3(a.heads, b.rows), dim3(512), ((size_t) a.Rp + 2048) * 4, s, b, a, part_o, part_ml, splits);
     return 0;
+}
+template <typename T, int KT> static void step_pick(const bamd_batch_dev & b, const bamd_latent_args & a, hipStream_t s) {
+    constexpr int VPP = 16 / (int) sizeof(T);
+    int lanes = 1; while (lanes < 64 && lanes < a.Rp / VPP) lanes *= 2;
+    const size_t lds = (size_t) 16 * (64 / lanes) * a.Rp * 4;
+    const dim3 grid(a.heads, b.rows);
+    if (a.Rp <= 256) hipLaunchKernelGGL((latent_step_kernel<T, KT, 1, 1>), grid, dim3(1024), lds, s, b, a);
+    else hipLaunchKernelGGL((latent_step_kernel<T, KT, 2, 16 / VPP / 2>), grid, dim3(1024), lds, s, b, a);
+}
+template <typename T> static void step_go(const bamd_batch_dev & b, const bamd_latent_args & a, hipStream_t s) {
+    if (a.D == 32) step_pick<T, 1>(b, a, s); else if (a.D == 64) step_pick<T, 2>(b, a, s); else step_pick<T, 4>(b, a, s);
+}
+bool bamd_latent_step_valid(int D, int Rp) { return D <= 128 && Rp <= 512; }
+// Every head reads the cache by itself in the one launch, sixteen share it in the three: 20 to 25 us less a layer against 12 ns a position of 256 bfloat16 numbers.  Steps of eight layers, three
+// launches and one, us: width 2048, rank 256, 16 heads: 60 positions 423 | 398, 155 427 | 408, 380 428 | 418, 800 432 | 438; sixteen rows 216 709 | 689, 500 707 | 692, 1000 711 | 716; 32-bit 155
+// 461 | 430, 380 460 | 452, 800 461 | 501.  Width 4096, rank 512, 32 heads: 155 830 | 809, 380 838 | 836, 800 827 | 884; sixteen rows 216 1280 | 1253, 500 1289 | 1317; 32-bit 155 907 | 849.
+// With more than two blocks to a CU the three are ahead: 48 rows of 16 heads, 100 positions 1200 | 1223
+bool bamd_latent_one_launch(int act, int D, int Rp, int rows, int heads, int most) {
+    return bamd_latent_step_valid(D, Rp) && most > 0 && (size_t) most * Rp <= (act == BAMD_ACT_F32 ? 112 * 1024 : 144 * 1024) && rows * heads <= 512;
+}
+void bamd_launch_latent_step(int act, const bamd_batch_dev & b, const bamd_latent_args & a, hipStream_t s) {
+    if (act == BAMD_ACT_F32) step_go<float>(b, a, s); else step_go<bamd_bf>(b, a, s);
 }
 int bamd_launch_latent_decode(int act, const bamd_batch_dev & b, const bamd_latent_args & a, void * qp, float * part_o, float * part_ml, int splits, hipStream_t s) {
     return act == BAMD_ACT_F32 ? decode_go<float>(b, a, qp, part_o, part_ml, splits, s) : decode_go<bamd_bf>(b, a, qp, part_o, part_ml, splits, s);

@@ -12,6 +12,7 @@
 #include "bamd_stack.h"
 
 #include <algorithm>
+#include <array>
 #include <chrono>
 #include <fstream>
 #include <iterator>
@@ -146,6 +147,7 @@ struct Mixer {
     virtual int run(Pass & p, MixState & st, Operand & o) = 0;       // p.y holds the input projection's rows
     virtual int f32_cols() const { return 0; }                       // columns of the f32 scratch row it wants
     virtual int latents() const { return 0; }
+    virtual bool one_launch(int, int, int) const { return false; }      // compute type, decoding rows, most positions of one: attention is one launch (more positions: it may not be)
     virtual int prompt_rows(int) const { return 0; }                 // query rows per tile of a prompt (0: no attention)
     virtual int scan_blocks() const { return 0; }                    // blocks of one segment of a prompt's scan (0: no segments)
     virtual void partials(int, size_t &, size_t &) const {}          // floats of the decoding shares' sums and of their maxima, for so many rows
@@ -208,13 +210,13 @@ struct Ctx {
     unsigned char * dev = nullptr; int32_t * pages = nullptr;
     static constexpr int RING = 4;
     unsigned char * pinned = nullptr, * host[RING] = {}; int32_t * pages_host[RING] = {}; hipEvent_t ev[RING] = {}; int ring = 0;
-    std::map<int, hipGraphExec_t> graphs;          // rows * 4 + what is in front and behind (STEP_*)
+    std::map<std::array<int, 3>, hipGraphExec_t> graphs;          // rows, what is in front and behind (STEP_*), layers whose attention is one launch
     bamd_step_box * box = nullptr; uint32_t * count_serial = nullptr; uint32_t serial = 0;      // decoding steps by way of pinned memory; serial: of the last one
 };
 struct Pass {                                      // one pass through the layers
     Ctx & c; Stack & st; hipStream_t s; bamd_batch_dev b; bool decode = false;
-    int n_tiles = 0, k_rows = 0, max_n = 1, n_segs = 0; float * x; float * xo; const float * pend = nullptr; int ldp = 0; const float * pend_g = nullptr; int pend_parts = 1;
-    Timer * tm = nullptr;
+    int n_tiles = 0, k_rows = 0, max_n = 1, n_segs = 0, most = 0; float * x; float * xo; const float * pend = nullptr; int ldp = 0; const float * pend_g = nullptr; int pend_parts = 1;
+    Timer * tm = nullptr;                          // most: positions of the longest sequence behind this pass (steps that are enqueued at once: behind the last)
     void begin(int kind, double bytes) { if (!tm) return; hipEvent_t e; hipEventCreate(&e); hipEventRecord(e, s); tm->ev.push_back(e); tm->kind.push_back(kind); tm->bytes.push_back(bytes); }
     void end() { if (!tm) return; hipEvent_t e; hipEventCreate(&e); hipEventRecord(e, s); tm->ev.push_back(e); }
 
@@ -311,6 +313,7 @@ struct LatentAttention : Mixer {
         return l.vec(p + "dkv.norm", { R }, &c_norm) || (dz.latent_sink && l.vec(p + "sink", { H }, &sink));
     }
     int latents() const override { return Rp; }
+    bool one_launch(int act, int rows, int most) const override { return bamd_latent_one_launch(act, D, Rp, rows, H, most); }
     int prompt_rows(int act) const override { return bamd_latent_prompt_rows(act, D); }
     double step_bytes(int len) const override { return (double) len * R * 2; }
     int state(Ctx & c, MixState & st) override;
@@ -694,7 +697,8 @@ int LatentAttention::run(Pass & p, MixState & st, Operand & o) {
     o.x = c.h; o.ldx = out.K;
     p.begin(1, p.tm ? step_bytes(c.seqs[0].len + 1) + (double) uk.bytes + (double) uv.bytes : 0);
     int rc = 0;
-    if (p.decode) rc = bamd_launch_latent_decode(act, p.b, a, c.qp, c.part_o, c.part_ml, splits_for(c, p.b.rows, (H + 15) / 16), p.s);
+    if (p.decode && one_launch(act, p.b.rows, p.most)) bamd_launch_latent_step(act, p.b, a, p.s);
+    else if (p.decode) rc = bamd_launch_latent_decode(act, p.b, a, c.qp, c.part_o, c.part_ml, splits_for(c, p.b.rows, (H + 15) / 16), p.s);
     else {
         const size_t kr = (size_t) p.k_rows, el = p.st.el();
         if (grow(c, &c.kc, &c.kc_n, kr * Rp * el, p.s) || grow(c, &c.kk, &c.kk_n, kr * H * D * el, p.s) || grow(c, &c.kv, &c.kv_n, kr * H * D * el, p.s)) return 1;
@@ -843,7 +847,7 @@ int send(Pass & p, const std::vector<Piece> & pc, const std::vector<int32_t> & w
             for (int i = 0; i < blocks; ++i) kblk[kb + i] = (int32_t) e;
             kb += blocks;
         }
-        rows += pc[e].n; p.max_n = std::max(p.max_n, pc[e].n);
+        rows += pc[e].n; p.max_n = std::max(p.max_n, pc[e].n); p.most = std::max(p.most, q.len + pc[e].n);
     }
     // longest key ranges first: the tail of the launch is short tiles
     if (!p.decode && tq) {
@@ -893,6 +897,7 @@ int leave(Pass & p, const std::vector<Piece> & pc) {
         Seq & q = c.seqs[(size_t) pc[e].seq];
         c.box->in.ent[e] = { pc[e].seq, (int32_t) e, 1, q.len, q.par, 0 };
         c.box->in.tok[e] = pc[e].tokens[0];
+        p.most = std::max(p.most, q.len + 1);
     }
     c.box->in.serial = ++c.serial;
     __atomic_thread_fence(__ATOMIC_RELEASE);
@@ -927,7 +932,9 @@ int decode_rows(Pass & p, int kind) {
         return 0;
     };
     if (!g_graph) return enqueue();
-    const int key = n * 4 + kind;
+    int ones = 0;                                                  // (layers whose attention is one launch for rows of this length: the same number, the same layers)
+    for (const Layer & ly : p.st.layers) ones += ly.mix->one_launch(p.st.act, n, p.most);
+    const std::array<int, 3> key = { n, kind, ones };
     auto it = c.graphs.find(key);
     if (it == c.graphs.end()) {
         hipGraph_t g = nullptr; hipGraphExec_t ex = nullptr;
@@ -1046,6 +1053,7 @@ int Stack::generate(bamd_context * bc, const int32_t * seqs, int n, int n_steps,
     HIPC(hipMemcpyAsync(c.step, &zero, 4, hipMemcpyHostToDevice, s));
     Pass p{ c, *this, s, {}, true };
     if (send(p, pc, want)) return 1;
+    p.most += n_steps - 1;
     hipEvent_t a = nullptr, b = nullptr;
     HIPC(hipEventCreate(&a));
     if (hipEventCreate(&b) != hipSuccess) { hipEventDestroy(a); return fail("hipEventCreate"); }
@@ -1329,6 +1337,7 @@ BAMD_OP bamd_op_latent_attention(int act, const float * q, const float * c, cons
     if (!q || !c || !c_norm || !uk || !uv || !out || rows < 1 || pos0 < 0 || (pos0 && !past) || heads < 1 || dim < 1 || dim > 256 || vdim < 1 || vdim > 256 || rank < 1 || rank > 1024 || (decode && rows != 1) || s.init(act) || s.one_entry(rows, pos0, b))
         return fail("bamd_op_latent_attention: bad arguments");
     int D = 32; while (D < std::max(dim, vdim)) D *= 2;
+    if (decode == 2 && !bamd_latent_step_valid(D, up(rank, 32))) return fail("bamd_op_latent_attention: no step of one launch for this shape");
     const int Rp = up(rank, 32), HD = heads * D, g_off = HD + up(rank, 16), ld = up(g_off + heads, 16), len = pos0 + rows, kr = up(len, BAMD_PAGE), hp = up(heads, 16);
     std::vector<float> in((size_t) rows * ld, 0.f);
     for (int r = 0; r < rows; ++r) {
@@ -1358,7 +1367,8 @@ BAMD_OP bamd_op_latent_attention(int act, const float * q, const float * c, cons
     if (s.up_(t.data(), t.size(), &tiles) || s.up_(kb.data(), kb.size(), &kblk)) return 1;
     a.in = din; a.ld = ld; a.c_off = HD; a.g_off = g_off; a.c_norm = dn; a.eps = eps; a.scale = scale; a.sink = dsink; a.gated = gate ? 1 : 0; a.heads = heads; a.D = D; a.R = rank; a.Rp = Rp; a.cache = cache; a.ukT = ukT; a.out = o; a.ldo = HD;
     int rc;
-    if (decode) rc = bamd_launch_latent_decode(act, b, a, qp, po, pm, splits, s.l.s);
+    if (decode == 2) { rc = 0; bamd_launch_latent_step(act, b, a, s.l.s); }
+    else if (decode) rc = bamd_launch_latent_decode(act, b, a, qp, po, pm, splits, s.l.s);
     else {
         bamd_launch_latent_store(act, b, a, s.l.s);
         bamd_launch_latent_gather(act, b, a, kblk, kr, kc, s.l.s);

@@ -448,6 +448,15 @@ def test_latent_attention(bamd, dtype, H, d, dv, R, T, pos0):
         near(got.reshape(T, -1), want.reshape(T, -1), dtype)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H,d,dv,R", [(1, 8, 8, 8), (3, 24, 40, 36), (17, 16, 32, 64), (2, 72, 128, 100), (2, 128, 64, 256), (3, 100, 96, 264), (2, 128, 128, 512)])
+@pytest.mark.parametrize("pos0", [0, 1, 15, 63, 64, 127, 128, 191, 192, 255, 256, 257, 520, 1100])
+def test_latent_attention_step_in_one_launch(bamd, dtype, H, d, dv, R, pos0):
+    """the token's own latent alone, first and last of a chunk of cached ones (64 to 256, by the rank and the type), whole chunks and a part"""
+    a = attention_case(H, d, dv, R, 1, pos0, H * d + pos0, dtype)
+    near(bamd.op_latent_attention(dtype=dtype, decode=2, **a).reshape(1, -1), plain_attention(H=H, **a).reshape(1, -1), dtype)
+
+
 @pytest.mark.parametrize("H,d,R,T,pos0", [(128, 24, 20, 257, 0), (128, 24, 20, 512, 70), (128, 24, 20, 513, 0), (85, 40, 36, 700, 130)])
 def test_latent_attention_in_paired_blocks(bamd, H, d, R, T, pos0):
     """tiles of 128 queries: one block per CU and a part of a second, two (taken the other way round), two and a part of a third (plain order), and heads that do not divide the CUs"""
@@ -485,7 +494,8 @@ def test_one_key_stands_out(bamd, dtype, pos0):
     for key in (0, 63, 64, 191, 298, 299):
         case = dict(a, q=rd(k[key][None] / (k[key] ** 2).sum(-1)[None, :, None]), c=a["c"][-1:], gate=a["gate"][-1:], past=rd(lat[:-1]), scale=24.0)
         want = plain_attention(H=H, **case)
-        near(bamd.op_latent_attention(dtype=dtype, decode=True, **case).reshape(1, -1), want.reshape(1, -1), dtype, 3)
+        for decode in (True, 2):
+            near(bamd.op_latent_attention(dtype=dtype, decode=decode, **case).reshape(1, -1), want.reshape(1, -1), dtype, 3)
 
 
 @pytest.mark.parametrize("scale", [0.125, 0.13])
@@ -509,7 +519,7 @@ def test_scores_far_from_zero(bamd, scale):
     near(bamd.op_latent_attention(dtype="float32", **a).reshape(T, -1), want.reshape(T, -1), "float32")
 
 
-@pytest.mark.parametrize("decode", [False, True])
+@pytest.mark.parametrize("decode", [False, True, 2])
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_sinks_and_gates(bamd, dtype, decode):
     """sinks from nothing to almost everything, none at all, gates open, shut and absent"""
