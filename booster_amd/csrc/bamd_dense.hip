@@ -491,6 +491,93 @@ static void few_go(const bamd_dense & w, const void * x, int ldx, int cb, int ro
     const int groups = (w.row_tiles + RT - 1) / RT;
     hipLaunchKernelGGL((dense_few_kernel<NT, RT, NS, GLU>), dim3(groups < 256 ? groups : 256, parts), dim3(512), (size_t) 8 * (NS * (NT + RT) + NT * RT) * 1024, s, w, (const bamd_bf *) x, ldx, cb, rows, out, ldo, cbo, limit, close);
 }
+// The same for up to sixteen rows where a block has several row tiles to go through and the rows' shares of K fit LDS: each wave copies its share of the rows once, in front of the loop, and its weights
+// go straight to registers, D requests of a kilobyte ahead, from one tile into the next.  Tiles are dealt out one by one (GLU: in pairs of gate and up), so that no CU has more than one above the
+// others — dense_few_kernel's groups of two or three leave up to a third of a round idle — and neighbours read neighbouring memory (a run of tiles per block: up to 18 % slower where the runs lie half a
+// megabyte apart).  The weights are requested first and everything is waited for once: rows first were 1 to 4 % slower.  Eight requests ahead: 1 to 6 % slower, sixteen: level.  Sums of up to `meet` tiles
+// wait in LDS for the eight waves to meet; they are the sums of dense_few_kernel, in its order.  us, that kernel and this one, behind a launch that writes the rows (its 2 us included): 16 rows x 14336 x
+// 4096 27.7 | 24.2 (5.2 TB/s), 16768 x 4096 32.8 | 28.5, 32000 x 4096 52.2 | 47.8, 28672 x 4096 with the gated unit 49.1 | 44.6, two rows x 8192 x 4096 18.1 | 15.8.
+template <int D, bool GLU>
+__global__ void __launch_bounds__(512) dense_share_kernel(bamd_dense w, const bamd_bf * x, int ldx, int cb, int rows, float * out, int ldo, int cbo, float limit, bamd_step_out close, int meet) {
+    constexpr int NW = 8, UNIT = GLU ? 2 : 1;
+    extern __shared__ __align__(16) unsigned char lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), stride = gridDim.x;
+    const int k0 = w.k_tiles * wave / NW, n = w.k_tiles * (wave + 1) / NW - k0, kn = (w.k_tiles + NW - 1) / NW;
+    float * red = (float *) (lds + (size_t) NW * kn * 1024);       // [wave][meet][64 lanes][4], behind the rows
+    const int tiles = (w.row_tiles / UNIT - (int) blockIdx.x + stride - 1) / stride * UNIT, steps = tiles * n;
+    auto tile_of = [&](int j) { return ((int) blockIdx.x + j / UNIT * stride) * UNIT + j % UNIT; };
+    const uint16_t * src = w.w + ((size_t) tile_of(0) * w.k_tiles + k0) * 512;
+    const size_t near = (size_t) (w.k_tiles - n + 1) * 512, far = near + (size_t) (stride - 1) * UNIT * w.k_tiles * 512;      // from a share's end to the next tile's
+    int rk = 0, rj = 0, left = steps;
+    bamd_u4 ring[D];
+    auto request = [&](int u) {                                   // (behind the last step: that one again, for nobody)
+        ring[u] = *(const bamd_u4 *) (src + lane * 8);
+        if (--left > 0) { if (++rk < n) src += 512; else { rk = 0; ++rj; src += GLU && (rj & 1) ? near : far; } }
+    };
+#pragma unroll
+    for (int u = 0; u < D; ++u) request(u);
+    {
+        int r = lane >> 2; r = r < rows ? r : rows - 1;
+        const uint32_t xo = (uint32_t) r * (uint32_t) ldx * 2u + (uint32_t) ((lane & 3) ^ ((lane >> 3) & 3)) * 16u, to = (uint32_t) (size_t) (bamd_lds_vp) lds + (uint32_t) (wave * kn) * 1024u;
+        for (int k = 0; k < n; ++k) lds_dma16_s((const unsigned char *) x + (size_t) (k0 + k) * cb * 2, xo, to + (uint32_t) k * 1024u);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const unsigned char * xs = lds + (size_t) wave * kn * 1024 + ((lane & 15) * 4 + ((lane >> 4) ^ ((lane >> 1) & 3))) * 16;
+    bamd_v4 acc = { 0, 0, 0, 0 };
+    int k = 0, waiting = 0, first = 0;                             // tiles whose sums wait; the first of them
+    auto all_here = [&] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); __builtin_amdgcn_s_barrier(); asm volatile("" ::: "memory"); };
+    auto join = [&](int count) {
+        all_here();
+        auto sum = [&](int t, int rl, int o) {                    // of column o, row rl of tile t
+            float v = 0.f;
+#pragma unroll
+            for (int q = 0; q < NW; ++q) v += red[(q * meet + t) * 256 + sum_slot((o >> 2) * 16 + rl) + (o & 3)];
+            return v;
+        };
+        for (int i = tid; i < count / UNIT * 256; i += 64 * NW) {
+            const int t = (i >> 8) * UNIT, oc = i & 15, r = (i >> 4) & 15, o = tile_of(first + t) / UNIT * 16 + oc;
+            if (r >= rows || o >= w.rows / UNIT) continue;
+            if constexpr (GLU) *row_out<bamd_bf>(out, r, ldo, cbo).at(o) = (bamd_bf) clamped_glu(sum(t, r, oc), sum(t + 1, r, oc), limit);
+            else {
+                const float v = sum(t, r, oc);
+                out[(size_t) r * ldo + o] = v;
+                to_host(close, (size_t) r * ldo + o, v);
+            }
+        }
+        first += count;
+    };
+    auto take = [&](int u) {
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bamd_bf8, ring[u]), *(const bamd_bf8 *) (xs + k * 1024), acc, 0, 0, 0);
+        if (++k < n) return;
+        *(bamd_v4 *) (red + (wave * meet + waiting) * 256 + sum_slot(lane)) = acc;
+        acc = bamd_v4{ 0, 0, 0, 0 }; k = 0;
+        if (++waiting == meet) { join(meet); waiting = 0; all_here(); }      // (every wave has as many tiles, and at least a column block of each)
+    };
+    int s = 0;
+    for (; s + D <= steps; s += D)
+#pragma unroll
+        for (int u = 0; u < D; ++u) { take(u); request(u); }
+#pragma unroll
+    for (int u = 0; u < D; ++u) if (s + u < steps) take(u);
+    if (waiting) join(waiting);
+    close_step(close);
+}
+// Where whole decoding steps are ahead, dense_few_kernel and this one, us, four layers each: width 4096 (Tupitar) two rows 562 | 546, sixteen 855 | 822; (Mafurax) six rows 793 | 775; width 3200,
+// thirteen rows 602 | 600; 3584, three rows 548 | 546.  Below K = 3072 the products by themselves are ahead (11328 x 2048 6 % at two rows), steps are not: width 2048, six rows 367 | 367, width 1024, twelve
+// rows 238 | 240.  With two tiles a block it takes K of about 4096 (two rows x 4640 x 3072 10.7 | 10.9, x 4096 13.1 | 12.4, x 4608 11.2 | 11.8), and K beyond 4608 leaves no room for the sums
+static bool share_fits(const bamd_dense & w, int rows) {
+    if (rows > 16 || w.k_tiles < 96 || w.k_tiles > 144) return false;
+    return w.row_tiles > 512 || (w.row_tiles > 256 && w.k_tiles >= 112 && w.k_tiles <= 128);
+}
+template <bool GLU>
+static void share_go(const bamd_dense & w, const void * x, int ldx, int cb, int rows, float * out, int ldo, hipStream_t s, const bamd_step_out & close, int cbo = 0, float limit = 0.f) {
+    constexpr int unit = GLU ? 2 : 1;
+    const int units = w.row_tiles / unit, grid = units < 256 ? units : 256, kn = (w.k_tiles + 7) / 8, most = (units + grid - 1) / grid * unit;
+    // A product that brings its results to the host meets after every tile: the bus is slower than the sums, and with eight tiles together all of them waited for it at the end (six rows of 32000: 31 | 40 us)
+    const int meet = close.host ? 1 : std::min(most, (20 - kn) / unit * unit);      // of 160 KiB, eight a tile
+    const size_t lds = (size_t) 8 * (kn + meet) * 1024;
+    hipLaunchKernelGGL((dense_share_kernel<12, GLU>), dim3(grid), dim3(512), lds, s, w, (const bamd_bf *) x, ldx, cb, rows, out, ldo, cbo, limit, close, meet);
+}
 bool bamd_dense_closes(int act, const bamd_dense & w, int rows, int ldo) { return act == BAMD_ACT_F32 || rows <= 32 || w.row_tiles <= 768 || (ldo & 3); }
 // RT by the rounds over the CUs; a round of 1, 2 or 3 tiles at K = 4096 takes 7.1, 12.7 and 16 us with up to 16 rows, one of 1 or 2 tiles 9.0 and 15.1 us with up to 32.
 // With more rows the 64 x 64 tiles of prompts are ahead once they fill the CUs (45 x 22672 x 4096: 49 against 74 us) and behind before (45 x 4096 x 14336: 136 against 48)
@@ -501,7 +588,8 @@ static int few_pick(const bamd_dense & w, const void * x, int ldx, int cb, int r
         few_go<4, 1, 3>(w, x, ldx, cb, rows, out, ldo, s, parts, close);
     } else if (rows > 16) {
         if (rounds[0] * 90 <= rounds[1] * 151) few_go<2, 1, 5>(w, x, ldx, cb, rows, out, ldo, s, parts, close); else few_go<2, 2, 4>(w, x, ldx, cb, rows, out, ldo, s, 1, close);
-    } else {
+    } else if (share_fits(w, rows)) share_go<false>(w, x, ldx, cb, rows, out, ldo, s, close);
+    else {
         const long t1 = rounds[0] * 71, t2 = rounds[1] * 127, t3 = rounds[2] * 160;
         if (t1 <= t2 && t1 <= t3) few_go<1, 1, 5>(w, x, ldx, cb, rows, out, ldo, s, parts, close);
         else if (t2 <= t3) few_go<1, 2, 5>(w, x, ldx, cb, rows, out, ldo, s, 1, close);
@@ -572,7 +660,9 @@ int bamd_launch_dense_few_glu(const bamd_dense & w, const void * x, int ldx, int
     if (!bamd_dense_few_glu(BAMD_ACT_BF16, w, rows) || !rows_fit(w, ldx, cb, rows, 32) || ldh < w.row_tiles * 8 || (ldh & 3)) return 1;
     if (cb) ldx = 32; else cb = 32;
     if (rows > 32) return gemm_tiles<bamd_bf, BAMD_OUT_GLU>(w, x, ldx, cb, rows, h, ldh, cbo, limit, s);
-    if (rows > 16) few_go<2, 2, 4, true>(w, x, ldx, cb, rows, (float *) h, ldh, s, 1, {}, cbo, limit); else few_go<1, 2, 5, true>(w, x, ldx, cb, rows, (float *) h, ldh, s, 1, {}, cbo, limit);
+    if (rows > 16) few_go<2, 2, 4, true>(w, x, ldx, cb, rows, (float *) h, ldh, s, 1, {}, cbo, limit);
+    else if (share_fits(w, rows)) share_go<true>(w, x, ldx, cb, rows, (float *) h, ldh, s, {}, cbo, limit);
+    else few_go<1, 2, 5, true>(w, x, ldx, cb, rows, (float *) h, ldh, s, 1, {}, cbo, limit);
     return 0;
 }
 int bamd_launch_dense_mv(int act, const bamd_dense & w, int pre, const bamd_batch_dev & b, const bamd_pre_args * p, const void * x, int ldx, int cb, int rows, float * out, int ldo, hipStream_t s, int * parts) {

@@ -250,6 +250,25 @@ def test_dense_few_rows(bamd, n, rows, k):
     assert (np.abs(bamd.op_dense(w, x, "bfloat16", 1) - want) <= 1e-5 * scale).all()                 # sqrt(k) <= 46 roundings of 2^-24 in a row, three times over
 
 
+# rows in LDS: the first and last sizes (257 row tiles, more than two a CU, the shortest and the longest K), shares of K that differ by a column block, tiles that meet in two goes (K = 4600), a CU with a
+# tile more than others, rows by rows and by blocks; sizes beside them for which dense_few_kernel stays
+@pytest.mark.parametrize("n,rows,k", [(4097, 5, 3553), (4097, 16, 4096), (4640, 2, 3300), (4640, 16, 4100), (8192, 4, 4090), (8193, 1, 3041), (8193, 3, 3040), (8210, 16, 4600), (8210, 16, 4640), (12290, 9, 3300)])
+def test_dense_rows_in_lds(bamd, n, rows, k):
+    r = np.random.default_rng(n + k + rows)
+    w = so.f32_to_bf16(r.standard_normal((n, k)).astype(np.float32))
+    x = so.round_bf16(r.standard_normal((rows, k)).astype(np.float32))
+    wf = so.bf16_to_f32(w)
+    want = x.astype(np.float64) @ wf.T.astype(np.float64)
+    scale = np.sqrt((x ** 2) @ (wf.T ** 2))
+    for impl in (1, 7):
+        assert (np.abs(bamd.op_dense(w, x, "bfloat16", impl) - want) <= 1.5e-5 * scale).all(), impl      # sqrt(k) <= 68 roundings of 2^-24 in a row, three times over (12e-6), and the scale's own
+
+
+@pytest.mark.parametrize("F,rows,k", [(2060, 5, 3553), (2060, 16, 4096), (4096, 4, 4090), (4112, 2, 3041), (4112, 16, 4600), (4128, 16, 4640), (6200, 3, 3300)])
+def test_dense_gated_rows_in_lds(bamd, F, rows, k):
+    gated(bamd, "bfloat16", F, rows, k)
+
+
 # K in two shares (few row tiles, many columns: an odd number of column blocks among them), and sizes just below that
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("n,k,rows", [(500, 2100, 131), (77, 2049, 300), (500, 1000, 70), (500, 2100, 1), (2048, 2080, 6), (2049, 2080, 6), (77, 2049, 20), (500, 2100, 45), (500, 2000, 6)])
