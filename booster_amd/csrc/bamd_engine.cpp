@@ -954,7 +954,8 @@ static int decode_to(bamd_context * c, const int32_t * tokens, int n_tokens, int
     bool gave = false;                                              // the step wrote the logits and the status words to the host itself
     if (c->cells.active && n_tokens > 1) { fail("after a context shift (bamd_kv_seq_add) tokens are evaluated one per call"); return 1; }
     if (!c->cells.active) c->n_cached = std::max(c->n_cached, n_past + n_tokens);
-    if (hipMemcpyAsync(c->forced, tokens, (size_t) n_tokens * 4, hipMemcpyHostToDevice, s) != hipSuccess) { fail("H2D tokens"); return 1; }
+    // (a single token goes its own way to the device, stage_step: in the inbox of the own queue's step, in front of the graph otherwise)
+    if (n_tokens > 1 && hipMemcpyAsync(c->forced, tokens, (size_t) n_tokens * 4, hipMemcpyHostToDevice, s) != hipSuccess) { fail("H2D tokens"); return 1; }
     if (n_tokens > 1 && (n_tokens <= BAMD_PREFILL_CAP || n_tokens <= c->bcap) && prefill_batch_supported(c, n_past + n_tokens - 1)) {
         // one part: every layer once for all tokens, lm_head for the last
         if (ensure_batch_buffers(c, n_tokens)) return 1;
