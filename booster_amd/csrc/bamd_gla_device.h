@@ -160,3 +160,70 @@ template <typename T> __device__ __forceinline__ void gla_norm_block(const bamd_
     }
     if (h0 + 16 >= a.heads) for (int c = a.heads * a.Pp + threadIdx.x; c < a.out_cols; c += 256) *out.at(a.out_off + c) = to_operand<Operand<T>>(0.f);
 }
+// A decoded token of one head in a whole block of 512: all its value columns (up to PT), so that the norm over them and the gate come behind the recurrence in the same launch.  NPL state rows per lane;
+// heads of up to 128 channels.  Everything is asked for before anything is waited for, the state first
+template <typename T, int PT, int NPL> struct GlaHead {
+    static constexpr int NW = 8, Q = PT / 4, NG = 64 / Q, GROUPS = NW * NG, NP = GROUPS * NPL;
+    static constexpr size_t lds = (size_t) (PT + 3 * NP + GROUPS * PT + 2) * 4;
+};
+template <typename T, int PT, int NPL>
+__device__ __forceinline__ void gla_head_block(const bamd_gla_args & a, int h, int row, bool first, float * st, unsigned char * lds) {
+    typedef GlaHead<T, PT, NPL> G;
+    constexpr int Q = G::Q, NP = G::NP, GROUPS = G::GROUPS;
+    static_assert(PT <= 128 && NP <= 128, "a quarter of the block per kind of operand");
+    float * vs = (float *) lds, * ks = vs + PT, * as = ks + NP, * qs = as + NP, * yp = qs + NP, * part = yp + GROUPS * PT;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, quad = lane % Q, grp = wave * G::NG + lane / Q, Np = a.Np, Pp = a.Pp, c = tid & 127, kind = tid >> 7;
+    const float * in = a.in + (size_t) row * a.ld;
+    bamd_v4 s[NPL];
+#pragma unroll
+    for (int j = 0; j < NPL; ++j) { const int r = grp * NPL + j; s[j] = !first && r < Np && quad * 4 < Pp ? *(const bamd_v4 *) (st + (size_t) r * Pp + quad * 4) : bamd_v4{ 0, 0, 0, 0 }; }
+    float gate = 0.f, norm = 0.f;
+    if (kind == 0) {                                              // decays; later the outputs
+        if (c < Pp) { norm = a.norm[c]; if (a.g_off >= 0) gate = in[a.g_off + h * Pp + c]; }
+        float z = 0.f;
+        if (c < Np) {
+            const size_t aw = (size_t) a.heads * Np;
+            z = a.a2b[h * Np + c];
+            for (int r0 = 0; r0 < a.rank; r0 += 16) {              // sixteen factors on their way at once
+                float w[16], t[16];
+#pragma unroll
+                for (int r = 0; r < 16; ++r) { const int i = min(r0 + r, a.rank - 1); w[r] = bf_f(a.a2[(size_t) i * aw + h * Np + c]); t[r] = in[a.t_off + i]; }
+#pragma unroll
+                for (int r = 0; r < 16; ++r) z = fmaf(r0 + r < a.rank ? w[r] : 0.f, t[r], z);
+            }
+        }
+        if (c < NP) as[c] = c < Np ? gla_alpha(z, a.inv_tau) : 0.f;
+    } else if (kind == 1) { if (c < NP) ks[c] = c < Np ? in[a.k_off + h * Np + c] : 0.f; }
+    else if (kind == 2) { if (c < NP) qs[c] = c < Np ? in[a.q_off + h * Np + c] : 0.f; }
+    else if (c < PT) vs[c] = c < Pp ? in[a.v_off + h * Pp + c] : 0.f;
+    __syncthreads();
+    const bamd_v4 v = *(const bamd_v4 *) (vs + quad * 4);
+    bamd_v4 y = { 0, 0, 0, 0 };
+#pragma unroll
+    for (int j = 0; j < NPL; ++j) {
+        const int r = grp * NPL + j;
+        const float k = ks[r], al = as[r], q = qs[r];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { s[j][i] = fmaf(al, s[j][i], k * v[i]); y[i] = fmaf(q, s[j][i], y[i]); }
+    }
+    *(bamd_v4 *) (yp + grp * PT + quad * 4) = y;
+#pragma unroll
+    for (int j = 0; j < NPL; ++j) { const int r = grp * NPL + j; if (r < Np && quad * 4 < Pp) *(bamd_v4 *) (st + (size_t) r * Pp + quad * 4) = s[j]; }
+    __syncthreads();
+    float o = 0.f;
+    if (tid < PT) {
+        float t[4] = { 0.f, 0.f, 0.f, 0.f };
+#pragma unroll
+        for (int g = 0; g < GROUPS; ++g) t[g & 3] += yp[g * PT + tid];
+        o = ((t[0] + t[1]) + (t[2] + t[3])) * a.q_scale;
+        const float ss = wave_sum(tid < Pp ? o * o : 0.f);
+        if (lane == 0) part[wave] = ss;
+    }
+    __syncthreads();
+    const RowOut<Operand<T>> out = row_out<Operand<T>>(a.out, row, a.ldo, a.cb);
+    if (tid < Pp) {
+        const float r = 1.0f / sqrtf((PT > 64 ? part[0] + part[1] : part[0]) / (float) a.P + a.eps);
+        *out.at(a.out_off + h * Pp + tid) = to_operand<Operand<T>>(o * r * norm * (a.g_off >= 0 ? gate / (1.0f + __expf(-gate)) : 1.f));
+    }
+    if (h == a.heads - 1) for (int i = a.heads * Pp + tid; i < a.out_cols; i += 512) *out.at(a.out_off + i) = to_operand<Operand<T>>(0.f);
+}

@@ -56,32 +56,35 @@ template <typename T, int ND> __device__ __forceinline__ void kv_head(const bamd
 }
 
 // LDS of a decoding block: the waves' weights, then their sums
-template <typename T, int ND> struct KvDecodeLds {
+template <typename T, int ND, int NW = 4> struct KvDecodeLds {
     static constexpr int D = ND * 32, NP = sizeof(T) == 2 ? 2 : 1, PS = 32 + 16 / sizeof(T);
-    static constexpr size_t weights = (size_t) 4 * NP * 16 * PS * sizeof(T), sums = ((size_t) 4 * 16 * D + 4 * 16 * 2) * 4, bytes = weights > sums ? weights : sums;
+    static constexpr size_t weights = (size_t) NW * NP * 16 * PS * sizeof(T), sums = ((size_t) NW * 16 * D + NW * 16 * 2) * 4, bytes = weights > sums ? weights : sums;
 };
-// one of `splits` shares of a row's keys for (kv head, group of 16 heads) = y; four waves take half pages in turn; the last wave of the last share brings the row's own key and value
-// and stores them in the cache
-template <typename T, int ND>
+// one of `splits` shares of a row's keys for (kv head, group of 16 heads) = y; NW waves take half pages in turn; the last wave of the last share brings the row's own key and value
+// and stores them in the cache.  ONE: there is one share, its last wave has nothing else to do, and its sums are gated and written as operand (kv_combine_block)
+template <typename T, int ND, int NW = 4, bool ONE = false>
 __device__ __forceinline__ void kv_decode_block(const bamd_batch_dev & b, const bamd_kv_args & a, int sp, int splits, int y, int row, float * part_o, float * part_ml, unsigned char * lds) {
-    typedef KvDecodeLds<T, ND> L;
+    typedef KvDecodeLds<T, ND, NW> L;
     constexpr int D = L::D, NV = ND * 2, NP = L::NP, PS = L::PS;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lr = lane & 15, lq = lane >> 4;
     const int rep = a.heads / a.kv_heads, hgs = (rep + 15) / 16, g = y / hgs, hg = y % hgs, h0 = g * rep + hg * 16, nh = min(16, rep - hg * 16);
     const bamd_entry e = b.ent[row];
-    const int pos = e.pos0, wi = sp * 4 + wave, nw = splits * 4;
+    const int pos = e.pos0, wi = sp * NW + wave, nw = ONE ? NW - 1 : splits * NW;
     const KvPages pg(a, pos - a.window + 1, (pos + BAMD_PAGE - 1) / BAMD_PAGE);
-    const int per = (2 * pg.count + nw - 1) / nw, t0 = wi * per, t1 = min(2 * pg.count, t0 + per);
-    const bool own = wi == nw - 1;
+    const int half_pages = 2 * pg.count - (ONE && pos % BAMD_PAGE && pos % BAMD_PAGE <= 32 && pg.page(pg.count - 1) == pos / BAMD_PAGE), per = (half_pages + nw - 1) / nw, t0 = wi * per, t1 = min(half_pages, t0 + per);
+    const bool own = wi == (ONE ? NW : nw) - 1;
     const size_t base = ((size_t) row * a.kv_heads * hgs + y) * splits + sp;
-    if (sp * 4 * per >= 2 * pg.count && sp != splits - 1) {        // a share without keys
-        for (int i = tid; i < nh * D; i += 256) part_o[base * 16 * D + i] = 0.f;
+    if (!ONE && sp * NW * per >= half_pages && sp != splits - 1) {        // a share without keys
+        for (int i = tid; i < nh * D; i += 64 * NW) part_o[base * 16 * D + i] = 0.f;
         if (tid < nh) { part_ml[(base * 16 + tid) * 2] = -INFINITY; part_ml[(base * 16 + tid) * 2 + 1] = 0.f; }
         return;
     }
     const int32_t * pages = b.pages + (size_t) e.seq * b.max_pages;
     const float * in = a.in + (size_t) row * a.ld;
     const KvCap cap = kv_cap(a);
+    __shared__ float gates[ONE ? 16 : 1];
+    float gate = 0.f;
+    if constexpr (ONE) if (a.gated && tid < nh) gate = in[a.g_off + h0 + tid];
     T * P = (T *) lds + (size_t) wave * NP * 16 * PS;
     // everything the first 32 keys need is on its way before the queries are normed (heads too wide for the registers read them as they go)
     constexpr bool AHEAD = ND * sizeof(T) <= 8;
@@ -215,9 +218,10 @@ __device__ __forceinline__ void kv_decode_block(const bamd_batch_dev & b, const 
                 }
         }
     }
-    // the four waves' sums
+    // the waves' sums
     __syncthreads();
-    float * so = (float *) lds, * sml = so + 4 * 16 * D;
+    float * so = (float *) lds, * sml = so + NW * 16 * D;
+    if constexpr (ONE) if (tid < nh) gates[tid] = (a.gated ? sigmoid_f(gate) : 1.f) * a.out_scale;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int hd = lq * 4 + r;
@@ -227,16 +231,17 @@ __device__ __forceinline__ void kv_decode_block(const bamd_batch_dev & b, const 
         for (int j = 0; j < NV; ++j) so[((size_t) wave * 16 + hd) * D + j * 16 + lr] = o[j][r];
     }
     __syncthreads();
-    for (int i = tid; i < nh * D; i += 256) {
+    for (int i = tid; i < nh * D; i += 64 * NW) {
         const int hd = i / D, d = i % D;
         float mx = -INFINITY, s = 0.f, t = 0.f;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) mx = fmaxf(mx, sml[(w * 16 + hd) * 2]);
+        for (int w = 0; w < NW; ++w) mx = fmaxf(mx, sml[(w * 16 + hd) * 2]);
         if (mx != -INFINITY)
 #pragma unroll
-            for (int w = 0; w < 4; ++w) { const float f = __builtin_amdgcn_exp2f(sml[(w * 16 + hd) * 2] - mx); s += f * sml[(w * 16 + hd) * 2 + 1]; t += f * so[((size_t) w * 16 + hd) * D + d]; }
-        part_o[(base * 16 + hd) * D + d] = t;
-        if (d == 0) { part_ml[(base * 16 + hd) * 2] = mx; part_ml[(base * 16 + hd) * 2 + 1] = s; }
+            for (int w = 0; w < NW; ++w) { const float f = __builtin_amdgcn_exp2f(sml[(w * 16 + hd) * 2] - mx); s += f * sml[(w * 16 + hd) * 2 + 1]; t += f * so[((size_t) w * 16 + hd) * D + d]; }
+        if constexpr (ONE) *row_out<Operand<T>>(a.out, row, a.ldo, a.cb).at(a.out_off + (h0 + hd) * D + d) = to_operand<Operand<T>>(t * (gates[hd] / s));
+        else part_o[(base * 16 + hd) * D + d] = t;
+        if (!ONE && d == 0) { part_ml[(base * 16 + hd) * 2] = mx; part_ml[(base * 16 + hd) * 2 + 1] = s; }
     }
 }
 // the shares of head h of a row summed, gated and written as operand; a whole block

@@ -467,6 +467,10 @@ struct Parallel : Mixer {
         return 0;
     }
     int run(Pass & p, MixState & st, Operand & o) override;
+    bool one_launch(int act, int rows, int most) const override {
+        auto * kv = dynamic_cast<KvAttention *>(br[0].get()); auto * gl = dynamic_cast<GatedLinear *>(br[1].get());
+        return kv && gl && bamd_kv_gla_one_launch(act, kv->a, gl->a, rows, most);
+    }
     double step_bytes(int len) const override { double t = 0; for (auto & b : br) t += b->step_bytes(len); return t; }
     int f32_cols() const override { int n = 0; for (auto & b : br) n = std::max(n, b->f32_cols()); return n; }
     int prompt_rows(int act) const override { int n = 0; for (auto & b : br) if (const int q = b->prompt_rows(act)) n = n ? std::min(n, q) : q; return n; }
@@ -751,7 +755,10 @@ int Parallel::run(Pass & p, MixState & st, Operand & o) {
     o.x = p.c.h; o.ldx = out.K;
     p.begin(1, p.tm ? step_bytes(p.c.seqs[0].len + 1) : 0);
     auto * kv = dynamic_cast<KvAttention *>(br[0].get()); auto * gl = dynamic_cast<GatedLinear *>(br[1].get());
-    if (p.decode && p.b.rows <= (p.st.act == BAMD_ACT_F32 ? PAIR_ROWS_F32 : PAIR_ROWS) && kv && gl) {           // few rows: the branches' blocks share their launches
+    if (p.decode && one_launch(p.st.act, p.b.rows, p.most)) {
+        const bamd_kv_args k = kv->args(p, st.sub[0], ld_of(in), out.K); const bamd_gla_args g = gl->args(p, st.sub[1], ld_of(in), out.K);
+        if (bamd_launch_kv_gla_one(p.st.act, p.b, &k, &g, p.s)) return fail("attention beside gated linear attention: unsupported shape");
+    } else if (p.decode && p.b.rows <= (p.st.act == BAMD_ACT_F32 ? PAIR_ROWS_F32 : PAIR_ROWS) && kv && gl) {           // few rows: the branches' blocks share their launches
         const bamd_kv_args k = kv->args(p, st.sub[0], ld_of(in), out.K);
         if (bamd_launch_kv_gla_decode(p.st.act, p.b, k, gl->args(p, st.sub[1], ld_of(in), out.K), p.c.part_o, p.c.part_ml, kv_splits(k, p.b.rows, p.c.max_pages), p.s)) return fail("attention beside gated linear attention: unsupported shape");
     } else for (size_t i = 0; i < br.size(); ++i) if (br[i]->run(p, st.sub[i], ld_of(in), out.K)) return 1;
@@ -1406,7 +1413,7 @@ BAMD_OP bamd_op_clamped_glu(int act, const float * gate, const float * upv, floa
     HIPC(hipGetLastError());
     return s.operand_back(dh, rows, F, ldh, out);
 }
-// past_k, past_v: what the cache holds in front of the rows (keys as they are cached), [pos0][kv_heads][dim / vdim]; rel: [rel_rows][heads] or null; splits: shares of a decoded row
+// past_k, past_v: what the cache holds in front of the rows (keys as they are cached), [pos0][kv_heads][dim / vdim]; rel: [rel_rows][heads] or null; splits: shares of a decoded row (-1: the step of one launch)
 BAMD_OP bamd_op_kv_attention(int act, const float * q, const float * k, const float * v, const float * gate, int rows, const float * past_k, const float * past_v, int pos0, int heads, int kv_heads, int dim, int vdim,
                              float scale, float cap, float eps, int unit, const float * rel, int rel_rows, int bias_max, int window, int keep, float out_scale, int splits, float * out) {
     OpScratch s; bamd_batch_dev b; bamd_kv_args a; memset((void *) &a, 0, sizeof a);
@@ -1437,7 +1444,8 @@ BAMD_OP bamd_op_kv_attention(int act, const float * q, const float * k, const fl
         s.alloc(&o, (size_t) rows * H * D * 6) || s.alloc((void **) &po, cells * 16 * D * 4) || s.alloc((void **) &pm, cells * 128)) return 1;
     a.in = din; a.bias = db; a.out = o;
     int rc;
-    if (splits) rc = bamd_launch_kv_decode(act, b, a, po, pm, splits, s.l.s);
+    if (splits < 0) rc = bamd_launch_kv_gla_one(act, b, &a, nullptr, s.l.s);
+    else if (splits) rc = bamd_launch_kv_decode(act, b, a, po, pm, splits, s.l.s);
     else { bamd_launch_kv_store(act, b, a, kblk, kr, s.l.s); rc = bamd_launch_kv_prompt(act, b, a, tiles, (int) t.size(), s.l.s); }
     if (rc) return fail("bamd_op_kv_attention: unsupported shape");
     HIPC(hipGetLastError());
@@ -1446,12 +1454,12 @@ BAMD_OP bamd_op_kv_attention(int act, const float * q, const float * k, const fl
     for (int r = 0; r < rows; ++r) for (int h = 0; h < H; ++h) memcpy(out + ((size_t) r * H + h) * vdim, &wide[((size_t) r * H + h) * D], (size_t) vdim * 4);
     return 0;
 }
-// q, k [rows][heads][dim], v, gate [rows][heads][vdim], low [rows][rank], a2 bfloat16 [heads * dim][rank]; state [heads][dim][vdim]; segment: tokens per scan segment (0: one).
-// y: outputs of the recurrence, out: normed and gated
+// q, k [rows][heads][dim], v, gate [rows][heads][vdim], low [rows][rank], a2 bfloat16 [heads * dim][rank]; state [heads][dim][vdim]; segment: tokens per scan segment (0: one; -1: a
+// decoded token, in one launch, which leaves y out).  y: outputs of the recurrence, out: normed and gated
 BAMD_OP bamd_op_gated_linear(int act, const float * q, const float * k, const float * v, const float * gate, const float * low, const uint16_t * a2, const float * a2b, const float * norm, int rows, int pos0, int heads, int dim,
                              int vdim, int rank, float tau, float q_scale, float eps, float out_scale, int segment, float * state, float * y, float * out) {
     OpScratch s; bamd_batch_dev b; bamd_gla_args a; memset((void *) &a, 0, sizeof a);
-    if (!q || !k || !v || !low || !a2 || !a2b || !norm || !state || !y || !out || rows < 1 || heads < 1 || dim < 1 || dim > 256 || vdim < 1 || rank < 1 || rank > 1024 || segment < 0 || s.init(act) || s.one_entry(rows, pos0, b))
+    if (!q || !k || !v || !low || !a2 || !a2b || !norm || !state || !y || !out || rows < 1 || heads < 1 || dim < 1 || dim > 256 || vdim < 1 || rank < 1 || rank > 1024 || segment < -1 || (segment < 0 && rows != 1) || s.init(act) || s.one_entry(rows, pos0, b))
         return fail("bamd_op_gated_linear: bad arguments");
     const int H = heads, Np = up(dim, 4), Pp = up(vdim, 4), ch = H * Np;
     a.q_off = 0; a.k_off = ch; a.v_off = 2 * ch; a.g_off = a.v_off + H * Pp; a.t_off = a.g_off + H * Pp; a.ld = up(a.t_off + rank, 16); a.rank = rank; a.inv_tau = 1.f / tau; a.q_scale = q_scale; a.ldy = H * Pp;
@@ -1474,7 +1482,7 @@ BAMD_OP bamd_op_gated_linear(int act, const float * q, const float * k, const fl
     }
     for (int i = 0; i < vdim; ++i) nm[(size_t) i] = norm[i] * out_scale;
     std::vector<bamd_segment> seg;
-    const int len = segment ? segment : rows;
+    const int len = segment > 0 ? segment : rows;
     for (int t = 0; t < rows; t += len) seg.push_back({ 0, t, std::min(len, rows - t), 0, 0 });
     for (bamd_segment & g : seg) g.last = (int) seg.size() - 1;
     float * din, * ds, * db, * dn, * dy; uint16_t * dw; bamd_segment * dseg; void * o;
@@ -1482,8 +1490,11 @@ BAMD_OP bamd_op_gated_linear(int act, const float * q, const float * k, const fl
         s.alloc((void **) &dy, (size_t) rows * H * Pp * 4) || s.alloc(&o, (size_t) rows * a.ldo * 6) || s.alloc((void **) &a.alpha, (size_t) rows * ch * 4) || s.alloc((void **) &a.seg_state, seg.size() * ch * Pp * 4) ||
         s.alloc((void **) &a.seg_decay, seg.size() * ch * 4)) return 1;
     a.in = din; a.a2 = dw; a.a2b = db; a.norm = dn; a.state = ds; a.y = dy; a.out = o;
-    if (bamd_launch_gla(b, a, rows, dseg, (int) seg.size(), s.l.s)) return fail("bamd_op_gated_linear: unsupported shape");
-    bamd_launch_gla_norm(act, a, rows, s.l.s);
+    if (segment < 0) { HIPC(hipMemsetAsync(dy, 0, (size_t) H * Pp * 4, s.l.s)); if (bamd_launch_kv_gla_one(act, b, nullptr, &a, s.l.s)) return fail("bamd_op_gated_linear: unsupported shape"); }
+    else {
+        if (bamd_launch_gla(b, a, rows, dseg, (int) seg.size(), s.l.s)) return fail("bamd_op_gated_linear: unsupported shape");
+        bamd_launch_gla_norm(act, a, rows, s.l.s);
+    }
     HIPC(hipGetLastError());
     std::vector<float> wy((size_t) rows * H * Pp), wo(wy.size());
     if (s.rows_back(dy, rows, H * Pp, H * Pp, wy.data(), true) || s.operand_back(o, rows, H * Pp, a.ldo, wo.data())) return 1;

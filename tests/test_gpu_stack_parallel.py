@@ -228,6 +228,17 @@ def test_window_attention(bamd, dtype, H, G, d, dv, T, pos0, window, keep):
         near(bamd.op_kv_attention(dtype=dtype, splits=splits, **a).reshape(T, -1), want, dtype)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H,G,d,dv", [(1, 1, 8, 8), (6, 2, 24, 40), (34, 2, 16, 32), (4, 4, 72, 128), (8, 2, 128, 64)])
+@pytest.mark.parametrize("pos0,window,keep", [(0, 5, 2), (1, 1, 0), (31, 100, 0), (63, 10, 3), (64, 64, 64), (255, 1 << 20, 0), (300, 63, 70), (513, 1 << 20, 0), (900, 700, 4)])
+def test_window_attention_step_in_one_launch(bamd, dtype, H, G, d, dv, pos0, window, keep):
+    """no key but the row's own, fewer half pages than waves, as many, more, and a share of them empty; groups of one, three, four and seventeen heads"""
+    a = case(dtype, H, G, d, dv, 1, pos0, window, keep)
+    near(bamd.op_kv_attention(dtype=dtype, splits=-1, out_scale=-0.7, **a).reshape(1, -1), -0.7 * plain(a, 1).reshape(1, -1), dtype)
+    a["gate"] = None
+    near(bamd.op_kv_attention(dtype=dtype, splits=-1, **a).reshape(1, -1), plain(a, 1).reshape(1, -1), dtype)
+
+
 @pytest.mark.parametrize("H,G,d,T,window", [(128, 8, 24, 257, 100), (128, 32, 24, 512, 1000), (128, 4, 24, 513, 70), (85, 5, 40, 700, 130)])
 def test_window_attention_in_paired_blocks(bamd, H, G, d, T, window):
     """tiles of 128 queries: one block per CU and a part of a second, two, two and a part of a third, and heads that do not divide the CUs"""
@@ -352,6 +363,21 @@ def test_gated_linear(bamd, H, d, dv, R):
         assert rel(gy, y) < 1e-5 and rel(gs, S) < 1e-5, pos
         assert np.abs(go - out).max() < (3e-4 if dv < 4 else 1e-4) * (1 + np.abs(out).max()), pos      # (a norm over few columns magnifies)
         pos += n
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H,d,dv,R", [(1, 1, 1, 1), (3, 10, 14, 5), (2, 64, 64, 3), (5, 66, 60, 16), (2, 60, 65, 17), (3, 128, 128, 16), (40, 24, 16, 2)])
+def test_gated_linear_step_in_one_launch(bamd, H, d, dv, R, dtype):
+    """a fresh state, then one that tokens left: the state's bits are those of two launches"""
+    a = gla_case(H, d, dv, R, 4, H * d + dv)
+    S, gs = np.zeros((H, d, dv)), np.full((H, d, dv), 7, np.float32)
+    for t in range(4):
+        _, out, S = plain_gla(a, S, t, t + 1)
+        _, _, two = bamd.op_gated_linear(pos0=t, state=gs, dtype=dtype, **part(a, t, t + 1))
+        _, go, gs = bamd.op_gated_linear(pos0=t, state=gs, dtype=dtype, out_scale=-0.6, segment=-1, **part(a, t, t + 1))
+        assert np.array_equal(gs.view(np.uint32), two.view(np.uint32)) and rel(gs, S) < 1e-5
+        e = np.abs(go + 0.6 * out)
+        assert (e <= (3e-4 if dv < 4 else 1e-4) * (1 + np.abs(out).max()) + (2.0 ** -8 if dtype == "bfloat16" else 0) * np.abs(out)).all(), t      # (as above, and the result's own rounding)
 
 
 @pytest.mark.parametrize("H,d,dv", [(2, 20, 24), (1, 130, 70), (3, 64, 16)])
