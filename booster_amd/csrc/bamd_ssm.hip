@@ -4,6 +4,7 @@
 //   decoding (one token): ssm_step_kernel, a block per (PT value columns, head, sequence), filters its own channels, one launch in all.  A lane keeps four columns of NPL state
 //     rows in registers (lane = column quad + group of state rows, so that a row's B and C serve four columns from one LDS read); y is summed over a lane's rows, then over the groups.
 // The state is read and written once per step; everything is 32-bit.
+#include <algorithm>
 #include "bamd_dense_device.h"
 #include <type_traits>
 
@@ -180,15 +181,26 @@ __global__ void __launch_bounds__(256) ssm_step_kernel(bamd_batch_dev b, bamd_ss
 // The products meet a later token's B, C and x with a factor of zero, which hides any finite value; an infinity, a NaN or a product that overflows shows as a y that is not finite.  Then the
 // wave takes the chunk again one token after the other, from the state in front of it, so that such a token reaches those behind it and none in front.  (A look at every value on
 // its way into LDS instead cost 264 us for 258; this one, under the stores of y, nothing.)
+// A prompt of few heads leaves CUs idle, and tokens one behind the other are its time: up to four parts of its tokens are taken at once, each by a block of its own, which brings the state along from the
+// first token on without the outputs (half a chunk's time) and so gets the bits that one block gets.  Borders are where all parts end together.  Four layers, us, one part and those taken: width 2048
+// (64 heads, two parts) 131 tokens 573 | 567, 1000 1228 | 1164, 2048 2051 | 1907; 1024 (32 heads, four) 300 473 | 448, 2048 1410 | 1217; 600 (13 heads) 1000 723 | 621.  Two parts to a CU (128 heads) were
+// no faster (2048 tokens of width 4096 4268 | 4271), and the registers that takes cost 2 %
+#define SSM_AGAIN 0.55f                             /* a chunk whose outputs are taken costs 1, one that only brings the state along 1 - this */
 template <int NT>
-__global__ void __launch_bounds__(512) ssm_chunk_kernel(bamd_batch_dev b, bamd_ssm_args a) {
+__global__ void __launch_bounds__(512) ssm_chunk_kernel(bamd_batch_dev b, bamd_ssm_args a, int cols) {
     constexpr int NQ = 4, NP = 16 * NQ * NT, LB = NP + 4, LX = 36, LD = 20, PF = 16 * NP / 512, KS = 512 / NP;      // row lengths in LDS: four rows on, 16 banks on
     __shared__ __align__(16) float Bs[2][16 * LB], Cs[2][16 * LB], xs[2][16 * LX], yp[2][NQ][16 * LX], dm[2][16 * LD];
     __shared__ __align__(16) float pre[2][16], fd[2][16], dts[2][16];
     const bamd_entry e = b.ent[blockIdx.z];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 15, q = lane >> 4, ct = wave & 1, part = wave >> 1;
-    const int h = blockIdx.y, p0 = blockIdx.x * 32, pw = min(32, a.P - p0), N = a.N, inner = a.heads * a.P, ch = inner + 2 * a.groups * N, g = h / (a.heads / a.groups);
+    const int h = blockIdx.y, p0 = (int) blockIdx.x % cols * 32, pw = min(32, a.P - p0), N = a.N, inner = a.heads * a.P, ch = inner + 2 * a.groups * N, g = h / (a.heads / a.groups);
     const int n0 = part * NT * 16;                                 // first state row of this wave
+    // this block's tokens [from, to).  The state in front of a part comes from a state that is fresh: one that a pass before left is where the last part's goes
+    const int parts = e.pos0 > 0 ? 1 : (int) gridDim.x / cols, at = (int) blockIdx.x / cols, chunks = (e.n + 15) / 16;
+    if (at >= parts) return;
+    auto border = [&](int k) { return k >= parts ? e.n : min(chunks - 1, (int) ((float) chunks * (1.f - __builtin_powif(SSM_AGAIN, k)) / (1.f - __builtin_powif(SSM_AGAIN, parts)) + 0.5f)) * 16; };
+    const int from = border(at), to = border(at + 1);              // (inner borders lie in front of the last chunk: no part reaches behind the tokens, and the last is never empty)
+    if (from >= to) return;
     float * st = a.state + (((size_t) e.seq * a.heads + h) * N) * a.P + p0;
     bamd_v4 S[NT];
 #pragma unroll
@@ -201,21 +213,23 @@ __global__ void __launch_bounds__(512) ssm_chunk_kernel(bamd_batch_dev b, bamd_s
     float bf[2][PF], cf[2][PF], xf[2], zf[2], fdt[2], fdec[2];
     const int kn = tid % NP, kt = tid / NP, xc = tid & 31, xt = tid >> 5;
     const uint32_t kb = (uint32_t) (inner + g * N + min(kn, N - 1)), kc = kb + (uint32_t) (a.groups * N), xo = (uint32_t) (h * a.P + p0 + min(xc, pw - 1));
-    auto request = [&](int t0, auto par) {
-        constexpr int R = decltype(par)::value;
-        const int nt = e.n - t0;
+    int end = to;                                                  // of the tokens that are gone through now
+    auto request = [&](int t0, auto par, auto full) {
+        constexpr int R = decltype(par)::value; constexpr bool F = decltype(full)::value;
+        const int nt = end - t0;
         if (nt <= 0) return;
         const float * f = a.filtered + (size_t) (e.row0 + t0) * ch, * z = a.in + (size_t) (e.row0 + t0) * a.ld;
         if (nt >= 16) {
             const uint32_t r = (uint32_t) (kt * ch);
 #pragma unroll
-            for (int i = 0; i < PF; ++i) { const float * fi = f + (size_t) (i * KS) * ch; bf[R][i] = fi[r + kb]; cf[R][i] = fi[r + kc]; }
+            for (int i = 0; i < PF; ++i) { const float * fi = f + (size_t) (i * KS) * ch; bf[R][i] = fi[r + kb]; if constexpr (F) cf[R][i] = fi[r + kc]; }
         } else {
 #pragma unroll
-            for (int i = 0; i < PF; ++i) { const uint32_t r = (uint32_t) (min(kt + i * KS, nt - 1) * ch); bf[R][i] = f[r + kb]; cf[R][i] = f[r + kc]; }
+            for (int i = 0; i < PF; ++i) { const uint32_t r = (uint32_t) (min(kt + i * KS, nt - 1) * ch); bf[R][i] = f[r + kb]; if constexpr (F) cf[R][i] = f[r + kc]; }
         }
         const int t = min(xt, nt - 1);
-        xf[R] = f[(uint32_t) (t * ch) + xo]; zf[R] = z[(uint32_t) (t * a.ld) + xo];
+        xf[R] = f[(uint32_t) (t * ch) + xo];
+        if constexpr (F) zf[R] = z[(uint32_t) (t * a.ld) + xo];
         const float * p = a.steps + ((size_t) (e.row0 + t0 + min(col, nt - 1)) * a.heads + h) * 2;
         fdt[R] = col < nt ? p[0] : 0.f; fdec[R] = col < nt ? p[1] : 1.f;
     };
@@ -225,14 +239,14 @@ __global__ void __launch_bounds__(512) ssm_chunk_kernel(bamd_batch_dev b, bamd_s
         v *= moved(v, std::integral_constant<int, 0x111>()); v *= moved(v, std::integral_constant<int, 0x112>());
         v *= moved(v, std::integral_constant<int, 0x114>()); return v * moved(v, std::integral_constant<int, 0x118>());
     };
-    auto put = [&](int nt, auto par) {                             // nt: the chunk's tokens and those behind
-        constexpr int w = decltype(par)::value;
+    auto put = [&](int nt, auto par, auto full) {                  // nt: the chunk's tokens and those behind
+        constexpr int w = decltype(par)::value; constexpr bool F = decltype(full)::value;
         if (nt >= 16 && N == NP) {
 #pragma unroll
-            for (int i = 0; i < PF; ++i) { Bs[w][(kt + i * KS) * LB + kn] = bf[w][i]; Cs[w][(kt + i * KS) * LB + kn] = cf[w][i]; }
+            for (int i = 0; i < PF; ++i) { Bs[w][(kt + i * KS) * LB + kn] = bf[w][i]; if constexpr (F) Cs[w][(kt + i * KS) * LB + kn] = cf[w][i]; }
         } else {
 #pragma unroll
-            for (int i = 0; i < PF; ++i) { const bool in = kn < N && kt + i * KS < nt; Bs[w][(kt + i * KS) * LB + kn] = in ? bf[w][i] : 0.f; Cs[w][(kt + i * KS) * LB + kn] = in ? cf[w][i] : 0.f; }
+            for (int i = 0; i < PF; ++i) { const bool in = kn < N && kt + i * KS < nt; Bs[w][(kt + i * KS) * LB + kn] = in ? bf[w][i] : 0.f; if constexpr (F) Cs[w][(kt + i * KS) * LB + kn] = in ? cf[w][i] : 0.f; }
         }
         xf[w] = xc < pw && xt < nt ? xf[w] : 0.f;
         xs[w][xt * LX + xc] = xf[w];
@@ -249,14 +263,50 @@ __global__ void __launch_bounds__(512) ssm_chunk_kernel(bamd_batch_dev b, bamd_s
             if (lane < 16) { dts[w][lane] = fdt[w]; pre[w][lane] = p; fd[w][lane] = f * fdt[w]; }
         }
     };
-    request(0, std::integral_constant<int, 0>()); request(16, std::integral_constant<int, 1>());
-    put(e.n, std::integral_constant<int, 0>());
-    __syncthreads();
+    // whole: outputs and state; the state alone is what a later part of the tokens starts from, in the same bits
+    const std::integral_constant<bool, true> whole; const std::integral_constant<bool, false> state_only;
+    auto state_chunk = [&](int t0, auto par) {
+        constexpr int w = decltype(par)::value;
+        const int nt = end - t0;
+        request(t0 + 32, par, state_only);
+        bamd_v4 T[NT];
+        float ba[NT][4], xw[4], sum = 0.f;
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) ba[j][i] = Bs[w][(q * 4 + i) * LB + n0 + j * 16 + col];
+        const bamd_v4 f4 = *(const bamd_v4 *) &fd[w][q * 4];
+        const float all = pre[w][15];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) xw[i] = xs[w][(q * 4 + i) * LX + ct * 16 + col] * f4[i];
+        if (nt > 16) put(nt - 16, std::integral_constant<int, w ^ 1>(), state_only);
+#pragma unroll
+        for (int j = 0; j < NT; ++j) T[j] = S[j] * all;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) T[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ba[j][i], xw[i], T[j], 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < NT; ++j) sum += (T[j][0] + T[j][1]) + (T[j][2] + T[j][3]);
+        if (!__any(!(fabsf(sum) < INFINITY))) {
+#pragma unroll
+            for (int j = 0; j < NT; ++j) S[j] = T[j];
+        } else for (int t = 0; t < 16; ++t) {
+            const float d = t ? dm[w][t * LD + t - 1] : pre[w][0], xv = dts[w][t] * xs[w][t * LX + ct * 16 + col];
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                const bamd_v4 B = *(const bamd_v4 *) &Bs[w][t * LB + n0 + j * 16 + q * 4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) S[j][i] = fmaf(d, S[j][i], B[i] * xv);
+            }
+        }
+        __syncthreads();
+    };
     auto chunk = [&](int t0, auto par) {
         constexpr int w = decltype(par)::value;
-        const int nt = e.n - t0;
+        const int nt = end - t0;
         const float xk = xf[w], zk = zf[w];
-        request(t0 + 32, par);
+        request(t0 + 32, par, whole);
         bamd_v4 cr[NT], br[NT], gt = { 0, 0, 0, 0 }, g2 = { 0, 0, 0, 0 }, y = { 0, 0, 0, 0 }, y2 = { 0, 0, 0, 0 };
         bamd_v4 T[NT];                                                // the state behind the chunk
         float ba[NT][4], xw[4], xd[4];
@@ -270,7 +320,7 @@ __global__ void __launch_bounds__(512) ssm_chunk_kernel(bamd_batch_dev b, bamd_s
         const float all = pre[w][15];
 #pragma unroll
         for (int i = 0; i < 4; ++i) { const float x = xs[w][(q * 4 + i) * LX + ct * 16 + col]; xd[i] = x * d4[i]; xw[i] = x * f4[i]; }
-        if (nt > 16) put(nt - 16, std::integral_constant<int, w ^ 1>());       // (requested a chunk ago; its place was read before the last barrier)
+        if (nt > 16) put(nt - 16, std::integral_constant<int, w ^ 1>(), whole);       // (requested a chunk ago; its place was read before the last barrier)
 #pragma unroll
         for (int j = 0; j < NT; ++j)
 #pragma unroll
@@ -311,7 +361,20 @@ __global__ void __launch_bounds__(512) ssm_chunk_kernel(bamd_batch_dev b, bamd_s
         const int o = xt * LX + xc;
         if (xt < nt && xc < pw) a.out[(size_t) (e.row0 + t0 + xt) * a.ldo + h * a.P + p0 + xc] = ((yp[w][0][o] + yp[w][1][o]) + (yp[w][2][o] + yp[w][3][o]) + D * xk) * silu_f(zk);
     };
-    for (int t0 = 0; t0 < e.n; t0 += 32) { chunk(t0, std::integral_constant<int, 0>()); if (t0 + 16 < e.n) chunk(t0 + 16, std::integral_constant<int, 1>()); }
+    const std::integral_constant<int, 0> even; const std::integral_constant<int, 1> odd;
+    if (from > 0) {
+        end = from;
+        request(0, even, state_only); request(16, odd, state_only);
+        put(end, even, state_only);
+        __syncthreads();
+        for (int t0 = 0; t0 < end; t0 += 32) { state_chunk(t0, even); if (t0 + 16 < end) state_chunk(t0 + 16, odd); }
+        end = to;
+    }
+    request(from, even, whole); request(from + 16, odd, whole);
+    put(end - from, even, whole);
+    __syncthreads();
+    for (int t0 = from; t0 < end; t0 += 32) { chunk(t0, even); if (t0 + 16 < end) chunk(t0 + 16, odd); }
+    if (at + 1 < parts) return;
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
@@ -342,10 +405,12 @@ int bamd_launch_ssm(const bamd_batch_dev & b, const bamd_ssm_args & a, int max_n
         return 0;
     }
     if (!a.filtered || !a.steps) return 1;
-    const dim3 cg((ch + 255) / 256, (b.rows + SSM_STRIP - 1) / SSM_STRIP), grid((a.P + 31) / 32, a.heads, b.n_entries);
+    const int cols = (a.P + 31) / 32, blocks = cols * a.heads * b.n_entries;
+    const int parts = max_n < 64 ? 1 : std::max(1, std::min(4, 256 / blocks));      // (of fewer tokens they are level)
+    const dim3 cg((ch + 255) / 256, (b.rows + SSM_STRIP - 1) / SSM_STRIP), grid(cols * parts, a.heads, b.n_entries);
     if (a.taps == 4) hipLaunchKernelGGL(ssm_conv_kernel<true>, cg, dim3(256), 0, s, b, a); else hipLaunchKernelGGL(ssm_conv_kernel<false>, cg, dim3(256), 0, s, b, a);
-    if (a.N <= 64) hipLaunchKernelGGL(ssm_chunk_kernel<1>, grid, dim3(512), 0, s, b, a);
-    else if (a.N <= 128) hipLaunchKernelGGL(ssm_chunk_kernel<2>, grid, dim3(512), 0, s, b, a);
-    else hipLaunchKernelGGL(ssm_chunk_kernel<4>, grid, dim3(512), 0, s, b, a);
+    if (a.N <= 64) hipLaunchKernelGGL(ssm_chunk_kernel<1>, grid, dim3(512), 0, s, b, a, cols);
+    else if (a.N <= 128) hipLaunchKernelGGL(ssm_chunk_kernel<2>, grid, dim3(512), 0, s, b, a, cols);
+    else hipLaunchKernelGGL(ssm_chunk_kernel<4>, grid, dim3(512), 0, s, b, a, cols);
     return 0;
 }

@@ -432,6 +432,50 @@ def test_ssm_tokens_that_are_not_finite(bamd, N, at, what, value):
         assert not ok.any() or rel(got[t][ok], want[t][ok]) < 2e-5, t                # as test_ssm
 
 
+@pytest.mark.parametrize("H,P,N,G", [(2, 40, 40, 1), (1, 31, 200, 1), (80, 10, 12, 2), (43, 33, 65, 1), (65, 40, 8, 1)])
+@pytest.mark.parametrize("n", [63, 64, 65, 100, 257])
+def test_ssm_prompts_in_parts(bamd, H, P, N, G, n):
+    """fresh prompts whose tokens are taken in four parts, three, two and one, last chunks of one token and of sixteen; a portion behind them starts from their state"""
+    r = np.random.default_rng(H * P + N + n)
+    inner, ch = H * P, H * P + 2 * G * N
+    f = lambda a: np.asarray(a, np.float32)
+    conv, cb, dtb, A, D = map(f, (r.standard_normal((ch, 4)), r.standard_normal(ch) * 0.3, r.uniform(-6, 1, H), r.uniform(-4, 3, H), r.standard_normal(H)))
+    rows = f(r.standard_normal((n + 70, inner + ch + H)))
+    rows[::9, -H:] -= 30
+    hist, S = np.zeros((3, ch)), np.zeros((H, N, P))
+    gh, gs = f(hist), f(S) + 7
+    for pos, end in ((0, n), (n, n + 70)):
+        want, hist, S = plain_ssm(rows[pos:end].astype(np.float64), H, P, N, G, conv, cb, dtb, A, D, hist, S)
+        got, gh, gs = bamd.op_ssm(rows[pos:end], pos, H, P, N, G, conv, cb, dtb, A, D, gh, gs)
+        assert rel(got, want) < 2e-5 and rel(gs, S) < 2e-5, pos      # as test_ssm
+
+
+@pytest.mark.parametrize("N,at", [(40, 0), (128, 3), (200, 17), (40, 47), (128, 60), (40, 110)])
+@pytest.mark.parametrize("what,value", [("x", np.inf), ("x", np.nan), ("B", np.inf), ("C", np.nan), ("dt", np.inf), ("far", 1e20)])
+def test_ssm_tokens_that_are_not_finite_in_parts(bamd, N, at, what, value):
+    """a token that the parts behind it meet on their way to a state, or that no part does"""
+    H, P, n = 2, 40, 130
+    r = np.random.default_rng(N + at)
+    inner, ch = H * P, H * P + 2 * N
+    f = lambda a: np.asarray(a, np.float32)
+    conv, cb, dtb, A, D = map(f, (r.uniform(0.5, 2, (ch, 1)), np.zeros(ch), r.uniform(-2, 1, H), r.uniform(-2, 1, H), r.standard_normal(H)))
+    rows = f(r.standard_normal((n, inner + ch + H)))
+    x, B, C = inner + P + 33, 2 * inner + N // 2, 2 * inner + N + 1                  # a column of the second head, a state row of both
+    if what == "far":
+        rows[at, 2 * inner + N + N // 2] = rows[at + 1, B] = value
+    else:
+        rows[at, {"x": x, "B": B, "C": C, "dt": -1}[what]] = value
+    with np.errstate(all="ignore"):
+        want, _, S = plain_ssm(rows.astype(np.float64), H, P, N, 1, conv, cb, dtb, A, D, np.zeros((0, ch)), np.zeros((H, N, P)))
+    got, _, gs = bamd.op_ssm(rows, 0, H, P, N, 1, conv, cb, dtb, A, D, np.zeros((0, ch)), np.zeros((H, N, P), np.float32))
+    assert np.isfinite(want[:at]).all() and (what == "far" or not np.isfinite(want).all())
+    assert np.array_equal(np.isfinite(gs), np.isfinite(S))
+    for t in range(n):
+        ok = np.isfinite(want[t])
+        assert (np.isfinite(got[t]) == ok).all(), t
+        assert not ok.any() or rel(got[t][ok], want[t][ok]) < 2e-5, t                # as test_ssm
+
+
 def plain_attention(q, c, gate, past, uk, uv, c_norm, sink, scale, eps, H):
     T, _, d = q.shape
     lat = np.stack([so.rms(v, eps) * c_norm for v in c])
