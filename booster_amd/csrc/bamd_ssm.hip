@@ -186,8 +186,9 @@ __global__ void __launch_bounds__(256) ssm_step_kernel(bamd_batch_dev b, bamd_ss
 // (64 heads, two parts) 131 tokens 573 | 567, 1000 1228 | 1164, 2048 2051 | 1907; 1024 (32 heads, four) 300 473 | 448, 2048 1410 | 1217; 600 (13 heads) 1000 723 | 621.  Two parts to a CU (128 heads) were
 // no faster (2048 tokens of width 4096 4268 | 4271), and the registers that takes cost 2 %
 #define SSM_AGAIN 0.55f                             /* a chunk whose outputs are taken costs 1, one that only brings the state along 1 - this */
+struct ssm_cut { float at[3]; };                   // inner borders, of all tokens
 template <int NT>
-__global__ void __launch_bounds__(512) ssm_chunk_kernel(bamd_batch_dev b, bamd_ssm_args a, int cols) {
+__global__ void __launch_bounds__(512) ssm_chunk_kernel(bamd_batch_dev b, bamd_ssm_args a, int cols, ssm_cut cut) {
     constexpr int NQ = 4, NP = 16 * NQ * NT, LB = NP + 4, LX = 36, LD = 20, PF = 16 * NP / 512, KS = 512 / NP;      // row lengths in LDS: four rows on, 16 banks on
     __shared__ __align__(16) float Bs[2][16 * LB], Cs[2][16 * LB], xs[2][16 * LX], yp[2][NQ][16 * LX], dm[2][16 * LD];
     __shared__ __align__(16) float pre[2][16], fd[2][16], dts[2][16];
@@ -198,7 +199,7 @@ __global__ void __launch_bounds__(512) ssm_chunk_kernel(bamd_batch_dev b, bamd_s
     // this block's tokens [from, to).  The state in front of a part comes from a state that is fresh: one that a pass before left is where the last part's goes
     const int parts = e.pos0 > 0 ? 1 : (int) gridDim.x / cols, at = (int) blockIdx.x / cols, chunks = (e.n + 15) / 16;
     if (at >= parts) return;
-    auto border = [&](int k) { return k >= parts ? e.n : min(chunks - 1, (int) ((float) chunks * (1.f - __builtin_powif(SSM_AGAIN, k)) / (1.f - __builtin_powif(SSM_AGAIN, parts)) + 0.5f)) * 16; };
+    auto border = [&](int k) { return k == 0 ? 0 : k >= parts ? e.n : min(chunks - 1, (int) ((float) chunks * (k == 1 ? cut.at[0] : k == 2 ? cut.at[1] : cut.at[2]) + 0.5f)) * 16; };
     const int from = border(at), to = border(at + 1);              // (inner borders lie in front of the last chunk: no part reaches behind the tokens, and the last is never empty)
     if (from >= to) return;
     float * st = a.state + (((size_t) e.seq * a.heads + h) * N) * a.P + p0;
@@ -407,10 +408,12 @@ int bamd_launch_ssm(const bamd_batch_dev & b, const bamd_ssm_args & a, int max_n
     if (!a.filtered || !a.steps) return 1;
     const int cols = (a.P + 31) / 32, blocks = cols * a.heads * b.n_entries;
     const int parts = max_n < 64 ? 1 : std::max(1, std::min(4, 256 / blocks));      // (of fewer tokens they are level)
+    ssm_cut cut = { { 1.f, 1.f, 1.f } };
+    for (int k = 1; k < parts; ++k) cut.at[k - 1] = (1.f - powf(SSM_AGAIN, (float) k)) / (1.f - powf(SSM_AGAIN, (float) parts));
     const dim3 cg((ch + 255) / 256, (b.rows + SSM_STRIP - 1) / SSM_STRIP), grid(cols * parts, a.heads, b.n_entries);
     if (a.taps == 4) hipLaunchKernelGGL(ssm_conv_kernel<true>, cg, dim3(256), 0, s, b, a); else hipLaunchKernelGGL(ssm_conv_kernel<false>, cg, dim3(256), 0, s, b, a);
-    if (a.N <= 64) hipLaunchKernelGGL(ssm_chunk_kernel<1>, grid, dim3(512), 0, s, b, a, cols);
-    else if (a.N <= 128) hipLaunchKernelGGL(ssm_chunk_kernel<2>, grid, dim3(512), 0, s, b, a, cols);
-    else hipLaunchKernelGGL(ssm_chunk_kernel<4>, grid, dim3(512), 0, s, b, a, cols);
+    if (a.N <= 64) hipLaunchKernelGGL(ssm_chunk_kernel<1>, grid, dim3(512), 0, s, b, a, cols, cut);
+    else if (a.N <= 128) hipLaunchKernelGGL(ssm_chunk_kernel<2>, grid, dim3(512), 0, s, b, a, cols, cut);
+    else hipLaunchKernelGGL(ssm_chunk_kernel<4>, grid, dim3(512), 0, s, b, a, cols, cut);
     return 0;
 }
