@@ -651,11 +651,12 @@ int bamd_prefill_mfma_supported(void) {
 // Token tiles (of 16) per block of the few-token kernel for this product, 0: one of the kernels with 64-row blocks.
 // Up to 64 tokens: whichever ends first.  Both take a start and a time per super-block, for every round of 256 blocks; the few-token kernel's goes by its token tiles.  Constants in ns,
 // fitted to 1323 sizes (three types, 8 to 64 tokens, 1024 to 24576 rows, K 1024 to 14336) with all records of the tiles copied: with fewer tokens the few-token kernel is faster than they say.
+// Q4_K with 33 to 48 tokens took 530 or 640 a step, by how the records lay to the lines; 572 keeps the sizes where those two were level (two rounds at K = 3840 and 4096) on the sides they were measured on.
 // Where the two part, K = 4096, 64-row blocks against 16-row ones in us: 8192 rows Q4_K 32 tokens 24.1 | 18.4, 48 tokens 24.0 | 22.7, 64 tokens 24.1 | 25.5; 12288 rows 32 tokens 25.2 | 27.9;
 // Q6_K 8192 rows 64 tokens 34.7 | 31.2
 struct x_cost { int start64, step64, extra, start[3], step[3]; };      // extra: what the few-token kernel's launch takes more, whatever its rounds
 static int x_few_tiles(int type, int nrows_pad, int nb, int T) {
-    static const x_cost costs[3] = { { 3010, 1300, 1150, { 1790, 2140, 2400 }, { 410, 530, 590 } },         // Q4_K
+    static const x_cost costs[3] = { { 3010, 1300, 1150, { 1790, 2140, 2400 }, { 410, 572, 590 } },         // Q4_K
                                      { 3410, 1240, 1800, { 1900, 2180, 2600 }, { 416, 520, 580 } },         // Q5_K
                                      { 3590, 1815, 1150, { 2040, 2400, 2740 }, { 680, 710, 750 } } };       // Q6_K
     if (T > 64) return 0;
