@@ -419,6 +419,28 @@ def test_head_norm_and_gate(bamd, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H,d,dv", [(6, 64, 65), (7, 20, 30), (2, 100, 128)])
+@pytest.mark.parametrize("rows", [1, 3, 9])
+def test_steps_that_outgrow_one_launch(bamd, dtype, H, d, dv, rows, tmp_path):
+    """sequences of different lengths around 224 and 448 positions, the most that one launch takes: the same graph key before, another behind"""
+    cfg = stack_cases.mafurax(64, 97, [stack_cases.parallel(stack_cases.attend(4, 2, 24, 20, 0.4, 6.0, 50, 1 << 20, 0), 0.7, (H, d, dv, 8.0), 1.3, ff=80, limit=0.8)])
+    case = Case(str(tmp_path / "m"), cfg, 3, dict(rel=8, rank=5))
+    m = bamd.Model(case.folder, dtype=dtype)
+    c = bamd.Context(m, 64 * 8 * rows, rows)
+    for most in (224, 448):
+        t = [tokens(cfg, most + 6, 30 + i) for i in range(min(rows, 3))]
+        want = [case.logits(x) for x in t]
+        at = [most - 4 - 30 * (s % 3) for s in range(rows)]
+        for s in range(rows): c.seq_free(s)
+        c.decode_batch([(s, t[s % 3][:at[s]], [at[s] - 1]) for s in range(rows)])
+        for _ in range(8):
+            got = c.decode_batch([(s, [t[s % 3][at[s]]], [0]) for s in range(rows)])
+            near(got, np.stack([want[s % 3][at[s]] for s in range(rows)]), dtype)
+            at = [a + 1 for a in at]
+    c.close(); m.close()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("H,d,dv,steps", [(3, 130, 70, (2, 21, 22, 42, 43, 64, 65)), (6, 64, 65, (5, 11, 22)), (7, 20, 30, (19, 37)), (2, 100, 9, (6, 64))])
 def test_decoding_rows_that_share_launches(bamd, dtype, H, d, dv, steps, tmp_path):
     """a step of that many sequences, whose recurrence takes 16, 32 or 64 columns a block; beyond 64 rows (48 in 32-bit) the branches have their own launches"""
