@@ -114,6 +114,7 @@ struct bamd_ssm_args {
     int heads, P, N, groups, taps;
 };
 int bamd_launch_ssm(const bamd_batch_dev & b, const bamd_ssm_args & a, int max_n, hipStream_t s);
+int bamd_ssm_chunk_blocks(int N, int parts);       // blocks of a prompt's scan per CU
 
 // ---- latent attention ------------------------------------------------------------------------------------------------------------------------------
 struct bamd_latent_args {

@@ -184,20 +184,21 @@ __global__ void __launch_bounds__(256) ssm_step_kernel(bamd_batch_dev b, bamd_ss
 // A prompt of few heads leaves CUs idle, and tokens one behind the other are its time: up to four parts of its tokens are taken at once, each by a block of its own, which brings the state along from the
 // first token on without the outputs (half a chunk's time) and so gets the bits that one block gets.  Borders are where all parts end together.  Four layers, us, one part and those taken: width 2048
 // (64 heads, two parts) 131 tokens 573 | 567, 1000 1228 | 1164, 2048 2051 | 1907; 1024 (32 heads, four) 300 473 | 448, 2048 1410 | 1217; 600 (13 heads) 1000 723 | 621.  Two parts to a CU (128 heads) were
-// no faster (2048 tokens of width 4096 4268 | 4271), and the registers that takes cost 2 %
+// no faster (2048 tokens of width 4096 4268 | 4271).  All these are state 128.  Tokens in one part have an instance of their own: with the parts' code in it a state of up to 64 takes 130 registers for
+// 128, one block per CU for two.  Eight prompts of 330 to 186 tokens, width 2048, state 64, 2320 us with, 2231 without, state 32 2312 | 2220; width 4096 (128 heads), two prompts of 900 and 675 3804 | 3700
 #define SSM_AGAIN 0.55f                             /* a chunk whose outputs are taken costs 1, one that only brings the state along 1 - this */
 struct ssm_cut { float at[3]; };                   // inner borders, of all tokens
-template <int NT>
+template <int NT, bool PARTS>
 __global__ void __launch_bounds__(512) ssm_chunk_kernel(bamd_batch_dev b, bamd_ssm_args a, int cols, ssm_cut cut) {
     constexpr int NQ = 4, NP = 16 * NQ * NT, LB = NP + 4, LX = 36, LD = 20, PF = 16 * NP / 512, KS = 512 / NP;      // row lengths in LDS: four rows on, 16 banks on
     __shared__ __align__(16) float Bs[2][16 * LB], Cs[2][16 * LB], xs[2][16 * LX], yp[2][NQ][16 * LX], dm[2][16 * LD];
     __shared__ __align__(16) float pre[2][16], fd[2][16], dts[2][16];
     const bamd_entry e = b.ent[blockIdx.z];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 15, q = lane >> 4, ct = wave & 1, part = wave >> 1;
-    const int h = blockIdx.y, p0 = (int) blockIdx.x % cols * 32, pw = min(32, a.P - p0), N = a.N, inner = a.heads * a.P, ch = inner + 2 * a.groups * N, g = h / (a.heads / a.groups);
+    const int h = blockIdx.y, p0 = (PARTS ? (int) blockIdx.x % cols : (int) blockIdx.x) * 32, pw = min(32, a.P - p0), N = a.N, inner = a.heads * a.P, ch = inner + 2 * a.groups * N, g = h / (a.heads / a.groups);
     const int n0 = part * NT * 16;                                 // first state row of this wave
     // this block's tokens [from, to).  The state in front of a part comes from a state that is fresh: one that a pass before left is where the last part's goes
-    const int parts = e.pos0 > 0 ? 1 : (int) gridDim.x / cols, at = (int) blockIdx.x / cols, chunks = (e.n + 15) / 16;
+    const int parts = !PARTS || e.pos0 > 0 ? 1 : (int) gridDim.x / cols, at = PARTS ? (int) blockIdx.x / cols : 0, chunks = (e.n + 15) / 16;
     if (at >= parts) return;
     auto border = [&](int k) { return k == 0 ? 0 : k >= parts ? e.n : min(chunks - 1, (int) ((float) chunks * (k == 1 ? cut.at[0] : k == 2 ? cut.at[1] : cut.at[2]) + 0.5f)) * 16; };
     const int from = border(at), to = border(at + 1);              // (inner borders lie in front of the last chunk: no part reaches behind the tokens, and the last is never empty)
@@ -363,7 +364,7 @@ __global__ void __launch_bounds__(512) ssm_chunk_kernel(bamd_batch_dev b, bamd_s
         if (xt < nt && xc < pw) a.out[(size_t) (e.row0 + t0 + xt) * a.ldo + h * a.P + p0 + xc] = ((yp[w][0][o] + yp[w][1][o]) + (yp[w][2][o] + yp[w][3][o]) + D * xk) * silu_f(zk);
     };
     const std::integral_constant<int, 0> even; const std::integral_constant<int, 1> odd;
-    if (from > 0) {
+    if (PARTS && from > 0) {
         end = from;
         request(0, even, state_only); request(16, odd, state_only);
         put(end, even, state_only);
@@ -393,6 +394,11 @@ template <int PT, bool FOUR> static void step_go(const bamd_batch_dev & b, const
         else if constexpr (PT >= 64) hipLaunchKernelGGL((ssm_step_kernel<PT, 16, FOUR>), grid, dim3(256), 0, s, b, a);
     }
 }
+static decltype(&ssm_chunk_kernel<1, false>) chunk_kernel(int N, int parts) {
+    if (N <= 64) return parts > 1 ? ssm_chunk_kernel<1, true> : ssm_chunk_kernel<1, false>;
+    if (N <= 128) return parts > 1 ? ssm_chunk_kernel<2, true> : ssm_chunk_kernel<2, false>;
+    return parts > 1 ? ssm_chunk_kernel<4, true> : ssm_chunk_kernel<4, false>;
+}
 // max_n: most tokens any entry brings.  a.filtered [rows][channels] and a.steps [rows][heads][2] are scratch of prompts
 int bamd_launch_ssm(const bamd_batch_dev & b, const bamd_ssm_args & a, int max_n, hipStream_t s) {
     if (a.N < 1 || a.N > 256 || a.taps < 1 || a.groups < 1 || a.heads % a.groups || max_n < 1) return 1;
@@ -412,8 +418,10 @@ int bamd_launch_ssm(const bamd_batch_dev & b, const bamd_ssm_args & a, int max_n
     for (int k = 1; k < parts; ++k) cut.at[k - 1] = (1.f - powf(SSM_AGAIN, (float) k)) / (1.f - powf(SSM_AGAIN, (float) parts));
     const dim3 cg((ch + 255) / 256, (b.rows + SSM_STRIP - 1) / SSM_STRIP), grid(cols * parts, a.heads, b.n_entries);
     if (a.taps == 4) hipLaunchKernelGGL(ssm_conv_kernel<true>, cg, dim3(256), 0, s, b, a); else hipLaunchKernelGGL(ssm_conv_kernel<false>, cg, dim3(256), 0, s, b, a);
-    if (a.N <= 64) hipLaunchKernelGGL(ssm_chunk_kernel<1>, grid, dim3(512), 0, s, b, a, cols, cut);
-    else if (a.N <= 128) hipLaunchKernelGGL(ssm_chunk_kernel<2>, grid, dim3(512), 0, s, b, a, cols, cut);
-    else hipLaunchKernelGGL(ssm_chunk_kernel<4>, grid, dim3(512), 0, s, b, a, cols, cut);
+    hipLaunchKernelGGL(chunk_kernel(a.N, parts), grid, dim3(512), 0, s, b, a, cols, cut);
     return 0;
+}
+int bamd_ssm_chunk_blocks(int N, int parts) {
+    int n = 0;
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, (const void *) chunk_kernel(N, parts), 512, 0) == hipSuccess ? n : -1;
 }

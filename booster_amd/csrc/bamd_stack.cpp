@@ -1233,6 +1233,8 @@ SafeTensor bf16_tensor(const uint16_t * p, std::vector<int64_t> shape) { SafeTen
 }  // namespace
 #define BAMD_OP extern "C" __attribute__((visibility("default"))) int
 
+// blocks of the state-space scan of prompts that a CU holds, for tokens taken in one part or in several; -1: no device
+BAMD_OP bamd_op_ssm_blocks(int N, int parts) { return N < 1 || N > 256 || parts < 1 ? -1 : bamd_ssm_chunk_blocks(N, parts); }
 BAMD_OP bamd_op_norm_threads(int n, int rows) { return bamd_norm_threads(n, rows); }
 BAMD_OP bamd_op_dense_route(int act, int nrows, int k, int rows, int pre, int most, int * shares) {
     if (nrows < 1 || k < 1 || rows < 1 || !shares) { fail("bamd_op_dense_route: bad arguments"); return -2; }

@@ -476,6 +476,12 @@ def test_ssm_tokens_that_are_not_finite_in_parts(bamd, N, at, what, value):
         assert not ok.any() or rel(got[t][ok], want[t][ok]) < 2e-5, t                # as test_ssm
 
 
+@pytest.mark.parametrize("N", [1, 64])
+def test_ssm_scan_in_one_part_has_two_blocks_per_cu(N):
+    """a block is eight waves, so that two need no more than 128 registers; what brings states along for parts of the tokens must not cost launches that fill the chip their second block"""
+    assert bamd_lib().bamd_op_ssm_blocks(N, 1) == 2
+
+
 def plain_attention(q, c, gate, past, uk, uv, c_norm, sink, scale, eps, H):
     T, _, d = q.shape
     lat = np.stack([so.rms(v, eps) * c_norm for v in c])
