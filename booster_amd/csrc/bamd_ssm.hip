@@ -182,7 +182,8 @@ __global__ void __launch_bounds__(256) ssm_step_kernel(bamd_batch_dev b, bamd_ss
 // wave takes the chunk again one token after the other, from the state in front of it, so that such a token reaches those behind it and none in front.  (A look at every value on
 // its way into LDS instead cost 264 us for 258; this one, under the stores of y, nothing.)
 // A prompt of few heads leaves CUs idle, and tokens one behind the other are its time: up to four parts of its tokens are taken at once, each by a block of its own, which brings the state along from the
-// first token on without the outputs (half a chunk's time) and so gets the bits that one block gets.  Borders are where all parts end together.  Four layers, us, one part and those taken: width 2048
+// first token on without the outputs (half a chunk's time).  Where values stay finite these are the bits that one block gets.  A chunk that one block takes again for its outputs (a C that is not finite) is
+// not taken again by those that bring only the state along: what stays finite behind it may be rounded otherwise, by the number of parts.  Borders are where all parts end together.  Four layers, us, one part and those taken: width 2048
 // (64 heads, two parts) 131 tokens 573 | 567, 1000 1228 | 1164, 2048 2051 | 1907; 1024 (32 heads, four) 300 473 | 448, 2048 1410 | 1217; 600 (13 heads) 1000 723 | 621.  Two parts to a CU (128 heads) were
 // no faster (2048 tokens of width 4096 4268 | 4271).  All these are state 128.  Tokens in one part have an instance of their own: with the parts' code in it a state of up to 64 takes 130 registers for
 // 128, one block per CU for two.  Eight prompts of 330 to 186 tokens, width 2048, state 64, 2320 us with, 2231 without, state 32 2312 | 2220; width 4096 (128 heads), two prompts of 900 and 675 3804 | 3700
@@ -265,7 +266,7 @@ __global__ void __launch_bounds__(512) ssm_chunk_kernel(bamd_batch_dev b, bamd_s
             if (lane < 16) { dts[w][lane] = fdt[w]; pre[w][lane] = p; fd[w][lane] = f * fdt[w]; }
         }
     };
-    // whole: outputs and state; the state alone is what a later part of the tokens starts from, in the same bits
+    // whole: outputs and state; the state alone is what a later part of the tokens starts from, in the same bits as long as neither takes a chunk again
     const std::integral_constant<bool, true> whole; const std::integral_constant<bool, false> state_only;
     auto state_chunk = [&](int t0, auto par) {
         constexpr int w = decltype(par)::value;

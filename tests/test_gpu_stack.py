@@ -450,6 +450,28 @@ def test_ssm_prompts_in_parts(bamd, H, P, N, G, n):
         assert rel(got, want) < 2e-5 and rel(gs, S) < 2e-5, pos      # as test_ssm
 
 
+@pytest.mark.parametrize("H,P,N,more", [(2, 40, 40, 66), (1, 31, 200, 130), (43, 33, 65, 86), (70, 20, 12, 140), (2, 64, 128, 128)])
+@pytest.mark.parametrize("n", [64, 81, 300])
+def test_ssm_parts_give_the_bits_of_one(bamd, H, P, N, more, n):
+    """the same heads in a launch that takes its tokens in four, three or two parts, and among so many that it takes one: outputs and state bit for bit"""
+    r = np.random.default_rng(H * P + N + n)
+    f = lambda a: np.asarray(a, np.float32)
+    chan = lambda H: H * P + 2 * N
+    cx, cbc, bx, bbc = r.standard_normal((H, P, 4)), r.standard_normal((2 * N, 4)), r.standard_normal((H, P)) * 0.3, r.standard_normal(2 * N) * 0.3
+    dtb, A, D = r.uniform(-6, 1, H), r.uniform(-4, 3, H), r.standard_normal(H)
+    z, x, bc, dt = r.standard_normal((n, H, P)), r.standard_normal((n, H, P)), r.standard_normal((n, 2 * N)), r.standard_normal((n, H))
+    dt[::9] -= 30
+    def go(heads):
+        k = np.arange(heads) % H
+        rows = np.concatenate([z[:, k].reshape(n, -1), x[:, k].reshape(n, -1), bc, dt[:, k]], 1)
+        got, _, S = bamd.op_ssm(f(rows), 0, heads, P, N, 1, f(np.concatenate([cx[k].reshape(-1, 4), cbc])), f(np.concatenate([bx[k].ravel(), bbc])), f(dtb[k]), f(A[k]), f(D[k]), np.zeros((3, chan(heads)), np.float32), np.zeros((heads, N, P), np.float32))
+        return got.reshape(n, heads, P), S
+    y, S = go(H)
+    ym, Sm = go(more)
+    k = np.arange(more) % H
+    assert (np.ascontiguousarray(ym).view(np.uint32) == np.ascontiguousarray(y[:, k]).view(np.uint32)).all() and (Sm.view(np.uint32) == np.ascontiguousarray(S[k]).view(np.uint32)).all()
+
+
 @pytest.mark.parametrize("N,at", [(40, 0), (128, 3), (200, 17), (40, 47), (128, 60), (40, 110)])
 @pytest.mark.parametrize("what,value", [("x", np.inf), ("x", np.nan), ("B", np.inf), ("C", np.nan), ("dt", np.inf), ("far", 1e20)])
 def test_ssm_tokens_that_are_not_finite_in_parts(bamd, N, at, what, value):
