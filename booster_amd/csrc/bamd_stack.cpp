@@ -216,7 +216,7 @@ struct Ctx {
 struct Pass {                                      // one pass through the layers
     Ctx & c; Stack & st; hipStream_t s; bamd_batch_dev b; bool decode = false;
     int n_tiles = 0, k_rows = 0, max_n = 1, n_segs = 0, most = 0; float * x; float * xo; const float * pend = nullptr; int ldp = 0; const float * pend_g = nullptr; int pend_parts = 1;
-    Timer * tm = nullptr;                          // most: positions of the longest sequence behind this pass (steps that are enqueued at once: behind the last)
+    Timer * tm = nullptr;                          // most: positions of the longest sequence behind this pass
     void begin(int kind, double bytes) { if (!tm) return; hipEvent_t e; hipEventCreate(&e); hipEventRecord(e, s); tm->ev.push_back(e); tm->kind.push_back(kind); tm->bytes.push_back(bytes); }
     void end() { if (!tm) return; hipEvent_t e; hipEventCreate(&e); hipEventRecord(e, s); tm->ev.push_back(e); }
 
@@ -1060,13 +1060,12 @@ int Stack::generate(bamd_context * bc, const int32_t * seqs, int n, int n_steps,
     HIPC(hipMemcpyAsync(c.step, &zero, 4, hipMemcpyHostToDevice, s));
     Pass p{ c, *this, s, {}, true };
     if (send(p, pc, want)) return 1;
-    p.most += n_steps - 1;
     hipEvent_t a = nullptr, b = nullptr;
     HIPC(hipEventCreate(&a));
     if (hipEventCreate(&b) != hipSuccess) { hipEventDestroy(a); return fail("hipEventCreate"); }
     int rc = 0;
     hipEventRecord(a, s);
-    for (int t = 0; t < n_steps && !rc; ++t) rc = decode_rows(p, STEP_GREEDY);
+    for (int t = 0; t < n_steps && !rc; ++t, ++p.most) rc = decode_rows(p, STEP_GREEDY);       // (each step's kernels are those that a step of its own takes)
     hipEventRecord(b, s);
     if (!rc) {
         for (const Piece & q : pc) { c.seqs[(size_t) q.seq].len += n_steps; c.seqs[(size_t) q.seq].par ^= n_steps & 1; }

@@ -647,6 +647,53 @@ def cases(tmp_path_factory):
     return {n: Case(str(d / n), c, SEEDS[n], ROWS.get(n)) for n, c in sorted(CONFIGS.items())}
 
 
+# a rank of 512: one launch for the latent attention of 288 to 310 positions in bfloat16, of 224 to 240 in 32-bit, three behind them; one rank that takes three throughout
+LONG_LATENT = config(64, 97, [latent(3, 24, 40, 512, 0.31, ff=70), mamba(3, 20, 24, 1, 5, 3), latent(2, 33, 12, 600, 0.2, ff=50)])
+
+
+@pytest.fixture(scope="module")
+def long_latent(tmp_path_factory):
+    return Case(str(tmp_path_factory.mktemp("long_latent") / "m"), LONG_LATENT, 5)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rows", [1, 3])
+def test_latent_steps_that_outgrow_one_launch(bamd, long_latent, dtype, rows):
+    """sequences of different lengths decoded across the most positions that one launch takes"""
+    m = bamd.Model(long_latent.folder, dtype=dtype)
+    c = bamd.Context(m, 448 * rows, rows)
+    for most in ((284, 304) if dtype == "bfloat16" else (220, 234)):
+        t = [tokens(LONG_LATENT, most + 12, 30 + i) for i in range(rows)]
+        want = [long_latent.logits(x) for x in t]
+        at = [most - 40 * s for s in range(rows)]
+        for s in range(rows): c.seq_free(s)
+        c.decode_batch([(s, t[s][:at[s]], [at[s] - 1]) for s in range(rows)])
+        for _ in range(12):
+            got = c.decode_batch([(s, [t[s][at[s]]], [0]) for s in range(rows)])
+            near(got, np.stack([want[s][at[s]] for s in range(rows)]), dtype)
+            at = [a + 1 for a in at]
+    c.close(); m.close()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_generating_across_the_limit_of_one_launch_is_stepping_across_it(bamd, long_latent, dtype):
+    """the logits behind steps enqueued at once are those, bit for bit, of the same steps one call each, however many of them run behind the limit"""
+    m = bamd.Model(long_latent.folder, dtype=dtype)
+    c = bamd.Context(m, 512, 1)
+    at = 280 if dtype == "bfloat16" else 216
+    p = tokens(LONG_LATENT, at, 7)
+    for steps in (4, 36):
+        c.seq_free(0)
+        c.decode(p, 0)
+        out, _ = c.generate_greedy(at, steps)
+        last = c.last_logits()
+        c.seq_free(0)
+        c.decode(p, 0)
+        for i in range(steps): one = c.decode([out[i]], at + i)
+        assert np.array_equal(last.view(np.uint32), one.view(np.uint32)), steps
+    c.close(); m.close()
+
+
 @pytest.fixture(params=[(n, t) for n in sorted(CONFIGS) for t in DTYPES], ids=lambda p: "-".join(p))
 def run(request, bamd, cases):
     name, dtype = request.param
