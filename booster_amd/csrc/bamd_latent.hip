@@ -381,6 +381,11 @@ template <typename T> __global__ void __launch_bounds__(512) latent_combine_kern
 // up-projection.  The three launches above become one; the pass over the cache that sixteen heads share there is every head's own here, out of the L2.  W_uk and the first latents are requested
 // before the token's row arrives.  Scores, weights and sums are 32-bit on the vector units: a head is one row of the matrix cores.
 // KT: D / 32; NRT: sixteen-row tiles of W_uk per wave (Rp <= 256 NRT); NP: pieces of sixteen bytes of a latent per lane
+// exp(x) of a share's maximum, x <= 0, to an ulp and a half.  __expf is off by half an ulp of x log2(e) (3e-6 at -62), and expf where products and sums may fuse is as well: its remainder enters twice
+__device__ __forceinline__ float share_weight(float x) {
+    const float hi = x * 1.4426950408889634f, lo = hi > -200.f ? fmaf(x, 1.9259629911266175e-8f, fmaf(x, 1.4426950408889634f, -hi)) : 0.f;
+    return __builtin_amdgcn_exp2f(hi) * fmaf(lo, 0.6931471805599453f, 1.f);
+}
 template <typename T> __device__ __forceinline__ void piece_of(const bamd_u4 & w, float * x) {
     if constexpr (sizeof(T) == 2) { x[0] = bf_lo(w.x); x[1] = bf_hi(w.x); x[2] = bf_lo(w.y); x[3] = bf_hi(w.y); x[4] = bf_lo(w.z); x[5] = bf_hi(w.z); x[6] = bf_lo(w.w); x[7] = bf_hi(w.w); }
     else { x[0] = __uint_as_float(w.x); x[1] = __uint_as_float(w.y); x[2] = __uint_as_float(w.z); x[3] = __uint_as_float(w.w); }
@@ -388,7 +393,7 @@ template <typename T> __device__ __forceinline__ void piece_of(const bamd_u4 & w
 template <typename T, int KT, int NRT, int NP> __global__ void __launch_bounds__(1024) latent_step_kernel(bamd_batch_dev b, bamd_latent_args a) {
     constexpr int VPP = 16 / (int) sizeof(T), D = 32 * KT, VT = D / 16, KP = 16 / VT, NKT = (8 * NRT + KP - 1) / KP, PF = NP == 2 ? 2 : NRT == 2 ? 3 : 4, RM = 256 * NRT;      // KP: shares of K per value tile
     extern __shared__ __align__(16) unsigned char lds[];
-    __shared__ float q[D], qp[RM], own[RM], red[32], ms[257], ls[257], part[16][16];
+    __shared__ float q[D], qp[RM], own[RM], red[32], ms[257], ls[257], wt[257], part[16][16];
     const int h = blockIdx.x, row = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int rt_n = a.Rp / 16, kt_n = a.Rp / 32, pr = a.Rp / VPP;
     bamd_u4 wk[NRT][KT];
@@ -522,15 +527,17 @@ template <typename T, int KT, int NRT, int NP> __global__ void __launch_bounds__
     float mx = fmaxf(snk, ms[n]);
     for (int i = lane; i < n; i += 64) mx = fmaxf(mx, ms[i]);
     mx = wave_max(mx);
+    if (tid <= n) wt[tid] = share_weight(ms[tid] - mx);
+    __syncthreads();
     float sum = 0.f;
-    for (int i = lane; i <= n; i += 64) sum += __expf(ms[i] - mx) * ls[i];
+    for (int i = lane; i <= n; i += 64) sum += wt[i] * ls[i];
     sum = wave_sum(sum);
     if (a.sink) sum += expf(snk - mx);
     const int th = a.Rp <= 256 ? 4 : 2, r = tid / th, g = tid % th;          // th threads per value of the latent: neighbours
     float v = 0.f;
     if (r < a.Rp) {
-        for (int i = g; i < n; i += th) v += __expf(ms[i] - mx) * ps[i * a.Rp + r];
-        if (g == 0) v += __expf(ms[n] - mx) * own[r];
+        for (int i = g; i < n; i += th) v += wt[i] * ps[i * a.Rp + r];
+        if (g == 0) v += wt[n] * own[r];
     }
     v += __shfl_xor(v, 1); if (th == 4) v += __shfl_xor(v, 2);
     if (r < a.Rp && g == 0) qp[r] = v;                             // (the scores are behind a barrier)

@@ -548,6 +548,26 @@ def test_latent_attention_step_in_one_launch(bamd, dtype, H, d, dv, R, pos0):
     near(bamd.op_latent_attention(dtype=dtype, decode=2, **a).reshape(1, -1), plain_attention(H=H, **a).reshape(1, -1), dtype)
 
 
+def test_latent_attention_step_weighs_shares_in_32_bits():
+    """scores that are whole numbers, a share for every key, and values that keep the keys apart: what is left of an output's error is its share's weight.  An exponential of a product rounded to 32 bits
+    is off by up to 3e-6 here (half an ulp of 62 log2(e)); one to an ulp and a half, the sum, the quotient and the products are no more than eight roundings of 2^-24"""
+    import booster_amd as bamd
+    n, d = 32, 8
+    scores = np.random.default_rng(2).permutation(np.arange(n) * 2 + 3).astype(np.float32)
+    past = np.zeros((n, n), np.float32)
+    past[:, 0] = scores
+    past[np.arange(1, n), np.arange(1, n)] = 1
+    uk, q, cn = np.zeros((d, n)), np.zeros((1, 1, d), np.float32), np.ones(n, np.float32)
+    uk[0, 0], q[0, 0, 0], cn[0] = 1, 1, 0                 # (the token's own score: zero)
+    c = np.zeros((1, n), np.float32)
+    c[0, 0] = 1
+    uv = np.eye(n)[1:]
+    a = dict(q=q, c=c, gate=None, past=past, uk=so.f32_to_bf16(uk), uv=so.f32_to_bf16(uv), c_norm=cn, sink=None, scale=1.0, eps=1e-5)
+    want = plain_attention(H=1, **a)
+    got = bamd.op_latent_attention(dtype="float32", decode=2, **a)
+    assert np.abs(got / want - 1).max() < 5e-7
+
+
 @pytest.mark.parametrize("H,d,R,T,pos0", [(128, 24, 20, 257, 0), (128, 24, 20, 512, 70), (128, 24, 20, 513, 0), (85, 40, 36, 700, 130)])
 def test_latent_attention_in_paired_blocks(bamd, H, d, R, T, pos0):
     """tiles of 128 queries: one block per CU and a part of a second, two (taken the other way round), two and a part of a third (plain order), and heads that do not divide the CUs"""
