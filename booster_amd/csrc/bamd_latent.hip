@@ -632,12 +632,15 @@ template <typename T> static void step_go(const bamd_batch_dev & b, const bamd_l
     if (a.D == 32) step_pick<T, 1>(b, a, s); else if (a.D == 64) step_pick<T, 2>(b, a, s); else step_pick<T, 4>(b, a, s);
 }
 bool bamd_latent_step_valid(int D, int Rp) { return D <= 128 && Rp <= 512; }
-// Every head reads the cache by itself in the one launch, sixteen share it in the three: 20 to 25 us less a layer against 12 ns a position of 256 bfloat16 numbers.  Steps of eight layers, three
+// Every head reads the cache by itself in the one launch, sixteen share it in the three: 20 to 25 us less a step against a time per position that goes by the rank and 42 numbers (a row's sum over its lanes
+// and its weight cost the same whatever it holds): where both are level, positions x (rank + 42) are 180k to 210k at ranks 32 to 512 in bfloat16 and 140k to 170k in 32-bit.  Steps of eight layers, three
 // launches and one, us: width 2048, rank 256, 16 heads: 60 positions 423 | 398, 155 427 | 408, 380 428 | 418, 800 432 | 438; sixteen rows 216 709 | 689, 500 707 | 692, 1000 711 | 716; 32-bit 155
 // 461 | 430, 380 460 | 452, 800 461 | 501.  Width 4096, rank 512, 32 heads: 155 830 | 809, 380 838 | 836, 800 827 | 884; sixteen rows 216 1280 | 1253, 500 1289 | 1317; 32-bit 155 907 | 849.
+// Lower ranks: width 1024, 8 heads, rank 32 2000 positions 267 | 261, 3000 266 | 267, 4000 264 | 273; 64 1500 265 | 261, 2000 266 | 268, 3000 266 | 280; 128 1000 277 | 271, 1500 279 | 284, 2000 280 | 297; 16
+// heads of width 2048, rank 64 1000 378 | 366, 2000 381 | 384, six rows 489 | 483, rank 256 520 392 | 384, 640 385 | 391; 32-bit rank 32 1700 272 | 268, 3000 276 | 284; 64 1000 274 | 265, 1700 277 | 281; 128 500 290 | 267, 1000 284 | 285; 256 430 415 | 406.
 // With more than two blocks to a CU the three are ahead: 48 rows of 16 heads, 100 positions 1200 | 1223
 bool bamd_latent_one_launch(int act, int D, int Rp, int rows, int heads, int most) {
-    return bamd_latent_step_valid(D, Rp) && most > 0 && (size_t) most * Rp <= (act == BAMD_ACT_F32 ? 112 * 1024 : 144 * 1024) && rows * heads <= 512;
+    return bamd_latent_step_valid(D, Rp) && most > 0 && (size_t) most * (Rp + 42) <= (act == BAMD_ACT_F32 ? 140000 : 180000) && rows * heads <= 512;
 }
 void bamd_launch_latent_step(int act, const bamd_batch_dev & b, const bamd_latent_args & a, hipStream_t s) {
     if (act == BAMD_ACT_F32) step_go<float>(b, a, s); else step_go<bamd_bf>(b, a, s);

@@ -1247,6 +1247,11 @@ BAMD_OP bamd_op_dense_cut(int nrows, int k, int rows, int gated) {
     d.rows = nrows; d.K = up(k, 32); d.row_tiles = up(nrows, 16) / 16; d.k_tiles = d.K / 32;
     return bamd_dense_cut(d, rows, gated ? BAMD_OUT_GLU : BAMD_OUT_F32) * 16;
 }
+// 1: a step of so many rows behind up to `positions` of them takes its latent attention in one launch
+BAMD_OP bamd_op_latent_route(int act, int dim, int rank, int rows, int heads, int positions) {
+    int D = 32; while (D < dim) D *= 2;
+    return bamd_latent_one_launch(act, D, up(rank, 32), rows, heads, positions);
+}
 BAMD_OP bamd_op_dense(int act, const uint16_t * w, int nrows, int k, const float * x, int rows, int impl, float * y) {
     OpScratch s; bamd_dense d; void * dx; float * dy = nullptr;
     const int planes = bamd_row_planes(act), cb = impl == 6 || impl == 7 ? planes * bamd_row_blocks(rows) : 0;                   // 6, 7: as impl 0 and 1, the operand rows by blocks

@@ -667,13 +667,14 @@ def cases(tmp_path_factory):
     return {n: Case(str(d / n), c, SEEDS[n], ROWS.get(n)) for n, c in sorted(CONFIGS.items())}
 
 
-# a rank of 512: one launch for the latent attention of 288 to 310 positions in bfloat16, of 224 to 240 in 32-bit, three behind them; one rank that takes three throughout
+# a rank of 512: one launch for the latent attention of up to 324 positions in bfloat16, 252 in 32-bit, three behind them; a rank that takes three throughout.
+# Weights by their condition: the oracle with every product's operands rounded to bfloat16 moves no row behind position 150 of the tests' tokens by more than 0.0112 (weights 5: 0.051)
 LONG_LATENT = config(64, 97, [latent(3, 24, 40, 512, 0.31, ff=70), mamba(3, 20, 24, 1, 5, 3), latent(2, 33, 12, 600, 0.2, ff=50)])
 
 
 @pytest.fixture(scope="module")
 def long_latent(tmp_path_factory):
-    return Case(str(tmp_path_factory.mktemp("long_latent") / "m"), LONG_LATENT, 5)
+    return Case(str(tmp_path_factory.mktemp("long_latent") / "m"), LONG_LATENT, 13)
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
@@ -682,7 +683,7 @@ def test_latent_steps_that_outgrow_one_launch(bamd, long_latent, dtype, rows):
     """sequences of different lengths decoded across the most positions that one launch takes"""
     m = bamd.Model(long_latent.folder, dtype=dtype)
     c = bamd.Context(m, 448 * rows, rows)
-    for most in ((284, 304) if dtype == "bfloat16" else (220, 234)):
+    for most in ((318,) if dtype == "bfloat16" else (246,)):
         t = [tokens(LONG_LATENT, most + 12, 30 + i) for i in range(rows)]
         want = [long_latent.logits(x) for x in t]
         at = [most - 40 * s for s in range(rows)]
@@ -700,7 +701,7 @@ def test_generating_across_the_limit_of_one_launch_is_stepping_across_it(bamd, l
     """the logits behind steps enqueued at once are those, bit for bit, of the same steps one call each, however many of them run behind the limit"""
     m = bamd.Model(long_latent.folder, dtype=dtype)
     c = bamd.Context(m, 512, 1)
-    at = 280 if dtype == "bfloat16" else 216
+    at = 318 if dtype == "bfloat16" else 246
     p = tokens(LONG_LATENT, at, 7)
     for steps in (4, 36):
         c.seq_free(0)

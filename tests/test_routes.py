@@ -90,3 +90,22 @@ def test_few_rows_are_halved_where_that_is_faster(L):
     for act in (BF16, F32):
         assert [share(act, n, k, ROWS, rows) for rows in (1, 64) for n, k in ((2048, 2048), (2049, 2048), (2048, 2016))] == [2, 1, 1] * 2
     assert [share(BF16, 512, 4096, pre) for pre in (1, 4, 6)] == [1, 1, 1]           # prologues that write state
+
+
+# type, rank, heads, rows, positions, measured us of a step of eight layers with latent attention in three launches and in one (where both are level, either is right)
+@pytest.mark.parametrize("act,rank,heads,rows,positions,three,one", [
+    (BF16, 32, 8, 1, 2000, 267, 261), (BF16, 32, 8, 1, 4000, 264, 273), (BF16, 64, 8, 1, 1500, 265, 261), (BF16, 64, 8, 1, 3000, 266, 280), (BF16, 64, 16, 1, 1000, 378, 366), (BF16, 64, 16, 1, 2000, 381, 384),
+    (BF16, 128, 8, 1, 1000, 277, 271), (BF16, 128, 8, 1, 1500, 279, 284), (BF16, 128, 16, 6, 1000, 490, 474), (BF16, 128, 16, 6, 2000, 494, 502), (BF16, 256, 16, 1, 520, 392, 384), (BF16, 256, 16, 1, 800, 432, 438),
+    (BF16, 512, 32, 1, 155, 830, 809), (BF16, 512, 32, 1, 800, 827, 884), (BF16, 512, 32, 16, 216, 1280, 1253), (BF16, 512, 32, 16, 500, 1289, 1317), (BF16, 256, 16, 48, 100, 1200, 1223), (BF16, 64, 16, 16, 1000, 595, 550),
+    (F32, 32, 8, 1, 1700, 272, 268), (F32, 32, 8, 1, 3000, 276, 284), (F32, 64, 8, 1, 1000, 274, 265), (F32, 64, 8, 1, 1700, 277, 281), (F32, 128, 8, 1, 500, 290, 267), (F32, 128, 8, 1, 1700, 287, 316),
+    (F32, 256, 16, 1, 380, 460, 452), (F32, 256, 16, 1, 800, 461, 501), (F32, 512, 32, 1, 155, 907, 849)])
+def test_latent_steps_take_the_faster_launches(L, act, rank, heads, rows, positions, three, one):
+    assert L.bamd_op_latent_route(act, 128, rank, rows, heads, positions) == (one < three)
+
+
+def test_latent_steps_of_shorter_sequences_are_no_slower_choice(L):
+    """the layers that take one launch are told apart by their number: what takes it at some length takes it at every shorter one"""
+    for act in (BF16, F32):
+        for rank in (32, 96, 256, 512, 544):
+            got = [L.bamd_op_latent_route(act, 128, rank, 1, 16, n) for n in range(1, 5000)]
+            assert got == sorted(got, reverse=True) and got[0] == (rank <= 512)
