@@ -649,21 +649,22 @@ int bamd_prefill_mfma_supported(void) {
     return 1;
 }
 // Token tiles (of 16) per block of the few-token kernel for this product, 0: one of the kernels with 64-row blocks.
-// Up to 64 tokens: whichever ends first.  Both take a start and a time per super-block, for every round of 256 blocks; the few-token kernel's goes by its token tiles.  Constants in ns,
-// fitted to 1323 sizes (three types, 8 to 64 tokens, 1024 to 24576 rows, K 1024 to 14336) with all records of the tiles copied: with fewer tokens the few-token kernel is faster than they say.
-// Q4_K with 33 to 48 tokens took 530 or 640 a step, by how the records lay to the lines; 572 keeps the sizes where those two were level (two rounds at K = 3840 and 4096) on the sides they were measured on.
-// Where the two part, K = 4096, 64-row blocks against 16-row ones in us: 8192 rows Q4_K 32 tokens 24.1 | 18.4, 48 tokens 24.0 | 22.7, 64 tokens 24.1 | 25.5; 12288 rows 32 tokens 25.2 | 27.9;
-// Q6_K 8192 rows 64 tokens 34.7 | 31.2
-struct x_cost { int start64, step64, extra, start[3], step[3]; };      // extra: what the few-token kernel's launch takes more, whatever its rounds
+// Up to 64 tokens and 16384 rows: whichever ends first.  The few-token kernel takes a start, and for every round of 256 blocks another and a time per super-block, which grows with the tokens whose records
+// are copied; the other (64 rows a block: matmul_mfma3_q4k_kernel, for Q6_K matmul_wide_kernel's four waves) is in its first round up to 16384 rows, and behind that faster everywhere (of 1755 sizes).
+// Constants in ns (token: tenths), fitted to 8190 sizes (three types, 6 to 64 tokens, 1024 to 16384 rows, K 1024 to 14336; weights from memory, launches one behind the other), of which this rule takes
+// the slower kernel for 13 by more than 1.5 %, at most 4.6 %; of 1500 others, drawn at random, for 4, at most 3.0 %.  Prompts of eight 8B layers, 50 tokens 1327 -> 1247 us, 61 1365 -> 1296; six 7B ones in
+// Q6_K, 26 942 -> 919, 48 1046 -> 1016.  Where the two part, us, few-token kernel and the other: Q4_K, K = 4096, 8192 rows 48 tokens 23.3 | 25.6, 64 26.4 | 26.1, 12288 rows 16 tokens
+// 25.8 | 25.6, 32 tokens 28.5 | 25.6; 6144 rows x 3840 40 tokens 20.3 | 23.6; Q6_K, K = 4096, 4096 rows 40 tokens 16.5 | 27.2, 6144 rows 16 tokens 26.2 | 23.5, 40 30.7 | 27.5
+struct x_cost { int extra, start[3], step[3], token[3], start64[3], step64[3]; };
 static int x_few_tiles(int type, int nrows_pad, int nb, int T) {
-    static const x_cost costs[3] = { { 3010, 1300, 1150, { 1790, 2140, 2400 }, { 410, 572, 590 } },         // Q4_K
-                                     { 3410, 1240, 1800, { 1900, 2180, 2600 }, { 416, 520, 580 } },         // Q5_K
-                                     { 3590, 1815, 1150, { 2040, 2400, 2740 }, { 680, 710, 750 } } };       // Q6_K
-    if (T > 64) return 0;
+    static const x_cost costs[3] = { { 1270, { 1950, 2230, 2490 }, { 335, 330, 334 }, { 30, 40, 43 }, { 3680, 3860, 3950 }, { 1346, 1335, 1355 } },         // Q4_K
+                                     { 1140, { 2060, 2320, 2570 }, { 335, 283, 302 }, { 36, 58, 53 }, { 3530, 3630, 3430 }, { 1318, 1344, 1429 } },         // Q5_K
+                                     { 1300, { 2250, 2670, 3080 }, { 541, 609, 751 }, { 54, 37, 10 }, { 3630, 4400, 4680 }, { 1243, 1429, 1637 } } };       // Q6_K
+    if (T > 64 || nrows_pad > 16384) return 0;
     const x_cost & c = costs[type == BAMD_Q6_K ? 2 : type == BAMD_Q5_K ? 1 : 0];
     const int i = T <= 32 ? 0 : T <= 48 ? 1 : 2;
-    const long few = c.extra + (long) ((nrows_pad + 15) / 16 + 255) / 256 * (c.start[i] + (long) c.step[i] * nb);
-    return few < ((long) x_row_blocks(nrows_pad) + 255) / 256 * (c.start64 + (long) c.step64 * nb) ? i + 2 : 0;
+    const long few = c.extra + (long) ((nrows_pad + 15) / 16 + 255) / 256 * (c.start[i] + (10L * c.step[i] + (long) c.token[i] * T) * nb / 10);
+    return few < c.start64[i] + (long) c.step64[i] * nb ? i + 2 : 0;
 }
 int bamd_prefill_few_tiles(int type, int nrows_pad, int K, int T) { return x_few_tiles(type, nrows_pad, K >> 8, T); }
 size_t bamd_prefill_route(int type, int nrows_pad, int K, int T, int * few_tiles, size_t * most) {

@@ -44,12 +44,13 @@ def test_the_launch_probe_covers_every_prompt_product(L):
     assert {s[0] for s in seen} == {0, 2, 3, 4} and max(s[1] for s in seen) == 159328 == most
 
 
-# type, K, rows, tokens, measured us of 64-row blocks and of the few-token kernel
+# type, K, rows, tokens, measured us of the other kernel (64-row blocks up to 16384 rows) and of the few-token kernel
 @pytest.mark.parametrize("t,k,rows,T,wide,few", [
-    (Q4_K, 4096, 4096, 37, 23.8, 12.3), (Q4_K, 4096, 8192, 32, 24.1, 18.4), (Q4_K, 4096, 8192, 48, 24.0, 22.7), (Q4_K, 4096, 8192, 64, 24.1, 25.5), (Q4_K, 3840, 6144, 36, 22.7, 25.2), (Q4_K, 4096, 6144, 36, 23.9, 22.8),
-    (Q4_K, 2048, 4352, 40, 13.8, 15.9), (Q4_K, 1536, 5120, 32, 11.2, 10.4), (Q4_K, 1536, 6144, 40, 11.4, 13.5), (Q4_K, 1024, 8192, 48, 8.9, 11.4), (Q4_K, 8960, 6144, 36, 48.8, 43.1), (Q4_K, 4096, 12288, 32, 25.2, 27.9),
-    (Q4_K, 2048, 24576, 16, 27.1, 33.5), (Q5_K, 3072, 6144, 64, 17.6, 20.5), (Q5_K, 2048, 6144, 48, 13.0, 14.9), (Q5_K, 13312, 6144, 48, 68.7, 59.7), (Q5_K, 14336, 4352, 32, 69.6, 52.5), (Q5_K, 4096, 14336, 48, 26.0, 44.8),
-    (Q6_K, 4096, 8192, 64, 34.7, 31.2), (Q6_K, 2048, 4352, 32, 18.2, 16.8), (Q6_K, 1024, 8192, 64, 12.1, 13.6), (Q6_K, 8192, 6144, 40, 62.2, 53.8), (Q6_K, 14336, 14336, 40, 108.0, 175.3), (Q6_K, 4096, 12288, 32, 33.9, 41.9)])
+    (Q4_K, 4096, 4096, 37, 24.7, 11.8), (Q4_K, 4096, 8192, 32, 25.0, 19.6), (Q4_K, 4096, 8192, 48, 25.4, 23.0), (Q4_K, 4096, 8192, 64, 26.0, 26.2), (Q4_K, 3840, 6144, 36, 23.5, 20.0), (Q4_K, 4096, 6144, 36, 24.8, 21.0),
+    (Q4_K, 2048, 4352, 40, 14.4, 13.2), (Q4_K, 1536, 5120, 32, 11.8, 10.5), (Q4_K, 1536, 6144, 40, 11.9, 11.6), (Q4_K, 1024, 8192, 48, 9.5, 10.4), (Q4_K, 8960, 6144, 36, 49.4, 38.7), (Q4_K, 4096, 12288, 32, 25.4, 28.3),
+    (Q4_K, 2048, 24576, 16, 15.2, 31.2), (Q4_K, 14336, 24576, 32, 75.4, 155.3), (Q5_K, 3072, 6144, 64, 20.9, 21.5), (Q5_K, 2048, 6144, 48, 14.9, 15.0), (Q5_K, 13312, 6144, 48, 74.9, 65.6), (Q5_K, 14336, 4352, 32, 74.1, 53.1),
+    (Q5_K, 4096, 14336, 48, 27.4, 46.6), (Q6_K, 4096, 8192, 64, 30.9, 33.2), (Q6_K, 2048, 4352, 32, 13.8, 17.1), (Q6_K, 1024, 8192, 64, 11.4, 14.4), (Q6_K, 8192, 6144, 40, 50.0, 53.7), (Q6_K, 14336, 14336, 40, 84.7, 175.7),
+    (Q6_K, 4096, 12288, 32, 24.2, 42.2), (Q6_K, 4096, 6144, 16, 23.3, 25.7), (Q6_K, 4096, 4352, 37, 27.1, 29.8), (Q6_K, 4096, 4096, 40, 27.2, 16.5), (Q6_K, 5120, 20480, 32, 38.8, 83.2)])
 def test_few_token_products_take_the_faster_kernel(L, t, k, rows, T, wide, few):
     assert (prefill(L, t, rows, k, T)[0] > 0) == (few < wide)
 
