@@ -443,7 +443,7 @@ def test_steps_that_outgrow_one_launch(bamd, dtype, H, d, dv, rows, tmp_path):
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("H,d,dv,steps", [(3, 130, 70, (2, 21, 22, 42, 43, 64, 65)), (6, 64, 65, (5, 11, 22)), (7, 20, 30, (19, 37)), (2, 100, 9, (6, 64))])
 def test_decoding_rows_that_share_launches(bamd, dtype, H, d, dv, steps, tmp_path):
-    """a step of that many sequences, whose recurrence takes 16, 32 or 64 columns a block; beyond 64 rows (48 in 32-bit) the branches have their own launches"""
+    """a step of that many short sequences: one launch up to 64 rows (48 in 32-bit) and 128 channels, two beyond the channels, the branches' own launches beyond the rows"""
     cfg = stack_cases.mafurax(64, 97, [stack_cases.parallel(stack_cases.attend(4, 2, 24, 20, 0.4, 6.0, 50, 19, 3), 0.7, (H, d, dv, 8.0), 1.3, ff=80, limit=0.8)])
     case = Case(str(tmp_path / "m"), cfg, 3, dict(rel=8, rank=5))
     m = bamd.Model(case.folder, dtype=dtype)
@@ -452,6 +452,26 @@ def test_decoding_rows_that_share_launches(bamd, dtype, H, d, dv, steps, tmp_pat
     want = [case.logits(x) for x in t]
     c.decode_batch([(s, t[s % 3][:5 + s % 3], [4 + s % 3]) for s in range(max(steps))])
     at = [5 + s % 3 for s in range(max(steps))]
+    for n in steps:
+        got = c.decode_batch([(s, [t[s % 3][at[s]]], [0]) for s in range(n)])
+        near(got, np.stack([want[s % 3][at[s]] for s in range(n)]), dtype)
+        for s in range(n): at[s] += 1
+    c.close(); m.close()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H,d,dv,steps", [(3, 130, 70, (2, 22, 43, 64, 65)), (6, 64, 65, (5, 11, 22)), (7, 20, 30, (19, 37)), (2, 100, 9, (6, 64)), (16, 128, 128, (3, 6, 8))])
+def test_decoding_long_rows_that_share_launches(bamd, dtype, H, d, dv, steps, tmp_path):
+    """the same behind 452 positions and more, which is two launches whatever the rows: the recurrence takes 16, 32 or 64 columns a block, up to 64, 128 and more channels.  (The oracle with every product's
+    operands rounded to bfloat16 moves no row of these by more than 0.0053.)"""
+    cfg = stack_cases.mafurax(64, 97, [stack_cases.parallel(stack_cases.attend(4, 2, 24, 20, 0.4, 6.0, 50, 1 << 20, 0), 0.7, (H, d, dv, 8.0), 1.3, ff=80, limit=0.8)])
+    case = Case(str(tmp_path / "m"), cfg, 3, dict(rel=8, rank=5))
+    m = bamd.Model(case.folder, dtype=dtype)
+    c = bamd.Context(m, 512 * max(steps), max(steps))
+    t = [tokens(cfg, 454 + len(steps), 30 + i) for i in range(3)]
+    want = [case.logits(x) for x in t]
+    c.decode_batch([(s, t[s % 3][:452 + s % 3], [451 + s % 3]) for s in range(max(steps))])
+    at = [452 + s % 3 for s in range(max(steps))]
     for n in steps:
         got = c.decode_batch([(s, [t[s % 3][at[s]]], [0]) for s in range(n)])
         near(got, np.stack([want[s % 3][at[s]] for s in range(n)]), dtype)
