@@ -191,8 +191,8 @@ bool bamd_gla_valid(const bamd_gla_args & a);
 
 // ---- both at once ------------------------------------------------------------------------------------------------------------------------------------
 // a decoded token through attention and gated linear attention that read the same projection: their blocks share two launches
+int bamd_launch_kv_gla_decode(int act, const bamd_batch_dev & b, const bamd_kv_args & kv, const bamd_gla_args & gla, float * part_o, float * part_ml, int splits, hipStream_t s);
 // the same in one launch (bamd_kv_gla_one_valid; null: without that mixer), which is the faster one for rows of up to `most` positions where bamd_kv_gla_one_launch says so (and then for shorter ones as well)
 bool bamd_kv_gla_one_valid(const bamd_kv_args * kv, const bamd_gla_args * gla);
 bool bamd_kv_gla_one_launch(int act, const bamd_kv_args & kv, const bamd_gla_args & gla, int rows, int most);
 int bamd_launch_kv_gla_one(int act, const bamd_batch_dev & b, const bamd_kv_args * kv, const bamd_gla_args * gla, hipStream_t s);
-int bamd_launch_kv_gla_decode(int act, const bamd_batch_dev & b, const bamd_kv_args & kv, const bamd_gla_args & gla, float * part_o, float * part_ml, int splits, hipStream_t s);

@@ -751,7 +751,7 @@ static int ensure_batch_buffers(bamd_context * c, int tokens) {
     return 0;
 }
 // Layout k of T quantised activations (0 rows of bytes, 1 f16 records, 2 f16 fragments), allocated when a product first reads it, by steps of BAMD_PREFILL_CAP tokens: most models read one or
-// two (of 2048 tokens at a feed-forward of 14336 all three would be 170 MB, the fragments are 64).  1: not allocated (what was there stays)
+// two (of 2048 tokens at a feed-forward of 14336 all three would be 193 MB: bytes 33, records 97, fragments 63).  1: not allocated (what was there stays)
 static int ensure_layout(bamd_context * c, int k, int T) {
     if (c->blay_tokens[k] >= T) return 0;
     const int cap = (T + BAMD_PREFILL_CAP - 1) / BAMD_PREFILL_CAP * BAMD_PREFILL_CAP, Kmax = std::max(c->m->E, c->m->F);

@@ -369,9 +369,9 @@ __global__ void __launch_bounds__(1024) matmul_mfma3_q4k_kernel(bamd_mma2_args a
 // each, four copy (all of it one after the other on four waves: 1230 ns a super-block at 37 tokens; copies spread over consumers and builders: 930 — a copy holds its wave until
 // the vector memory path takes it); the arithmetic, its order and the layouts are those above.  Everything a step reads travels global -> LDS by DMA — token records two
 // super-blocks ahead, the row tile's quants, scales and headers four — and the wait at the end of a step leaves what was issued in it (and the weights issued in the one before)
-// in flight, so that a step is not as long as the memory's latency.  37 tokens, 4096 rows: K = 4096 25.0 -> 12.9 us, K = 14336 77 -> 38 us (Q6_K 105 -> 46 us).  The copies of
-// the token records, the same to every block, were 24 us of the 38: of the tokens that there are and half a line out of step (BAMD_B16_MEM), 38 -> 34.6 us, a prompt 4681 -> 4511 (48 tokens,
-// no fewer copies, level).
+// in flight, so that a step is not as long as the memory's latency.  37 tokens, 4096 rows, launches one behind the other, 64-row blocks and this: K = 4096 24.7 and 11.3 us, K = 14336 77
+// and 31.4 (Q5_K 74 and 32.1, Q6_K on matmul_wide_kernel 84 and 44.6).  The copies of the token records are the same to every block: of the tokens that there are and half a line out of step
+// (BAMD_B16_MEM), a launch in a prompt 38 -> 34.6 us, a prompt 4681 -> 4511 (48 tokens, no fewer copies, level).  Without them the 31.4 us are 27.4 (Q6_K 38.5 of 44.6, 48 tokens 27.5 of 34.4).
 //   W slot of a super-block   Q4_K / Q5_K: 2 x 1 KiB quants of the two record groups | 1 KiB builder operands | 1 KiB consumer header | Q5_K: 2 x 256 B fifth bits
 //                             Q6_K: 2 x 1 KiB low bits | 2 x 512 B high bits | 2 x 1 KiB builder operands of the e-halves | 64 B of d
 template <int TYPE> struct FewW { static constexpr int SLOT = TYPE == BAMD_Q6_K ? 5184 : TYPE == BAMD_Q5_K ? 4608 : 4096, COPIES = TYPE == BAMD_Q4_K ? 1 : 2; };

@@ -15,7 +15,7 @@
 //     per super-block.  Quants and headers come through LDS too (private to the wave, two super-blocks ahead), which makes every request of the loop a counted copy; except with Q6_K on
 //     eight waves, where two registers are kept in scratch memory and the compiler's wait for the one it reads back at the top of a super-block waits for the copies in flight as well.
 // 2048 tokens, K = 4096, Q4_K, in a running prompt: 14336 rows 708 -> 523 us (343 -> 460 TFLOP/s), 6144 rows 312 -> 222, 4096 rows 216 -> 152; Q6_K, K = 14336, 4096 rows 880 -> 510.
-// Per super-block of 128 rows x 64 tokens 2.3 us; by itself the 14336-row launch takes 553 us (2.5 per super-block), 427 without the min pass, in Q5_K 528 and 453.  Tried: the eight e on two waves (four waves per SIMD, half the registers): 3.0
+// Per super-block of 128 rows x 64 tokens 2.1 us: by itself the 14336-row launch takes 471 us, 366 without the min pass, in Q5_K 459 and 394, in Q6_K 530.  Tried, when that was 2.3: the eight e on two waves (four waves per SIMD, half the registers): 3.0
 // us; matrix instructions and chains pinned in turn: no faster; a loop without a seam between super-blocks: 2.5 us, 3.4 for Q6_K.
 #include "bamd_device.h"
 #include "bamd_mfma_common.h"
