@@ -210,7 +210,7 @@ struct Ctx {
     unsigned char * dev = nullptr; int32_t * pages = nullptr;
     static constexpr int RING = 4;
     unsigned char * pinned = nullptr, * host[RING] = {}; int32_t * pages_host[RING] = {}; hipEvent_t ev[RING] = {}; int ring = 0;
-    std::map<std::array<int, 3>, hipGraphExec_t> graphs;          // rows, what is in front and behind (STEP_*), layers whose attention is one launch
+    std::map<std::array<int, 3>, hipGraphExec_t> graphs;          // rows, what is in front and behind (STEP_*), layers whose attention is one launch (kept as long as the context: no more than numbers of rows x STEP_* x choices that its steps have met)
     bamd_step_box * box = nullptr; uint32_t * count_serial = nullptr; uint32_t serial = 0;      // decoding steps by way of pinned memory; serial: of the last one
 };
 struct Pass {                                      // one pass through the layers
